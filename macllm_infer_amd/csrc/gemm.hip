@@ -9,8 +9,9 @@
 // products of a chunk in turn, wave 0 to 3), never on M, on the tiling or on the rows beside it: a
 // row's result is bit for bit the same alone, in a small step and in a large one.
 //
-// A step of up to 16 rows is bound by reading W once: every wave keeps eight 1 KiB fragments of it in
-// flight.  A large M re-reads x once per 64 features and W once per 64 rows, from the caches.
+// A step of up to 32 rows is bound by reading W once: every wave keeps its 1 KiB fragments in flight.  More rows are
+// bound by the matrix cores and go through tiled_f32_kernel, which shares its operands through LDS and keeps that
+// order of the sums (K a multiple of 32, rows of whole 16-byte pieces; other sizes stay with the first kernel).
 #include "common.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -126,6 +127,144 @@ gemm_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict__
   }
 }
 
+// Many rows: a group of 2 x 2 waves owns 32 MT rows x 32 NT features, stages 32 columns of both operands in LDS (two
+// buffers; the next stage is on its way to registers while this one is multiplied) and sums the four runs of chunks
+// one after the other, each from zero, adding the runs' sums in their order: bit for bit the sums above.
+// GROUPS = 4: four such groups of a workgroup take a run each and group 0 adds their tiles, for products of too few
+// tiles to fill 256 compute units one wave a SIMD (a wave's chain of products is then a quarter as long).
+// LDS: a row of a stage is eight 16-byte pieces; piece p of row r lies at r * 8 + (p ^ (r & 7)), so that the eight rows
+// that a quarter-wave reads at once fall into different banks, and a thread's stores are one run.
+// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32, 152 TFLOP/s in a large library product) where the tiles
+// fill the chip (512 x 4,096 x 1,024: 105 TFLOP/s, 86 with the waves' operands straight from the caches, each row of
+// 64 bytes a chunk), else the tiles' serial walk over K (512 x 1,024 x 2,048: 27 us, 53 before; 100 x 1,024 x 2,048: 16
+// us, 50 before).  A second stage on its way (102 TFLOP/s), 128 x 128 tiles (92) and an order of the tiles by die gain nothing.
+template <int MT, int NT, int GROUPS>
+__global__ void __launch_bounds__(GF_THREADS * GROUPS)
+tiled_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict__ W, long ldw,
+                 const float* __restrict__ bias, float* __restrict__ out, long ldo, bool whole, int M, int N, int K) {
+  constexpr int BM = 32 * MT, BN = 32 * NT, ROWS = BM + BN;
+  constexpr int PIECES = ROWS * 8 / GF_THREADS;                // 16-byte pieces a thread moves a stage
+  constexpr int STAGED = GROUPS * 2 * ROWS * 8, PARTIAL = (GROUPS - 1) * BM * BN / 4;
+  __shared__ floatx4 lds[STAGED > PARTIAL ? STAGED : PARTIAL];
+  const int group = GROUPS == 1 ? 0 : threadIdx.x / GF_THREADS;
+  const int tid = threadIdx.x % GF_THREADS;
+  const int lane = tid & (WAVE - 1);
+  const int wave = tid / WAVE;
+  const int q = lane / 16;
+  const int r = lane % 16;
+  const int first_m = (wave & 1) * MT * 16, first_n = (wave >> 1) * NT * 16;     // the wave's part of the tile
+  const long n0 = (long)blockIdx.x * BN;
+  const long m0 = (long)blockIdx.y * BM;
+  floatx4* const stage_of_group = lds + group * 2 * ROWS * 8;
+
+  const int chunks = K / 16;
+  const int run = (chunks + GF_WAVES - 1) / GF_WAVES;          // chunks of one of the four runs
+  const int first_chunk = group * run;
+  const int mine = GROUPS == 1 ? chunks : max(0, min(run, chunks - first_chunk));
+  const int stages = GROUPS == 1 ? chunks / 2 : (run + 1) / 2;
+  const float* source[PIECES];
+  int column[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int slot = p * GF_THREADS + tid;
+    const int row = slot / 8;
+    source[p] = row < BN ? W + min(n0 + row, (long)N - 1) * ldw : x + min(m0 + row - BN, (long)M - 1) * ldx;
+    column[p] = first_chunk * 16 + 4 * ((slot % 8) ^ (row & 7));
+  }
+  floatx4 on_the_way[PIECES];
+  auto ask = [&](int stage) {                                  // (columns past the row's end repeat its last ones and are not multiplied)
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+      on_the_way[p] = *reinterpret_cast<const floatx4*>(source[p] + min(column[p] + 32 * stage, K - 4));
+  };
+  auto lay_down = [&](int buffer) {
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) stage_of_group[buffer * ROWS * 8 + p * GF_THREADS + tid] = on_the_way[p];
+  };
+
+  floatx4 acc[NT][MT], total[NT][MT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = total[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  int left = run;
+  ask(0);
+  lay_down(0);
+  __syncthreads();
+  for (int stage = 0; stage < stages; ++stage) {
+    const floatx4* const staged = stage_of_group + (stage & 1) * ROWS * 8;
+    ask(stage + 1);
+    __builtin_amdgcn_sched_barrier(0);                         // the loads before the products, their stores to LDS behind them
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if (GROUPS > 1 && 2 * stage + c >= mine) continue;
+      floatx4 weights[NT], rows[MT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const int row = first_n + nt * 16 + r;
+        weights[nt] = staged[row * 8 + ((4 * c + q) ^ (row & 7))];
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int row = BN + first_m + mt * 16 + r;
+        rows[mt] = staged[row * 8 + ((4 * c + q) ^ (row & 7))];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(weights[nt][i], rows[mt][i], acc[nt][mt], 0, 0, 0);
+      if (GROUPS == 1 && --left == 0) {                        // a run ends
+        left = run;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            total[nt][mt] += acc[nt][mt];
+            acc[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    lay_down((stage + 1) & 1);
+    __syncthreads();
+  }
+
+  if (GROUPS > 1) {                                            // behind the loop's last barrier: the stages are read
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        if (group > 0) lds[((group - 1) * NT * MT + nt * MT + mt) * GF_THREADS + tid] = acc[nt][mt];
+    __syncthreads();
+    if (group > 0) return;
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      floatx4 value = total[nt][mt] + acc[nt][mt];             // (the last run's sum, or a shorter run's behind it)
+#pragma unroll
+      for (int g = 1; g < GROUPS; ++g) value += lds[((g - 1) * NT * MT + nt * MT + mt) * GF_THREADS + tid];
+      const long n = n0 + first_n + nt * 16 + 4 * q;
+      const long m = m0 + first_m + mt * 16 + r;
+      if (m >= M) continue;
+      if (bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) value[i] += bias[min(n + i, (long)N - 1)];
+      }
+      if (whole && n + 3 < N) {
+        *reinterpret_cast<floatx4*>(out + m * ldo + n) = value;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) out[m * ldo + n + i] = value[i];
+      }
+    }
+}
+
 template <int MT, int NT, int DEPTH>
 static void launch_gemm_f32(bool vec, dim3 grid, hipStream_t stream, const float* x, long ldx, const float* W,
                             long ldw, const float* bias, float* out, long ldo, int M, int N, int K) {
@@ -138,6 +277,31 @@ extern "C" int mi_gemm_f32(const float* x, long ldx, const float* W, long ldw, c
   if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldw < K || ldo < N) return ERR_BAD_ARGUMENT;
   const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && ((unsigned long long)x % 16) == 0 &&
                    ((unsigned long long)W % 16) == 0;
+  if (M > 32 && vec && K % 32 == 0) {
+    // The tiling that the rounds of workgroups over 256 compute units make cheapest: microseconds a round at K =
+    // 1,024, in tenths, as measured over 33 to 512 rows and 768 to 32,784 features (32 x 32 in four groups: 9.1, 15.7,
+    // 22.5, 28.7 for one to four rounds; 32 x 64 in four groups: 14.3, 28; 64 x 64 in one group: 24.5, 41, then two
+    // workgroups a compute unit hide each other's waits).  From 33 rows on the best of them is at least as fast as
+    // the first kernel at every size measured (64 x 1,024 x 2,048: 16 us against 21; 33 x 3,352 x 1,024: 9.7 against 11).
+    auto rounds = [&](long rows, long features) {
+      return (((M + rows - 1) / rows) * ((N + features - 1) / features) + 255) / 256;
+    };
+    const long small = 25 + 66 * rounds(32, 32), middle = 5 + 139 * rounds(32, 64);
+    const long large = rounds(64, 64) == 1 ? 245 : 205 * rounds(64, 64);
+    const bool whole = ldo % 4 == 0 && ((unsigned long long)out % 16) == 0;
+    const int bm = large < small && large < middle ? 64 : 32, bn = bm == 64 || middle < small ? 64 : 32;
+    const dim3 tiles((unsigned)(((long)N + bn - 1) / bn), (unsigned)(((long)M + bm - 1) / bm));
+    if (((long)M + bm - 1) / bm <= 65535) {
+      if (bm == 64)
+        tiled_f32_kernel<2, 2, 1><<<tiles, GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
+      else if (bn == 64)
+        tiled_f32_kernel<1, 2, 4><<<tiles, 4 * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
+      else
+        tiled_f32_kernel<1, 1, 4><<<tiles, 4 * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
+      RETURN_IF_LAUNCH_FAILED();
+      return 0;
+    }
+  }
   // rows and features of a workgroup: one tile of features while the step is small (W is read once, by as
   // many workgroups as there are tiles of it); 64 x 64 for many rows (x and W come from the caches)
   const int row_tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;

@@ -128,6 +128,22 @@ def test_float32_product_is_true_float32(ops, shape):
     assert (got.cpu() - (wide[:, 8:8 + K].double() @ w.double().T).float()).abs().max() < 2e-5 * math.sqrt(K)
 
 
+@pytest.mark.parametrize("shape", [(33, 70, 32), (65, 129, 96), (130, 2100, 96), (64, 1000, 224), (448, 4100, 160), (449, 4098, 1024)])
+def test_tiled_float32_product_sums_in_the_order_of_the_small_one(ops, shape):
+    """More than 32 rows with K a multiple of 32 go through the tiles that LDS shares (32 x 32, 32 x 64 and 64 x 64, runs
+    of chunks of unequal length, ragged edges, rows of the result that are no whole 16-byte pieces): the bits of the
+    product of a single row, and float32 rounding away from float64."""
+    M, N, K = shape
+    x, w, b = rand(M, K, seed=6).to(DEV), rand(N, K, seed=7).to(DEV), rand(N, seed=8).to(DEV)
+    got = ops.linear(x, w, b)
+    want = x.double() @ w.double().T + b.double()
+    # K products of N(0, 1) factors summed in four chains: below 2e-5 sqrt(K), as for the general kernel above
+    assert (got - want).abs().max() < 2e-5 * math.sqrt(K)
+    for row in (0, 15, 16, 31, 32, M - 1):
+        assert torch.equal(ops.linear(x[row:row + 1], w, b)[0], got[row]), row
+    assert torch.equal(ops.linear(x[:17], w, None), ops.linear(x, w, None)[:17])
+
+
 def test_mixed_product_keeps_a_32bit_weight(ops):
     x, w = rand(4, 96, seed=10, dtype=torch.bfloat16), rand(50, 96, seed=11)
     got = ops.linear(x.to(DEV), w.to(DEV), None)
