@@ -807,6 +807,31 @@ def test_penalties_match_the_plain_rule(ops):
     assert int(counts[0].sum()) == 0 and int(counts[1].sum()) == 0
 
 
+@pytest.mark.parametrize("V", [3, 700, 40000])
+def test_penalties_count_histories_longer_than_a_walk(ops, V):
+    """Histories around a workgroup's 1,024 tokens a trip and 4,096 a round, full of repeats: every token's penalties
+    once, the counts zero again, whatever shares them."""
+    generator = torch.Generator().manual_seed(V)
+    lengths = [1, 1023, 1024, 1025, 4096, 4097, 9001]
+    prompt_lens = [1, 0, 1024, 700, 4000, 4097, 5]
+    flat = torch.randint(0, V, (sum(lengths),), generator=generator, dtype=torch.int32)
+    offsets = i32([sum(lengths[:count]) for count in range(len(lengths) + 1)])
+    rows = len(lengths)
+    rep, pres, freq = (torch.rand(rows, generator=generator) + offset for offset in (0.6, -0.5, 0.0))
+    pres[::2] = freq[::2] = 0.0                      # a repetition penalty alone
+    source, extra_rows = i32([V - 1, 0]), i32([0, -1, 1, 0, -1, 1, 0])
+    logits = rand(rows, V, seed=V)
+    want = logits.clone()
+    ref_ops.apply_penalties(want, flat, offsets, i32(prompt_lens), rep, pres, freq, None, None, source, extra_rows)
+    got = logits.clone().to(DEV)
+    counts = [torch.zeros(rows * V, dtype=torch.int32, device=DEV) for _ in range(2)]
+    ops.apply_penalties(got, flat.to(DEV), offsets.to(DEV), i32(prompt_lens).to(DEV), rep.to(DEV), pres.to(DEV),
+                        freq.to(DEV), *counts, source.to(DEV), extra_rows.to(DEV))
+    # two float32 roundings of numbers up to the penalty of the commonest token
+    assert (got.cpu() - want).abs().max() <= 2 ** -22 * want.abs().max()
+    assert int(counts[0].sum()) == 0 and int(counts[1].sum()) == 0
+
+
 def test_allowed_tokens_keep_their_logits_and_the_rest_is_minus_infinity(ops):
     """Rows with a list keep exactly the listed logits (a list may name a token twice, and the last and the first of
     a vocabulary that is no multiple of anything); a row without one is untouched; argmax then takes the best
