@@ -102,6 +102,15 @@ _SIGNATURES = {
                               _c_long, _c_int, _c_ptr],
         "mi_tanh_rows": [_c_ptr, _c_int, _c_long, _c_ptr, _c_long, _c_int, _c_int, _c_ptr],
     },
+    "linear_matrix": {
+        "mi_linear_matrix_supported": [_c_int, _c_int, _c_int],
+        "mi_linear_matrix_run": [_c_int],
+        "mi_linear_matrix_chunk_tokens": [],
+        "mi_linear_matrix_floats": [_c_int, _c_int, _c_int, _c_int, _c_int],
+        "mi_linear_matrix_scan": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr,
+                                  _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_int,
+                                  _c_ptr, _c_long, _c_ptr, _c_float, _c_float, _c_ptr, _c_ptr, _c_long, _c_ptr],
+    },
     "linear_chunk": {
         "mi_linear_chunk_supported": [_c_int, _c_int],
         "mi_linear_chunk_tokens": [],
@@ -1152,6 +1161,72 @@ def linear_state_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, nu
         _p(decay_logits), logits_ld, _p(decay_bias), float(decay_floor), float(key_eps),
         float(gate_power) if gated else 0.0, float(query_scale), 1 if silu else 0, _stream()),
         "linear_state_scan", f"(dk={dk}, dv={dv})")
+
+
+# the delta rule's matrices hold the reciprocal of a run's decays: its logarithm stays this far within float32's range
+LINEAR_MATRIX_MOST_LOG = 60.0
+
+
+def linear_matrix_supported(dtype, key_dim: int, value_dim: int, decay_floor: Optional[float] = None) -> bool:
+    """Whether the float32 matrix-core kernels of retention (``decay_floor`` None) or of the delta rule cover these heads
+    and, for the delta rule, this strongest decay."""
+    delta = decay_floor is not None
+    if dtype != torch.bfloat16 or not _fn("linear_matrix", "mi_linear_matrix_supported")(int(delta), int(key_dim), int(value_dim)):
+        return False
+    run = _fn("linear_matrix", "mi_linear_matrix_run")(int(delta))
+    return not delta or 0.0 <= decay_floor * run <= LINEAR_MATRIX_MOST_LOG
+
+
+def linear_matrix_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, num_heads: int, key_dim: int, value_dim: int,
+                       state: torch.Tensor, slot_ids: torch.Tensor, out: torch.Tensor, chunks,
+                       head_decay: Optional[torch.Tensor] = None, key_scale: float = 1.0,
+                       positions: Optional[torch.Tensor] = None, inv_freq: Optional[torch.Tensor] = None, rotary_dim: int = 0,
+                       removal_col: int = -1, decay_logits: Optional[torch.Tensor] = None,
+                       decay_bias: Optional[torch.Tensor] = None, decay_floor: float = 0.0, key_eps: float = 0.0) -> None:
+    """``linear_state_scan`` (retention, or with ``removal_col`` >= 0 the delta rule) for prompt portions in bfloat16, a run
+    of tokens at a time on the float32 matrix cores: the same arguments, and ``chunks``, the step's lanes cut into chunks of
+    128 tokens (``chunks`` int32 [n, 4], ``lane_chunks`` int32 [lanes, 2], ``num_chunks``, ``chunk_size``)."""
+    ld = _row_major(u, "u")
+    T = u.shape[0]
+    H, dk, dv = int(num_heads), int(key_dim), int(value_dim)
+    delta = removal_col >= 0
+    _need(linear_matrix_supported(u.dtype, dk, dv, decay_floor if delta else None),
+          "linear_matrix_scan: heads not covered; use linear_state_scan")
+    widest = max(q_col + H * dk, k_col + H * dk, v_col + H * dv, removal_col + H * dk if delta else 0)
+    _need(min(q_col, k_col, v_col) >= 0 and u.shape[1] >= widest, "linear_matrix_scan: u is too narrow for its columns")
+    _need(state.dtype == torch.float32 and state.dim() == 4 and state.shape[1:] == (H, dv, dk) and state.is_contiguous()
+          and state.is_cuda, "linear_matrix_scan: state must be contiguous float32 [slots, H, dv, dk] on the GPU")
+    _need(out.dtype == torch.float32 and out.shape == (T, H * dv) and out.is_contiguous(),
+          "linear_matrix_scan: out must be contiguous float32 [T, H * dv]")
+    logits_ld = 0
+    if delta:
+        _need(decay_logits is not None and decay_logits.dtype == torch.float32 and decay_logits.shape == (T, H * dk),
+              "linear_matrix_scan: decay_logits must be float32 [T, H * dk]")
+        logits_ld = _row_major(decay_logits, "decay_logits")
+        _need(decay_bias is not None and decay_bias.dtype == torch.float32 and decay_bias.numel() == H * dk
+              and decay_bias.is_contiguous() and decay_bias.is_cuda, "linear_matrix_scan: decay_bias must be float32 [H * dk]")
+    else:
+        _need(head_decay is not None and head_decay.dtype == torch.float32 and head_decay.numel() == H
+              and head_decay.is_cuda, "linear_matrix_scan: head_decay must be float32 [H] on the GPU")
+    if inv_freq is not None:
+        _i32(positions, "positions")
+        _need(not delta and positions.numel() == T and inv_freq.dtype == torch.float32 and inv_freq.numel() == rotary_dim // 2
+              and inv_freq.is_cuda and 0 < rotary_dim <= dk, "linear_matrix_scan: the rotation does not fit the heads")
+    _i32(slot_ids, "slot_ids")
+    _i32(chunks.chunks, "chunks")
+    _i32(chunks.lane_chunks, "lane_chunks")
+    lanes, count = slot_ids.numel(), int(chunks.num_chunks)
+    _need(chunks.chunk_size == _fn("linear_matrix", "mi_linear_matrix_chunk_tokens")() and count > 0
+          and chunks.chunks.numel() >= 4 * count and chunks.lane_chunks.numel() >= 2 * lanes,
+          "linear_matrix_scan: the chunk table does not cover the step")
+    local = torch.empty((_fn("linear_matrix", "mi_linear_matrix_floats", _c_long)(int(delta), count, H, dk, dv),),
+                        dtype=torch.float32, device=u.device)
+    _check(_fn("linear_matrix", "mi_linear_matrix_scan")(
+        _p(u), ld, int(q_col), int(k_col), int(v_col), int(removal_col), H, dk, dv, _p(state), _p(slot_ids), lanes,
+        _p(chunks.chunks), _p(chunks.lane_chunks), count, int(chunks.chunk_size), _p(head_decay), float(key_scale),
+        _p(positions) if inv_freq is not None else None, _p(inv_freq), int(rotary_dim) if inv_freq is not None else 0,
+        _p(decay_logits), logits_ld, _p(decay_bias), float(decay_floor), float(key_eps), _p(local), _p(out), out.stride(0),
+        _stream()), "linear_matrix_scan", f"(dk={dk}, dv={dv}, chunks={count})")
 
 
 def linear_chunk_supported(dtype, key_dim: int, value_dim: int) -> bool:

@@ -41,12 +41,28 @@ def chunk_table(step):
     return step.derived[key]
 
 
+# Tokens of the longest lane from which on runs of tokens on the matrix cores are faster than the walk token by token
+MATRIX_FROM = 32
+
+
+def run_scan(u: torch.Tensor, step, columns: dict, recurrence: dict) -> None:
+    """The scan of retention or the delta rule: a run of tokens at a time on the float32 matrix cores for prompt portions in
+    bfloat16 whose heads those kernels cover, else token by token (single tokens, short portions, float32, other sizes)."""
+    floor = recurrence.get("decay_floor")
+    if (u.is_cuda and step.max_query_len >= MATRIX_FROM
+            and ops.linear_matrix_supported(u.dtype, columns["key_dim"], columns["value_dim"], floor)):
+        ops.linear_matrix_scan(u, **columns, **recurrence, slot_ids=step.slot_ids, chunks=chunk_table(step))
+        return
+    ops.linear_state_scan(u, **columns, **recurrence, cu_seqlens=step.cu_seqlens, slot_ids=step.slot_ids,
+                          max_query_len=step.max_query_len, chunks=scan_chunks(step))
+
+
 @register_part("retention")
 class Retention(Mixer):
     """[q | k | v | g] = one projection of the normed rows; q and k rotated by position, k scaled;
     S <- decay[h] S + k v^T, o = S^T q per head; o / rms(o) per head, times SiLU(g), output projection."""
     graph_safe = True
-    kernel_modules = ("common", "linear_state", "gemm")
+    kernel_modules = ("common", "linear_state", "linear_matrix", "gemm")
     chunk_tokens = CHUNK_TOKENS
 
     @classmethod
@@ -88,11 +104,10 @@ class Retention(Mixer):
         keys, values = spec.num_heads * spec.key_dim, spec.num_heads * spec.value_dim
         u = self.in_proj(x)                                              # [T, q | k | v | g]
         raw = torch.empty((x.shape[0], values), dtype=torch.float32, device=x.device)
-        ops.linear_state_scan(u, q_col=0, k_col=keys, v_col=2 * keys, num_heads=spec.num_heads, key_dim=spec.key_dim,
-                              value_dim=spec.value_dim, state=cache.states["state"], cu_seqlens=step.cu_seqlens,
-                              slot_ids=step.slot_ids, out=raw, max_query_len=step.max_query_len,
-                              head_decay=self.decay, key_scale=spec.key_scale, positions=step.positions,
-                              inv_freq=self.inv_freq, rotary_dim=self.rotary_dim, chunks=scan_chunks(step))
+        run_scan(u, step, dict(q_col=0, k_col=keys, v_col=2 * keys, num_heads=spec.num_heads, key_dim=spec.key_dim,
+                               value_dim=spec.value_dim, state=cache.states["state"], out=raw),
+                 dict(head_decay=self.decay, key_scale=spec.key_scale, positions=step.positions, inv_freq=self.inv_freq,
+                      rotary_dim=self.rotary_dim))
         gated = torch.empty((x.shape[0], values), dtype=u.dtype, device=x.device)
         ops.head_norm_gate(raw, u[:, 2 * keys + values:], None, spec.num_heads, spec.norm_eps, "silu", gated)
         return self.out_proj(gated)
@@ -105,7 +120,7 @@ class GeneralDelta(Mixer):
     a = sigmoid(a part), u = k / sqrt(sum k^2 + key_eps), S <- diag(w) S - (a u)(u^T S) + k v^T, o = S^T r;
     then o / rms(o) per head times the weight ``norm``, times sigmoid(g), output projection."""
     graph_safe = True
-    kernel_modules = ("common", "linear_state", "gemm")
+    kernel_modules = ("common", "linear_state", "linear_matrix", "gemm")
     chunk_tokens = CHUNK_TOKENS
 
     @classmethod
@@ -157,12 +172,10 @@ class GeneralDelta(Mixer):
         ops.tanh_rows(u[:, 5 * inner:], bent)
         logits = ops.linear(bent, self.decay_proj.weight, None, keep_float32=True)     # float32 [T, inner]
         raw = torch.empty((x.shape[0], inner), dtype=torch.float32, device=x.device)
-        ops.linear_state_scan(u, q_col=0, k_col=inner, v_col=2 * inner, num_heads=spec.num_heads,
-                              key_dim=spec.head_dim, value_dim=spec.head_dim, state=cache.states["state"],
-                              cu_seqlens=step.cu_seqlens, slot_ids=step.slot_ids, out=raw,
-                              max_query_len=step.max_query_len, removal_col=4 * inner, decay_logits=logits,
-                              decay_bias=self.decay_bias, decay_floor=spec.decay_floor, key_eps=spec.key_eps,
-                              chunks=scan_chunks(step))
+        run_scan(u, step, dict(q_col=0, k_col=inner, v_col=2 * inner, num_heads=spec.num_heads, key_dim=spec.head_dim,
+                               value_dim=spec.head_dim, state=cache.states["state"], out=raw),
+                 dict(removal_col=4 * inner, decay_logits=logits, decay_bias=self.decay_bias, decay_floor=spec.decay_floor,
+                      key_eps=spec.key_eps))
         gated = torch.empty((x.shape[0], inner), dtype=u.dtype, device=x.device)
         ops.head_norm_gate(raw, u[:, 3 * inner:4 * inner], self.norm_weight, spec.num_heads, spec.norm_eps, "sigmoid",
                            gated)

@@ -124,6 +124,62 @@ def test_scans_walk_lanes_and_chunks_alike(dtype, delta, H, dk, dv, rotary):
         assert float((got_state - want_state).abs().max()) <= 2e-4 * max(1.0, float(want_state.abs().max())), name
 
 
+@pytest.mark.parametrize("delta, H, dk, dv, rotary", [
+    (False, 2, 64, 16, 0), (False, 3, 64, 128, 64), (False, 1, 64, 64, 20), (False, 1, 128, 256, 128),
+    (True, 2, 64, 64, 0), (True, 1, 64, 16, 0), (True, 1, 64, 192, 0), (True, 2, 128, 128, 0)])
+def test_runs_on_the_matrix_cores_give_the_walk_s_numbers(delta, H, dk, dv, rotary):
+    """Lanes that end around the edges of tiles (16), runs (32, 64) and chunks (128) and one of several chunks, from states
+    that are not empty in slots out of order, rows that begin at odd columns, decays of one and of zero: as far from a
+    float64 recurrence as float32 rounding puts the walk."""
+    from macllm_infer_amd.kernels import ops, build
+    build.ensure_modules(["linear_state", "linear_matrix"])
+    lengths = [1, 15, 16, 17, 31, 33, 63, 64, 65, 127, 128, 129, 300]
+    T, lanes = sum(lengths), len(lengths)
+    generator = torch.Generator().manual_seed(dk + dv)
+    u = (torch.randn(T, 1 + 3 * H * dk + H * dv + 3, generator=generator) * 0.7).to(torch.bfloat16)
+    state = torch.randn(lanes + 2, H, dv, dk, generator=generator) * 0.3
+    cu = torch.tensor([0] + list(np.cumsum(lengths)), dtype=torch.int32)
+    slots = torch.randperm(lanes + 2, generator=generator)[:lanes].to(torch.int32)
+    columns = dict(q_col=1, k_col=1 + H * dk, v_col=1 + 2 * H * dk, num_heads=H, key_dim=dk, value_dim=dv)
+    if delta:
+        recurrence = dict(removal_col=1 + 2 * H * dk + H * dv, decay_logits=torch.randn(T, H * dk, generator=generator) * 3.0,
+                          decay_bias=torch.randn(H * dk, generator=generator), decay_floor=math.exp(-0.5), key_eps=1e-6)
+    else:
+        recurrence = dict(head_decay=torch.tensor([0.97, 1.0, 0.0][:H]), key_scale=dk ** -0.5)
+        if rotary:
+            recurrence.update(positions=torch.arange(T, dtype=torch.int32) * 3 % 5000, rotary_dim=rotary,
+                              inv_freq=torch.tensor([1e4 ** (-2.0 * i / rotary) for i in range(rotary // 2)]))
+    double = lambda values: {name: value.double() if isinstance(value, torch.Tensor) and value.is_floating_point() else value
+                             for name, value in values.items()}
+    want, want_state = torch.zeros(T, H * dv, dtype=torch.float64), state.double()
+    before = ref_ops._f
+    ref_ops._f = lambda value: value.double()
+    try:
+        ref_ops.linear_state_scan(u, **columns, **double(recurrence), state=want_state, cu_seqlens=cu, slot_ids=slots, out=want)
+    finally:
+        ref_ops._f = before
+    on = lambda values: {name: value.to(DEV) if isinstance(value, torch.Tensor) else value for name, value in values.items()}
+    assert ops.linear_matrix_supported(torch.bfloat16, dk, dv, recurrence.get("decay_floor"))
+    got, got_state = torch.full((T, H * dv), float("nan"), device=DEV), state.clone().to(DEV)
+    ops.linear_matrix_scan(u.to(DEV), **columns, **on(recurrence), state=got_state, slot_ids=slots.to(DEV), out=got,
+                           chunks=ops.SsdChunks(lengths, 128, DEV))
+    # outputs are sums of some dk float32 products of terms up to the outputs' own scale: 2^-24 sqrt(dk) of it a rounding, and
+    # the angles of a rotation are products in float32 (up to 5,000 radians, half a unit in the last place of that: 2.4e-4)
+    bound = (2e-6 if not rotary else 5e-4) * float(want.abs().max())
+    assert float((got.cpu().double() - want).abs().max()) <= bound
+    assert float((got_state.cpu().double() - want_state).abs().max()) <= (2e-6 if not rotary else 5e-4) * float(want_state.abs().max())
+    untouched = sorted(set(range(lanes + 2)) - set(slots.tolist()))
+    assert torch.equal(got_state.cpu()[untouched], state[untouched])
+
+
+def test_heads_the_matrix_cores_do_not_cover_stay_with_the_walk():
+    from macllm_infer_amd.kernels import ops
+    covered = lambda *sizes, dtype=torch.bfloat16, floor=None: ops.linear_matrix_supported(dtype, *sizes, floor)
+    assert covered(64, 256) and covered(128, 128, floor=0.6) and not covered(64, 64, dtype=torch.float32)
+    assert not covered(32, 64) and not covered(64, 24) and not covered(96, 96) and not covered(64, 272)
+    assert not covered(128, 144, floor=0.6) and not covered(64, 64, floor=2.0) and not covered(64, 64, floor=-1.0)
+
+
 # ------------------------------------------------------------------ the parts alone
 def attention_tensors(hidden, H, G, D, V, seed):
     return {"q_proj.weight": rand(H * D, hidden, seed=seed + 1, scale=hidden ** -0.5),
