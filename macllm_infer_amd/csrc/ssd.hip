@@ -524,13 +524,13 @@ ssd_chunk_scan_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t*
   }
 }
 
+#define SSD_SCAN_WAVES 8
 // The same with the operands that the eight tiles of 128 tokens share staged in LDS: one
 // workgroup of eight waves per (chunk, head, 128 tokens), a tile of 16 tokens a wave.  S_in of
 // the head (64 rows at a time), then, 64 tokens s at a time, the rows of B and the columns of
 // x^T go through LDS once for all tiles instead of once per tile from the caches; only C, the
 // skip and the gate are read per tile.  Rows are padded by 16 bytes so that the 16 rows a
 // matrix-core operand reads fall in different banks.  Head sizes up to 128.
-#define SSD_SCAN_WAVES 8
 template <int NK, int PT>
 __global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
 ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
@@ -718,6 +718,317 @@ ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf1
   }
 }
 
+// ---------------------------------------------------------------- lanes of one chunk
+// Every lane of the step is one chunk of at most SSD_SINGLE_TOKENS tokens, so that a chunk starts from its request's state
+// and leaves it: the chunk's state, the pass and the scan in one launch, with their products and sums in their order (the
+// state read in float32, rounded to bfloat16 where it is an operand of the outputs, as the pass rounds it).  One workgroup
+// of eight waves a (lane, head), a tile of 16 tokens a wave; rows of the grid past the heads update the lanes' conv tails,
+// as in the pass.  A short prompt waits for round trips, not for bytes: everything that the first 64 tokens need, the old
+// state and the operands of the new one are asked for at the top and laid in LDS behind one barrier.  37 tokens, 24 heads
+// of 64 x 128: 8.0 + 7.0 + 7.8 us in three launches, 13.5 in this one (14.7 with every stage asking for its own).
+#define SSD_SINGLE_TOKENS (SSD_SCAN_WAVES * 16)
+struct SsdSingle {
+  float* state;                    // [slots, H, P, N]
+  const int* slot_ids;
+  const bf16_t* u;                 // the conv's raw rows and tails, where the conv ran in the launch before
+  long u_ld;
+  int C, K;
+  bf16_t* conv_state;
+  const int* lane_chunks;
+};
+template <int NK, int PT>
+__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
+ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                  const float* __restrict__ delta, const float* __restrict__ cum, const float* __restrict__ D,
+                  const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y, long y_ld,
+                  const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated, long gated_ld, const SsdSingle one) {
+  constexpr int N = 32 * NK;
+  constexpr int P = 16 * PT;
+  constexpr int LD1 = N + 8;                     // row stride of the S and B buffers
+  constexpr int LDX = 64 + 8;                    // row stride of the x^T buffer
+  constexpr int THREADS = SSD_SCAN_WAVES * WAVE;
+  constexpr int S_PIECES = (P * (N / 8) + THREADS - 1) / THREADS;      // eight elements a piece
+  constexpr int B_PIECES = (64 * (N / 8) + THREADS - 1) / THREADS;
+  constexpr int X_PIECES = (P * 8 + THREADS - 1) / THREADS;
+  constexpr int QK = SSD_SINGLE_TOKENS / 32;
+  constexpr int PB = PT < 4 ? PT : 4;            // tiles of state rows that share the weighted B fragments
+  constexpr int ITEMS = (N / 16) * (PT / PB);
+  extern __shared__ __align__(16) unsigned char scan_smem[];
+  bf16_t* s_rows = reinterpret_cast<bf16_t*>(scan_smem);               // [P][LD1]
+  bf16_t* b_lds = s_rows + P * LD1;                                    // [64][LD1]
+  bf16_t* x_lds = b_lds + 64 * LD1;                                    // [P][LDX]
+  float* L = reinterpret_cast<float*>(x_lds + P * LDX);                // [SSD_SINGLE_TOKENS] each
+  float* step = L + SSD_SINGLE_TOKENS;
+  float* weight = step + SSD_SINGLE_TOKENS;
+  const int chunk = blockIdx.x;
+  const int head = blockIdx.y;
+  const int step_lane = chunks[4 * chunk];
+  const int t0 = chunks[4 * chunk + 1];
+  const int length = chunks[4 * chunk + 2];
+  if (length <= 0) return;                    // a row of the table past the step's own chunks: the whole workgroup leaves
+  const int tid = threadIdx.x;
+  if (head >= H) {
+    ssd_tail_block(one.u, one.u_ld, one.C, one.K, one.conv_state, chunks, one.lane_chunks, one.slot_ids, Q, step_lane,
+                   (head - H) * THREADS + tid);
+    return;
+  }
+  const int group = head / (H / G);
+  const int lane = tid & (WAVE - 1);
+  const int wave = tid / WAVE;
+  const int q = lane / 16;
+  const int n = lane % 16;
+  const int GN = G * N;
+  const int b_col = E + group * N;
+  const int c_col = E + GN + group * N;
+  const int t = wave * 16 + n;
+  const bool tile_live = wave * 16 < length;
+  const bool has_t = t < length;
+  const long t_row = t0 + min(t, length - 1);
+  float* const slot = one.state + ((long)one.slot_ids[step_lane] * H + head) * P * N;
+  const bf16_t* x_rows = TT + ((long)chunk * (E + GN) + (long)head * P) * Q;
+  const bf16_t* b_rows = TT + ((long)chunk * (E + GN) + E + (long)group * N) * Q;
+
+  // ---- everything is asked for
+  const int token = min(tid, length - 1);
+  const float own_cum = cum[(long)(t0 + token) * H + head];            // (the first 128 threads' count)
+  const float own_delta = delta[(long)(t0 + token) * H + head];
+  s_bf16x8 c_frag[NK], b_piece[B_PIECES], x_piece[X_PIECES];
+  s_floatx4 s_piece[S_PIECES][2];
+#pragma unroll
+  for (int i = 0; i < S_PIECES; ++i) {
+    const int at = min(tid + i * THREADS, P * (N / 8) - 1) * 8;        // (the state of a head is one run)
+    s_piece[i][0] = *reinterpret_cast<const s_floatx4*>(slot + at);
+    s_piece[i][1] = *reinterpret_cast<const s_floatx4*>(slot + at + 4);
+  }
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk)
+    c_frag[kk] = *reinterpret_cast<const s_bf16x8*>(xbc + t_row * xbc_ld + c_col + 32 * kk + 8 * q);
+  auto ask_block = [&](int sb) {                                       // 64 tokens s: B's rows and x^T's columns
+#pragma unroll
+    for (int i = 0; i < B_PIECES; ++i) {
+      const int index = min(tid + i * THREADS, 64 * (N / 8) - 1);
+      const long row = t0 + min(64 * sb + index / (N / 8), length - 1);
+      b_piece[i] = *reinterpret_cast<const s_bf16x8*>(xbc + row * xbc_ld + b_col + 8 * (index % (N / 8)));
+    }
+#pragma unroll
+    for (int i = 0; i < X_PIECES; ++i) {
+      const int index = min(tid + i * THREADS, P * 8 - 1);
+      const int at = 64 * sb + 8 * (index % 8);                        // (past Q: the last there are, whose weights are zero)
+      x_piece[i] = *reinterpret_cast<const s_bf16x8*>(x_rows + (long)(index / 8) * Q + min(at, Q - 8));
+    }
+  };
+  auto lay_block = [&]() {
+#pragma unroll
+    for (int i = 0; i < B_PIECES; ++i) {
+      const int index = tid + i * THREADS;
+      if (index < 64 * (N / 8)) *reinterpret_cast<s_bf16x8*>(b_lds + (index / (N / 8)) * LD1 + 8 * (index % (N / 8))) = b_piece[i];
+    }
+#pragma unroll
+    for (int i = 0; i < X_PIECES; ++i) {
+      const int index = tid + i * THREADS;
+      if (index < P * 8) *reinterpret_cast<s_bf16x8*>(x_lds + (index / 8) * LDX + 8 * (index % 8)) = x_piece[i];
+    }
+  };
+  ask_block(0);
+  s_bf16x8 b_raw[QK], x[PB][QK];
+  s_floatx4 before[PB];
+  auto ask_state = [&](int item) {
+    const int nt = item % (N / 16), pt0 = item / (N / 16) * PB;
+#pragma unroll
+    for (int ks = 0; ks < QK; ++ks)
+      b_raw[ks] = *reinterpret_cast<const s_bf16x8*>(b_rows + (long)(nt * 16 + n) * Q + min(32 * ks, Q - 32) + 8 * q);
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+#pragma unroll
+      for (int ks = 0; ks < QK; ++ks)
+        x[i][ks] = *reinterpret_cast<const s_bf16x8*>(x_rows + (long)((pt0 + i) * 16 + n) * Q + min(32 * ks, Q - 32) + 8 * q);
+      before[i] = *reinterpret_cast<const s_floatx4*>(slot + (long)((pt0 + i) * 16 + n) * N + nt * 16 + 4 * q);
+    }
+  };
+  constexpr bool EARLY = NK <= 4;                // (256 state columns and the operands of the new state do not fit the registers)
+  if (EARLY) ask_state(min(wave, ITEMS - 1));
+  s_bf16x4 x_skip[PT], gate[PT];
+#pragma unroll
+  for (int pi = 0; pi < PT; ++pi) {
+    const long column = (long)head * P + pi * 16 + 4 * q;
+    x_skip[pi] = *reinterpret_cast<const s_bf16x4*>(xbc + t_row * xbc_ld + column);
+    gate[pi] = *reinterpret_cast<const s_bf16x4*>((z != nullptr ? z + t_row * z_ld : xbc + t_row * xbc_ld) + column);
+  }
+
+  // ---- and laid down
+  if (tid < SSD_SINGLE_TOKENS) {
+    L[tid] = own_cum;
+    step[tid] = own_delta;
+  }
+#pragma unroll
+  for (int i = 0; i < S_PIECES; ++i) {
+    const int index = tid + i * THREADS;
+    s_bf16x8 value;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      value[e] = (bf16_t)s_piece[i][0][e];
+      value[4 + e] = (bf16_t)s_piece[i][1][e];
+    }
+    if (index < P * (N / 8)) *reinterpret_cast<s_bf16x8*>(s_rows + (index / (N / 8)) * LD1 + 8 * (index % (N / 8))) = value;
+  }
+  lay_block();
+  if (!has_t) {
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) c_frag[kk][j] = (bf16_t)0.f;
+  }
+  __syncthreads();
+  const float total = L[length - 1];
+  if (tid < SSD_SINGLE_TOKENS) weight[tid] = tid < length ? __expf(total - own_cum) * own_delta : 0.f;
+
+  // ---- the state's part of the outputs, then the chunk's own tokens, 64 at a time
+  s_floatx4 acc[PT];
+#pragma unroll
+  for (int pi = 0; pi < PT; ++pi) acc[pi] = s_floatx4{0.f, 0.f, 0.f, 0.f};
+  const float l_t = L[min(t, length - 1)];
+  if (tile_live) {
+    const float carry = __expf(l_t);
+#pragma unroll
+    for (int pi = 0; pi < PT; ++pi) {
+#pragma unroll
+      for (int kk = 0; kk < NK; ++kk) {
+        const s_bf16x8 a = *reinterpret_cast<const s_bf16x8*>(s_rows + (pi * 16 + n) * LD1 + 32 * kk + 8 * q);
+        acc[pi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, c_frag[kk], acc[pi], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[pi][i] *= carry;
+    }
+  }
+  for (int sb = 0; sb * 64 < length; ++sb) {
+    if (sb > 0) {
+      ask_block(sb);
+      __syncthreads();                                                 // the block before is read
+      lay_block();
+      __syncthreads();
+    }
+    if (!tile_live) continue;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int s0 = sb * 64 + 32 * j;
+      if (s0 > wave * 16 + 15 || s0 >= length) continue;
+      s_floatx4 w[2];
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        w[half] = s_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+          const s_bf16x8 a = *reinterpret_cast<const s_bf16x8*>(b_lds + (32 * j + 16 * half + n) * LD1 + 32 * kk + 8 * q);
+          w[half] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, c_frag[kk], w[half], 0, 0, 0);
+        }
+      }
+      s_bf16x8 p_frag;
+#pragma unroll
+      for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = s0 + 16 * half + 4 * q + i;
+          const int s_safe = min(s, length - 1);
+          const bool visible = has_t && s <= t && s < length;
+          const float value = visible ? w[half][i] * __expf(l_t - L[s_safe]) * step[s_safe] : 0.f;
+          p_frag[4 * half + i] = (bf16_t)value;
+        }
+#pragma unroll
+      for (int pi = 0; pi < PT; ++pi) {
+        const bf16_t* x_row = x_lds + (pi * 16 + n) * LDX + 32 * j + 4 * q;
+        const s_bf16x4 lo = *reinterpret_cast<const s_bf16x4*>(x_row);
+        const s_bf16x4 hi = *reinterpret_cast<const s_bf16x4*>(x_row + 16);
+        s_bf16x8 a;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          a[e] = lo[e];
+          a[4 + e] = hi[e];
+        }
+        acc[pi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, p_frag, acc[pi], 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();                                                     // the weights are there
+
+  // ---- the state the chunk leaves: sum_s weight_s x_s (outer) B_s beside what is left of the old one
+  const float decay = __expf(total);
+  for (int item = wave; item < ITEMS; item += SSD_SCAN_WAVES) {
+    const int nt = item % (N / 16), pt0 = item / (N / 16) * PB;
+    if (!EARLY || item != wave) ask_state(item);
+    s_floatx4 sum[PB];
+#pragma unroll
+    for (int i = 0; i < PB; ++i) sum[i] = s_floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < QK; ++ks) {
+      s_bf16x8 a;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] = (bf16_t)((float)b_raw[ks][j] * weight[32 * ks + 8 * q + j]);
+#pragma unroll
+      for (int i = 0; i < PB; ++i) sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, x[i][ks], sum[i], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) before[i][j] = decay * before[i][j] + sum[i][j];
+      *reinterpret_cast<s_floatx4*>(slot + (long)((pt0 + i) * 16 + n) * N + nt * 16 + 4 * q) = before[i];
+    }
+  }
+
+  // ---- y[t, h*P + 16 pi + 4q + i] = acc + D x
+  if (!has_t) return;
+  const float skip = D[head];
+#pragma unroll
+  for (int pi = 0; pi < PT; ++pi) {
+    const long column = (long)head * P + pi * 16 + 4 * q;
+    s_floatx4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = acc[pi][i] + skip * (float)x_skip[pi][i];
+    if (z != nullptr) {
+      s_bf16x4 packed;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)(out[i] * silu_bf16_f((float)gate[pi][i]));
+      *reinterpret_cast<s_bf16x4*>(gated + t_row * gated_ld + column) = packed;
+    } else {
+      *reinterpret_cast<s_floatx4*>(y + t_row * y_ld + column) = out;
+    }
+  }
+}
+
+static size_t ssd_single_lds_bytes(int P, int N) {
+  return (size_t)(P + 64) * (N + 8) * 2 + (size_t)P * (64 + 8) * 2 + (size_t)3 * SSD_SINGLE_TOKENS * 4;
+}
+
+static bool ssd_staged_sizes(int P, int N) {
+  return (P == 16 || P == 32 || P == 64 || P == 128) && (N == 32 || N == 64 || N == 128 || N == 256);
+}
+
+// Whether a step whose longest lane holds `longest` tokens (0: not known) is worked on in one launch behind the conv.
+extern "C" int mi_ssd_single(int Q, int P, int N, int longest) {
+  return longest > 0 && longest <= Q && longest <= SSD_SINGLE_TOKENS && ssd_staged_sizes(P, N) ? 1 : 0;
+}
+
+template <int NK, int PT>
+static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, long xbc_ld, const bf16_t* TT, int E,
+                             const float* delta, const float* cum, const float* D, const int* chunks, int Q, int H, int G,
+                             float* y, long y_ld, const bf16_t* z, long z_ld, bf16_t* gated, long gated_ld,
+                             const SsdSingle& one) {
+  const size_t lds = ssd_single_lds_bytes(16 * PT, 32 * NK);
+  // beyond 64 KiB a kernel has to be told once per device that it may have that much (gfx950 has 160 KiB)
+  static bool told[64] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return ERR_BAD_ARGUMENT;
+  if (lds > 64 * 1024 && !told[device]) {
+    if (hipFuncSetAttribute((const void*)ssd_single_kernel<NK, PT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+      (void)hipGetLastError();
+      return ERR_UNSUPPORTED_SIZE;
+    }
+    told[device] = true;
+  }
+  ssd_single_kernel<NK, PT><<<grid, SSD_SCAN_WAVES * WAVE, lds, stream>>>(xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y,
+                                                                          y_ld, z, z_ld, gated, gated_ld, one);
+  return 0;
+}
+
 static size_t ssd_scan_lds_bytes(int Q, int P, int N) {
   return (size_t)64 * (N + 8) * 2 + (size_t)P * (64 + 8) * 2 + (size_t)2 * Q * 4;
 }
@@ -736,7 +1047,7 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
                               int G, float* delta, float* cum, void* TT, float* chunk_state,
                               float* chunk_decay, void* state_in, float* y, long y_ld, const void* z, long z_ld,
                               void* gated, long gated_ld, const void* u, long u_ld, const float* conv_w,
-                              const float* conv_b, void* conv_state, int conv_k, hipStream_t stream) {
+                              const float* conv_b, void* conv_state, int conv_k, int longest, hipStream_t stream) {
   if (n_chunks <= 0 || n_lanes <= 0 || H <= 0 || G <= 0 || H % G != 0) return ERR_BAD_ARGUMENT;
   const int E = H * P;
   const int GN = G * N;
@@ -769,6 +1080,25 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
                                                            (const bf16_t*)xbc, xbc_ld, E + GN, Q, (bf16_t*)TT);
     RETURN_IF_LAUNCH_FAILED();
   }
+  if (mi_ssd_single(Q, P, N, longest)) {
+    const int tail_rows = conv_here ? (C + SSD_SCAN_WAVES * WAVE - 1) / (SSD_SCAN_WAVES * WAVE) : 0;
+    const SsdSingle one = {ssm_state, slot_ids, (const bf16_t*)u, u_ld, C, conv_k, (bf16_t*)conv_state, lane_chunks};
+    int status = ERR_UNSUPPORTED_SIZE;
+#define SINGLE_CASE(NK_, PT_)                                                                                     \
+  if (N == 32 * NK_ && P == 16 * PT_)                                                                             \
+    status = launch_ssd_single<NK_, PT_>(dim3(n_chunks, H + tail_rows), stream, (const bf16_t*)xbc, xbc_ld,       \
+                                         (const bf16_t*)TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld,           \
+                                         (const bf16_t*)z, z_ld, (bf16_t*)gated, gated_ld, one);
+    SINGLE_CASE(1, 1) SINGLE_CASE(1, 2) SINGLE_CASE(1, 4) SINGLE_CASE(1, 8)
+    SINGLE_CASE(2, 1) SINGLE_CASE(2, 2) SINGLE_CASE(2, 4) SINGLE_CASE(2, 8)
+    SINGLE_CASE(4, 1) SINGLE_CASE(4, 2) SINGLE_CASE(4, 4) SINGLE_CASE(4, 8)
+    SINGLE_CASE(8, 1) SINGLE_CASE(8, 2) SINGLE_CASE(8, 4) SINGLE_CASE(8, 8)
+#undef SINGLE_CASE
+    if (status != 0) return status;
+    RETURN_IF_LAUNCH_FAILED();
+    return 0;
+  }
+  if (!chunk_state || !chunk_decay || !state_in) return ERR_BAD_ARGUMENT;
   {
     const dim3 grid(n_chunks, H);
 #define STATE_CASE(QK_)                                                                                         \
@@ -791,8 +1121,7 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
                                                     (bf16_t*)conv_state, chunks, Q);
     RETURN_IF_LAUNCH_FAILED();
   }
-  const bool staged = (P == 16 || P == 32 || P == 64 || P == 128) && (N == 32 || N == 64 || N == 128 || N == 256) &&
-                      ssd_scan_lds_bytes(Q, P, N) <= 64 * 1024;
+  const bool staged = ssd_staged_sizes(P, N) && ssd_scan_lds_bytes(Q, P, N) <= 64 * 1024;
   if (staged) {
     const dim3 grid(n_chunks, H, (Q + 127) / 128);
     const size_t lds = ssd_scan_lds_bytes(Q, P, N);

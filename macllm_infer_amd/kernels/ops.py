@@ -165,7 +165,8 @@ _SIGNATURES = {
         "mi_ssd_prefill": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr,
                            _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_long,
-                           _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
+                           _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
+        "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int],
     },
     "gemm": {
         "mi_gemm_f32": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr],
@@ -1834,13 +1835,14 @@ def ssd_supported(chunk_size: int, head_dim: int, state_size: int, num_groups: i
 def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: torch.Tensor, D: torch.Tensor,
                 ssm_state: torch.Tensor, table: SsdChunks, slot_ids: torch.Tensor, num_groups: int,
                 y: Optional[torch.Tensor], z: Optional[torch.Tensor] = None,
-                gated: Optional[torch.Tensor] = None, conv: Optional[dict] = None) -> None:
+                gated: Optional[torch.Tensor] = None, conv: Optional[dict] = None, longest: int = 0) -> None:
     """The selective scan of ``ssm_scan`` (same arguments and results beyond rounding) for bfloat16,
     in chunks on the matrix cores.  ``table`` cuts this step's lanes into chunks.  With ``z`` and
     ``gated`` (bfloat16 [T, E], column views are fine) it writes gated = y * SiLU(z) and no y.
     With ``conv`` = {u, weight, bias, state} the conv runs here too: ``xbc`` is then written (what
     ``conv1d_silu`` would put there from the raw rows ``u`` [T, C]) and the tails ``state`` updated
-    (as ``conv_state_update`` would); see ``ssd_conv_supported``."""
+    (as ``conv_state_update`` would); see ``ssd_conv_supported``.  ``longest``: the longest lane's tokens, or
+    more (0: not known): where every lane is one chunk of up to 128 tokens the scan and its states are one launch."""
     xbc_ld = _row_major(xbc, "xbc")
     dt_ld = _row_major(dt, "dt")
     fused_gate = z is not None
@@ -1874,9 +1876,11 @@ def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: t
     device = xbc.device
     delta = torch.empty((2, T, H), dtype=torch.float32, device=device)
     transposed = torch.empty((chunks * (E + GN) * Q,), dtype=torch.bfloat16, device=device)
-    chunk_state = torch.empty((chunks * H * P * N + chunks * H,), dtype=torch.float32, device=device)
-    state_in = torch.empty((chunks * H * P * N,), dtype=torch.bfloat16, device=device)
-    decay = chunk_state[chunks * H * P * N:]
+    chunk_state = state_in = decay = None
+    if not _fn("ssd", "mi_ssd_single")(Q, P, N, int(longest)):
+        chunk_state = torch.empty((chunks * H * P * N + chunks * H,), dtype=torch.float32, device=device)
+        state_in = torch.empty((chunks * H * P * N,), dtype=torch.bfloat16, device=device)
+        decay = chunk_state[chunks * H * P * N:]
     raw = conv_w = conv_b = conv_state = None
     raw_ld = taps = 0
     if conv is not None:
@@ -1895,7 +1899,7 @@ def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: t
         _p(xbc), xbc_ld, _p(dt), dt_ld, _p(dt_bias), _p(A), _p(D), _p(ssm_state), _p(table.chunks), chunks,
         _p(table.lane_chunks), _p(slot_ids), table.num_lanes, Q, H, P, N, num_groups, _p(delta[0]), _p(delta[1]),
         _p(transposed), _p(chunk_state), _p(decay), _p(state_in), _p(y), y_ld, _p(z), z_ld, _p(gated), gated_ld,
-        _p(raw), raw_ld, _p(conv_w), _p(conv_b), _p(conv_state), int(taps), _stream()),
+        _p(raw), raw_ld, _p(conv_w), _p(conv_b), _p(conv_state), int(taps), int(longest), _stream()),
         "ssd_prefill", f"(Q={Q}, P={P}, N={N})")
 
 

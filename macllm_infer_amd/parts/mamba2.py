@@ -139,10 +139,11 @@ class Mamba2(Mixer):
             arguments = (xbc, u[:, E + C:], self.dt_bias, self.A, self.D, ssm_state, self._chunk_table(step),
                          step.slot_ids, spec.num_groups)
             if self.norm_weight is None and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0:
-                ops.ssd_prefill(*arguments, None, z=u[:, :E], gated=gated, conv=conv)      # the gate on the scan's way out
+                ops.ssd_prefill(*arguments, None, z=u[:, :E], gated=gated, conv=conv,
+                                longest=step.max_query_len)                 # the gate on the scan's way out
                 return
             y = torch.empty((T, E), dtype=torch.float32, device=u.device)
-            ops.ssd_prefill(*arguments, y, conv=conv)
+            ops.ssd_prefill(*arguments, y, conv=conv, longest=step.max_query_len)
         else:
             y = torch.empty((T, E), dtype=torch.float32, device=u.device)
             ops.ssm_scan(xbc, u[:, E + C:], self.dt_bias, self.A, self.D, ssm_state, step.cu_seqlens,

@@ -579,6 +579,37 @@ def test_chunked_scan_with_the_conv_inside(ops, K, Q, bias):
     close(got_xbc, plain_xbc, torch.bfloat16, 4.0)
 
 
+@pytest.mark.parametrize("Q, H, P, N, G, gate", [(32, 4, 16, 32, 2, False), (64, 3, 32, 64, 1, True), (128, 6, 64, 128, 2, True),
+                                                 (128, 2, 128, 256, 1, True), (256, 2, 64, 128, 1, False), (128, 1, 128, 32, 1, False)])
+def test_lanes_of_one_chunk_scan_in_one_launch(ops, Q, H, P, N, G, gate):
+    """Where no lane is longer than a chunk (and 128 tokens) the chunk's state, the pass and the scan are one launch: the
+    numbers of the three, outputs, states and conv tails, for lanes at the edges of the tiles of 16 and of the chunk."""
+    E, GN, K = H * P, G * N, 4
+    C = E + 2 * GN
+    longest = min(Q, 128)
+    counts = [1, 2, 3, 15, 16, 17, longest - 1, longest, 33 if Q > 32 else 31]
+    T = sum(counts)
+    slots = len(counts) + 2
+    ids = i32(torch.randperm(slots, generator=torch.Generator().manual_seed(Q)).tolist()[:len(counts)]).to(DEV)
+    wide = rand(T, E + C + H + (-(E + C + H)) % 8, seed=190, dtype=torch.bfloat16).to(DEV)
+    z, raw, dt = wide[:, :E], wide[:, E:E + C], wide[:, E + C:E + C + H]
+    weight, bias = gpu(rand(C, K, seed=191, scale=0.5), rand(C, seed=192))
+    dt_bias, A, D = gpu(rand(H, seed=194) - 1.0, -torch.exp(torch.linspace(-3.0, 1.0, H)), rand(H, seed=195))
+    tails, state = rand(slots, K - 1, C, seed=193, dtype=torch.bfloat16).to(DEV), rand(slots, H, P, N, seed=196, scale=0.5).to(DEV)
+    results = []
+    for known in (0, longest):
+        now_tails, now_state = tails.clone(), state.clone()
+        xbc = torch.full((T, C), float("nan"), dtype=torch.bfloat16, device=DEV)
+        y = None if gate else torch.full((T, E), float("nan"), device=DEV)
+        gated = torch.full((T, E), float("nan"), dtype=torch.bfloat16, device=DEV) if gate else None
+        ops.ssd_prefill(xbc, dt, dt_bias, A, D, now_state, ops.SsdChunks(counts, Q, DEV), ids, G, y, z=z if gate else None,
+                        gated=gated, conv=dict(u=raw, weight=weight, bias=bias, state=now_tails), longest=known)
+        results.append((gated if gate else y, now_state, now_tails))
+    for one, three in zip(results[1], results[0]):
+        assert torch.equal(one, three) and bool(torch.isfinite(one).all())
+    assert not torch.equal(results[1][1], state) and not torch.equal(results[1][2], tails)
+
+
 def test_chunked_scan_carries_a_far_token_through_many_chunks(ops):
     """One token with a large x and a head that barely decays: 600 tokens later its state is what
     the output consists of; every chunk boundary between must pass it on."""
