@@ -397,231 +397,164 @@ moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* _
     }
 }
 
-// Where piece `piece` (0..3) of row `row` of an LDS stage lies: a row is 64 bytes, and the pieces of rows 4 apart
-// are swapped among themselves so that the sixteen rows a quarter of a wave reads at once fall into sixteen
-// different groups of banks.
-__device__ __forceinline__ int stage_slot(int row, int piece) { return row * 4 + (piece ^ ((row >> 2) & 3)); }
+// Four neighbouring results of one place: in one store where the rows of the output are whole groups of four.
+template <typename TO>
+__device__ __forceinline__ void store_four(TO* row, long n, int width, bool whole, const float (&value)[4]) {
+  typedef TO four_t __attribute__((ext_vector_type(4)));
+  if (whole && n + 3 < width) {
+    four_t packed;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) packed[i] = from_float<TO>(value[i]);
+    *reinterpret_cast<four_t*>(row + n) = packed;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (n + i < width) row[n + i] = from_float<TO>(value[i]);
+}
 
 // The same product for prompt portions whose rows and matrices are whole 16-byte pieces: a workgroup owns a tile
-// of 64 places and 128 rows of its expert's matrix (GLU: 64 gate rows and the 64 up rows that go with them, which
-// make 64 outputs; else 128 outputs), walks K one chunk at a time through two LDS stages (the next chunk's pieces
-// are asked for before the current one's products), and every wave owns all 64 places and a quarter of the
-// features: no sum crosses a wave, a row's result is summed in k order by one lane's accumulator.
-template <typename T, typename TO, bool GLU>
-__global__ void __launch_bounds__(TILE_THREADS)
+// of ROWS places (128 where experts get hundreds of rows each, else 64) and 128 rows of its expert's matrix (GLU: 64
+// gate rows and the 64 up rows that go with them, which make 64 outputs; else 128 outputs), every one of its four waves
+// half the places and half the features (GLU: 32 gate rows and their 32 up rows): no sum crosses a wave, a row's result
+// is summed in k order by one lane's accumulator.  K is walked in stages of eight pieces a row, whole lines of 128 bytes
+// (64 columns of bfloat16, 32 of float32), through two LDS stages; the next stage's pieces are asked for before the
+// current one's products.  Piece p of row r of a stage lies at r * 8 + (p ^ (r & 7)): the eight rows that a quarter of a
+// wave reads at once fall into different groups of banks, and a thread's stores are one run.
+// What bounds it: the bytes in flight of a compute unit (a stage a workgroup, 24 or 32 KB).  Three of sixteen experts of
+// 512 x 1,024 in bfloat16, us for the two products of 1,554 / 700 tokens: stages of 64 bytes a row 75 / 50 with
+// tiles of 128 / 64 places; now 51 / 41 with 128 and 45 / 35 with 64.  (Bounds of two workgroups a compute unit keep the
+// sums out of the accumulator registers, whose moves cost 20 us; two or three stages on their way: 55 and 62 with 128.)
+template <typename T, typename TO, bool GLU, int ROWS>
+__global__ void __launch_bounds__(TILE_THREADS, 2)
 moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* __restrict__ W, long expert_stride,
                             long ldw, int N, int K, const int* __restrict__ source, const int* __restrict__ tile_expert,
                             int gather, float limit, float alpha, float offset, int squared_relu,
-                            const float* __restrict__ row_scale, TO* __restrict__ out, long ldo) {
+                            const float* __restrict__ row_scale, TO* __restrict__ out, long ldo, int whole) {
   typedef typename TileTraits<T>::Piece Piece;
-  constexpr int CHUNK = TileTraits<T>::CHUNK;
   constexpr int PIECE = TileTraits<T>::PIECE;
-  constexpr int ROWS = 64, FEATURES = 128;
-  __shared__ Piece stage[2][(ROWS + FEATURES) * 4];
+  constexpr int STAGE_K = 8 * PIECE;
+  constexpr int FEATURES = 128;
+  constexpr int MT = ROWS / 32;                                // tiles of 16 places a wave
+  constexpr int X_PIECES = ROWS * 8 / TILE_THREADS, W_PIECES = FEATURES * 8 / TILE_THREADS;
+  __shared__ Piece stage[2][(ROWS + FEATURES) * 8];
   const int tile = blockIdx.y;
   const int expert = tile_expert[tile];
   if (expert < 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
   const int wave = tid / WAVE;
-  const int q = lane / 16;
-  const int r = lane % 16;
-  const int width = GLU ? N / 2 : N;
-  const long n0 = (long)blockIdx.x * (GLU ? 64 : 128);
-  const T* matrix = W + (long)expert * expert_stride;
-  // what this thread brings into a stage: piece `part` of one row of x and of two rows of the matrix
-  const int lrow = tid / 4;
-  const int part = tid % 4;
-  const int place_in = tile * ROWS + lrow;
-  const long x_at = gather ? max(source[place_in], 0) : place_in;
-  const T* x_from = x + min(x_at, (long)x_rows - 1) * ldx;
-  const T* w_from[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int s = lrow + 64 * j;                                // row of the stage's matrix part
-    long feature;
-    if (GLU) feature = (j == 0 ? 0 : width) + min(n0 + lrow, (long)width - 1);
-    else feature = min(n0 + s, (long)width - 1);
-    w_from[j] = matrix + feature * ldw;
-  }
-  tile_floatx4 acc[2][4];
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
-  const int chunks = (K + CHUNK - 1) / CHUNK;
-  Piece gx = tile_load<T, true>(x_from, PIECE * part, K);
-  Piece gw0 = tile_load<T, true>(w_from[0], PIECE * part, K);
-  Piece gw1 = tile_load<T, true>(w_from[1], PIECE * part, K);
-  stage[0][stage_slot(lrow, part)] = gx;
-  stage[0][stage_slot(ROWS + lrow, part)] = gw0;
-  stage[0][stage_slot(ROWS + 64 + lrow, part)] = gw1;
-  __syncthreads();
-  for (int c = 0; c < chunks; ++c) {
-    const int cur = c & 1;
-    const int k_next = c + 1 < chunks ? (c + 1) * CHUNK + PIECE * part : K;      // past the end: zeros, never used
-    gx = tile_load<T, true>(x_from, k_next, K);
-    gw0 = tile_load<T, true>(w_from[0], k_next, K);
-    gw1 = tile_load<T, true>(w_from[1], k_next, K);
-    Piece a[2], b[4];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const int row = GLU ? 64 * nt + 16 * wave + r : 32 * wave + 16 * nt + r;
-      a[nt] = stage[cur][stage_slot(ROWS + row, q)];
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) b[mt] = stage[cur][stage_slot(16 * mt + r, q)];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = tile_mfma(a[nt], b[mt], acc[nt][mt]);
-    stage[cur ^ 1][stage_slot(lrow, part)] = gx;
-    stage[cur ^ 1][stage_slot(ROWS + lrow, part)] = gw0;
-    stage[cur ^ 1][stage_slot(ROWS + 64 + lrow, part)] = gw1;
-    __syncthreads();
-  }
-#pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int place = tile * ROWS + 16 * mt + r;
-    const bool live = source[place] >= 0;
-    const float scale = row_scale ? row_scale[place] : 1.0f;
-    TO* row = out + (long)place * ldo;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (GLU) {
-        const long n = n0 + 16 * wave + 4 * q + i;
-        const float g = fminf(acc[0][mt][i] * scale, limit);
-        const float u = fminf(fmaxf(acc[1][mt][i] * scale, -limit), limit);
-        const float value = g / (1.0f + expf(-alpha * g)) * (u + offset);
-        if (n < width) row[n] = from_float<TO>(live ? value : 0.f);
-      } else {
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-          const long n = n0 + 32 * wave + 16 * nt + 4 * q + i;
-          float value = acc[nt][mt][i] * scale;
-          if (squared_relu) {
-            value = fmaxf(value, 0.f);
-            value *= value;
-          }
-          if (n < width) row[n] = from_float<TO>(live ? value : 0.f);
-        }
-      }
-    }
-  }
-}
-
-// The widest form, for prompt portions whose experts get hundreds of rows each: 128 places x 128 matrix rows a
-// workgroup, every wave a quarter of it as 64 places x 64 matrix rows (GLU: 32 gate rows and their 32 up rows), so
-// that eight fragments from LDS feed sixteen matrix instructions.
-template <typename T, typename TO, bool GLU>
-__global__ void __launch_bounds__(TILE_THREADS)
-moe_expert_gemm_widest_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* __restrict__ W, long expert_stride,
-                              long ldw, int N, int K, const int* __restrict__ source, const int* __restrict__ tile_expert,
-                              int gather, float limit, float alpha, float offset, int squared_relu,
-                              const float* __restrict__ row_scale, TO* __restrict__ out, long ldo) {
-  typedef typename TileTraits<T>::Piece Piece;
-  constexpr int CHUNK = TileTraits<T>::CHUNK;
-  constexpr int PIECE = TileTraits<T>::PIECE;
-  constexpr int ROWS = 128, FEATURES = 128;
-  __shared__ Piece stage[2][(ROWS + FEATURES) * 4];
-  const int tile = blockIdx.y;
-  const int expert = tile_expert[tile];
-  if (expert < 0) return;
-  const int tid = threadIdx.x;
-  const int lane = tid & (WAVE - 1);
-  const int wave = tid / WAVE;
-  const int wm = wave / 2;                                     // which 64 places
+  const int wm = wave / 2;                                     // which half of the places
   const int wn = wave % 2;                                     // which half of the features
   const int q = lane / 16;
   const int r = lane % 16;
   const int width = GLU ? N / 2 : N;
   const long n0 = (long)blockIdx.x * (GLU ? 64 : 128);
   const T* matrix = W + (long)expert * expert_stride;
-  const int lrow = tid / 4;
-  const int part = tid % 4;
-  const T* x_from[2];
-  const T* w_from[2];
+  // what this thread brings into a stage: one piece each of X_PIECES rows of x and W_PIECES of the matrix, 32 rows apart
+  const int lrow = tid / 8;
+  const int column = PIECE * ((tid % 8) ^ (lrow & 7));
+  const T* x_from[X_PIECES];
+  const T* w_from[W_PIECES];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int place_in = tile * ROWS + lrow + 64 * j;
+  for (int j = 0; j < X_PIECES; ++j) {
+    const int place_in = tile * ROWS + lrow + 32 * j;
     const long x_at = gather ? max(source[place_in], 0) : place_in;
     x_from[j] = x + min(x_at, (long)x_rows - 1) * ldx;
-    long feature;
-    if (GLU) feature = (j == 0 ? 0 : width) + min(n0 + lrow, (long)width - 1);
-    else feature = min(n0 + lrow + 64 * j, (long)width - 1);
+  }
+#pragma unroll
+  for (int j = 0; j < W_PIECES; ++j) {
+    const int row = lrow + 32 * j;                             // of the stage's matrix part
+    const long feature = GLU ? (row < 64 ? 0 : width) + min(n0 + row % 64, (long)width - 1) : min(n0 + row, (long)width - 1);
     w_from[j] = matrix + feature * ldw;
   }
-  tile_floatx4 acc[4][4];
+  tile_floatx4 acc[4][MT];
 #pragma unroll
   for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
-  const int chunks = (K + CHUNK - 1) / CHUNK;
-  Piece gx[2], gw[2];
+    for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
+  const int stages = (K + STAGE_K - 1) / STAGE_K;
+  Piece gx[X_PIECES], gw[W_PIECES];
+  auto ask = [&](int stage_number) {                           // (a piece past the end: the row's last one, laid as zeros)
+    const int k = min(stage_number * STAGE_K + column, K - PIECE);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    gx[j] = tile_load<T, true>(x_from[j], PIECE * part, K);
-    gw[j] = tile_load<T, true>(w_from[j], PIECE * part, K);
-    stage[0][stage_slot(lrow + 64 * j, part)] = gx[j];
-    stage[0][stage_slot(ROWS + lrow + 64 * j, part)] = gw[j];
-  }
+    for (int j = 0; j < X_PIECES; ++j) gx[j] = *reinterpret_cast<const Piece*>(x_from[j] + k);
+#pragma unroll
+    for (int j = 0; j < W_PIECES; ++j) gw[j] = *reinterpret_cast<const Piece*>(w_from[j] + k);
+  };
+  auto lay = [&](int stage_number) {
+    const bool there = stage_number * STAGE_K + column < K;
+    Piece* const into = stage[stage_number & 1];
+    const Piece none = {};
+#pragma unroll
+    for (int j = 0; j < X_PIECES; ++j) into[tid + TILE_THREADS * j] = there ? gx[j] : none;
+#pragma unroll
+    for (int j = 0; j < W_PIECES; ++j) into[ROWS * 8 + tid + TILE_THREADS * j] = there ? gw[j] : none;
+  };
+  auto multiply = [&](const Piece* staged) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      Piece a[4], b[MT];
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt) {
+        // GLU: nt 0, 1 are gate rows, nt 2, 3 the up rows of the same outputs (the stage's second 64 rows)
+        const int row = GLU ? 64 * (nt / 2) + 32 * wn + 16 * (nt % 2) + r : 64 * wn + 16 * nt + r;
+        a[nt] = staged[(ROWS + row) * 8 + ((4 * c + q) ^ (row & 7))];
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const int row = 16 * MT * wm + 16 * mt + r;
+        b[mt] = staged[row * 8 + ((4 * c + q) ^ (row & 7))];
+      }
+#pragma unroll
+      for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = tile_mfma(a[nt], b[mt], acc[nt][mt]);
+    }
+  };
+  ask(0);
+  lay(0);
   __syncthreads();
-  for (int c = 0; c < chunks; ++c) {
-    const int cur = c & 1;
-    const int k_next = c + 1 < chunks ? (c + 1) * CHUNK + PIECE * part : K;      // past the end: zeros, never used
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      gx[j] = tile_load<T, true>(x_from[j], k_next, K);
-      gw[j] = tile_load<T, true>(w_from[j], k_next, K);
-    }
-    Piece a[4], b[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      // GLU: nt 0, 1 are gate rows, nt 2, 3 the up rows of the same outputs (the stage's second 64 rows)
-      const int row = GLU ? 64 * (nt / 2) + 32 * wn + 16 * (nt % 2) + r : 64 * wn + 16 * nt + r;
-      a[nt] = stage[cur][stage_slot(ROWS + row, q)];
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) b[mt] = stage[cur][stage_slot(64 * wm + 16 * mt + r, q)];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) acc[nt][mt] = tile_mfma(a[nt], b[mt], acc[nt][mt]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      stage[cur ^ 1][stage_slot(lrow + 64 * j, part)] = gx[j];
-      stage[cur ^ 1][stage_slot(ROWS + lrow + 64 * j, part)] = gw[j];
-    }
+  for (int s = 0; s < stages; ++s) {
+    ask(s + 1);
+    __builtin_amdgcn_sched_barrier(0);                         // (left to itself the scheduler moves the loads behind the products)
+    multiply(stage[s & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    lay(s + 1);
     __syncthreads();
   }
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int place = tile * ROWS + 64 * wm + 16 * mt + r;
+  for (int mt = 0; mt < MT; ++mt) {
+    const int place = tile * ROWS + 16 * MT * wm + 16 * mt + r;
     const bool live = source[place] >= 0;
     const float scale = row_scale ? row_scale[place] : 1.0f;
     TO* row = out + (long)place * ldo;
+    if (GLU) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (GLU) {
+      for (int h = 0; h < 2; ++h) {
+        float value[4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const long n = n0 + 32 * wn + 16 * h + 4 * q + i;
+        for (int i = 0; i < 4; ++i) {
           const float g = fminf(acc[h][mt][i] * scale, limit);
           const float u = fminf(fmaxf(acc[2 + h][mt][i] * scale, -limit), limit);
-          const float value = g / (1.0f + expf(-alpha * g)) * (u + offset);
-          if (n < width) row[n] = from_float<TO>(live ? value : 0.f);
+          value[i] = live ? g / (1.0f + expf(-alpha * g)) * (u + offset) : 0.f;
         }
-      } else {
+        store_four<TO>(row, n0 + 32 * wn + 16 * h + 4 * q, width, whole != 0, value);
+      }
+    } else {
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-          const long n = n0 + 64 * wn + 16 * nt + 4 * q + i;
-          float value = acc[nt][mt][i] * scale;
+      for (int nt = 0; nt < 4; ++nt) {
+        float value[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          value[i] = acc[nt][mt][i] * scale;
           if (squared_relu) {
-            value = fmaxf(value, 0.f);
-            value *= value;
+            value[i] = fmaxf(value[i], 0.f);
+            value[i] *= value[i];
           }
-          if (n < width) row[n] = from_float<TO>(live ? value : 0.f);
+          if (!live) value[i] = 0.f;
         }
+        store_four<TO>(row, n0 + 64 * wn + 16 * nt + 4 * q, width, whole != 0, value);
       }
     }
   }
@@ -640,22 +573,18 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
   const int width = glu ? N / 2 : N;
 #define EXPERT_LAUNCH(VEC_, GLU_, MT_, PAIRS_)                                                                           moe_expert_gemm_kernel<T, TO, VEC_, GLU_, MT_, PAIRS_>                                                                    <<<dim3((unsigned)((width + 16 * PAIRS_ - 1) / (16 * PAIRS_)), (unsigned)tiles), TILE_THREADS, 0, stream>>>(               x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo)
 #define EXPERT_SHAPE(MT_, PAIRS_GLU_, PAIRS_PLAIN_)                                                                      do {                                                                                                                    if (vec && glu) EXPERT_LAUNCH(true, true, MT_, PAIRS_GLU_);                                                            else if (vec) EXPERT_LAUNCH(true, false, MT_, PAIRS_PLAIN_);                                                           else if (glu) EXPERT_LAUNCH(false, true, MT_, PAIRS_GLU_);                                                             else EXPERT_LAUNCH(false, false, MT_, PAIRS_PLAIN_);                                                                 } while (0)
-  if (pad == 128) {      // (only plans of rows and matrices in whole pieces are made so wide)
+  if ((pad == 128 || pad == 64) && vec) {      // (plans of 128 places are made of rows and matrices in whole pieces only)
     const dim3 grid((unsigned)((width + (glu ? 64 : 128) - 1) / (glu ? 64 : 128)), (unsigned)tiles);
-    if (glu)
-      moe_expert_gemm_widest_kernel<T, TO, true><<<grid, TILE_THREADS, 0, stream>>>(
-          x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo);
-    else
-      moe_expert_gemm_widest_kernel<T, TO, false><<<grid, TILE_THREADS, 0, stream>>>(
-          x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo);
-  } else if (pad == 64 && vec) {
-    const dim3 grid((unsigned)((width + (glu ? 64 : 128) - 1) / (glu ? 64 : 128)), (unsigned)tiles);
-    if (glu)
-      moe_expert_gemm_wide_kernel<T, TO, true><<<grid, TILE_THREADS, 0, stream>>>(
-          x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo);
-    else
-      moe_expert_gemm_wide_kernel<T, TO, false><<<grid, TILE_THREADS, 0, stream>>>(
-          x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo);
+    const int whole = ldo % 4 == 0 && ((unsigned long long)out % 16) == 0;
+#define EXPERT_WIDE(GLU_, ROWS_)                                                                                  \
+  moe_expert_gemm_wide_kernel<T, TO, GLU_, ROWS_><<<grid, TILE_THREADS, 0, stream>>>(                             \
+      x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, \
+      row_scale, out, ldo, whole)
+    if (pad == 128 && glu) EXPERT_WIDE(true, 128);
+    else if (pad == 128) EXPERT_WIDE(false, 128);
+    else if (glu) EXPERT_WIDE(true, 64);
+    else EXPERT_WIDE(false, 64);
+#undef EXPERT_WIDE
   } else if (pad == 64) {
     EXPERT_SHAPE(4, 2, 4);
   } else {

@@ -179,7 +179,9 @@ def test_the_router_and_the_grouping_of_rows_by_expert(T, experts, top):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T, experts, top, hidden, inner, pad", [
     (1, 4, 2, 32, 16, None), (45, 6, 3, 64, 40, None), (130, 9, 2, 48, 24, None), (7, 3, 1, 20, 12, None),
-    (400, 5, 2, 72, 88, None), (300, 3, 2, 36, 20, None), (700, 3, 2, 64, 40, 128), (530, 2, 2, 136, 264, 128)])
+    (400, 5, 2, 72, 88, None), (300, 3, 2, 36, 20, None), (700, 3, 2, 64, 40, 128), (530, 2, 2, 136, 264, 128),
+    # the wide tiles where their stages of K and their rows of outputs end early
+    (45, 6, 3, 8, 56, 64), (90, 3, 2, 72, 66, 64), (130, 3, 2, 128, 200, 64), (257, 2, 1, 200, 128, 128)])
 def test_the_grouped_products_and_the_weighted_sum(dtype, T, experts, top, hidden, inner, pad):
     from macllm_infer_amd.config import ClampedGLUSpec
     glu = ClampedGLUSpec(limit=0.9)
