@@ -143,6 +143,11 @@ _SIGNATURES = {
                                       _c_ptr, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr,
                                       _c_long, _c_ptr],
     },
+    "attention_shared": {
+        "mi_prefill_attention_shared": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_long, _c_int,
+                                        _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int, _c_int,
+                                        _c_ptr, _c_long, _c_ptr],
+    },
     "attention_widths": {
         "mi_prefill_attention_padded": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_long, _c_int,
                                         _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int, _c_int, _c_ptr,
@@ -1546,6 +1551,38 @@ def prefill_attention_supported(dtype, num_heads: int, num_kv_heads: int, head_d
     return value_dim is not None and head_dim % 8 == 0 and head_dim <= 128 and value_dim % 4 == 0 and value_dim <= 128
 
 
+SHARED_PREFILL_KEYS = (576, 2048)         # of the longest walk, heads of 64: of any grid, of one that fills half the chip
+SHARED_PREFILL_WORKGROUPS = 128           # half of the chip's compute units
+COMPUTE_UNITS = 256
+
+
+def shared_prefill_heads(tiles: int, num_heads: int, num_kv_heads: int, head_dim: int, max_seq_len: int,
+                         span: int) -> int:
+    """How many query heads a workgroup of the prompt attention with shared keys takes, 0: the kernel whose waves
+    read their keys themselves is the faster one.
+
+    The other kernel splits a tile's keys eight ways instead of two and, of heads of 64, shares a key fragment among up
+    to four heads: it is the faster one where a few heavy tiles bound the launch.  Heads of 64 (us, other | this one): 8
+    over 2 kv heads, 300 tokens 13.9 | 9.9, 515 14.2 | 13.8, 2,048 34.9 | 28.2, 2,048 behind 2,048 45.6 | 50.9, 4,096
+    58.4 | 71.9; 6 over 2, 600 tokens 13.6 | 14.6; 16 over 16, 600 tokens 17.4 | 15.1, 2,048 behind 4,096 252 | 111 and
+    256 behind 4,096 28.9 | 52.9.  Heads of 128: 12 over 2, 515 tokens 18.1 | 20.5, 1,024 37.1 | 23.6, 256 behind 4,096
+    57.7 | 78.3, 1,024 behind 4,096 128 | 93.
+    Heads of 64 go one to a workgroup: two workgroups then share a compute unit.  Of heads of 128 a unit holds one
+    workgroup either way: one head while there is a unit for each, else two, which read K and V half as often (2,048
+    tokens behind 2,048: 132 us with one head, 114 with two; 1,024 tokens 23.6 and 33.6)."""
+    heads_per_kv = num_heads // num_kv_heads
+    workgroups = tiles * num_heads
+    if head_dim == 64:
+        longest = min(max_seq_len, abs(span) + 64) if span else max_seq_len
+        short, long = SHARED_PREFILL_KEYS
+        fits = (0 < longest <= short or (0 < longest <= long and workgroups >= SHARED_PREFILL_WORKGROUPS)
+                or (heads_per_kv == 1 and workgroups >= COMPUTE_UNITS))
+        return 1 if fits else 0
+    if workgroups < SHARED_PREFILL_WORKGROUPS:
+        return 0
+    return 1 if heads_per_kv == 1 or workgroups <= COMPUTE_UNITS else 2
+
+
 def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, k_cache: torch.Tensor,
                       v_cache: torch.Tensor, block_tables: torch.Tensor, query_tiles: torch.Tensor,
                       cu_seqlens: torch.Tensor, start_pos: torch.Tensor, scale: float, window: Optional[int],
@@ -1590,6 +1627,17 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     gate_ld = _gate_rows(gate, out, "prefill_attention")
     _need(gate is None or (gate_ld % 4 == 0 and gate.data_ptr() % 8 == 0), "prefill_attention: the gate's rows lie in pieces of four")
     own_width = head_dim in (64, 128) and value_dim == head_dim
+    if (own_width and log_bias is None and sinks is None and slopes is None and gate is None and keep_first == 0
+            and page_size >= 8 and page_size & (page_size - 1) == 0 and page_stride % 8 == 0
+            and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and out_ld % 4 == 0):
+        heads = shared_prefill_heads(query_tiles.shape[0], num_heads, num_kv_heads, head_dim, int(max_seq_len or 0),
+                                     span_code)
+        if heads:
+            _check(_fn("attention_shared", "mi_prefill_attention_shared")(
+                _p(q), q_ld, num_heads, num_kv_heads, head_dim, _p(k_cache), _p(v_cache), page_stride, page_size,
+                _p(block_tables), block_tables.shape[1], _p(query_tiles), query_tiles.shape[0], _p(cu_seqlens),
+                _p(start_pos), float(scale), span_code, heads, _p(out), out_ld, _stream()), "prefill_attention")
+            return
     _need(own_width or log_bias is None, "prefill_attention: the logarithmic bias comes with heads of 64 or 128 and values as wide")
     _check(_fn(*(("attention", "mi_prefill_attention") if own_width else ("attention_widths", "mi_prefill_attention_padded")))(
         _p(q), q_ld, num_heads, num_kv_heads, head_dim, *(() if own_width else (value_dim,)), _p(k_cache), _p(v_cache),

@@ -40,7 +40,7 @@ class Attention(Mixer):
     ``key_multiplier`` the k projection's output (weights and bias), ``out_multiplier``
     the output projection's output."""
     graph_safe = True
-    kernel_modules = ("common", "attention", "attention_widths", "gemm", "mamba2")
+    kernel_modules = ("common", "attention", "attention_shared", "attention_widths", "gemm", "mamba2")
     query_tile = 64          # tokens of one lane that a workgroup of the prompt attention kernels takes
 
     @classmethod
@@ -49,6 +49,8 @@ class Attention(Mixer):
         unused = {"mamba2"} if spec.conv_kernel == 0 else set()                  # the convolutions' kernels
         if own_width or spec.head_dim % 8 or spec.head_dim > 128:                # the prompt kernel at padded widths
             unused.add("attention_widths")
+        if not own_width:                                                        # and the one at these two
+            unused.add("attention_shared")
         return tuple(name for name in cls.kernel_modules if name not in unused)
 
     @classmethod

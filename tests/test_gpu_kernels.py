@@ -1551,6 +1551,55 @@ def test_prefill_attention_many_short_portions(ops, Hq, Hkv, dh):
     close(got, want, dtype, 2.0)
 
 
+@pytest.mark.parametrize("Hq, Hkv, dh, page_size, window", [(8, 2, 64, 16, None), (3, 1, 64, 8, None), (2, 2, 64, 128, 70),
+                                                              (12, 2, 128, 16, None), (4, 4, 128, 64, 33), (5, 1, 128, 8, 1)])
+@pytest.mark.parametrize("copies", [1, 12])
+def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_size, window, copies):
+    """The kernel whose waves share their keys, held against the one whose waves read them alone: portions that end
+    at and beside the edges of a wave's 16 tokens, a tile of 64 and a stage of 64 keys, behind prefixes that do the same;
+    few workgroups and many, with one query head and with two.  Unwritten cells hold NaN, as do the cells of passed
+    pages.  Both round their weights to bfloat16 and sum in float32: they may differ by the rounding of an output."""
+    dtype = torch.bfloat16
+    starts = [0, 37, 0, 64, 127, 500, 0, 129, 9000 if copies == 1 and page_size == 8 else 700] * copies
+    counts = [64, 83, 150, 64, 65, 2, 1, 1, 15] * copies
+    lengths = [s + c for s, c in zip(starts, counts)]
+    pool, table = paged_setup(lengths, page_size, Hkv, dh, dtype, seed=23)
+    for lane, length in enumerate(lengths):
+        fill_cache(pool, table, lane, rand(length, Hkv, dh, seed=1200 + lane, dtype=dtype),
+                   rand(length, Hkv, dh, seed=1400 + lane, dtype=dtype), page_size)
+    T = sum(counts)
+    q = rand(T, Hq * dh + 8, seed=612, dtype=dtype).to(DEV)
+    cu = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    cu[1:] = torch.cumsum(torch.tensor(counts), 0)
+    tiles = i32([(lane, row) for lane in range(len(counts)) for row in range(int(cu[lane]), int(cu[lane + 1]), 64)]
+                + [(-1, 0)])
+    assert ops.shared_prefill_heads(tiles.shape[0], Hq, Hkv, dh, 2000, window or 0) in (0, 1, 2)
+    got = {}
+    device_pool, live = pool.to(DEV), table.clone()
+    for lane, start in enumerate(starts if window else []):      # pages that every query has passed were given back
+        live[lane, :max(0, start - window + 1) // page_size] = -1
+    for heads in (0, 1) if dh == 64 else (0, 1, 2):
+        monkeypatch.setattr(ops, "shared_prefill_heads", lambda *args: heads)
+        got[heads] = torch.full((T, Hq * dh), float("nan"), dtype=dtype, device=DEV)
+        ops.prefill_attention(q, Hq, Hkv, dh, *views(device_pool, page_size), (live if heads else table).to(DEV),
+                              tiles.to(DEV), cu.to(DEV), i32(starts).to(DEV), 0.21, window, got[heads], max(lengths))
+    for heads in list(got)[1:]:
+        assert torch.isfinite(got[heads].float()).all()
+        close(got[heads], got[0].cpu(), dtype, 2.0)
+
+
+def test_rule_of_the_prompt_attention(ops):
+    """Heads of 64: short walks, longer ones on half the chip, any where every head has its own keys and the chip is
+    full.  Heads of 128: grids of half the chip on, two heads a workgroup once every compute unit has one."""
+    rule = ops.shared_prefill_heads
+    assert rule(1, 8, 2, 64, 576, 0) == 1 and rule(9, 8, 2, 64, 577, 0) == 0 and rule(1, 8, 2, 64, 0, 0) == 0
+    assert rule(16, 8, 2, 64, 2048, 0) == 1 and rule(15, 8, 2, 64, 2048, 0) == 0 and rule(64, 8, 2, 64, 2049, 0) == 0
+    assert rule(15, 8, 2, 64, 9000, 512) == 1 and rule(15, 8, 2, 64, 9000, -513) == 0
+    assert rule(16, 16, 16, 64, 9000, 0) == 1 and rule(15, 16, 16, 64, 9000, 0) == 0
+    assert rule(10, 12, 2, 128, 9000, 0) == 0 and rule(11, 12, 2, 128, 9000, 0) == 1 and rule(22, 12, 2, 128, 9000, 0) == 2
+    assert rule(300, 8, 8, 128, 0, 0) == 1
+
+
 def test_prefill_attention_finds_far_keys_and_edges(ops):
     """Queries at the end of a 700-token prompt; one chosen key takes all the weight."""
     Hq, Hkv, dh, length, page_size = 4, 2, 64, 700, 16
