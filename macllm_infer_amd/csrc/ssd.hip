@@ -7,7 +7,8 @@
 //     y_t   = exp(L_t) (S_in . C_t) + sum_{s<=t} exp(L_t - L_s) delta_s (C_t . B_s) x_s + D_h x_t
 //     S_out = exp(L_end) S_in + sum_s exp(L_end - L_s) delta_s x_s (outer) B_s
 // Every exponent is a difference of a non-increasing sequence taken forwards, so it is <= 0 and
-// nothing overflows.  The result does not depend on Q beyond rounding.  Five kernels:
+// nothing overflows.  The result does not depend on Q beyond rounding.  Five kernels (the last three are one launch
+// where every lane is one chunk, see ssd_single_kernel):
 //     prepare     delta, L                                    (one workgroup per chunk and head)
 //     transpose   x and B of each chunk, token-contiguous and zero-padded to Q: [chunk, E + G*N, Q]
 //     chunk_state sum_s exp(L_end - L_s) delta_s x_s (outer) B_s  per chunk and head (matrix cores)
@@ -312,11 +313,49 @@ ssd_chunk_state_kernel(const bf16_t* __restrict__ TT, int E, int GN, const float
 // Per lane, serially over its chunks: state_in[chunk] = running (rounded to bfloat16: it is a
 // matrix-core operand); running = decay[chunk] * running + chunk_state[chunk].  The running state
 // starts from the request's slot and goes back to it, in float32.
+// V neighbouring elements a thread.  Bound by memory: 10 bytes for every element of a chunk's state; four elements a
+// thread ask for 16 bytes a load and write 8 (one element a thread: 4 and 2), in workgroups of one wave so that small
+// states still reach every compute unit.  A lane's chunks come in rounds of AT_ONCE whose loads are all asked for
+// before the recurrence; lanes of up to four chunks take the short round, which asks for nothing twice over.  Measured
+// (one element a thread -> now, beside the prompt attention): 16 chunks of 24 heads of 64 x 128 12.4 -> 8.4 us, of 128 x
+// 256 55 -> 25; 25 lanes of one to five chunks 67 -> 25.
+template <int V, int AT_ONCE>
+__device__ __forceinline__ void ssd_pass_rounds(const float* __restrict__ chunk_state, const float* __restrict__ chunk_decay,
+                                                bf16_t* __restrict__ state_in, int first, int count, int H, int head,
+                                                long per_head, long element, float (&running)[V]) {
+  typedef float floats __attribute__((ext_vector_type(V)));
+  typedef __bf16 halves __attribute__((ext_vector_type(V)));
+  for (int c0 = first; c0 < first + count; c0 += AT_ONCE) {
+    floats added[AT_ONCE];
+    float decay[AT_ONCE];
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) {
+      const int c = min(c0 + j, first + count - 1);
+      added[j] = *reinterpret_cast<const floats*>(chunk_state + ((long)c * H + head) * per_head + element);
+      decay[j] = chunk_decay[(long)c * H + head];
+    }
+#pragma unroll
+    for (int j = 0; j < AT_ONCE; ++j) {
+      if (c0 + j < first + count) {
+        halves entering;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+          entering[i] = (bf16_t)running[i];
+          running[i] = decay[j] * running[i] + added[j][i];
+        }
+        *reinterpret_cast<halves*>(state_in + ((long)(c0 + j) * H + head) * per_head + element) = entering;
+      }
+    }
+  }
+}
+
+template <int V>
 __global__ void ssd_state_pass_kernel(const float* __restrict__ chunk_state, const float* __restrict__ chunk_decay,
                                       const int* __restrict__ lane_chunks, const int* __restrict__ slot_ids, int H,
                                       long per_head, float* __restrict__ ssm_state, bf16_t* __restrict__ state_in,
                                       const bf16_t* __restrict__ u, long u_ld, int C, int K,
                                       bf16_t* __restrict__ conv_state, const int* __restrict__ chunks, int Q) {
+  typedef float floats __attribute__((ext_vector_type(V)));
   const int lane = blockIdx.z;
   if ((int)blockIdx.y >= H) {                // rows past the heads (when the conv ran here): the lane's conv tail
     if (blockIdx.x == 0)
@@ -325,30 +364,22 @@ __global__ void ssd_state_pass_kernel(const float* __restrict__ chunk_state, con
     return;
   }
   const int head = blockIdx.y;
-  const long element = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long element = V * ((long)blockIdx.x * blockDim.x + threadIdx.x);
   if (element >= per_head) return;
   const int first = lane_chunks[2 * lane];
   const int count = lane_chunks[2 * lane + 1];
   float* slot = ssm_state + ((long)slot_ids[lane] * H + head) * per_head + element;
-  float running = *slot;
-  constexpr int AT_ONCE = 16;                               // chunks whose loads are asked for at once, then the recurrence
-  for (int c0 = first; c0 < first + count; c0 += AT_ONCE) { // (a portion of 2,048 tokens in chunks of 128: one round)
-    float added[AT_ONCE], decay[AT_ONCE];
+  floats state = *reinterpret_cast<const floats*>(slot);
+  float running[V];
 #pragma unroll
-    for (int j = 0; j < AT_ONCE; ++j) {
-      const int c = min(c0 + j, first + count - 1);
-      added[j] = chunk_state[((long)c * H + head) * per_head + element];
-      decay[j] = chunk_decay[(long)c * H + head];
-    }
+  for (int i = 0; i < V; ++i) running[i] = state[i];
+  if (count <= 4)
+    ssd_pass_rounds<V, 4>(chunk_state, chunk_decay, state_in, first, count, H, head, per_head, element, running);
+  else
+    ssd_pass_rounds<V, 16>(chunk_state, chunk_decay, state_in, first, count, H, head, per_head, element, running);
 #pragma unroll
-    for (int j = 0; j < AT_ONCE; ++j) {
-      if (c0 + j < first + count) {
-        state_in[((long)(c0 + j) * H + head) * per_head + element] = (bf16_t)running;
-        running = decay[j] * running + added[j];
-      }
-    }
-  }
-  *slot = running;
+  for (int i = 0; i < V; ++i) state[i] = running[i];
+  *reinterpret_cast<floats*>(slot) = state;
 }
 
 // ---------------------------------------------------------------- chunk scan
@@ -1114,11 +1145,20 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
     RETURN_IF_LAUNCH_FAILED();
   }
   {
+    // states and their areas are whole pieces of four (P * N is a multiple of 512) unless a caller's view begins
+    // in the middle of one
     const long per_head = (long)P * N;
-    const dim3 grid((unsigned)((per_head + 255) / 256), H + (conv_here ? (C + 255) / 256 : 0), n_lanes);
-    ssd_state_pass_kernel<<<grid, 256, 0, stream>>>(chunk_state, chunk_decay, lane_chunks, slot_ids, H, per_head,
-                                                    ssm_state, (bf16_t*)state_in, (const bf16_t*)u, u_ld, C, conv_k,
-                                                    (bf16_t*)conv_state, chunks, Q);
+    const bool pieces = (((uintptr_t)chunk_state | (uintptr_t)ssm_state) % 16) == 0 && ((uintptr_t)state_in % 8) == 0;
+    const int threads = pieces ? 64 : 256, each = pieces ? 4 : 1;
+    const dim3 grid((unsigned)((per_head / each + threads - 1) / threads),
+                    H + (conv_here ? (C + threads - 1) / threads : 0), n_lanes);
+#define PASS_CASE(V_)                                                                                              \
+  ssd_state_pass_kernel<V_><<<grid, threads, 0, stream>>>(chunk_state, chunk_decay, lane_chunks, slot_ids, H, per_head, \
+                                                          ssm_state, (bf16_t*)state_in, (const bf16_t*)u, u_ld, C,     \
+                                                          conv_k, (bf16_t*)conv_state, chunks, Q)
+    if (pieces) PASS_CASE(4);
+    else PASS_CASE(1);
+#undef PASS_CASE
     RETURN_IF_LAUNCH_FAILED();
   }
   const bool staged = ssd_staged_sizes(P, N) && ssd_scan_lds_bytes(Q, P, N) <= 64 * 1024;

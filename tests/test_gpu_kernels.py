@@ -610,6 +610,29 @@ def test_lanes_of_one_chunk_scan_in_one_launch(ops, Q, H, P, N, G, gate):
     assert not torch.equal(results[1][1], state) and not torch.equal(results[1][2], tails)
 
 
+@pytest.mark.parametrize("P, N", [(16, 32), (64, 128)])
+def test_states_pass_through_chunks_in_pieces_and_one_by_one(ops, P, N):
+    """The pass moves four neighbours a thread where the states lie at whole pieces and one where they do not: the same
+    numbers, for lanes of one chunk, of a short round and beside it, and of more than a long one."""
+    H, G, Q = 3, 1, 32
+    E = H * P
+    counts = [5, 4 * Q, 4 * Q + 1, 16 * Q, 17 * Q + 3]
+    T, slots = sum(counts), len(counts) + 1
+    xbc, dt = rand(T, E + 2 * N, seed=290, dtype=torch.bfloat16).to(DEV), rand(T, H, seed=291, dtype=torch.bfloat16).to(DEV)
+    dt_bias, A, D = gpu(rand(H, seed=292) - 1.0, -torch.exp(torch.linspace(-3.0, 1.0, H)), rand(H, seed=293))
+    start, ids = rand(slots, H, P, N, seed=294, scale=0.5).to(DEV), i32([3, 0, 5, 1, 4]).to(DEV)
+    results = []
+    for offset in (0, 1):
+        held = torch.zeros(start.numel() + 4, device=DEV)
+        state = held[offset:offset + start.numel()].view(start.shape)
+        state.copy_(start)
+        y = torch.full((T, E), float("nan"), device=DEV)
+        ops.ssd_prefill(xbc, dt, dt_bias, A, D, state, ops.SsdChunks(counts, Q, DEV), ids, G, y)
+        results.append((y, state))
+    for pieces, single in zip(*results):
+        assert bool(torch.isfinite(pieces).all()) and torch.equal(pieces, single)
+
+
 def test_chunked_scan_carries_a_far_token_through_many_chunks(ops):
     """One token with a large x and a head that barely decays: 600 tokens later its state is what
     the output consists of; every chunk boundary between must pass it on."""
