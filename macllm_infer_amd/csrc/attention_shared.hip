@@ -31,13 +31,16 @@
 #define SHARED_SPARE 32              // entries for the four stages that are asked for past the end, in pages of 8
 
 // U: steps of 32 keys whose scores are formed before the softmax.
-template <int DH, int NSET, int U>
-__global__ void __launch_bounds__(SHARED_WAVES * WAVE, DH * NSET == 64 ? 4 : 2)
+// BIAS: BIAS_LOG, the scores lose log_bias[head] = (r1, r2) -> r1 * ln(1 + r2 * distance).  sinks (may be null): one more term
+// exp(sinks[head]) of the softmax's denominator.
+template <int DH, int NSET, int U, int BIAS = BIAS_NONE>
+__global__ void __launch_bounds__(SHARED_WAVES * WAVE, DH * NSET == 64 && BIAS == BIAS_NONE ? 4 : 2)
 prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, const bf16_t* __restrict__ k_base,
                       const bf16_t* __restrict__ v_base, long page_stride, int page_shift,
                       const int* __restrict__ block_tables, int max_pages, const int* __restrict__ tiles,
                       const int* __restrict__ cu_seqlens, const int* __restrict__ start_pos, float scale, int window,
-                      bf16_t* __restrict__ out, long out_ld) {
+                      bf16_t* __restrict__ out, long out_ld, const float* __restrict__ log_bias,
+                      const float* __restrict__ sinks) {
   constexpr int FRAGMENTS = DH / 8;              // of K in a stage, and as many of V
   constexpr int PIECES = FRAGMENTS / 4;          // of either that a thread moves
   // two heads of 128: fragments are asked for four at a time, or they would spill
@@ -96,6 +99,14 @@ prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, 
 #pragma unroll
   for (int s = 0; s < NSET; ++s) highest[s] = -INFINITY;
   const float scale_log2 = scale * 1.4426950408889634f;
+  const float unit = BIAS == BIAS_NONE ? scale_log2 : 1.f;   // of a score towards units of log2: biased ones are there already
+  float bias_r1[NSET], bias_r2[NSET];
+#pragma unroll
+  for (int s = 0; s < NSET; ++s) {
+    const int head = min(head0 + s, Hq - 1);
+    bias_r1[s] = BIAS == BIAS_LOG ? log_bias[2 * head] : 0.f;
+    bias_r2[s] = BIAS == BIAS_LOG ? log_bias[2 * head + 1] : 0.f;
+  }
   const int page_mask = (1 << page_shift) - 1;
   const int key_lo = first_visible_key(base_position + tile_token, window) / SHARED_STAGE * SHARED_STAGE;
   const int key_hi = tile_last + 1;
@@ -132,6 +143,15 @@ prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, 
     float top[NSET][U];
 #pragma unroll
     for (int s = 0; s < NSET; ++s) {
+      if (BIAS == BIAS_LOG) {                    // a key past the column's position gets a bias of anything: it is masked
+#pragma unroll
+        for (int t = 0; t < 2 * U; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float distance = (float)(col_pos[s] - (k0 + 8 * qd + 32 * (t / 2) + 4 * (t % 2) + i));
+            score[s][t][i] = fmaf(score[s][t][i], scale_log2, -bias_r1[s] * __log2f(fmaf(bias_r2[s], fmaxf(distance, 0.f), 1.f)));
+          }
+      }
       if (MASKED) {
         // visible keys of the column relative to the lane's first: lo .. lo + span, one unsigned compare a score (an
         // empty range gets a lo that no offset reaches)
@@ -164,7 +184,7 @@ prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, 
       for (int st = 0; st < U; ++st) {
         // The sums are held relative to the largest score of the step's keys, not of all keys so far, as long as that is
         // within 2^16 of it: the largest weight of every step is then one, which bfloat16 holds exactly.
-        const float most = top[s][st] * scale_log2;                             // scale > 0: the maximum stays the maximum
+        const float most = top[s][st] * unit;                                   // scale > 0: the maximum stays the maximum
         highest[s] = fmaxf(highest[s], most);
         const float reference = fmaxf(most, highest[s] - 16.f);
         const float m_safe = reference == -INFINITY ? 0.f : reference;          // nothing visible yet
@@ -175,7 +195,7 @@ prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, 
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float p = __builtin_amdgcn_exp2f(fmaf(score[s][2 * st + t][i], scale_log2, -m_safe));
+            const float p = __builtin_amdgcn_exp2f(fmaf(score[s][2 * st + t][i], unit, -m_safe));
             sum += p;
             p_frag[s][st][4 * t + i] = (bf16_t)p;
           }
@@ -293,12 +313,15 @@ prefill_shared_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, 
   for (int s = 0; s < NSET; ++s) {
     const float* const other = part + (w * NSET + s) * ITEMS * WAVE + lane;
     const float m_other = other[0];
-    const float m = fmaxf(acc.m[s], m_other);
+    // the sink, in the scores' units of log2: it may be the largest term
+    const float sink = sinks ? sinks[min(head0 + s, Hq - 1)] * 1.4426950408889634f : -INFINITY;
+    const float m = fmaxf(fmaxf(acc.m[s], m_other), sink);
     const float factor = acc.m[s] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(acc.m[s] - m);
     const float factor_other = m_other == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_other - m);
     float l = acc.l[s] * factor + other[WAVE] * factor_other;
     l += __shfl_xor(l, 16, WAVE);
     l += __shfl_xor(l, 32, WAVE);
+    if (sinks) l += __builtin_amdgcn_exp2f(sink - m);       // once for the column: no key, no value
     if (col_pos[s] < 0) continue;
     const float inverse = 1.f / l;
     bf16_t* const o = out + (long)token * out_ld + (long)(head0 + s) * DH;
@@ -319,7 +342,7 @@ extern "C" int mi_prefill_attention_shared(const void* q, long q_ld, int Hq, int
                                            const void* v_base, long page_stride, int page_size, const int* block_tables,
                                            int max_pages, const int* tiles, int n_tiles, const int* cu_seqlens,
                                            const int* start_pos, float scale, int window, int nset, void* out,
-                                           long out_ld, hipStream_t stream) {
+                                           long out_ld, const float* log_bias, const float* sinks, hipStream_t stream) {
   if (n_tiles <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || page_size <= 0 || max_pages <= 0)
     return ERR_BAD_ARGUMENT;
   const int G = Hq / Hkv;
@@ -331,12 +354,17 @@ extern "C" int mi_prefill_attention_shared(const void* q, long q_ld, int Hq, int
   int page_shift = 0;
   while ((1 << page_shift) < page_size) ++page_shift;
   const dim3 grid(n_tiles, Hkv, (G + nset - 1) / nset);
-#define SHARED_CASE(DH_, NSET_, U_)                                                                                  \
-  if (dh == DH_ && nset == NSET_)                                                                                \
-    prefill_shared_kernel<DH_, NSET_, U_><<<grid, SHARED_WAVES * WAVE, 0, stream>>>(                                 \
-        (const bf16_t*)q, q_ld, Hq, Hkv, (const bf16_t*)k_base, (const bf16_t*)v_base, page_stride, page_shift,  \
-        block_tables, max_pages, tiles, cu_seqlens, start_pos, scale, window, (bf16_t*)out, out_ld);
+#define SHARED_LAUNCH(DH_, NSET_, U_, BIAS_)                                                                      \
+  prefill_shared_kernel<DH_, NSET_, U_, BIAS_><<<grid, SHARED_WAVES * WAVE, 0, stream>>>(                        \
+      (const bf16_t*)q, q_ld, Hq, Hkv, (const bf16_t*)k_base, (const bf16_t*)v_base, page_stride, page_shift,    \
+      block_tables, max_pages, tiles, cu_seqlens, start_pos, scale, window, (bf16_t*)out, out_ld, log_bias, sinks)
+#define SHARED_CASE(DH_, NSET_, U_)                                                                              \
+  if (dh == DH_ && nset == NSET_) {                                                                              \
+    if (log_bias) SHARED_LAUNCH(DH_, NSET_, U_, BIAS_LOG);                                                       \
+    else SHARED_LAUNCH(DH_, NSET_, U_, BIAS_NONE);                                                               \
+  }
   SHARED_CASE(64, 1, 2) SHARED_CASE(128, 1, 2) SHARED_CASE(128, 2, 1)
+#undef SHARED_LAUNCH
 #undef SHARED_CASE
   RETURN_IF_LAUNCH_FAILED();
   return 0;

@@ -146,7 +146,7 @@ _SIGNATURES = {
     "attention_shared": {
         "mi_prefill_attention_shared": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_long, _c_int,
                                         _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int, _c_int,
-                                        _c_ptr, _c_long, _c_ptr],
+                                        _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr],
     },
     "attention_widths": {
         "mi_prefill_attention_padded": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_long, _c_int,
@@ -1627,7 +1627,7 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     gate_ld = _gate_rows(gate, out, "prefill_attention")
     _need(gate is None or (gate_ld % 4 == 0 and gate.data_ptr() % 8 == 0), "prefill_attention: the gate's rows lie in pieces of four")
     own_width = head_dim in (64, 128) and value_dim == head_dim
-    if (own_width and log_bias is None and sinks is None and slopes is None and gate is None and keep_first == 0
+    if (own_width and slopes is None and gate is None and keep_first == 0
             and page_size >= 8 and page_size & (page_size - 1) == 0 and page_stride % 8 == 0
             and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and out_ld % 4 == 0):
         heads = shared_prefill_heads(query_tiles.shape[0], num_heads, num_kv_heads, head_dim, int(max_seq_len or 0),
@@ -1636,7 +1636,8 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
             _check(_fn("attention_shared", "mi_prefill_attention_shared")(
                 _p(q), q_ld, num_heads, num_kv_heads, head_dim, _p(k_cache), _p(v_cache), page_stride, page_size,
                 _p(block_tables), block_tables.shape[1], _p(query_tiles), query_tiles.shape[0], _p(cu_seqlens),
-                _p(start_pos), float(scale), span_code, heads, _p(out), out_ld, _stream()), "prefill_attention")
+                _p(start_pos), float(scale), span_code, heads, _p(out), out_ld, _p(log_bias),
+                _p(sinks), _stream()), "prefill_attention")
             return
     _need(own_width or log_bias is None, "prefill_attention: the logarithmic bias comes with heads of 64 or 128 and values as wide")
     _check(_fn(*(("attention", "mi_prefill_attention") if own_width else ("attention_widths", "mi_prefill_attention_padded")))(

@@ -2,7 +2,8 @@
 retention and lightning attention (a fixed decay per head), gated linear attention (a decay per key channel) and the
 generalized delta rule (a decay per key channel and a removal of what the state holds along the unit key).  All keep their state [heads, value dim, key dim] in float32 in the
 request's state slot and run through one scan kernel (``ops.linear_state_scan``), for prompt portions and for
-single decoded tokens alike; rotation, decays, gates of the recurrence and unit keys are formed in float32 inside
+single decoded tokens alike, but that retention and the delta rule take bfloat16 portions of ``MATRIX_FROM`` tokens on to
+the float32 matrix cores (``ops.linear_matrix_scan``) and lightning attention has chunks of its own; rotation, decays, gates of the recurrence and unit keys are formed in float32 inside
 it.  The head-wise root-mean-square norm, its weight and the output gate are one more launch.
 """
 from __future__ import annotations

@@ -1576,11 +1576,11 @@ def test_prefill_attention_many_short_portions(ops, Hq, Hkv, dh):
 
 @pytest.mark.parametrize("Hq, Hkv, dh, page_size, window", [(8, 2, 64, 16, None), (3, 1, 64, 8, None), (2, 2, 64, 128, 70),
                                                               (12, 2, 128, 16, None), (4, 4, 128, 64, 33), (5, 1, 128, 8, 1)])
-@pytest.mark.parametrize("copies", [1, 12])
-def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_size, window, copies):
+@pytest.mark.parametrize("copies, terms", [(1, False), (12, False), (1, True)])
+def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_size, window, copies, terms):
     """The kernel whose waves share their keys, held against the one whose waves read them alone: portions that end
     at and beside the edges of a wave's 16 tokens, a tile of 64 and a stage of 64 keys, behind prefixes that do the same;
-    few workgroups and many, with one query head and with two.  Unwritten cells hold NaN, as do the cells of passed
+    few workgroups and many, with one query head and with two, with and without a logarithmic bias and sinks.  Unwritten cells hold NaN, as do the cells of passed
     pages.  Both round their weights to bfloat16 and sum in float32: they may differ by the rounding of an output."""
     dtype = torch.bfloat16
     starts = [0, 37, 0, 64, 127, 500, 0, 129, 9000 if copies == 1 and page_size == 8 else 700] * copies
@@ -1599,13 +1599,15 @@ def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_
     assert ops.shared_prefill_heads(tiles.shape[0], Hq, Hkv, dh, 2000, window or 0) in (0, 1, 2)
     got = {}
     device_pool, live = pool.to(DEV), table.clone()
+    bias, sinks = gpu(rand(Hq, 2, seed=613).abs(), 3.0 * rand(Hq, seed=614)) if terms else (None, None)
     for lane, start in enumerate(starts if window else []):      # pages that every query has passed were given back
         live[lane, :max(0, start - window + 1) // page_size] = -1
     for heads in (0, 1) if dh == 64 else (0, 1, 2):
         monkeypatch.setattr(ops, "shared_prefill_heads", lambda *args: heads)
         got[heads] = torch.full((T, Hq * dh), float("nan"), dtype=dtype, device=DEV)
         ops.prefill_attention(q, Hq, Hkv, dh, *views(device_pool, page_size), (live if heads else table).to(DEV),
-                              tiles.to(DEV), cu.to(DEV), i32(starts).to(DEV), 0.21, window, got[heads], max(lengths))
+                              tiles.to(DEV), cu.to(DEV), i32(starts).to(DEV), 0.21, window, got[heads], max(lengths),
+                              log_bias=bias, sinks=sinks)
     for heads in list(got)[1:]:
         assert torch.isfinite(got[heads].float()).all()
         close(got[heads], got[0].cpu(), dtype, 2.0)
