@@ -83,6 +83,36 @@ __device__ __forceinline__ lm_floatx4 lm_columns(const float* at, int stride, in
   return value;
 }
 
+// acc + a tile on a triangle's diagonal (16 x 16 at `at`, zero above the diagonal, STRICT: and on it) times `right`.  A row
+// of the result is a token's and takes the tokens up to its own (STRICT: before it); a later token's infinity or NaN must
+// not reach it through a product with zero: such values stay out of the product and are added to their own rows.
+template <bool STRICT>
+__device__ __forceinline__ lm_floatx4 lm_diagonal(const float* at, int stride, int q, int r, const lm_floatx4& right, lm_floatx4 acc) {
+  lm_floatx4 numbers;
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool number = __builtin_isfinite(right[i]);
+    finite &= number;
+    numbers[i] = number ? right[i] : 0.f;
+  }
+  acc = lm_mfma(lm_rows(at, stride, q, r), numbers, acc);
+  if (__all(finite)) return acc;
+#pragma unroll 1
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int s = 4 * g + j;
+      const float value = __shfl(right[j], 16 * g + r, WAVE);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = 4 * q + i;
+        if (!__builtin_isfinite(value) && (STRICT ? s < t : s <= t)) acc[i] = fmaf(at[t * stride + s], value, acc[i]);
+      }
+    }
+  return acc;
+}
+
 template <int KIND, int DK, int N>
 static constexpr long lm_run_floats(int dv) { return (long)N * DK + (long)dv * DK + (KIND == LM_DELTA ? DK * DK : 0); }
 
@@ -289,7 +319,8 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
       for (int ti = 0; ti < T; ++ti) {
         z[ti] = lm_floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int tj = 0; tj <= ti; ++tj) z[ti] = lm_mfma(lm_rows(P + 16 * ti * TS + 16 * tj, TS, q, r), v[tj], z[ti]);
+        for (int tj = 0; tj < ti; ++tj) z[ti] = lm_mfma(lm_rows(P + 16 * ti * TS + 16 * tj, TS, q, r), v[tj], z[ti]);
+        z[ti] = lm_diagonal<true>(P + 16 * ti * TS + 16 * ti, TS, q, r, v[ti], z[ti]);
       }
     }
     __syncthreads();
@@ -300,7 +331,7 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
       lm_floatx4 known = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int tj = 0; tj < ti; ++tj) known = lm_mfma(lm_rows(L + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], known);
-      z[ti] = lm_mfma(lm_rows(inverse + ti * 16 * 20, 20, q, r), z[ti] - known, lm_floatx4{0.f, 0.f, 0.f, 0.f});
+      z[ti] = lm_diagonal<false>(inverse + ti * 16 * 20, 20, q, r, z[ti] - known, lm_floatx4{0.f, 0.f, 0.f, 0.f});
     }
   } else if (!has_values) {
     return;
@@ -312,7 +343,8 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
     for (int ti = 0; ti < T; ++ti) {
       lm_floatx4 removed = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int tj = 0; tj <= ti; ++tj) removed = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], removed);
+      for (int tj = 0; tj < ti; ++tj) removed = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], removed);
+      removed = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], removed);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 16 * ti + 4 * q + i;
@@ -338,10 +370,12 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
   for (int ti = 0; ti < T; ++ti) {
     lm_floatx4 given = {0.f, 0.f, 0.f, 0.f}, removed = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int tj = 0; tj <= ti; ++tj) {
+    for (int tj = 0; tj < ti; ++tj) {
       given = lm_mfma(lm_rows(RK + 16 * ti * TS + 16 * tj, TS, q, r), v[tj], given);
       if (DELTA) removed = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], removed);
     }
+    given = lm_diagonal<false>(RK + 16 * ti * TS + 16 * ti, TS, q, r, v[ti], given);
+    if (DELTA) removed = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], removed);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = 16 * ti + 4 * q + i;

@@ -172,6 +172,54 @@ def test_runs_on_the_matrix_cores_give_the_walk_s_numbers(delta, H, dk, dv, rota
     assert torch.equal(got_state.cpu()[untouched], state[untouched])
 
 
+@pytest.mark.parametrize("delta, dk, dv", [(False, 64, 64), (False, 128, 32), (True, 64, 64)])
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+@pytest.mark.parametrize("part", ["v", "k", "r", "removal", "decay"])
+def test_a_token_that_is_no_number_leaves_the_tokens_before_it_alone(delta, dk, dv, bad, part):
+    """An infinity or NaN in a token's value, key, query, removal rate or decay, at the first, a middle and the last place
+    of a tile of 16: the tokens before it keep their bits, and what is finite behind it is what the walk has finite."""
+    if not delta and part in ("removal", "decay"):
+        pytest.skip("retention has no such part")
+    from macllm_infer_amd.kernels import ops, build
+    build.ensure_modules(["linear_state", "linear_matrix"])
+    H, T = 2, 90
+    generator = torch.Generator().manual_seed(dk)
+    u = (torch.randn(T, 3 * H * dk + H * dv, generator=generator) * 0.7).to(torch.bfloat16).to(DEV)
+    state = (torch.randn(1, H, dv, dk, generator=generator) * 0.3).to(DEV)
+    columns = dict(q_col=0, k_col=H * dk, v_col=2 * H * dk, num_heads=H, key_dim=dk, value_dim=dv)
+    if delta:
+        logits = torch.randn(T, H * dk, generator=generator).to(DEV)
+        recurrence = dict(removal_col=2 * H * dk + H * dv, decay_bias=torch.zeros(H * dk, device=DEV), decay_floor=math.exp(-0.5), key_eps=1e-6)
+    else:
+        logits, recurrence = None, dict(head_decay=torch.tensor([0.97, 0.0], device=DEV), key_scale=dk ** -0.5)
+    i32 = lambda values: torch.tensor(values, dtype=torch.int32, device=DEV)
+
+    def run(scan, token):
+        rows, decay_logits = u.clone(), logits.clone() if delta else None
+        if token is not None:
+            if part == "decay":
+                decay_logits[token, 3] = bad if bad != math.inf else math.nan      # (an infinite one is a decay of the floor)
+            else:
+                rows[token, {"v": 2 * H * dk, "k": H * dk, "r": 0, "removal": 2 * H * dk + H * dv}[part] + 3] = bad if part != "removal" else math.nan
+        out, now = torch.zeros(T, H * dv, device=DEV), state.clone()
+        common = dict(**columns, **recurrence, state=now, slot_ids=i32([0]), out=out)
+        if delta:
+            common.update(decay_logits=decay_logits)
+        if scan == "matrix":
+            ops.linear_matrix_scan(rows, **common, chunks=ops.SsdChunks([T], 128, DEV))
+        else:
+            ops.linear_state_scan(rows, **common, cu_seqlens=i32([0, T]), max_query_len=T)
+        return out, now
+
+    clean, _ = run("matrix", None)
+    for token in (32, 37, 47, 63, 64, 79):
+        out, now = run("matrix", token)
+        walked, walked_state = run("walk", token)
+        assert torch.equal(out[:token], clean[:token]), token
+        assert torch.equal(torch.isfinite(out), torch.isfinite(walked)), token
+        assert torch.equal(torch.isfinite(now), torch.isfinite(walked_state)), token
+
+
 def test_heads_the_matrix_cores_do_not_cover_stay_with_the_walk():
     from macllm_infer_amd.kernels import ops
     covered = lambda *sizes, dtype=torch.bfloat16, floor=None: ops.linear_matrix_supported(dtype, *sizes, floor)
