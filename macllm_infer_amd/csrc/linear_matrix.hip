@@ -15,17 +15,25 @@
 //     carry   a workgroup a (lane of the step, head, 16 value channels) walks the lane's runs: O = Ov + Ro S, S <- M S + Nv
 //             (retention: S <- decay^N S + Nv), the next runs' matrices on their way meanwhile
 // Every w_t is at least exp(-decay_floor), and 1 / d_t at most exp(N decay_floor): the caller keeps that within float32.
-// log d_t is summed in double and its exponential taken in two parts, so that d_t / d_s keeps float32's precision.
+// What is in float32 and what in 64 bits: states, operands and the products over tokens are float32.  The d_t are 64-bit
+// products of the w_t, so that B, A, K, R (and A and K as they stand at the run's end, for M and Nv) are rounded once; the
+// triangles, whose sums over all key channels are the longest, are summed in 64 bits (v_mfma_f64_16x16x4_f64) and rounded
+// once; the sums over tokens run from the oldest to the newest, whose terms are as a rule the largest; the carry's sums
+// over key channels are chains of 16.  Off 64 bits, in units of the result's norm, outputs and (states) of the walk and of
+// this, 300 tokens: delta rule with 16 heads of 64 channels 1.01e-7 (7.4e-8) and 7.4e-8 (5.8e-8), decays near their floor
+// of exp(-0.6) 8.4e-8 (4.8e-8) and 6.3e-8 (4.7e-8), near one 5.9e-7 (7.5e-7) and 1.9e-7 (2.1e-7), 8 heads of 128 channels
+// 1.07e-7 (7.5e-8) and 7.5e-8 (5.9e-8); retention 3.0e-7 (3.5e-7) and 1.6e-7 (1.5e-7).  (All in float32, one chain a sum:
+// 1.6e-7 (1.0e-7), 1.35e-7 (9.4e-8), 2.6e-7 (2.8e-7), 2.0e-7 (1.1e-7), 2.0e-7 (1.5e-7), and 98 instead of the 104 us below.)
 // What bounds it: the chunk kernel its products (some 110 matrix instructions a value wave and run of 32 tokens) and the
 // waits between its stages; the carry what one compute unit can fetch, 30 KB a run at 28 KB a microsecond, of M alone 16.
-// 1,999 tokens, in microseconds with both kernels, before (the three passes of linear_state.hip) and now: delta rule with 16
-// heads of 64 channels 292 and 101, retention with 8 heads of 64 and 128 channels 139 and 48; 100 tokens, where the walk
-// went from end to end: 98 and 21, 64 and 19.  Off 64 bits by 1.6e-7 (delta rule, 1.0e-7 before) and 2.3e-7 (3.3e-7) of the
-// outputs' norm: float32's own rounding, in front of a norm that rounds to bfloat16.
+// 1,999 tokens, in microseconds with both kernels, the three passes of linear_state.hip and this: delta rule with 16
+// heads of 64 channels 244 and 104, retention with 8 heads of 64 and 128 channels 125 and 48; 100 tokens, where the walk
+// goes from end to end: 96 and 23, 63 and 21.
 #include "common.h"
 #include <cstdint>
 
 typedef float lm_floatx4 __attribute__((ext_vector_type(4)));
+typedef double lm_doublex4 __attribute__((ext_vector_type(4)));
 
 #define LM_RETENTION 0
 #define LM_DELTA 1
@@ -58,16 +66,16 @@ struct LinearMatrixArgs {
 
 __device__ __forceinline__ float lm_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// exp(sign * x) of a double: its float and what that leaves
-__device__ __forceinline__ float lm_exp(double x, float sign) {
-  const float whole = (float)x;
-  const float rest = (float)(x - (double)whole);
-  return expf(sign * whole) * (1.0f + sign * rest);
-}
-
 __device__ __forceinline__ lm_floatx4 lm_mfma(const lm_floatx4& a, const lm_floatx4& b, lm_floatx4 acc) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], acc, 0, 0, 0);
+  return acc;
+}
+
+// the same with products and sums in 64 bits
+__device__ __forceinline__ lm_doublex4 lm_mfma_double(const lm_floatx4& a, const lm_floatx4& b, lm_doublex4 acc) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[i], (double)b[i], acc, 0, 0, 0);
   return acc;
 }
 
@@ -82,6 +90,10 @@ __device__ __forceinline__ lm_floatx4 lm_columns(const float* at, int stride, in
   for (int i = 0; i < 4; ++i) value[i] = at[(4 * q + i) * stride + r];
   return value;
 }
+
+// The rows of LDS that belong to a tile of 16 tokens are permuted (row 4a + b is token 4b + a, and the other way round): one
+// matrix instruction then sums four neighbouring tokens, and a product's chain runs from the oldest token to the newest.
+__device__ __forceinline__ constexpr int lm_place(int at) { return (at & ~15) + 4 * (at & 3) + ((at >> 2) & 3); }
 
 // acc + a tile on a triangle's diagonal (16 x 16 at `at`, zero above the diagonal, STRICT: and on it) times `right`.  A row
 // of the result is a token's and takes the tokens up to its own (STRICT: before it); a later token's infinity or NaN must
@@ -107,7 +119,8 @@ __device__ __forceinline__ lm_floatx4 lm_diagonal(const float* at, int stride, i
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 4 * q + i;
-        if (!__builtin_isfinite(value) && (STRICT ? s < t : s <= t)) acc[i] = fmaf(at[t * stride + s], value, acc[i]);
+        const bool sees = STRICT ? lm_place(s) < lm_place(t) : lm_place(s) <= lm_place(t);
+        if (!__builtin_isfinite(value) && sees) acc[i] = fmaf(at[t * stride + s], value, acc[i]);
       }
     }
   return acc;
@@ -141,7 +154,7 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
   float* const A = B + N * KS;
   float* const inverse = A + N * KS;                    // [T][16][20]: the inverses of I + L's diagonal blocks
   float* const last = inverse + T * 16 * 20;            // d_N
-  double* const sums = reinterpret_cast<double*>(last + DK);   // [waves][DK]
+  double* const products = reinterpret_cast<double*>(last + DK);   // [waves][DK]: of the waves' decays
 
   const int* row = a.chunks + 4 * (blockIdx.x / RUNS);
   if (row[0] < 0) return;                               // a row past the step's own chunks
@@ -163,17 +176,18 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
   float* const Nv = Ro + N * DK;                        // [dv][DK], transposed as the state is
   float* const M = Nv + (long)dv * DK;                  // [DK][DK]
 
-  lm_floatx4 v[T];                                      // the values as right operands: row 16j + 4q + i, column r
+  lm_floatx4 v[T];                                      // the values as right operands: row 16j + 4q + i (lm_place), column r
 #pragma unroll
   for (int j = 0; j < T; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int t = 16 * j + 4 * q + i;
+      const int t = 16 * j + 4 * i + q;
       const float value = (float)a.u[(t0 + min(t, count - 1)) * a.ld + a.v_col + (long)head * dv + (has_values ? 16 * value_tile + r : 0)];
       v[j][i] = t < count ? value : 0.f;
     }
 
-  // ---- B, A, K and R, a wave PT tokens in a row, a lane PC channels
+  // ---- B, A, K and R, a wave PT tokens in a row, a lane PC channels (and A and K as they stand at the run's end)
+  float a_end[PT][PC], k_end[PT][PC];
   if (!DELTA) {
     const float decay = a.head_decay[head];
     for (int n = threadIdx.x; n <= N; n += blockDim.x) powers[n] = n == 0 ? 1.f : powf(decay, (float)n);
@@ -199,14 +213,15 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
             rx = low ? rx * cosine - r_pair * sine : rx * cosine + r_pair * sine;
             kx = low ? kx * cosine - k_pair * sine : kx * cosine + k_pair * sine;
           }
-          R[t * KS + c] = valid ? rx : 0.f;
-          K[t * KS + c] = valid ? kx * a.key_scale : 0.f;
+          R[lm_place(t) * KS + c] = valid ? rx : 0.f;
+          K[lm_place(t) * KS + c] = valid ? kx * a.key_scale : 0.f;
           Ro[t * DK + c] = valid ? rx * powers[t + 1] : 0.f;
         }
       }
     }
   } else {
-    float kx[PT][PC], rx[PT][PC], removal[PT][PC], step[PT][PC];
+    float kx[PT][PC], rx[PT][PC], removal[PT][PC], logit[PT][PC];
+    double w[PT][PC];
     if (wave < LM_PREP_WAVES) {
 #pragma unroll
       for (int j = 0; j < PT; ++j) {
@@ -218,32 +233,38 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
           kx[j][pc] = (float)from[a.k_col + c];
           rx[j][pc] = (float)from[a.r_col + c];
           removal[j][pc] = (float)from[a.removal_col + c];
-          step[j][pc] = a.decay_logits[token * a.logits_ld + (long)head * DK + c];
+          logit[j][pc] = a.decay_logits[token * a.logits_ld + (long)head * DK + c];
         }
       }
-      double before[PC];
+      double kept[PC];                                  // of a state over this wave's tokens
 #pragma unroll
-      for (int pc = 0; pc < PC; ++pc) before[pc] = 0.0;
+      for (int pc = 0; pc < PC; ++pc) kept[pc] = 1.0;
 #pragma unroll
       for (int j = 0; j < PT; ++j) {
         const bool valid = wave * PT + j < count;
 #pragma unroll
         for (int pc = 0; pc < PC; ++pc) {
           const int c = lane + WAVE * pc;
-          step[j][pc] = valid ? -a.decay_floor * lm_sigmoid(step[j][pc] + a.decay_bias[head * DK + c]) : 0.f;
-          before[pc] += (double)step[j][pc];
+          const float rate = lm_sigmoid(logit[j][pc] + a.decay_bias[head * DK + c]);
+          w[j][pc] = valid ? exp((double)(-a.decay_floor * rate)) : 1.0;
+          kept[pc] *= w[j][pc];
         }
       }
 #pragma unroll
-      for (int pc = 0; pc < PC; ++pc) sums[wave * DK + lane + WAVE * pc] = before[pc];
+      for (int pc = 0; pc < PC; ++pc) products[wave * DK + lane + WAVE * pc] = kept[pc];
     }
     __syncthreads();
     if (wave < LM_PREP_WAVES) {
-      double log_d[PC];
+      double d[PC], d_last[PC];                         // d_(t-1), d_N
 #pragma unroll
       for (int pc = 0; pc < PC; ++pc) {
-        log_d[pc] = 0.0;
-        for (int w = 0; w < wave; ++w) log_d[pc] += sums[w * DK + lane + WAVE * pc];
+        d[pc] = d_last[pc] = 1.0;
+        for (int other = 0; other < LM_PREP_WAVES; ++other) {
+          const double product = products[other * DK + lane + WAVE * pc];
+          if (other < wave) d[pc] *= product;
+          d_last[pc] *= product;
+        }
+        if (wave == 0) last[lane + WAVE * pc] = (float)d_last[pc];
       }
 #pragma unroll
       for (int j = 0; j < PT; ++j) {
@@ -257,13 +278,15 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
         for (int pc = 0; pc < PC; ++pc) {
           const int c = lane + WAVE * pc;
           const float unit = kx[j][pc] / length;
-          B[t * KS + c] = valid ? lm_exp(log_d[pc], 1.f) * unit : 0.f;
-          log_d[pc] += (double)step[j][pc];
-          const float shrunk = lm_exp(log_d[pc], 1.f), grown = lm_exp(log_d[pc], -1.f);
-          A[t * KS + c] = valid ? grown * (lm_sigmoid(removal[j][pc]) * unit) : 0.f;
-          K[t * KS + c] = valid ? grown * kx[j][pc] : 0.f;
-          R[t * KS + c] = valid ? shrunk * rx[j][pc] : 0.f;
-          if (t == N - 1) last[c] = shrunk;
+          const double key = kx[j][pc], away = lm_sigmoid(removal[j][pc]) * unit;
+          B[lm_place(t) * KS + c] = valid ? (float)(d[pc] * (double)unit) : 0.f;
+          d[pc] *= w[j][pc];
+          const double grown = 1.0 / d[pc], to_end = d_last[pc] * grown;
+          A[lm_place(t) * KS + c] = valid ? (float)(grown * away) : 0.f;
+          K[lm_place(t) * KS + c] = valid ? (float)(grown * key) : 0.f;
+          R[lm_place(t) * KS + c] = valid ? (float)(d[pc] * (double)rx[j][pc]) : 0.f;
+          a_end[j][pc] = valid ? (float)(to_end * away) : 0.f;
+          k_end[j][pc] = valid ? (float)(to_end * key) : 0.f;
         }
       }
     }
@@ -280,19 +303,27 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
     const float* left = (which < 2 ? R : B) + 16 * ti * KS;
     const float* right = ((which & 1) ? A : K) + 16 * tj * KS;
     float* into = which == 0 ? RK : which == 1 ? RA : which == 2 ? P : L;
-    lm_floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    lm_doublex4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int c = 0; c < KT; ++c) acc = lm_mfma(lm_rows(left + 16 * c, KS, q, r), lm_rows(right + 16 * c, KS, q, r), acc);
-    const int s = 16 * tj + r;
+    for (int c = 0; c < KT; ++c) acc = lm_mfma_double(lm_rows(left + 16 * c, KS, q, r), lm_rows(right + 16 * c, KS, q, r), acc);
+    const int s = lm_place(16 * tj + r);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * ti + 4 * q + i;
-      float value = acc[i];
-      if (!DELTA) value *= powers[max(t - s, 0)];
-      into[t * TS + s] = (which < 2 ? s <= t : s < t) ? value : 0.f;
+    for (int i = 0; i < 4; ++i) {                       // (rows of a result in 64 bits lie four apart in a lane)
+      const int at = 16 * ti + 4 * i + q, t = lm_place(at);
+      if (!DELTA) acc[i] *= (double)powers[max(t - s, 0)];
+      into[at * TS + 16 * tj + r] = (which < 2 ? s <= t : s < t) ? (float)acc[i] : 0.f;
     }
   }
   __syncthreads();
+  if (DELTA && wave < LM_PREP_WAVES) {                  // (read behind the next barrier)
+#pragma unroll
+    for (int j = 0; j < PT; ++j)
+#pragma unroll
+      for (int pc = 0; pc < PC; ++pc) {
+        A[lm_place(wave * PT + j) * KS + lane + WAVE * pc] = a_end[j][pc];
+        K[lm_place(wave * PT + j) * KS + lane + WAVE * pc] = k_end[j][pc];
+      }
+  }
 
   lm_floatx4 z[T];                                      // this wave's 16 columns of [Zk | Zv], rows 16j + 4q + i
   if (DELTA) {
@@ -304,14 +335,14 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
         const float* block = L + (16 * wave) * TS + 16 * wave;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          float sum = i == r ? 1.f : 0.f;
+          float sum = i == lm_place(r) ? 1.f : 0.f;
 #pragma unroll
-          for (int m = 0; m < i; ++m) sum = fmaf(-block[i * TS + m], x[m], sum);
+          for (int m = 0; m < i; ++m) sum = fmaf(-block[lm_place(i) * TS + lm_place(m)], x[m], sum);
           x[i] = sum;
         }
         if (q == 0) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) inverse[(wave * 16 + i) * 20 + r] = x[i];
+          for (int i = 0; i < 16; ++i) inverse[(wave * 16 + lm_place(i)) * 20 + r] = x[i];
         }
       }
     } else if (has_values) {
@@ -333,6 +364,8 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
       for (int tj = 0; tj < ti; ++tj) known = lm_mfma(lm_rows(L + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], known);
       z[ti] = lm_diagonal<false>(inverse + ti * 16 * 20, 20, q, r, z[ti] - known, lm_floatx4{0.f, 0.f, 0.f, 0.f});
     }
+#pragma unroll
+    for (int ti = 0; ti < T; ++ti) z[ti] = -z[ti];      // what is taken away
   } else if (!has_values) {
     return;
   }
@@ -341,65 +374,61 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
     // 16 columns of Ro and M
 #pragma unroll
     for (int ti = 0; ti < T; ++ti) {
-      lm_floatx4 removed = {0.f, 0.f, 0.f, 0.f};
+      lm_floatx4 taken = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int tj = 0; tj < ti; ++tj) removed = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], removed);
-      removed = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], removed);
+      for (int tj = 0; tj < ti; ++tj) taken = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], taken);
+      taken = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], taken);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int t = 16 * ti + 4 * q + i;
-        Ro[t * DK + 16 * wave + r] = R[t * KS + 16 * wave + r] - removed[i];
+        const int at = 16 * ti + 4 * q + i;
+        Ro[lm_place(at) * DK + 16 * wave + r] = R[at * KS + 16 * wave + r] + taken[i];
       }
     }
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
-      lm_floatx4 removed = {0.f, 0.f, 0.f, 0.f};
+      lm_floatx4 taken = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int tj = 0; tj < T; ++tj) removed = lm_mfma(lm_columns(A + 16 * tj * KS + 16 * kt, KS, q, r), z[tj], removed);
+      for (int tj = 0; tj < T; ++tj) taken = lm_mfma(lm_columns(A + 16 * tj * KS + 16 * kt, KS, q, r), z[tj], taken);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int k = 16 * kt + 4 * q + i, c = 16 * wave + r;
-        M[k * DK + c] = last[k] * ((k == c ? 1.f : 0.f) - removed[i]);
+        M[k * DK + c] = (k == c ? last[k] : 0.f) + taken[i];
       }
     }
     return;
   }
 
-  // ---- 16 value channels of Ov and Nv
+  // ---- 16 value channels of Ov and Nv: one chain of sums each, from the oldest tokens to the newest, whose terms are as a rule
+  // the largest
 #pragma unroll
   for (int ti = 0; ti < T; ++ti) {
-    lm_floatx4 given = {0.f, 0.f, 0.f, 0.f}, removed = {0.f, 0.f, 0.f, 0.f};
+    lm_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int tj = 0; tj < ti; ++tj) {
-      given = lm_mfma(lm_rows(RK + 16 * ti * TS + 16 * tj, TS, q, r), v[tj], given);
-      if (DELTA) removed = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], removed);
+      if (DELTA) sum = lm_mfma(lm_rows(RA + 16 * ti * TS + 16 * tj, TS, q, r), z[tj], sum);
+      sum = lm_mfma(lm_rows(RK + 16 * ti * TS + 16 * tj, TS, q, r), v[tj], sum);
     }
-    given = lm_diagonal<false>(RK + 16 * ti * TS + 16 * ti, TS, q, r, v[ti], given);
-    if (DELTA) removed = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], removed);
+    if (DELTA) sum = lm_diagonal<false>(RA + 16 * ti * TS + 16 * ti, TS, q, r, z[ti], sum);
+    sum = lm_diagonal<false>(RK + 16 * ti * TS + 16 * ti, TS, q, r, v[ti], sum);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int t = 16 * ti + 4 * q + i;
-      if (t < count) a.out[(t0 + t) * a.out_ld + (long)head * dv + 16 * value_tile + r] = given[i] - removed[i];
+      const int t = 16 * ti + 4 * i + q;
+      if (t < count) a.out[(t0 + t) * a.out_ld + (long)head * dv + 16 * value_tile + r] = sum[i];
     }
   }
   if (!DELTA) {                                         // the keys' way to the run's end, laid on the values
 #pragma unroll
     for (int j = 0; j < T; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[j][i] *= powers[max(count - 1 - (16 * j + 4 * q + i), 0)];
+      for (int i = 0; i < 4; ++i) v[j][i] *= powers[max(count - 1 - (16 * j + 4 * i + q), 0)];
   }
 #pragma unroll
   for (int kt = 0; kt < KT; ++kt) {
-    lm_floatx4 given = {0.f, 0.f, 0.f, 0.f}, removed = {0.f, 0.f, 0.f, 0.f};
+    lm_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int tj = 0; tj < T; ++tj) {
-      given = lm_mfma(lm_columns(K + 16 * tj * KS + 16 * kt, KS, q, r), v[tj], given);
-      if (DELTA) removed = lm_mfma(lm_columns(A + 16 * tj * KS + 16 * kt, KS, q, r), z[tj], removed);
-    }
-    lm_floatx4 sum = given - removed;
-    if (DELTA) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sum[i] *= last[16 * kt + 4 * q + i];
+      if (DELTA) sum = lm_mfma(lm_columns(A + 16 * tj * KS + 16 * kt, KS, q, r), z[tj], sum);
+      sum = lm_mfma(lm_columns(K + 16 * tj * KS + 16 * kt, KS, q, r), v[tj], sum);
     }
     *reinterpret_cast<lm_floatx4*>(Nv + (long)(16 * value_tile + r) * DK + 16 * kt + 4 * q) = sum;
   }
@@ -478,7 +507,12 @@ __global__ void __launch_bounds__((KIND == LM_DELTA ? N / 16 + DK / 16 : 4) * WA
       lm_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
       if (DELTA || outputs) {
 #pragma unroll
-        for (int c = 0; c < KT; ++c) sum = lm_mfma(lm_rows(s_now + 16 * c, KS, q, r), rows[at][c], sum);
+        for (int c = 0; c < KT; c += 4) {               // a chain for every 16 channels, added in pairs
+          lm_floatx4 part[4];
+#pragma unroll
+          for (int p = 0; p < 4; ++p) part[p] = lm_mfma(lm_rows(s_now + 16 * (c + p), KS, q, r), rows[at][c + p], lm_floatx4{0.f, 0.f, 0.f, 0.f});
+          sum += (part[0] + part[1]) + (part[2] + part[3]);
+        }
       }
       if (outputs) {                                    // value channels 4q + i of token r
         const int t = j * N + 16 * wave + r;

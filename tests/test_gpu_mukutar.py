@@ -172,6 +172,46 @@ def test_runs_on_the_matrix_cores_give_the_walk_s_numbers(delta, H, dk, dv, rota
     assert torch.equal(got_state.cpu()[untouched], state[untouched])
 
 
+@pytest.mark.parametrize("delta, dk, dv, floor, shift", [
+    (False, 64, 128, 0.0, 0.0), (False, 128, 64, 0.0, 0.0), (True, 64, 64, 0.625, 0.0), (True, 64, 64, 0.625, 5.0),
+    (True, 64, 64, 0.625, -6.0), (True, 128, 128, 0.625, 0.0), (True, 64, 64, 1.875, 5.0)])
+def test_runs_on_the_matrix_cores_are_no_further_from_64_bits_than_the_walk(delta, dk, dv, floor, shift):
+    """Outputs and states, by their norm, for decays spread out, near their floor and near one, and for the strongest floor
+    that is taken (whose reciprocals over a run reach exp(60)).  Both are float32 throughout; 3 in 100 is what two
+    orders of the same sums differ by over these sizes."""
+    from macllm_infer_amd.kernels import ops, build
+    build.ensure_modules(["linear_state", "linear_matrix"])
+    H, T = 4, 300
+    generator = torch.Generator().manual_seed(int(10 * floor) + dk)
+    u = (torch.randn(T, 3 * H * dk + H * dv, generator=generator) * 0.7).to(torch.bfloat16)
+    state = torch.randn(1, H, dv, dk, generator=generator) * 0.3
+    common = dict(q_col=0, k_col=H * dk, v_col=2 * H * dk, num_heads=H, key_dim=dk, value_dim=dv, slot_ids=torch.zeros(1, dtype=torch.int32))
+    if delta:
+        common.update(removal_col=2 * H * dk + H * dv, decay_logits=torch.randn(T, H * dk, generator=generator),
+                      decay_bias=torch.full((H * dk,), shift), decay_floor=floor, key_eps=2.0 ** -20)
+    else:
+        common.update(head_decay=1.0 - 2.0 ** -torch.arange(3.0, 3.0 + H), key_scale=0.125)
+    cu = torch.tensor([0, T], dtype=torch.int32)
+    wide = {name: value.double() if isinstance(value, torch.Tensor) and value.is_floating_point() else value for name, value in common.items()}
+    want, want_state = torch.zeros(T, H * dv, dtype=torch.float64), state.double()
+    before = ref_ops._f
+    ref_ops._f = lambda value: value.double()
+    try:
+        ref_ops.linear_state_scan(u, **wide, state=want_state, cu_seqlens=cu, out=want)
+    finally:
+        ref_ops._f = before
+    on = {name: value.to(DEV) if isinstance(value, torch.Tensor) else value for name, value in common.items()}
+    off = {}
+    for name in ("walk", "matrix"):
+        out, now = torch.zeros(T, H * dv, device=DEV), state.clone().to(DEV)
+        if name == "walk":
+            ops.linear_state_scan(u.to(DEV), **on, state=now, out=out, cu_seqlens=cu.to(DEV), max_query_len=T)
+        else:
+            ops.linear_matrix_scan(u.to(DEV), **on, state=now, out=out, chunks=ops.SsdChunks([T], 128, DEV))
+        off[name] = [float((got.cpu().double() - true).norm() / true.norm()) for got, true in ((out, want), (now, want_state))]
+    assert off["matrix"][0] <= 1.03 * off["walk"][0] and off["matrix"][1] <= 1.03 * off["walk"][1], off
+
+
 @pytest.mark.parametrize("delta, dk, dv", [(False, 64, 64), (False, 128, 32), (True, 64, 64)])
 @pytest.mark.parametrize("bad", [math.nan, math.inf])
 @pytest.mark.parametrize("part", ["v", "k", "r", "removal", "decay"])
