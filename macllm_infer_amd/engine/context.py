@@ -16,7 +16,7 @@ from __future__ import annotations
 
 from dataclasses import dataclass, field
 from itertools import chain
-from typing import Callable, Hashable, List, Optional, Sequence
+from typing import Callable, Hashable, List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -58,6 +58,9 @@ class StepContext:
     lane_starts: Optional[List[int]] = field(default_factory=list)
     max_query_len: int = 0           # the longest lane (its upper bound in a step of fixed capacity)
     max_seq_len: int = 0             # an upper bound of the longest context in the batch
+    # (lanes, tokens, longest context) that a choice between kernels of different rounding goes by: those of the
+    # captured graph of the step's capacity, also where the step is launched kernel by kernel
+    sizes: Tuple[int, int, int] = (0, 0, 0)
     derived: dict = field(default_factory=dict)   # tables parts derive from the step, shared by the layers
     chunk_tables: dict = field(default_factory=dict)   # chunk size -> ChunkTable, for the sizes the model's mixers name
     tables: dict = field(default_factory=dict)         # name -> int32 tensor, for the tables the model's mixers declare
@@ -88,6 +91,11 @@ def lower_lanes(lanes: Sequence[Lane], cache) -> LoweredLanes:
     if wants.size and (wants.min() < -(1 << 31) or wants.max() >= (1 << 31)):
         raise OverflowError("a wanted place does not fit 32 bits")
     return LoweredLanes(slots, lengths, tokens.astype(np.int32), want_counts, wants.astype(np.int32))
+
+
+def longest_context(lowered: LoweredLanes, cache) -> int:
+    """Tokens of the longest request behind a step of these lanes."""
+    return int((cache.lengths_of(lowered.slots) + lowered.lengths).max())
 
 
 def apply_feeds(token_ids: torch.Tensor, feeds) -> None:
@@ -219,7 +227,7 @@ def _pack(lowered: LoweredLanes, cache, out: Optional[np.ndarray], pad_lengths: 
 
 
 def _assemble(views, group_shapes, lengths, starts, max_seq_len, chunk_sizes=(), num_tokens=None, num_lanes=None,
-              max_query_len=None, query_tile: int = 0, tables: Sequence[StepTable] = ()) -> StepContext:
+              max_query_len=None, query_tile: int = 0, tables: Sequence[StepTable] = (), sizes=None) -> StepContext:
     """``lengths`` / ``starts``: the lanes' host copies, or None for a step of fixed capacity, whose lanes
     differ from fill to fill (``num_tokens``, ``num_lanes`` and ``max_query_len`` are then its capacities)."""
     tokens = sum(lengths) if lengths is not None else num_tokens
@@ -230,7 +238,8 @@ def _assemble(views, group_shapes, lengths, starts, max_seq_len, chunk_sizes=(),
         want_rows=views[7], query_tiles=views[8].view(-1, 2), query_tile=int(query_tile or 0),
         lane_lengths=list(lengths) if lengths is not None else None,
         lane_starts=list(starts) if starts is not None else None,
-        max_query_len=max(lengths) if lengths is not None else max_query_len, max_seq_len=max_seq_len)
+        max_query_len=max(lengths) if lengths is not None else max_query_len, max_seq_len=max_seq_len,
+        sizes=sizes or (lanes, tokens, max_seq_len))
     groups = len(group_shapes)
     for index, shape in enumerate(group_shapes):
         context.slot_mappings.append(views[9 + 2 * index])
@@ -254,10 +263,10 @@ def _split(buffer: torch.Tensor, sizes):
 
 def build_step_context(lanes: Sequence[Lane], cache, device, lowered: Optional[LoweredLanes] = None,
                        query_tile: int = 0, chunk_sizes: Sequence[int] = (),
-                       tables: Sequence[StepTable] = ()) -> StepContext:
+                       tables: Sequence[StepTable] = (), sizes: Optional[Tuple[int, int, int]] = None) -> StepContext:
     """``cache``: the CacheManager, after the step's pages were reserved.  ``query_tile``, ``chunk_sizes``:
     see ``_pack``; ``tables``: the tables the model's mixers declare (``DecoderModel.step_layout`` holds all
-    three for a whole model)."""
+    three for a whole model).  ``sizes``: see ``StepContext``; by default the step's own."""
     if lowered is None:
         lowered = lower_lanes(lanes, cache)
     needed, _, _, _, _ = _pack(lowered, cache, None, query_tile=query_tile, chunk_sizes=chunk_sizes)
@@ -265,12 +274,12 @@ def build_step_context(lanes: Sequence[Lane], cache, device, lowered: Optional[L
     host = torch.empty(-needed + sum(table_sizes), dtype=torch.int32)
     if torch.device(device).type == "cuda":
         host = host.pin_memory()
-    _, sizes, shapes, longest, _ = _pack(lowered, cache, host.numpy(), query_tile=query_tile, chunk_sizes=chunk_sizes)
-    _fill_tables(tables, host.numpy(), sizes, table_sizes, cache)
+    _, sections, shapes, longest, _ = _pack(lowered, cache, host.numpy(), query_tile=query_tile, chunk_sizes=chunk_sizes)
+    _fill_tables(tables, host.numpy(), sections, table_sizes, cache)
     packed = host.to(device, non_blocking=True)
     starts = cache.lengths_of(lowered.slots).tolist()
-    context = _assemble(_split(packed, sizes + table_sizes), shapes, lowered.lengths.tolist(), starts, longest,
-                        chunk_sizes, query_tile=query_tile, tables=tables)
+    context = _assemble(_split(packed, sections + table_sizes), shapes, lowered.lengths.tolist(), starts, longest,
+                        chunk_sizes, query_tile=query_tile, tables=tables, sizes=sizes)
     context._keepalive = host
     return context
 

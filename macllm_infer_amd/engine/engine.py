@@ -28,7 +28,8 @@ from ..kernels import build as kernel_build
 from ..kernels import ops
 from ..parts.base import BuildContext
 from ..weights.loader import WeightSource, bind
-from .context import Lane, LoweredLanes, apply_feeds, build_step_context, lower_lanes
+from .context import Lane, LoweredLanes, apply_feeds, build_step_context, longest_context, lower_lanes
+from .graphs import DecodeGraphs
 from .model import DecoderModel
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "fp32": torch.float32,
@@ -147,13 +148,12 @@ class Engine:
         self._beside = None                          # and the stream they are replayed on
         self._in_halves: Optional[bool] = None
         self.halves_share: Optional[float] = None
+        # the pool bounds a request's length only where some layer keeps every key: a model whose attention
+        # layers all have windows or chunks (or that has none) gives passed pages back, and a request outgrows the pool
+        bound = any(group.need.keeps_every_key for group in self.cache.groups)
+        self._longest_captured = min(self.max_context, capacity) if bound else self.max_context
         if decode_graphs and check_device and self.model.graph_safe:
-            from .graphs import DecodeGraphs
-            # the pool bounds a request's length only where some layer keeps every key: a model whose attention
-            # layers all have windows or chunks (or that has none) gives passed pages back, and a request outgrows the pool
-            bound = any(group.need.keeps_every_key for group in self.cache.groups)
-            self.graphs = DecodeGraphs(self.model, self.cache, self.device,
-                                       min(self.max_context, capacity) if bound else self.max_context)
+            self.graphs = DecodeGraphs(self.model, self.cache, self.device, self._longest_captured)
 
     @property
     def split_from_lanes(self) -> int:
@@ -208,7 +208,6 @@ class Engine:
                 whole.append((lanes, tokens))
         done = self.graphs.warm_up(whole + [(first, first) for first, _ in halves], context)
         if halves:
-            from .graphs import DecodeGraphs
             if self.graphs_beside is None:
                 self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len)
                 self._beside = torch.cuda.Stream(device=self.device)
@@ -332,7 +331,9 @@ class Engine:
             else:
                 logits = graphs.run_bucket(lanes, lowered)            # prompt portions: a graph of their capacity
         if logits is None:
-            context = build_step_context(lanes, self.cache, self.device, lowered, **self.model.step_layout)
+            sizes = DecodeGraphs.step_sizes(len(lanes), int(lowered.lengths.sum()), longest_context(lowered, self.cache),
+                                            self._longest_captured)
+            context = build_step_context(lanes, self.cache, self.device, lowered, sizes=sizes, **self.model.step_layout)
             apply_feeds(context.token_ids, lowered.feeds)
             logits = self.model.forward(context, self.cache)
         return logits
@@ -345,7 +346,6 @@ class Engine:
         contents nobody reads; their graphs have memory pools of their own."""
         main = torch.cuda.current_stream(self.device)
         if self.graphs_beside is None:
-            from .graphs import DecodeGraphs
             self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len)
             self._beside = torch.cuda.Stream(device=self.device)
         half = (len(lanes) + 1) // 2

@@ -27,7 +27,7 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
 
-from .context import Lane, LoweredLanes, StaticStep, apply_feeds
+from .context import Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
 
 
 def bucket_for(lanes: int) -> int:
@@ -38,6 +38,14 @@ def bucket_for(lanes: int) -> int:
 
 
 CONTEXT_BUCKET_FROM = 2048
+
+
+def context_bucket(longest: int, most: int) -> int:
+    """The smallest bucket of context length that holds ``longest`` tokens, at most ``most``."""
+    bucket = CONTEXT_BUCKET_FROM
+    while bucket < longest:
+        bucket <<= 1
+    return min(bucket, most)
 
 
 def token_capacities(most: int) -> List[int]:
@@ -77,23 +85,32 @@ class DecodeGraphs:
 
     def context_bucket(self, lowered: LoweredLanes, at_least: int = 0) -> int:
         """The smallest bucket of context length that holds every lane of the step after it ran."""
-        longest = max(int((self.cache.lengths_of(lowered.slots) + lowered.lengths).max()), at_least)
-        bucket = CONTEXT_BUCKET_FROM
-        while bucket < longest:
-            bucket <<= 1
-        return min(bucket, self.max_seq_len)
+        return context_bucket(max(longest_context(lowered, self.cache), at_least), self.max_seq_len)
 
-    def capacity_for(self, lanes: int, tokens: int, wants: int) -> Optional[Tuple[int, int, int]]:
+    @classmethod
+    def capacity_for(cls, lanes: int, tokens: int, wants: int) -> Optional[Tuple[int, int, int]]:
         """(lanes, tokens, wanted rows) of the smallest capacity that holds such a step, or None."""
-        if tokens > self.BUCKET_MOST_TOKENS:
+        if tokens > cls.BUCKET_MOST_TOKENS:
             return None
         lane_cap = bucket_for(lanes)
         for _ in range(2):                                   # the lanes' own bucket, or the next one (room for padding lanes)
-            for token_cap in token_capacities(self.BUCKET_MOST_TOKENS):
+            for token_cap in token_capacities(cls.BUCKET_MOST_TOKENS):
                 if token_cap >= tokens and StaticStep.fits(lane_cap, token_cap, lanes, tokens):
                     return lane_cap, token_cap, lane_cap if wants <= lane_cap else token_cap
             lane_cap <<= 1
         return None
+
+    @classmethod
+    def step_sizes(cls, lanes: int, tokens: int, longest: int, max_seq_len: int) -> Tuple[int, int, int]:
+        """(lanes, tokens, longest context) of the captured graph that a step with prompt portions replays, or would
+        replay once it is captured; the step's own where no graph holds it.  Kernels whose results differ in their
+        last bits are picked by these, so that a step gives the same numbers launched and replayed."""
+        capacity = cls.capacity_for(lanes, tokens, lanes)
+        if capacity is not None:
+            context = context_bucket(max(longest, capacity[1]), max_seq_len)
+            if context >= capacity[1]:
+                return capacity[0], capacity[1], context
+        return lanes, tokens, longest
 
     def token_target(self, lanes: int, tokens: int) -> int:
         """For a scheduler that is free to cut a prompt portion shorter: the largest number of tokens, at most

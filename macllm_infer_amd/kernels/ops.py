@@ -1556,10 +1556,10 @@ SHARED_PREFILL_WORKGROUPS = 128           # half of the chip's compute units
 COMPUTE_UNITS = 256
 
 
-def shared_prefill_heads(tiles: int, num_heads: int, num_kv_heads: int, head_dim: int, max_seq_len: int,
-                         span: int) -> int:
+def shared_prefill_heads(tiles: int, num_heads: int, num_kv_heads: int, head_dim: int, longest: int, span: int) -> int:
     """How many query heads a workgroup of the prompt attention with shared keys takes, 0: the kernel whose waves
-    read their keys themselves is the faster one.
+    read their keys themselves is the faster one.  ``tiles``: of 64 tokens; ``longest``: the bound of the step's contexts
+    that a captured step has, 2,048 at the least, so that only a window or chunk makes a walk short.
 
     The other kernel splits a tile's keys eight ways instead of two and, of heads of 64, shares a key fragment among up
     to four heads: it is the faster one where a few heavy tiles bound the launch.  Heads of 64 (us, other | this one): 8
@@ -1573,9 +1573,9 @@ def shared_prefill_heads(tiles: int, num_heads: int, num_kv_heads: int, head_dim
     heads_per_kv = num_heads // num_kv_heads
     workgroups = tiles * num_heads
     if head_dim == 64:
-        longest = min(max_seq_len, abs(span) + 64) if span else max_seq_len
+        walk = min(longest, abs(span) + 64) if span else longest
         short, long = SHARED_PREFILL_KEYS
-        fits = (0 < longest <= short or (0 < longest <= long and workgroups >= SHARED_PREFILL_WORKGROUPS)
+        fits = ((span and 0 < walk <= short) or (0 < walk <= long and workgroups >= SHARED_PREFILL_WORKGROUPS)
                 or (heads_per_kv == 1 and workgroups >= COMPUTE_UNITS))
         return 1 if fits else 0
     if workgroups < SHARED_PREFILL_WORKGROUPS:
@@ -1589,12 +1589,14 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
                       out: torch.Tensor, max_seq_len: int = 0, log_bias: Optional[torch.Tensor] = None,
                       sinks: Optional[torch.Tensor] = None, keep_first: int = 0, chunk: Optional[int] = None,
                       slopes: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
-                      value_dim: Optional[int] = None) -> None:
+                      value_dim: Optional[int] = None, sizes: Optional[tuple] = None) -> None:
     """``paged_attention`` on the matrix cores for bfloat16 (flash-style, online softmax in
     float32).  ``query_tiles`` [tiles, 2]: (lane, first token row) of runs of up to 64 tokens of
     one lane; the keys and values of the step's own tokens must be in the cache already.
     ``max_seq_len``: an upper bound of the step's longest context if known (it picks how many heads share
-    a key fragment, never the result).  ``keep_first`` (with a window): keys at positions below it stay visible.
+    a key fragment, never the result).  ``sizes`` (lanes, tokens, longest context; by default those of the arguments)
+    pick between the kernel whose waves share their keys and the one whose waves read them alone, which round
+    differently: a caller whose steps run launched and replayed gives both the same (``StepContext.sizes``).  ``keep_first`` (with a window): keys at positions below it stay visible.
     ``chunk``, ``slopes``, ``gate``, ``value_dim``: as for ``paged_attention``.  Heads of 64 or 128 with values as wide
     take the kernel of their width; any other width up to 128 the one that pads to the next of its own."""
     _need(keep_first >= 0 and (keep_first == 0 or window), "prefill_attention: first keys are kept behind a window")
@@ -1630,8 +1632,8 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     if (own_width and slopes is None and gate is None and keep_first == 0
             and page_size >= 8 and page_size & (page_size - 1) == 0 and page_stride % 8 == 0
             and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and out_ld % 4 == 0):
-        heads = shared_prefill_heads(query_tiles.shape[0], num_heads, num_kv_heads, head_dim, int(max_seq_len or 0),
-                                     span_code)
+        _, tokens, longest = sizes or (start_pos.numel(), T, int(max_seq_len or 0))
+        heads = shared_prefill_heads(-(-tokens // 64), num_heads, num_kv_heads, head_dim, longest, span_code)
         if heads:
             _check(_fn("attention_shared", "mi_prefill_attention_shared")(
                 _p(q), q_ld, num_heads, num_kv_heads, head_dim, _p(k_cache), _p(v_cache), page_stride, page_size,

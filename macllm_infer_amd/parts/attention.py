@@ -222,7 +222,7 @@ class Attention(Mixer):
                 ops.prefill_attention(qkv, *geometry, cache.k_cache, cache.v_cache, step.block_tables[cache.group],
                                       step.query_tiles, step.cu_seqlens, step.start_pos, spec.scale, spec.window,
                                       attended, step.max_seq_len, log_bias=self.position.score_log_bias,
-                                      sinks=self.sink)
+                                      sinks=self.sink, sizes=step.sizes)
                 return
             ops.paged_attention(qkv, *geometry, cache.k_cache, cache.v_cache, step.block_tables[cache.group],
                                 step.lane_of_token, step.positions, spec.scale, spec.window, attended,
@@ -246,7 +246,7 @@ class Attention(Mixer):
         elif ops.prefill_attention_supported(qkv.dtype, *geometry, cache.k_cache.shape[2]):
             ops.prefill_attention(qkv, *geometry, cache.k_cache, cache.v_cache, step.block_tables[cache.group],
                                   step.query_tiles, step.cu_seqlens, step.start_pos, spec.scale, spec.window,
-                                  attended, step.max_seq_len)
+                                  attended, step.max_seq_len, sizes=step.sizes)
         else:
             ops.paged_attention(qkv, *geometry, cache.k_cache, cache.v_cache, step.block_tables[cache.group],
                                 step.lane_of_token, step.positions, spec.scale, spec.window, attended,
@@ -325,7 +325,7 @@ class Attention(Mixer):
                                  value_dim=spec.value_width, head_scales=self.head_scales, score_bias=self.score_bias,
                                  sigmoid=sigmoid, **terms)
         elif portions and plain and gate_fits and own_width:
-            ops.prefill_attention(*prompt, **terms)
+            ops.prefill_attention(*prompt, sizes=step.sizes, **terms)
         elif (portions and all(value is None or isinstance(value, int) and value == 0 for value in terms.values())
                 and ops.prefill_attention_forms_supported(qkv.dtype, *geometry, spec.value_width, page, sigmoid,
                                                           self.head_scales is not None)):

@@ -277,6 +277,7 @@ def test_a_step_of_fixed_capacity_holds_any_lanes_that_fit_it(seed):
     ends_at = static.context.tables["ends"].data_ptr()
     assert static.context.lane_lengths is None and static.context.num_tokens == token_cap
     assert static.context.num_lanes == lane_cap and static.context.max_query_len == token_cap
+    assert static.context.sizes == (lane_cap, token_cap, 512)
     addresses = [static.context.token_ids.data_ptr(), static.context.query_tiles.data_ptr(),
                  static.context.chunk_tables[8].chunks.data_ptr(), static.context.block_tables[0].data_ptr()]
     names = ["a", "b", "c", "d", "e"]
@@ -383,3 +384,32 @@ def test_the_cores_packing_of_a_step_matches_a_plain_packing(seed, decode_only):
         compare(static.context, dict(plain_packing(cache, lanes, [1] * (4 - len(lanes)), static.max_pages),
                                      want_rows=[0, 1, 2, 3]))
     cache.check()
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_a_launched_step_is_sized_like_the_graph_of_its_capacity(seed):
+    """What a choice between kernels goes by (``StepContext.sizes``): of a step that is launched, the lanes, tokens and
+    context of the captured step that would hold it; the step's own where none does."""
+    from macllm_infer_amd.engine.context import Lane, StaticStep, build_step_context, longest_context, lower_lanes
+    from macllm_infer_amd.engine.graphs import DecodeGraphs
+    rng = random.Random(40 + seed)
+    cache = make(capacity=9000, page=16, requests=6)
+    most = 8192
+    for name in "abcd":
+        cache.add_request(name)
+    for _ in range(10):
+        lanes = [Lane(name, [1] * rng.choice([1, 1, 7, 37, 300, 515, 1000]), [0]) for name in rng.sample("abcd", rng.randrange(1, 5))]
+        lowered = lower_lanes(lanes, cache)
+        tokens = int(lowered.lengths.sum())
+        sizes = DecodeGraphs.step_sizes(len(lanes), tokens, longest_context(lowered, cache), most)
+        cache.reserve_slots(lowered.slots, lowered.lengths)
+        launched = build_step_context(lanes, cache, "cpu", lowered, query_tile=64, sizes=sizes)
+        lane_cap, token_cap, wants = DecodeGraphs.capacity_for(len(lanes), tokens, len(lanes))
+        context = 2048
+        while context < max(longest_context(lowered, cache), token_cap):
+            context *= 2
+        static = StaticStep(cache, lane_cap, context, "cpu", query_tile=64, tokens=token_cap, wants=wants)
+        assert launched.sizes == static.context.sizes == (lane_cap, token_cap, context)
+        assert build_step_context(lanes, cache, "cpu", lowered).sizes == (len(lanes), tokens, longest_context(lowered, cache))
+    assert DecodeGraphs.step_sizes(2, 20000, 30000, 65536) == (2, 20000, 30000)      # more tokens than graphs are made for
+    assert DecodeGraphs.step_sizes(1, 100, 100, 64) == (1, 100, 100)                 # more than the cache's graphs can hold

@@ -1477,6 +1477,44 @@ def test_configurations_drawn_at_random_match_the_plain_model(seed, odd, dtype):
     engine.cache.check()
 
 
+@pytest.mark.parametrize("shape, vocab", [("0.5b", 1003), ("7b", 1003)])
+def test_a_prompt_takes_the_same_attention_kernel_launched_and_replayed(monkeypatch, shape, vocab):
+    """A portion of any length, alone or beside decoded tokens, is launched the first time its capacity is met and
+    captured and replayed from then on: the rule that picks the attention kernel says the same both times."""
+    import bench
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.kernels import ops
+    from macllm_infer_amd.weights.random_init import random_tensors
+    config = FalconH1Config.from_dict(dict(bench.SHAPES[shape], num_hidden_layers=1, vocab_size=vocab))
+    engine = Engine(config=config, tensors=random_tensors(config, 7, torch.bfloat16, "unit"), dtype="bfloat16",
+                    kv_cache_capacity_tokens=12288, max_active_sequences=8)
+    picked, rule = [], ops.shared_prefill_heads
+
+    def spy(*sizes):
+        picked.append(rule(*sizes))
+        return picked[-1]
+    monkeypatch.setattr(ops, "shared_prefill_heads", spy)
+    for name in ("a", "b", "c"):
+        engine.add_request(name)
+        engine.step([Lane(name, tokens_for(vocab, 70, 9))])
+    for length, beside in ((37, 0), (100, 0), (200, 0), (300, 0), (515, 0), (576, 0), (777, 0), (1300, 0), (2048, 0), (2500, 0),
+                           (100, 2), (515, 3), (1000, 1)):
+        seen = []
+        before = dict(engine.graphs.counts)
+        for _ in range(3):
+            picked.clear()
+            engine.add_request("prompt")
+            engine.step([Lane("prompt", tokens_for(vocab, length, 3), [length - 1])]
+                        + [Lane(name, [5], [0]) for name in ("a", "b", "c")[:beside]])
+            engine.finish("prompt")
+            seen.append(list(picked))
+        after = engine.graphs.counts
+        if after["bucket_eager"] > before["bucket_eager"]:        # (else a graph of this capacity was there)
+            assert seen[0] and seen[1] and set(seen[0]) == set(seen[1]), (length, beside, seen)
+        assert not seen[2]
+
+
 @pytest.mark.parametrize("shape, layers, vocab", [("0.5b", 2, None), ("7b", 1, 1003)])
 def test_layers_of_the_benchmark_shapes_match_the_plain_model(shape, layers, vocab):
     """Layers with the sizes bench.py measures (0.5B shape: width 1024, 8 query heads on 2, 24
