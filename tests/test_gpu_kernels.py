@@ -1613,16 +1613,34 @@ def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_
 
 
 def test_rule_of_the_prompt_attention(ops):
-    """Heads of 64: short windows, longer walks on half the chip, any where every head has its own keys and the chip is
-    full.  Heads of 128: grids of half the chip on, two heads a workgroup once every compute unit has one."""
+    """Heads of 64: short windows, longer walks in full tiles on half the chip.  One head a kv head: half the chip.  Heads of
+    128: full tiles on half the chip, two heads a workgroup once every compute unit has one."""
     rule = ops.shared_prefill_heads
-    assert rule(1, 8, 2, 64, 2048, 512) == 1 and rule(9, 8, 2, 64, 577, 0) == 0 and rule(1, 8, 2, 64, 0, 0) == 0
-    assert rule(1, 8, 2, 64, 300, 0) == 0            # (no captured step has so short a bound: replays would differ)
-    assert rule(16, 8, 2, 64, 2048, 0) == 1 and rule(15, 8, 2, 64, 2048, 0) == 0 and rule(64, 8, 2, 64, 2049, 0) == 0
-    assert rule(15, 8, 2, 64, 9000, 512) == 1 and rule(15, 8, 2, 64, 9000, -513) == 0
-    assert rule(16, 16, 16, 64, 9000, 0) == 1 and rule(15, 16, 16, 64, 9000, 0) == 0
-    assert rule(10, 12, 2, 128, 9000, 0) == 0 and rule(11, 12, 2, 128, 9000, 0) == 1 and rule(22, 12, 2, 128, 9000, 0) == 2
-    assert rule(300, 8, 8, 128, 0, 0) == 1
+    assert rule(64, 1, 8, 2, 64, 2048, 512) == 1 and rule(64, 1, 8, 2, 64, 9000, -512) == 1      # a window, a chunk of 512 keys
+    assert rule(64, 1, 8, 2, 64, 2048, 513) == 0 and rule(300, 1, 8, 2, 64, 300, 0) == 0
+    assert rule(1536, 1, 8, 2, 64, 2048, 0) == 1 and rule(1024, 1, 8, 2, 64, 2048, 0) == 0
+    assert rule(2048, 1, 8, 2, 64, 2049, 0) == 0 and rule(2048, 1, 8, 2, 64, 0, 0) == 0
+    assert rule(2048, 2, 8, 2, 64, 4096, 1024) == 1 and rule(2048, 2, 6, 2, 64, 4096, 1024) == 0
+    assert rule(640, 2, 16, 16, 64, 9000, 0) == 1 and rule(320, 2, 16, 16, 64, 9000, 0) == 0
+    assert rule(1024, 1, 8, 8, 128, 0, 0) == 1 and rule(1024, 4, 8, 8, 128, 0, 0) == 0
+    assert rule(640, 2, 12, 2, 128, 2048, 0) == 0 and rule(1024, 1, 12, 2, 128, 9000, 0) == 1 and rule(2048, 1, 12, 2, 128, 9000, 0) == 2
+    assert rule(777, 1, 12, 2, 128, 2048, 0) == 1 and rule(777, 1, 12, 2, 128, 4096, 0) == 0
+
+
+def test_rule_of_the_prompt_attention_knows_tiles_of_a_few_tokens(ops):
+    """Steps of many short lanes, and of single tokens beside a portion: their tiles hold a few tokens each and are no
+    reason for the kernel that works on whole tiles, unless there are more of them than fill the chip."""
+    rule = ops.shared_prefill_heads
+    for lanes, tokens in ((16, 16), (16, 128), (32, 32), (32, 512), (16, 576), (32, 1664)):
+        assert rule(tokens, lanes, 8, 2, 64, 2048, 0) == 0, (lanes, tokens)
+    assert rule(64, 64, 8, 2, 64, 2048, 0) == 1 and rule(64, 64, 8, 2, 64, 4096, 0) == 0
+    assert rule(2048, 32, 8, 2, 64, 2048, 0) == 1            # 32 lanes that may all be a tile long
+    for lanes, tokens in ((16, 16), (16, 256), (32, 32), (64, 1024)):
+        assert rule(tokens, lanes, 12, 2, 128, 4096, 0) == 0, (lanes, tokens)
+    assert rule(16, 16, 12, 2, 128, 2048, 0) == 0 and rule(32, 32, 12, 2, 128, 2048, 0) == 2
+    assert rule(1024, 16, 12, 2, 128, 4096, 0) == 1
+    assert rule(16, 16, 32, 8, 128, 4096, 0) == 0 and rule(16, 16, 32, 8, 128, 2048, 0) == 2
+    assert rule(32, 32, 8, 8, 128, 9000, 0) == 1 and rule(16, 16, 8, 8, 128, 9000, 0) == 0
 
 
 def test_prefill_attention_finds_far_keys_and_edges(ops):
