@@ -349,7 +349,8 @@ extern "C" int mi_prefill_attention_shared(const void* q, long q_ld, int Hq, int
   const int G = Hq / Hkv;
   if ((dh != 64 && dh != 128) || page_size < 8 || (page_size & (page_size - 1)) != 0 || page_stride % 8 != 0 ||
       (uintptr_t)k_base % 16 != 0 || (uintptr_t)v_base % 16 != 0 || q_ld % 8 != 0 || (uintptr_t)q % 16 != 0 ||
-      out_ld % 4 != 0 || (uintptr_t)out % 8 != 0 || Hkv > 65535 || G > 64 || n_tiles > (1 << 28))
+      out_ld % 4 != 0 || (uintptr_t)out % 8 != 0 || Hkv > 65535 || G > 64 || n_tiles > (1 << 28) ||
+      2L * Hkv * dh * page_size > (1L << 32))      // (offsets into a page are 32 bits)
     return ERR_UNSUPPORTED_SIZE;
   if (nset != 1 && (nset != 2 || dh != 128)) return ERR_BAD_ARGUMENT;
   int page_shift = 0;

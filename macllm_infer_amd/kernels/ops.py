@@ -1604,6 +1604,13 @@ def shared_prefill_heads(tokens: int, lanes: int, num_heads: int, num_kv_heads: 
     return 2 if -(-tokens // 64) * num_heads > 256 else 1           # compute units
 
 
+def shared_prefill_covers(num_kv_heads: int, head_dim: int, page_size: int, page_stride: int, k_address: int, v_address: int) -> bool:
+    """Whether the prompt attention with shared keys takes this cache: pages of a power of two of 8 tokens or more in whole
+    16-byte pieces, and a page's keys and values within the 32 bits of an offset into it."""
+    return (page_size >= 8 and page_size & (page_size - 1) == 0 and page_stride % 8 == 0
+            and k_address % 16 == 0 and v_address % 16 == 0 and 2 * num_kv_heads * head_dim * page_size <= 1 << 32)
+
+
 def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, k_cache: torch.Tensor,
                       v_cache: torch.Tensor, block_tables: torch.Tensor, query_tiles: torch.Tensor,
                       cu_seqlens: torch.Tensor, start_pos: torch.Tensor, scale: float, window: Optional[int],
@@ -1651,8 +1658,7 @@ def prefill_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     _need(gate is None or (gate_ld % 4 == 0 and gate.data_ptr() % 8 == 0), "prefill_attention: the gate's rows lie in pieces of four")
     own_width = head_dim in (64, 128) and value_dim == head_dim
     if (own_width and slopes is None and gate is None and keep_first == 0
-            and page_size >= 8 and page_size & (page_size - 1) == 0 and page_stride % 8 == 0
-            and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0 and out_ld % 4 == 0):
+            and shared_prefill_covers(num_kv_heads, head_dim, page_size, page_stride, k_cache.data_ptr(), v_cache.data_ptr())):
         lanes, tokens, longest = sizes or (start_pos.numel(), T, int(max_seq_len or 0))
         heads = shared_prefill_heads(tokens, lanes, num_heads, num_kv_heads, head_dim, longest, span_code)
         if heads:

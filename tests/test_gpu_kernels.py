@@ -1643,6 +1643,15 @@ def test_rule_of_the_prompt_attention_knows_tiles_of_a_few_tokens(ops):
     assert rule(32, 32, 8, 8, 128, 9000, 0) == 1 and rule(16, 16, 8, 8, 128, 9000, 0) == 0
 
 
+def test_pages_beyond_32_bits_stay_with_the_other_prompt_kernel(ops):
+    """The kernel with shared keys reaches into a page by 32-bit offsets: a page of 2^32 bytes of keys is its largest."""
+    covers = ops.shared_prefill_covers
+    assert covers(8, 128, 16, 4096, 0, 32) and covers(16, 128, 1 << 20, 8, 0, 0) and not covers(16, 128, 1 << 21, 8, 0, 0)
+    assert not covers(33, 64, 1 << 20, 8, 0, 0) and covers(32, 64, 1 << 20, 8, 0, 0)
+    assert not covers(2, 64, 24, 8, 0, 0) and not covers(2, 64, 4, 8, 0, 0) and not covers(2, 64, 16, 12, 0, 0)
+    assert not covers(2, 64, 16, 8, 8, 0) and not covers(2, 64, 16, 8, 0, 24)
+
+
 def test_prefill_attention_finds_far_keys_and_edges(ops):
     """Queries at the end of a 700-token prompt; one chosen key takes all the weight."""
     Hq, Hkv, dh, length, page_size = 4, 2, 64, 700, 16
