@@ -1033,9 +1033,10 @@ static bool ssd_staged_sizes(int P, int N) {
   return (P == 16 || P == 32 || P == 64 || P == 128) && (N == 32 || N == 64 || N == 128 || N == 256);
 }
 
-// Whether a step whose longest lane holds `longest` tokens (0: not known) is worked on in one launch behind the conv.
-extern "C" int mi_ssd_single(int Q, int P, int N, int longest) {
-  return longest > 0 && longest <= Q && longest <= SSD_SINGLE_TOKENS && ssd_staged_sizes(P, N) ? 1 : 0;
+// Whether a step whose longest lane holds `longest` tokens (0: not known) is worked on in one launch behind the conv: with
+// states that begin at whole 16-byte pieces, as that launch moves them.
+extern "C" int mi_ssd_single(int Q, int P, int N, int longest, const float* ssm_state) {
+  return (uintptr_t)ssm_state % 16 == 0 && longest > 0 && longest <= Q && longest <= SSD_SINGLE_TOKENS && ssd_staged_sizes(P, N) ? 1 : 0;
 }
 
 template <int NK, int PT>
@@ -1111,7 +1112,7 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
                                                            (const bf16_t*)xbc, xbc_ld, E + GN, Q, (bf16_t*)TT);
     RETURN_IF_LAUNCH_FAILED();
   }
-  if (mi_ssd_single(Q, P, N, longest)) {
+  if (mi_ssd_single(Q, P, N, longest, ssm_state)) {
     const int tail_rows = conv_here ? (C + SSD_SCAN_WAVES * WAVE - 1) / (SSD_SCAN_WAVES * WAVE) : 0;
     const SsdSingle one = {ssm_state, slot_ids, (const bf16_t*)u, u_ld, C, conv_k, (bf16_t*)conv_state, lane_chunks};
     int status = ERR_UNSUPPORTED_SIZE;

@@ -171,7 +171,7 @@ _SIGNATURES = {
                            _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_long,
                            _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
-        "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int],
+        "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int, _c_ptr],
     },
     "gemm": {
         "mi_gemm_f32": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr],
@@ -1961,7 +1961,7 @@ def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: t
     delta = torch.empty((2, T, H), dtype=torch.float32, device=device)
     transposed = torch.empty((chunks * (E + GN) * Q,), dtype=torch.bfloat16, device=device)
     chunk_state = state_in = decay = None
-    if not _fn("ssd", "mi_ssd_single")(Q, P, N, int(longest)):
+    if not _fn("ssd", "mi_ssd_single")(Q, P, N, int(longest), _p(ssm_state)):
         chunk_state = torch.empty((chunks * H * P * N + chunks * H,), dtype=torch.float32, device=device)
         state_in = torch.empty((chunks * H * P * N,), dtype=torch.bfloat16, device=device)
         decay = chunk_state[chunks * H * P * N:]

@@ -611,6 +611,30 @@ def test_lanes_of_one_chunk_scan_in_one_launch(ops, Q, H, P, N, G, gate):
 
 
 @pytest.mark.parametrize("P, N", [(16, 32), (64, 128)])
+def test_states_that_begin_within_a_piece_of_16_bytes_scan_in_three_launches(ops, P, N):
+    """Lanes of one chunk whose states do not begin at 16 bytes, as a view into a caller's pool may: the numbers of the
+    one launch, which moves whole pieces, from the launches that do not."""
+    H, G, Q = 3, 1, 128
+    E = H * P
+    counts = [5, 128, 33]
+    T, slots = sum(counts), len(counts) + 1
+    xbc, dt = rand(T, E + 2 * N, seed=490, dtype=torch.bfloat16).to(DEV), rand(T, H, seed=491, dtype=torch.bfloat16).to(DEV)
+    dt_bias, A, D = gpu(rand(H, seed=492) - 1.0, -torch.exp(torch.linspace(-3.0, 1.0, H)), rand(H, seed=493))
+    start, ids = rand(slots, H, P, N, seed=494, scale=0.5).to(DEV), i32([3, 0, 1]).to(DEV)
+    results = []
+    for offset in (0, 1, 2):
+        held = torch.zeros(start.numel() + 4, device=DEV)
+        state = held[offset:offset + start.numel()].view(start.shape)
+        state.copy_(start)
+        assert ops._fn("ssd", "mi_ssd_single")(Q, P, N, 128, state.data_ptr()) == (offset == 0)
+        y = torch.full((T, E), float("nan"), device=DEV)
+        ops.ssd_prefill(xbc, dt, dt_bias, A, D, state, ops.SsdChunks(counts, Q, DEV), ids, G, y, longest=128)
+        results.append((y, state))
+    for y, state in results:
+        assert bool(torch.isfinite(y).all()) and torch.equal(y, results[0][0]) and torch.equal(state, results[0][1])
+
+
+@pytest.mark.parametrize("P, N", [(16, 32), (64, 128)])
 def test_states_pass_through_chunks_in_pieces_and_one_by_one(ops, P, N):
     """The pass moves four neighbours a thread where the states lie at whole pieces and one where they do not: the same
     numbers, for lanes of one chunk, of a short round and beside it, and of more than a long one."""
