@@ -991,6 +991,7 @@ ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __r
     for (int i = 0; i < PB; ++i) sum[i] = s_floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < QK; ++ks) {
+      if (32 * ks >= Q) continue;              // (a chunk's own columns once more, whose infinities a weight of zero would not stop)
       s_bf16x8 a;
 #pragma unroll
       for (int j = 0; j < 8; ++j) a[j] = (bf16_t)((float)b_raw[ks][j] * weight[32 * ks + 8 * q + j]);

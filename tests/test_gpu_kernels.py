@@ -610,6 +610,28 @@ def test_lanes_of_one_chunk_scan_in_one_launch(ops, Q, H, P, N, G, gate):
     assert not torch.equal(results[1][1], state) and not torch.equal(results[1][2], tails)
 
 
+@pytest.mark.parametrize("Q", [32, 64, 128])
+def test_lanes_of_one_chunk_keep_infinities_as_the_three_launches_do(ops, Q):
+    """An infinite element of x in the last 32 tokens of a chunk: infinities in the states stay what they are, in a chunk of
+    any size (a shorter one than the launch's 128 tokens meets its last columns again, with weights of zero)."""
+    H, G, P, N = 2, 1, 32, 64
+    E = H * P
+    counts = [Q, Q - 3]
+    T = sum(counts)
+    xbc, dt = rand(T, E + 2 * N, seed=590, dtype=torch.bfloat16), rand(T, H, seed=591, dtype=torch.bfloat16).to(DEV)
+    xbc[Q - 8, 5] = math.inf
+    dt_bias, A, D = gpu(rand(H, seed=592) - 1.0, -torch.exp(torch.linspace(-3.0, 1.0, H)), rand(H, seed=593))
+    start, ids = rand(2, H, P, N, seed=594, scale=0.5).to(DEV), i32([1, 0]).to(DEV)
+    results = []
+    for known in (0, Q):
+        state, y = start.clone(), torch.zeros(T, E, device=DEV)
+        ops.ssd_prefill(xbc.to(DEV), dt, dt_bias, A, D, state, ops.SsdChunks(counts, Q, DEV), ids, G, y, longest=known)
+        results.append((y, state))
+    for three, one in zip(*results):
+        assert torch.equal(torch.isnan(one), torch.isnan(three)) and torch.equal(torch.nan_to_num(one), torch.nan_to_num(three))
+    assert bool(torch.isinf(results[0][1]).any())
+
+
 @pytest.mark.parametrize("P, N", [(16, 32), (64, 128)])
 def test_states_that_begin_within_a_piece_of_16_bytes_scan_in_three_launches(ops, P, N):
     """Lanes of one chunk whose states do not begin at 16 bytes, as a view into a caller's pool may: the numbers of the
