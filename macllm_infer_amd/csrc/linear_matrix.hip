@@ -59,7 +59,7 @@ struct LinearMatrixArgs {
   long logits_ld;
   const float* decay_bias;          // [H * dk]
   float decay_floor, key_eps;
-  float* local;                     // [chunks * runs a chunk, H, Ro | Nv | M]
+  float* local;                     // [runs (lm_first_run), H, Ro | Nv | M]
   float* out;                       // [T, out_ld]
   long out_ld;
 };
@@ -129,6 +129,11 @@ __device__ __forceinline__ lm_floatx4 lm_diagonal(const float* at, int stride, i
 template <int KIND, int DK, int N>
 static constexpr long lm_run_floats(int dv) { return (long)N * DK + (long)dv * DK + (KIND == LM_DELTA ? DK * DK : 0); }
 
+// Where the runs of a lane that begins at token row `row` lie in the work area: a lane of n tokens has ceil(n / N) runs, and
+// floor((row + n) / N) + lane + 1 is never before its last.  The area holds floor(tokens / N) + lanes of them.
+template <int N>
+__device__ __forceinline__ long lm_first_run(int lane, long row) { return row / N + lane; }
+
 template <int KIND, int DK, int N>
 static constexpr int lm_chunk_lds_floats() {
   constexpr int KS = DK + 4, TS = N + 4, T = N / 16;
@@ -171,7 +176,7 @@ __global__ void __launch_bounds__(LM_MOST_WAVES * WAVE) linear_matrix_chunk_kern
   const int dv = a.dv;
   const int value_tile = wave - (DELTA ? KT : 0);       // this wave's 16 value channels, if it has some
   const bool has_values = value_tile >= 0 && value_tile < dv / 16;
-  float* const run = a.local + ((long)blockIdx.x * a.H + head) * lm_run_floats<KIND, DK, N>(dv);
+  float* const run = a.local + ((lm_first_run<N>(row[0], row[1] - row[3] * LM_CHUNK_TOKENS) + row[3] * RUNS + part) * a.H + head) * lm_run_floats<KIND, DK, N>(dv);
   float* const Ro = run;                                // [N][DK]
   float* const Nv = Ro + N * DK;                        // [dv][DK], transposed as the state is
   float* const M = Nv + (long)dv * DK;                  // [DK][DK]
@@ -440,7 +445,6 @@ template <int KIND, int DK, int N, int AHEAD>
 __global__ void __launch_bounds__((KIND == LM_DELTA ? N / 16 + DK / 16 : 4) * WAVE) linear_matrix_carry_kernel(const LinearMatrixArgs a) {
   constexpr bool DELTA = KIND == LM_DELTA;
   constexpr int T = N / 16, KT = DK / 16, KS = DK + 4;
-  constexpr int RUNS = LM_CHUNK_TOKENS / N;
   constexpr int WAVES = DELTA ? T + KT : 4;
   constexpr int FOURS = DELTA ? 1 : 16 * DK / 4 / (WAVES * WAVE);      // retention: groups of four elements of a thread
   static_assert(DELTA || (T <= 4 && FOURS >= 1), "four waves hold the outputs' rows and the state");
@@ -462,7 +466,7 @@ __global__ void __launch_bounds__((KIND == LM_DELTA ? N / 16 + DK / 16 : 4) * WA
   const int dv = a.dv;
   const bool outputs = wave < T;
   const long run_floats = lm_run_floats<KIND, DK, N>(dv), run_stride = run_floats * a.H;
-  const float* const local = a.local + ((long)first * RUNS * a.H + head) * run_floats;
+  const float* const local = a.local + (lm_first_run<N>(lane_of_step, row0) * a.H + head) * run_floats;
   const float* const matrix = local + (outputs ? (long)(16 * wave + r) * DK
                                                : (long)N * DK + (long)dv * DK + (long)(16 * (wave - T) + r) * DK) + 4 * q;
   const float* const Nv = local + N * DK + (long)value0 * DK;
@@ -558,9 +562,10 @@ extern "C" int mi_linear_matrix_supported(int delta, int dk, int dv) {
 extern "C" int mi_linear_matrix_run(int delta) { return delta ? LM_DELTA_RUN : LM_RETENTION_RUN; }
 extern "C" int mi_linear_matrix_chunk_tokens(void) { return LM_CHUNK_TOKENS; }
 
-extern "C" long mi_linear_matrix_floats(int delta, int num_chunks, int H, int dk, int dv) {
+// of the work area for a step of so many tokens in so many lanes
+extern "C" long mi_linear_matrix_floats(int delta, int tokens, int lanes, int H, int dk, int dv) {
   const long run = mi_linear_matrix_run(delta);
-  return (long)num_chunks * (LM_CHUNK_TOKENS / run) * H * (run * dk + (long)dv * dk + (delta ? (long)dk * dk : 0));
+  return (tokens / run + lanes) * H * (run * dk + (long)dv * dk + (delta ? (long)dk * dk : 0));
 }
 
 template <int KIND, int DK, int N, int AHEAD>

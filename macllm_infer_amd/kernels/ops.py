@@ -106,7 +106,7 @@ _SIGNATURES = {
         "mi_linear_matrix_supported": [_c_int, _c_int, _c_int],
         "mi_linear_matrix_run": [_c_int],
         "mi_linear_matrix_chunk_tokens": [],
-        "mi_linear_matrix_floats": [_c_int, _c_int, _c_int, _c_int, _c_int],
+        "mi_linear_matrix_floats": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
         "mi_linear_matrix_scan": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr,
                                   _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_int,
                                   _c_ptr, _c_long, _c_ptr, _c_float, _c_float, _c_ptr, _c_ptr, _c_long, _c_ptr],
@@ -1229,9 +1229,10 @@ def linear_matrix_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, n
     _i32(chunks.lane_chunks, "lane_chunks")
     lanes, count = slot_ids.numel(), int(chunks.num_chunks)
     _need(chunks.chunk_size == _fn("linear_matrix", "mi_linear_matrix_chunk_tokens")() and count > 0
-          and chunks.chunks.numel() >= 4 * count and chunks.lane_chunks.numel() >= 2 * lanes,
+          and chunks.chunks.numel() >= 4 * count and chunks.lane_chunks.numel() >= 2 * lanes
+          and chunks.num_tokens == T and chunks.num_lanes == lanes,
           "linear_matrix_scan: the chunk table does not cover the step")
-    local = torch.empty((_fn("linear_matrix", "mi_linear_matrix_floats", _c_long)(int(delta), count, H, dk, dv),),
+    local = torch.empty((_fn("linear_matrix", "mi_linear_matrix_floats", _c_long)(int(delta), T, lanes, H, dk, dv),),
                         dtype=torch.float32, device=u.device)
     _check(_fn("linear_matrix", "mi_linear_matrix_scan")(
         _p(u), ld, int(q_col), int(k_col), int(v_col), int(removal_col), H, dk, dv, _p(state), _p(slot_ids), lanes,

@@ -260,6 +260,38 @@ def test_a_token_that_is_no_number_leaves_the_tokens_before_it_alone(delta, dk, 
         assert torch.equal(torch.isfinite(now), torch.isfinite(walked_state)), token
 
 
+@pytest.mark.parametrize("delta", [False, True])
+def test_work_area_of_the_runs_is_that_of_the_tokens(delta):
+    """Lanes of every length around a run and a chunk, most of them of one token: the area has room for the tokens' runs and
+    one run a lane, and none is shared: outputs and states are the walk's, whose lanes meet nowhere."""
+    import ctypes
+    from macllm_infer_amd.kernels import ops, build
+    build.ensure_modules(["linear_state", "linear_matrix"])
+    H, dk, dv, run = 2, 64, 32, 32 if delta else 64
+    lengths = [1] * 9 + [31, 1, 32, 33, 2, 63, 64, 65, 1, 127, 128, 129, 1, 1, 200, 5, 95, 1]
+    T, lanes = sum(lengths), len(lengths)
+    floats = ops._fn("linear_matrix", "mi_linear_matrix_floats", ctypes.c_long)(int(delta), T, lanes, H, dk, dv)
+    assert floats == (T // run + lanes) * H * dk * (run + dv + (dk if delta else 0))
+    generator = torch.Generator().manual_seed(5)
+    u = (torch.randn(T, 3 * H * dk + H * dv, generator=generator) * 0.7).to(torch.bfloat16).to(DEV)
+    state = (torch.randn(lanes, H, dv, dk, generator=generator) * 0.3).to(DEV)
+    common = dict(q_col=0, k_col=H * dk, v_col=2 * H * dk, num_heads=H, key_dim=dk, value_dim=dv,
+                  slot_ids=torch.arange(lanes, dtype=torch.int32, device=DEV))
+    if delta:
+        common.update(removal_col=2 * H * dk + H * dv, decay_logits=torch.randn(T, H * dk, generator=generator).to(DEV),
+                      decay_bias=torch.zeros(H * dk, device=DEV), decay_floor=math.exp(-0.5), key_eps=1e-6)
+    else:
+        common.update(head_decay=torch.tensor([0.97, 0.99], device=DEV), key_scale=dk ** -0.5)
+    walked, walked_state = torch.zeros(T, H * dv, device=DEV), state.clone()
+    cu = torch.tensor([0] + list(np.cumsum(lengths)), dtype=torch.int32, device=DEV)
+    ops.linear_state_scan(u, **common, state=walked_state, out=walked, cu_seqlens=cu, max_query_len=max(lengths))
+    out, now = torch.zeros(T, H * dv, device=DEV), state.clone()
+    ops.linear_matrix_scan(u, **common, state=now, out=out, chunks=ops.SsdChunks(lengths, 128, DEV))
+    # float32 rounding of sums of some 64 products, as in the test above
+    assert float((out - walked).abs().max()) <= 4e-6 * float(walked.abs().max())
+    assert float((now - walked_state).abs().max()) <= 4e-6 * float(walked_state.abs().max())
+
+
 def test_heads_the_matrix_cores_do_not_cover_stay_with_the_walk():
     from macllm_infer_amd.kernels import ops
     covered = lambda *sizes, dtype=torch.bfloat16, floor=None: ops.linear_matrix_supported(dtype, *sizes, floor)
