@@ -31,6 +31,7 @@
 // goes from end to end: 96 and 23, 63 and 21.
 #include "common.h"
 #include <cstdint>
+#include <type_traits>
 
 typedef float lm_floatx4 __attribute__((ext_vector_type(4)));
 typedef double lm_doublex4 __attribute__((ext_vector_type(4)));
@@ -478,73 +479,81 @@ __global__ void __launch_bounds__((KIND == LM_DELTA ? N / 16 + DK / 16 : 4) * WA
     decay_last = powf(a.head_decay[head], (float)(tokens - (runs - 1) * N));
   }
 
-  lm_floatx4 rows[AHEAD][KT], beside[AHEAD][FOURS], known[AHEAD];
-  auto ask = [&](int at, int j) {
-    const int run = min(j, runs - 1);
-    const float* from = matrix + run * run_stride;
+  // `in_flight` runs' operands are on their way (a run past the lane's last is asked for as that run again)
+  auto walk = [&](auto in_flight) {
+    constexpr int IN_FLIGHT = decltype(in_flight)::value;
+    lm_floatx4 rows[IN_FLIGHT][KT], beside[IN_FLIGHT][FOURS], known[IN_FLIGHT];
+    auto ask = [&](int at, int j) {
+      const int run = min(j, runs - 1);
+      const float* from = matrix + run * run_stride;
 #pragma unroll
-    for (int c = 0; c < KT; ++c) rows[at][c] = *reinterpret_cast<const lm_floatx4*>(from + 16 * c);
-    if (DELTA) {
+      for (int c = 0; c < KT; ++c) rows[at][c] = *reinterpret_cast<const lm_floatx4*>(from + 16 * c);
+      if (DELTA) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        beside[at][0][i] = Nv[run * run_stride + (4 * q + i) * DK + (outputs ? 0 : 16 * (wave - T) + r)];
-    } else {
+        for (int i = 0; i < 4; ++i)
+          beside[at][0][i] = Nv[run * run_stride + (4 * q + i) * DK + (outputs ? 0 : 16 * (wave - T) + r)];
+      } else {
 #pragma unroll
-      for (int g = 0; g < FOURS; ++g)
-        beside[at][g] = *reinterpret_cast<const lm_floatx4*>(Nv + run * run_stride + 4 * (tid + g * WAVES * WAVE));
+        for (int g = 0; g < FOURS; ++g)
+          beside[at][g] = *reinterpret_cast<const lm_floatx4*>(Nv + run * run_stride + 4 * (tid + g * WAVES * WAVE));
+      }
+      const long row = row0 + min(run * N + 16 * (outputs ? wave : 0) + r, tokens - 1);
+      known[at] = *reinterpret_cast<const lm_floatx4*>(a.out + row * a.out_ld + (long)head * dv + value0 + 4 * q);
+    };
+#pragma unroll
+    for (int j = 0; j < IN_FLIGHT; ++j) ask(j, j);
+    __syncthreads();
+    for (int j0 = 0; j0 < runs; j0 += IN_FLIGHT) {
+#pragma unroll
+      for (int at = 0; at < IN_FLIGHT; ++at) {
+        // (no way out of the turns of a round: behind one the compiler waits for every load in flight.  A turn past the
+        // last run repeats that run's products, stores nothing and hands the state on)
+        const int j = j0 + at;
+        const bool live = j < runs;
+        const float* const s_now = s_lds[j & 1];
+        float* const s_next = s_lds[(j + 1) & 1];
+        lm_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+        if (DELTA || outputs) {
+#pragma unroll
+          for (int c = 0; c < KT; c += 4) {               // a chain for every 16 channels, added in pairs
+            lm_floatx4 part[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) part[p] = lm_mfma(lm_rows(s_now + 16 * (c + p), KS, q, r), rows[at][c + p], lm_floatx4{0.f, 0.f, 0.f, 0.f});
+            sum += (part[0] + part[1]) + (part[2] + part[3]);
+          }
+        }
+        if (outputs) {                                    // value channels 4q + i of token r
+          const int t = j * N + 16 * wave + r;
+          if (t < tokens)
+            *reinterpret_cast<lm_floatx4*>(a.out + (row0 + t) * a.out_ld + (long)head * dv + value0 + 4 * q) = known[at] + sum;
+        } else if (DELTA) {                               // value channels 4q + i of key channel r
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int place = (4 * q + i) * KS + 16 * (wave - T) + r;
+            s_next[place] = live ? sum[i] + beside[at][0][i] : s_now[place];
+          }
+        }
+        if (!DELTA) {
+          const int own = min(N, tokens - j * N);
+          const float shrink = own == N ? decay_run : decay_last;
+#pragma unroll
+          for (int g = 0; g < FOURS; ++g) {
+            const int e = 4 * (tid + g * WAVES * WAVE);
+            const int place = (e / DK) * KS + e % DK;
+            const lm_floatx4 before = *reinterpret_cast<const lm_floatx4*>(s_now + place);
+            *reinterpret_cast<lm_floatx4*>(s_next + place) = live ? shrink * before + beside[at][g] : before;
+          }
+        }
+        ask(at, j + IN_FLIGHT);
+        __syncthreads();
+      }
     }
-    const long row = row0 + min(run * N + 16 * (outputs ? wave : 0) + r, tokens - 1);
-    known[at] = *reinterpret_cast<const lm_floatx4*>(a.out + row * a.out_ld + (long)head * dv + value0 + 4 * q);
+    return (runs + IN_FLIGHT - 1) / IN_FLIGHT * IN_FLIGHT;      // turns made
   };
-#pragma unroll
-  for (int j = 0; j < AHEAD; ++j) ask(j, j);
-  __syncthreads();
-  for (int j0 = 0; j0 < runs; j0 += AHEAD) {
-#pragma unroll
-    for (int at = 0; at < AHEAD; ++at) {
-      // (no way out of the turns of a round: behind one the compiler waits for every load in flight.  A turn past the
-      // last run repeats that run's products, stores nothing and hands the state on)
-      const int j = j0 + at;
-      const bool live = j < runs;
-      const float* const s_now = s_lds[j & 1];
-      float* const s_next = s_lds[(j + 1) & 1];
-      lm_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-      if (DELTA || outputs) {
-#pragma unroll
-        for (int c = 0; c < KT; c += 4) {               // a chain for every 16 channels, added in pairs
-          lm_floatx4 part[4];
-#pragma unroll
-          for (int p = 0; p < 4; ++p) part[p] = lm_mfma(lm_rows(s_now + 16 * (c + p), KS, q, r), rows[at][c + p], lm_floatx4{0.f, 0.f, 0.f, 0.f});
-          sum += (part[0] + part[1]) + (part[2] + part[3]);
-        }
-      }
-      if (outputs) {                                    // value channels 4q + i of token r
-        const int t = j * N + 16 * wave + r;
-        if (t < tokens)
-          *reinterpret_cast<lm_floatx4*>(a.out + (row0 + t) * a.out_ld + (long)head * dv + value0 + 4 * q) = known[at] + sum;
-      } else if (DELTA) {                               // value channels 4q + i of key channel r
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int place = (4 * q + i) * KS + 16 * (wave - T) + r;
-          s_next[place] = live ? sum[i] + beside[at][0][i] : s_now[place];
-        }
-      }
-      if (!DELTA) {
-        const int own = min(N, tokens - j * N);
-        const float shrink = own == N ? decay_run : decay_last;
-#pragma unroll
-        for (int g = 0; g < FOURS; ++g) {
-          const int e = 4 * (tid + g * WAVES * WAVE);
-          const int place = (e / DK) * KS + e % DK;
-          const lm_floatx4 before = *reinterpret_cast<const lm_floatx4*>(s_now + place);
-          *reinterpret_cast<lm_floatx4*>(s_next + place) = live ? shrink * before + beside[at][g] : before;
-        }
-      }
-      ask(at, j + AHEAD);
-      __syncthreads();
-    }
-  }
-  const float* const s_end = s_lds[((runs + AHEAD - 1) / AHEAD * AHEAD) & 1];
+  // a lane of one run or two, as single tokens beside a portion are, does not ask for their operands again and again
+  const int turns = runs == 1 ? walk(std::integral_constant<int, 1>()) : runs <= 2 ? walk(std::integral_constant<int, 2>())
+                                                                      : walk(std::integral_constant<int, AHEAD>());
+  const float* const s_end = s_lds[turns & 1];
   for (int e = tid; e < 16 * DK; e += WAVES * WAVE) state[e] = s_end[(e / DK) * KS + e % DK];
 }
 

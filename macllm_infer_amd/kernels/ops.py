@@ -1177,6 +1177,8 @@ def linear_state_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, nu
 
 # the delta rule's matrices hold the reciprocal of a run's decays: its logarithm stays this far within float32's range
 LINEAR_MATRIX_MOST_LOG = 60.0
+# the largest work area: 2,048 tokens of 64 heads of 128 channels take 604 MB, three times that of the walk's passes
+LINEAR_MATRIX_MOST_BYTES = 1 << 30
 
 
 def linear_matrix_supported(dtype, key_dim: int, value_dim: int, decay_floor: Optional[float] = None) -> bool:
@@ -1187,6 +1189,12 @@ def linear_matrix_supported(dtype, key_dim: int, value_dim: int, decay_floor: Op
         return False
     run = _fn("linear_matrix", "mi_linear_matrix_run")(int(delta))
     return not delta or 0.0 <= decay_floor * run <= LINEAR_MATRIX_MOST_LOG
+
+
+def linear_matrix_bytes(tokens: int, lanes: int, num_heads: int, key_dim: int, value_dim: int, delta: bool) -> int:
+    """The work area of ``linear_matrix_scan`` for a step of so many tokens in so many lanes."""
+    return 4 * _fn("linear_matrix", "mi_linear_matrix_floats", _c_long)(int(delta), int(tokens), int(lanes), int(num_heads),
+                                                                        int(key_dim), int(value_dim))
 
 
 def linear_matrix_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, num_heads: int, key_dim: int, value_dim: int,
@@ -1232,8 +1240,7 @@ def linear_matrix_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, n
           and chunks.chunks.numel() >= 4 * count and chunks.lane_chunks.numel() >= 2 * lanes
           and chunks.num_tokens == T and chunks.num_lanes == lanes,
           "linear_matrix_scan: the chunk table does not cover the step")
-    local = torch.empty((_fn("linear_matrix", "mi_linear_matrix_floats", _c_long)(int(delta), T, lanes, H, dk, dv),),
-                        dtype=torch.float32, device=u.device)
+    local = torch.empty((linear_matrix_bytes(T, lanes, H, dk, dv, delta) // 4,), dtype=torch.float32, device=u.device)
     _check(_fn("linear_matrix", "mi_linear_matrix_scan")(
         _p(u), ld, int(q_col), int(k_col), int(v_col), int(removal_col), H, dk, dv, _p(state), _p(slot_ids), lanes,
         _p(chunks.chunks), _p(chunks.lane_chunks), count, int(chunks.chunk_size), _p(head_decay), float(key_scale),

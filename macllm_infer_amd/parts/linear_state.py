@@ -1,10 +1,11 @@
 """Mixers that carry a matrix-valued state per head from token to token instead of a cache of keys:
 retention and lightning attention (a fixed decay per head), gated linear attention (a decay per key channel) and the
-generalized delta rule (a decay per key channel and a removal of what the state holds along the unit key).  All keep their state [heads, value dim, key dim] in float32 in the
-request's state slot and run through one scan kernel (``ops.linear_state_scan``), for prompt portions and for
-single decoded tokens alike, but that retention and the delta rule take bfloat16 portions of ``MATRIX_FROM`` tokens on to
-the float32 matrix cores (``ops.linear_matrix_scan``) and lightning attention has chunks of its own; rotation, decays, gates of the recurrence and unit keys are formed in float32 inside
-it.  The head-wise root-mean-square norm, its weight and the output gate are one more launch.
+generalized delta rule (a decay per key channel and a removal of what the state holds along the unit key).  All keep
+their state [heads, value dim, key dim] in float32 in the request's state slot and run through one scan kernel
+(``ops.linear_state_scan``), for prompt portions and for single decoded tokens alike, but that retention and the delta
+rule take bfloat16 portions to the float32 matrix cores where that pays (``runs_pay``, ``ops.linear_matrix_scan``) and
+lightning attention has chunks of its own; rotation, decays, gates of the recurrence and unit keys are formed in float32
+inside it.  The head-wise root-mean-square norm, its weight and the output gate are one more launch.
 """
 from __future__ import annotations
 
@@ -42,16 +43,44 @@ def chunk_table(step):
     return step.derived[key]
 
 
-# Tokens of the longest lane from which on runs of tokens on the matrix cores are faster than the walk token by token
-MATRIX_FROM = 32
+# (delta rule, key channels) -> the tokens from which on runs on the matrix cores pay; the lanes x heads up to which they do
+# in a step of up to 8 lanes that holds so many tokens a lane; the lanes x heads a token of the average lane, of at most so many tokens,
+# up to which they do in any case.  See ``runs_pay``.
+RUNS_PAY = {(True, 64): (32, 128, 10, 3.0, 128), (True, 128): (48, 64, 40, 1.0, 256),
+            (False, 64): (32, 128, 10, 3.0, 128), (False, 128): (64, 128, 40, 0.9, 256)}
+
+
+def runs_pay(tokens: int, lanes: int, heads: int, key_dim: int, delta: bool) -> bool:
+    """Whether a step of so many tokens in so many lanes (those of a captured step, which does not know how its tokens fall
+    into lanes) is faster in runs on the matrix cores than token by token, end to end or in chunks of 128.
+
+    A lane costs a run's matrices however few tokens it has, the walk its longest lane.  us a layer, token by token | in
+    runs, steps of a capacity (token by token: end to end up to 128 tokens, in chunks beyond):
+
+    * delta rule, 16 heads of 64: one lane of 32 tokens 33 | 23, 100 96 | 23, 2,048 244 | 104; 3 single tokens beside 60 59 |
+      21, beside 512 169 | 46; 8 lanes of 16 18 | 29, of 32 30 | 31, of 64 52 | 37; 16 lanes of 32 31 | 56, of 64 53 | 64,
+      of 128 111 | 80; 32 lanes of 8 18 | 97, of 64 69 | 120.  48 heads: 4 lanes of 64 53 | 50, 8 of 64 65 | 90, of 128 123 | 117.
+    * delta rule, heads of 128: 8 of them, one lane of 32 36 | 37, of 48 52 | 37, of 2,048 354 | 241; 8 lanes of 64 69 | 56, 16
+      of 64 73 | 103, of 128 136 | 127; 3 single tokens beside 256 227 | 59.  32 heads: 2 lanes of 64 68 | 56, 4 of 64 73 |
+      103, of 128 136 | 127, 8 of 128 142 | 257, of 256 676 | 467.
+    * retention, 8 heads of 64: one lane of 32 22 | 20, 2,048 125 | 48; 8 lanes of 16 13 | 21, of 32 23 | 21; 16 of 32 24 | 28, of
+      64 39 | 30; 32 of 64 45 | 46.  16 heads of 128 (values of 256): one lane of 48 37 | 38, of 64 49 | 39; 4 lanes of 64 46 |
+      54, of 128 85 | 62; 8 of 64 58 | 65, of 128 97 | 80; 3 single tokens beside 256 139 | 67."""
+    least, sure, few, slope, longest = RUNS_PAY[delta, key_dim]
+    return tokens >= least and ((lanes <= 8 and lanes * heads <= sure and tokens >= few * lanes)
+                                or (lanes * heads <= slope * min(tokens / lanes, longest) and tokens >= least * lanes))
 
 
 def run_scan(u: torch.Tensor, step, columns: dict, recurrence: dict) -> None:
     """The scan of retention or the delta rule: a run of tokens at a time on the float32 matrix cores for prompt portions in
-    bfloat16 whose heads those kernels cover, else token by token (single tokens, short portions, float32, other sizes)."""
+    bfloat16 whose heads those kernels cover, else token by token (single tokens, many short lanes, float32, other sizes)."""
     floor = recurrence.get("decay_floor")
-    if (u.is_cuda and step.max_query_len >= MATRIX_FROM
-            and ops.linear_matrix_supported(u.dtype, columns["key_dim"], columns["value_dim"], floor)):
+    lanes, tokens, _ = step.sizes
+    heads, sizes = columns["num_heads"], (columns["key_dim"], columns["value_dim"])
+    if (u.is_cuda and step.max_query_len > 1 and ops.linear_matrix_supported(u.dtype, *sizes, floor)
+            and runs_pay(tokens, lanes, heads, sizes[0], floor is not None)
+            and ops.linear_matrix_bytes(tokens, lanes, heads, *sizes, floor is not None) <= ops.LINEAR_MATRIX_MOST_BYTES
+            and columns["state"].data_ptr() % 16 == 0):
         ops.linear_matrix_scan(u, **columns, **recurrence, slot_ids=step.slot_ids, chunks=chunk_table(step))
         return
     ops.linear_state_scan(u, **columns, **recurrence, cu_seqlens=step.cu_seqlens, slot_ids=step.slot_ids,

@@ -292,6 +292,40 @@ def test_work_area_of_the_runs_is_that_of_the_tokens(delta):
     assert float((now - walked_state).abs().max()) <= 4e-6 * float(walked_state.abs().max())
 
 
+def test_a_step_takes_the_same_scan_launched_and_replayed(monkeypatch):
+    """Portions alone and beside others, and crowds of short ones: the scan that a step's first pass launches is the one
+    its capacity's graph holds, runs on the matrix cores for the former and the walk for the latter."""
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import config_from_dict
+    from macllm_infer_amd.kernels import ops
+    from macllm_infer_amd.weights.random_init import random_tensors
+    retention = {"type": "retention", "mixer": {"heads": 8, "dim": 64, "vdim": 128, "rot": {"base": 1e6, "dims": 64},
+                                                "decay": [0.9 + 0.01 * head for head in range(8)]}}
+    delta = {"type": "general_delta", "mixer": {"heads": 16, "dim": 64, "decay_rank": 32}}
+    raw = {"architecture": "Mukutar", "width": 256, "vocab": 300, "norm": {"eps": 1e-5}, "max_context": 4096,
+           "layers": [dict(layer, mlp={"kind": "dense", "ff": 256}) for layer in (delta, retention)]}
+    config = config_from_dict(raw)
+    engine = Engine(config=config, tensors=random_tensors(config, 3, torch.bfloat16, "baseline"), dtype="bfloat16",
+                    kv_cache_capacity_tokens=8192, max_active_sequences=40)
+    taken = []
+    for name in ("linear_matrix_scan", "linear_state_scan"):
+        plain = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda *args, name=name, plain=plain, **kw: (taken.append(name), plain(*args, **kw))[1])
+    for lengths, runs in (([300], True), ([20], True), ([14], False), ([60, 1, 1], True), ([16] * 16, False), ([8] * 32, False), ([128] * 4, True)):
+        seen = []
+        for _ in range(3):
+            taken.clear()
+            names = [f"r{index}" for index in range(len(lengths))]
+            for name in names:
+                engine.add_request(name)
+            engine.step([Lane(name, [7] * length, [length - 1]) for name, length in zip(names, lengths)])
+            for name in names:
+                engine.finish(name)
+            seen.append(set(taken))
+        want = {"linear_matrix_scan"} if runs else {"linear_state_scan"}
+        assert seen[0] == want and seen[1] == want and not seen[2], (lengths, seen)
+
+
 def test_heads_the_matrix_cores_do_not_cover_stay_with_the_walk():
     from macllm_infer_amd.kernels import ops
     covered = lambda *sizes, dtype=torch.bfloat16, floor=None: ops.linear_matrix_supported(dtype, *sizes, floor)

@@ -160,3 +160,18 @@ def test_greedy_generation_through_the_scheduler(host_ops, tmp_path):
         assert finished[index].generated == mukutar_plain.greedy(raw, tensors, prompt, 6)
     stats = engine.cache.stats()
     assert stats["live_requests"] == 0 and stats["free_slots"] == 3
+
+
+def test_many_short_lanes_are_walked_and_portions_go_in_runs():
+    """Which scan a step of retention or the delta rule takes, by the lanes and tokens of its captured step: a portion alone
+    or beside a few single tokens in runs on the matrix cores, a crowd of short lanes token by token."""
+    from macllm_infer_amd.parts.linear_state import RUNS_PAY, runs_pay
+    for (delta, key_dim), (least, *_) in RUNS_PAY.items():
+        assert runs_pay(2048, 1, 16, key_dim, delta) and runs_pay(least + least % 16, 1, 4, key_dim, delta)
+        assert not runs_pay(least - 1, 1, 4, key_dim, delta) and not runs_pay(16, 4, 4, key_dim, delta)
+        assert not runs_pay(64, 64, 4, key_dim, delta) and not runs_pay(256, 64, 8, key_dim, delta)
+        assert not runs_pay(256, 32, 16, key_dim, delta) and not runs_pay(2048, 64, 16, key_dim, delta)
+    # three single tokens beside 60 or 512, in the captured steps that hold them
+    assert runs_pay(80, 8, 16, 64, True) and runs_pay(640, 8, 8, 64, False) and runs_pay(640, 8, 8, 128, True)
+    assert runs_pay(2048, 16, 16, 64, True) and not runs_pay(1024, 16, 16, 64, True)          # lanes of 128 and of 64
+    assert runs_pay(512, 4, 32, 128, True) and not runs_pay(256, 4, 32, 128, True)
