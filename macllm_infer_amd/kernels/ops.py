@@ -866,20 +866,43 @@ def latent_decode_attention(q: torch.Tensor, num_heads: int, kv_rank: int, rope_
 # --------------------------------------------------------------------------- routed experts
 MOE_TILE_ROWS = 16          # places of a tile of the grouped products: steps of few rows
 MOE_WIDE_TILE_ROWS = 64     # steps whose experts get 64 rows or more each on average
-MOE_WIDEST_TILE_ROWS = 128  # and 256 or more, if rows and matrices are whole 16-byte pieces (``whole_pieces``)
-# In bfloat16 (and whole pieces) the wide tiles pay earlier and longer: sixteen experts of 512 x 1,024 take 36 us with tiles
-# of 16 places and 31 with 64 at 38 rows each, 31 and 31 at 28 (of 3,072 x 3,072: 419 and 181 at 28); 45 with 64 places and
-# 51 with 128 at 338 rows each (the tiles of 64 still fit the GPU at once), 65 and 54 at 384.
-MOE_WIDE_ROWS_16 = 32
-MOE_WIDEST_ROWS_16 = 352
+MOE_WIDEST_TILE_ROWS = 128  # and 256 or more, if rows and matrices are whole 16-byte pieces (``whole_pieces``); see below
+MOE_COLUMNS = 128           # matrix rows of a workgroup of the wide tiles
+MOE_UNITS = 256             # compute units
+MOE_WIDE_RESIDENT = 3       # workgroups of 64 places whose LDS fits a compute unit
+MOE_WIDEST_RESIDENT = 2     # and of 128
 
 
-def moe_tile_rows(tokens: int, top_k: int, num_experts: int, whole_pieces: bool = False, dtype=torch.float32) -> int:
-    """The tile of the grouped products for a step: it depends on the step's size alone, never on its tokens."""
-    short = whole_pieces and dtype == torch.bfloat16
-    if whole_pieces and tokens * top_k >= (MOE_WIDEST_ROWS_16 if short else 2 * MOE_WIDEST_TILE_ROWS) * num_experts:
-        return MOE_WIDEST_TILE_ROWS
-    return MOE_WIDE_TILE_ROWS if tokens * top_k >= (MOE_WIDE_ROWS_16 if short else MOE_WIDE_TILE_ROWS) * num_experts else MOE_TILE_ROWS
+def moe_tile_rows(tokens: int, top_k: int, num_experts: int, whole_pieces: bool = False, dtype=torch.float32,
+                  columns: Optional[int] = None) -> int:
+    """The tile of the grouped products for a step: it depends on the step's size alone, never on its tokens.
+
+    In bfloat16 (and whole pieces), with ``columns`` rows in an expert's first matrix: tiles of 128 places read the
+    matrices half as often as tiles of 64, and a chip full of them takes about 1.1 times as long as one full of 64, of
+    which it holds half as many again.  So the tiles are counted in fills of the chip (an expert's last tile is half full
+    on average), and 128 places taken where 64 would need more than 1.1 times as many.  us of both products, 64 | 128
+    places, by rows an expert (experts x width x expert width):
+
+    * 16 x 1,024 x 512: 256 44 | 50, 338 45 | 50, 384 59 | 51; 4 of them 512 34 | 38, 1,024 43 | 48
+    * 64 x 1,024 x 512: 128 87 | 97, 192 114 | 111, 256 129 | 140, 300 151 | 153, 350 167 | 176, 400 188 | 189
+    * 8 x 3,072 x 3,072: 192 194 | 203, 256 270 | 212, 300 282 | 290, 350 302 | 296, 400 341 | 332, 512 418 | 362
+    * 16 x 3,072 x 3,072: 128 323 | 334, 192 382 | 357, 256 473 | 425, 300 508 | 526, 350 587 | 525
+    * 64 x 2,048 x 1,024: 128 284 | 299, 192 342 | 332, 256 430 | 401, 350 563 | 501; 128 x 1,024 x 256: 300 172 | 184
+
+    Tiles of 64 take the place of 16 from 32 rows an expert on where one tile an expert gives every other compute unit a
+    workgroup: 16 x 1,024 x 512 at 28 rows 31 | 31, 32 32 | 29, 64 53 | 30; 8 x 3,072 x 3,072 at 16 165 | 122; but
+    4 x 1,024 x 512 at 32 16 | 24, 64 20 | 24."""
+    rows = tokens * top_k
+    if not whole_pieces or dtype != torch.bfloat16 or columns is None:
+        if whole_pieces and rows >= 2 * MOE_WIDEST_TILE_ROWS * num_experts:
+            return MOE_WIDEST_TILE_ROWS
+        return MOE_WIDE_TILE_ROWS if rows >= MOE_WIDE_TILE_ROWS * num_experts else MOE_TILE_ROWS
+    blocks = -(-columns // MOE_COLUMNS)
+    if rows < (32 if 2 * num_experts * blocks >= MOE_UNITS else MOE_WIDE_TILE_ROWS) * num_experts:
+        return MOE_TILE_ROWS
+    fills = [-(-(2 * rows + tile * num_experts) * blocks // (2 * tile * MOE_UNITS * resident))
+             for tile, resident in ((MOE_WIDE_TILE_ROWS, MOE_WIDE_RESIDENT), (MOE_WIDEST_TILE_ROWS, MOE_WIDEST_RESIDENT))]
+    return MOE_WIDEST_TILE_ROWS if 10 * fills[0] > 11 * fills[1] else MOE_WIDE_TILE_ROWS
 
 
 ROUTINGS = {"softmax_then_top": 0, "top_then_softmax": 1, "sigmoid_then_top": 2}

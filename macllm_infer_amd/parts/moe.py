@@ -122,7 +122,8 @@ class RoutedExperts(FeedForward):
         how = dict(routing=spec.routing, renormalize=spec.renormalize, groups=spec.groups, kept_groups=spec.kept_groups)
         choice = (logits, spec.router_outputs, spec.top_k, self.correction, spec.route_scale, spec.weight_eps,
                   self.shared and spec.shared_gated)
-        pad = ops.moe_tile_rows(tokens, spec.top_k, spec.num_experts, self.whole_pieces, x.dtype)
+        pad = ops.moe_tile_rows(tokens, spec.top_k, spec.num_experts, self.whole_pieces, self.gate_up.dtype,
+                                self.gate_up.shape[1])
         if tokens <= ops.ROUTE_PLAN_TOKENS:
             _, weights, gate, plan = ops.moe_route_plan(*choice, experts_with_matrices=spec.num_experts, pad=pad,
                                                          place_weights=spec.input_weighted, **how)

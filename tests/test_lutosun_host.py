@@ -174,3 +174,19 @@ def test_greedy_generation_through_the_scheduler(host_ops, tmp_path):
         assert finished[index].generated == tokens[len(prompt):], index
     stats = engine.cache.stats()
     assert stats["live_requests"] == 0 and stats["free_slots"] == 3
+
+
+def test_tiles_of_the_grouped_products_go_by_the_matrices_too():
+    """The places of a tile of the experts' products: by fills of the chip, which the number of experts and their width
+    decide as much as the rows an expert gets; 16-bit tiles of 64 need a workgroup for every other compute unit; matrices
+    kept in float32, or not in whole pieces, keep their own lines."""
+    from macllm_infer_amd.kernels import ops
+    tile = lambda rows, experts, columns, dtype=torch.bfloat16, whole=True: ops.moe_tile_rows(rows * experts // 2, 2, experts, whole, dtype, columns)
+    assert [tile(rows, 16, 1024) for rows in (28, 32, 256, 338, 384)] == [16, 64, 64, 64, 128]
+    assert [tile(rows, 8, 6144) for rows in (128, 192, 256, 300, 400, 512)] == [64, 64, 128, 64, 128, 128]
+    assert [tile(rows, 64, 2048) for rows in (192, 256, 350)] == [128, 128, 128]
+    assert [tile(rows, 4, 1024) for rows in (32, 63, 64, 512, 1024, 8192)] == [16, 16, 64, 64, 64, 128]
+    for columns in (None, 1024, 6144):
+        assert [tile(rows, 8, columns, torch.float32) for rows in (63, 64, 255, 256)] == [16, 64, 64, 128]
+        assert [tile(rows, 8, columns, torch.float32, False) for rows in (63, 64, 255, 256)] == [16, 64, 64, 64]
+        assert [tile(rows, 8, columns, torch.bfloat16, False) for rows in (63, 64, 255, 256)] == [16, 64, 64, 64]
