@@ -124,7 +124,7 @@ class Engine:
         if check_device:
             # (bfloat16 products of few rows go through the skinny kernels)
             skinny = ["decode"] if self.dtype == torch.bfloat16 else []
-            kernel_build.ensure_modules(DecoderModel.kernel_modules(self.spec) + skinny + list(kernel_build.HOST_MODULES))
+            kernel_build.ensure_modules(DecoderModel.kernel_modules(self.spec, self.dtype) + skinny + list(kernel_build.HOST_MODULES))
         source.apply_aliases(self.spec.tensor_aliases, root_prefix=self.spec.root_namespace)
         expected = DecoderModel.expected_tensors(self.spec)
         if self.spec.stored_name_rules:

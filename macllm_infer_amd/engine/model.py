@@ -9,7 +9,7 @@ from typing import Dict, Hashable, List
 import torch
 
 from ..config.spec import ModelSpec
-from ..kernels import ops
+from ..kernels import build as kernel_build, ops
 from ..cache.manager import StateNeed
 from ..parts.base import BuildContext, Residual, RowVector, WeightedBranch, part_class
 from ..parts.block import arrangement_class
@@ -69,11 +69,13 @@ class DecoderModel:
         return list(dict.fromkeys(found))
 
     @staticmethod
-    def kernel_modules(spec: ModelSpec) -> List[str]:
+    def kernel_modules(spec: ModelSpec, dtype: torch.dtype = torch.bfloat16) -> List[str]:
+        """The HIP modules that a model of this spec launches in ``dtype``."""
         modules = ["common", "gemm"]
         for layer in spec.layers:
             modules += arrangement_class(layer.arrangement).kernel_modules(layer)
-        return list(dict.fromkeys(modules))
+        never = kernel_build.BFLOAT16_MODULES if dtype != torch.bfloat16 else ()
+        return [module for module in dict.fromkeys(modules) if module not in never]
 
     @staticmethod
     def cache_layout(spec: ModelSpec):

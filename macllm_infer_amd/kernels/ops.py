@@ -1200,6 +1200,7 @@ def linear_state_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, nu
 
 # the delta rule's matrices hold the reciprocal of a run's decays: its logarithm stays this far within float32's range
 LINEAR_MATRIX_MOST_LOG = 60.0
+LINEAR_MATRIX_KEY_DIMS = (64, 128)
 # the largest work area: 2,048 tokens of 64 heads of 128 channels take 604 MB, three times that of the walk's passes
 LINEAR_MATRIX_MOST_BYTES = 1 << 30
 
@@ -1208,7 +1209,9 @@ def linear_matrix_supported(dtype, key_dim: int, value_dim: int, decay_floor: Op
     """Whether the float32 matrix-core kernels of retention (``decay_floor`` None) or of the delta rule cover these heads
     and, for the delta rule, this strongest decay."""
     delta = decay_floor is not None
-    if dtype != torch.bfloat16 or not _fn("linear_matrix", "mi_linear_matrix_supported")(int(delta), int(key_dim), int(value_dim)):
+    if dtype != torch.bfloat16 or key_dim not in LINEAR_MATRIX_KEY_DIMS or value_dim % 16:      # (nothing is loaded for these)
+        return False
+    if not _fn("linear_matrix", "mi_linear_matrix_supported")(int(delta), int(key_dim), int(value_dim)):
         return False
     run = _fn("linear_matrix", "mi_linear_matrix_run")(int(delta))
     return not delta or 0.0 <= decay_floor * run <= LINEAR_MATRIX_MOST_LOG

@@ -49,7 +49,8 @@ class Attention(Mixer):
         unused = {"mamba2"} if spec.conv_kernel == 0 else set()                  # the convolutions' kernels
         if own_width or spec.head_dim % 8 or spec.head_dim > 128:                # the prompt kernel at padded widths
             unused.add("attention_widths")
-        if not own_width:                                                        # and the one at these two
+        if (not own_width or spec.out_gate or spec.weighting != "softmax" or spec.head_temperature
+                or (spec.window and spec.keep_first) or hasattr(spec.position, "slopes")):   # the one that shares its keys
             unused.add("attention_shared")
         return tuple(name for name in cls.kernel_modules if name not in unused)
 

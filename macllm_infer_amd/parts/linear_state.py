@@ -87,6 +87,12 @@ def run_scan(u: torch.Tensor, step, columns: dict, recurrence: dict) -> None:
                           max_query_len=step.max_query_len, chunks=scan_chunks(step))
 
 
+def scan_modules(modules: tuple, key_dim: int, value_dim: int) -> tuple:
+    """Without the kernels of runs on the matrix cores for heads that they do not cover."""
+    covered = key_dim in ops.LINEAR_MATRIX_KEY_DIMS and value_dim % 16 == 0
+    return tuple(name for name in modules if covered or name != "linear_matrix")
+
+
 @register_part("retention")
 class Retention(Mixer):
     """[q | k | v | g] = one projection of the normed rows; q and k rotated by position, k scaled;
@@ -94,6 +100,10 @@ class Retention(Mixer):
     graph_safe = True
     kernel_modules = ("common", "linear_state", "linear_matrix", "gemm")
     chunk_tokens = CHUNK_TOKENS
+
+    @classmethod
+    def modules_of(cls, spec) -> tuple:
+        return scan_modules(cls.kernel_modules, spec.key_dim, spec.value_dim)
 
     @classmethod
     def expected_tensors(cls, spec, prefix: str, hidden_size: int):
@@ -152,6 +162,10 @@ class GeneralDelta(Mixer):
     graph_safe = True
     kernel_modules = ("common", "linear_state", "linear_matrix", "gemm")
     chunk_tokens = CHUNK_TOKENS
+
+    @classmethod
+    def modules_of(cls, spec) -> tuple:
+        return scan_modules(cls.kernel_modules, spec.head_dim, spec.head_dim)
 
     @classmethod
     def expected_tensors(cls, spec, prefix: str, hidden_size: int):

@@ -175,3 +175,32 @@ def test_many_short_lanes_are_walked_and_portions_go_in_runs():
     assert runs_pay(80, 8, 16, 64, True) and runs_pay(640, 8, 8, 64, False) and runs_pay(640, 8, 8, 128, True)
     assert runs_pay(2048, 16, 16, 64, True) and not runs_pay(1024, 16, 16, 64, True)          # lanes of 128 and of 64
     assert runs_pay(512, 4, 32, 128, True) and not runs_pay(256, 4, 32, 128, True)
+
+
+def test_a_model_loads_the_kernels_it_can_launch():
+    """The prompt attention that shares its keys and the runs on the matrix cores take bfloat16 at their own sizes: models in
+    float32, or with other heads, forms of attention or state sizes, list neither."""
+    import dataclasses
+    from macllm_infer_amd.config.spec import AttentionSpec, LinearDistanceBiasSpec
+    from macllm_infer_amd.parts.base import part_class
+    modules = lambda spec: part_class(spec).modules_of(spec)
+    attention = AttentionSpec(num_heads=8, num_kv_heads=2, head_dim=64, scale=0.125, window=256)
+    assert "attention_shared" in modules(attention) and "attention" in modules(attention)
+    for other in (dict(head_dim=96), dict(value_dim=128), dict(keep_first=4), dict(out_gate=True), dict(weighting="sigmoid"),
+                  dict(head_temperature=True), dict(position=LinearDistanceBiasSpec(8))):
+        assert "attention_shared" not in modules(dataclasses.replace(attention, **other)), other
+    spec = config_from_dict(mukutar_configs.MUK_B).to_model_spec()
+    widths = {"retention": ("key_dim", "value_dim"), "general_delta": ("head_dim",), "attention": ("head_dim", "value_dim")}
+    sized = lambda part, width: dataclasses.replace(part, **{size: width for size in widths[part.kind]})
+    scans = {slot.spec.kind: slot.spec for layer in spec.layers for slot in layer.mixers}
+    assert set(scans) == set(widths)
+    for kind in ("retention", "general_delta"):
+        for width, covered in ((64, True), (128, True), (32, False), (72, False)):
+            names = modules(sized(scans[kind], width))
+            assert ("linear_matrix" in names) == covered and "linear_state" in names, (kind, width)
+    wide = dataclasses.replace(spec, layers=[dataclasses.replace(layer, mixers=[
+        dataclasses.replace(slot, spec=sized(slot.spec, 64)) for slot in layer.mixers]) for layer in spec.layers])
+    for dtype in (torch.bfloat16, torch.float32):
+        listed = DecoderModel.kernel_modules(wide, dtype)
+        assert ("linear_matrix" in listed) == ("attention_shared" in listed) == (dtype == torch.bfloat16)
+        assert {"linear_state", "attention"} <= set(listed)
