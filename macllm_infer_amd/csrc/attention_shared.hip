@@ -18,10 +18,11 @@
 // What bounds it: the instructions of the softmax (about 850 cycles of a wave for 64 keys and 16 columns), the reads of
 // the fragments from LDS and the fetches from L2, about a third of the time each; they overlap only in part.  Heads of
 // 64 fit two workgroups on a compute unit, heads of 128 one; of those two heads a workgroup halve the reads and the
-// fetches of a column.  Measured against the kernel whose waves read their own keys (prefill_attention_kernel), pages
-// of 16: 8 heads of 64 over 2 kv heads, 2,048 tokens 34.9 -> 28.2 us; 12 heads of 128 over 2, 2,048 tokens 82.1 -> 60.2,
-// behind 2,048 more 147 -> 114; 20 prompts of 200 behind 500, 32 heads of 128 over 8, 375 -> 146; with the
-// logarithmic bias and sinks, 2,048 tokens of 8 heads of 64 42.0 -> 34.5, 1,024 behind 1,024 of 12 of 128 127 -> 49.  The error of its
+// fetches of a column.  Measured against the kernel whose waves read their own keys (prefill_attention_kernel) in
+// replayed steps, pages of 16: 8 heads of 64 over 2 kv heads, 1,536 tokens 28.4 -> 21.9 us, 4 prompts of 512 28.3 -> 14.1;
+// 12 heads of 128 over 2, 1,999 tokens 95 -> 79, 1,536 behind 6,000 249 -> 199; 8 prompts of 256, 32 heads of 128 over 8,
+// 123 -> 36.5; with the logarithmic bias 1,999 tokens of 12 of 128 225 -> 90, with a window of 1,024 too 1,536 of 8 of 64
+// 30.3 -> 20.6.  Where it is the slower one is at ops.shared_prefill_heads, with both sides.  The error of its
 // results against 64 bits is the smaller one (2,048 tokens, scores of deviation one: 0.00195 against 0.00198, relative;
 // behind 1,024: 0.00203 against 0.00213), because every step of 32 keys has its own reference.
 // Tried without gain: the two groups half a turn apart (the phases only get longer: 36.7 us in place of 28.2), two

@@ -1588,64 +1588,51 @@ def prefill_attention_supported(dtype, num_heads: int, num_kv_heads: int, head_d
 def shared_prefill_heads(tokens: int, lanes: int, num_heads: int, num_kv_heads: int, head_dim: int, longest: int,
                          span: int, biased: bool = False) -> int:
     """How many query heads a workgroup of the prompt attention with shared keys takes, 0: the kernel whose waves
-    read their keys themselves is the faster one.  ``tokens`` and ``lanes`` say how full the tiles of 64 tokens are,
-    ``longest`` bounds the step's contexts (0: not known); all three are those of a captured step (at least 2,048 for
-    ``longest``), which does not know how its tokens fall into lanes.  ``biased``: with the logarithmic bias.
+    read their keys themselves is the faster one.  ``tokens`` and ``lanes`` size the step, ``longest`` bounds its contexts
+    (0: not known); all three are those of a captured step (at least 2,048 for ``longest``), which does not know how its
+    tokens fall into lanes.  ``biased``: with the logarithmic bias.
 
     The other kernel works on 16 tokens a workgroup and splits their keys eight ways instead of two, so that a tile of a
-    few tokens, or a grid that leaves compute units idle, costs it little; of heads of 64 it shares a key fragment
-    among up to two heads, or four where contexts may be longer than 2,048.  This one pays where full tiles fill the
-    chip, and forms a bias once a key and token where the other forms it in every wave.  Measured over nine shapes of
-    heads, contexts to 8,192 and windows, 1,364 steps without a bias and 1,332 with one; us, other | this one (n: two
-    heads a workgroup):
+    few tokens, or a grid that leaves compute units idle, costs it little.  This one walks a tile's keys in longer chains
+    but reads them once for 64 tokens, and forms a bias once a key and token where the other forms it in every wave.
+    us of the kernel in replayed steps (three layers of a model, so that keys come from memory), other | this one
+    (n: two heads a workgroup); over 1,526 such steps the rule's choice costs 92.7 ms, always the better kernel 92.0,
+    always the other one 134.8:
 
-    * one query head a kv head: from half a chip of workgroups on, or many lanes.  16 heads of 64: 515 tokens 15.7 | 14.2,
-      300 behind 500 16.6 | 18.9, 2,048 behind 4,096 246 | 108; 8 of 128: 1,024 tokens 32.5 | 24.9, 3 of 300 behind 4,000
-      106 | 119, 16 single tokens behind 500 25.7 | 19.3, 32 behind 1,500 99 | 55.
-    * heads of 64 that share keys, contexts of up to 2,048: 8 over 2, 1,024 tokens 12.9 | 16.3, 1,536 25.4 | 22.0,
-      2 prompts of 777 21.3 | 18.5, 32 of 64 behind 500 24.7 | 13.4, but 8 single tokens beside 1,500 32.1 | 36.4, 8 beside
-      515 17.7 | 29.4, 32 lanes of 8 behind 1,500 20.2 | 31.4 (64: 52.9 | 49.2); 32 over 8, 300 tokens 15.4 | 10.3; with a
-      bias 8 over 2, 1,024 tokens 15.0 | 18.9, behind 500 20.2 | 25.9.  A walk of 128 keys: 777 tokens 8.1 | 8.0, 1,999
-      14.6 | 8.4; of 512: 64 tokens 7.0 | 6.0, 777 11.8 | 14.4.
-    * the same with longer contexts: 2,048 behind 2,048 44.4 | 50.1, 4,096 58.1 | 71.8; with a window of 1,024, 1,999 behind
-      4,000, 23.6 | 23.4 (6 over 2: 19.4 | 23.2; 32 over 8: 84 | 57), of 512 18.3 | 15.0; with a bias and that window, 1,280
-      behind 3,000, 42.7 | 22.2, and without the window 8 over 2, 4,096 behind 2,048, 161 | 171 (6 over 2: 111 | 144).
-    * heads of 128 that share keys: 12 over 2, 515 tokens 18.7 | 20.9, 777 30.2 | 27.5, 1,024 38.5 | 24.3; behind 4,096
-      tokens 777 121 | 131, 1,024 128 | 93; 32 over 8, 515 behind 4,096 180 | 174n; 16 lanes of 8 behind 1,500 32.2 | 48.4,
-      32 of 8 behind 500 38.7 | 25.5n, behind 1,500 66.6 | 62.4n, behind 4,000 133 | 154n; 16 over 2 with a window of 1,024,
-      24 single tokens beside 515 71 | 82n.  With a bias: 12 over 2, 515 tokens 50 | 23, 16 single tokens behind 4,000 234 |
-      123, 64 tokens behind 6,000 97 | 127.
+    * one query head a kv head.  16 of 64: a prompt of 300 tokens 11.6 | 10.8, behind 1,500 28.8 | 35.0, 515 19.7 | 14.9, 515
+      behind 3,000 66 | 64, 1,999 82 | 46; 16 lanes of 8 behind 400 28 | 18, behind 3,500 107 | 95 (with a bias 119 | 145).  8
+      of 128: 515 21.2 | 21.6, 777 28.5 | 27.5, 1,024 31.5 | 25.1, 16 lanes of 2 behind 1,500 53 | 49.
+    * heads of 64 that share keys, contexts to 2,048.  8 over 2: 515 tokens 11.7 | 15.1, 1,024 14.7 | 16.6, 1,300 31 | 27, 1,536
+      28 | 22; 3 prompts of 311 15.5 | 10.5 (behind 1,000 21.6 | 26.7), 8 of 100 13.6 | 7.3, 8 single tokens beside 515 18.5 |
+      23.0; 32 lanes of 8 behind 400 13.3 | 22.5, 60 of 8 65 | 58.  32 over 8: 100 tokens 8.1 | 6.6, behind 500 12.7 | 14.7; 300
+      16.0 | 11.3, behind 1,500 36.8 | 35.4.
+    * the same with longer contexts.  8 over 2: 1,024 behind 3,000 44 | 51, 1,999 behind 1,500 54 | 82; 32 over 8: 1,999
+      behind 1,500 156 | 142, 515 behind 6,000 145 | 159, 8 prompts of 100 behind 3,000 138 | 162.  With a bias 37 tokens
+      behind 3,000 94 | 65, 1,999 behind 6,000 218 | 159; with a window of 1,024 too 43 | 26 and 63 | 26.
+    * heads of 128 that share keys.  12 over 2: 300 tokens 17.3 | 15.4, behind 500 23.5 | 27.8, 515 behind 500 34.8 | 32.3, 1,999
+      95 | 79n; 32 lanes of 2 behind 400 37 | 24n, 16 of them 19 | 19; 515 behind 3,000 64 | 97, 1,024 101 | 76, 8 prompts of
+      256 183 | 100n, 60 lanes of 8 behind 3,500 338 | 315n; 32 over 8, these lanes, 575 | 709n, 32 of them 287 | 329n.  With a
+      bias 12 over 2: 37 tokens behind 6,000 263 | 175, 1,500 beside a single token 172 | 69n.
     Heads of 64 go one to a workgroup: two workgroups then share a compute unit.  Of heads of 128 a unit holds one
     workgroup either way: one head while there is a unit for each, else two, which read K and V half as often (12 over 2,
-    2,048 tokens behind 2,048 132 with one head, 114 with two; 1,024 tokens 24.3 and 34.2)."""
+    1,536 tokens behind 6,000 256 and 199n; 1,024 tokens 125 and 187n)."""
     heads_per_kv = num_heads // num_kv_heads
     longest = longest or 1 << 30
     walk = min(longest, abs(span) + 64) if span else longest        # keys of the longest walk
-    sure = max(0, tokens - 63 * lanes) // 64                        # full tiles, however the tokens fall into lanes
-    full = tokens // 64 if tokens >= 64 * lanes else sure           # and where lanes are tiles long on the average
-    many = lanes // 2 * num_heads                                   # workgroups of short lanes (a bucket is more than half real lanes)
-    grid = full * num_heads
     if heads_per_kv == 1:
-        return 1 if ((max(grid, many) >= 128 and (sure * num_heads >= 112 or lanes >= 8))
-                     or (lanes >= 16 and many >= 64 and walk <= 2048)) else 0
+        many = 32 if biased and longest > 2048 else 16
+        return 1 if tokens * num_heads >= 128 * 64 or (lanes >= many and lanes * num_heads >= 128) else 0
     if head_dim == 64:
+        grid = tokens * num_kv_heads // 64                          # tiles of 64 tokens, by kv head
         if longest > 2048:
-            if biased:
-                return 1 if heads_per_kv >= 4 or span else 0
-            return 1 if walk <= 576 or (walk <= 2048 and grid >= 240) else 0
-        if walk <= 192 or (walk <= 576 and tokens <= 320 and lanes <= 2):
-            return 1
-        return 1 if (sure >= (19 if biased else 22) or full >= 31 or many >= 192
-                     or (num_heads >= 24 and sure * num_heads >= 96)) else 0
-    if biased:
-        if walk > 4096 and tokens <= 128:
+            return 1 if biased or walk <= 576 or (grid >= 80 and tokens >= 128 * lanes) else 0
+        least = 28 if lanes >= 16 else 32 if lanes >= 4 or walk <= 576 else 40
+        return 1 if walk <= 192 or grid >= least or (lanes >= 32 and lanes * num_kv_heads >= 128) else 0
+    if not biased:
+        grid = tokens * num_heads // 64
+        if not (grid >= 96 or lanes >= 32 if walk <= 2048 else grid >= 192 and tokens >= 32 * lanes):
             return 0
-    elif walk > 2048:
-        if grid < 192 or (full < 16 and grid < 256):
-            return 0
-    elif grid < 128:
-        return 2 if max(grid, many) >= (192 if walk <= 576 or heads_per_kv <= 6 else 512) else 0
-    return 2 if max(-(-tokens // 64), lanes) * num_heads > 256 else 1      # compute units
+    return 2 if max(-(-tokens // 64), lanes) * num_heads >= 256 else 1      # compute units
 
 
 def shared_prefill_covers(num_kv_heads: int, head_dim: int, page_size: int, page_stride: int, k_address: int, v_address: int) -> bool:

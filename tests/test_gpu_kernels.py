@@ -1673,24 +1673,26 @@ def test_prefill_attention_with_shared_keys(ops, monkeypatch, Hq, Hkv, dh, page_
 
 
 def test_rule_of_the_prompt_attention(ops):
-    """Heads of 64: walks of a few keys, longer ones in full tiles on more than half the chip.  One head a kv head: half
-    the chip.  Heads of 128: full tiles on half the chip, two heads a workgroup once every compute unit has one.  With the
-    logarithmic bias: wherever this kernel forms it less often."""
+    """Heads of 64: walks of a few keys, longer ones in many tiles.  One head a kv head: half the chip.  Heads of 128: full
+    tiles on a third of the chip (longer contexts: three quarters), two heads a workgroup once every compute unit has
+    one.  With the logarithmic bias: wherever this kernel forms it less often."""
     rule = ops.shared_prefill_heads
-    assert rule(64, 1, 8, 2, 64, 2048, 512) == 1 and rule(64, 1, 8, 2, 64, 9000, -512) == 1      # a window, a chunk of 512 keys
-    assert rule(777, 1, 8, 2, 64, 2048, 512) == 0 and rule(777, 1, 8, 2, 64, 2048, 128) == 1
-    assert rule(64, 1, 8, 2, 64, 2048, 513) == 0 and rule(300, 1, 8, 2, 64, 2048, 0) == 0
-    assert rule(1536, 1, 8, 2, 64, 2048, 0) == 1 and rule(1024, 1, 8, 2, 64, 2048, 0) == 0
+    assert rule(64, 1, 8, 2, 64, 9000, 512) == 1 and rule(64, 1, 8, 2, 64, 9000, -512) == 1      # a window, a chunk of 512 keys
+    assert rule(64, 1, 8, 2, 64, 9000, 513) == 0 and rule(300, 1, 8, 2, 64, 2048, 0) == 0
+    assert rule(896, 2, 8, 2, 64, 2048, 512) == 0 and rule(1024, 1, 8, 2, 64, 2048, 512) == 1 and rule(48, 2, 8, 2, 64, 2048, 128) == 1
+    assert rule(1408, 2, 8, 2, 64, 2048, 0) == 1 and rule(1024, 1, 8, 2, 64, 2048, 0) == 0
+    assert rule(1024, 4, 8, 2, 64, 2048, 0) == 1 and rule(896, 4, 8, 2, 64, 2048, 0) == 0 and rule(896, 16, 8, 2, 64, 2048, 0) == 1
     assert rule(2048, 1, 8, 2, 64, 2049, 0) == 0 and rule(2048, 1, 8, 2, 64, 0, 0) == 0
-    assert rule(2048, 2, 8, 2, 64, 4096, 1024) == 1 and rule(1024, 2, 8, 2, 64, 4096, 1024) == 0
-    assert rule(320, 1, 32, 8, 64, 2048, 0) == 1 and rule(128, 1, 32, 8, 64, 2048, 0) == 0
+    assert rule(2048, 2, 8, 2, 64, 4096, 1024) == 0 and rule(2048, 2, 32, 8, 64, 4096, 1024) == 1
+    assert rule(640, 2, 32, 8, 64, 4096, 0) == 1 and rule(320, 2, 32, 8, 64, 4096, 0) == 0 and rule(896, 16, 32, 8, 64, 4096, 0) == 0
+    assert rule(320, 2, 32, 8, 64, 2048, 0) == 1 and rule(112, 2, 32, 8, 64, 2048, 0) == 0
     assert rule(640, 2, 16, 16, 64, 9000, 0) == 1 and rule(320, 2, 16, 16, 64, 9000, 0) == 0
-    assert rule(1024, 1, 8, 8, 128, 0, 0) == 1 and rule(960, 3, 8, 8, 128, 4096, 0) == 0
-    assert rule(576, 1, 12, 2, 128, 2048, 0) == 0 and rule(777, 1, 12, 2, 128, 2048, 0) == 1
-    assert rule(777, 1, 12, 2, 128, 4096, 0) == 0 and rule(1024, 1, 12, 2, 128, 9000, 0) == 1
-    assert rule(2048, 1, 12, 2, 128, 9000, 0) == 2
-    for sizes, plain, biased in (((2048, 1, 8, 2, 64, 4096, 0), 0, 1), ((2048, 1, 6, 2, 64, 8192, 0), 0, 0), ((1408, 1, 8, 2, 64, 2048, 0), 0, 1),
-                                 ((515, 1, 12, 2, 128, 2048, 0), 0, 1), ((64, 1, 12, 2, 128, 8192, 0), 0, 0), ((32, 32, 12, 2, 128, 4096, 0), 0, 2)):
+    assert rule(1024, 4, 8, 8, 128, 0, 0) == 1 and rule(896, 2, 8, 8, 128, 0, 0) == 0
+    assert rule(320, 2, 12, 2, 128, 2048, 0) == 0 and rule(640, 2, 12, 2, 128, 2048, 0) == 1 and rule(1408, 2, 12, 2, 128, 2048, 0) == 2
+    assert rule(896, 2, 12, 2, 128, 4096, 0) == 0 and rule(896, 2, 12, 2, 128, 4096, 1024) == 1 and rule(1024, 1, 12, 2, 128, 9000, 0) == 1
+    assert rule(2048, 1, 12, 2, 128, 9000, 0) == 2 and rule(1024, 1, 16, 2, 128, 4096, 0) == 2
+    for sizes, plain, biased in (((48, 2, 8, 2, 64, 4096, 0), 0, 1), ((2048, 1, 6, 2, 64, 8192, 0), 0, 1), ((640, 2, 8, 2, 64, 2048, 0), 0, 0),
+                                 ((48, 2, 12, 2, 128, 8192, 0), 0, 1), ((32, 32, 12, 2, 128, 4096, 0), 0, 2), ((16, 16, 16, 16, 64, 4096, 0), 1, 0)):
         assert rule(*sizes) == plain and rule(*sizes, True) == biased, sizes
 
 
@@ -1698,16 +1700,16 @@ def test_rule_of_the_prompt_attention_knows_tiles_of_a_few_tokens(ops):
     """Steps of many short lanes, and of single tokens beside a portion: their tiles hold a few tokens each and are no
     reason for the kernel that works on whole tiles, unless there are more of them than fill the chip."""
     rule = ops.shared_prefill_heads
-    for lanes, tokens in ((16, 16), (16, 128), (32, 32), (32, 512), (16, 576), (32, 1664)):
+    for lanes, tokens in ((8, 80), (16, 16), (16, 128), (32, 32), (32, 512), (16, 640)):
         assert rule(tokens, lanes, 8, 2, 64, 2048, 0) == 0, (lanes, tokens)
     assert rule(64, 64, 8, 2, 64, 2048, 0) == 1 and rule(64, 64, 8, 2, 64, 4096, 0) == 0
-    assert rule(2048, 32, 8, 2, 64, 2048, 0) == 1            # 32 lanes that may all be a tile long
     for lanes, tokens in ((16, 16), (16, 256), (32, 32), (64, 1024)):
         assert rule(tokens, lanes, 12, 2, 128, 4096, 0) == 0, (lanes, tokens)
     assert rule(16, 16, 12, 2, 128, 2048, 0) == 0 and rule(32, 32, 12, 2, 128, 2048, 0) == 2
     assert rule(1024, 16, 12, 2, 128, 4096, 0) == 1 and rule(960, 16, 12, 2, 128, 4096, 0) == 0
-    assert rule(16, 16, 32, 8, 128, 4096, 0) == 0 and rule(16, 16, 32, 8, 128, 2048, 0) == 2
-    assert rule(32, 32, 8, 8, 128, 9000, 0) == 1 and rule(16, 16, 8, 8, 128, 9000, 0) == 0
+    assert rule(16, 16, 32, 8, 128, 4096, 0) == 0 and rule(16, 16, 32, 8, 128, 2048, 0) == 0 and rule(32, 32, 32, 8, 128, 2048, 0) == 2
+    assert rule(512, 64, 32, 8, 128, 4096, 0) == 0 and rule(2048, 64, 32, 8, 128, 4096, 0) == 2
+    assert rule(16, 16, 8, 8, 128, 9000, 0) == 1 and rule(8, 8, 8, 8, 128, 9000, 0) == 0
 
 
 def test_pages_beyond_32_bits_stay_with_the_other_prompt_kernel(ops):
