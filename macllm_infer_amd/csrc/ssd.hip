@@ -313,12 +313,14 @@ ssd_chunk_state_kernel(const bf16_t* __restrict__ TT, int E, int GN, const float
 // Per lane, serially over its chunks: state_in[chunk] = running (rounded to bfloat16: it is a
 // matrix-core operand); running = decay[chunk] * running + chunk_state[chunk].  The running state
 // starts from the request's slot and goes back to it, in float32.
-// V neighbouring elements a thread.  Bound by memory: 10 bytes for every element of a chunk's state; four elements a
+// V neighbouring elements a thread.  An element of a chunk's state is 6 bytes, float32 in and bfloat16 out; four elements a
 // thread ask for 16 bytes a load and write 8 (one element a thread: 4 and 2), in workgroups of one wave so that small
 // states still reach every compute unit.  A lane's chunks come in rounds of AT_ONCE whose loads are all asked for
-// before the recurrence; lanes of up to four chunks take the short round, which asks for nothing twice over.  Measured
-// (one element a thread -> now, beside the prompt attention): 16 chunks of 24 heads of 64 x 128 12.4 -> 8.4 us, of 128 x
-// 256 55 -> 25; 25 lanes of one to five chunks 67 -> 25.
+// before the recurrence; lanes of up to four chunks take the short round, which asks for nothing twice over.  Few chunks
+// are bound by the launch and the round trips, many by their bytes, which come from the caches that the launch before
+// filled.  Alone, 24 heads, in us: 64 x 128, 1 chunk 3.0, 4 3.8, 16 7.6 (2.5 TB/s), 32 12.4, so 0.29 for each chunk more
+// (4.1 TB/s); 128 x 256, 1 chunk 5.2, 16 14.3 (5.3 TB/s), 32 26.1.  Beside the prompt attention (one element a thread ->
+// now): 16 chunks of 64 x 128 12.4 -> 8.4, of 128 x 256 55 -> 25; 25 lanes of one to five chunks of 64 x 128 67 -> 25.
 template <int V, int AT_ONCE>
 __device__ __forceinline__ void ssd_pass_rounds(const float* __restrict__ chunk_state, const float* __restrict__ chunk_decay,
                                                 bf16_t* __restrict__ state_in, int first, int count, int H, int head,
@@ -756,7 +758,8 @@ ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf1
 // of eight waves a (lane, head), a tile of 16 tokens a wave; rows of the grid past the heads update the lanes' conv tails,
 // as in the pass.  A short prompt waits for round trips, not for bytes: everything that the first 64 tokens need, the old
 // state and the operands of the new one are asked for at the top and laid in LDS behind one barrier.  37 tokens, 24 heads
-// of 64 x 128: 8.0 + 7.0 + 7.8 us in three launches, 13.5 in this one (14.7 with every stage asking for its own).
+// of 64 x 128: 8.0 + 7.0 + 7.8 us in three launches, 13.5 in this one (14.7 with every stage asking for its own); with the
+// conv's launch before, replayed alone, 23.6 -> 19.2 (100 tokens 27.5 -> 23.1, 128 27.9 -> 24.0; 37 of 128 x 256 44.7 -> 40.2).
 #define SSD_SINGLE_TOKENS (SSD_SCAN_WAVES * 16)
 struct SsdSingle {
   float* state;                    // [slots, H, P, N]
