@@ -21,6 +21,7 @@ from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from ..kernels import ops
 from . import native
 from .pages import BlockTable, CacheExhausted, PagePool, SlotPool
 
@@ -228,6 +229,7 @@ class CacheManager:
                 else:
                     raise TypeError(f"unknown cache need {need!r}")
             self.entries[key] = entry
+        self._slot_states = ops.SlotStates(self._state_tensors) if self.device.type == "cuda" else None
         self.core = Core([group.page_size for group in self.groups], [group.num_pages for group in self.groups],
                          [group.need.span for group in self.groups], max_requests,
                          [getattr(group.need, "keep_first", 0) for group in self.groups])
@@ -266,7 +268,10 @@ class CacheManager:
         for index, group in enumerate(self.groups):
             group.tables[request] = BlockTable(self.core, index, slot)
         if self._state_tensors:                       # a fresh request starts from zeros
-            torch._foreach_zero_([tensor[slot] for tensor in self._state_tensors])
+            if self._slot_states is not None:
+                self._slot_states.zero(slot)
+            else:
+                torch._foreach_zero_([tensor[slot] for tensor in self._state_tensors])
         return record
 
     def can_ever_fit(self, total_tokens: int) -> bool:

@@ -33,6 +33,7 @@ _SIGNATURES = {
         "mi_embed": [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_int, _c_int, _c_ptr],
         "mi_embed_rmsnorm": [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_float, _c_ptr, _c_int, _c_int, _c_ptr],
         "mi_feed_tokens": [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
+        "mi_zero_slot": [_c_ptr, _c_ptr, _c_int, _c_long, _c_ptr],
         "mi_add_rmsnorm": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_float, _c_ptr, _c_int, _c_ptr, _c_int,
                            _c_int, _c_float, _c_float, _c_ptr],
         "mi_add_partials_rmsnorm": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_float, _c_ptr, _c_int, _c_ptr, _c_int, _c_int,
@@ -335,6 +336,27 @@ def feed_tokens(token_ids: torch.Tensor, source: torch.Tensor, dst: Sequence[int
     _check(_fn("common", "mi_feed_tokens")(_p(token_ids), token_ids.numel(), _p(source), source.numel(),
                                            ctypes.addressof(places), ctypes.addressof(sources), count, _stream()),
            "feed_tokens")
+
+
+class SlotStates:
+    """The state tensors [slots, ...] of a cache on the device, whose slots are set to zero in one launch."""
+
+    def __init__(self, tensors: Sequence[torch.Tensor]):
+        self.tensors = [tensor for tensor in tensors if tensor.numel() > 0]
+        self.slots = min((tensor.shape[0] for tensor in self.tensors), default=0)
+        for tensor in self.tensors:
+            _need(tensor.is_cuda and tensor.is_contiguous(), "zero_slot: states must be contiguous tensors on the device")
+        count = len(self.tensors)
+        self._bases = (_c_ptr * count)(*[tensor.data_ptr() for tensor in self.tensors])
+        self._bytes = (_c_long * count)(*[tensor[0].numel() * tensor.element_size() for tensor in self.tensors])
+
+    def zero(self, slot: int) -> None:
+        if not self.tensors:
+            return
+        _need(0 <= slot < self.slots, "zero_slot: no such slot")
+        with torch.cuda.device(self.tensors[0].device):
+            _check(_fn("common", "mi_zero_slot")(ctypes.addressof(self._bases), ctypes.addressof(self._bytes),
+                                                 len(self.tensors), int(slot), _stream()), "zero_slot")
 
 
 def add_rmsnorm(h: torch.Tensor, deltas: Sequence[torch.Tensor], weight: torch.Tensor, eps: float,

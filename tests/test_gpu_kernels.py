@@ -1744,3 +1744,19 @@ def test_prefill_attention_finds_far_keys_and_edges(ops):
             position = length - T + row
             hit = (out.float().cpu()[row] - expected).abs().max() < 1e-2
             assert hit == (chosen <= position), f"key {chosen}, query at {position}"
+
+
+@pytest.mark.parametrize("count", [1, 3, 121])
+def test_zero_slot_clears_one_slot_of_every_tensor_and_nothing_beside_it(ops, count):
+    """Slots of odd sizes (bytes before and behind the 16-byte pieces), of one element, and of more than a block's
+    share; more tensors than one launch takes."""
+    shapes = [((5, 3), torch.bfloat16), ((7,), torch.uint8), ((1,), torch.float32), ((40, 1027), torch.float32),
+              ((64,), torch.float32), ((), torch.bfloat16)]
+    tensors = [torch.ones((4,) + shapes[i % len(shapes)][0], dtype=shapes[i % len(shapes)][1], device=DEV) for i in range(count)]
+    states = ops.SlotStates(tensors)
+    for slot in (1, 3):
+        states.zero(slot)
+        for tensor in tensors:
+            assert (tensor[slot] == 0).all() and (tensor[0] == 1).all() and (tensor[2] == 1).all()
+    with pytest.raises(ops.KernelError):
+        states.zero(4)
