@@ -1760,3 +1760,70 @@ def test_zero_slot_clears_one_slot_of_every_tensor_and_nothing_beside_it(ops, co
             assert (tensor[slot] == 0).all() and (tensor[0] == 1).all() and (tensor[2] == 1).all()
     with pytest.raises(ops.KernelError):
         states.zero(4)
+
+
+def within_rounding(got, want, dtype):
+    """One rounding of the result (half an ulp of bfloat16, 2^-9 of the value) and float32 sums of up to 8,192 terms in
+    another order (8192^0.5 ulps of 2^-24, 5e-6) taken through a quotient and a product."""
+    got, want = got.double().cpu(), want.double()
+    assert got.shape == want.shape and torch.isfinite(got).all()
+    share = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) + 2e-5
+    assert ((got - want).abs() <= share * want.abs() + 2e-5).all(), float((got - want).abs().max())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [3, 513])
+@pytest.mark.parametrize("d", [4, 1020, 1022, 1024, 1028, 2052, 4100, 8192, 8196])
+def test_scaled_rmsnorm_in_pieces_of_four(ops, dtype, T, d):
+    h, scale, weight = rand(T, d, seed=1), rand(d, seed=2), rand(d, seed=3)
+    delta = rand(T, d, seed=4, dtype=dtype)
+    stream = h.double() + scale.double() * delta.double()
+    want = stream / torch.sqrt(stream.square().mean(-1, keepdim=True) + 1e-5) * weight.double()
+    dh, dd, ds, dw = gpu(h, delta, scale, weight)
+    out = torch.empty(T, d, dtype=dtype, device=DEV)
+    rows = i32([T - 1, 0, T - 1]).to(DEV)
+    gathered = torch.empty(3, d, dtype=dtype, device=DEV)
+    ops.add_scaled_rmsnorm(dh, dd, ds, dw, 1e-5, gathered, rows=rows)
+    assert torch.equal(dh.cpu(), h)
+    ops.add_scaled_rmsnorm(dh, dd, ds, dw, 1e-5, out)
+    within_rounding(dh, stream, torch.float32)
+    within_rounding(out, want, dtype)
+    within_rounding(gathered, want[[T - 1, 0, T - 1]], dtype)
+    dh.copy_(h)
+    ops.add_scaled_rmsnorm(dh, dd, ds, dw, 1e-5, None)
+    within_rounding(dh, stream, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [3, 513])
+@pytest.mark.parametrize("width, ld", [(8, 8), (2044, 2048), (2048, 2048), (2056, 2064), (2048, 2052), (8200, 8200), (32776, 32776)])
+def test_polynorm_with_the_row_in_registers(ops, dtype, T, width, ld):
+    z = rand(T, ld, seed=1, dtype=dtype)[:, :width]
+    c = torch.tensor([0.7, -0.4, 0.25, 0.1])
+    x = z.double()
+    rms = lambda p: p / torch.sqrt(p.square().mean(-1, keepdim=True) + 1e-5)
+    want = 0.7 * rms(x) - 0.4 * rms(x ** 2) + 0.25 * rms(x ** 3) + 0.1
+    on = torch.empty(T, ld, dtype=dtype, device=DEV)
+    on[:, :width] = z.to(DEV)
+    out = torch.full((T, ld), 7.0, dtype=dtype, device=DEV)
+    ops.polynorm(on[:, :width], c.to(DEV), 1e-5, out[:, :width])
+    assert (out[:, width:] == 7.0).all()
+    within_rounding(out[:, :width], want, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("activation", ["silu", "sigmoid"])
+@pytest.mark.parametrize("T, H, dv, gap", [(1, 1, 32, 0), (7, 3, 64, 8), (129, 5, 128, 4), (33, 3, 256, 0), (5, 3, 64, 2), (5, 3, 60, 0)])
+def test_head_norms_in_pieces_of_four(ops, dtype, activation, T, H, dv, gap):
+    width = H * dv
+    raw, gate, weight = rand(T, width, seed=1), rand(T, width + gap, seed=2, dtype=dtype), rand(width, seed=3)
+    heads = raw.double().unflatten(1, (H, dv))
+    z = gate[:, gap:].double()
+    normed = (heads / torch.sqrt(heads.square().mean(-1, keepdim=True) + 1e-5)).flatten(1)
+    want = normed * (z * torch.sigmoid(z) if activation == "silu" else torch.sigmoid(z))
+    d_raw, d_gate, d_weight = gpu(raw, gate, weight)
+    for one, expected in ((None, want), (d_weight, want * weight.double())):
+        out = torch.full((T, width + gap), 7.0, dtype=dtype, device=DEV)
+        ops.head_norm_gate(d_raw, d_gate[:, gap:], one, H, 1e-5, activation, out[:, gap:])
+        assert (out[:, :gap] == 7.0).all()
+        within_rounding(out[:, gap:], expected, dtype)
