@@ -327,10 +327,9 @@ extern "C" int mi_conv_step(void* u, int dtype, long ld, int col_offset, int M, 
 // elements (1, 2, 4 or 8: the smallest number that covers N; one load where alignment allows); 256/R rows per block.
 //
 // The recurrence is serial in the tokens, so what a token costs is what its step waits for.  The tokens of a
-// lane come in blocks of up to 16: a block's B, C, x, delta and decay are asked for two blocks ahead by all threads
+// lane come in blocks of up to 64: a block's B, C, x, delta and decay are asked for two blocks ahead by all threads
 // of the workgroup, a few elements each and each element once a workgroup, laid in LDS one block ahead, and read
-// from there into the registers of the threads that use them, eight tokens (16 / PER) at a time before the first of
-// them; softplus and the exponential are taken once a token and head, by a small kernel ahead of the scan.  What
+// from there into the registers of the threads that use them, a few tokens at a time before the first of them; softplus and the exponential are taken once a token and head, by a small kernel ahead of the scan.  What
 // the R lanes of a row add up for a token's output is added in registers (scan_lanes_sum: a butterfly over the
 // lanes in which both partners of every step add the same two numbers), the outputs of a block wait in a register
 // of the lane with the token's number and leave with one store a block.  Every token goes through the same
@@ -338,9 +337,14 @@ extern "C" int mi_conv_step(void* u, int dtype, long ld, int col_offset, int M, 
 // nothing staged, few registers, many workgroups a compute unit): a step of one token and a prompt of thousands
 // give a position the same bits.
 #define SCAN_MAX_PER_THREAD 8
-#define SCAN_BLOCK_ELEMENTS 16      // tokens of a run that goes without a condition, times PER
-#define SCAN_BLOCK_TOKENS 16        // tokens of a block that a workgroup stages, at most
-#define SCAN_THREAD_PIECES 4        // loads of four elements of B|C that a thread sends for, a block
+#define SCAN_BLOCK_ELEMENTS 16      // tokens of a run that goes without a condition, times PER, where they are summed one by one
+// Tokens of a block that a workgroup stages, at most (a row narrower than a wave keeps a block's outputs in 16 lanes), and
+// loads of four elements of B|C that a thread sends for, a block.  512 tokens, 24 heads of 64 with 128 states: 60 us (72
+// with the tokens' sums one by one and B and C apart in LDS), with 256 states and heads of 128: 113 (228).  Eight loads a
+// thread (blocks of 32 tokens) gain 5 us there and lose 3 on every lane of a few tokens; asking LDS for a run's operands
+// while the run before is worked on costs registers and gains nothing.
+#define SCAN_BLOCK_TOKENS(eight) ((eight) ? 64 : 16)
+#define SCAN_THREAD_PIECES 4
 
 template <int CONTROL, int ROW_MASK>
 __device__ __forceinline__ float scan_dpp(float v) {
@@ -348,21 +352,53 @@ __device__ __forceinline__ float scan_dpp(float v) {
 }
 
 // The sum of a value over the R lanes of a row (R a power of two, rows at multiples of R), in the last 16 lanes of
-// the row (in all of them if R <= 16), the same bits in each of those: within 16 lanes step k adds what the lane's
-// group of 2^k lanes holds to what its neighbour group holds, and the lanes of both groups add the same two numbers
+// the row (in all of them if R <= 16 or R = 64), the same bits in each of those: within 16 lanes step k adds what the
+// lane's group of 2^k lanes holds to what its neighbour group holds, and the lanes of both groups add the same two numbers
 // (neighbours within a quad by quad permutation, then the mirrors of half a row and of a row of 16: after the steps
-// before, every lane of a group holds the group's sum, so any lane of the neighbour group will do); the sums of the
-// 16-lane rows then travel upwards, the last lane of a row to every lane of the next, and of the first two rows to
-// the last two: ((s3 + s2) + (s1 + s0)) in a row of 64.  All in the vector pipeline, nothing through LDS.
+// before, every lane of a group holds the group's sum, so any lane of the neighbour group will do); of a row of 32
+// the last lane of the first 16 adds to the others.  A row of 64 begins from afar: lanes 32 apart, 16, 8, then the
+// neighbours 1, 2 and 4 apart, an order in which scan_eight_sums below can add up eight tokens at once.
+// All in the vector pipeline, nothing through LDS.
+__device__ __forceinline__ float scan_halves_sum(float low, float high) {      // lanes below 32: the sums of `low`, the others: of `high`
+  const auto swapped = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, low), __builtin_bit_cast(unsigned, high), false, false);
+  const unsigned first = swapped[0], second = swapped[1];      // (a bit cast of an element itself takes the first one)
+  return __builtin_bit_cast(float, first) + __builtin_bit_cast(float, second);
+}
+__device__ __forceinline__ float scan_rows_sum(float even, float odd) {        // even rows of 16 lanes: the sums of `even`, the others: of `odd`
+  const auto swapped = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, even), __builtin_bit_cast(unsigned, odd), false, false);
+  const unsigned first = swapped[0], second = swapped[1];      // (a bit cast of an element itself takes the first one)
+  return __builtin_bit_cast(float, first) + __builtin_bit_cast(float, second);
+}
+
 template <int R>
 __device__ __forceinline__ float scan_lanes_sum(float v) {
+  if (R == 64) {
+    v = scan_halves_sum(v, v);
+    v = scan_rows_sum(v, v);
+    v += scan_dpp<0x128, 0xf>(v);                     // row_ror 8
+  }
   if (R >= 2) v += scan_dpp<0xB1, 0xf>(v);            // quad_perm [1, 0, 3, 2]
   if (R >= 4) v += scan_dpp<0x4E, 0xf>(v);            // quad_perm [2, 3, 0, 1]
   if (R >= 8) v += scan_dpp<0x141, 0xf>(v);           // row_half_mirror
-  if (R >= 16) v += scan_dpp<0x140, 0xf>(v);          // row_mirror
-  if (R >= 32) v += scan_dpp<0x142, 0xa>(v);          // row_bcast15 into rows 1 and 3 (the others add 0)
-  if (R >= 64) v += scan_dpp<0x143, 0xc>(v);          // row_bcast31 into rows 2 and 3
+  if (R >= 16 && R < 64) v += scan_dpp<0x140, 0xf>(v);          // row_mirror
+  if (R == 32) v += scan_dpp<0x142, 0xa>(v);          // row_bcast15 into rows 1 and 3 (the others add 0)
   return v;
+}
+
+// The sums over a row of 64 lanes of eight values at once, value j in lanes 8 j to 8 j + 7: every step halves the number of
+// registers as well as the lanes that a value is spread over (18 instructions, where eight sums one by one take 80), and
+// adds the pairs that scan_lanes_sum<64> adds: the same bits.
+__device__ __forceinline__ float scan_eight_sums(const float (&v)[8], bool upper_eight) {
+  float far[4], near[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) far[i] = scan_halves_sum(v[i], v[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) near[i] = scan_rows_sum(far[i], far[i + 2]);
+  float sum = (upper_eight ? near[1] : near[0]) + scan_dpp<0x128, 0xf>(upper_eight ? near[0] : near[1]);
+  sum += scan_dpp<0xB1, 0xf>(sum);
+  sum += scan_dpp<0x4E, 0xf>(sum);
+  sum += scan_dpp<0x141, 0xf>(sum);
+  return sum;
 }
 
 // A barrier of the workgroup for what went through LDS, and nothing else.  __syncthreads() also waits for every load
@@ -382,7 +418,8 @@ ssm_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt
                 float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ slot_ids,
                 int H, int P, int N, int G, int block_tokens, const float* __restrict__ delta_decay,
                 float* __restrict__ y, long y_ld) {
-  constexpr int TB = PER == 1 ? SCAN_BLOCK_ELEMENTS / 2 : SCAN_BLOCK_ELEMENTS / PER;    // tokens of a run that goes without a condition
+  constexpr bool EIGHT = R == WAVE && PER <= 4;        // the sums of eight tokens are added up together
+  constexpr int TB = EIGHT || PER == 1 ? 8 : SCAN_BLOCK_ELEMENTS / PER;    // tokens of a run that goes without a condition
   constexpr int ROWS = 256 / R;                        // rows of a workgroup
   constexpr int SUM_LANES = R < 16 ? R : 16;           // the last lanes of a row, which hold its sums
   constexpr int FIRST_SUM_LANE = R - SUM_LANES;
@@ -445,81 +482,98 @@ ssm_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt
     // them (which a wave can only state for all it has asked of memory at once, stores included) never meets a
     // load or a store of a moment ago.  Every element comes in once a workgroup: the rows of a head, and the
     // heads of a group, read the same B and C.
-    const int row_floats = 2 * N;
-    float* b_l = staged_l;                                      // [2][block_tokens][2 N]: B then C of a token
+    // a token's B and C as its lanes read them: PER elements of B, then the PER of C, lane after lane
+    const int row_floats = 2 * PER * ((N + PER - 1) / PER);
+    auto place = [&](int n) { return n / PER * 2 * PER + n % PER; };       // of B's element n; C's lies PER further
+    float* b_l = staged_l;                                      // [2][block_tokens][row_floats]
     float* x_l = b_l + 2 * block_tokens * row_floats;           // [2][block_tokens][ROWS]
     float* dd_l = x_l + 2 * block_tokens * ROWS;                // [2][block_tokens][2]: delta, decay
     typedef T pieces __attribute__((ext_vector_type(4)));
-    const int pieces_a_row = (row_floats + 3) / 4;
+    const int pieces_a_row = (2 * N + 3) / 4;
     const bool whole_rows = N == R * PER;                       // no lane of a row is idle
-    float staged_bc[SCAN_THREAD_PIECES][4], staged_x = 0.f, staged_dd = 0.f;
-    // where this thread's pieces lie in a block (the same for every block: worked out once, a division each)
-    int piece_token[SCAN_THREAD_PIECES], piece_col[SCAN_THREAD_PIECES];
+    constexpr int PIECES = SCAN_THREAD_PIECES;
+    float staged_bc[PIECES][4], staged_x = 0.f, staged_dd = 0.f;
+    // where this thread's pieces lie in a block, in memory from the block's first row on and in LDS (the same for
+    // every block: worked out once, a division each).  A piece past the block is its last token's once more: two
+    // threads then move the same numbers to the same place.
+    int piece_token[PIECES], piece_col[PIECES], piece_from[PIECES], piece_to[PIECES];
 #pragma unroll
-    for (int j = 0; j < SCAN_THREAD_PIECES; ++j) {
+    for (int j = 0; j < PIECES; ++j) {
       const int index = tid + j * 256;
-      piece_token[j] = index / pieces_a_row;
-      piece_col[j] = (index - piece_token[j] * pieces_a_row) * 4;
+      const int token = index / pieces_a_row;
+      const int col = (index - token * pieces_a_row) * 4;
+      piece_token[j] = min(token, block_tokens - 1);
+      piece_col[j] = col;
+      piece_from[j] = piece_token[j] * (int)xbc_ld + (int)(col < N ? b_col + col : c_col + (col - N));
+      piece_to[j] = piece_token[j] * row_floats + (col < N ? place(col) : place(col - N) + PER);
     }
     const int x_token = tid / ROWS, x_row = tid % ROWS;
-    // this thread's share of block `block` of the lane into its registers (nothing if the lane has no such block)
+    // this thread's share of block `block` of the lane into its registers (nothing if the lane has no such block); of a
+    // short block the rows behind its last one repeat that one, and nobody reads them
     auto fetch = [&](int block) {
       const long t0 = t_begin + (long)block * block_tokens;
       const int count = (int)max(0L, min((long)block_tokens, t_end - t0));
       if (count <= 0) return;
+      const T* rows = xbc + t0 * xbc_ld;
 #pragma unroll
-      for (int j = 0; j < SCAN_THREAD_PIECES; ++j) {
-        const int token = min(piece_token[j], count - 1);           // a piece past the block reads its last token, unused
-        const int col = piece_col[j];
+      for (int j = 0; j < PIECES; ++j) {
         if (VECTORS) {
-          // B and C of a group lie apart in a row: columns N .. 2 N of the staged row are C
-          const pieces four = *reinterpret_cast<const pieces*>(xbc + (t0 + token) * xbc_ld + (col < N ? b_col + col : c_col + (col - N)));
+          int from = piece_from[j];
+          if (count < block_tokens) from -= max(0, piece_token[j] - (count - 1)) * (int)xbc_ld;
+          const pieces four = *reinterpret_cast<const pieces*>(rows + from);
 #pragma unroll
           for (int i = 0; i < 4; ++i) staged_bc[j][i] = to_float<T>(four[i]);
         } else {
+          const T* row = rows + min(piece_token[j], count - 1) * xbc_ld;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {                         // element by element: a piece may straddle B and C
-            const int at = min(col + i, row_floats - 1);
-            staged_bc[j][i] = to_float(xbc[(t0 + token) * xbc_ld + (at < N ? b_col + at : c_col + (at - N))]);
+            const int at = min(piece_col[j] + i, 2 * N - 1);
+            staged_bc[j][i] = to_float(row[at < N ? b_col + at : c_col + (at - N)]);
           }
         }
       }
       const int row = p0 + x_row;
-      staged_x = row < P ? to_float(xbc[(t0 + min(x_token, count - 1)) * xbc_ld + (long)head * P + row]) : 0.f;
-      staged_dd = delta_decay[((t0 + min(tid >> 1, count - 1)) * H + head) * 2 + (tid & 1)];
+      staged_x = row < P ? to_float(rows[min(x_token, count - 1) * xbc_ld + (long)head * P + row]) : 0.f;
+      staged_dd = delta_decay[(t0 * H + head) * 2 + (long)min(tid >> 1, count - 1) * H * 2 + (tid & 1)];
     };
     // this thread's registers (block `block`) into LDS
     auto lay_down = [&](int block) {
-      const long t0 = t_begin + (long)block * block_tokens;
-      const int count = (int)max(0L, min((long)block_tokens, t_end - t0));
-      if (count <= 0) return;
+      if (t_begin + (long)block * block_tokens >= t_end) return;
       const int phase = block & 1;
       float* rows_l = b_l + phase * block_tokens * row_floats;
 #pragma unroll
-      for (int j = 0; j < SCAN_THREAD_PIECES; ++j) {
-        const int token = piece_token[j];
-        const int col = piece_col[j];
-        if (token < count) {
-          float* to = rows_l + token * row_floats + col;
-          if (VECTORS) {
-            *reinterpret_cast<float4*>(to) = make_float4(staged_bc[j][0], staged_bc[j][1], staged_bc[j][2], staged_bc[j][3]);
+      for (int j = 0; j < PIECES; ++j) {
+        if (VECTORS) {                                          // four elements of B or four of C (N is a multiple of 4)
+          float* four = rows_l + piece_to[j];
+          if (PER >= 4) {
+            *reinterpret_cast<float4*>(four) = make_float4(staged_bc[j][0], staged_bc[j][1], staged_bc[j][2], staged_bc[j][3]);
+          } else if (PER == 2) {
+            *reinterpret_cast<float2*>(four) = make_float2(staged_bc[j][0], staged_bc[j][1]);
+            *reinterpret_cast<float2*>(four + 4) = make_float2(staged_bc[j][2], staged_bc[j][3]);
           } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (col + i < row_floats) to[i] = staged_bc[j][i];
+            for (int i = 0; i < 4; ++i) four[2 * i] = staged_bc[j][i];
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int at = piece_col[j] + i;
+            if (at < 2 * N) rows_l[piece_token[j] * row_floats + (at < N ? place(at) : place(at - N) + PER)] = staged_bc[j][i];
           }
         }
       }
-      if (x_token < count) x_l[phase * block_tokens * ROWS + tid] = staged_x;
-      if (tid < 2 * count) dd_l[phase * block_tokens * 2 + tid] = staged_dd;
+      if (x_token < block_tokens) x_l[phase * block_tokens * ROWS + tid] = staged_x;
+      if (tid < 2 * block_tokens) dd_l[phase * block_tokens * 2 + tid] = staged_dd;
     };
     // the outputs of the block before: token i of the block waits in the i-th of the row's lanes that hold sums
-    // (block_tokens <= SUM_LANES)
+    // (block_tokens <= SUM_LANES), where eight tokens are added up together in the (i / 8)-th of the eight lanes from 8 (i % 8) on
+    auto kept_token = [&]() { return EIGHT ? (r & 7) * 8 + r / 8 : r - FIRST_SUM_LANE; };
     float kept = 0.f;
     long kept_t0 = 0;
     int kept_count = 0;
     auto store_kept = [&]() {
-      if (r >= FIRST_SUM_LANE && r - FIRST_SUM_LANE < kept_count && active) y_mine[(kept_t0 + r - FIRST_SUM_LANE) * y_ld] = kept;
+      const int token = kept_token();
+      if (token >= 0 && token < kept_count && active) y_mine[(kept_t0 + token) * y_ld] = kept;
     };
     fetch(0);
     lay_down(0);
@@ -539,7 +593,7 @@ ssm_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt
       const float* rows_l = b_l + phase * block_tokens * row_floats;
       const float* x_now = x_l + phase * block_tokens * ROWS + row_in_block;
       const float* dd_now = dd_l + phase * block_tokens * 2;
-      const float* mine_l = rows_l + min(r * PER, N - PER > 0 ? N - PER : 0);    // this thread's columns of B (C: N further)
+      const float* mine_l = rows_l + r * 2 * PER;                 // this thread's elements of B and C, in rows without idle lanes
       // runs of TB tokens of a row whose lanes all hold PER elements go without a condition: straight code that
       // asks LDS for the run's operands at once; what is left of a block, and rows with idle lanes, take the
       // guarded loop
@@ -552,29 +606,56 @@ ssm_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt
             const float2 delta_and_decay = *reinterpret_cast<const float2*>(dd_now + (done + token) * 2);
             decay[token] = delta_and_decay.y;
             dx[token] = delta_and_decay.x * x_now[(done + token) * ROWS];
+            const float* from = mine_l + (done + token) * row_floats;
+            if (PER == 1) {
+              const float2 both = *reinterpret_cast<const float2*>(from);
+              b[token][0] = both.x;
+              c[token][0] = both.y;
+            } else if (PER == 2) {
+              const float4 both = *reinterpret_cast<const float4*>(from);
+              b[token][0] = both.x;
+              b[token][PER - 1] = both.y;
+              c[token][0] = both.z;
+              c[token][PER - 1] = both.w;
+            } else {
 #pragma unroll
-            for (int i = 0; i < PER; ++i) {
-              b[token][i] = mine_l[(done + token) * row_floats + i];
-              c[token][i] = mine_l[(done + token) * row_floats + N + i];
+              for (int i = 0; i < PER; i += 4) {
+                const float4 of_b = *reinterpret_cast<const float4*>(from + i);
+                const float4 of_c = *reinterpret_cast<const float4*>(from + PER + i);
+                const float bs[4] = {of_b.x, of_b.y, of_b.z, of_b.w}, cs[4] = {of_c.x, of_c.y, of_c.z, of_c.w};
+#pragma unroll
+                for (int j = 0; j < 4 && i + j < PER; ++j) {
+                  b[token][i + j] = bs[j];
+                  c[token][i + j] = cs[j];
+                }
+              }
             }
           }
-          // the x of the token whose output this lane keeps (any token of the run for the other lanes)
-          const int my_token = done + ((r - FIRST_SUM_LANE - done) & (TB - 1));
+          // the token of the run whose sum this lane keeps, and its x
+          const int my_token = done + (EIGHT ? r / 8 : (r - FIRST_SUM_LANE - done) & (TB - 1));
           const float my_x = x_now[my_token * ROWS];
+          float partial[TB];
           float my_sum = 0.f;
 #pragma unroll
           for (int token = 0; token < TB; ++token) {
-            float partial = 0.f;
+            partial[token] = 0.f;
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
               const float next_s = fmaf(decay[token], s[i], dx[token] * b[token][i]);
               s[i] = next_s;
-              partial = fmaf(next_s, c[token][i], partial);
+              partial[token] = fmaf(next_s, c[token][i], partial[token]);
             }
-            const float sum = scan_lanes_sum<R>(partial);
-            my_sum = my_token == done + token ? sum : my_sum;
+            if constexpr (!EIGHT) {
+              const float sum = scan_lanes_sum<R>(partial[token]);
+              my_sum = my_token == done + token ? sum : my_sum;
+            }
           }
-          kept = (r >= FIRST_SUM_LANE + done && r < FIRST_SUM_LANE + done + TB) ? fmaf(skip, my_x, my_sum) : kept;
+          if constexpr (EIGHT) {
+            my_sum = scan_eight_sums(partial, (r & 8) != 0);
+            if ((r & 7) == done / TB) kept = fmaf(skip, my_x, my_sum);
+          } else {
+            kept = (r >= FIRST_SUM_LANE + done && r < FIRST_SUM_LANE + done + TB) ? fmaf(skip, my_x, my_sum) : kept;
+          }
         }
       }
       for (int token = done; token < count; ++token) {
@@ -586,13 +667,13 @@ ssm_scan_kernel(const T* __restrict__ xbc, long xbc_ld, const T* __restrict__ dt
         for (int i = 0; i < PER; ++i) {
           const int n = r * PER + i;
           if (n < N) {
-            const float next_s = fmaf(decay, s[i], dx * rows_l[token * row_floats + n]);
+            const float next_s = fmaf(decay, s[i], dx * rows_l[token * row_floats + place(n)]);
             s[i] = next_s;
-            partial = fmaf(next_s, rows_l[token * row_floats + N + n], partial);
+            partial = fmaf(next_s, rows_l[token * row_floats + place(n) + PER], partial);
           }
         }
         const float out = fmaf(skip, x, scan_lanes_sum<R>(partial));
-        kept = r == FIRST_SUM_LANE + token ? out : kept;
+        kept = kept_token() == token ? out : kept;
       }
       kept_t0 = t0;
       kept_count = count;
@@ -661,12 +742,13 @@ extern "C" int mi_ssm_scan(const void* xbc, int dtype, long xbc_ld, const void* 
   if (!single && (!delta_decay || tokens <= 0)) return ERR_BAD_ARGUMENT;
   // tokens of a block: no more than R (a block's x values, one a row and token, are one a thread, and its outputs
   // wait one a lane of the row), and B and C of a block no more than SCAN_THREAD_PIECES loads of four elements a thread
-  int block_tokens = SCAN_BLOCK_TOKENS;
+  const bool eight = R == WAVE && per <= 4;
+  int block_tokens = SCAN_BLOCK_TOKENS(eight);
   if (block_tokens > R) block_tokens = R;
   while (block_tokens > 1 && (long)block_tokens * ((2 * N + 3) / 4) > 256L * SCAN_THREAD_PIECES) block_tokens /= 2;
-  const size_t bytes = single ? 0 : 2 * (size_t)block_tokens * (2 * N + rows_per_block + 2) * sizeof(float);
+  const size_t bytes = single ? 0 : 2 * (size_t)block_tokens * (2 * per * ((N + per - 1) / per) + rows_per_block + 2) * sizeof(float);
   // four elements a load: every head's and group's columns of B and C start at multiples of 4
-  const bool vectors = !single && N % 4 == 0 && xbc_ld % 4 == 0 && ((long)H * P) % 4 == 0 &&
+  const bool vectors = !single && N % 4 == 0 && xbc_ld % 4 == 0 && ((long)H * P) % 4 == 0 && xbc_ld < (1L << 24) &&
                        ((uintptr_t)xbc % (dtype == DT_F32 ? 16 : 8)) == 0;
   if (!single) {
     const long total = tokens * H;

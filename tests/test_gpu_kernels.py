@@ -1827,3 +1827,31 @@ def test_head_norms_in_pieces_of_four(ops, dtype, activation, T, H, dv, gap):
         ops.head_norm_gate(d_raw, d_gate[:, gap:], one, H, 1e-5, activation, out[:, gap:])
         assert (out[:, :gap] == 7.0).all()
         within_rounding(out[:, gap:], expected, dtype)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N", [17, 40, 64, 100, 128, 200, 256, 260, 512])
+def test_scan_gives_the_same_bits_however_its_tokens_are_cut(ops, dtype, N):
+    """Lanes whose blocks and runs of eight tokens end at, before and behind a cut, and single tokens: rows of 32 and of 64
+    lanes, with and without idle lanes, one to eight states a lane."""
+    H, P, G, T = 2, 9, 1, 83
+    E = H * P
+    xbc, dt = rand(T, E + 2 * N, seed=1, dtype=dtype), rand(T, H, seed=2, dtype=dtype)
+    dt_bias, A, D = rand(H, seed=3), -torch.tensor([0.05, 1.0]), rand(H, seed=4)
+    start = rand(1, H, P, N, seed=5, scale=0.5)
+    want_y, want_state = torch.empty(T, E), start.clone()
+    ref_ops.ssm_scan(xbc, dt, dt_bias, A, D, want_state, i32([0, T]), i32([0]), G, want_y)
+    on = gpu(xbc, dt, dt_bias, A, D)
+    slot = i32([0]).to(DEV)
+    results = []
+    for sizes in ([83], [8, 16, 32, 27], [7, 1, 9, 15, 17, 34], [1] * 83, [64, 19]):
+        state, y, first = start.to(DEV), torch.full((T, E), float("nan"), device=DEV), 0
+        for size in sizes:
+            rows = slice(first, first + size)
+            ops.ssm_scan(on[0][rows], on[1][rows], *on[2:], state, i32([0, size]).to(DEV), slot, G, y[rows], size)
+            first += size
+        results.append((y, state))
+    for y, state in results[1:]:
+        assert torch.equal(y, results[0][0]) and torch.equal(state, results[0][1])
+    close(results[0][0], want_y, torch.float32, max(1.0, want_y.abs().max().item()))
+    close(results[0][1], want_state, torch.float32, max(1.0, want_state.abs().max().item()))
