@@ -167,6 +167,24 @@ extern "C" int mi_zero_slot(void* const* bases, const long* bytes, int count, lo
   return 0;
 }
 
+// ---------------------------------------------------------------- a known length of nothing
+// One wave that is busy for `microseconds` by the constant 100 MHz clock (and for so many rounds at most, whatever the
+// clock says): by two of them the host finds out whether two streams run beside each other.
+__global__ void wait_kernel(int microseconds) {
+  const unsigned long long begin = wall_clock64();
+  for (int round = 0; round < 100 * microseconds; ++round) {
+    if (wall_clock64() - begin >= 100ull * microseconds) return;
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+extern "C" int mi_wait(int microseconds, hipStream_t stream) {
+  if (microseconds <= 0 || microseconds > 10000) return ERR_BAD_ARGUMENT;
+  wait_kernel<<<1, WAVE, 0, stream>>>(microseconds);
+  RETURN_IF_LAUNCH_FAILED();
+  return 0;
+}
+
 // ---------------------------------------------------------------- add + rmsnorm
 // For each processed row r:  v = h[r] (+ factor0 * delta0[r]) (+ factor1 * delta1[r]);  if update: h[r] = v;
 // out[i] = v / sqrt(mean(v^2) + eps) * weight.

@@ -27,9 +27,10 @@ from ..config.spec import ConfigError
 from ..kernels import build as kernel_build
 from ..kernels import ops
 from ..parts.base import BuildContext
+from ..parts.block import OVERLAP_MIN_TOKENS
 from ..weights.loader import WeightSource, bind
 from .context import Lane, LoweredLanes, apply_feeds, build_step_context, longest_context, lower_lanes
-from .graphs import DecodeGraphs
+from .graphs import BESIDE_CANDIDATES, SINGLES, DecodeGraphs, replayed_beside
 from .model import DecoderModel
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "fp32": torch.float32,
@@ -61,15 +62,15 @@ def resolve_dtype(dtype) -> torch.dtype:
     return _DTYPES[dtype]
 
 
-# A step with portions of prompts beside several single decoded tokens runs as two batches (see
+# A step with portions of prompts beside several single decoded tokens runs as two batches side by side (see
 # ``Engine._run_in_two``) when the single tokens cost more as part of the portions' batch than as a batch of their
 # own.  As part of it every one of them is a prompt of one token to the prompt kernels (beside 2,048 prompt tokens
 # of the 0.5B shape, 8 decoded tokens cost 2.7 ms and 63 cost 13); a batch of their own reads every weight once
-# more and pays its dependent kernels.  Both depend on the model and on the GPU, so the clock decides when the
+# more and shares the GPU with the portions.  Both depend on the model and on the GPU, so the clock decides when the
 # first step that could be split comes (``DecodeGraphs.measure_split``): from so many single tokens on that they
-# cost, beside the portions, what a batch of their own costs (the 0.5B shape: 17 beside a portion of 256 tokens, 9
-# beside one of 2,048; eight layers of the 7B shape: 20 and 7; a third of a second for the three graphs).  Without a clock (no graphs, or ``measured_paths=False``) a step
-# is split from SPLIT_FROM_LANES single tokens on, which is also the fewest the clock can say.
+# cost, as part of the portions' batch, what a batch of their own adds to the portions beside it (a third of a second
+# for the three graphs).  Without a clock (no graphs, or ``measured_paths=False``) a step is split from SPLIT_FROM_LANES
+# single tokens on, which is also the fewest the clock can say.
 SPLIT_FROM_LANES = 4
 SPLIT_NEVER = 1 << 30
 # A step of more single decoded tokens than the skinny kernels take rows runs as two halves at once, each a
@@ -88,8 +89,8 @@ HALVES_MARGIN = 0.95
 
 def split_from_lanes(lane_share: Optional[float]) -> int:
     """From how many single decoded tokens beside portions of prompts on a step runs as two batches.
-    ``lane_share``: what one of them costs beside the portions, as a share of what a batch of them costs alone
-    (None: not measured)."""
+    ``lane_share``: what one of them costs as part of the portions' batch, as a share of what a batch of them adds to the
+    portions beside it (None: not measured)."""
     if lane_share is None:
         return SPLIT_FROM_LANES
     if lane_share <= 0:
@@ -145,7 +146,8 @@ class Engine:
         self.max_context = self.spec.max_context
         self.graphs = None
         self.graphs_beside = None                    # the graphs of the second half of a step that runs as two halves at once
-        self._beside = None                          # and the stream they are replayed on
+        self._beside = {}                            # and the streams they are replayed on, by the caller's stream
+        self._beside_portions = []                   # the streams among which the clock finds one for single tokens beside portions
         self._in_halves: Optional[bool] = None
         self.halves_share: Optional[float] = None
         # the pool bounds a request's length only where some layer keeps every key: a model whose attention
@@ -161,7 +163,7 @@ class Engine:
         the clock when it is first needed (or by ``warm_up``), where there is one."""
         if self._split_from_lanes is None:
             if self._measure_split and self.graphs is not None:
-                self.lane_share = self.graphs.measure_split()
+                self.lane_share = self.graphs.measure_split(self._candidates())
                 self._split_from_lanes = split_from_lanes(self.lane_share) if self.lane_share is not None else SPLIT_NEVER
             else:
                 self._split_from_lanes = split_from_lanes(None)
@@ -178,7 +180,7 @@ class Engine:
         if self._in_halves is None:
             self._in_halves = False
             if self._measure_split and self.graphs is not None:
-                self.halves_share = self.graphs.measure_halves()
+                self.halves_share = self.graphs.measure_halves(self._second_stream())
                 self._in_halves = self.halves_share is not None and self.halves_share < HALVES_MARGIN
         return self._in_halves
 
@@ -208,9 +210,7 @@ class Engine:
                 whole.append((lanes, tokens))
         done = self.graphs.warm_up(whole + [(first, first) for first, _ in halves], context)
         if halves:
-            if self.graphs_beside is None:
-                self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len)
-                self._beside = torch.cuda.Stream(device=self.device)
+            self._make_graphs_beside()
             done += self.graphs_beside.warm_up([(second, second) for _, second in halves], context)
         return done
 
@@ -338,6 +338,26 @@ class Engine:
             logits = self.model.forward(context, self.cache)
         return logits
 
+    def _second_stream(self) -> torch.cuda.Stream:
+        """The stream that a step's second half is queued on, beside the caller's: found by the clock when a caller's
+        stream first needs one."""
+        main = torch.cuda.current_stream(self.device)
+        if main.cuda_stream not in self._beside:
+            self._beside[main.cuda_stream] = ops.stream_beside(main)
+        return self._beside[main.cuda_stream]
+
+    def _candidates(self) -> list:
+        """The streams that the single tokens beside portions of prompts may be queued on."""
+        if not self._beside_portions:
+            self._beside_portions = [torch.cuda.Stream(device=self.device) for _ in range(BESIDE_CANDIDATES + 1)]
+        main = torch.cuda.current_stream(self.device)
+        return [stream for stream in self._beside_portions if stream != main][:BESIDE_CANDIDATES]
+
+    def _make_graphs_beside(self) -> None:
+        if self.graphs_beside is None:
+            apart = [self.graphs._capture_stream(SINGLES)]
+            self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len, apart)
+
     def _run_in_halves(self, lanes: Sequence[Lane]) -> torch.Tensor:
         """A step of many single decoded tokens as two halves at once: the second half's graph is replayed on a
         stream of its own, which starts behind everything queued so far (the tokens that lanes are fed from
@@ -345,34 +365,49 @@ class Engine:
         different requests, so they share no page and no slot but the scratch ones of their padding lanes, whose
         contents nobody reads; their graphs have memory pools of their own."""
         main = torch.cuda.current_stream(self.device)
-        if self.graphs_beside is None:
-            self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len)
-            self._beside = torch.cuda.Stream(device=self.device)
+        self._make_graphs_beside()
         half = (len(lanes) + 1) // 2
         first, second = list(lanes[:half]), list(lanes[half:])
         lowered_second = self.validate(second)
-        self._beside.wait_stream(main)
+        beside = self._second_stream()
         try:
-            with torch.cuda.stream(self._beside):
+            with replayed_beside(main, beside):
                 rows_second = self._run(second, lowered_second, self.graphs_beside)
             rows_first = self._run(first, self.validate(first))
         finally:
             # whatever happens, nothing queued behind this step (pages given back and used again among it) may
             # overtake what the second stream still has to do
-            main.wait_stream(self._beside)
+            main.wait_stream(beside)
         rows_second.record_stream(main)
         return torch.cat([rows_first, rows_second])
 
     def _run_in_two(self, lanes: Sequence[Lane], lowered: LoweredLanes, single: np.ndarray) -> torch.Tensor:
-        """A step that holds portions of prompts beside several single decoded tokens, as two batches one after
-        the other: the portions through the prompt kernels, the single tokens through the decode kernels.  (As
-        one batch the prompt kernels take every single token as a prompt of its own, a tile of the attention
-        kernel and a chunk of the scan each: 2,048 prompt tokens beside 63 decoded ones took 19.4 ms on the
-        0.5B shape, where the two batches take 6.3 and 3.1.)  The logits come back in the order of the lanes."""
-        parts = []
+        """A step that holds portions of prompts beside several single decoded tokens, as two batches side by side:
+        the portions through the prompt kernels, and on a second stream the single tokens through the graph of a decode
+        step, whose small kernels wait for each other most of their time (515 prompt tokens of the 0.5B shape beside 24 decoded
+        ones: 4.8 ms, 6.1 with one batch behind the other).  (As one batch the prompt kernels take every single token as
+        a prompt of its own, a tile of the attention kernel and a chunk of the scan each: 2,048 prompt tokens beside 63
+        decoded ones took 19.4 ms, where the two batches take 6.3 and 3.1.)  The batches belong to different requests,
+        and graphs of the two kinds share neither a memory pool nor a library's workspace.  (From OVERLAP_MIN_TOKENS single
+        tokens on, whose mixers may use a second stream themselves, the batches follow each other.)  The logits come
+        back in the order of the lanes."""
+        batches = []
         for chosen in (~single, single):
             members = [lane for lane, mine in zip(lanes, chosen) if mine]
-            parts.append(self._run(members, self.validate(members)))
+            batches.append((members, self.validate(members)))
+        portions, singles = batches
+        if self.graphs is None or len(singles[0]) >= OVERLAP_MIN_TOKENS:
+            parts = [self._run(*portions), self._run(*singles)]
+        else:
+            main = torch.cuda.current_stream(self.device)
+            beside = self.graphs.stream_beside(portions[0], portions[1], singles[1], self._candidates())
+            try:
+                with replayed_beside(main, beside):
+                    rows_of_singles = self._run(*singles)
+                parts = [self._run(*portions), rows_of_singles]
+            finally:
+                main.wait_stream(beside)               # as in ``_run_in_halves``
+            rows_of_singles.record_stream(main)
         # the rows of the two batches, back in the order of the lanes: runs of lanes of one kind are slices of that
         # kind's rows (no index travels to the device: that copy would wait for everything queued before it)
         pieces, cursor = [], [0, 0]

@@ -23,11 +23,12 @@ launches), and ``warm_up`` captures a list of them before the first request.
 from __future__ import annotations
 
 from collections import OrderedDict
+from contextlib import contextmanager
 from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
 
-from .context import Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
+from .context import _NO_LANES, Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
 
 
 def bucket_for(lanes: int) -> int:
@@ -62,16 +63,42 @@ def token_capacities(most: int) -> List[int]:
         value += max(16, power // (8 if value >= 1024 else 4))
 
 
+SINGLES, PORTIONS = "single tokens", "portions"          # kinds of captured steps
+
+
+# The runtime lays its streams on a few hardware queues (four by default), in turn, and what lies on one queue runs one
+# after the other.  A graph of a long portion runs its mixers on two queues, of which the second is the runtime's own
+# choice when the graph is made: of four streams made in a row some stand in the way of one of the two, and the clock
+# says which does not (515 prompt tokens of the 0.5B shape beside 24 decoded ones: 4.8 ms on two of four streams, 6.05 on
+# the others).
+BESIDE_CANDIDATES = 4
+
+
+@contextmanager
+def replayed_beside(main: torch.cuda.Stream, beside: torch.cuda.Stream):
+    """What is queued inside goes onto ``beside``, behind everything that ``main`` holds so far."""
+    beside.wait_stream(main)
+    with torch.cuda.stream(beside):
+        yield
+
+
 class DecodeGraphs:
-    def __init__(self, model, cache, device, max_seq_len: int):
+    def __init__(self, model, cache, device, max_seq_len: int, apart_from: Sequence[torch.cuda.Stream] = ()):
+        """``apart_from``: streams on which other graphs are recorded that are replayed beside these."""
         self.model = model
+        self.apart_from = tuple(apart_from)
         self.cache = cache
         self.device = device
         self.max_seq_len = max_seq_len
         self._graphs: Dict[tuple, tuple] = {}
         self._bucket_graphs: "OrderedDict[tuple, tuple]" = OrderedDict()
         self._seen: "OrderedDict[tuple, int]" = OrderedDict()
-        self._pool = None
+        # graphs of single tokens and graphs of portions are replayed beside each other (``Engine._run_in_two``): each
+        # kind has a memory pool of its own and is recorded on a stream of its own, by which the libraries keep
+        # their workspaces apart
+        self._pools: Dict[str, object] = {}
+        self._streams: Dict[str, torch.cuda.Stream] = {}
+        self._besides: Dict[tuple, Dict[int, torch.cuda.Stream]] = {}
         self.counts = {"decode_replays": 0, "bucket_replays": 0, "bucket_captures": 0, "bucket_eager": 0}
 
     # captured capacities kept; the least recently used one goes.  A capture costs about as much as thirty replays
@@ -128,18 +155,23 @@ class DecodeGraphs:
                     best = max(best, fill)
         return best if best >= tokens - tokens // 8 else tokens
 
-    def run_bucket(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[torch.Tensor]:
-        """Logits of a step with prompt portions from the captured graph of its capacity, or None when that
-        capacity has no graph (yet): the caller then launches the step kernel by kernel."""
+    def _bucket_key(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[tuple]:
+        """The capacity and context of the graph that such a step replays, or None where no graph can hold it."""
         capacity = self.capacity_for(len(lanes), int(lowered.lengths.sum()), int(lowered.want_counts.sum()))
         if capacity is None:
-            self.counts["bucket_eager"] += 1
             return None
         context = self.context_bucket(lowered, at_least=capacity[1])
         if context < capacity[1]:                           # the cache cannot hold a padding lane of that many tokens
+            return None
+        return capacity + (context,)
+
+    def run_bucket(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[torch.Tensor]:
+        """Logits of a step with prompt portions from the captured graph of its capacity, or None when that
+        capacity has no graph (yet): the caller then launches the step kernel by kernel."""
+        key = self._bucket_key(lanes, lowered)
+        if key is None:
             self.counts["bucket_eager"] += 1
             return None
-        key = capacity + (context,)
         entry = self._bucket_graphs.get(key)
         if entry is None:
             self._seen[key] = self._seen.get(key, 0) + 1
@@ -166,7 +198,8 @@ class DecodeGraphs:
         entry = self._capture(0, static, warm_runs=1)
         self.counts["bucket_captures"] += 1
         while len(self._bucket_graphs) >= self.BUCKET_GRAPHS:
-            self._bucket_graphs.popitem(last=False)
+            gone, _ = self._bucket_graphs.popitem(last=False)
+            self._besides.pop(gone, None)
         self._bucket_graphs[key] = entry
         return entry
 
@@ -193,17 +226,18 @@ class DecodeGraphs:
                 done.append(key)
         return done
 
-    def measure_split(self, prompt_tokens: int = 1024, singles: int = 16, replays: int = 5) -> Optional[float]:
-        """The clock's answer to what a single decoded token costs beside a portion of a prompt, in units of what
-        a batch of single tokens of its own costs: (time of ``prompt_tokens`` + ``singles`` single tokens as one
-        batch - time of the portion alone) / ``singles`` / time of the ``singles`` alone.  Each of the three is
-        a captured step whose lanes are all padding (nothing but the scratch page and slot is touched), replayed
-        ``replays`` times; the median counts.  None when the single tokens cost nothing measurable."""
+    def measure_split(self, candidates: Sequence[torch.cuda.Stream], prompt_tokens: int = 1024, singles: int = 16, replays: int = 5) -> Optional[float]:
+        """The clock's answer to what a single decoded token costs as part of a portion's batch, in units of what
+        a batch of single tokens costs that runs beside the portion on a stream of its own: (time of ``prompt_tokens`` +
+        ``singles`` single tokens as one batch - time of the portion alone) / ``singles`` / (time of the two batches
+        side by side, the single tokens on the best of ``candidates``, - time of the portion alone).  Each of the three graphs is a captured step whose lanes are all
+        padding (nothing but the scratch page and slot is touched), replayed ``replays`` times; the median counts.
+        None when the single tokens cost nothing measurable as part of the batch."""
         prompt_tokens = min(prompt_tokens, self.max_seq_len)
         if prompt_tokens < 2:
             return None
-        times = []
-        for lengths in ([prompt_tokens], [prompt_tokens] + [1] * singles, [1] * singles):
+        captured = []
+        for lengths, kind in (([prompt_tokens], PORTIONS), ([prompt_tokens] + [1] * singles, PORTIONS), ([1] * singles, SINGLES)):
             ends, row = [], 0
             for length in lengths:
                 row += length
@@ -211,22 +245,57 @@ class DecodeGraphs:
             static = StaticStep(self.cache, len(lengths), max(prompt_tokens, 64), self.device, lengths=lengths,
                                 want_rows=ends, **self.model.step_layout)
             # (a memory pool of its own: the graphs' shared pool ends with the last graph in it)
-            _, graph, _ = self._capture(0, static, warm_runs=1, pool=torch.cuda.graph_pool_handle())
-            marks = [torch.cuda.Event(enable_timing=True) for _ in range(replays + 1)]
-            graph.replay()
-            marks[0].record()
-            for mark in marks[1:]:
-                graph.replay()
-                mark.record()
-            torch.cuda.synchronize(self.device)
-            times.append(sorted(a.elapsed_time(b) for a, b in zip(marks, marks[1:]))[replays // 2])
-            del graph, static
-        portion, both, alone = times
-        if both <= portion or alone <= 0:
+            captured.append(self._capture(0, static, warm_runs=1, pool=torch.cuda.graph_pool_handle(), kind=kind))
+        portion, both = self._clock(captured[0][1].replay, replays), self._clock(captured[1][1].replay, replays)
+        two = min(self._clock_beside(captured[0][1], captured[2][1], stream, replays) for stream in candidates)
+        del captured
+        if both <= portion:
             return None
-        return (both - portion) / singles / alone
+        return (both - portion) / singles / max(two - portion, 0.01 * portion)
 
-    def measure_halves(self, lanes: int = 128, replays: int = 5) -> Optional[float]:
+    def _clock(self, run, replays: int) -> float:
+        """The median time of ``replays`` calls of ``run`` in a row, behind a first one, in milliseconds."""
+        marks = [torch.cuda.Event(enable_timing=True) for _ in range(replays + 1)]
+        run()
+        marks[0].record()
+        for mark in marks[1:]:
+            run()
+            mark.record()
+        torch.cuda.synchronize(self.device)
+        return sorted(a.elapsed_time(b) for a, b in zip(marks, marks[1:]))[replays // 2]
+
+    def _clock_beside(self, graph, other, beside: torch.cuda.Stream, replays: int) -> float:
+        """The time of ``graph`` with ``other`` on ``beside``."""
+        main = torch.cuda.current_stream(self.device)
+
+        def side_by_side():
+            with replayed_beside(main, beside):
+                other.replay()
+            graph.replay()
+            main.wait_stream(beside)
+        return self._clock(side_by_side, replays)
+
+    def stream_beside(self, lanes: Sequence[Lane], portions: LoweredLanes, singles: LoweredLanes,
+                      candidates: Sequence[torch.cuda.Stream]) -> torch.cuda.Stream:
+        """The stream of ``candidates`` on which the graph of ``singles`` runs best beside that of ``portions``: asked of
+        the clock once for every graph of portions (and stream of the caller), with nothing but padding in either; the
+        first where one of the two has no graph yet."""
+        key = self._bucket_key(lanes, portions)
+        decode_key = (bucket_for(len(singles.slots)), self.context_bucket(singles))
+        if key not in self._bucket_graphs or decode_key not in self._graphs:
+            return candidates[0]
+        main = torch.cuda.current_stream(self.device).cuda_stream
+        chosen = self._besides.setdefault(key, {})
+        if main not in chosen:
+            graphs = []
+            for static, graph, _ in (self._bucket_graphs[key], self._graphs[decode_key]):
+                static.fill(_NO_LANES)
+                graphs.append(graph)
+            times = [self._clock_beside(*graphs, stream, 3) for stream in candidates]
+            chosen[main] = candidates[times.index(min(times))]
+        return chosen[main]
+
+    def measure_halves(self, beside: torch.cuda.Stream, lanes: int = 128, replays: int = 5) -> Optional[float]:
         """The clock's answer to whether a step of ``lanes`` single tokens is faster as two halves at once, each a
         graph of its own on a stream of its own, than as one graph: the time of the two halves over the time of the
         one.  The halves read every weight twice, which a model whose steps wait for its weights cannot afford
@@ -239,33 +308,33 @@ class DecodeGraphs:
         halves = [self._capture(bucket_for((lanes + 1) // 2), context=context, warm_runs=1,
                                 pool=torch.cuda.graph_pool_handle()) for _ in range(2)]
         main = torch.cuda.current_stream(self.device)
-        beside = torch.cuda.Stream(device=self.device)
 
         def as_one():
             whole[1].replay()
 
         def as_halves():
-            beside.wait_stream(main)
-            with torch.cuda.stream(beside):
+            with replayed_beside(main, beside):
                 halves[1][1].replay()
             halves[0][1].replay()
             main.wait_stream(beside)
 
-        times = []
-        for run in (as_one, as_halves):
-            marks = [torch.cuda.Event(enable_timing=True) for _ in range(replays + 1)]
-            run()
-            marks[0].record()
-            for mark in marks[1:]:
-                run()
-                mark.record()
-            torch.cuda.synchronize(self.device)
-            times.append(sorted(a.elapsed_time(b) for a, b in zip(marks, marks[1:]))[replays // 2])
+        one, two = (self._clock(run, replays) for run in (as_one, as_halves))
         del whole, halves
-        return times[1] / times[0] if times[0] > 0 else None
+        return two / one if one > 0 else None
+
+    def _capture_stream(self, kind: str) -> torch.cuda.Stream:
+        if kind not in self._streams:
+            # (streams come from a pool that hands them out in turn)
+            taken = [torch.cuda.current_stream(self.device)] + list(self._streams.values()) + list(self.apart_from)
+            stream = torch.cuda.Stream(device=self.device)
+            while stream in taken:
+                stream = torch.cuda.Stream(device=self.device)
+            self._streams[kind] = stream
+        return self._streams[kind]
 
     def _capture(self, bucket: int, static: Optional[StaticStep] = None, warm_runs: int = 2, context: int = 0,
-                 pool=None):
+                 pool=None, kind: Optional[str] = None):
+        kind = kind or (PORTIONS if static is not None and static.capacity else SINGLES)
         if static is None:
             static = StaticStep(self.cache, bucket, context or self.max_seq_len, self.device,
                                 **self.model.step_layout)
@@ -279,12 +348,10 @@ class DecodeGraphs:
         torch.cuda.current_stream(self.device).wait_stream(side)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
-        # one pool for every graph: replays never overlap, so their intermediate buffers may share memory
+        # one pool for every graph of a kind: their replays never overlap, so their intermediate buffers may share memory
         if pool is None:
-            if self._pool is None:
-                self._pool = torch.cuda.graph_pool_handle()
-            pool = self._pool
-        with torch.cuda.graph(graph, pool=pool):
+            pool = self._pools.setdefault(kind, torch.cuda.graph_pool_handle())
+        with torch.cuda.graph(graph, pool=pool, stream=self._capture_stream(kind)):
             logits = self.model.forward(static.context, self.cache)
         return static, graph, logits
 

@@ -33,6 +33,7 @@ _SIGNATURES = {
         "mi_embed": [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_int, _c_int, _c_ptr],
         "mi_embed_rmsnorm": [_c_ptr, _c_ptr, _c_int, _c_float, _c_ptr, _c_float, _c_ptr, _c_int, _c_int, _c_ptr],
         "mi_feed_tokens": [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
+        "mi_wait": [_c_int, _c_ptr],
         "mi_zero_slot": [_c_ptr, _c_ptr, _c_int, _c_long, _c_ptr],
         "mi_add_rmsnorm": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_float, _c_ptr, _c_int, _c_ptr, _c_int,
                            _c_int, _c_float, _c_float, _c_ptr],
@@ -336,6 +337,33 @@ def feed_tokens(token_ids: torch.Tensor, source: torch.Tensor, dst: Sequence[int
     _check(_fn("common", "mi_feed_tokens")(_p(token_ids), token_ids.numel(), _p(source), source.numel(),
                                            ctypes.addressof(places), ctypes.addressof(sources), count, _stream()),
            "feed_tokens")
+
+
+def stream_beside(main: "torch.cuda.Stream", candidates: int = 8, microseconds: int = 200) -> "torch.cuda.Stream":
+    """A stream (default priority) whose kernels run beside those of ``main``.  The runtime lays its streams on a few
+    hardware queues, and what lies on one queue runs one after the other: of up to ``candidates`` streams the first on
+    which a wait of so many microseconds is over together with one on ``main`` (or, if none is, the last)."""
+    wait = _fn("common", "mi_wait")
+    with torch.cuda.device(main.device):
+        for _ in range(candidates):
+            beside = torch.cuda.Stream(device=main.device)
+            if beside == main:
+                continue
+            took = []
+            for _ in range(2):                       # the first round warms both streams up
+                torch.cuda.synchronize(main.device)
+                begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                begin.record(main)
+                beside.wait_event(begin)
+                for stream in (main, beside):
+                    _check(wait(microseconds, stream.cuda_stream), "wait")
+                main.wait_stream(beside)
+                end.record(main)
+                torch.cuda.synchronize(main.device)
+                took.append(1000.0 * begin.elapsed_time(end))
+            if took[1] < 1.6 * microseconds:
+                break
+    return beside
 
 
 class SlotStates:
