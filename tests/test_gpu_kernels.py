@@ -1855,3 +1855,38 @@ def test_scan_gives_the_same_bits_however_its_tokens_are_cut(ops, dtype, N):
         assert torch.equal(y, results[0][0]) and torch.equal(state, results[0][1])
     close(results[0][0], want_y, torch.float32, max(1.0, want_y.abs().max().item()))
     close(results[0][1], want_state, torch.float32, max(1.0, want_state.abs().max().item()))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T", [3, 300])
+@pytest.mark.parametrize("d", [4, 1020, 1022, 1024, 1028, 2052, 4096, 4100])
+def test_layer_norm_in_pieces_of_four(ops, dtype, T, d):
+    h, vector = rand(T, d, seed=1), rand(d, seed=2)
+    first, second = rand(T, d, seed=3, dtype=dtype), rand(T, d, seed=4)
+    weight, bias, bw, bb = (rand(d, seed=seed) for seed in (5, 6, 7, 8))
+    branch = 0.25 * first.double() - 1.5 * second.double()
+
+    def norm(x, weight, bias):
+        centred = x - x.mean(-1, keepdim=True)
+        return centred / torch.sqrt(centred.square().mean(-1, keepdim=True) + 1e-5) * weight.double() + bias.double()
+    for normed in (False, True):
+        stream = h.double() + (norm(branch, bw, bb) if normed else branch) + vector.double()
+        dh, d1, d2, dv, dw, db, dbw, dbb = gpu(h.clone(), first, second, vector, weight, bias, bw, bb)
+        branches = [(d1, 0.25), (d2, -1.5)]
+        out = torch.empty(T, d, dtype=dtype, device=DEV)
+        ops.add_layernorm(dh, branches, dv, dw, db, 1e-5, out, branch_norm=(dbw, dbb, 1e-5) if normed else None)
+        # (the deviations cancel: a rounding of the largest element, not of the result, and with four columns a variance that
+        # may be small beside the mean)
+        assert (dh.cpu().double() - stream).abs().max() <= 4e-6 * max(1.0, stream.abs().max().item()) * 4
+        want = norm(stream, weight, bias)
+        share = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+        assert ((out.cpu().double() - want).abs() <= share * want.abs() + 1e-4).all()
+        if not normed:
+            dh.copy_(h)
+            rows = i32([T - 1, 0, T - 1]).to(DEV)
+            gathered = torch.empty(3, d, dtype=dtype, device=DEV)
+            ops.add_layernorm(dh, branches, dv, dw, db, 1e-5, gathered, rows=rows)
+            assert torch.equal(dh.cpu(), h)
+            if d % 4 == 0 and (d <= 4096 and (d > 1024 or T <= 256)):     # (the sums of other rows go by the number of rows too)
+                assert torch.equal(gathered, out[[T - 1, 0, T - 1]])
+            assert ((gathered.cpu().double() - want[[T - 1, 0, T - 1]]).abs() <= share * want[[T - 1, 0, T - 1]].abs() + 1e-4).all()
