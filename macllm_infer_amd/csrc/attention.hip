@@ -12,83 +12,18 @@
 // (The reference pages its cache the same way, K and V both token-major:
 // crates/macllm-kv/src/cache.rs:558-566, crates/macllm-kernels/src/metal/paged_decode.metal:109-113.)
 #include "common.h"
+#include "rope_rows.h"
 #include <type_traits>
 
 // ---------------------------------------------------------------- rope + cache write
-// For token t at absolute position p:
-//   q[t, h, :] is rotated in place; k[t, h, :] is rotated and stored; v[t, h, :] is stored.
-//   Rotation (half-split, first rotary_dim dims): angle = (float)p * inv_freq[j];
-//   out[j] = x[j] cos - x[j+half] sin;  out[j+half] = x[j+half] cos + x[j] sin.
-//   (reference: src/decoder.rs:186-195, 226-229; K is cached after rotation, :953-962)
-// slot_mapping[t] = page*page_size + offset of the token's cache cell; null = nothing is stored.
 template <typename T>
 __global__ void rope_kv_store_kernel(T* __restrict__ qkv, long ld, int Hq, int Hkv, int dh, int dv,
                                      const int* __restrict__ positions, const float* __restrict__ inv_freq,
                                      int rotary_dim, const int* __restrict__ slot_mapping,
                                      T* __restrict__ k_base, T* __restrict__ v_base, long page_stride,
                                      int page_size) {
-  const long token = blockIdx.x;
-  T* row = qkv + token * ld;
-  const float position = (float)positions[token];
-  const int half = rotary_dim / 2;
-  long cell = -1;
-  long page = 0;
-  int offset = 0;
-  if (slot_mapping) {
-    cell = slot_mapping[token];
-    page = cell / page_size;
-    offset = (int)(cell - page * page_size);
-  }
-  // q heads then k heads: (head, pair) items
-  const int rotary_heads = Hq + Hkv;
-  const int pairs = rotary_heads * (dh / 2);   // items cover dh/2 "columns": rotated pairs and pass-through pairs
-  for (int item = threadIdx.x; item < pairs; item += blockDim.x) {
-    const int head = item / (dh / 2);
-    const int j = item - head * (dh / 2);
-    T* x = row + (long)head * dh;
-    // column j pairs with j+half when j < half; columns >= rotary_dim pass through.
-    // Enumerate so that every element of the head is visited exactly once:
-    //   j in [0, half): rotated pair (j, j+half)
-    //   j in [half, dh/2): pass-through elements (rotary_dim + 2*(j-half)) and the next one
-    float a, b;
-    int ia, ib;
-    if (j < half) {
-      ia = j;
-      ib = j + half;
-      const float x0 = to_float(x[ia]);
-      const float x1 = to_float(x[ib]);
-      float s = 0.f, c = 1.f;
-      if (inv_freq) {
-        const float angle = position * inv_freq[j];
-        s = sinf(angle);
-        c = cosf(angle);
-      }
-      a = x0 * c - x1 * s;
-      b = x1 * c + x0 * s;
-    } else {
-      ia = rotary_dim + 2 * (j - half);
-      ib = ia + 1;
-      a = to_float(x[ia]);
-      b = to_float(x[ib]);
-    }
-    if (head < Hq) {
-      x[ia] = from_float<T>(a);
-      x[ib] = from_float<T>(b);
-    } else if (cell >= 0) {
-      const int kvh = head - Hq;
-      T* dst = k_base + page * page_stride + ((long)kvh * page_size + offset) * dh;
-      dst[ia] = from_float<T>(a);
-      dst[ib] = from_float<T>(b);
-    }
-  }
-  if (cell >= 0) {
-    const T* v = row + (long)(Hq + Hkv) * dh;
-    for (int item = threadIdx.x; item < Hkv * dv; item += blockDim.x) {
-      const int kvh = item / dv;
-      const int i = item - kvh * dv;
-      v_base[page * page_stride + ((long)kvh * dv + i) * page_size + offset] = v[item];
-    }
-  }
+  rope_kv_store_row<T>(blockIdx.x, qkv, ld, Hq, Hkv, dh, dv, positions, inv_freq, rotary_dim, slot_mapping, k_base, v_base,
+                       page_stride, page_size);
 }
 
 // dv: the width of a value head (the v heads follow the k heads in a row of qkv).
@@ -1521,17 +1456,8 @@ extern "C" int mi_prefill_attention(const void* q, long q_ld, int Hq, int Hkv, i
   const int G = Hq / Hkv;
   if ((dh != 64 && dh != 128) || page_size % 4 != 0 || q_ld % 8 != 0 || out_ld % 4 != 0 || Hkv > 65535 || G > 64)
     return ERR_UNSUPPORTED_SIZE;
-  // up to four query heads share every K and V fragment; head size 128 holds twice the registers per head, and
-  // more than two heads would spill.  A grid that would leave compute units with fewer than two workgroups, over
-  // contexts of up to 2,048 keys (max_seq_len: an upper bound of the step's longest context, 0 = not known), is
-  // bound by the softmax arithmetic of its longest tiles: it takes sets of two heads, so that twice the
-  // workgroups, every other pass from the light end, spread that work.  Over longer contexts the keys and
-  // values that four heads share count for more (a 2,048-token portion of the 0.5B shape behind 2,048 tokens
-  // of context: 7.29 ms with two heads a set, 6.85 with four; behind 30,000 tokens 19.0 and 16.4).
-  int most = dh == 128 ? 2 : 4;
-  if (most > 2 && max_seq_len <= 2048 && 4L * n_tiles * Hkv * ((G + most - 1) / most) < PREFILL_FILL_BLOCKS) most = 2;
-  const int passes = (G + most - 1) / most;
-  const int nset = (G + passes - 1) / passes;
+  const int nset = prefill_head_set(dh, G, n_tiles, Hkv, max_seq_len);
+  const int passes = (G + nset - 1) / nset;
   if (n_tiles > (1 << 28)) return ERR_UNSUPPORTED_SIZE;
   const dim3 grid(4 * n_tiles, Hkv, passes);
 #define PREFILL_LAUNCH(DH_, NSET_, BIAS_)                                                                      \

@@ -14,6 +14,24 @@
 #define PREFILL_WAVES 8
 #define PREFILL_FILL_BLOCKS 512   // two workgroups for each of the 256 compute units
 
+// How many query heads of a kv head share a workgroup of the launch (G of them in all).
+// up to four query heads share every K and V fragment; head size 128 holds twice the registers per head, and
+// more than two heads would spill.  A grid that would leave compute units with fewer than two workgroups, over
+// contexts of up to 2,048 keys (max_seq_len: an upper bound of the step's longest context, 0 = not known), is
+// bound by the softmax arithmetic of its longest tiles: it takes sets of two heads, so that twice the
+// workgroups, every other pass from the light end, spread that work.  Over longer contexts the keys and
+// values that four heads share count for more (a 2,048-token portion of the 0.5B shape behind 2,048 tokens
+// of context: 7.29 ms with two heads a set, 6.85 with four; behind 30,000 tokens 19.0 and 16.4).
+static inline int prefill_head_set(int dh, int G, int n_tiles, int Hkv, int max_seq_len) {
+  int most = dh == 128 ? 2 : 4;
+  if (most > 2 && max_seq_len <= 2048 && 4L * n_tiles * Hkv * ((G + most - 1) / most) < PREFILL_FILL_BLOCKS) most = 2;
+  const int passes = (G + most - 1) / most;
+  return (G + passes - 1) / passes;
+}
+
+// LDS of a workgroup: m, l and the accumulator of one set from every wave, and the waves' page ids
+constexpr int prefill_lds_bytes(int DV) { return PREFILL_WAVES * WAVE * 4 * (2 + 4 * (DV / 16) + 1); }
+
 // BIAS: BIAS_LOG, the scores lose log_bias[head] = (r1, r2) -> r1 * ln(1 + r2 * distance); BIAS_LINEAR, they lose
 // slopes[head] * distance.  sinks (may be null): one more term exp(sinks[head]) of the softmax's denominator.
 // DV: the width the values are computed with, the keys' or, PADDED, the next width of the launch's table above
@@ -24,27 +42,23 @@
 // key_dim wide, a multiple of 8 and at most DH.  out_gate: see output_gate (softmax weights; rows in pieces of four).
 template <int DH, int NSET, int BIAS = BIAS_NONE, int DV = DH, bool SIGMOID = false, bool PADDED = false,
           bool PADDED_KEYS = false>
-__global__ void __launch_bounds__(PREFILL_WAVES * WAVE)
-prefill_attention_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, const bf16_t* __restrict__ k_base,
-                         const bf16_t* __restrict__ v_base, long page_stride, int page_size,
-                         const int* __restrict__ block_tables, int max_pages, const int* __restrict__ tiles,
-                         const int* __restrict__ cu_seqlens, const int* __restrict__ start_pos, float scale,
-                         int window, bf16_t* __restrict__ out, long out_ld,
-                         const float* __restrict__ log_bias = nullptr, const float* __restrict__ sinks = nullptr,
-                         int value_dim = DV, const float* __restrict__ head_scales = nullptr,
-                         const float* __restrict__ score_bias = nullptr, int kept = 0,
-                         const float* __restrict__ slopes = nullptr, const bf16_t* __restrict__ out_gate = nullptr,
-                         long gate_ld = 0, int key_dim = DH) {
+__device__ __forceinline__ void prefill_attention_block(
+    unsigned char* __restrict__ smem, const int place, const int places, const int kvh, const int pass,
+    const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, const bf16_t* __restrict__ k_base,
+    const bf16_t* __restrict__ v_base, long page_stride, int page_size, const int* __restrict__ block_tables, int max_pages,
+    const int* __restrict__ tiles, const int* __restrict__ cu_seqlens, const int* __restrict__ start_pos, float scale,
+    int window, bf16_t* __restrict__ out, long out_ld, const float* __restrict__ log_bias, const float* __restrict__ sinks,
+    int value_dim, const float* __restrict__ head_scales, const float* __restrict__ score_bias, int kept,
+    const float* __restrict__ slopes, const bf16_t* __restrict__ out_gate, long gate_ld, int key_dim) {
   constexpr int ITEMS = 2 + 4 * (DV / 16);                    // m, l and the accumulator of one set
-  __shared__ float part[PREFILL_WAVES][ITEMS][WAVE];
-  __shared__ int wave_pages[PREFILL_WAVES][WAVE];
+  float (*const part)[ITEMS][WAVE] = reinterpret_cast<float (*)[ITEMS][WAVE]>(smem);
+  int (*const wave_pages)[WAVE] = reinterpret_cast<int (*)[WAVE]>(smem + sizeof(float) * PREFILL_WAVES * ITEMS * WAVE);
   // heavy ones first; every other head pass the other way round, so that workgroups of two passes that
   // run side by side bring about the same work together
-  const int block = (blockIdx.z & 1) ? blockIdx.x : gridDim.x - 1 - blockIdx.x;
+  const int block = (pass & 1) ? place : places - 1 - place;
   const int tile = block / 4;
-  const int kvh = blockIdx.y;
   const int G = Hq / Hkv;
-  const int head0 = kvh * G + blockIdx.z * NSET;             // first head of this pass
+  const int head0 = kvh * G + pass * NSET;             // first head of this pass
   const int request = tiles[2 * tile];
   if (request < 0) return;                                    // a row of the table past the step's own runs
   const int lane = threadIdx.x & (WAVE - 1);
@@ -61,13 +75,13 @@ prefill_attention_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hk
   const int last_position = base_position + min(first_token + 15, lane_end - 1);
   const int first_position = base_position + first_token;
   // every column of the wave holds a query (16 tokens, and the head sets divide the heads): the wave's bounds are known
-  const bool full_tile = first_token + 16 <= lane_end && (blockIdx.z + 1) * NSET <= G;
+  const bool full_tile = first_token + 16 <= lane_end && (pass + 1) * NSET <= G;
 
   mfma_bf16x8 q_frag[NSET][DH / 32];
   int col_pos[NSET];
 #pragma unroll
   for (int s = 0; s < NSET; ++s) {
-    const bool valid = has_query && blockIdx.z * NSET + s < G;
+    const bool valid = has_query && pass * NSET + s < G;
     col_pos[s] = valid ? position : -1;
 #pragma unroll
     for (int kk = 0; kk < DH / 32; ++kk) {
@@ -213,4 +227,24 @@ prefill_attention_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hk
       *reinterpret_cast<mfma_bf16x4*>(o + 16 * dt + 4 * qd) = packed;
     }
   }
+}
+
+template <int DH, int NSET, int BIAS = BIAS_NONE, int DV = DH, bool SIGMOID = false, bool PADDED = false,
+          bool PADDED_KEYS = false>
+__global__ void __launch_bounds__(PREFILL_WAVES * WAVE)
+prefill_attention_kernel(const bf16_t* __restrict__ q, long q_ld, int Hq, int Hkv, const bf16_t* __restrict__ k_base,
+                         const bf16_t* __restrict__ v_base, long page_stride, int page_size,
+                         const int* __restrict__ block_tables, int max_pages, const int* __restrict__ tiles,
+                         const int* __restrict__ cu_seqlens, const int* __restrict__ start_pos, float scale,
+                         int window, bf16_t* __restrict__ out, long out_ld,
+                         const float* __restrict__ log_bias = nullptr, const float* __restrict__ sinks = nullptr,
+                         int value_dim = DV, const float* __restrict__ head_scales = nullptr,
+                         const float* __restrict__ score_bias = nullptr, int kept = 0,
+                         const float* __restrict__ slopes = nullptr, const bf16_t* __restrict__ out_gate = nullptr,
+                         long gate_ld = 0, int key_dim = DH) {
+  __shared__ __align__(16) unsigned char smem[prefill_lds_bytes(DV)];
+  prefill_attention_block<DH, NSET, BIAS, DV, SIGMOID, PADDED, PADDED_KEYS>(
+      smem, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, q, q_ld, Hq, Hkv, k_base, v_base, page_stride, page_size, block_tables,
+      max_pages, tiles, cu_seqlens, start_pos, scale, window, out, out_ld, log_bias, sinks, value_dim, head_scales, score_bias,
+      kept, slopes, out_gate, gate_ld, key_dim);
 }

@@ -20,7 +20,8 @@
 // contiguous, which is the state index n for C . B^T and S_in . C, and the token for the other
 // two products, hence the transposed copies.
 // (reference recurrence: crates/macllm-kernels/src/mamba2.rs:259-288; the reference scans token by token.)
-#include "common.h"
+#include "attn_prefill.h"
+#include "rope_rows.h"
 
 typedef __bf16 s_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 s_bf16x4 __attribute__((ext_vector_type(4)));
@@ -198,22 +199,62 @@ __device__ void ssd_conv_block(const bf16_t* __restrict__ u, long u_ld, int C, c
   }
 }
 
-// prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch
-template <int K>
+// ---------------------------------------------------------------- attention beside the scan
+// A layer whose attention and state-space mixer read the same projected rows runs two chains of small launches that do
+// not depend on each other: rotation and cache write, then the attention; conv and prepare, then the scan.  In a short
+// prompt none of them fills the GPU and each costs its launch and its round trips, so the attention's two run as further
+// workgroups of the scan's two.  37 tokens of the 0.5B shape through 36
+// layers: 2,314 us in four launches, 1,954 in two; 128 tokens of twelve layers of the 7B shape 3,100 and 2,872.
+struct PromptBeside {
+  void* qkv;                       // rows [q | k | v] of T tokens, bfloat16
+  long ld;
+  int T, Hq, Hkv, dh;
+  const int* positions;
+  const float* inv_freq;
+  int rotary_dim;
+  const int* slot_mapping;
+  void* k_base;
+  void* v_base;
+  long page_stride;
+  int page_size;
+  int attend;                      // 1: the attention too, beside the second launch
+  const int* block_tables;
+  int max_pages;
+  const int* tiles;
+  int n_tiles;
+  const int* cu_seqlens;
+  const int* start_pos;
+  float scale;
+  int window, max_seq_len;
+  void* out;
+  long out_ld;
+};
+
+// prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch; with BESIDE the
+// rows from `first_beside` on rotate and store a token each
+template <int K, bool BESIDE>
 __global__ void __launch_bounds__(256)
 ssd_prepare_conv_kernel(const bf16_t* __restrict__ dt, long dt_ld, const float* __restrict__ dt_bias,
                         const float* __restrict__ A, const int* __restrict__ chunks, int H, float* __restrict__ delta,
                         float* __restrict__ cum, const bf16_t* __restrict__ u, long u_ld, int C,
                         const float* __restrict__ conv_w, const float* __restrict__ conv_b,
                         const bf16_t* __restrict__ conv_state, const int* __restrict__ slot_ids, int Q,
-                        bf16_t* __restrict__ xbc, long xbc_ld, int tt_channels, bf16_t* __restrict__ TT) {
+                        bf16_t* __restrict__ xbc, long xbc_ld, int tt_channels, bf16_t* __restrict__ TT, int first_beside,
+                        PromptBeside beside) {
   __shared__ __align__(4) bf16_t tile[64 * (SSD_MAX_Q + 2)];
   __shared__ float wave_total[SSD_MAX_Q / WAVE];
   if ((int)blockIdx.y < H)
     ssd_prepare_block(dt, dt_ld, dt_bias, A, chunks, H, delta, cum, blockIdx.x, blockIdx.y, wave_total);
-  else
+  else if (!BESIDE || (int)blockIdx.y < first_beside)
     ssd_conv_block<K>(u, u_ld, C, conv_w, conv_b, conv_state, chunks, slot_ids, Q, xbc, xbc_ld, tt_channels, TT,
                       blockIdx.x, ((int)blockIdx.y - H) * 64, tile);
+  else {
+    const long token = (long)((int)blockIdx.y - first_beside) * gridDim.x + blockIdx.x;
+    if (token < beside.T)
+      rope_kv_store_row<bf16_t>(token, (bf16_t*)beside.qkv, beside.ld, beside.Hq, beside.Hkv, beside.dh, beside.dh, beside.positions,
+                                beside.inv_freq, beside.rotary_dim, beside.slot_mapping, (bf16_t*)beside.k_base,
+                                (bf16_t*)beside.v_base, beside.page_stride, beside.page_size);
+  }
 }
 
 // The conv tail of a lane after its tokens: the last K-1 rows of [old tail ; the lane's raw rows]
@@ -771,11 +812,12 @@ struct SsdSingle {
   const int* lane_chunks;
 };
 template <int NK, int PT>
-__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
-ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+__device__ __forceinline__ void ssd_single_block(
+    unsigned char* __restrict__ scan_smem, const int chunk, const int head, const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
                   const float* __restrict__ delta, const float* __restrict__ cum, const float* __restrict__ D,
                   const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y, long y_ld,
                   const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated, long gated_ld, const SsdSingle one) {
+
   constexpr int N = 32 * NK;
   constexpr int P = 16 * PT;
   constexpr int LD1 = N + 8;                     // row stride of the S and B buffers
@@ -787,15 +829,12 @@ ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __r
   constexpr int QK = SSD_SINGLE_TOKENS / 32;
   constexpr int PB = PT < 4 ? PT : 4;            // tiles of state rows that share the weighted B fragments
   constexpr int ITEMS = (N / 16) * (PT / PB);
-  extern __shared__ __align__(16) unsigned char scan_smem[];
   bf16_t* s_rows = reinterpret_cast<bf16_t*>(scan_smem);               // [P][LD1]
   bf16_t* b_lds = s_rows + P * LD1;                                    // [64][LD1]
   bf16_t* x_lds = b_lds + 64 * LD1;                                    // [P][LDX]
   float* L = reinterpret_cast<float*>(x_lds + P * LDX);                // [SSD_SINGLE_TOKENS] each
   float* step = L + SSD_SINGLE_TOKENS;
   float* weight = step + SSD_SINGLE_TOKENS;
-  const int chunk = blockIdx.x;
-  const int head = blockIdx.y;
   const int step_lane = chunks[4 * chunk];
   const int t0 = chunks[4 * chunk + 1];
   const int length = chunks[4 * chunk + 2];
@@ -1029,6 +1068,41 @@ ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __r
   }
 }
 
+template <int NK, int PT>
+__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
+ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                  const float* __restrict__ delta, const float* __restrict__ cum, const float* __restrict__ D,
+                  const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y, long y_ld,
+                  const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated, long gated_ld, const SsdSingle one) {
+  extern __shared__ __align__(16) unsigned char scan_smem[];
+  ssd_single_block<NK, PT>(scan_smem, blockIdx.x, blockIdx.y, xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld, one);
+}
+
+// The same beside the prompt attention of the layer (see PromptBeside): workgroups 0 .. scan_groups - 1 are the scan's, the
+// longer ones, and those after them the attention's, of as many threads; either uses the workgroup's LDS.
+static_assert(SSD_SCAN_WAVES == PREFILL_WAVES, "workgroups of one launch");
+template <int NK, int PT, int DH, int NSET>
+__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
+ssd_single_beside_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                  const float* __restrict__ delta, const float* __restrict__ cum, const float* __restrict__ D,
+                  const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y, long y_ld,
+                  const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated, long gated_ld, const SsdSingle one,
+                         int n_chunks, int scan_groups, int passes, const PromptBeside beside) {
+  extern __shared__ __align__(16) unsigned char scan_smem[];
+  if ((int)blockIdx.x < scan_groups) {
+    ssd_single_block<NK, PT>(scan_smem, blockIdx.x % n_chunks, blockIdx.x / n_chunks, xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld, one);
+    return;
+  }
+  const int index = blockIdx.x - scan_groups;
+  const int places = 4 * beside.n_tiles;
+  prefill_attention_block<DH, NSET>(scan_smem, index % places, places, index / places % beside.Hkv, index / places / beside.Hkv,
+                                    (const bf16_t*)beside.qkv, beside.ld, beside.Hq, beside.Hkv, (const bf16_t*)beside.k_base,
+                                    (const bf16_t*)beside.v_base, beside.page_stride, beside.page_size, beside.block_tables,
+                                    beside.max_pages, beside.tiles, beside.cu_seqlens, beside.start_pos, beside.scale,
+                                    beside.window, (bf16_t*)beside.out, beside.out_ld, nullptr, nullptr, DH, nullptr, nullptr, 0,
+                                    nullptr, nullptr, 0, DH);
+}
+
 static size_t ssd_single_lds_bytes(int P, int N) {
   return (size_t)(P + 64) * (N + 8) * 2 + (size_t)P * (64 + 8) * 2 + (size_t)3 * SSD_SINGLE_TOKENS * 4;
 }
@@ -1043,26 +1117,60 @@ extern "C" int mi_ssd_single(int Q, int P, int N, int longest, const float* ssm_
   return (uintptr_t)ssm_state % 16 == 0 && longest > 0 && longest <= Q && longest <= SSD_SINGLE_TOKENS && ssd_staged_sizes(P, N) ? 1 : 0;
 }
 
+// beyond 64 KiB a kernel has to be told once per device that it may have that much (gfx950 has 160 KiB)
+template <typename Kernel>
+static int allow_lds(Kernel kernel, size_t lds, bool (&told)[64]) {
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return ERR_BAD_ARGUMENT;
+  if (lds <= 64 * 1024 || told[device]) return 0;
+  if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+    (void)hipGetLastError();
+    return ERR_UNSUPPORTED_SIZE;
+  }
+  told[device] = true;
+  return 0;
+}
+
+#define SINGLE_ARGUMENTS xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld, one
 template <int NK, int PT>
 static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, long xbc_ld, const bf16_t* TT, int E,
                              const float* delta, const float* cum, const float* D, const int* chunks, int Q, int H, int G,
                              float* y, long y_ld, const bf16_t* z, long z_ld, bf16_t* gated, long gated_ld,
-                             const SsdSingle& one) {
+                             const SsdSingle& one, const PromptBeside* beside, int nset) {
   const size_t lds = ssd_single_lds_bytes(16 * PT, 32 * NK);
-  // beyond 64 KiB a kernel has to be told once per device that it may have that much (gfx950 has 160 KiB)
-  static bool told[64] = {};
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return ERR_BAD_ARGUMENT;
-  if (lds > 64 * 1024 && !told[device]) {
-    if (hipFuncSetAttribute((const void*)ssd_single_kernel<NK, PT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-      (void)hipGetLastError();
-      return ERR_UNSUPPORTED_SIZE;
-    }
-    told[device] = true;
+  if constexpr ((NK == 4 && PT == 4) || (NK == 8 && PT == 8)) {
+    if (beside) {
+      const int passes = (beside->Hq / beside->Hkv + nset - 1) / nset;
+      const int scan_groups = (int)(grid.x * grid.y);
+      const unsigned groups = (unsigned)(scan_groups + 4 * beside->n_tiles * beside->Hkv * passes);
+#define BESIDE_CASE(DH_, NSET_)                                                                                             \
+  if (beside->dh == DH_ && nset == NSET_) {                                                                                 \
+    static bool told[64] = {};                                                                                              \
+    const size_t both = lds > (size_t)prefill_lds_bytes(DH_) ? lds : (size_t)prefill_lds_bytes(DH_);                        \
+    const int code = allow_lds(ssd_single_beside_kernel<NK, PT, DH_, NSET_>, both, told);                                   \
+    if (code) return code;                                                                                                  \
+    ssd_single_beside_kernel<NK, PT, DH_, NSET_><<<groups, SSD_SCAN_WAVES * WAVE, both, stream>>>(                          \
+        SINGLE_ARGUMENTS, (int)grid.x, scan_groups, passes, *beside);                                                       \
+    return 0;                                                                                                               \
   }
-  ssd_single_kernel<NK, PT><<<grid, SSD_SCAN_WAVES * WAVE, lds, stream>>>(xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y,
-                                                                          y_ld, z, z_ld, gated, gated_ld, one);
+      BESIDE_CASE(64, 2) BESIDE_CASE(64, 4) BESIDE_CASE(128, 2)
+#undef BESIDE_CASE
+    }
+  }
+  if (beside) return ERR_UNSUPPORTED_SIZE;
+  static bool told[64] = {};
+  const int code = allow_lds(ssd_single_kernel<NK, PT>, lds, told);
+  if (code) return code;
+  ssd_single_kernel<NK, PT><<<grid, SSD_SCAN_WAVES * WAVE, lds, stream>>>(SINGLE_ARGUMENTS);
   return 0;
+}
+#undef SINGLE_ARGUMENTS
+
+// Whether mi_ssd_prefill takes the attention of such heads beside its second launch (of a step that mi_ssd_single covers).
+extern "C" int mi_ssd_beside(int P, int N, int Hq, int Hkv, int dh, int n_tiles, int max_seq_len) {
+  if (Hkv <= 0 || Hq % Hkv != 0 || n_tiles <= 0 || !((P == 64 && N == 128) || (P == 128 && N == 256))) return 0;
+  const int nset = prefill_head_set(dh, Hq / Hkv, n_tiles, Hkv, max_seq_len);
+  return (dh == 64 && (nset == 2 || nset == 4)) || (dh == 128 && nset == 2) ? 1 : 0;
 }
 
 static size_t ssd_scan_lds_bytes(int Q, int P, int N) {
@@ -1077,13 +1185,15 @@ extern "C" int mi_ssd_supported(int Q, int P, int N, int G, int E) {
           (E % 8) == 0 && ((long)G * N) % 8 == 0) ? 1 : 0;
 }
 
+// beside: null, or the attention that reads the same step's rows (bfloat16, values as wide as the keys, a cache to write to
+// or none); its rotation needs the conv here, its attention a step that mi_ssd_single and mi_ssd_beside cover.
 extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long dt_ld, const float* dt_bias,
                               const float* A, const float* D, float* ssm_state, const int* chunks, int n_chunks,
                               const int* lane_chunks, const int* slot_ids, int n_lanes, int Q, int H, int P, int N,
                               int G, float* delta, float* cum, void* TT, float* chunk_state,
                               float* chunk_decay, void* state_in, float* y, long y_ld, const void* z, long z_ld,
                               void* gated, long gated_ld, const void* u, long u_ld, const float* conv_w,
-                              const float* conv_b, void* conv_state, int conv_k, int longest, hipStream_t stream) {
+                              const float* conv_b, void* conv_state, int conv_k, int longest, const PromptBeside* beside, hipStream_t stream) {
   if (n_chunks <= 0 || n_lanes <= 0 || H <= 0 || G <= 0 || H % G != 0) return ERR_BAD_ARGUMENT;
   const int E = H * P;
   const int GN = G * N;
@@ -1098,17 +1208,44 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
       n_chunks > 65535 * 32 ||
       H + (E + GN + 63) / 64 > 65535 || n_lanes > 65535)
     return ERR_UNSUPPORTED_SIZE;
+  int nset = 0;
+  if (beside) {
+    const PromptBeside& b = *beside;
+    if (!conv_here || !b.qkv || b.T <= 0 || b.Hq <= 0 || b.Hkv <= 0 || b.Hq % b.Hkv != 0 || b.dh <= 0 || (b.dh & 1) || !b.positions ||
+        b.ld < (long)(b.Hq + 2 * b.Hkv) * b.dh || b.rotary_dim < 0 || b.rotary_dim > b.dh || (b.rotary_dim & 1) ||
+        (b.rotary_dim > 0 && !b.inv_freq) || (b.slot_mapping && (!b.k_base || !b.v_base || b.page_size <= 0)))
+      return ERR_BAD_ARGUMENT;
+    if (b.attend) {
+      if (!b.block_tables || b.max_pages <= 0 || !b.tiles || b.n_tiles <= 0 || !b.cu_seqlens || !b.start_pos || !b.out || !b.k_base ||
+          !b.v_base || b.page_size <= 0)
+        return ERR_BAD_ARGUMENT;
+      if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
+          b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0 ||
+          b.n_tiles > (1 << 20) || b.Hkv > 256)
+        return ERR_UNSUPPORTED_SIZE;
+      nset = prefill_head_set(b.dh, b.Hq / b.Hkv, b.n_tiles, b.Hkv, b.max_seq_len);
+    }
+  }
   if (conv_here) {
-    const dim3 grid(n_chunks, H + (C + 63) / 64);
+    const int own_rows = H + (C + 63) / 64;
+    const int rows = own_rows + (beside ? (beside->T + n_chunks - 1) / n_chunks : 0);
+    if (rows > 65535) return ERR_UNSUPPORTED_SIZE;
+    const dim3 grid(n_chunks, rows);
+    const PromptBeside none = {};
+#define CONV_LAUNCH(K_, BESIDE_)                                                                                   \
+  ssd_prepare_conv_kernel<K_, BESIDE_><<<grid, 256, 0, stream>>>(                                                  \
+      (const bf16_t*)dt, dt_ld, dt_bias, A, chunks, H, delta, cum, (const bf16_t*)u, u_ld, C, conv_w, conv_b,      \
+      (const bf16_t*)conv_state, slot_ids, Q, (bf16_t*)xbc, xbc_ld, E + GN, (bf16_t*)TT, own_rows, beside ? *beside : none)
 #define CONV_CASE(K_)                                                                                              \
-  ssd_prepare_conv_kernel<K_><<<grid, 256, 0, stream>>>((const bf16_t*)dt, dt_ld, dt_bias, A, chunks, H, delta, cum,  \
-                                                        (const bf16_t*)u, u_ld, C, conv_w, conv_b,                  \
-                                                        (const bf16_t*)conv_state, slot_ids, Q, (bf16_t*)xbc,       \
-                                                        xbc_ld, E + GN, (bf16_t*)TT)
+  do {                                                                                                             \
+    if (beside) CONV_LAUNCH(K_, true);                                                                             \
+    else CONV_LAUNCH(K_, false);                                                                                   \
+  } while (0)
     if (conv_k == 2) CONV_CASE(2);
     else if (conv_k == 3) CONV_CASE(3);
     else CONV_CASE(4);
 #undef CONV_CASE
+#undef CONV_LAUNCH
     RETURN_IF_LAUNCH_FAILED();
   } else {
     const dim3 grid(n_chunks, H + (E + GN + 63) / 64);       // x and B are neighbours in a row of xbc
@@ -1124,7 +1261,8 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
   if (N == 32 * NK_ && P == 16 * PT_)                                                                             \
     status = launch_ssd_single<NK_, PT_>(dim3(n_chunks, H + tail_rows), stream, (const bf16_t*)xbc, xbc_ld,       \
                                          (const bf16_t*)TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld,           \
-                                         (const bf16_t*)z, z_ld, (bf16_t*)gated, gated_ld, one);
+                                         (const bf16_t*)z, z_ld, (bf16_t*)gated, gated_ld, one,                       \
+                                         beside && beside->attend ? beside : nullptr, nset);
     SINGLE_CASE(1, 1) SINGLE_CASE(1, 2) SINGLE_CASE(1, 4) SINGLE_CASE(1, 8)
     SINGLE_CASE(2, 1) SINGLE_CASE(2, 2) SINGLE_CASE(2, 4) SINGLE_CASE(2, 8)
     SINGLE_CASE(4, 1) SINGLE_CASE(4, 2) SINGLE_CASE(4, 4) SINGLE_CASE(4, 8)

@@ -169,10 +169,11 @@ _SIGNATURES = {
     },
     "ssd": {
         "mi_ssd_supported": [_c_int, _c_int, _c_int, _c_int, _c_int],
+        "mi_ssd_beside": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
         "mi_ssd_prefill": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr,
                            _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_long,
-                           _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
+                           _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr],
         "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int, _c_ptr],
     },
     "gemm": {
@@ -1997,17 +1998,100 @@ def ssd_supported(chunk_size: int, head_dim: int, state_size: int, num_groups: i
     return bool(_fn("ssd", "mi_ssd_supported")(chunk_size, head_dim, state_size, num_groups, inner_size))
 
 
+class _PromptBeside(ctypes.Structure):
+    _fields_ = [("qkv", _c_ptr), ("ld", _c_long), ("T", _c_int), ("Hq", _c_int), ("Hkv", _c_int), ("dh", _c_int),
+                ("positions", _c_ptr), ("inv_freq", _c_ptr), ("rotary_dim", _c_int), ("slot_mapping", _c_ptr),
+                ("k_base", _c_ptr), ("v_base", _c_ptr), ("page_stride", _c_long), ("page_size", _c_int), ("attend", _c_int),
+                ("block_tables", _c_ptr), ("max_pages", _c_int), ("tiles", _c_ptr), ("n_tiles", _c_int),
+                ("cu_seqlens", _c_ptr), ("start_pos", _c_ptr), ("scale", _c_float), ("window", _c_int),
+                ("max_seq_len", _c_int), ("out", _c_ptr), ("out_ld", _c_long)]
+
+
+@dataclass
+class PromptBeside:
+    """The attention of a layer whose state-space mixer reads the same step: what ``rope_kv_store`` and (``attend``)
+    ``prefill_attention`` take, to be run by ``ssd_prefill`` in its own launches."""
+    qkv: torch.Tensor
+    num_heads: int
+    num_kv_heads: int
+    head_dim: int
+    positions: torch.Tensor
+    inv_freq: Optional[torch.Tensor]
+    rotary_dim: int
+    slot_mapping: Optional[torch.Tensor]
+    k_cache: torch.Tensor
+    v_cache: torch.Tensor
+    block_tables: torch.Tensor
+    query_tiles: torch.Tensor
+    cu_seqlens: torch.Tensor
+    start_pos: torch.Tensor
+    scale: float
+    window: Optional[int]
+    out: torch.Tensor
+    max_seq_len: int
+    sizes: Optional[tuple]
+    attend: bool = True
+
+    def fits(self, longest: int, ssm_state: torch.Tensor, chunk_size: int) -> bool:
+        """Whether ``ssd_prefill`` of a step with lanes of up to ``longest`` tokens takes this attention in its two
+        launches: lanes of one chunk, heads and states of the sizes it knows, and a step that ``prefill_attention`` gives
+        to the kernel whose waves read their keys themselves."""
+        q, out = self.qkv, self.out
+        if not (q.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and q.dim() == 2 and q.stride(1) == 1 and q.stride(0) % 8 == 0
+                and q.data_ptr() % 16 == 0 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0):
+            return False
+        page_size = self.k_cache.shape[2]
+        if not prefill_attention_supported(q.dtype, self.num_heads, self.num_kv_heads, self.head_dim, page_size):
+            return False
+        _, _, P, N = ssm_state.shape
+        if not (_fn("ssd", "mi_ssd_single")(chunk_size, P, N, int(longest), _p(ssm_state))
+                and _fn("ssd", "mi_ssd_beside")(P, N, self.num_heads, self.num_kv_heads, self.head_dim,
+                                                self.query_tiles.shape[0], int(self.max_seq_len or 0))):
+            return False
+        if not shared_prefill_covers(self.num_kv_heads, self.head_dim, page_size, self.k_cache.stride(0), self.k_cache.data_ptr(),
+                                     self.v_cache.data_ptr()):
+            return True
+        lanes, tokens, most = self.sizes or (self.start_pos.numel(), q.shape[0], int(self.max_seq_len or 0))
+        return not shared_prefill_heads(tokens, lanes, self.num_heads, self.num_kv_heads, self.head_dim, most,
+                                        _span(self.window, None, "prefill_attention"))
+
+    def lowered(self) -> _PromptBeside:
+        q_ld, out_ld = _row_major(self.qkv, "qkv"), _row_major(self.out, "out")
+        T = self.qkv.shape[0]
+        _need(self.qkv.shape[1] == (self.num_heads + 2 * self.num_kv_heads) * self.head_dim and self.qkv.is_cuda
+              and self.out.shape == (T, self.num_heads * self.head_dim), "prompt beside: qkv or out does not fit")
+        page_stride, page_size = _cache_view(self.k_cache, self.v_cache, self.num_kv_heads, self.head_dim, self.qkv.dtype)
+        for name in ("positions", "block_tables", "query_tiles", "cu_seqlens", "start_pos"):
+            _i32(getattr(self, name), name)
+        if self.slot_mapping is not None:
+            _i32(self.slot_mapping, "slot_mapping")
+        _need(self.positions.numel() == T and (self.slot_mapping is None or self.slot_mapping.numel() == T)
+              and self.block_tables.dim() == 2 and self.query_tiles.dim() == 2 and self.query_tiles.shape[1] == 2
+              and self.cu_seqlens.numel() == self.start_pos.numel() + 1, "prompt beside: metadata shapes do not match")
+        rotary = int(self.rotary_dim) if self.inv_freq is not None else 0
+        _need(self.inv_freq is None or (self.inv_freq.dtype == torch.float32 and self.inv_freq.numel() >= rotary // 2
+                                        and self.inv_freq.is_cuda), "prompt beside: inv_freq must be float32 [rotary_dim / 2]")
+        return _PromptBeside(_p(self.qkv), q_ld, T, self.num_heads, self.num_kv_heads, self.head_dim, _p(self.positions),
+                             _p(self.inv_freq), rotary, _p(self.slot_mapping), _p(self.k_cache), _p(self.v_cache), page_stride,
+                             page_size, 1 if self.attend else 0, _p(self.block_tables), self.block_tables.shape[1],
+                             _p(self.query_tiles), self.query_tiles.shape[0], _p(self.cu_seqlens), _p(self.start_pos),
+                             float(self.scale), _span(self.window, None, "prefill_attention"), int(self.max_seq_len or 0),
+                             _p(self.out), out_ld)
+
+
 def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: torch.Tensor, D: torch.Tensor,
                 ssm_state: torch.Tensor, table: SsdChunks, slot_ids: torch.Tensor, num_groups: int,
                 y: Optional[torch.Tensor], z: Optional[torch.Tensor] = None,
-                gated: Optional[torch.Tensor] = None, conv: Optional[dict] = None, longest: int = 0) -> None:
+                gated: Optional[torch.Tensor] = None, conv: Optional[dict] = None, longest: int = 0,
+                beside: Optional[PromptBeside] = None) -> None:
     """The selective scan of ``ssm_scan`` (same arguments and results beyond rounding) for bfloat16,
     in chunks on the matrix cores.  ``table`` cuts this step's lanes into chunks.  With ``z`` and
     ``gated`` (bfloat16 [T, E], column views are fine) it writes gated = y * SiLU(z) and no y.
     With ``conv`` = {u, weight, bias, state} the conv runs here too: ``xbc`` is then written (what
     ``conv1d_silu`` would put there from the raw rows ``u`` [T, C]) and the tails ``state`` updated
     (as ``conv_state_update`` would); see ``ssd_conv_supported``.  ``longest``: the longest lane's tokens, or
-    more (0: not known): where every lane is one chunk of up to 128 tokens the scan and its states are one launch."""
+    more (0: not known): where every lane is one chunk of up to 128 tokens the scan and its states are one launch.  ``beside``
+    (with ``conv``; see ``PromptBeside.fits``): the attention of the same step, run by further workgroups of the two."""
     xbc_ld = _row_major(xbc, "xbc")
     dt_ld = _row_major(dt, "dt")
     fused_gate = z is not None
@@ -2060,11 +2144,14 @@ def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: t
         _need(conv_state.dim() == 3 and conv_state.shape[1:] == (taps - 1, C) and conv_state.dtype == torch.bfloat16
               and conv_state.is_contiguous(), "ssd_prefill: bad conv state")
         _need(ssd_conv_supported(taps, C, raw), "ssd_prefill: the conv does not fit (see ssd_conv_supported)")
+    lowered = beside.lowered() if beside is not None else None
+    _need(lowered is None or (conv is not None and lowered.T == T), "ssd_prefill: the attention beside is of another step")
     _check(_fn("ssd", "mi_ssd_prefill")(
         _p(xbc), xbc_ld, _p(dt), dt_ld, _p(dt_bias), _p(A), _p(D), _p(ssm_state), _p(table.chunks), chunks,
         _p(table.lane_chunks), _p(slot_ids), table.num_lanes, Q, H, P, N, num_groups, _p(delta[0]), _p(delta[1]),
         _p(transposed), _p(chunk_state), _p(decay), _p(state_in), _p(y), y_ld, _p(z), z_ld, _p(gated), gated_ld,
-        _p(raw), raw_ld, _p(conv_w), _p(conv_b), _p(conv_state), int(taps), int(longest), _stream()),
+        _p(raw), raw_ld, _p(conv_w), _p(conv_b), _p(conv_state), int(taps), int(longest),
+        ctypes.addressof(lowered) if lowered is not None else None, _stream()),
         "ssd_prefill", f"(Q={Q}, P={P}, N={N})")
 
 

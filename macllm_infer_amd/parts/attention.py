@@ -197,6 +197,20 @@ class Attention(Mixer):
         self.mix(self.qkv(x), step, cache, attended)
         return self.out(attended)
 
+    def prompt_beside(self, qkv: torch.Tensor, step, cache, attended: torch.Tensor):
+        """What ``mix`` would launch for this step, for another mixer to run in its launches (``ops.PromptBeside``), or None
+        where that is more or other than a rotation with the cache write and the prompt attention."""
+        spec = self.spec
+        rotation = getattr(self.position, "plain_rotation", None)
+        if (rotation is None or self.prepared or self.general_only or self.position.score_slopes is not None
+                or step.max_query_len == 1 or not cache.owns_kv or spec.value_width != spec.head_dim):
+            return None
+        inv_freq, rotary_dim = rotation()
+        return ops.PromptBeside(qkv, spec.num_heads, spec.num_kv_heads, spec.head_dim, step.positions, inv_freq, rotary_dim,
+                                step.slot_mappings[cache.group], cache.k_cache, cache.v_cache, step.block_tables[cache.group],
+                                step.query_tiles, step.cu_seqlens, step.start_pos, spec.scale, spec.window, attended,
+                                step.max_seq_len, step.sizes)
+
     def mix(self, qkv: torch.Tensor, step, cache, attended: torch.Tensor) -> None:
         """From the projected rows [q | k | v] (rotated and stored in place) to the attended rows
         ``attended`` [T, Hq * dh]; both may be column views of wider matrices."""

@@ -662,9 +662,27 @@ class LayerFusion:
         return False
 
     def _mix_each(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, order=None) -> None:
+        if order is None and self._mix_side_by_side(u, step, caches, mixed):
+            return
         for index in (range(len(self.mixers)) if order is None else order):
             (lo, hi), (mixed_lo, mixed_hi) = self.in_cols[index], self.mixed_cols[index]
             self.mixers[index].mix(u[:, lo:hi], step, caches[self.names[index]], mixed[:, mixed_lo:mixed_hi])
+
+    def _mix_side_by_side(self, u: torch.Tensor, step, caches, mixed: torch.Tensor) -> bool:
+        """Short portions: an attention mixer's launches inside those of a state-space mixer (False: nothing was done)."""
+        if len(self.mixers) != 2 or step.max_query_len == 1:
+            return False
+        first, second = self.mixers
+        make, takes = getattr(first, "prompt_beside", None), getattr(second, "takes_beside", None)
+        if make is None or takes is None:
+            return False
+        rows = [(u[:, lo:hi], step, caches[name], mixed[:, mixed_lo:mixed_hi])
+                for (lo, hi), (mixed_lo, mixed_hi), name in zip(self.in_cols, self.mixed_cols, self.names)]
+        beside = make(*rows[0])
+        if beside is None or not takes(*rows[1], beside):
+            return False
+        second.mix(*rows[1], beside=beside)
+        return True
 
     def forward_general(self, residual: Residual, step, caches) -> None:
         block = self.block

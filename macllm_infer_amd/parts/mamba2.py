@@ -112,9 +112,16 @@ class Mamba2(Mixer):
         self.mix(u, step, cache, gated)
         return self.out_proj(gated)
 
-    def mix(self, u: torch.Tensor, step, cache, gated: torch.Tensor) -> None:
+    def takes_beside(self, u: torch.Tensor, step, cache, gated: torch.Tensor, beside) -> bool:
+        """Whether ``mix`` runs the attention ``beside`` (``ops.PromptBeside``) in its own launches."""
+        spec = self.spec
+        return (self.norm_weight is None and self._chunked(u, step) and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0
+                and ops.ssd_conv_supported(spec.conv_kernel, spec.conv_width, u[:, spec.inner_size:spec.inner_size + spec.conv_width])
+                and beside.fits(step.max_query_len, cache.states["ssm"], spec.chunk_size))
+
+    def mix(self, u: torch.Tensor, step, cache, gated: torch.Tensor, beside=None) -> None:
         """From the projected rows [z | x B C | dt] to the gated (and normed) scan output
-        ``gated`` [T, E]; both may be column views of wider matrices."""
+        ``gated`` [T, E]; both may be column views of wider matrices.  ``beside``: see ``takes_beside``."""
         spec = self.spec
         E, C = spec.inner_size, spec.conv_width
         T = u.shape[0]
@@ -140,7 +147,7 @@ class Mamba2(Mixer):
                          step.slot_ids, spec.num_groups)
             if self.norm_weight is None and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0:
                 ops.ssd_prefill(*arguments, None, z=u[:, :E], gated=gated, conv=conv,
-                                longest=step.max_query_len)                 # the gate on the scan's way out
+                                longest=step.max_query_len, beside=beside)  # the gate on the scan's way out
                 return
             y = torch.empty((T, E), dtype=torch.float32, device=u.device)
             ops.ssd_prefill(*arguments, y, conv=conv, longest=step.max_query_len)

@@ -124,6 +124,10 @@ class Rope(PositionEncoding):
     def pair_rotation(self):
         return self.inv_freq, self.rotary_dim, False
 
+    def plain_rotation(self):
+        """(inv_freq, rotary_dim): ``rotate_and_store`` is this rotation and the cache write, and nothing else."""
+        return self.inv_freq, self.rotary_dim
+
     def rotate_and_store(self, qkv, num_heads, num_kv_heads, head_dim, step, cache) -> None:
         owns = cache.owns_kv
         ops.rope_kv_store(qkv, num_heads, num_kv_heads, head_dim, step.positions, self.inv_freq,

@@ -1890,3 +1890,74 @@ def test_layer_norm_in_pieces_of_four(ops, dtype, T, d):
             if d % 4 == 0 and (d <= 4096 and (d > 1024 or T <= 256)):     # (the sums of other rows go by the number of rows too)
                 assert torch.equal(gathered, out[[T - 1, 0, T - 1]])
             assert ((gathered.cpu().double() - want[[T - 1, 0, T - 1]]).abs() <= share * want[[T - 1, 0, T - 1]].abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("H, P, N, Hq, Hkv, dh", [(24, 64, 128, 8, 2, 64), (3, 64, 128, 4, 1, 64), (4, 128, 256, 12, 2, 128),
+                                                  (5, 128, 256, 2, 1, 64), (2, 64, 128, 4, 2, 128)])
+@pytest.mark.parametrize("counts, starts, window, longest", [([37], [0], None, 2048), ([1, 5, 128, 64], [0, 700, 0, 33], None, 4096),
+                                                             ([16] * 5, [3, 0, 950, 16, 690], 600, 2048)])
+def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, window, longest):
+    """Lanes of one chunk of up to 128 tokens behind contexts: the rotation, the cache, the attended rows, the scan's outputs,
+    states and tails are the same bits in two launches and in four; a row of the table of runs that holds none."""
+    page_size, G, K, Q = 16, 1, 4, 128
+    E, GN, T, lanes = H * P, G * N, sum(counts), len(counts)
+    C, A_cols = E + 2 * GN, (Hq + 2 * Hkv) * dh
+    lengths = [start + count for start, count in zip(starts, counts)]
+    pool, block_table = paged_setup(lengths, page_size, Hkv, dh, torch.bfloat16, seed=3)
+    pool = rand(*pool.shape, seed=4, dtype=torch.bfloat16)
+    cu = [0] + torch.tensor(counts).cumsum(0).tolist()
+    positions, cells, tiles = [], [], []
+    for lane, (start, count) in enumerate(zip(starts, counts)):
+        for offset in range(count):
+            position = start + offset
+            positions.append(position)
+            cells.append(int(block_table[lane, position // page_size]) * page_size + position % page_size)
+        tiles += [(lane, cu[lane] + first) for first in range(0, count, 64)]
+    tiles.append((-1, 0))
+    u = rand(T, A_cols + E + C + H + (-(A_cols + E + C + H)) % 8, seed=5, dtype=torch.bfloat16).to(DEV)
+    weight, bias = rand(C, K, seed=6, scale=0.5).to(DEV), rand(C, seed=7).to(DEV)
+    dt_bias, A, D = gpu(rand(H, seed=8) - 1.0, -torch.exp(torch.linspace(-3.0, 1.0, H)), rand(H, seed=9))
+    state, tails = rand(lanes + 1, H, P, N, seed=10, scale=0.5).to(DEV), rand(lanes + 1, K - 1, C, seed=11, dtype=torch.bfloat16).to(DEV)
+    slots = i32(torch.randperm(lanes + 1, generator=torch.Generator().manual_seed(1))[:lanes].tolist()).to(DEV)
+    inv_freq = (1e4 ** (-torch.arange(dh // 2).float() / (dh // 2))).to(DEV)
+    index = {name: i32(values).to(DEV) for name, values in (("positions", positions), ("cells", cells), ("tiles", tiles), ("cu", cu), ("starts", starts))}
+    block_table = block_table.to(DEV)
+    table = ops.SsdChunks(counts, Q, DEV)
+    results = []
+    for together in (False, True):
+        rows, pages, s, t = u.clone(), pool.to(DEV), state.clone(), tails.clone()
+        mixed = torch.full((T, Hq * dh + E), float("nan"), dtype=torch.bfloat16, device=DEV)
+        qkv, z, raw, dt = rows[:, :A_cols], rows[:, A_cols:A_cols + E], rows[:, A_cols + E:A_cols + E + C], rows[:, A_cols + E + C:A_cols + E + C + H]
+        beside = ops.PromptBeside(qkv, Hq, Hkv, dh, index["positions"], inv_freq, dh, index["cells"], *views(pages, page_size), block_table,
+                                  index["tiles"], index["cu"], index["starts"], 0.11, window, mixed[:, :Hq * dh], longest,
+                                  (1, 16, 4096))          # (of a step that goes to the kernel whose waves read their keys)
+        if not together:
+            ops.rope_kv_store(qkv, Hq, Hkv, dh, beside.positions, inv_freq, dh, beside.slot_mapping, *views(pages, page_size))
+            ops.prefill_attention(qkv, Hq, Hkv, dh, *views(pages, page_size), block_table, beside.query_tiles, beside.cu_seqlens,
+                                  beside.start_pos, 0.11, window, beside.out, longest, sizes=beside.sizes)
+        else:
+            assert beside.fits(max(counts), s, Q)
+        xbc = torch.empty(T, C, dtype=torch.bfloat16, device=DEV)
+        ops.ssd_prefill(xbc, dt, dt_bias, A, D, s, table, slots, G, None, z=z, gated=mixed[:, Hq * dh:], longest=max(counts),
+                        conv=dict(u=raw, weight=weight, bias=bias, state=t), beside=beside if together else None)
+        results.append((rows, pages, s, t, mixed))
+    for apart, joined in zip(*results):
+        assert torch.isfinite(joined.float()).all() and torch.equal(apart, joined)
+
+
+def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
+    state = torch.zeros(2, 4, 64, 128, device=DEV)
+    q, out = torch.zeros(8, 1024, dtype=torch.bfloat16, device=DEV), torch.zeros(8, 512, dtype=torch.bfloat16, device=DEV)
+    cache = torch.zeros(4, 4, 16, 64, dtype=torch.bfloat16, device=DEV)
+    one = i32([0, 0]).to(DEV)
+    make = lambda **other: ops.PromptBeside(**dict(dict(
+        qkv=q, num_heads=8, num_kv_heads=4, head_dim=64, positions=one, inv_freq=None, rotary_dim=0, slot_mapping=None,
+        k_cache=cache, v_cache=cache.transpose(2, 3).contiguous(), block_tables=one.view(1, 2), query_tiles=one.view(1, 2),
+        cu_seqlens=one, start_pos=one[:1], scale=1.0, window=None, out=out, max_seq_len=64, sizes=(1, 16, 4096)), **other))
+    assert make().fits(8, state, 128)
+    assert not make().fits(129, state, 128) and not make().fits(0, state, 128)          # a lane of two chunks, or of unknown length
+    assert not make().fits(8, torch.zeros(2, 4, 32, 128, device=DEV), 128)              # states of other sizes
+    assert not make(num_heads=4).fits(8, state, 128)                                    # one head a kv head
+    assert not make(qkv=q.float()).fits(8, state, 128)
+    assert not make(qkv=torch.zeros(8, 1028, dtype=torch.bfloat16, device=DEV)[:, 4:]).fits(8, state, 128)
+    assert not make(sizes=(1, 2048, 2048)).fits(8, state, 128)                          # the kernel whose waves share their keys
