@@ -324,12 +324,18 @@ class DecodeGraphs:
 
     def _capture_stream(self, kind: str) -> torch.cuda.Stream:
         if kind not in self._streams:
-            # (streams come from a pool that hands them out in turn)
-            taken = [torch.cuda.current_stream(self.device)] + list(self._streams.values()) + list(self.apart_from)
-            stream = torch.cuda.Stream(device=self.device)
-            while stream in taken:
+            usual = torch.cuda.graph.default_capture_stream           # the one torch records graphs on by default
+            if usual is None:
+                usual = torch.cuda.graph.default_capture_stream = torch.cuda.Stream(device=self.device)
+            if kind == SINGLES and not self.apart_from:
+                self._streams[kind] = usual
+            else:
+                # (streams come from a pool that hands them out in turn)
+                taken = [torch.cuda.current_stream(self.device), usual] + list(self._streams.values()) + list(self.apart_from)
                 stream = torch.cuda.Stream(device=self.device)
-            self._streams[kind] = stream
+                while stream in taken:
+                    stream = torch.cuda.Stream(device=self.device)
+                self._streams[kind] = stream
         return self._streams[kind]
 
     def _capture(self, bucket: int, static: Optional[StaticStep] = None, warm_runs: int = 2, context: int = 0,
