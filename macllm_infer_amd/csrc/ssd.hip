@@ -34,7 +34,7 @@ typedef float s_floatx4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- prepare
 // delta[t, h] = softplus(dt + bias); cum[t, h] = sum of delta*A over the chunk up to t (inclusive).
-__device__ void ssd_prepare_block(const bf16_t* __restrict__ dt, long dt_ld, const float* __restrict__ dt_bias,
+__device__ __forceinline__ void ssd_prepare_block(const bf16_t* __restrict__ dt, long dt_ld, const float* __restrict__ dt_bias,
                                   const float* __restrict__ A, const int* __restrict__ chunks, int H,
                                   float* __restrict__ delta, float* __restrict__ cum, int chunk, int head,
                                   float* wave_total) {
@@ -70,7 +70,7 @@ __device__ void ssd_prepare_block(const bf16_t* __restrict__ dt, long dt_ld, con
 // 64 channels of a chunk per workgroup: 16-byte loads along the channels, 2-byte stores into a
 // transposed LDS tile whose row stride (Q + 2 elements = an odd number of banks) keeps them
 // apart, 4-byte LDS reads and 16-byte stores along the tokens.
-__device__ void ssd_transpose_block(const bf16_t* __restrict__ xbc, long ld, int channels, const int* __restrict__ chunks,
+__device__ __forceinline__ void ssd_transpose_block(const bf16_t* __restrict__ xbc, long ld, int channels, const int* __restrict__ chunks,
                                     int Q, bf16_t* __restrict__ out, int chunk, int c0, bf16_t* tile) {
   const int stride = Q + 2;
   const int t0 = chunks[4 * chunk + 1];
@@ -126,7 +126,7 @@ ssd_prepare_transpose_kernel(const bf16_t* __restrict__ dt, long dt_ld, const fl
 // not exist are clamped and dropped).  The tail itself is updated later, by ssd_tail_block, once every
 // chunk has read it.
 template <int K>
-__device__ void ssd_conv_block(const bf16_t* __restrict__ u, long u_ld, int C, const float* __restrict__ conv_w,
+__device__ __forceinline__ void ssd_conv_block(const bf16_t* __restrict__ u, long u_ld, int C, const float* __restrict__ conv_w,
                                const float* __restrict__ conv_b, const bf16_t* __restrict__ conv_state,
                                const int* __restrict__ chunks, const int* __restrict__ slot_ids, int Q,
                                bf16_t* __restrict__ xbc, long xbc_ld, int tt_channels, bf16_t* __restrict__ TT,
@@ -203,8 +203,8 @@ __device__ void ssd_conv_block(const bf16_t* __restrict__ u, long u_ld, int C, c
 // A layer whose attention and state-space mixer read the same projected rows runs two chains of small launches that do
 // not depend on each other: rotation and cache write, then the attention; conv and prepare, then the scan.  In a short
 // prompt none of them fills the GPU and each costs its launch and its round trips, so the attention's two run as further
-// workgroups of the scan's two.  37 tokens of the 0.5B shape through 36
-// layers: 2,314 us in four launches, 1,954 in two; 128 tokens of twelve layers of the 7B shape 3,100 and 2,872.
+// workgroups of the scan's two.  37 tokens of the 0.5B shape through 36 layers: 2,314 us in four launches, 1,954 in two; 128 tokens of
+// twelve layers of the 7B shape 3,100 and 2,872.
 struct PromptBeside {
   void* qkv;                       // rows [q | k | v] of T tokens, bfloat16
   long ld;
@@ -230,8 +230,9 @@ struct PromptBeside {
   long out_ld;
 };
 
-// prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch; with BESIDE the
-// rows from `first_beside` on rotate and store a token each
+// prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch (their code inlined in
+// both instances: as a function called from two kernels the conv took 30 us where it takes 16); with BESIDE the rows
+// from `first_beside` on rotate and store a token each
 template <int K, bool BESIDE>
 __global__ void __launch_bounds__(256)
 ssd_prepare_conv_kernel(const bf16_t* __restrict__ dt, long dt_ld, const float* __restrict__ dt_bias,
@@ -259,7 +260,7 @@ ssd_prepare_conv_kernel(const bf16_t* __restrict__ dt, long dt_ld, const float* 
 
 // The conv tail of a lane after its tokens: the last K-1 rows of [old tail ; the lane's raw rows]
 // (conv_state_update of mamba2.hip), one thread per channel; every old value is read before the first is written.
-__device__ void ssd_tail_block(const bf16_t* __restrict__ u, long u_ld, int C, int K, bf16_t* __restrict__ conv_state,
+__device__ __forceinline__ void ssd_tail_block(const bf16_t* __restrict__ u, long u_ld, int C, int K, bf16_t* __restrict__ conv_state,
                                const int* __restrict__ chunks, const int* __restrict__ lane_chunks,
                                const int* __restrict__ slot_ids, int Q, int lane, int channel) {
   if (channel >= C) return;
