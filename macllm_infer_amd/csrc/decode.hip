@@ -1299,8 +1299,11 @@ extern "C" int mi_fused_gemm_supported(int pro, int M, int K) {
 #define MX_MAX_PAGES 132       // page ids of one run of keys (at most MX_SPLIT_MOST / 8 + 2)
 #define MX_SPLIT_LEAST 256     // keys of one attention workgroup: between these two, see mi_mixer_split_keys
 #define MX_SPLIT_MOST 1024
-#define MX_WALK_BLOCKS 256      // attention workgroups from which on a workgroup walks over several runs
-#define MX_SPLIT_BLOCKS 128    // attention workgroups a step should at least have before its runs grow
+// attention workgroups from which on a workgroup walks over several runs, and those that a step should at least have before
+// its runs grow: a workgroup of heads of 128 moves twice the bytes of one of heads of 64
+#define MX_WALK_BLOCKS(dh) ((dh) == 128 ? 128 : 256)
+#define MX_SPLIT_BLOCKS(dh, groups) ((dh) == 128 && (groups) >= 16 ? 64 : 128)
+#define MX_WHOLE_SPAN 2048     // contexts up to which a large step gives a whole request to one workgroup, see mi_mixer_runs
 #define MX_SCAN_PER_THREAD 8
 #define MX_FEW_BLOCKS 512       // state-space workgroups of a step up to which each takes one row per thread group
 
@@ -1702,11 +1705,11 @@ __global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p)
 // 64 tokens at 2,100 keys 61.0 / 56.0 / 52.0, at 6,000 keys 100 / 85 / 80.  So: the longest run that still
 // leaves MX_SPLIT_BLOCKS workgroups (up to 512 keys for steps of up to 16 tokens, 1,024 beyond), and never
 // more than 16 runs for a request.  `span`: the most keys a request of the step can have.
-extern "C" int mi_mixer_split_keys(int M, int Hkv, int page_size, long span) {
-  if (M <= 0 || Hkv <= 0 || page_size <= 0 || span <= 0) return 0;
+extern "C" int mi_mixer_split_keys(int M, int Hkv, int dh, int page_size, long span) {
+  if (M <= 0 || Hkv <= 0 || dh <= 0 || page_size <= 0 || span <= 0) return 0;
   long split = MX_SPLIT_LEAST;
   for (long candidate = M <= 16 ? MX_SPLIT_MOST / 2 : MX_SPLIT_MOST; candidate > MX_SPLIT_LEAST; candidate /= 2)
-    if ((long)Hkv * M * ((span + candidate - 1) / candidate) >= MX_SPLIT_BLOCKS) {
+    if ((long)Hkv * M * ((span + candidate - 1) / candidate) >= MX_SPLIT_BLOCKS(dh, (long)Hkv * M)) {
       split = candidate;
       break;
     }
@@ -1718,12 +1721,23 @@ extern "C" int mi_mixer_split_keys(int M, int Hkv, int page_size, long span) {
 // The runs of keys of a step, as mi_mixer_decode cuts them: keys of a run and workgroups (partial results) per
 // (token, kv head): one per run while the step is small, fewer (each walks over several runs) once the step has
 // MX_WALK_BLOCKS of them anyway.  `span`: the most keys a request of the step can have.
-extern "C" int mi_mixer_runs(int M, int Hkv, int page_size, long span, int* run_keys, int* runs) {
-  const int keys = mi_mixer_split_keys(M, Hkv, page_size, span);
+// A step of half as many requests as that, or of heads of 128 a quarter, gives each request's kv head to one workgroup, which
+// writes the attended heads itself: the merge's launch (4.7 us) counts for more than the longer walk, up to contexts of
+// MX_WHOLE_SPAN keys.  Mixer and merge of a layer in us, several workgroups a request | one: heads of 64, 64 tokens behind
+// 300 keys 33.8 | 29.2, 1,500 39.9 | 34.9, 4,500 62.6 | 64.3; 32 tokens behind 1,500 24.9 | 26.5.  (Contexts of all lengths up to
+// 3,500 keys wait for the longest walk: a step of 64 of them takes 2,870 and 2,884.)  Heads
+// of 128 over states of 128 x 256, 32 tokens behind 300 keys 57.1 | 54.4, 1,500 64.9 | 58.8, but 4,000 88 | 92.  The line at
+// 128 workgroups for those heads (256 before | 128): 8 tokens behind 4,500 keys 37.7 | 33.8, 16 behind 2,500 48.9 | 42.8, behind
+// 4,500 63.0 | 50.4, 32 behind 2,500 79.0 | 71.0; their runs of 512 keys from 64 workgroups on (128 before | 64): 8 tokens
+// behind 300 keys 21.8 | 18.2, behind 1,500 26.2 | 23.7, but 4 behind 2,500 17.7 | 18.8.
+extern "C" int mi_mixer_runs(int M, int Hkv, int dh, int page_size, long span, int* run_keys, int* runs) {
+  const int keys = mi_mixer_split_keys(M, Hkv, dh, page_size, span);
   if (keys <= 0 || !run_keys || !runs) return ERR_BAD_ARGUMENT;
   const long whole = (span + keys - 1) / keys;
+  const long groups = (long)Hkv * M;
+  const long most = 2 * groups >= MX_WALK_BLOCKS(dh) && span <= MX_WHOLE_SPAN ? 1 : max(1L, (MX_WALK_BLOCKS(dh) + groups - 1) / groups);
   *run_keys = keys;
-  *runs = (int)min(whole, max(1L, (MX_WALK_BLOCKS + (long)Hkv * M - 1) / ((long)Hkv * M)));
+  *runs = (int)min(whole, most);
   return 0;
 }
 
@@ -1809,7 +1823,7 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
   p.ssm_out = (bf16_t*)ssm_out;
   p.ssm_y = ssm_y;
   p.out_ld = out_ld;
-  if (mi_mixer_runs(M, Hkv, page_size, span, &p.split_keys, &p.splits) != 0) return ERR_UNSUPPORTED_SIZE;
+  if (mi_mixer_runs(M, Hkv, dh, page_size, span, &p.split_keys, &p.splits) != 0) return ERR_UNSUPPORTED_SIZE;
   if ((long)Hkv * M * p.splits > 0x3fffffffL || M > 65535 || Hq > 65535) return ERR_UNSUPPORTED_SIZE;
   if (!partial || partial_floats < (long)M * Hq * p.splits * (dh + 2)) return ERR_BAD_ARGUMENT;
   p.partial = partial;

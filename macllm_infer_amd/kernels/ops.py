@@ -193,8 +193,8 @@ _SIGNATURES = {
                                 _c_ptr],
         "mi_shared_rows_gemm_split": [_c_ptr, _c_long, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_int,
                                       _c_int, _c_ptr],
-        "mi_mixer_split_keys": [_c_int, _c_int, _c_int, _c_long],
-        "mi_mixer_runs": [_c_int, _c_int, _c_int, _c_long, _c_ptr, _c_ptr],
+        "mi_mixer_split_keys": [_c_int, _c_int, _c_int, _c_int, _c_long],
+        "mi_mixer_runs": [_c_int, _c_int, _c_int, _c_int, _c_long, _c_ptr, _c_ptr],
         "mi_fused_gemm_merge": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_long, _c_ptr,
                                 _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_long, _c_int, _c_ptr, _c_ptr, _c_long, _c_ptr,
                                 _c_ptr, _c_ptr],
@@ -2455,11 +2455,11 @@ def mixer_decode_supported(num_heads: int, num_kv_heads: int, head_dim: int, pag
 MERGE_AT_ONCE = 8          # runs of keys a merge asks for at once (decode.hip)
 
 
-def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int):
+def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: int = 64):
     """(keys of a run, runs per token and kv head) as ``mixer_decode`` cuts the contexts of a step of M tokens
     whose requests hold up to ``span`` keys."""
     run_keys, runs = ctypes.c_int(0), ctypes.c_int(0)
-    _check(_fn("decode", "mi_mixer_runs")(M, num_kv_heads, page_size, span, ctypes.addressof(run_keys),
+    _check(_fn("decode", "mi_mixer_runs")(M, num_kv_heads, head_dim, page_size, span, ctypes.addressof(run_keys),
                                           ctypes.addressof(runs)), "mixer_decode", "(no run length for these sizes)")
     return run_keys.value, runs.value
 
@@ -2503,7 +2503,7 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
                  z_col + E, x_col + E + 2 * num_groups * state_size, dt_col + ssm_heads)
     _need(u.shape[1] >= widest, "mixer_decode: u is too narrow")
     span = max(1, int(max_seq_len)) if not window else window + page_size
-    run_keys, runs = mixer_runs(M, num_kv_heads, page_size, span)        # the launcher's own rule
+    run_keys, runs = mixer_runs(M, num_kv_heads, page_size, span, head_dim)        # the launcher's own rule
     partial = torch.empty((M * num_heads * runs * (head_dim + 2),), dtype=torch.float32, device=u.device)
     _check(_fn("decode", "mi_mixer_decode")(
         _p(u), u_ld, M, num_heads, num_kv_heads, head_dim, q_col, k_col, v_col, _p(inv_freq), rotary_dim,

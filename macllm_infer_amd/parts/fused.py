@@ -997,7 +997,7 @@ class AttentionMamba2Step:
         a = self.attention.spec
         rows, page_size = step.num_tokens, caches[self.attention_name].k_cache.shape[2]
         span = max(1, int(step.max_seq_len)) if not a.window else a.window + page_size
-        runs = ops.mixer_runs(rows, a.num_kv_heads, page_size, span)[1]
+        runs = ops.mixer_runs(rows, a.num_kv_heads, page_size, span, a.head_dim)[1]
         return a.num_heads * a.head_dim, rows * a.num_heads * min(runs, ops.MERGE_AT_ONCE) * (a.head_dim + 2) * 4
 
     def run(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, merge: bool = True):

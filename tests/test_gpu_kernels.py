@@ -1961,3 +1961,12 @@ def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
     assert not make(qkv=q.float()).fits(8, state, 128)
     assert not make(qkv=torch.zeros(8, 1028, dtype=torch.bfloat16, device=DEV)[:, 4:]).fits(8, state, 128)
     assert not make(sizes=(1, 2048, 2048)).fits(8, state, 128)                          # the kernel whose waves share their keys
+
+
+def test_runs_of_keys_go_by_the_heads_width_and_the_steps_size(ops):
+    """Where a large step gives a request's kv head to one workgroup (no merge), and the lines beside it."""
+    runs = lambda M, dh, span: ops.mixer_runs(M, 2, 16, span, dh)
+    assert runs(64, 64, 2048)[1] == 1 and runs(64, 64, 4096)[1] == 2 and runs(63, 64, 2048)[1] == 2 and runs(32, 64, 2048)[1] == 2
+    assert runs(32, 128, 2048)[1] == 1 and runs(32, 128, 4096)[1] == 2 and runs(16, 128, 2048)[1] == 4
+    assert runs(8, 128, 2048) == (512, 4) and runs(4, 128, 2048) == (256, 8) and runs(8, 64, 2048) == (256, 8)
+    assert runs(8, 128, 8192) == (512, 8) and runs(8, 64, 8192) == (512, 16)
