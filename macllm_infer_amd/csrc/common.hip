@@ -1234,138 +1234,6 @@ static void launch_add_layernorm_rows(int per, int n_rows, int threads, hipStrea
 #undef ROWS_CASE
 }
 
-template <int VEC>
-__device__ __forceinline__ void floats_at(const float* from, float (&to)[VEC]) {
-  if constexpr (VEC == 4) {
-    const float4 piece = *reinterpret_cast<const float4*>(from);
-    to[0] = piece.x; to[1] = piece.y; to[2] = piece.z; to[3] = piece.w;
-  } else {
-    to[0] = from[0];
-  }
-}
-
-typedef __bf16 common_bf16x4 __attribute__((ext_vector_type(4)));
-
-template <int VEC>
-__device__ __forceinline__ void add_branch(const NormBranch& branch, long at, float (&to)[VEC]) {
-  if (!branch.rows) return;
-  if (branch.dtype == DT_BF16) {
-    if constexpr (VEC == 4) {
-      const common_bf16x4 piece = *reinterpret_cast<const common_bf16x4*>((const bf16_t*)branch.rows + at);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) to[j] += branch.factor * (float)piece[j];
-    } else {
-      to[0] += branch.factor * (float)((const bf16_t*)branch.rows)[at];
-    }
-    return;
-  }
-  float piece[VEC];
-  floats_at<VEC>((const float*)branch.rows + at, piece);
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) to[j] += branch.factor * piece[j];
-}
-
-// The same in pieces of four columns, PIECES of them a thread in registers and all asked for at the start (rows of a
-// multiple of four columns at aligned addresses, up to 4,096): the order of the sums goes by d alone.  24 MB of traffic and
-// up to eight crossings of the workgroup, which fewer waves cross faster: 1,554 rows of 1,024 with a norm on the branch
-// 9.5 us through the first kernel, 8.0 here (without that norm 7.1 and 5.7);
-// 12 rows of 3,072 6.6 through the second, 5.5 here.
-template <typename TO, int PIECES, int THREADS>
-__global__ void __launch_bounds__(THREADS)
-add_layernorm_fours_kernel(float* __restrict__ h, NormBranch b0, NormBranch b1, NormBranch b2,
-                           const float* __restrict__ vector, const float* __restrict__ weight,
-                           const float* __restrict__ bias, float eps, const float* __restrict__ branch_weight,
-                           const float* __restrict__ branch_bias, float branch_eps, TO* __restrict__ out,
-                           const int* __restrict__ rows, int d) {
-  typedef TO four __attribute__((ext_vector_type(4)));
-  __shared__ float scratch[16];
-  const long out_row = blockIdx.x;
-  const long row = rows ? (long)rows[out_row] : out_row;
-  float branch[PIECES][4], v[PIECES][4], bw[PIECES][4], bb[PIECES][4], w[PIECES][4], b[PIECES][4], extra[PIECES][4];
-#pragma unroll
-  for (int k = 0; k < PIECES; ++k) {
-    const int i = ((int)threadIdx.x + k * THREADS) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) branch[k][j] = v[k][j] = bw[k][j] = bb[k][j] = w[k][j] = b[k][j] = extra[k][j] = 0.f;
-    if (i < d) {
-      add_branch<4>(b0, row * d + i, branch[k]);
-      add_branch<4>(b1, row * d + i, branch[k]);
-      add_branch<4>(b2, row * d + i, branch[k]);
-      floats_at<4>(h + row * d + i, v[k]);
-      if (branch_weight) {
-        floats_at<4>(branch_weight + i, bw[k]);
-        floats_at<4>(branch_bias + i, bb[k]);
-      }
-      if (out) {
-        floats_at<4>(weight + i, w[k]);
-        floats_at<4>(bias + i, b[k]);
-      }
-      if (vector) floats_at<4>(vector + i, extra[k]);
-    }
-  }
-  auto mean_of = [&](const float (&x)[PIECES][4]) {
-    float sum = 0.f;
-#pragma unroll
-    for (int k = 0; k < PIECES; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum += x[k][j];                    // (columns past the end hold zeros)
-    return block_sum(sum, scratch) / (float)d;
-  };
-  auto deviation_of = [&](const float (&x)[PIECES][4], float mean, float least) {
-    float squares = 0.f;
-#pragma unroll
-    for (int k = 0; k < PIECES; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float centred = ((int)threadIdx.x + k * THREADS) * 4 < d ? x[k][j] - mean : 0.f;
-        squares += centred * centred;
-      }
-    return sqrtf(block_sum(squares, scratch) / (float)d + least);
-  };
-  if (branch_weight) {
-    const float mean = mean_of(branch);
-    const float denominator = deviation_of(branch, mean, branch_eps);
-#pragma unroll
-    for (int k = 0; k < PIECES; ++k)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) branch[k][j] = (branch[k][j] - mean) / denominator * bw[k][j] + bb[k][j];
-  }
-#pragma unroll
-  for (int k = 0; k < PIECES; ++k) {
-    const int i = ((int)threadIdx.x + k * THREADS) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[k][j] = i < d ? v[k][j] + branch[k][j] + extra[k][j] : 0.f;
-    if (i < d && !rows) *reinterpret_cast<float4*>(h + row * d + i) = make_float4(v[k][0], v[k][1], v[k][2], v[k][3]);
-  }
-  if (!out) return;
-  const float mean = mean_of(v);
-  const float denominator = deviation_of(v, mean, eps);
-#pragma unroll
-  for (int k = 0; k < PIECES; ++k) {
-    const int i = ((int)threadIdx.x + k * THREADS) * 4;
-    if (i >= d) continue;
-    four piece;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) piece[j] = from_float<TO>((v[k][j] - mean) / denominator * w[k][j] + b[k][j]);
-    *reinterpret_cast<four*>(out + out_row * d + i) = piece;
-  }
-}
-
-template <typename TO>
-static void launch_add_layernorm_fours(int n_rows, hipStream_t stream, float* h, NormBranch b0, NormBranch b1,
-                                       NormBranch b2, const float* vector, const float* weight, const float* bias,
-                                       float eps, const float* branch_weight, const float* branch_bias,
-                                       float branch_eps, TO* out, const int* rows, int d) {
-#define FOURS_CASE(PIECES_, THREADS_)                                                                            \
-  if (d <= 4 * PIECES_ * THREADS_) {                                                                             \
-    add_layernorm_fours_kernel<TO, PIECES_, THREADS_><<<n_rows, THREADS_, 0, stream>>>(                          \
-        h, b0, b1, b2, vector, weight, bias, eps, branch_weight, branch_bias, branch_eps, out, rows, d);         \
-    return;                                                                                                      \
-  }
-  FOURS_CASE(1, 256) FOURS_CASE(1, 512) FOURS_CASE(2, 512)
-#undef FOURS_CASE
-}
-
 extern "C" int mi_add_layernorm(float* h, const void* rows0, int dtype0, float factor0, const void* rows1, int dtype1,
                                 float factor1, const void* rows2, int dtype2, float factor2, const float* vector,
                                 const float* weight, const float* bias, float eps, const float* branch_weight,
@@ -1376,20 +1244,6 @@ extern "C" int mi_add_layernorm(float* h, const void* rows0, int dtype0, float f
   if (branch_weight && (!branch_bias || rows || !rows0)) return ERR_BAD_ARGUMENT;
   if ((size_t)d * sizeof(float) > 64 * 1024) return ERR_UNSUPPORTED_SIZE;
   const NormBranch b0 = {rows0, dtype0, factor0}, b1 = {rows1, dtype1, factor1}, b2 = {rows2, dtype2, factor2};
-  const uintptr_t addresses = (uintptr_t)h | (uintptr_t)rows0 | (uintptr_t)rows1 | (uintptr_t)rows2 | (uintptr_t)vector |
-                              (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)branch_weight | (uintptr_t)branch_bias |
-                              (uintptr_t)out;
-  // (a few rows of up to 1,024 numbers stay with one number a thread: 12 rows in a decode step 4.1 us there, 4.3 in pieces)
-  if (d % 4 == 0 && d <= 4096 && (n_rows > 256 || d > 1024) && addresses % 16 == 0 && (out_dtype == DT_F32 || out_dtype == DT_BF16)) {
-    if (out_dtype == DT_F32)
-      launch_add_layernorm_fours<float>(n_rows, stream, h, b0, b1, b2, vector, weight, bias, eps, branch_weight, branch_bias,
-                                        branch_eps, (float*)out, rows, d);
-    else
-      launch_add_layernorm_fours<bf16_t>(n_rows, stream, h, b0, b1, b2, vector, weight, bias, eps, branch_weight, branch_bias,
-                                         branch_eps, (bf16_t*)out, rows, d);
-    RETURN_IF_LAUNCH_FAILED();
-    return 0;
-  }
   if (n_rows <= 256 && d <= 8192 && (out_dtype == DT_F32 || out_dtype == DT_BF16)) {
     // few rows: the kernel that keeps a row in registers, as many threads as a row has elements where that fits
     const int per = d <= 1024 ? 1 : d <= 2048 ? 2 : d <= 4096 ? 4 : 8;
@@ -1422,6 +1276,37 @@ extern "C" int mi_add_layernorm(float* h, const void* rows0, int dtype0, float f
 // are gathered); out (if wanted) = v / sqrt(mean(v^2) + eps) * weight.  One workgroup a row, which stays in registers: a
 // thread keeps CHUNKS pieces of VEC neighbouring elements (piece threadIdx.x + k * blockDim.x), and everything the later
 // stages read from memory is asked for at the start, beside the branches' rows.
+template <int VEC>
+__device__ __forceinline__ void floats_at(const float* from, float (&to)[VEC]) {
+  if constexpr (VEC == 4) {
+    const float4 piece = *reinterpret_cast<const float4*>(from);
+    to[0] = piece.x; to[1] = piece.y; to[2] = piece.z; to[3] = piece.w;
+  } else {
+    to[0] = from[0];
+  }
+}
+
+typedef __bf16 common_bf16x4 __attribute__((ext_vector_type(4)));
+
+template <int VEC>
+__device__ __forceinline__ void add_branch(const NormBranch& branch, long at, float (&to)[VEC]) {
+  if (!branch.rows) return;
+  if (branch.dtype == DT_BF16) {
+    if constexpr (VEC == 4) {
+      const common_bf16x4 piece = *reinterpret_cast<const common_bf16x4*>((const bf16_t*)branch.rows + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) to[j] += branch.factor * (float)piece[j];
+    } else {
+      to[0] += branch.factor * (float)((const bf16_t*)branch.rows)[at];
+    }
+    return;
+  }
+  float piece[VEC];
+  floats_at<VEC>((const float*)branch.rows + at, piece);
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) to[j] += branch.factor * piece[j];
+}
+
 template <typename TO, int CHUNKS, int VEC>
 __global__ void __launch_bounds__(1024)
 add_normed_rmsnorm_kernel(float* __restrict__ h, NormBranch b0, NormBranch b1, NormBranch b2,

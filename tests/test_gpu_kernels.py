@@ -1860,7 +1860,7 @@ def test_scan_gives_the_same_bits_however_its_tokens_are_cut(ops, dtype, N):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T", [3, 300])
 @pytest.mark.parametrize("d", [4, 1020, 1022, 1024, 1028, 2052, 4096, 4100])
-def test_layer_norm_in_pieces_of_four(ops, dtype, T, d):
+def test_layer_norm_of_the_stream_and_its_branches(ops, dtype, T, d):
     h, vector = rand(T, d, seed=1), rand(d, seed=2)
     first, second = rand(T, d, seed=3, dtype=dtype), rand(T, d, seed=4)
     weight, bias, bw, bb = (rand(d, seed=seed) for seed in (5, 6, 7, 8))
@@ -1887,7 +1887,7 @@ def test_layer_norm_in_pieces_of_four(ops, dtype, T, d):
             gathered = torch.empty(3, d, dtype=dtype, device=DEV)
             ops.add_layernorm(dh, branches, dv, dw, db, 1e-5, gathered, rows=rows)
             assert torch.equal(dh.cpu(), h)
-            if d % 4 == 0 and (d <= 4096 and (d > 1024 or T <= 256)):     # (the sums of other rows go by the number of rows too)
+            if T <= 256:                                 # (of more rows the sums go in another order than of three)
                 assert torch.equal(gathered, out[[T - 1, 0, T - 1]])
             assert ((gathered.cpu().double() - want[[T - 1, 0, T - 1]]).abs() <= share * want[[T - 1, 0, T - 1]].abs() + 1e-4).all()
 
@@ -1961,6 +1961,43 @@ def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
     assert not make(qkv=q.float()).fits(8, state, 128)
     assert not make(qkv=torch.zeros(8, 1028, dtype=torch.bfloat16, device=DEV)[:, 4:]).fits(8, state, 128)
     assert not make(sizes=(1, 2048, 2048)).fits(8, state, 128)                          # the kernel whose waves share their keys
+
+
+@pytest.mark.parametrize("T, d", [(257, 64), (300, 1024), (300, 1028), (513, 2052)])
+def test_layer_norm_of_many_rows_adds_a_row_up_in_one_order(ops, T, d):
+    """The bits of more than 256 rows: number i of a row belongs to thread i % 256, a thread's numbers are added one after the
+    other, the lanes of a wave in halves, the four waves from the first on.  (Behind such a norm a router chooses experts: another
+    order of the sums turns a choice, and with it a whole row of logits.)"""
+    import numpy as np
+    h, branch, weight, bias = rand(T, d, seed=1), rand(T, d, seed=2), rand(d, seed=3), rand(d, seed=4)
+    f32 = np.float32
+    v = (h.numpy() + branch.numpy()).astype(f32)
+
+    def total(numbers, squared):
+        sums = np.zeros((T, 256), dtype=f32)
+        for first in range(0, d, 256):
+            piece = numbers[:, first:first + 256].astype(np.float64)
+            # (a product and a sum with one rounding: float64 holds the product whole)
+            added = (sums[:, :piece.shape[1]].astype(np.float64) + (piece * piece if squared else piece)).astype(f32)
+            sums[:, :piece.shape[1]] = added
+        waves = sums.reshape(T, 4, 64)
+        while waves.shape[2] > 1:
+            half = waves.shape[2] // 2
+            waves = waves[:, :, :half] + waves[:, :, half:]
+        out = np.zeros(T, dtype=f32)
+        for wave in range(4):
+            out = out + waves[:, wave, 0]
+        return out
+    mean = total(v, False) / f32(d)
+    centred = v - mean[:, None]
+    denominator = np.sqrt(total(centred, True) / f32(d) + f32(1e-5))
+    share = centred / denominator[:, None]
+    want = (share.astype(np.float64) * weight.numpy() + bias.numpy()).astype(f32)
+    dh, d1, dw, db = gpu(h, branch, weight, bias)
+    out = torch.empty(T, d, device=DEV)
+    ops.add_layernorm(dh, [(d1, 1.0)], None, dw, db, 1e-5, out)
+    assert torch.equal(dh.cpu(), torch.from_numpy(v))
+    assert torch.equal(out.cpu(), torch.from_numpy(want))
 
 
 def test_runs_of_keys_go_by_the_heads_width_and_the_steps_size(ops):
