@@ -27,10 +27,10 @@ from ..config.spec import ConfigError
 from ..kernels import build as kernel_build
 from ..kernels import ops
 from ..parts.base import BuildContext
-from ..parts.block import OVERLAP_MIN_TOKENS
+from ..parts.streams import SECOND_HALF, SINGLES
 from ..weights.loader import WeightSource, bind
 from .context import Lane, LoweredLanes, apply_feeds, build_step_context, longest_context, lower_lanes
-from .graphs import BESIDE_CANDIDATES, SINGLES, DecodeGraphs, replayed_beside
+from .graphs import DecodeGraphs, replayed_beside
 from .model import DecoderModel
 
 _DTYPES = {"bfloat16": torch.bfloat16, "bf16": torch.bfloat16, "float32": torch.float32, "fp32": torch.float32,
@@ -85,6 +85,7 @@ SPLIT_NEVER = 1 << 30
 HALVES_FROM_LANES = 65
 HALVES_MOST_LANES = 128        # beyond, a half would leave the skinny kernels too: one graph, as measured for no such size
 HALVES_MARGIN = 0.95
+CALLERS_STREAMS = 32           # callers' streams whose second streams are remembered
 
 
 def split_from_lanes(lane_share: Optional[float]) -> int:
@@ -146,8 +147,7 @@ class Engine:
         self.max_context = self.spec.max_context
         self.graphs = None
         self.graphs_beside = None                    # the graphs of the second half of a step that runs as two halves at once
-        self._beside = {}                            # and the streams they are replayed on, by the caller's stream
-        self._beside_portions = []                   # the streams among which the clock finds one for single tokens beside portions
+        self._beside = {}                            # the streams that a step's second batch may be queued on, by the caller's stream
         self._in_halves: Optional[bool] = None
         self.halves_share: Optional[float] = None
         # the pool bounds a request's length only where some layer keeps every key: a model whose attention
@@ -163,7 +163,7 @@ class Engine:
         the clock when it is first needed (or by ``warm_up``), where there is one."""
         if self._split_from_lanes is None:
             if self._measure_split and self.graphs is not None:
-                self.lane_share = self.graphs.measure_split(self._candidates())
+                self.lane_share = self.graphs.measure_split(self._streams_beside())
                 self._split_from_lanes = split_from_lanes(self.lane_share) if self.lane_share is not None else SPLIT_NEVER
             else:
                 self._split_from_lanes = split_from_lanes(None)
@@ -180,7 +180,7 @@ class Engine:
         if self._in_halves is None:
             self._in_halves = False
             if self._measure_split and self.graphs is not None:
-                self.halves_share = self.graphs.measure_halves(self._second_stream())
+                self.halves_share = self.graphs.measure_halves(self._streams_beside()[0])
                 self._in_halves = self.halves_share is not None and self.halves_share < HALVES_MARGIN
         return self._in_halves
 
@@ -338,25 +338,26 @@ class Engine:
             logits = self.model.forward(context, self.cache)
         return logits
 
-    def _second_stream(self) -> torch.cuda.Stream:
-        """The stream that a step's second half is queued on, beside the caller's: found by the clock when a caller's
-        stream first needs one."""
+    def _streams_beside(self) -> list:
+        """The streams that a step's second batch may be queued on.  Kernels on the first of them run beside those of the
+        caller's stream: the clock is asked when a caller's stream first needs one."""
         main = torch.cuda.current_stream(self.device)
         if main.cuda_stream not in self._beside:
-            self._beside[main.cuda_stream] = ops.stream_beside(main)
+            others = [stream for stream in self.graphs.streams.beside if stream != main]
+            first = ops.stream_beside(main, others)
+            if len(self._beside) >= CALLERS_STREAMS:
+                self._beside.clear()
+            self._beside[main.cuda_stream] = [first] + [stream for stream in others if stream != first]
         return self._beside[main.cuda_stream]
 
-    def _candidates(self) -> list:
-        """The streams that the single tokens beside portions of prompts may be queued on."""
-        if not self._beside_portions:
-            self._beside_portions = [torch.cuda.Stream(device=self.device) for _ in range(BESIDE_CANDIDATES + 1)]
-        main = torch.cuda.current_stream(self.device)
-        return [stream for stream in self._beside_portions if stream != main][:BESIDE_CANDIDATES]
+    def _apart(self) -> bool:
+        """Whether single tokens may run beside portions: the caller's stream must be none that the single tokens' graphs
+        use (a portion that is launched kernel by kernel leaves a library's workspace there)."""
+        return self.graphs is not None and not self.graphs.streams.belongs_to(SINGLES, torch.cuda.current_stream(self.device))
 
     def _make_graphs_beside(self) -> None:
         if self.graphs_beside is None:
-            apart = [self.graphs._capture_stream(SINGLES)]
-            self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len, apart)
+            self.graphs_beside = DecodeGraphs(self.model, self.cache, self.device, self.graphs.max_seq_len, SECOND_HALF)
 
     def _run_in_halves(self, lanes: Sequence[Lane]) -> torch.Tensor:
         """A step of many single decoded tokens as two halves at once: the second half's graph is replayed on a
@@ -369,7 +370,7 @@ class Engine:
         half = (len(lanes) + 1) // 2
         first, second = list(lanes[:half]), list(lanes[half:])
         lowered_second = self.validate(second)
-        beside = self._second_stream()
+        beside = self._streams_beside()[0]
         try:
             with replayed_beside(main, beside):
                 rows_second = self._run(second, lowered_second, self.graphs_beside)
@@ -385,22 +386,22 @@ class Engine:
         """A step that holds portions of prompts beside several single decoded tokens, as two batches side by side:
         the portions through the prompt kernels, and on a second stream the single tokens through the graph of a decode
         step, whose small kernels wait for each other most of their time (515 prompt tokens of the 0.5B shape beside 24 decoded
-        ones: 4.8 ms, 6.1 with one batch behind the other).  (As one batch the prompt kernels take every single token as
+        ones: 4.8 ms, 6.1 with one batch behind the other; beside 130, whose graph of 256 rows forks too, 7.2 and 9.4).  (As one batch the prompt kernels take every single token as
         a prompt of its own, a tile of the attention kernel and a chunk of the scan each: 2,048 prompt tokens beside 63
         decoded ones took 19.4 ms, where the two batches take 6.3 and 3.1.)  The batches belong to different requests,
-        and graphs of the two kinds share neither a memory pool nor a library's workspace.  (From OVERLAP_MIN_TOKENS single
-        tokens on, whose mixers may use a second stream themselves, the batches follow each other.)  The logits come
+        and what they are recorded, warmed up and forked on are streams of their own, by which they share neither a memory pool
+        nor a library's workspace (``BatchStreams``).  Where they are not, the batches follow each other.  The logits come
         back in the order of the lanes."""
         batches = []
         for chosen in (~single, single):
             members = [lane for lane, mine in zip(lanes, chosen) if mine]
             batches.append((members, self.validate(members)))
         portions, singles = batches
-        if self.graphs is None or len(singles[0]) >= OVERLAP_MIN_TOKENS:
+        if not self._apart():
             parts = [self._run(*portions), self._run(*singles)]
         else:
             main = torch.cuda.current_stream(self.device)
-            beside = self.graphs.stream_beside(portions[0], portions[1], singles[1], self._candidates())
+            beside = self.graphs.stream_beside(portions[0], portions[1], singles[1], self._streams_beside())
             try:
                 with replayed_beside(main, beside):
                     rows_of_singles = self._run(*singles)

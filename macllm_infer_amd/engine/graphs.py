@@ -28,6 +28,7 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
 
+from ..parts.streams import PORTIONS, SECOND_HALF, SINGLES, batch_streams
 from .context import _NO_LANES, Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
 
 
@@ -63,17 +64,6 @@ def token_capacities(most: int) -> List[int]:
         value += max(16, power // (8 if value >= 1024 else 4))
 
 
-SINGLES, PORTIONS = "single tokens", "portions"          # kinds of captured steps
-
-
-# The runtime lays its streams on a few hardware queues (four by default), in turn, and what lies on one queue runs one
-# after the other.  A graph of a long portion runs its mixers on two queues, of which the second is the runtime's own
-# choice when the graph is made: of four streams made in a row some stand in the way of one of the two, and the clock
-# says which does not (515 prompt tokens of the 0.5B shape beside 24 decoded ones: 4.8 ms on two of four streams, 6.05 on
-# the others).
-BESIDE_CANDIDATES = 4
-
-
 @contextmanager
 def replayed_beside(main: torch.cuda.Stream, beside: torch.cuda.Stream):
     """What is queued inside goes onto ``beside``, behind everything that ``main`` holds so far."""
@@ -83,21 +73,21 @@ def replayed_beside(main: torch.cuda.Stream, beside: torch.cuda.Stream):
 
 
 class DecodeGraphs:
-    def __init__(self, model, cache, device, max_seq_len: int, apart_from: Sequence[torch.cuda.Stream] = ()):
-        """``apart_from``: streams on which other graphs are recorded that are replayed beside these."""
+    def __init__(self, model, cache, device, max_seq_len: int, singles: str = SINGLES):
+        """``singles``: the kind of its graphs of single tokens (``SECOND_HALF``: they are replayed beside those of another
+        bank of graphs)."""
         self.model = model
-        self.apart_from = tuple(apart_from)
+        self.singles = singles
+        self.streams = batch_streams(torch.device(device))
         self.cache = cache
         self.device = device
         self.max_seq_len = max_seq_len
         self._graphs: Dict[tuple, tuple] = {}
         self._bucket_graphs: "OrderedDict[tuple, tuple]" = OrderedDict()
         self._seen: "OrderedDict[tuple, int]" = OrderedDict()
-        # graphs of single tokens and graphs of portions are replayed beside each other (``Engine._run_in_two``): each
-        # kind has a memory pool of its own and is recorded on a stream of its own, by which the libraries keep
-        # their workspaces apart
+        # graphs of two kinds are replayed beside each other (``Engine._run_in_two``, ``Engine._run_in_halves``): each kind
+        # has a memory pool of its own, and streams of its own that it is recorded and forked on (see ``BatchStreams``)
         self._pools: Dict[str, object] = {}
-        self._streams: Dict[str, torch.cuda.Stream] = {}
         self._besides: Dict[tuple, Dict[int, torch.cuda.Stream]] = {}
         self.counts = {"decode_replays": 0, "bucket_replays": 0, "bucket_captures": 0, "bucket_eager": 0}
 
@@ -247,7 +237,7 @@ class DecodeGraphs:
             # (a memory pool of its own: the graphs' shared pool ends with the last graph in it)
             captured.append(self._capture(0, static, warm_runs=1, pool=torch.cuda.graph_pool_handle(), kind=kind))
         portion, both = self._clock(captured[0][1].replay, replays), self._clock(captured[1][1].replay, replays)
-        two = min(self._clock_beside(captured[0][1], captured[2][1], stream, replays) for stream in candidates)
+        two = min(self._clock_beside(captured[0][1], captured[2][1], stream, replays) for stream in candidates[:4])
         del captured
         if both <= portion:
             return None
@@ -306,7 +296,7 @@ class DecodeGraphs:
         context = min(CONTEXT_BUCKET_FROM, self.max_seq_len)
         whole = self._capture(bucket_for(lanes), context=context, warm_runs=1, pool=torch.cuda.graph_pool_handle())
         halves = [self._capture(bucket_for((lanes + 1) // 2), context=context, warm_runs=1,
-                                pool=torch.cuda.graph_pool_handle()) for _ in range(2)]
+                                pool=torch.cuda.graph_pool_handle(), kind=kind) for kind in (SINGLES, SECOND_HALF)]
         main = torch.cuda.current_stream(self.device)
 
         def as_one():
@@ -322,42 +312,27 @@ class DecodeGraphs:
         del whole, halves
         return two / one if one > 0 else None
 
-    def _capture_stream(self, kind: str) -> torch.cuda.Stream:
-        if kind not in self._streams:
-            usual = torch.cuda.graph.default_capture_stream           # the one torch records graphs on by default
-            if usual is None:
-                usual = torch.cuda.graph.default_capture_stream = torch.cuda.Stream(device=self.device)
-            if kind == SINGLES and not self.apart_from:
-                self._streams[kind] = usual
-            else:
-                # (streams come from a pool that hands them out in turn)
-                taken = [torch.cuda.current_stream(self.device), usual] + list(self._streams.values()) + list(self.apart_from)
-                stream = torch.cuda.Stream(device=self.device)
-                while stream in taken:
-                    stream = torch.cuda.Stream(device=self.device)
-                self._streams[kind] = stream
-        return self._streams[kind]
-
     def _capture(self, bucket: int, static: Optional[StaticStep] = None, warm_runs: int = 2, context: int = 0,
                  pool=None, kind: Optional[str] = None):
-        kind = kind or (PORTIONS if static is not None and static.capacity else SINGLES)
+        kind = kind or (PORTIONS if static is not None and static.capacity else self.singles)
         if static is None:
             static = StaticStep(self.cache, bucket, context or self.max_seq_len, self.device,
                                 **self.model.step_layout)
         # a first run outside the graph lets the libraries set themselves up; every lane is padding,
-        # so only the scratch page and slot are touched
-        side = torch.cuda.Stream(device=self.device)
-        side.wait_stream(torch.cuda.current_stream(self.device))
-        with torch.cuda.stream(side):
+        # so only the scratch page and slot are touched.  It runs on the kind's own stream: a graph of another kind may be
+        # under way, and the library's workspace on a stream drawn for the moment might be that graph's
+        stream = self.streams.recording[kind]
+        stream.wait_stream(torch.cuda.current_stream(self.device))
+        with torch.cuda.stream(stream):
             for _ in range(warm_runs):
                 self.model.forward(static.context, self.cache)
-        torch.cuda.current_stream(self.device).wait_stream(side)
+        torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
         # one pool for every graph of a kind: their replays never overlap, so their intermediate buffers may share memory
         if pool is None:
             pool = self._pools.setdefault(kind, torch.cuda.graph_pool_handle())
-        with torch.cuda.graph(graph, pool=pool, stream=self._capture_stream(kind)):
+        with torch.cuda.graph(graph, pool=pool, stream=stream):
             logits = self.model.forward(static.context, self.cache)
         return static, graph, logits
 

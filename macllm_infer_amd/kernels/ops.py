@@ -340,16 +340,13 @@ def feed_tokens(token_ids: torch.Tensor, source: torch.Tensor, dst: Sequence[int
            "feed_tokens")
 
 
-def stream_beside(main: "torch.cuda.Stream", candidates: int = 8, microseconds: int = 200) -> "torch.cuda.Stream":
-    """A stream (default priority) whose kernels run beside those of ``main``.  The runtime lays its streams on a few
-    hardware queues, and what lies on one queue runs one after the other: of up to ``candidates`` streams the first on
-    which a wait of so many microseconds is over together with one on ``main`` (or, if none is, the last)."""
+def stream_beside(main: "torch.cuda.Stream", candidates: Sequence["torch.cuda.Stream"], microseconds: int = 200) -> "torch.cuda.Stream":
+    """Of ``candidates`` (none of them ``main``) a stream whose kernels run beside those of ``main``.  The runtime lays its
+    streams on a few hardware queues, and what lies on one queue runs one after the other: the first on which a wait
+    of so many microseconds is over together with one on ``main`` (or, if none is, the last)."""
     wait = _fn("common", "mi_wait")
     with torch.cuda.device(main.device):
-        for _ in range(candidates):
-            beside = torch.cuda.Stream(device=main.device)
-            if beside == main:
-                continue
+        for beside in candidates:
             took = []
             for _ in range(2):                       # the first round warms both streams up
                 torch.cuda.synchronize(main.device)

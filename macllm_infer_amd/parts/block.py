@@ -7,6 +7,7 @@ import torch
 
 from ..weights.loader import Expect
 from .base import BuildContext, NormedBranches, NormedRows, Residual, ScaledBranch, StreamTail, WeightedBranch, part_class
+from .streams import batch_streams
 
 _ARRANGEMENTS: Dict[str, type] = {}
 _FUSIONS: Dict[str, object] = {}
@@ -16,16 +17,21 @@ _side_streams: Dict[int, list] = {}
 
 
 def side_stream(device: torch.device, beside: "torch.cuda.Stream") -> "torch.cuda.Stream":
-    """A second stream of the device (default priority) that is not ``beside``.  Streams come from a pool of a
-    few dozen that hands them out in turn, so the one drawn may be the very stream a graph is being captured on:
-    work recorded "beside" it would queue behind (a 2,048-token prompt of the 0.5B shape: 7.2 ms instead of 6.3)."""
+    """The stream (default priority) that work on ``beside`` forks to, which is not ``beside`` itself (work recorded "beside"
+    it would queue behind: a 2,048-token prompt of the 0.5B shape took 7.2 ms instead of 6.3).  Every kind of batch that may
+    run beside another one has a stream of its own for it (``streams.BatchStreams``); work on any other stream forks
+    to one of two that belong to no such batch."""
     index = device.index if device.index is not None else torch.cuda.current_device()
+    batches = batch_streams(device)
+    side = batches.side_of(beside)
+    if side is not None:
+        return side
     streams = _side_streams.setdefault(index, [])
     for stream in streams:
         if stream != beside:
             return stream
     while True:
-        streams.append(torch.cuda.Stream(device=device))
+        streams.append(batches.apart())
         if streams[-1] != beside:
             return streams[-1]
 

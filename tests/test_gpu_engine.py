@@ -1302,6 +1302,45 @@ def test_long_portions_overlap_their_mixers(tmp_path, name):
     assert engine.graphs.counts["bucket_replays"] >= 5
 
 
+@pytest.mark.parametrize("name, dtype", [("A", "float32"), ("D", "bfloat16")])
+@pytest.mark.parametrize("count", [40, 130])
+def test_single_tokens_beside_portions_give_the_bits_of_one_batch_behind_the_other(tmp_path, monkeypatch, name, dtype, count):
+    """A portion of 300 tokens, whose graph forks, beside 40 decoded tokens and beside 130, whose graph of 256 rows forks too:
+    launched kernel by kernel, captured and replayed, the caller on the default stream and on streams of torch's pool
+    (on the one that the single tokens' graphs are recorded on, one batch behind the other), the same bits as an engine that never runs two
+    batches at once."""
+    from macllm_infer_amd import Engine, Lane
+    folder = tiny_configs.make_model_dir(name, tmp_path, torch.float32 if dtype == "float32" else torch.bfloat16)
+    cfg, _ = plain_impl.load_model_dir(folder)
+    make = lambda: Engine(folder, dtype=dtype, kv_cache_block_tokens=16, kv_cache_capacity_tokens=4096 + 32 * count,
+                          max_active_sequences=count + 2, measured_paths=False)
+    two, one = make(), make()
+    assert two.split_from_lanes == one.split_from_lanes == 4
+    beside = []
+    real = two._apart
+    monkeypatch.setattr(two, "_apart", lambda: (beside.append(real()), beside[-1])[1])
+    monkeypatch.setattr(one, "_apart", lambda: False)
+    streams = [torch.cuda.current_stream()] * 4 + [torch.cuda.Stream() for _ in range(2)] + [two.graphs.streams.recording["single tokens"]]
+    for engine in (two, one):
+        for index in range(count):
+            engine.add_request(index)
+        for first in range(0, count, 20):
+            engine.step([Lane(index, tokens_for(cfg["vocab_size"], 3 + index % 5, index)) for index in range(first, min(first + 20, count))])
+    for turn, stream in enumerate(streams):
+        lanes = [Lane(index, [(7 * index + turn) % cfg["vocab_size"]], [0]) for index in range(count)]
+        lanes.insert(3, Lane(f"prompt {turn}", tokens_for(cfg["vocab_size"], 300, 3000 + turn), [0, 299]))
+        rows = []
+        for engine in (two, one):
+            engine.add_request(f"prompt {turn}")
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                rows.append(engine.step(lanes).cpu())
+            engine.finish(f"prompt {turn}")
+        assert rows[0].shape[0] == count + 2 and torch.equal(rows[0], rows[1]), turn
+    assert beside == [True] * 6 + [False]
+    assert two.graphs.counts["bucket_replays"] >= 5 and two.graphs._besides
+
+
 def test_the_second_stream_is_never_the_stream_it_runs_beside(monkeypatch):
     """Streams come from a pool that hands them out in turn; whichever of them a graph is captured on, the
     stream that the first mixer of a long portion runs on is another one (on the same one the two mixers

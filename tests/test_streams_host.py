@@ -1,0 +1,139 @@
+"""Batches that run at once share no stream that a library keeps a workspace by: over a stand-in for torch's pool of
+streams, which hands 32 of them out in turn."""
+import contextlib
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from macllm_infer_amd.engine import engine as engine_module
+from macllm_infer_amd.engine import graphs as graphs_module
+from macllm_infer_amd.parts import block, streams
+
+POOL = 32
+DEVICE = torch.device("cuda", 0)
+
+
+class FakeStream:
+    turn = 0
+
+    def __init__(self, device=None, number=None):
+        if number is None:
+            number = FakeStream.turn % POOL
+            FakeStream.turn += 1
+        self.number, self.device, self.cuda_stream = number, DEVICE, 1000 + number
+
+    def __eq__(self, other):
+        return self.number == other.number
+
+    def __hash__(self):
+        return self.number
+
+    def wait_stream(self, other):
+        pass
+
+
+@pytest.fixture()
+def cuda(monkeypatch):
+    """torch.cuda's streams and captures without a GPU; ``current`` is the stream that work would be queued on."""
+    state = SimpleNamespace(current=FakeStream(number=-1))
+
+    @contextlib.contextmanager
+    def on(stream):
+        before, state.current = state.current, stream
+        try:
+            yield
+        finally:
+            state.current = before
+
+    class FakeGraph:
+        default_capture_stream = None
+
+        def __init__(self, graph, pool=None, stream=None):
+            if stream is None and FakeGraph.default_capture_stream is None:
+                FakeGraph.default_capture_stream = FakeStream()
+            self.on = on(stream if stream is not None else FakeGraph.default_capture_stream)
+
+        def __enter__(self):
+            return self.on.__enter__()
+
+        def __exit__(self, *error):
+            return self.on.__exit__(*error)
+
+    FakeStream.turn = 0
+    for name, value in (("Stream", FakeStream), ("stream", on), ("graph", FakeGraph), ("CUDAGraph", object),
+                        ("current_stream", lambda device=None: state.current), ("synchronize", lambda device=None: None),
+                        ("graph_pool_handle", object), ("current_device", lambda: 0)):
+        monkeypatch.setattr(torch.cuda, name, value)
+    monkeypatch.setattr(block, "_side_streams", {})
+    monkeypatch.setattr(streams, "_of_device", {})
+    return state
+
+
+def captures(state, kind, drawn_between=0):
+    """A function that captures a graph of ``kind`` and returns the streams worked on so far, warm-up and fork included."""
+    used = set()
+
+    def forward(context, cache):
+        used.add(state.current)
+        used.add(block.side_stream(DEVICE, state.current))
+    bank = graphs_module.DecodeGraphs(SimpleNamespace(forward=forward, blocks=[], step_layout={}), None, DEVICE, 4096)
+
+    def capture():
+        for _ in range(drawn_between):
+            FakeStream()
+        bank._capture(0, SimpleNamespace(capacity=kind == "portions", context=None))
+        return used
+    return capture
+
+
+@pytest.mark.parametrize("drawn_between", [0, 1, 2, 5])
+def test_no_capture_of_portions_works_on_a_stream_of_the_single_tokens(cuda, drawn_between):
+    """33 captures in a row, other parts of the program drawing streams in between, while single tokens may be under way."""
+    singles = set(captures(cuda, "singles")())
+    capture = captures(cuda, "portions", drawn_between)
+    for _ in range(POOL + 1):
+        assert not singles & capture()
+
+
+def test_every_kind_of_batch_has_streams_of_its_own(cuda):
+    of_device = streams.batch_streams(DEVICE)
+    assert streams.batch_streams(DEVICE) is of_device
+    own = [stream for kind in streams.KINDS for stream in (of_device.recording[kind], of_device.side[kind])]
+    assert len(set(own + of_device.beside)) == len(own) + len(of_device.beside)
+    assert of_device.recording[streams.SINGLES] == torch.cuda.graph.default_capture_stream
+    for _ in range(2 * POOL):
+        assert of_device.apart() not in own + of_device.beside
+    for kind in streams.KINDS:
+        assert block.side_stream(DEVICE, of_device.recording[kind]) == of_device.side[kind]
+    for number in range(POOL):                           # work on any other stream forks to none of a kind's
+        main = FakeStream(number=number)
+        side = block.side_stream(DEVICE, main)
+        assert side != main and (main in [of_device.recording[kind] for kind in streams.KINDS] or side not in own)
+
+
+def engine_on(monkeypatch):
+    monkeypatch.setattr(engine_module.ops, "stream_beside", lambda main, candidates: candidates[-1])
+    engine = SimpleNamespace(graphs=SimpleNamespace(streams=streams.batch_streams(DEVICE)), device=DEVICE, _beside={})
+    engine._streams_beside = lambda: engine_module.Engine._streams_beside(engine)
+    return engine
+
+
+def test_single_tokens_run_beside_portions_only_where_their_streams_are_apart(cuda, monkeypatch):
+    """Whatever stream of the pool the caller is on: beside it only if it is none of the single tokens' own (a portion
+    that is launched kernel by kernel works on the caller's), on a stream that is neither the caller's nor a kind's."""
+    engine = engine_on(monkeypatch)
+    of_device = engine.graphs.streams
+    for number in [-1] + list(range(POOL)):
+        cuda.current = FakeStream(number=number)
+        assert engine_module.Engine._apart(engine) != of_device.belongs_to(streams.SINGLES, cuda.current)
+        assert all(stream != cuda.current and stream in of_device.beside for stream in engine._streams_beside())
+    assert len(engine._beside) <= engine_module.CALLERS_STREAMS
+
+
+def test_the_streams_of_a_callers_stream_begin_with_the_one_the_clock_found(cuda, monkeypatch):
+    engine = engine_on(monkeypatch)
+    found = engine._streams_beside()
+    assert found[0] == engine.graphs.streams.beside[-1] and set(found) == set(engine.graphs.streams.beside)
+    monkeypatch.setattr(engine_module.ops, "stream_beside", None)               # not asked again
+    assert engine._streams_beside() is found
