@@ -212,6 +212,8 @@ class Engine:
         if halves:
             self._make_graphs_beside()
             done += self.graphs_beside.warm_up([(second, second) for _, second in halves], context)
+        if self.split_from_lanes < SPLIT_NEVER:
+            self.graphs.ask_beside(done, self._streams_beside())
         return done
 
     def step_token_target(self, lanes: int, tokens: int) -> int:
@@ -295,19 +297,25 @@ class Engine:
         """Run one batch; returns float32 logits [wanted, vocab] in the order of the lanes and
         of each lane's ``want``.  Raises StepError or CacheExhausted with nothing changed, or
         StepFailed with the lanes' requests ended and everything they held given back.  The work is
-        queued on the GPU; nothing here waits for it (a lane with ``feed`` takes its token from the device,
-        so a caller may queue the next step before it has read this one's tokens)."""
+        queued on the GPU and not waited for (a lane with ``feed`` takes its token from the device,
+        so a caller may queue the next step before it has read this one's tokens), but in a step that is the first to
+        need a graph, or an answer of the clock, which ``warm_up`` gets ahead for the steps it is told of."""
         lowered = self.validate(lanes)
         single = lowered.lengths == 1
         singles = int(single.sum())
-        # (the clock is asked, once, only by a step that may need its answer, and before anything is reserved)
+        # (the clock is asked only by a step that may need its answer, and before anything is reserved)
         in_two = SPLIT_FROM_LANES <= singles < len(lanes) and self.split_from_lanes <= singles
         in_halves = (singles == len(lanes) and HALVES_FROM_LANES <= singles <= HALVES_MOST_LANES
                      and self.graphs is not None and self.in_halves)
+        if in_two:
+            batches = self._two_batches(lanes, single)
+            beside = self._stream_for_singles(*batches[0])
+        elif in_halves:
+            self._streams_beside()
         self.cache.reserve_slots(lowered.slots, lowered.lengths)
         try:
             if in_two:
-                logits = self._run_in_two(lanes, lowered, single)
+                logits = self._run_in_two(batches, beside, lowered, single)
             elif in_halves:
                 logits = self._run_in_halves(lanes)
             else:
@@ -350,10 +358,16 @@ class Engine:
             self._beside[main.cuda_stream] = [first] + [stream for stream in others if stream != first]
         return self._beside[main.cuda_stream]
 
-    def _apart(self) -> bool:
-        """Whether single tokens may run beside portions: the caller's stream must be none that the single tokens' graphs
-        use (a portion that is launched kernel by kernel leaves a library's workspace there)."""
-        return self.graphs is not None and not self.graphs.streams.belongs_to(SINGLES, torch.cuda.current_stream(self.device))
+    def _stream_for_singles(self, portions: Sequence[Lane], lowered: LoweredLanes) -> Optional[torch.cuda.Stream]:
+        """The stream for the single tokens of a step beside these portions, or None: one batch behind the other.  The
+        caller's stream must be none that the single tokens' graphs use: a portion that is launched kernel by kernel
+        leaves a library's workspace there."""
+        if self.graphs is None or self.graphs.streams.belongs_to(SINGLES, torch.cuda.current_stream(self.device)):
+            return None
+        candidates = self._streams_beside()
+        key = self.graphs.bucket_key(portions, lowered)
+        self.graphs.ask_beside([key], candidates)
+        return self.graphs.stream_beside(key, candidates)
 
     def _make_graphs_beside(self) -> None:
         if self.graphs_beside is None:
@@ -382,26 +396,29 @@ class Engine:
         rows_second.record_stream(main)
         return torch.cat([rows_first, rows_second])
 
-    def _run_in_two(self, lanes: Sequence[Lane], lowered: LoweredLanes, single: np.ndarray) -> torch.Tensor:
+    def _two_batches(self, lanes: Sequence[Lane], single: np.ndarray) -> list:
+        """The portions and the single tokens of a step, each as (lanes, lowered)."""
+        batches = []
+        for chosen in (~single, single):
+            members = [lane for lane, mine in zip(lanes, chosen) if mine]
+            batches.append((members, self.validate(members)))
+        return batches
+
+    def _run_in_two(self, batches: list, beside: Optional[torch.cuda.Stream], lowered: LoweredLanes, single: np.ndarray) -> torch.Tensor:
         """A step that holds portions of prompts beside several single decoded tokens, as two batches side by side:
-        the portions through the prompt kernels, and on a second stream the single tokens through the graph of a decode
+        the portions through the prompt kernels, and on the stream ``beside`` the single tokens through the graph of a decode
         step, whose small kernels wait for each other most of their time (515 prompt tokens of the 0.5B shape beside 24 decoded
         ones: 4.8 ms, 6.1 with one batch behind the other; beside 130, whose graph of 256 rows forks too, 7.2 and 9.4).  (As one batch the prompt kernels take every single token as
         a prompt of its own, a tile of the attention kernel and a chunk of the scan each: 2,048 prompt tokens beside 63
         decoded ones took 19.4 ms, where the two batches take 6.3 and 3.1.)  The batches belong to different requests,
         and what they are recorded, warmed up and forked on are streams of their own, by which they share neither a memory pool
-        nor a library's workspace (``BatchStreams``).  Where they are not, the batches follow each other.  The logits come
+        nor a library's workspace (``BatchStreams``).  Without ``beside`` the batches follow each other.  The logits come
         back in the order of the lanes."""
-        batches = []
-        for chosen in (~single, single):
-            members = [lane for lane, mine in zip(lanes, chosen) if mine]
-            batches.append((members, self.validate(members)))
         portions, singles = batches
-        if not self._apart():
+        if beside is None:
             parts = [self._run(*portions), self._run(*singles)]
         else:
             main = torch.cuda.current_stream(self.device)
-            beside = self.graphs.stream_beside(portions[0], portions[1], singles[1], self._streams_beside())
             try:
                 with replayed_beside(main, beside):
                     rows_of_singles = self._run(*singles)

@@ -28,6 +28,8 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
 
+from ..kernels import ops
+from ..parts.block import OVERLAP_MIN_TOKENS
 from ..parts.streams import PORTIONS, SECOND_HALF, SINGLES, batch_streams
 from .context import _NO_LANES, Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
 
@@ -88,7 +90,7 @@ class DecodeGraphs:
         # graphs of two kinds are replayed beside each other (``Engine._run_in_two``, ``Engine._run_in_halves``): each kind
         # has a memory pool of its own, and streams of its own that it is recorded and forked on (see ``BatchStreams``)
         self._pools: Dict[str, object] = {}
-        self._besides: Dict[tuple, Dict[int, torch.cuda.Stream]] = {}
+        self._besides: Dict[tuple, torch.cuda.Stream] = {}
         self.counts = {"decode_replays": 0, "bucket_replays": 0, "bucket_captures": 0, "bucket_eager": 0}
 
     # captured capacities kept; the least recently used one goes.  A capture costs about as much as thirty replays
@@ -145,7 +147,7 @@ class DecodeGraphs:
                     best = max(best, fill)
         return best if best >= tokens - tokens // 8 else tokens
 
-    def _bucket_key(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[tuple]:
+    def bucket_key(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[tuple]:
         """The capacity and context of the graph that such a step replays, or None where no graph can hold it."""
         capacity = self.capacity_for(len(lanes), int(lowered.lengths.sum()), int(lowered.want_counts.sum()))
         if capacity is None:
@@ -158,7 +160,7 @@ class DecodeGraphs:
     def run_bucket(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> Optional[torch.Tensor]:
         """Logits of a step with prompt portions from the captured graph of its capacity, or None when that
         capacity has no graph (yet): the caller then launches the step kernel by kernel."""
-        key = self._bucket_key(lanes, lowered)
+        key = self.bucket_key(lanes, lowered)
         if key is None:
             self.counts["bucket_eager"] += 1
             return None
@@ -265,25 +267,48 @@ class DecodeGraphs:
             main.wait_stream(beside)
         return self._clock(side_by_side, replays)
 
-    def stream_beside(self, lanes: Sequence[Lane], portions: LoweredLanes, singles: LoweredLanes,
-                      candidates: Sequence[torch.cuda.Stream]) -> torch.cuda.Stream:
-        """The stream of ``candidates`` on which the graph of ``singles`` runs best beside that of ``portions``: asked of
-        the clock once for every graph of portions (and stream of the caller), with nothing but padding in either; the
-        first where one of the two has no graph yet."""
-        key = self._bucket_key(lanes, portions)
-        decode_key = (bucket_for(len(singles.slots)), self.context_bucket(singles))
-        if key not in self._bucket_graphs or decode_key not in self._graphs:
-            return candidates[0]
-        main = torch.cuda.current_stream(self.device).cuda_stream
-        chosen = self._besides.setdefault(key, {})
-        if main not in chosen:
-            graphs = []
-            for static, graph, _ in (self._bucket_graphs[key], self._graphs[decode_key]):
-                static.fill(_NO_LANES)
-                graphs.append(graph)
-            times = [self._clock_beside(*graphs, stream, 3) for stream in candidates]
-            chosen[main] = candidates[times.index(min(times))]
-        return chosen[main]
+    def forks(self, key: tuple) -> bool:
+        """Whether the graph of the portions' capacity ``key`` runs its mixers on two streams."""
+        return key[1] >= OVERLAP_MIN_TOKENS and any(len(getattr(block, "mixers", ())) == 2 for block in self.model.blocks)
+
+    def ask_beside(self, keys: Iterable[tuple], candidates: Sequence[torch.cuda.Stream]) -> None:
+        """The clock's answer to which of ``candidates`` does not stand in the way of the graphs of these capacities, for
+        those that fork and have no answer yet (nothing but padding is touched).  Such a graph takes two hardware queues, of
+        which the second is the runtime's choice when the graph is made, another one from graph to graph: a stream that
+        lies on it makes the graph wait (640 tokens of the 0.5B shape beside 24 decoded ones: 4.5 ms on two of four streams,
+        5.6 on the others, which are others for the graph of 1,024 tokens).  Asked by a kernel that does nothing but wait, for
+        a quarter of the graph's time: five to seven replays, about what the capture cost."""
+        for key in keys:
+            if key not in self._bucket_graphs or key in self._besides or not self.forks(key):
+                continue
+            static, graph, _ = self._bucket_graphs[key]
+            static.fill(_NO_LANES)
+            at_once = self._clock_behind_wait(graph, candidates[0], 1, 3)
+            wait = min(max(at_once / 4, 0.02), 5.0)
+            for stream in candidates:
+                self._besides[key] = stream
+                if self._clock_behind_wait(graph, stream, int(1000 * wait), 2) - at_once < wait / 2:
+                    break
+
+    def _clock_behind_wait(self, graph, beside: torch.cuda.Stream, microseconds: int, replays: int) -> float:
+        """The least time of ``graph`` beside a kernel on ``beside`` that waits, in milliseconds."""
+        main = torch.cuda.current_stream(self.device)
+        marks = [[torch.cuda.Event(enable_timing=True) for _ in range(2)] for _ in range(replays)]
+        for begin, end in marks:
+            begin.record()
+            with replayed_beside(main, beside):
+                ops.wait(microseconds)
+            graph.replay()
+            main.wait_stream(beside)
+            end.record()
+        torch.cuda.synchronize(self.device)
+        return min(begin.elapsed_time(end) for begin, end in marks)
+
+    def stream_beside(self, key: Optional[tuple], candidates: Sequence[torch.cuda.Stream]) -> torch.cuda.Stream:
+        """The stream of ``candidates`` to run single tokens on beside portions of the capacity ``key``: the clock's answer
+        where there is one (``ask_beside``), else the first."""
+        chosen = self._besides.get(key)
+        return chosen if chosen is not None and any(chosen == stream for stream in candidates) else candidates[0]
 
     def measure_halves(self, beside: torch.cuda.Stream, lanes: int = 128, replays: int = 5) -> Optional[float]:
         """The clock's answer to whether a step of ``lanes`` single tokens is faster as two halves at once, each a

@@ -340,11 +340,15 @@ def feed_tokens(token_ids: torch.Tensor, source: torch.Tensor, dst: Sequence[int
            "feed_tokens")
 
 
+def wait(microseconds: int) -> None:
+    """A kernel of one wave on the current stream that does nothing for so long (at most 10,000)."""
+    _check(_fn("common", "mi_wait")(int(microseconds), _stream()), "wait")
+
+
 def stream_beside(main: "torch.cuda.Stream", candidates: Sequence["torch.cuda.Stream"], microseconds: int = 200) -> "torch.cuda.Stream":
     """Of ``candidates`` (none of them ``main``) a stream whose kernels run beside those of ``main``.  The runtime lays its
     streams on a few hardware queues, and what lies on one queue runs one after the other: the first on which a wait
     of so many microseconds is over together with one on ``main`` (or, if none is, the last)."""
-    wait = _fn("common", "mi_wait")
     with torch.cuda.device(main.device):
         for beside in candidates:
             took = []
@@ -354,7 +358,8 @@ def stream_beside(main: "torch.cuda.Stream", candidates: Sequence["torch.cuda.St
                 begin.record(main)
                 beside.wait_event(begin)
                 for stream in (main, beside):
-                    _check(wait(microseconds, stream.cuda_stream), "wait")
+                    with torch.cuda.stream(stream):
+                        wait(microseconds)
                 main.wait_stream(beside)
                 end.record(main)
                 torch.cuda.synchronize(main.device)

@@ -97,6 +97,21 @@ def test_portions_beside_several_decoded_tokens_run_as_two_batches_in_the_caller
     engine.cache.check()
 
 
+def test_the_clock_is_asked_for_a_second_stream_before_anything_is_reserved(host_ops, tmp_path, monkeypatch):
+    """The question replays graphs and waits for them: by then nothing of the step may have changed."""
+    engine, cfg, _ = engine_for("A", tmp_path, capacity=400, page=8, requests=7)
+    streams = {key: tokens_for(cfg, 20, 60 + index) for index, key in enumerate("abcde")}
+    for key in streams:
+        engine.add_request(key)
+    engine.step([Lane(key, streams[key][:10], []) for key in "abcd"])
+    order = []
+    reserve = engine.cache.reserve_slots
+    monkeypatch.setattr(engine.cache, "reserve_slots", lambda *arguments: (order.append("reserve"), reserve(*arguments))[1])
+    monkeypatch.setattr(engine, "_stream_for_singles", lambda portions, lowered: order.append([lane.request for lane in portions]))
+    engine.step([Lane(key, streams[key][10:11], [0]) for key in "abcd"] + [Lane("e", streams["e"][:9], [8])])
+    assert order == [["e"], "reserve"]
+
+
 def test_refused_steps_change_nothing(host_ops, tmp_path):
     engine, cfg, tensors = engine_for("A", tmp_path, capacity=32, page=8, requests=2)
     engine.add_request("a")

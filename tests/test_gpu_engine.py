@@ -1317,9 +1317,9 @@ def test_single_tokens_beside_portions_give_the_bits_of_one_batch_behind_the_oth
     two, one = make(), make()
     assert two.split_from_lanes == one.split_from_lanes == 4
     beside = []
-    real = two._apart
-    monkeypatch.setattr(two, "_apart", lambda: (beside.append(real()), beside[-1])[1])
-    monkeypatch.setattr(one, "_apart", lambda: False)
+    real = two._stream_for_singles
+    monkeypatch.setattr(two, "_stream_for_singles", lambda *batches: (beside.append(real(*batches)), beside[-1])[1])
+    monkeypatch.setattr(one, "_stream_for_singles", lambda *batches: None)
     streams = [torch.cuda.current_stream()] * 4 + [torch.cuda.Stream() for _ in range(2)] + [two.graphs.streams.recording["single tokens"]]
     for engine in (two, one):
         for index in range(count):
@@ -1337,8 +1337,48 @@ def test_single_tokens_beside_portions_give_the_bits_of_one_batch_behind_the_oth
                 rows.append(engine.step(lanes).cpu())
             engine.finish(f"prompt {turn}")
         assert rows[0].shape[0] == count + 2 and torch.equal(rows[0], rows[1]), turn
-    assert beside == [True] * 6 + [False]
+    assert [stream is None for stream in beside] == [False] * 6 + [True]
     assert two.graphs.counts["bucket_replays"] >= 5 and two.graphs._besides
+
+
+def test_warm_up_asks_the_clock_ahead_which_stream_runs_beside_a_long_portion(tmp_path, monkeypatch):
+    """For the graphs that fork, and for nothing that a step needs afterwards; the requests that are live then, and the step
+    behind it, are as if it had not been asked."""
+    import gates
+    from macllm_infer_amd import Engine, Lane
+    folder = tiny_configs.make_model_dir("D", tmp_path, torch.bfloat16)
+    cfg, tensors = plain_impl.load_model_dir(folder)
+    engine = Engine(folder, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=4096, max_active_sequences=8)
+    engine.split_from_lanes = 4
+    tokens = {index: tokens_for(cfg["vocab_size"], 400, 50 + index) for index in range(6)}
+    for index in range(6):
+        engine.add_request(index)
+    engine.step([Lane(index, tokens[index][:9]) for index in range(5)])
+    engine.warm_up([(5, 5), (1, 40), (1, 300), (1, 384)])
+    graphs = engine.graphs
+    assert sorted(key[1] for key in graphs._bucket_graphs if key in graphs._besides) == [320, 384]
+    before = dict(graphs._besides)
+    asked = []
+    real = graphs._clock_behind_wait
+    monkeypatch.setattr(graphs, "_clock_behind_wait", lambda *arguments: (asked.append(1), real(*arguments))[1])
+
+    def check(got, wanted):
+        for row, (index, place) in enumerate(wanted):
+            want = plain_impl.falcon_h1_logits(cfg, tensors, tokens[index][:place + 1])[-1]
+            assert gates.bfloat16_close(got[row:row + 1].float().cpu().numpy(), want[None].numpy()), (index, place)
+    check(engine.step([Lane(index, tokens[index][9:10], [0]) for index in range(5)] + [Lane(5, tokens[5][:300], [299])]),
+          [(index, 9) for index in range(5)] + [(5, 299)])
+    assert graphs._besides == before and not asked and graphs.counts["bucket_replays"] == 1
+    graphs._besides.clear()                                  # asked in between, of a graph that holds a step's lanes
+    check(engine.step([Lane(index, tokens[index][10:11], [0]) for index in range(5)] + [Lane(5, tokens[5][300:399], [98])]),
+          [(index, 10) for index in range(5)] + [(5, 398)])
+    engine.add_request(6)
+    tokens[6] = tokens_for(cfg["vocab_size"], 300, 60)
+    check(engine.step([Lane(index, tokens[index][11:12], [0]) for index in range(5)] + [Lane(6, tokens[6], [299])]),
+          [(index, 11) for index in range(5)] + [(6, 299)])
+    assert asked and len(graphs._besides) == 1
+    check(engine.step([Lane(index, tokens[index][12:13], [0]) for index in range(6 - 1)] + [Lane(5, tokens[5][399:400], [0])]),
+          [(index, 12) for index in range(5)] + [(5, 399)])
 
 
 def test_the_second_stream_is_never_the_stream_it_runs_beside(monkeypatch):

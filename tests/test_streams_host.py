@@ -112,9 +112,11 @@ def test_every_kind_of_batch_has_streams_of_its_own(cuda):
         assert side != main and (main in [of_device.recording[kind] for kind in streams.KINDS] or side not in own)
 
 
-def engine_on(monkeypatch):
+def engine_on(monkeypatch, asked):
+    bank = SimpleNamespace(streams=streams.batch_streams(DEVICE), bucket_key=lambda lanes, lowered: "key",
+                           ask_beside=lambda keys, candidates: asked.append(keys), stream_beside=lambda key, candidates: candidates[0])
     monkeypatch.setattr(engine_module.ops, "stream_beside", lambda main, candidates: candidates[-1])
-    engine = SimpleNamespace(graphs=SimpleNamespace(streams=streams.batch_streams(DEVICE)), device=DEVICE, _beside={})
+    engine = SimpleNamespace(graphs=bank, device=DEVICE, _beside={})
     engine._streams_beside = lambda: engine_module.Engine._streams_beside(engine)
     return engine
 
@@ -122,17 +124,22 @@ def engine_on(monkeypatch):
 def test_single_tokens_run_beside_portions_only_where_their_streams_are_apart(cuda, monkeypatch):
     """Whatever stream of the pool the caller is on: beside it only if it is none of the single tokens' own (a portion
     that is launched kernel by kernel works on the caller's), on a stream that is neither the caller's nor a kind's."""
-    engine = engine_on(monkeypatch)
+    asked = []
+    engine = engine_on(monkeypatch, asked)
     of_device = engine.graphs.streams
     for number in [-1] + list(range(POOL)):
         cuda.current = FakeStream(number=number)
-        assert engine_module.Engine._apart(engine) != of_device.belongs_to(streams.SINGLES, cuda.current)
-        assert all(stream != cuda.current and stream in of_device.beside for stream in engine._streams_beside())
+        asked.clear()
+        stream = engine_module.Engine._stream_for_singles(engine, [object()], None)
+        if of_device.belongs_to(streams.SINGLES, cuda.current):
+            assert stream is None and not asked
+        else:
+            assert stream != cuda.current and stream in of_device.beside and asked == [["key"]]
     assert len(engine._beside) <= engine_module.CALLERS_STREAMS
 
 
 def test_the_streams_of_a_callers_stream_begin_with_the_one_the_clock_found(cuda, monkeypatch):
-    engine = engine_on(monkeypatch)
+    engine = engine_on(monkeypatch, [])
     found = engine._streams_beside()
     assert found[0] == engine.graphs.streams.beside[-1] and set(found) == set(engine.graphs.streams.beside)
     monkeypatch.setattr(engine_module.ops, "stream_beside", None)               # not asked again
