@@ -883,7 +883,7 @@ polynorm_kernel(const T* __restrict__ z, long ld, const float* __restrict__ coef
 
 // The same with the row in registers, PIECES pieces of 16 bytes a thread (piece threadIdx.x + k * blockDim.x), the three
 // sums through one barrier, one read of the row: rows of whole pieces from aligned addresses.  (1,999 rows of 2,048 in
-// bfloat16: 8.9 us through the kernel above, 5.9 here, of which the 16 MB alone take 3.3.)
+// bfloat16: 8.9 us through the kernel above, 5.6 here, of which the 16 MB alone take 3.3.)
 template <typename T, int PIECES>
 __global__ void __launch_bounds__(1024)
 polynorm_rows_kernel(const T* __restrict__ z, long ld, const float* __restrict__ coefficients, float eps,
@@ -952,8 +952,10 @@ static bool launch_polynorm_rows(const T* z, long ld, const float* coefficients,
   if (I % VEC != 0 || ld % VEC != 0 || out_ld % VEC != 0 || ((uintptr_t)z | (uintptr_t)out) % 16 != 0) return false;
   const int pieces = I / VEC;
   if (pieces > 4096) return false;
-  const int most = rows <= 512 ? 1024 : 256;                 // few rows: the shortest chain a row
-  const int each = pieces <= most ? 1 : pieces <= 2 * most ? 2 : 4;
+  // by the width alone, never by the number of rows: a position's sums are the same bits however its prompt is cut.  Few waves
+  // cross the barrier faster than many, whatever the rows (12 rows of 4,096 in float32: 3.7 us with one piece a thread, 3.1
+  // with four; 1,999 rows 17.2 and 10.6)
+  const int each = pieces <= 256 ? 1 : pieces <= 512 ? 2 : 4;
   const int threads = ((pieces + each - 1) / each + WAVE - 1) / WAVE * WAVE;
   if (each == 1) polynorm_rows_kernel<T, 1><<<rows, threads, 0, stream>>>(z, ld, coefficients, eps, out, out_ld, I);
   else if (each == 2) polynorm_rows_kernel<T, 2><<<rows, threads, 0, stream>>>(z, ld, coefficients, eps, out, out_ld, I);

@@ -1812,6 +1812,19 @@ def test_polynorm_with_the_row_in_registers(ops, dtype, T, width, ld):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [1024, 1028, 1536, 2048, 2056, 4096, 8192])
+def test_polynorm_of_a_row_is_the_same_bits_whatever_rows_stand_beside_it(ops, dtype, width):
+    z, c = rand(513, width, seed=1, dtype=dtype).to(DEV), torch.tensor([0.7, -0.4, 0.25, 0.1], device=DEV)
+    outs = []
+    for rows in (1, 3, 512, 513):
+        out = torch.empty(rows, width, dtype=dtype, device=DEV)
+        ops.polynorm(z[:rows], c, 1e-5, out)
+        outs.append(out)
+    for fewer in outs[:-1]:
+        assert torch.equal(fewer, outs[-1][:fewer.shape[0]])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("activation", ["silu", "sigmoid"])
 @pytest.mark.parametrize("T, H, dv, gap", [(1, 1, 32, 0), (7, 3, 64, 8), (129, 5, 128, 4), (33, 3, 256, 0), (5, 3, 64, 2), (5, 3, 60, 0)])
 def test_head_norms_in_pieces_of_four(ops, dtype, activation, T, H, dv, gap):
