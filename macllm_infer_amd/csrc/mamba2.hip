@@ -327,24 +327,26 @@ extern "C" int mi_conv_step(void* u, int dtype, long ld, int col_offset, int M, 
 // elements (1, 2, 4 or 8: the smallest number that covers N; one load where alignment allows); 256/R rows per block.
 //
 // The recurrence is serial in the tokens, so what a token costs is what its step waits for.  The tokens of a
-// lane come in blocks of up to 64: a block's B, C, x, delta and decay are asked for two blocks ahead by all threads
+// lane come in blocks of up to 32: a block's B, C, x, delta and decay are asked for two blocks ahead by all threads
 // of the workgroup, a few elements each and each element once a workgroup, laid in LDS one block ahead, and read
-// from there into the registers of the threads that use them, a few tokens at a time before the first of them; softplus and the exponential are taken once a token and head, by a small kernel ahead of the scan.  What
-// the R lanes of a row add up for a token's output is added in registers (scan_lanes_sum: a butterfly over the
-// lanes in which both partners of every step add the same two numbers), the outputs of a block wait in a register
+// from there into the registers of the threads that use them, a few tokens at a time before the first of them; softplus
+// and the exponential are taken once a token and head, by a small kernel ahead of the scan.  What the R lanes of a row add up
+// for a token's output is added in registers (scan_lanes_sum: a butterfly over the lanes in which both partners of every step add the same two numbers), the outputs of a block wait in a register
 // of the lane with the token's number and leave with one store a block.  Every token goes through the same
 // operations in the same order whatever block it falls into, and in the kernel for steps of single tokens (SINGLE:
 // nothing staged, few registers, many workgroups a compute unit): a step of one token and a prompt of thousands
 // give a position the same bits.
 #define SCAN_MAX_PER_THREAD 8
 #define SCAN_BLOCK_ELEMENTS 16      // tokens of a run that goes without a condition, times PER, where they are summed one by one
-// Tokens of a block that a workgroup stages, at most (a row narrower than a wave keeps a block's outputs in 16 lanes), and
+// Tokens of a block that a workgroup stages, at most (a row narrower than a wave keeps a block's outputs in 16 lanes; one as
+// wide as a wave holds 33 states or more, 64 tokens of which are more loads than its threads send for), and
 // loads of four elements of B|C that a thread sends for, a block.  512 tokens, 24 heads of 64 with 128 states: 60 us (72
 // with the tokens' sums one by one and B and C apart in LDS), with 256 states and heads of 128: 113 (228).  Eight loads a
 // thread (blocks of 32 tokens) gain 5 us there and lose 3 on every lane of a few tokens; asking LDS for a run's operands
 // while the run before is worked on costs registers and gains nothing.
-#define SCAN_BLOCK_TOKENS(eight) ((eight) ? 64 : 16)
+#define SCAN_BLOCK_TOKENS(eight) ((eight) ? 32 : 16)
 #define SCAN_THREAD_PIECES 4
+static_assert(64 * ((2 * (WAVE / 2 + 1) + 3) / 4) > 256 * SCAN_THREAD_PIECES, "blocks of 64 tokens could be staged");
 
 template <int CONTROL, int ROW_MASK>
 __device__ __forceinline__ float scan_dpp(float v) {
