@@ -217,7 +217,6 @@ struct PromptBeside {
   void* v_base;
   long page_stride;
   int page_size;
-  int attend;                      // 1: the attention too, beside the second launch
   const int* block_tables;
   int max_pages;
   const int* tiles;
@@ -1187,7 +1186,7 @@ extern "C" int mi_ssd_supported(int Q, int P, int N, int G, int E) {
 }
 
 // beside: null, or the attention that reads the same step's rows (bfloat16, values as wide as the keys, a cache to write to
-// or none); its rotation needs the conv here, its attention a step that mi_ssd_single and mi_ssd_beside cover.
+// or none): needs the conv here and a step that mi_ssd_single and mi_ssd_beside cover.
 extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long dt_ld, const float* dt_bias,
                               const float* A, const float* D, float* ssm_state, const int* chunks, int n_chunks,
                               const int* lane_chunks, const int* slot_ids, int n_lanes, int Q, int H, int P, int N,
@@ -1214,18 +1213,16 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
     const PromptBeside& b = *beside;
     if (!conv_here || !b.qkv || b.T <= 0 || b.Hq <= 0 || b.Hkv <= 0 || b.Hq % b.Hkv != 0 || b.dh <= 0 || (b.dh & 1) || !b.positions ||
         b.ld < (long)(b.Hq + 2 * b.Hkv) * b.dh || b.rotary_dim < 0 || b.rotary_dim > b.dh || (b.rotary_dim & 1) ||
-        (b.rotary_dim > 0 && !b.inv_freq) || (b.slot_mapping && (!b.k_base || !b.v_base || b.page_size <= 0)))
+        (b.rotary_dim > 0 && !b.inv_freq))
       return ERR_BAD_ARGUMENT;
-    if (b.attend) {
-      if (!b.block_tables || b.max_pages <= 0 || !b.tiles || b.n_tiles <= 0 || !b.cu_seqlens || !b.start_pos || !b.out || !b.k_base ||
-          !b.v_base || b.page_size <= 0)
-        return ERR_BAD_ARGUMENT;
-      if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
-          b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0 ||
-          b.n_tiles > (1 << 20) || b.Hkv > 256)
-        return ERR_UNSUPPORTED_SIZE;
-      nset = prefill_head_set(b.dh, b.Hq / b.Hkv, b.n_tiles, b.Hkv, b.max_seq_len);
-    }
+    if (!b.block_tables || b.max_pages <= 0 || !b.tiles || b.n_tiles <= 0 || !b.cu_seqlens || !b.start_pos || !b.out || !b.k_base ||
+        !b.v_base || b.page_size <= 0)
+      return ERR_BAD_ARGUMENT;
+    if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
+        b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0 ||
+        b.n_tiles > (1 << 20) || b.Hkv > 256)
+      return ERR_UNSUPPORTED_SIZE;
+    nset = prefill_head_set(b.dh, b.Hq / b.Hkv, b.n_tiles, b.Hkv, b.max_seq_len);
   }
   if (conv_here) {
     const int own_rows = H + (C + 63) / 64;
@@ -1262,8 +1259,7 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
   if (N == 32 * NK_ && P == 16 * PT_)                                                                             \
     status = launch_ssd_single<NK_, PT_>(dim3(n_chunks, H + tail_rows), stream, (const bf16_t*)xbc, xbc_ld,       \
                                          (const bf16_t*)TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld,           \
-                                         (const bf16_t*)z, z_ld, (bf16_t*)gated, gated_ld, one,                       \
-                                         beside && beside->attend ? beside : nullptr, nset);
+                                         (const bf16_t*)z, z_ld, (bf16_t*)gated, gated_ld, one, beside, nset);
     SINGLE_CASE(1, 1) SINGLE_CASE(1, 2) SINGLE_CASE(1, 4) SINGLE_CASE(1, 8)
     SINGLE_CASE(2, 1) SINGLE_CASE(2, 2) SINGLE_CASE(2, 4) SINGLE_CASE(2, 8)
     SINGLE_CASE(4, 1) SINGLE_CASE(4, 2) SINGLE_CASE(4, 4) SINGLE_CASE(4, 8)

@@ -2003,7 +2003,7 @@ def ssd_supported(chunk_size: int, head_dim: int, state_size: int, num_groups: i
 class _PromptBeside(ctypes.Structure):
     _fields_ = [("qkv", _c_ptr), ("ld", _c_long), ("T", _c_int), ("Hq", _c_int), ("Hkv", _c_int), ("dh", _c_int),
                 ("positions", _c_ptr), ("inv_freq", _c_ptr), ("rotary_dim", _c_int), ("slot_mapping", _c_ptr),
-                ("k_base", _c_ptr), ("v_base", _c_ptr), ("page_stride", _c_long), ("page_size", _c_int), ("attend", _c_int),
+                ("k_base", _c_ptr), ("v_base", _c_ptr), ("page_stride", _c_long), ("page_size", _c_int),
                 ("block_tables", _c_ptr), ("max_pages", _c_int), ("tiles", _c_ptr), ("n_tiles", _c_int),
                 ("cu_seqlens", _c_ptr), ("start_pos", _c_ptr), ("scale", _c_float), ("window", _c_int),
                 ("max_seq_len", _c_int), ("out", _c_ptr), ("out_ld", _c_long)]
@@ -2011,7 +2011,7 @@ class _PromptBeside(ctypes.Structure):
 
 @dataclass
 class PromptBeside:
-    """The attention of a layer whose state-space mixer reads the same step: what ``rope_kv_store`` and (``attend``)
+    """The attention of a layer whose state-space mixer reads the same step: what ``rope_kv_store`` and
     ``prefill_attention`` take, to be run by ``ssd_prefill`` in its own launches."""
     qkv: torch.Tensor
     num_heads: int
@@ -2032,7 +2032,6 @@ class PromptBeside:
     out: torch.Tensor
     max_seq_len: int
     sizes: Optional[tuple]
-    attend: bool = True
 
     def fits(self, longest: int, ssm_state: torch.Tensor, chunk_size: int) -> bool:
         """Whether ``ssd_prefill`` of a step with lanes of up to ``longest`` tokens takes this attention in its two
@@ -2075,7 +2074,7 @@ class PromptBeside:
                                         and self.inv_freq.is_cuda), "prompt beside: inv_freq must be float32 [rotary_dim / 2]")
         return _PromptBeside(_p(self.qkv), q_ld, T, self.num_heads, self.num_kv_heads, self.head_dim, _p(self.positions),
                              _p(self.inv_freq), rotary, _p(self.slot_mapping), _p(self.k_cache), _p(self.v_cache), page_stride,
-                             page_size, 1 if self.attend else 0, _p(self.block_tables), self.block_tables.shape[1],
+                             page_size, _p(self.block_tables), self.block_tables.shape[1],
                              _p(self.query_tiles), self.query_tiles.shape[0], _p(self.cu_seqlens), _p(self.start_pos),
                              float(self.scale), _span(self.window, None, "prefill_attention"), int(self.max_seq_len or 0),
                              _p(self.out), out_ld)
