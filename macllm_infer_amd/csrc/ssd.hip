@@ -1141,8 +1141,10 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
   if constexpr ((NK == 4 && PT == 4) || (NK == 8 && PT == 8)) {
     if (beside) {
       const int passes = (beside->Hq / beside->Hkv + nset - 1) / nset;
+      const long all = (long)grid.x * grid.y + 4L * beside->n_tiles * beside->Hkv * passes;
+      if (all > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
       const int scan_groups = (int)(grid.x * grid.y);
-      const unsigned groups = (unsigned)(scan_groups + 4 * beside->n_tiles * beside->Hkv * passes);
+      const unsigned groups = (unsigned)all;
 #define BESIDE_CASE(DH_, NSET_)                                                                                             \
   if (beside->dh == DH_ && nset == NSET_) {                                                                                 \
     static bool told[64] = {};                                                                                              \
@@ -1166,11 +1168,18 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
 }
 #undef SINGLE_ARGUMENTS
 
-// Whether mi_ssd_prefill takes the attention of such heads beside its second launch (of a step that mi_ssd_single covers).
-extern "C" int mi_ssd_beside(int P, int N, int Hq, int Hkv, int dh, int n_tiles, int max_seq_len) {
-  if (Hkv <= 0 || Hq % Hkv != 0 || n_tiles <= 0 || !((P == 64 && N == 128) || (P == 128 && N == 256))) return 0;
+// Whether mi_ssd_prefill takes the attention of such heads beside its second launch (of a step that mi_ssd_single covers,
+// whose H heads of the scan may have a group each): what it would refuse is refused here, before anything is launched.
+extern "C" int mi_ssd_beside(int H, int P, int N, int Hq, int Hkv, int dh, int n_tiles, int max_seq_len) {
+  if (H <= 0 || Hkv <= 0 || Hkv > 256 || Hq % Hkv != 0 || n_tiles <= 0 || n_tiles > (1 << 20) ||
+      !((P == 64 && N == 128) || (P == 128 && N == 256)))
+    return 0;
   const int nset = prefill_head_set(dh, Hq / Hkv, n_tiles, Hkv, max_seq_len);
-  return (dh == 64 && (nset == 2 || nset == 4)) || (dh == 128 && nset == 2) ? 1 : 0;
+  if (!((dh == 64 && (nset == 2 || nset == 4)) || (dh == 128 && nset == 2))) return 0;
+  // rows of the first launch, with a lane's tokens beside each chunk; workgroups of the second (a lane of one chunk has a tile)
+  const long own_rows = H + ((long)H * (P + 2 * N) + 63) / 64;
+  const long passes = (Hq / Hkv + nset - 1) / nset;
+  return own_rows + SSD_SINGLE_TOKENS <= 65535 && n_tiles * (2 * own_rows + 4 * Hkv * passes) <= 0x7fffffffL ? 1 : 0;
 }
 
 static size_t ssd_scan_lds_bytes(int Q, int P, int N) {
@@ -1218,9 +1227,8 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
     if (!b.block_tables || b.max_pages <= 0 || !b.tiles || b.n_tiles <= 0 || !b.cu_seqlens || !b.start_pos || !b.out || !b.k_base ||
         !b.v_base || b.page_size <= 0)
       return ERR_BAD_ARGUMENT;
-    if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
-        b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0 ||
-        b.n_tiles > (1 << 20) || b.Hkv > 256)
+    if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(H, P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
+        b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0)
       return ERR_UNSUPPORTED_SIZE;
     nset = prefill_head_set(b.dh, b.Hq / b.Hkv, b.n_tiles, b.Hkv, b.max_seq_len);
   }

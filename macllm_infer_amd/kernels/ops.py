@@ -169,7 +169,7 @@ _SIGNATURES = {
     },
     "ssd": {
         "mi_ssd_supported": [_c_int, _c_int, _c_int, _c_int, _c_int],
-        "mi_ssd_beside": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
+        "mi_ssd_beside": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
         "mi_ssd_prefill": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr,
                            _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_long,
@@ -2044,9 +2044,9 @@ class PromptBeside:
         page_size = self.k_cache.shape[2]
         if not prefill_attention_supported(q.dtype, self.num_heads, self.num_kv_heads, self.head_dim, page_size):
             return False
-        _, _, P, N = ssm_state.shape
+        _, H, P, N = ssm_state.shape
         if not (_fn("ssd", "mi_ssd_single")(chunk_size, P, N, int(longest), _p(ssm_state))
-                and _fn("ssd", "mi_ssd_beside")(P, N, self.num_heads, self.num_kv_heads, self.head_dim,
+                and _fn("ssd", "mi_ssd_beside")(H, P, N, self.num_heads, self.num_kv_heads, self.head_dim,
                                                 self.query_tiles.shape[0], int(self.max_seq_len or 0))):
             return False
         if not shared_prefill_covers(self.num_kv_heads, self.head_dim, page_size, self.k_cache.stride(0), self.k_cache.data_ptr(),

@@ -1976,6 +1976,23 @@ def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
     assert not make(sizes=(1, 2048, 2048)).fits(8, state, 128)                          # the kernel whose waves share their keys
 
 
+def test_sizes_that_the_scans_launches_refuse_keep_the_attention_in_its_own(ops):
+    """More kv heads than the second launch takes, more rows than the first has, more workgroups than a launch has: what
+    ``ssd_prefill`` would refuse, ``fits`` refuses before anything is launched."""
+    state = torch.zeros(1, 1, 64, 128, device=DEV)
+    one = i32([0, 0]).to(DEV)
+
+    def fits(scan_heads=4, kv_heads=2, tiles=1):
+        q, out = torch.zeros(1, 1024, dtype=torch.bfloat16, device=DEV), torch.zeros(1, 512, dtype=torch.bfloat16, device=DEV)
+        cache = torch.zeros(1, 1, 16, 64, dtype=torch.bfloat16, device=DEV).expand(1, kv_heads, 16, 64)
+        beside = ops.PromptBeside(q, 4 * kv_heads, kv_heads, 64, one, None, 0, None, cache, cache.transpose(2, 3), one.view(1, 2),
+                                  one.view(1, 2).expand(tiles, 2), one, one[:1], 1.0, None, out, 64, (1, 16, 4096))
+        return beside.fits(8, state.expand(1, scan_heads, 64, 128), 128)
+    assert fits() and fits(scan_heads=10000) and fits(kv_heads=256) and fits(tiles=1 << 16)
+    assert not fits(scan_heads=11000) and not fits(kv_heads=257) and not fits(tiles=(1 << 20) + 1)
+    assert not fits(scan_heads=10000, tiles=1 << 16)
+
+
 @pytest.mark.parametrize("T, d", [(257, 64), (300, 1024), (300, 1028), (513, 2052)])
 def test_layer_norm_of_many_rows_adds_a_row_up_in_one_order(ops, T, d):
     """The bits of more than 256 rows: number i of a row belongs to thread i % 256, a thread's numbers are added one after the
