@@ -2456,9 +2456,9 @@ def mixer_decode_supported(num_heads: int, num_kv_heads: int, head_dim: int, pag
 MERGE_AT_ONCE = 8          # runs of keys a merge asks for at once (decode.hip)
 
 
-def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: int = 64):
+def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: int):
     """(keys of a run, runs per token and kv head) as ``mixer_decode`` cuts the contexts of a step of M tokens
-    whose requests hold up to ``span`` keys."""
+    whose requests hold up to ``span`` keys, for heads of ``head_dim``."""
     run_keys, runs = ctypes.c_int(0), ctypes.c_int(0)
     _check(_fn("decode", "mi_mixer_runs")(M, num_kv_heads, head_dim, page_size, span, ctypes.addressof(run_keys),
                                           ctypes.addressof(runs)), "mixer_decode", "(no run length for these sizes)")

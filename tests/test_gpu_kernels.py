@@ -2037,3 +2037,5 @@ def test_runs_of_keys_go_by_the_heads_width_and_the_steps_size(ops):
     assert runs(32, 128, 2048)[1] == 1 and runs(32, 128, 4096)[1] == 2 and runs(16, 128, 2048)[1] == 4
     assert runs(8, 128, 2048) == (512, 4) and runs(4, 128, 2048) == (256, 8) and runs(8, 64, 2048) == (256, 8)
     assert runs(8, 128, 8192) == (512, 8) and runs(8, 64, 8192) == (512, 16)
+    with pytest.raises(TypeError):                          # no width is the right one by default
+        ops.mixer_runs(8, 2, 16, 2048)
