@@ -1081,6 +1081,14 @@ ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __r
 // The same beside the prompt attention of the layer (see PromptBeside): workgroups 0 .. scan_groups - 1 are the scan's, the
 // longer ones, and those after them the attention's, of as many threads; either uses the workgroup's LDS.
 static_assert(SSD_SCAN_WAVES == PREFILL_WAVES, "workgroups of one launch");
+// Heads that share their keys and states of 64 x 128 and more: two launches are the faster way at every such size, by what the
+// launches and the attention behind the scan cost.  37 tokens | 128 | five lanes of 16 behind 700 keys, four launches and two in us, 24 heads
+// of the scan: states of 64 x 128 beside 8 / 2 heads of 64 28.5, 19.2 | 33.8, 24.2 | 33.5, 19.0; 64 x 256 beside 6 / 2 of
+// 64 31.2, 22.5 | 37.5, 28.5 | 36.8, 22.7; 128 x 128 beside 12 / 2 of 128 41.5, 26.6 | 49.8, 33.6 | 53.4, 29.9; 128 x 256
+// beside 8 / 2 of 64 50.6, 41.4 | 58.7, 48.9 | 59.7, 43.9.  (Smaller states, and a key for every query head, are in no shape of this
+// framework and would be six times the instances: 100 s to compile and 5.3 MB, 31 and 1.7 with these.)
+#define BESIDE_LEAST_P 64
+#define BESIDE_LEAST_N 128
 template <int NK, int PT, int DH, int NSET>
 __global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
 ssd_single_beside_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
@@ -1138,7 +1146,7 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
                              float* y, long y_ld, const bf16_t* z, long z_ld, bf16_t* gated, long gated_ld,
                              const SsdSingle& one, const PromptBeside* beside, int nset) {
   const size_t lds = ssd_single_lds_bytes(16 * PT, 32 * NK);
-  if constexpr ((NK == 4 && PT == 4) || (NK == 8 && PT == 8)) {
+  if constexpr (32 * NK >= BESIDE_LEAST_N && 16 * PT >= BESIDE_LEAST_P) {
     if (beside) {
       const int passes = (beside->Hq / beside->Hkv + nset - 1) / nset;
       const long all = (long)grid.x * grid.y + 4L * beside->n_tiles * beside->Hkv * passes;
@@ -1155,7 +1163,7 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
         SINGLE_ARGUMENTS, (int)grid.x, scan_groups, passes, *beside);                                                       \
     return 0;                                                                                                               \
   }
-      BESIDE_CASE(64, 2) BESIDE_CASE(64, 4) BESIDE_CASE(128, 2)
+      BESIDE_CASE(64, 2) BESIDE_CASE(64, 3) BESIDE_CASE(64, 4) BESIDE_CASE(128, 2)
 #undef BESIDE_CASE
     }
   }
@@ -1171,11 +1179,10 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
 // Whether mi_ssd_prefill takes the attention of such heads beside its second launch (of a step that mi_ssd_single covers,
 // whose H heads of the scan may have a group each): what it would refuse is refused here, before anything is launched.
 extern "C" int mi_ssd_beside(int H, int P, int N, int Hq, int Hkv, int dh, int n_tiles, int max_seq_len) {
-  if (H <= 0 || Hkv <= 0 || Hkv > 256 || Hq % Hkv != 0 || n_tiles <= 0 || n_tiles > (1 << 20) ||
-      !((P == 64 && N == 128) || (P == 128 && N == 256)))
+  if (H <= 0 || Hkv <= 0 || Hkv > 256 || Hq <= Hkv || Hq % Hkv != 0 || n_tiles <= 0 || n_tiles > (1 << 20) || (dh != 64 && dh != 128) ||
+      !ssd_staged_sizes(P, N) || P < BESIDE_LEAST_P || N < BESIDE_LEAST_N)
     return 0;
   const int nset = prefill_head_set(dh, Hq / Hkv, n_tiles, Hkv, max_seq_len);
-  if (!((dh == 64 && (nset == 2 || nset == 4)) || (dh == 128 && nset == 2))) return 0;
   // rows of the first launch, with a lane's tokens beside each chunk; workgroups of the second (a lane of one chunk has a tile)
   const long own_rows = H + ((long)H * (P + 2 * N) + 63) / 64;
   const long passes = (Hq / Hkv + nset - 1) / nset;

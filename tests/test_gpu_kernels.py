@@ -1906,7 +1906,8 @@ def test_layer_norm_of_the_stream_and_its_branches(ops, dtype, T, d):
 
 
 @pytest.mark.parametrize("H, P, N, Hq, Hkv, dh", [(24, 64, 128, 8, 2, 64), (3, 64, 128, 4, 1, 64), (4, 128, 256, 12, 2, 128),
-                                                  (5, 128, 256, 2, 1, 64), (2, 64, 128, 4, 2, 128)])
+                                                  (5, 128, 256, 2, 1, 64), (2, 64, 128, 4, 2, 128), (3, 64, 256, 6, 2, 64),
+                                                  (4, 128, 128, 10, 2, 64), (3, 64, 256, 12, 2, 128), (2, 128, 128, 4, 1, 64)])
 @pytest.mark.parametrize("counts, starts, window, longest", [([37], [0], None, 2048), ([1, 5, 128, 64], [0, 700, 0, 33], None, 4096),
                                                              ([16] * 5, [3, 0, 950, 16, 690], 600, 2048)])
 def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, window, longest):
