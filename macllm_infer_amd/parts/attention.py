@@ -199,13 +199,16 @@ class Attention(Mixer):
 
     def prompt_beside(self, qkv: torch.Tensor, step, cache, attended: torch.Tensor):
         """What ``mix`` would launch for this step, for another mixer to run in its launches (``ops.PromptBeside``), or None
-        where that is more or other than a rotation with the cache write and the prompt attention."""
+        where that is more or other than a rotation with the cache write and the prompt attention (a subclass with a ``mix`` of
+        its own among it)."""
+        if getattr(self.mix, "__func__", None) is not Attention.mix:
+            return None
         spec = self.spec
-        rotation = getattr(self.position, "plain_rotation", None)
+        rotation = self.position.plain_rotation()
         if (rotation is None or self.prepared or self.general_only or self.position.score_slopes is not None
                 or step.max_query_len == 1 or not cache.owns_kv or spec.value_width != spec.head_dim):
             return None
-        inv_freq, rotary_dim = rotation()
+        inv_freq, rotary_dim = rotation
         return ops.PromptBeside(qkv, spec.num_heads, spec.num_kv_heads, spec.head_dim, step.positions, inv_freq, rotary_dim,
                                 step.slot_mappings[cache.group], cache.k_cache, cache.v_cache, step.block_tables[cache.group],
                                 step.query_tiles, step.cu_seqlens, step.start_pos, spec.scale, spec.window, attended,

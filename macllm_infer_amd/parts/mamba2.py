@@ -113,9 +113,11 @@ class Mamba2(Mixer):
         return self.out_proj(gated)
 
     def takes_beside(self, u: torch.Tensor, step, cache, gated: torch.Tensor, beside) -> bool:
-        """Whether ``mix`` runs the attention ``beside`` (``ops.PromptBeside``) in its own launches."""
+        """Whether ``mix`` runs the attention ``beside`` (``ops.PromptBeside``) in its own launches (a subclass's own ``mix`` knows
+        nothing of it)."""
         spec = self.spec
-        return (self.norm_weight is None and self._chunked(u, step) and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0
+        return (getattr(self.mix, "__func__", None) is Mamba2.mix and self.norm_weight is None
+                and self._chunked(u, step) and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0
                 and ops.ssd_conv_supported(spec.conv_kernel, spec.conv_width, u[:, spec.inner_size:spec.inner_size + spec.conv_width])
                 and beside.fits(step.max_query_len, cache.states["ssm"], spec.chunk_size))
 

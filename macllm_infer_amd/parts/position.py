@@ -44,6 +44,11 @@ class PositionEncoding(Part):
         mixers whose kernels turn a part of their rows themselves."""
         return None
 
+    def plain_rotation(self):
+        """``(inv_freq, rotary_dim)`` where ``rotate_and_store`` is that rotation and the cache write, and nothing else: a
+        launch of another kind may then do both in its place.  None: it has to be called."""
+        return None
+
     def rotate(self, qkv, num_heads, num_kv_heads, head_dim, step) -> None:
         return None
 
@@ -125,7 +130,9 @@ class Rope(PositionEncoding):
         return self.inv_freq, self.rotary_dim, False
 
     def plain_rotation(self):
-        """(inv_freq, rotary_dim): ``rotate_and_store`` is this rotation and the cache write, and nothing else."""
+        # (a subclass may have a ``rotate_and_store`` of its own)
+        if getattr(self.rotate_and_store, "__func__", None) is not Rope.rotate_and_store:
+            return None
         return self.inv_freq, self.rotary_dim
 
     def rotate_and_store(self, qkv, num_heads, num_kv_heads, head_dim, step, cache) -> None:

@@ -112,6 +112,51 @@ def test_the_clock_is_asked_for_a_second_stream_before_anything_is_reserved(host
     assert order == [["e"], "reserve"]
 
 
+def test_a_part_with_a_method_of_its_own_keeps_it_in_short_prompts():
+    """The launches that run a short prompt's attention beside the state-space scan stand in for ``Rope.rotate_and_store``,
+    ``Attention.mix`` and ``Mamba2.mix`` as they are: what a subclass, or a program, puts in their place is called."""
+    from types import SimpleNamespace
+    from macllm_infer_amd.config import RopeSpec
+    from macllm_infer_amd.parts.attention import Attention
+    from macllm_infer_amd.parts.base import BuildContext
+    from macllm_infer_amd.parts.mamba2 import Mamba2
+    from macllm_infer_amd.parts.position import Rope
+
+    class OwnRope(Rope):
+        def rotate_and_store(self, *arguments):
+            pass
+
+    class OwnAttention(Attention):
+        def mix(self, *arguments):
+            pass
+
+    class OwnMamba2(Mamba2):
+        def mix(self, *arguments):
+            pass
+    build = BuildContext(hidden_size=64, dtype=torch.float32, device=torch.device("cpu"), max_context=64)
+    rope = Rope(RopeSpec(1e4, 16), 16, build)
+    assert rope.plain_rotation()[1] == 16 and OwnRope(RopeSpec(1e4, 16), 16, build).plain_rotation() is None
+    step = SimpleNamespace(max_query_len=5, positions=None, slot_mappings=[None], block_tables=[None], query_tiles=None,
+                           cu_seqlens=None, start_pos=None, max_seq_len=64, sizes=None)
+    cache = SimpleNamespace(owns_kv=True, group=0, k_cache=None, v_cache=None)
+
+    def attention(kind, position):
+        made = object.__new__(kind)
+        made.spec = SimpleNamespace(num_heads=4, num_kv_heads=2, head_dim=16, value_width=16, scale=1.0, window=None)
+        made.prepared = made.general_only = False
+        made.position = position
+        return made
+    assert attention(Attention, rope).prompt_beside(None, step, cache, None) is not None
+    assert attention(Attention, OwnRope(RopeSpec(1e4, 16), 16, build)).prompt_beside(None, step, cache, None) is None
+    assert attention(OwnAttention, rope).prompt_beside(None, step, cache, None) is None
+    patched = attention(Attention, rope)
+    patched.mix = lambda *arguments: None
+    assert patched.prompt_beside(None, step, cache, None) is None
+    scan = object.__new__(OwnMamba2)
+    scan.spec = scan.norm_weight = None
+    assert scan.takes_beside(None, step, cache, None, None) is False
+
+
 def test_refused_steps_change_nothing(host_ops, tmp_path):
     engine, cfg, tensors = engine_for("A", tmp_path, capacity=32, page=8, requests=2)
     engine.add_request("a")
