@@ -344,20 +344,20 @@ class DecodeGraphs:
             static = StaticStep(self.cache, bucket, context or self.max_seq_len, self.device,
                                 **self.model.step_layout)
         # a first run outside the graph lets the libraries set themselves up; every lane is padding,
-        # so only the scratch page and slot are touched.  It runs on the kind's own stream: a graph of another kind may be
+        # so only the scratch page and slot are touched.  It runs on a stream of the kind's own: a graph of another kind may be
         # under way, and the library's workspace on a stream drawn for the moment might be that graph's
-        stream = self.streams.recording[kind]
-        stream.wait_stream(torch.cuda.current_stream(self.device))
-        with torch.cuda.stream(stream):
+        warming = self.streams.warming[kind]
+        warming.wait_stream(torch.cuda.current_stream(self.device))
+        with torch.cuda.stream(warming):
             for _ in range(warm_runs):
                 self.model.forward(static.context, self.cache)
-        torch.cuda.current_stream(self.device).wait_stream(stream)
+        torch.cuda.current_stream(self.device).wait_stream(warming)
         torch.cuda.synchronize(self.device)
         graph = torch.cuda.CUDAGraph()
         # one pool for every graph of a kind: their replays never overlap, so their intermediate buffers may share memory
         if pool is None:
             pool = self._pools.setdefault(kind, torch.cuda.graph_pool_handle())
-        with torch.cuda.graph(graph, pool=pool, stream=stream):
+        with torch.cuda.graph(graph, pool=pool, stream=self.streams.recording[kind]):
             logits = self.model.forward(static.context, self.cache)
         return static, graph, logits
 

@@ -23,19 +23,25 @@ BESIDE_STREAMS = 5
 
 
 class BatchStreams:
-    """``recording[kind]``: the stream that graphs of the kind are warmed up and recorded on; ``side[kind]``: the stream that
-    they fork their first mixer to; ``beside``: streams that a graph may be replayed on beside the caller's stream."""
+    """``warming[kind]``: the stream that a step of the kind runs on before its graph is recorded (not the recording one: a
+    library's workspace that is there before the first recording is not the graph's own, and a decode step of 12 requests
+    of the experts' model takes 1,248 us instead of 1,242); ``recording[kind]``: the stream that its graphs are recorded on;
+    ``side[kind]``: the stream that they fork their first mixer to; ``beside``: streams that a graph may be replayed on beside
+    the caller's stream."""
 
     def __init__(self, draw: Callable, usual: Optional["torch.cuda.Stream"] = None):
         """``draw()``: a stream, perhaps one that is taken.  ``usual``: the stream that torch records graphs on by default."""
         self._draw = draw
         self._taken = []
-        self.recording, self.side = {}, {}
+        self.warming, self.recording, self.side = {}, {}, {}
+        if usual is not None:
+            self.recording[SINGLES] = usual
+            self._taken.append(usual)
         for kind in KINDS:
-            self.recording[kind] = self.apart() if usual is None or kind != SINGLES else usual
-            self._taken.append(self.recording[kind])
-            self.side[kind] = self.apart()
-            self._taken.append(self.side[kind])
+            for streams in (self.recording, self.side, self.warming):
+                if kind not in streams:
+                    streams[kind] = self.apart()
+                    self._taken.append(streams[kind])
         self.beside = []
         for _ in range(BESIDE_STREAMS):
             self.beside.append(self.apart())
@@ -49,14 +55,14 @@ class BatchStreams:
                 return stream
 
     def side_of(self, main: "torch.cuda.Stream") -> Optional["torch.cuda.Stream"]:
-        """The stream that work recorded on ``main`` forks to (None: no kind of batch is recorded there)."""
+        """The stream that work on ``main`` forks to (None: no kind of batch is warmed up or recorded there)."""
         for kind in KINDS:
-            if main == self.recording[kind]:
+            if main == self.recording[kind] or main == self.warming[kind]:
                 return self.side[kind]
         return None
 
     def belongs_to(self, kind: str, stream: "torch.cuda.Stream") -> bool:
-        return stream == self.recording[kind] or stream == self.side[kind]
+        return any(stream == streams[kind] for streams in (self.warming, self.recording, self.side))
 
 
 _of_device: Dict[int, BatchStreams] = {}

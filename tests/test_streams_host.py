@@ -99,17 +99,18 @@ def test_no_capture_of_portions_works_on_a_stream_of_the_single_tokens(cuda, dra
 def test_every_kind_of_batch_has_streams_of_its_own(cuda):
     of_device = streams.batch_streams(DEVICE)
     assert streams.batch_streams(DEVICE) is of_device
-    own = [stream for kind in streams.KINDS for stream in (of_device.recording[kind], of_device.side[kind])]
+    own = [stream for kind in streams.KINDS for stream in (of_device.warming[kind], of_device.recording[kind], of_device.side[kind])]
     assert len(set(own + of_device.beside)) == len(own) + len(of_device.beside)
     assert of_device.recording[streams.SINGLES] == torch.cuda.graph.default_capture_stream
     for _ in range(2 * POOL):
         assert of_device.apart() not in own + of_device.beside
     for kind in streams.KINDS:
         assert block.side_stream(DEVICE, of_device.recording[kind]) == of_device.side[kind]
+        assert block.side_stream(DEVICE, of_device.warming[kind]) == of_device.side[kind]
     for number in range(POOL):                           # work on any other stream forks to none of a kind's
         main = FakeStream(number=number)
         side = block.side_stream(DEVICE, main)
-        assert side != main and (main in [of_device.recording[kind] for kind in streams.KINDS] or side not in own)
+        assert side != main and (of_device.side_of(main) is not None or side not in own)
 
 
 def engine_on(monkeypatch, asked):
