@@ -23,22 +23,20 @@ BESIDE_STREAMS = 5
 
 
 class BatchStreams:
-    """``warming[kind]``: the stream that a step of the kind runs on before its graph is recorded (not the recording one: a
-    library's workspace that is there before the first recording is not the graph's own, and a decode step of 12 requests
-    of the experts' model takes 1,248 us instead of 1,242); ``recording[kind]``: the stream that its graphs are recorded on;
-    ``side[kind]``: the stream that they fork their first mixer to; ``beside``: streams that a graph may be replayed on beside
-    the caller's stream."""
+    """``recording[kind]``: the stream that graphs of the kind are recorded on; ``side[kind]``: the stream that they fork their
+    first mixer to; ``beside``: streams that a graph may be replayed on beside the caller's stream.  What runs ahead of a
+    recording, or forks elsewhere, is on a stream ``apart`` from all of these."""
 
     def __init__(self, draw: Callable, usual: Optional["torch.cuda.Stream"] = None):
         """``draw()``: a stream, perhaps one that is taken.  ``usual``: the stream that torch records graphs on by default."""
         self._draw = draw
         self._taken = []
-        self.warming, self.recording, self.side = {}, {}, {}
+        self.recording, self.side = {}, {}
         if usual is not None:
             self.recording[SINGLES] = usual
             self._taken.append(usual)
         for kind in KINDS:
-            for streams in (self.recording, self.side, self.warming):
+            for streams in (self.recording, self.side):
                 if kind not in streams:
                     streams[kind] = self.apart()
                     self._taken.append(streams[kind])
@@ -55,14 +53,14 @@ class BatchStreams:
                 return stream
 
     def side_of(self, main: "torch.cuda.Stream") -> Optional["torch.cuda.Stream"]:
-        """The stream that work on ``main`` forks to (None: no kind of batch is warmed up or recorded there)."""
+        """The stream that work recorded on ``main`` forks to (None: no kind of batch is recorded there)."""
         for kind in KINDS:
-            if main == self.recording[kind] or main == self.warming[kind]:
+            if main == self.recording[kind]:
                 return self.side[kind]
         return None
 
     def belongs_to(self, kind: str, stream: "torch.cuda.Stream") -> bool:
-        return any(stream == streams[kind] for streams in (self.warming, self.recording, self.side))
+        return stream == self.recording[kind] or stream == self.side[kind]
 
 
 _of_device: Dict[int, BatchStreams] = {}

@@ -36,7 +36,7 @@ class FakeStream:
 @pytest.fixture()
 def cuda(monkeypatch):
     """torch.cuda's streams and captures without a GPU; ``current`` is the stream that work would be queued on."""
-    state = SimpleNamespace(current=FakeStream(number=-1))
+    state = SimpleNamespace(current=FakeStream(number=-1), capturing=False, recorded=set())
 
     @contextlib.contextmanager
     def on(stream):
@@ -55,9 +55,11 @@ def cuda(monkeypatch):
             self.on = on(stream if stream is not None else FakeGraph.default_capture_stream)
 
         def __enter__(self):
+            state.capturing = True
             return self.on.__enter__()
 
         def __exit__(self, *error):
+            state.capturing = False
             return self.on.__exit__(*error)
 
     FakeStream.turn = 0
@@ -76,7 +78,9 @@ def captures(state, kind, drawn_between=0):
 
     def forward(context, cache):
         used.add(state.current)
-        used.add(block.side_stream(DEVICE, state.current))
+        if state.capturing:                                  # (only what is recorded forks)
+            used.add(block.side_stream(DEVICE, state.current))
+            state.recorded |= {state.current, block.side_stream(DEVICE, state.current)}
     bank = graphs_module.DecodeGraphs(SimpleNamespace(forward=forward, blocks=[], step_layout={}), None, DEVICE, 4096)
 
     def capture():
@@ -89,8 +93,10 @@ def captures(state, kind, drawn_between=0):
 
 @pytest.mark.parametrize("drawn_between", [0, 1, 2, 5])
 def test_no_capture_of_portions_works_on_a_stream_of_the_single_tokens(cuda, drawn_between):
-    """33 captures in a row, other parts of the program drawing streams in between, while single tokens may be under way."""
-    singles = set(captures(cuda, "singles")())
+    """33 captures in a row, other parts of the program drawing streams in between, while single tokens may be under way: their
+    graph works on the streams that it was recorded and forked on."""
+    captures(cuda, "singles")()
+    singles = set(cuda.recorded)
     capture = captures(cuda, "portions", drawn_between)
     for _ in range(POOL + 1):
         assert not singles & capture()
@@ -99,14 +105,13 @@ def test_no_capture_of_portions_works_on_a_stream_of_the_single_tokens(cuda, dra
 def test_every_kind_of_batch_has_streams_of_its_own(cuda):
     of_device = streams.batch_streams(DEVICE)
     assert streams.batch_streams(DEVICE) is of_device
-    own = [stream for kind in streams.KINDS for stream in (of_device.warming[kind], of_device.recording[kind], of_device.side[kind])]
+    own = [stream for kind in streams.KINDS for stream in (of_device.recording[kind], of_device.side[kind])]
     assert len(set(own + of_device.beside)) == len(own) + len(of_device.beside)
     assert of_device.recording[streams.SINGLES] == torch.cuda.graph.default_capture_stream
     for _ in range(2 * POOL):
         assert of_device.apart() not in own + of_device.beside
     for kind in streams.KINDS:
         assert block.side_stream(DEVICE, of_device.recording[kind]) == of_device.side[kind]
-        assert block.side_stream(DEVICE, of_device.warming[kind]) == of_device.side[kind]
     for number in range(POOL):                           # work on any other stream forks to none of a kind's
         main = FakeStream(number=number)
         side = block.side_stream(DEVICE, main)
