@@ -1147,6 +1147,179 @@ add_layernorm_kernel(float* __restrict__ h, NormBranch b0, NormBranch b1, NormBr
     o[i] = from_float<TO>((wide_row[i] - mean) / denominator * weight[i] + bias[i]);
 }
 
+template <int VEC>
+__device__ __forceinline__ void floats_at(const float* from, float (&to)[VEC]) {
+  if constexpr (VEC == 4) {
+    const float4 piece = *reinterpret_cast<const float4*>(from);
+    to[0] = piece.x; to[1] = piece.y; to[2] = piece.z; to[3] = piece.w;
+  } else {
+    to[0] = from[0];
+  }
+}
+
+typedef __bf16 common_bf16x4 __attribute__((ext_vector_type(4)));
+
+// The same bits by one wave a row, up to 2,048 columns in whole pieces of four at aligned addresses, without a barrier: lane l
+// keeps the pieces 4 l + 256 k, which are the numbers of four neighbouring threads above.  It adds those up in the same
+// order, and the lanes then add what the threads' waves add: pairs of threads 32 apart are lanes 8 apart, and so on
+// down to 4 threads and 1 lane, pairs 2 and 1 apart lie in one lane, and the four waves are the rows of 16 lanes.  What bounds it
+// is the rows' traffic and the chain of one row: 1,554 rows of 1,024 7.2 us above, 5.4 here (21 MB, 4.2 at the rate of a large
+// copy), with a norm on the branch 9.7 and 7.2; 300 rows 4.7 and 3.7, 6.5 and 4.5; 1,999 rows of 2,048 12.4 and 9.0.  Beyond
+// that a wave keeps too much of a row (1,999 rows of 3,072: 18.7 above, 23.9 here).
+template <int CONTROL>
+__device__ __forceinline__ float layernorm_dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CONTROL, 0xf, 0xf, true));
+}
+
+// (a factor times a branch is rounded before it is added, as above)
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
+
+template <int PIECES>
+__device__ __forceinline__ float layernorm_row_sum(const float (&x)[PIECES][4], bool squares) {
+  float mine[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) mine[j] = squares ? fmaf(x[k][j], x[k][j], mine[j]) : mine[j] + x[k][j];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    mine[j] += layernorm_dpp<0x128>(mine[j]);           // row_ror 8: the lane 8 apart
+    mine[j] += layernorm_dpp<0x124>(mine[j]);           // row_ror 4: 4 apart, as lanes 8 apart hold the same now
+    mine[j] += layernorm_dpp<0x4E>(mine[j]);            // quad_perm [2, 3, 0, 1]
+    mine[j] += layernorm_dpp<0xB1>(mine[j]);            // quad_perm [1, 0, 3, 2]
+  }
+  const float sum = (mine[0] + mine[2]) + (mine[1] + mine[3]);
+  float total = 0.f;
+#pragma unroll
+  for (int wave = 0; wave < 4; ++wave)
+    total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sum), 16 * wave));
+  return total;
+}
+
+template <typename TO, int PIECES>
+__global__ void __launch_bounds__(WAVE)
+add_layernorm_wave_kernel(float* __restrict__ h, NormBranch b0, NormBranch b1, NormBranch b2,
+                          const float* __restrict__ vector, const float* __restrict__ weight,
+                          const float* __restrict__ bias, float eps, const float* __restrict__ branch_weight,
+                          const float* __restrict__ branch_bias, float branch_eps, TO* __restrict__ out,
+                          const int* __restrict__ rows, int d) {
+  typedef TO four __attribute__((ext_vector_type(4)));
+  constexpr bool AT_ONCE = PIECES <= 4;          // the norms' weights beside the rows; longer rows leave no registers for them
+  const long out_row = blockIdx.x;
+  const long row = rows ? (long)rows[out_row] : out_row;
+  float v[PIECES][4], branch[3][PIECES][4], w[PIECES][4], b[PIECES][4], bw[PIECES][4], bb[PIECES][4], extra[PIECES][4];
+  const NormBranch of[3] = {b0, b1, b2};
+  auto column = [&](int k) { return ((int)threadIdx.x + k * WAVE) * 4; };
+#pragma unroll
+  for (int k = 0; k < PIECES; ++k) {
+    // a piece past the end is zeros, which change no sum
+    const bool live = column(k) < d;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[k][j] = 0.f;
+    if (live) floats_at<4>(h + row * d + column(k), v[k]);
+    if (AT_ONCE && live) {
+      if (branch_weight) {
+        floats_at<4>(branch_weight + column(k), bw[k]);
+        floats_at<4>(branch_bias + column(k), bb[k]);
+      }
+      if (vector) floats_at<4>(vector + column(k), extra[k]);
+      if (out) {
+        floats_at<4>(weight + column(k), w[k]);
+        floats_at<4>(bias + column(k), b[k]);
+      }
+    }
+  }
+  // (a branch's pieces one after the other: all are under way before the first is waited for)
+#pragma unroll
+  for (int which = 0; which < 3; ++which) {
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) branch[which][k][j] = 0.f;
+    if (!of[which].rows) continue;
+    if (of[which].dtype == DT_BF16) {
+      common_bf16x4 piece[PIECES];
+#pragma unroll
+      for (int k = 0; k < PIECES; ++k)             // (past the end: the last piece, dropped)
+        piece[k] = *reinterpret_cast<const common_bf16x4*>((const bf16_t*)of[which].rows + row * d + min(column(k), d - 4));
+#pragma unroll
+      for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) branch[which][k][j] = column(k) < d ? (float)piece[k][j] : 0.f;
+    } else {
+#pragma unroll
+      for (int k = 0; k < PIECES; ++k)
+        if (column(k) < d) floats_at<4>((const float*)of[which].rows + row * d + column(k), branch[which][k]);
+    }
+  }
+  if (branch_weight) {
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float sum = rounded_product(b0.factor, branch[0][k][j]);
+        sum += rounded_product(b1.factor, branch[1][k][j]);
+        sum += rounded_product(b2.factor, branch[2][k][j]);
+        branch[0][k][j] = sum;
+      }
+    const float mean = layernorm_row_sum<PIECES>(branch[0], false) / (float)d;
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) branch[0][k][j] = column(k) < d ? branch[0][k][j] - mean : 0.f;
+    const float denominator = sqrtf(layernorm_row_sum<PIECES>(branch[0], true) / (float)d + branch_eps);
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+      if (column(k) >= d) continue;
+      if (!AT_ONCE) {
+        floats_at<4>(branch_weight + column(k), bw[k]);
+        floats_at<4>(branch_bias + column(k), bb[k]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[k][j] += branch[0][k][j] / denominator * bw[k][j] + bb[k][j];
+    }
+  } else {
+#pragma unroll
+    for (int which = 0; which < 3; ++which)
+#pragma unroll
+      for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[k][j] += rounded_product(of[which].factor, branch[which][k][j]);
+  }
+#pragma unroll
+  for (int k = 0; k < PIECES; ++k) {
+    if (column(k) >= d) continue;
+    if (vector) {
+      if (!AT_ONCE) floats_at<4>(vector + column(k), extra[k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[k][j] += extra[k][j];
+    }
+    if (!rows) *reinterpret_cast<float4*>(h + row * d + column(k)) = make_float4(v[k][0], v[k][1], v[k][2], v[k][3]);
+  }
+  if (!out) return;
+  const float mean = layernorm_row_sum<PIECES>(v, false) / (float)d;
+#pragma unroll
+  for (int k = 0; k < PIECES; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[k][j] = column(k) < d ? v[k][j] - mean : 0.f;
+  const float denominator = sqrtf(layernorm_row_sum<PIECES>(v, true) / (float)d + eps);
+#pragma unroll
+  for (int k = 0; k < PIECES; ++k) {
+    if (column(k) >= d) continue;
+    if (!AT_ONCE) {
+      floats_at<4>(weight + column(k), w[k]);
+      floats_at<4>(bias + column(k), b[k]);
+    }
+    four piece;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) piece[j] = from_float<TO>(v[k][j] / denominator * w[k][j] + b[k][j]);
+    *reinterpret_cast<four*>(out + out_row * d + column(k)) = piece;
+  }
+}
+
 // The same for steps of few rows, whose time is the chain of waits: a thread keeps PER elements of the row in
 // registers (element threadIdx.x + k * blockDim.x), and everything the later stages read from memory (the stream's
 // row, the norms' weights and biases) is asked for at the start, beside the branches' rows.
@@ -1260,6 +1433,22 @@ extern "C" int mi_add_layernorm(float* h, const void* rows0, int dtype0, float f
     return 0;
   }
   const int threads = (d > 2048 && n_rows <= 512) ? 1024 : 256;
+  const uintptr_t addresses = (uintptr_t)h | (uintptr_t)rows0 | (uintptr_t)rows1 | (uintptr_t)rows2 | (uintptr_t)vector |
+                              (uintptr_t)weight | (uintptr_t)bias | (uintptr_t)branch_weight | (uintptr_t)branch_bias |
+                              (uintptr_t)out;
+  if (d % 4 == 0 && d <= 2048 && addresses % 16 == 0 && (out_dtype == DT_F32 || out_dtype == DT_BF16)) {
+#define WAVE_LAUNCH(TO_, PIECES_)                                                                                  \
+  add_layernorm_wave_kernel<TO_, PIECES_><<<n_rows, WAVE, 0, stream>>>(h, b0, b1, b2, vector, weight, bias, eps,   \
+                                                                       branch_weight, branch_bias, branch_eps,     \
+                                                                       (TO_*)out, rows, d)
+    if (d <= 1024 && out_dtype == DT_F32) WAVE_LAUNCH(float, 4);
+    else if (d <= 1024) WAVE_LAUNCH(bf16_t, 4);
+    else if (out_dtype == DT_F32) WAVE_LAUNCH(float, 8);
+    else WAVE_LAUNCH(bf16_t, 8);
+#undef WAVE_LAUNCH
+    RETURN_IF_LAUNCH_FAILED();
+    return 0;
+  }
   const size_t lds = (size_t)d * sizeof(float);
   if (out_dtype == DT_F32)
     add_layernorm_kernel<float><<<n_rows, threads, lds, stream>>>(h, b0, b1, b2, vector, weight, bias, eps, branch_weight,
@@ -1278,18 +1467,6 @@ extern "C" int mi_add_layernorm(float* h, const void* rows0, int dtype0, float f
 // are gathered); out (if wanted) = v / sqrt(mean(v^2) + eps) * weight.  One workgroup a row, which stays in registers: a
 // thread keeps CHUNKS pieces of VEC neighbouring elements (piece threadIdx.x + k * blockDim.x), and everything the later
 // stages read from memory is asked for at the start, beside the branches' rows.
-template <int VEC>
-__device__ __forceinline__ void floats_at(const float* from, float (&to)[VEC]) {
-  if constexpr (VEC == 4) {
-    const float4 piece = *reinterpret_cast<const float4*>(from);
-    to[0] = piece.x; to[1] = piece.y; to[2] = piece.z; to[3] = piece.w;
-  } else {
-    to[0] = from[0];
-  }
-}
-
-typedef __bf16 common_bf16x4 __attribute__((ext_vector_type(4)));
-
 template <int VEC>
 __device__ __forceinline__ void add_branch(const NormBranch& branch, long at, float (&to)[VEC]) {
   if (!branch.rows) return;

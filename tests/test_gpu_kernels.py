@@ -1977,6 +1977,40 @@ def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
     assert not make(sizes=(1, 2048, 2048)).fits(8, state, 128)                          # the kernel whose waves share their keys
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d", [4, 252, 260, 1024, 1028, 2044, 2048])
+@pytest.mark.parametrize("count, normed", [(0, False), (1, False), (2, False), (3, False), (1, True), (3, True)])
+def test_layer_norm_of_many_rows_by_waves_has_the_bits_of_workgroups(ops, dtype, d, count, normed):
+    """The same numbers at addresses that are not aligned go through the kernel of a workgroup a row: the stream and the
+    normed rows, all of them and gathered, are the same bits for any branches and factors."""
+    T = 300
+
+    def placed(tensor, shift):
+        buffer = torch.empty(tensor.numel() + 4, dtype=tensor.dtype, device=DEV)
+        view = buffer[shift:shift + tensor.numel()].view(tensor.shape)
+        view.copy_(tensor)
+        return view
+    h, vector, weight, bias, bw, bb = rand(T, d, seed=1), *(rand(d, seed=seed) for seed in range(2, 7))
+    branches = [(rand(T, d, seed=10 + index, dtype=dtype if index != 1 else torch.float32), factor)
+                for index, factor in zip(range(count), (0.3, -1.7, 1.0))]
+    outcomes = []
+    for shift in (0, 1):
+        stream, extra, w, b = placed(h, shift), placed(vector, shift), placed(weight, shift), placed(bias, shift)
+        placed_branches = [(placed(rows, shift), factor) for rows, factor in branches]
+        norm = (placed(bw, shift), placed(bb, shift), 1e-5) if normed else None
+        out = placed(torch.zeros(T, d, dtype=dtype), shift)
+        results = []
+        if not normed:
+            rows = i32([(7 * i) % T for i in range(260)]).to(DEV)
+            gathered = placed(torch.zeros(260, d, dtype=dtype), shift)
+            ops.add_layernorm(stream, placed_branches, extra, w, b, 1e-5, gathered, rows=rows)
+            results.append(gathered)
+        ops.add_layernorm(stream, placed_branches, None if count == 2 else extra, w, b, 1e-5, out, branch_norm=norm)
+        outcomes.append(results + [stream, out])
+    for by_waves, by_workgroups in zip(*outcomes):
+        assert torch.equal(by_waves, by_workgroups)
+
+
 def test_sizes_that_the_scans_launches_refuse_keep_the_attention_in_its_own(ops):
     """More kv heads than the second launch takes, more rows than the first has, more workgroups than a launch has: what
     ``ssd_prefill`` would refuse, ``fits`` refuses before anything is launched."""
@@ -1994,7 +2028,7 @@ def test_sizes_that_the_scans_launches_refuse_keep_the_attention_in_its_own(ops)
     assert not fits(scan_heads=10000, tiles=1 << 16)
 
 
-@pytest.mark.parametrize("T, d", [(257, 64), (300, 1024), (300, 1028), (513, 2052)])
+@pytest.mark.parametrize("T, d", [(257, 4), (257, 64), (300, 1020), (300, 1022), (300, 1024), (300, 1028), (300, 2048), (513, 2052)])
 def test_layer_norm_of_many_rows_adds_a_row_up_in_one_order(ops, T, d):
     """The bits of more than 256 rows: number i of a row belongs to thread i % 256, a thread's numbers are added one after the
     other, the lanes of a wave in halves, the four waves from the first on.  (Behind such a norm a router chooses experts: another
