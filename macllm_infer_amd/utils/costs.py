@@ -223,7 +223,7 @@ def total(costs: Dict[str, Cost]) -> Cost:
 DECODE_GROUPS: List[Tuple[str, str]] = [
     (r"mixer_decode_kernel|mixer_merge_kernel|decode_attention_kernel|decode_merge_kernel|ssm_scan_kernel|conv_step_kernel|"
      r"gate_norm_kernel|rope_kv_store_kernel|paged_attention_kernel|paged_attention_tile_kernel|"
-     r"paged_attention_merge_kernel|linear_state_|head_norm_gate_kernel|wide_norm_gate_kernel|tanh_rows_kernel|latent_|rotate_heads_kernel|attention_prepare_kernel", "mixers"),
+     r"paged_attention_merge_kernel|linear_state_|head_norm_gate_|wide_norm_gate_kernel|tanh_rows_kernel|latent_|rotate_heads_kernel|attention_prepare_kernel", "mixers"),
     (r"fused_gemm_kernel<\d+, \d+, 2|shared_rows_gemm_kernel<\d+, \d+, 2", "input projections"),
     (r"moe_expert_gemm_kernel<[^>]*(?:true|false), false|moe_expert_gemm_kernelI\w*Lb[01]ELb0E|moe_combine",
      "output projections + down projections"),                   # (the experts' down products: not gated)
@@ -232,11 +232,12 @@ DECODE_GROUPS: List[Tuple[str, str]] = [
      "output projections + down projections"),
 ]
 PLAIN_PRODUCT = r"fused_gemm_kernel<\d+, [01], 0"
+# (of lanes of one chunk, up to 128 tokens, the scan's two launches hold the attention too)
 PREFILL_GROUPS: List[Tuple[str, str]] = [
     (r"^Cijk_|gemm_f32_kernel|tiled_f32_kernel|head_gemm_kernel|moe_expert_gemm", "matrix products"),
     (r"prefill_attention|prefill_shared|paged_attention_kernel|paged_attention_tile_kernel|paged_attention_merge_kernel|"
      r"rope_kv_store_kernel|latent_|attention_prepare_kernel|rotate_heads_kernel", "attention"),
-    (r"ssd_|ssm_scan_kernel|conv1d_silu|conv_state_update|gate_norm_kernel|linear_state_|linear_chunk_|linear_matrix_|head_norm_gate_kernel|"
+    (r"ssd_|ssm_scan_kernel|conv1d_silu|conv_state_update|gate_norm_kernel|linear_state_|linear_chunk_|linear_matrix_|head_norm_gate_|"
      r"wide_norm_gate_kernel|tanh_rows_kernel", "state-space scan"),
 ]
 
