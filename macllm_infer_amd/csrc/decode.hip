@@ -31,6 +31,9 @@
 //     waves split K and feed the matrix cores (v_mfma_f32_16x16x32_bf16: A = 16 weight rows x 32 k,
 //     B = 16 batch rows x 32 k, both contiguous in k), then sum their partial tiles through LDS.
 //
+//   skinny : the same behind the plain prologue with one tile of 16 features a workgroup, which is what the four
+//     products of a small step are: fewer instructions and everything in flight at once (see there).
+//
 //   shared_rows_gemm : the same product behind the plain prologue where the rows of x, fetched by every wave
 //     of fused_gemm, cross the caches as often as the weights (16 rows) or several times as often: a workgroup's
 //     four waves own tiles of 16 features each and walk the same columns, which go through LDS once a
@@ -123,49 +126,22 @@ __device__ __forceinline__ float gate_act_f(int kind, float z) {
 
 // the activation of a gate and the up value beside it; clamped: g sigmoid(alpha g) (u + offset) with g = min(gate, limit),
 // u = clamp(up, -limit, limit)
-__device__ __forceinline__ float gated_f(const FusedGemmParams& p, float gate, float up) {
+template <typename Params>
+__device__ __forceinline__ float gated_f(const Params& p, float gate, float up) {
   if (p.gate_act != 2) return gate_act_f(p.gate_act, gate) * up;
   const float g = fminf(gate, p.act_limit);
   const float u = fminf(fmaxf(up, -p.act_limit), p.act_limit);
   return g / (1.0f + expf(-p.act_alpha * g)) * (u + p.act_offset);
 }
 
-// What is left of a step for a workgroup that takes `rows` of its rows from row0 on (plain prologue).
-__device__ __forceinline__ void take_rows(FusedGemmParams& p, int row0, int rows) {
-  if (p.x) p.x += (long)row0 * p.x_ld;
-  if (p.out) p.out = p.out_f32 ? (void*)(reinterpret_cast<float*>(p.out) + (long)row0 * p.out_ld)
-                               : (void*)(reinterpret_cast<bf16_t*>(p.out) + (long)row0 * p.out_ld);
-  if (p.slot_ids) p.slot_ids += row0;
-  if (p.res_h) {
-    p.res_h += (long)row0 * p.N;
-    if (p.res_hb) p.res_hb += (long)row0 * p.res_hb_ld;
-    if (p.ssq_out) p.ssq_out += row0;
-  }
-  if (p.ssq_in) p.ssq_in += row0;
-  p.M = min(rows, p.M - row0);
-}
-
 __device__ __forceinline__ float round_bf16(float v) { return (float)(bf16_t)v; }
 
-template <int MT, int PRO, int EPI, int FG_WAVES, int NT, bool ROW_TILES = false>
-__global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmParams whole_step) {
+template <int MT, int PRO, int EPI, int FG_WAVES, int NT>
+__global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmParams p) {
   static_assert(NT == 1 || PRO == PRO_PLAIN, "several feature tiles a workgroup: plain prologue only");
-  // Row tiles: a workgroup takes MT tiles of 16 rows of the step and row_tiles workgroups share a tile of
-  // features.  Workgroups go to the eight dies in turn and each die has a cache of its own, so those that share
-  // weights are given numbers that are 8 apart and follow each other: the weights leave memory once.
-  FusedGemmParams p = whole_step;
   const int slab_rows = p.M;
-  int block_x = blockIdx.x;
-  int ssq_rows = p.ssq_ld;              // rows of the tables of partial sums of squares from this workgroup's first row on
-  if (ROW_TILES) {
-    static_assert(!ROW_TILES || (PRO == PRO_PLAIN && NT == 1), "rows dealt out: plain prologue, one tile of features");
-    const int die = block_x % 8, turn = block_x / 8;
-    block_x = (turn / p.row_tiles) * 8 + die;
-    if (block_x * 16 * NT >= p.N) return;
-    const int row0 = (turn % p.row_tiles) * MT * 16;
-    ssq_rows -= row0;
-    take_rows(p, row0, MT * 16);
-  }
+  const int block_x = blockIdx.x;
+  const int ssq_rows = p.ssq_ld;        // rows of the tables of partial sums of squares
   static_assert(PRO != PRO_MERGE || EPI == EPI_PLAIN || EPI == EPI_RESIDUAL, "the merge prologue comes with the plain or the residual epilogue");
   static_assert(EPI != EPI_RESIDUAL || (NT == 1 && PRO != PRO_NORM), "the residual epilogue: one tile of features, rows given as they are");
   static_assert(EPI != EPI_TANH || (NT == 1 && PRO == PRO_PLAIN), "the tanh epilogue: one tile of features, the plain prologue");
@@ -623,10 +599,10 @@ __global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmPa
     if (EPI == EPI_RESIDUAL) {
       __syncthreads();
       if (tid < min(MT * 16, ssq_rows)) {
-        float squares = 0.f;
+        float squares[4];                       // in the order of skinny_kernel: fours, then pairs of them
 #pragma unroll
-        for (int f = 0; f < 16; ++f) squares += tile[f * (MT * 16) + tid];
-        p.ssq_out[(long)block_x * p.ssq_ld + tid] = squares;
+        for (int f = 0; f < 16; ++f) squares[f / 4] = (f % 4 ? squares[f / 4] : 0.f) + tile[f * (MT * 16) + tid];
+        p.ssq_out[(long)block_x * p.ssq_ld + tid] = (squares[0] + squares[1]) + (squares[2] + squares[3]);
       }
     }
     if (EPI == EPI_SWIGLU) {
@@ -657,6 +633,393 @@ static size_t fused_gemm_lds(int MT, int pro, int K, int M, int staged = 0) {
   return bytes;
 }
 
+// ---------------------------------------------------------------- skinny product
+// fused_gemm behind rows given in bfloat16 (no prologue), one tile of 16 features a workgroup: four products of every
+// layer of a decode step.  Such a launch is bound by a chain of round trips (its arguments, the weights, the rows that the
+// launch before has just written on other dies, LDS) and by its instructions (64 of them cost a wave 0.1 us), not by
+// bandwidth, so: what does not change with the sizes is fixed at compile time, all of a wave's weights and rows are asked
+// for before the first product (EXACT: CH chunks of 32 columns a wave; longer K in two buffers of CH chunks), the partial
+// tiles lie in LDS as they leave the matrix cores, and one wave a tile of 16 rows finishes it, four neighbouring features
+// a lane, behind the only barrier.  The sums of a tile have the order of fused_gemm_kernel's: the waves' runs of K, each
+// in order, then the waves in order.  One behind the other, the weights of 36 layers in turn (one MI355X): 4,096 x 1,024
+// (gate and up) and 1,024 x 2,048 into the stream 10.0 -> 8.5 us at one row, 10.9 -> 9.4 at 8, 11.9 -> 10.4 at 16, 14.0 -> 11.9
+// at 37, 16.6 -> 13.8 at 64; 4,120 x 1,024 with the conv step and 1,024 x 2,048 10.9 -> 9.0, 11.8 -> 9.9, 13.4 -> 11.0; of
+// 8 rows 8,728 x 3,072 17.5 -> 15.8, 3,072 x 4,608 8.2 -> 7.4.
+struct SkinnyParams {
+  const bf16_t* W;       // [N, K], or (TILED) in fragment order
+  const bf16_t* x;
+  int x_ld, M, N, chunks;
+  const float* ssq_in;   // row scale
+  int ssq_blocks, ssq_ld;
+  const int* slot_ids;
+  void* out;             // rows, or the residual stream (RESIDUAL, TANH: leading dimension N)
+  long out_ld;
+  const float* bias;
+  float out_scale, ssq_inverse_width, ssq_eps;
+  int out_f32, gate_act;
+  const float* res_w;
+  bf16_t* res_hb;
+  long res_hb_ld;
+  float* ssq_out;
+  const float* conv_w;
+  const float* conv_b;
+  bf16_t* conv_state;
+  int conv_lo, conv_hi;
+  const float *post_w, *post_b, *next_w, *next_b;
+  float post_alpha, next_alpha;
+  float act_limit, act_alpha, act_offset;
+};
+
+// the sum over the lanes 16, then 32 apart, in every lane, in the vector pipeline
+__device__ __forceinline__ float quarters_sum(float v) {
+  const auto rows = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned even = rows[0], odd = rows[1];
+  const float pair = __builtin_bit_cast(float, even) + __builtin_bit_cast(float, odd);
+  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, pair), __builtin_bit_cast(unsigned, pair), false, false);
+  const unsigned low = halves[0], high = halves[1];
+  return __builtin_bit_cast(float, low) + __builtin_bit_cast(float, high);
+}
+
+// v of the lane 32 further, in the lanes below 32
+__device__ __forceinline__ float upper_half(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned high = halves[1];
+  return __builtin_bit_cast(float, high);
+}
+
+// v * v, rounded before anything is added to it (fused_gemm_kernel's squares pass through LDS)
+__device__ __forceinline__ float square_rounded(float v) {
+#pragma clang fp contract(off)
+  return v * v;
+}
+
+// EPI_PLAIN ... EPI_TANH as above.  SQ: partial sums of squares a thread asks for early (0: no row scale).  TILED: W in
+// fragment order.  Row y of the grid takes the MT tiles of 16 rows from row 16 MT y on; with several of them a row of
+// the grid is a multiple of 8 workgroups, so that those of a tile of features run on one die and its weights leave memory once.
+template <int MT, int EPI, int WAVES, int CH, bool EXACT, int SQ, bool TILED>
+__global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
+  __shared__ floatx4 red[WAVES][MT][WAVE];
+  __shared__ float parts[SQ > 0 ? WAVES : 1][MT * 16];
+  const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int q = lane / 16, r = lane % 16;
+  // (a workgroup past the last tile, which fills up a row of the grid, does that tile's work again and stores nothing: a
+  // branch up here would have the arguments behind it fetched after the branch)
+  const int own = blockIdx.x, tile = min(own, (p.N - 1) / 16), row0 = blockIdx.y * (MT * 16);
+  const int last_row = p.M - 1 - row0;                          // of this workgroup's rows (the launch gives it at least one)
+  const int ssq_rows = p.ssq_ld - row0;
+  const int mine = WAVES > MT && wave >= MT ? MT - 1 : wave;    // the tile of rows that this wave finishes (or stands beside)
+  const int m = min(mine * 16 + r, last_row);                   // its row, from row0 on
+  const int n = tile * 16 + 4 * q, n_safe = min(n, p.N - 4);
+  int slot = 0;
+  if (EPI == EPI_CONV) slot = p.slot_ids[row0 + m];
+
+  // ---- the weights, then the rows: everything of a wave at once (EXACT), or the first two buffers
+  constexpr int BUFFERS = EXACT ? 1 : 2;
+  constexpr int STEP = TILED ? 512 : 32;
+  bf16x8_t a[BUFFERS][CH], b[BUFFERS][CH][MT];
+  const int chunks = EXACT ? WAVES * CH : p.chunks;
+  const int per_wave = EXACT ? CH : (chunks + WAVES - 1) / WAVES;
+  const int first = wave * per_wave;
+  const int count = EXACT ? CH : max(0, min(per_wave, chunks - first));
+  const bf16_t* w_at = TILED ? p.W + ((long)tile * chunks + first) * 512 + lane * 8
+                             : p.W + ((long)min(tile * 16 + r, p.N - 1) * chunks + first) * 32 + 8 * q;
+  const bf16_t* x_at[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) x_at[mt] = p.x + (long)(row0 + min(mt * 16 + r, last_row)) * p.x_ld + first * 32 + 8 * q;
+  // (no condition around a load: a chunk past the wave's run reads a valid one and is multiplied as zeros)
+  auto chunk_at = [&](int c) { return EXACT ? c : min(c, max(count, 1) - 1) - (count ? 0 : first); };
+  auto ask_weights = [&](int buffer, int c0) {
+#pragma unroll
+    for (int j = 0; j < CH; ++j) a[buffer][j] = *reinterpret_cast<const bf16x8_t*>(w_at + (long)chunk_at(c0 + j) * STEP);
+  };
+  auto ask_rows = [&](int buffer, int c0) {
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) b[buffer][j][mt] = *reinterpret_cast<const bf16x8_t*>(x_at[mt] + chunk_at(c0 + j) * 32);
+  };
+#pragma unroll
+  for (int buffer = 0; buffer < BUFFERS; ++buffer) ask_weights(buffer, buffer * CH);
+#pragma unroll
+  for (int buffer = 0; buffer < BUFFERS; ++buffer) ask_rows(buffer, buffer * CH);
+
+  // ---- what the last stage needs, behind them: sums of squares, the stream's elements, conv tails
+  constexpr int PARTS = WAVES * 4;
+  const int part = threadIdx.x / 16;
+  float sq[MT][SQ > 0 ? SQ : 1];
+  if (SQ > 0) {
+    const int last = p.ssq_blocks - 1;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      const float* at = p.ssq_in + row0 + min(mt * 16 + r, ssq_rows - 1);
+#pragma unroll
+      for (int i = 0; i < SQ; ++i) sq[mt][i] = at[(long)min(part + i * PARTS, last) * p.ssq_ld];
+    }
+  }
+  floatx4 h_old, res_w, post_w, post_b, next_w, next_b;
+  float* h_at = reinterpret_cast<float*>(p.out) + (long)(row0 + m) * p.N + n_safe;
+  if (EPI == EPI_RESIDUAL || EPI == EPI_TANH) h_old = *reinterpret_cast<const floatx4*>(h_at);
+  if (EPI == EPI_RESIDUAL) res_w = *reinterpret_cast<const floatx4*>(p.res_w + n_safe);
+  if (EPI == EPI_TANH) {
+    const float* following_w = p.res_hb ? p.next_w : p.post_w;          // without a next norm: valid and not used
+    const float* following_b = p.res_hb ? p.next_b : p.post_b;
+    post_w = *reinterpret_cast<const floatx4*>(p.post_w + n_safe);
+    post_b = *reinterpret_cast<const floatx4*>(p.post_b + n_safe);
+    next_w = *reinterpret_cast<const floatx4*>(following_w + n_safe);
+    next_b = *reinterpret_cast<const floatx4*>(following_b + n_safe);
+  }
+  bf16x4_t tail[3];
+  floatx4 taps[4], tap_bias = {0.f, 0.f, 0.f, 0.f};
+  const int channels = p.conv_hi - p.conv_lo;
+  bf16_t* tail_at = nullptr;
+  if (EPI == EPI_CONV && wave < MT) {          // four taps; four channels a lane
+    const int channel = min(max(n - p.conv_lo, 0), channels - 4);
+    tail_at = p.conv_state + (long)slot * 3 * channels + channel;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) tail[k] = *reinterpret_cast<const bf16x4_t*>(tail_at + (long)k * channels);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) taps[i] = *reinterpret_cast<const floatx4*>(p.conv_w + (long)(channel + i) * 4);
+    if (p.conv_b) tap_bias = *reinterpret_cast<const floatx4*>(p.conv_b + channel);
+  }
+
+  // the last stage's arguments now, while the weights are on their way; and no load moves behind the first products
+  asm volatile("" ::"s"(p.bias), "s"(p.out), "s"(p.out_ld), "s"(p.out_scale), "s"(p.out_f32));
+  if (EPI == EPI_SWIGLU) asm volatile("" ::"s"(p.gate_act));
+  if (EPI == EPI_RESIDUAL) asm volatile("" ::"s"(p.res_hb), "s"(p.res_hb_ld), "s"(p.ssq_out));
+  if (SQ > 0) asm volatile("" ::"s"(p.ssq_inverse_width), "s"(p.ssq_eps));
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- the products
+  floatx4 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int buffer, int c0, bool whole) {
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      floatx4 weights = *reinterpret_cast<const floatx4*>(&a[buffer][j]);
+      if (!whole) weights = c0 + j < count ? weights : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(&weights), b[buffer][j][mt], acc[mt], 0, 0, 0);
+    }
+  };
+  if (EXACT) {
+    multiply(0, 0, true);
+  } else {
+    int c = 0;
+    for (; c + 2 * CH < count; c += 2 * CH) {
+#pragma unroll
+      for (int buffer = 0; buffer < 2; ++buffer) {
+        multiply(buffer, c + buffer * CH, true);
+        ask_weights(buffer, c + (2 + buffer) * CH);
+        ask_rows(buffer, c + (2 + buffer) * CH);
+      }
+    }
+#pragma unroll
+    for (int buffer = 0; buffer < 2; ++buffer) multiply(buffer, c + buffer * CH, false);
+  }
+  if (SQ > 0) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < SQ; ++i) sum += part + i * PARTS < p.ssq_blocks ? sq[mt][i] : 0.f;
+      // wider rows than SQ sums a thread: the rest now
+      for (int block = part + SQ * PARTS; block < p.ssq_blocks; block += PARTS)
+        sum += p.ssq_in[(long)block * p.ssq_ld + row0 + min(mt * 16 + r, ssq_rows - 1)];
+      sum = quarters_sum(sum);
+      if (lane < 16) parts[wave][mt * 16 + lane] = sum;
+    }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) red[wave][mt][lane] = acc[mt];
+  __syncthreads();
+  if (wave >= MT) return;
+
+  // ---- lane (q, r): features n .. n + 3 of row m
+  floatx4 v = red[0][mine][lane];
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) v += red[w][mine][lane];
+  if (SQ > 0) {                                // the norm's division, on the float32 sums
+    float squares = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) squares += parts[w][mine * 16 + r];
+    const float mean = squares * p.ssq_inverse_width + p.ssq_eps;
+    float inverse = __builtin_amdgcn_rsqf(mean);
+    inverse = inverse * (1.5f - 0.5f * mean * inverse * inverse);         // (a step of Newton's: as close as 1 / sqrtf)
+    v *= inverse;
+  }
+  if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + n_safe);
+  const bool live = mine * 16 + r <= last_row && n < p.N && own == tile;
+  const long row = row0 + m;
+  if (EPI == EPI_RESIDUAL) {
+    floatx4 updated;
+    float square = 0.f;
+    if (live) {
+      bf16x4_t rows;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        updated[i] = h_old[i] + v[i];
+        rows[i] = (bf16_t)(updated[i] * res_w[i]);
+        square += square_rounded(updated[i]);
+      }
+      *reinterpret_cast<floatx4*>(h_at) = updated;
+      *reinterpret_cast<bf16x4_t*>(p.res_hb + row * p.res_hb_ld + n) = rows;
+    }
+    square = quarters_sum(square);
+    if (own == tile && lane < min(16, ssq_rows - mine * 16)) p.ssq_out[(long)tile * p.ssq_ld + row0 + mine * 16 + lane] = square;
+  } else if (EPI == EPI_TANH) {
+    if (!live) return;
+    floatx4 updated;
+    bf16x4_t rows;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      updated[i] = h_old[i] + tanh_norm_f(v[i], p.post_alpha, post_w[i], post_b[i]);
+      if (p.res_hb) rows[i] = (bf16_t)tanh_norm_f(updated[i], p.next_alpha, next_w[i], next_b[i]);
+    }
+    *reinterpret_cast<floatx4*>(h_at) = updated;
+    if (p.res_hb) *reinterpret_cast<bf16x4_t*>(p.res_hb + row * p.res_hb_ld + n) = rows;
+  } else if (EPI == EPI_SWIGLU) {
+    // a tile is 8 gate features, then the 8 up features of the same columns: lanes q = 0, 1 take theirs from q + 2
+    floatx4 up;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) up[i] = upper_half(v[i]);
+    if (q >= 2 || !live) return;
+    bf16x4_t packed;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)(silu_bf16_f(round_bf16(v[i])) * round_bf16(up[i]));
+    if (p.gate_act) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)gated_f(p, round_bf16(v[i]), round_bf16(up[i]));
+    }
+    *reinterpret_cast<bf16x4_t*>(reinterpret_cast<bf16_t*>(p.out) + row * p.out_ld + tile * 8 + 4 * q) = packed;
+  } else {
+    if (!live) return;
+    if (EPI == EPI_PLAIN && p.out_f32) {
+      *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(p.out) + row * p.out_ld + n) = v * p.out_scale;
+      return;
+    }
+    bf16x4_t packed;
+    if (EPI == EPI_CONV && n >= p.conv_lo && n < p.conv_hi) {
+      bf16x4_t sample;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sample[i] = (bf16_t)v[i];
+        float sum = tap_bias[i];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) sum += taps[i][k] * (float)tail[k][i];
+        sum += taps[i][3] * (float)sample[i];
+        packed[i] = (bf16_t)silu_bf16_f(sum);
+      }
+      *reinterpret_cast<bf16x4_t*>(tail_at) = tail[1];                    // the tail rolls by one
+      *reinterpret_cast<bf16x4_t*>(tail_at + channels) = tail[2];
+      *reinterpret_cast<bf16x4_t*>(tail_at + 2L * channels) = sample;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)(v[i] * p.out_scale);
+    }
+    *reinterpret_cast<bf16x4_t*>(reinterpret_cast<bf16_t*>(p.out) + row * p.out_ld + n) = packed;
+  }
+}
+
+// Whether skinny_kernel takes this product: whole pieces of four features wherever it moves them at once.
+static bool skinny_takes(const FusedGemmParams& p, int epi) {
+  auto aligned = [](const void* at, size_t bytes) { return ((uintptr_t)at & (bytes - 1)) == 0; };
+  if (p.w_tiled ? epi == EPI_TANH : p.ssq_in || epi == EPI_CONV || epi == EPI_RESIDUAL) return false;     // forms without an instance
+  if (p.N % 4 || p.x_ld > 0x7fffffffL || !aligned(p.W, 16) || !aligned(p.x, 16) || (p.bias && !aligned(p.bias, 16))) return false;
+  if (epi == EPI_RESIDUAL || epi == EPI_TANH) {
+    if (!aligned(p.res_h, 16) || (p.res_hb && (p.res_hb_ld % 4 || !aligned(p.res_hb, 8)))) return false;
+    if (epi == EPI_RESIDUAL) return aligned(p.res_w, 16);
+    return aligned(p.post_w, 16) && aligned(p.post_b, 16) && (!p.res_hb || (aligned(p.next_w, 16) && aligned(p.next_b, 16)));
+  }
+  if (p.out_ld % 4 || !aligned(p.out, p.out_f32 ? 16 : 8)) return false;
+  if (epi == EPI_CONV)
+    return p.conv_k == 4 && p.conv_lo % 4 == 0 && p.conv_hi % 4 == 0 && aligned(p.conv_state, 8) && aligned(p.conv_w, 16) &&
+           (!p.conv_b || aligned(p.conv_b, 16));
+  return true;
+}
+
+template <int MT, int EPI, int WAVES, int CH, bool EXACT>
+static void launch_skinny_scaled(const SkinnyParams& p, bool tiled, dim3 blocks, hipStream_t stream) {
+  if (!tiled) {
+    if constexpr (EPI == EPI_PLAIN || EPI == EPI_SWIGLU || EPI == EPI_TANH) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, false><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+    return;
+  }
+  if constexpr (EPI == EPI_TANH) return;
+  else if constexpr (EPI == EPI_RESIDUAL) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+  else {
+    if (!p.ssq_in) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+    else if (WAVES == 4 || p.ssq_blocks <= 4 * 4 * WAVES) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 4, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+    else if (p.ssq_blocks <= 6 * 4 * 8) skinny_kernel<MT, EPI, 8, CH, EXACT, 6, true><<<blocks, 8 * WAVE, 0, stream>>>(p);
+    else skinny_kernel<MT, EPI, 8, CH, EXACT, 12, true><<<blocks, 8 * WAVE, 0, stream>>>(p);
+  }
+}
+
+// All of a wave's run of K at once where that is a fixed number of chunks (K of 512 and 1,024 over four waves, 2,048 over
+// eight), else two buffers of a few chunks in turn: eight waves of a long K wait for each other's registers, not for
+// latency.  At 8 rows two buffers of 2 / 3 / 4 / 6 chunks take 15.5 / 15.8 / 19.5 / 20.5 us for 8,728 x 3,072 (all 12 chunks of
+// a wave at once 16.6), 29.6 / 29.1 / 38.4 / 40.0 for 24,576 x 3,072, 7.5 / 7.4 / 8.5 / 8.9 for 3,072 x 4,608.
+template <int MT, int EPI>
+static void launch_skinny_sized(const SkinnyParams& p, bool tiled, int waves, dim3 blocks, hipStream_t stream) {
+  if (waves == 4 && p.chunks == 32) launch_skinny_scaled<MT, EPI, 4, 8, true>(p, tiled, blocks, stream);
+  else if (waves == 8 && p.chunks == 64) launch_skinny_scaled<MT, EPI, 8, 8, true>(p, tiled, blocks, stream);
+  else if (MT == 1 && waves == 4 && p.chunks == 16) launch_skinny_scaled<1, EPI, 4, 4, true>(p, tiled, blocks, stream);
+  else if (waves == 4) launch_skinny_scaled<MT, EPI, 4, MT <= 2 ? 4 : 2, false>(p, tiled, blocks, stream);
+  else launch_skinny_scaled<MT, EPI, 8, MT == 1 ? 3 : 2, false>(p, tiled, blocks, stream);
+}
+
+template <int MT>
+static int launch_skinny(const FusedGemmParams& f, int epi, hipStream_t stream) {
+  SkinnyParams p = {};
+  p.W = f.W;
+  p.x = f.x;
+  p.x_ld = (int)f.x_ld;
+  p.M = f.M;
+  p.N = f.N;
+  p.chunks = f.K / 32;
+  p.ssq_in = f.ssq_in;
+  p.ssq_blocks = f.ssq_blocks;
+  p.ssq_ld = f.ssq_ld;
+  p.ssq_inverse_width = f.ssq_width > 0 ? 1.0f / (float)f.ssq_width : 0.f;
+  p.ssq_eps = f.ssq_eps;
+  p.out = epi == EPI_RESIDUAL || epi == EPI_TANH ? (void*)f.res_h : f.out;
+  p.out_ld = f.out_ld;
+  p.out_f32 = f.out_f32;
+  p.out_scale = f.out_scale;
+  p.bias = f.bias;
+  p.res_hb = f.res_hb;
+  p.res_hb_ld = f.res_hb_ld;
+  p.res_w = f.res_w;
+  p.ssq_out = f.ssq_out;
+  p.conv_w = f.conv_w;
+  p.conv_b = f.conv_b;
+  p.conv_state = f.conv_state;
+  p.slot_ids = f.slot_ids;
+  p.conv_lo = f.conv_lo;
+  p.conv_hi = f.conv_hi;
+  p.post_w = f.post_w;
+  p.post_b = f.post_b;
+  p.next_w = f.next_w;
+  p.next_b = f.next_b;
+  p.post_alpha = f.post_alpha;
+  p.next_alpha = f.next_alpha;
+  p.gate_act = f.gate_act;
+  p.act_limit = f.act_limit;
+  p.act_alpha = f.act_alpha;
+  p.act_offset = f.act_offset;
+  const int tiles = (p.N + 15) / 16;
+  const dim3 blocks(f.row_tiles > 1 ? (tiles + 7) / 8 * 8 : tiles, f.row_tiles);
+  const int waves = fused_gemm_waves(f.K);
+  const bool tiled = f.w_tiled;
+  if (epi == EPI_PLAIN) launch_skinny_sized<MT, EPI_PLAIN>(p, tiled, waves, blocks, stream);
+  else if (epi == EPI_SWIGLU) launch_skinny_sized<MT, EPI_SWIGLU>(p, tiled, waves, blocks, stream);
+  else if (epi == EPI_CONV) launch_skinny_sized<MT, EPI_CONV>(p, tiled, waves, blocks, stream);
+  else if (epi == EPI_RESIDUAL) launch_skinny_sized<MT, EPI_RESIDUAL>(p, tiled, waves, blocks, stream);
+  else if (epi == EPI_TANH) launch_skinny_sized<MT, EPI_TANH>(p, tiled, waves, blocks, stream);
+  else return ERR_BAD_ARGUMENT;
+  return 0;
+}
+
 // feature_tiles: how many tiles of 16 output features a workgroup owns (1, 2 or 4).  With one, the rows of x
 // cross the caches once per 16 features, which is what bounds a step of many rows; with more, fewer
 // workgroups (of four waves) each keep more weight fragments in flight.  Plain prologue only.
@@ -679,33 +1042,13 @@ static int launch_fused_gemm(const FusedGemmParams& p, int pro, int epi, hipStre
 #undef FG_WIDE
     return 0;
   }
-  const int feature_blocks = (p.N + 15) / 16;
-  const dim3 blocks(p.row_tiles > 1 ? (feature_blocks + 7) / 8 * 8 * p.row_tiles : feature_blocks, k_splits);
+  const dim3 blocks((p.N + 15) / 16, k_splits);
   const int waves = fused_gemm_waves(p.K / k_splits);
 #define FG_LAUNCH(PRO_, EPI_)                                                                      \
   do {                                                                                             \
     if (waves == 8) fused_gemm_kernel<MT, PRO_, EPI_, 8, 1><<<blocks, 8 * WAVE, lds, stream>>>(p); \
     else fused_gemm_kernel<MT, PRO_, EPI_, 4, 1><<<blocks, 4 * WAVE, lds, stream>>>(p);            \
   } while (0)
-#define FG_LAUNCH_ROWS(EPI_)                                                                                  \
-  do {                                                                                                        \
-    if (waves == 8) fused_gemm_kernel<MT, PRO_PLAIN, EPI_, 8, 1, true><<<blocks, 8 * WAVE, lds, stream>>>(p); \
-    else fused_gemm_kernel<MT, PRO_PLAIN, EPI_, 4, 1, true><<<blocks, 4 * WAVE, lds, stream>>>(p);            \
-  } while (0)
-  if (p.row_tiles > 1) {           // MT of 1 or 2: the tiles of a step of up to 64 rows over two workgroups or more
-    if (pro != PRO_PLAIN) return ERR_BAD_ARGUMENT;
-    if constexpr (MT <= 2) {
-      if (epi == EPI_RESIDUAL) FG_LAUNCH_ROWS(EPI_RESIDUAL);
-      else if (epi == EPI_TANH) FG_LAUNCH_ROWS(EPI_TANH);
-      else if (epi == EPI_PLAIN) FG_LAUNCH_ROWS(EPI_PLAIN);
-      else if (epi == EPI_SWIGLU) FG_LAUNCH_ROWS(EPI_SWIGLU);
-      else if (epi == EPI_CONV) FG_LAUNCH_ROWS(EPI_CONV);
-      else return ERR_BAD_ARGUMENT;
-      return 0;
-    } else {
-      return ERR_BAD_ARGUMENT;
-    }
-  }
   if (pro == PRO_MERGE && epi == EPI_PLAIN) FG_LAUNCH(PRO_MERGE, EPI_PLAIN);
   else if (pro == PRO_MERGE && epi == EPI_RESIDUAL) FG_LAUNCH(PRO_MERGE, EPI_RESIDUAL);
   else if (pro == PRO_PLAIN && epi == EPI_RESIDUAL) FG_LAUNCH(PRO_PLAIN, EPI_RESIDUAL);
@@ -718,7 +1061,6 @@ static int launch_fused_gemm(const FusedGemmParams& p, int pro, int epi, hipStre
   else if (pro == PRO_PLAIN && epi == EPI_CONV) FG_LAUNCH(PRO_PLAIN, EPI_CONV);
   else return ERR_BAD_ARGUMENT;
 #undef FG_LAUNCH
-#undef FG_LAUNCH_ROWS
   return 0;
 }
 
@@ -732,11 +1074,17 @@ static int launch_fused_gemm_rows(FusedGemmParams& p, int pro, int epi, hipStrea
   int MT = step_tiles;
   p.ssq_ld = 16 * step_tiles;
   p.row_tiles = 1;
-  if (row_tiles > 1) {
-    if (pro != PRO_PLAIN || feature_tiles != 1) return ERR_BAD_ARGUMENT;
+  if (row_tiles > 1 && (pro != PRO_PLAIN || feature_tiles != 1)) return ERR_BAD_ARGUMENT;
+  if (pro == PRO_PLAIN && feature_tiles == 1 && k_splits == 1 && skinny_takes(p, epi)) {
     MT = (step_tiles + row_tiles - 1) / row_tiles;
     p.row_tiles = (step_tiles + MT - 1) / MT;
+    if (MT == 1) return launch_skinny<1>(p, epi, stream);
+    if (MT == 2) return launch_skinny<2>(p, epi, stream);
+    if (MT == 3) return launch_skinny<3>(p, epi, stream);
+    if (MT == 4) return launch_skinny<4>(p, epi, stream);
+    return ERR_UNSUPPORTED_SIZE;
   }
+  // (features that are no whole pieces of four: every workgroup takes all rows, the same sums)
   if (MT == 1) return launch_fused_gemm<1>(p, pro, epi, stream, k_splits, feature_tiles);
   if (MT == 2) return launch_fused_gemm<2>(p, pro, epi, stream, k_splits, feature_tiles);
   if (MT == 3) return launch_fused_gemm<3>(p, pro, epi, stream, k_splits, feature_tiles);

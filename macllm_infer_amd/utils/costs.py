@@ -216,7 +216,8 @@ def total(costs: Dict[str, Cost]) -> Cost:
 
 # Which kernels do the work of which group (name patterns of this package's kernels and of the BLAS library's).
 # fused_gemm_kernel<row tiles, prologue (0 norm, 1 plain, 2 merge of the attention runs), epilogue (0 plain,
-# 1 SiLU(g)*u, 2 conv, 3 add to the residual stream, 4 the same through tanh norms), ...>; shared_rows_gemm_kernel<row tiles, feature tiles a
+# 1 SiLU(g)*u, 2 conv, 3 add to the residual stream, 4 the same through tanh norms), ...>; skinny_kernel<row
+# tiles, epilogue, ...>; shared_rows_gemm_kernel<row tiles, feature tiles a
 # wave, epilogue (0 float32 slabs, 1 SiLU(g)*u, 2 conv or plain rows)>.  A product with the plain epilogue that is
 # launched once a step is the output head; launched more often, an output or down projection (the library's
 # products carry no such mark and stay with the other kernels).
@@ -224,14 +225,14 @@ DECODE_GROUPS: List[Tuple[str, str]] = [
     (r"mixer_decode_kernel|mixer_merge_kernel|decode_attention_kernel|decode_merge_kernel|ssm_scan_kernel|conv_step_kernel|"
      r"gate_norm_kernel|rope_kv_store_kernel|paged_attention_kernel|paged_attention_tile_kernel|"
      r"paged_attention_merge_kernel|linear_state_|head_norm_gate_|wide_norm_gate_kernel|tanh_rows_kernel|latent_|rotate_heads_kernel|attention_prepare_kernel", "mixers"),
-    (r"fused_gemm_kernel<\d+, \d+, 2|shared_rows_gemm_kernel<\d+, \d+, 2", "input projections"),
+    (r"fused_gemm_kernel<\d+, \d+, 2|skinny_kernel<\d+, 2|shared_rows_gemm_kernel<\d+, \d+, 2", "input projections"),
     (r"moe_expert_gemm_kernel<[^>]*(?:true|false), false|moe_expert_gemm_kernelI\w*Lb[01]ELb0E|moe_combine",
      "output projections + down projections"),                   # (the experts' down products: not gated)
-    (r"fused_gemm_kernel<\d+, \d+, 1|shared_rows_gemm_kernel<\d+, \d+, 1|moe_|clamped_glu_kernel", "gate and up projections"),
-    (r"fused_gemm_kernel<\d+, \d+, [34]|fused_gemm_kernel<\d+, 2, 0|shared_rows_gemm_kernel<\d+, \d+, 0|fused_gemm_split_kernel",
+    (r"fused_gemm_kernel<\d+, \d+, 1|skinny_kernel<\d+, 1|shared_rows_gemm_kernel<\d+, \d+, 1|moe_|clamped_glu_kernel", "gate and up projections"),
+    (r"fused_gemm_kernel<\d+, \d+, [34]|skinny_kernel<\d+, [34]|fused_gemm_kernel<\d+, 2, 0|shared_rows_gemm_kernel<\d+, \d+, 0|fused_gemm_split_kernel",
      "output projections + down projections"),
 ]
-PLAIN_PRODUCT = r"fused_gemm_kernel<\d+, [01], 0"
+PLAIN_PRODUCT = r"fused_gemm_kernel<\d+, [01], 0|skinny_kernel<\d+, 0"
 # (of lanes of one chunk, up to 128 tokens, the scan's two launches hold the attention too)
 PREFILL_GROUPS: List[Tuple[str, str]] = [
     (r"^Cijk_|gemm_f32_kernel|tiled_f32_kernel|head_gemm_kernel|moe_expert_gemm", "matrix products"),

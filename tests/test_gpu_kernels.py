@@ -1152,6 +1152,57 @@ def test_a_product_that_joins_the_residual_stream_and_the_product_behind_the_nex
                 close(got, want, torch.bfloat16, 16.0)
 
 
+@pytest.mark.parametrize("M, N, K, blocks", [(1, 48, 512, 1), (8, 4120, 1024, 64), (5, 100, 96, 6), (16, 52, 2048, 130), (17, 136, 3104, 192),
+                                             (40, 264, 1024, 250), (33, 36, 4608, 400), (64, 72, 2048, 128)])
+def test_skinny_products_of_weights_in_fragment_order(ops, M, N, K, blocks):
+    """Weights in fragment order go through the kernel whose runs of K are fixed at compile time or taken in two buffers
+    (K of 512, 1,024 and 2,048; others, also with fewer chunks than waves), its last tile partly past the end, its rows in
+    tiles that the step does not fill, rows dealt out with tiles that are no multiple of 8.  Into the stream: the bits of the
+    row-major weight, whose waves add up in the same order.  Behind a row scale of few and of many partial sums: plain rows,
+    SiLU(g) * u and the conv step with its tails against the plain versions; sums of K products of order 0.1 in
+    float32, then one rounding to bfloat16, as for the other products of this file."""
+    x, W, b = rand(M, K, seed=360, dtype=torch.bfloat16), rand(N, K, seed=361, scale=0.1, dtype=torch.bfloat16), rand(N, seed=362)
+    weight, fragments = W.to(DEV), ops.fragment_order(W.to(DEV))
+    h, next_w = rand(M, N, seed=363, scale=2.0), rand(N, seed=364, scale=0.1) + 1.0
+    ssq = torch.zeros(blocks, 16 * (-(-M // 16)))
+    ssq[:, :M] = rand(blocks, M, seed=365).abs() * 16.0 + 1.0
+    scale, on_gpu = ops.RowScale(ssq, 16 * blocks, 1e-5), ops.RowScale(ssq.to(DEV), 16 * blocks, 1e-5)
+    first = None
+    for operand, row_tiles in ((None, 1), (fragments, 1), (fragments, 2), (fragments, 3), (fragments, 4)):
+        got_h, got_hb = h.clone().to(DEV), torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        got_ssq = ops.residual_workspace(M, N, DEV)
+        ops.fused_gemm_residual(weight, b.to(DEV), x.to(DEV), got_h, got_hb, next_w.to(DEV), got_ssq, operand, row_tiles=row_tiles)
+        first = first or (got_h, got_hb, got_ssq[:, :M])
+        assert all(torch.equal(one, other) for one, other in zip(first, (got_h, got_hb, got_ssq[:, :M])))
+    for row_tiles in (1, 2, 4):
+        for dtype, out_scale in ((torch.bfloat16, 1.0), (torch.float32, 0.6)):
+            want, got = torch.empty(M, N, dtype=dtype), torch.full((M + 1, N), float("nan"), dtype=dtype, device=DEV)
+            ref_ops.fused_gemm(W, b, want, x=x, row_scale=scale, out_scale=out_scale)
+            ops.fused_gemm(weight, b.to(DEV), got[:M], x=x.to(DEV), row_scale=on_gpu, out_scale=out_scale, fragments=fragments, row_tiles=row_tiles)
+            assert torch.isnan(got[M].float()).all()
+            close(got[:M], want, dtype, 6.0 if dtype == torch.bfloat16 else 200.0)
+        if N % 16 == 0:
+            want, got = torch.empty(M, N // 2, dtype=torch.bfloat16), torch.full((M + 1, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+            ref_ops.fused_gemm(W, b, want, x=x, row_scale=scale, epilogue=ref_ops.EPI_SWIGLU)
+            ops.fused_gemm(weight, b.to(DEV), got[:M], x=x.to(DEV), row_scale=on_gpu, epilogue=ops.EPI_SWIGLU, fragments=fragments, row_tiles=row_tiles)
+            assert torch.isnan(got[M].float()).all()
+            close(got[:M], want, torch.bfloat16, 16.0)
+        lo, hi = 12, N - 8                          # (four channels a lane: the columns of a conv begin and end at fours)
+        state = rand(M + 2, 3, hi - lo, seed=366, dtype=torch.bfloat16)
+        slot_ids = torch.randperm(M + 2, generator=torch.Generator().manual_seed(M))[:M].to(torch.int32)
+        conv = dict(lo=lo, hi=hi, taps=4, weight=rand(hi - lo, 4, seed=367, scale=0.5), bias=rand(hi - lo, seed=368, scale=0.1))
+        want, want_state, got_state = torch.empty(M, N, dtype=torch.bfloat16), state.clone(), state.clone().to(DEV)
+        ref_ops.fused_gemm(W, b, want, x=x, row_scale=scale, epilogue=ref_ops.EPI_CONV, conv=dict(conv, state=want_state, slot_ids=slot_ids))
+        got = torch.full((M + 1, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.fused_gemm(weight, b.to(DEV), got[:M], x=x.to(DEV), row_scale=on_gpu, epilogue=ops.EPI_CONV, fragments=fragments, row_tiles=row_tiles,
+                       conv=dict(conv, weight=conv["weight"].to(DEV), bias=conv["bias"].to(DEV), state=got_state, slot_ids=slot_ids.to(DEV)))
+        assert torch.isnan(got[M].float()).all()
+        close(got[:M], want, torch.bfloat16, 8.0)
+        close(got_state, want_state, torch.bfloat16, 8.0)
+        unused = [slot for slot in range(M + 2) if slot not in slot_ids.tolist()]
+        assert torch.equal(got_state[unused].cpu(), state[unused])
+
+
 @pytest.mark.parametrize("M, N, K, S", [(64, 1024, 2048, 8), (33, 100, 2048, 16), (17, 48, 96, 3), (64, 136, 3072, 5),
                                         (5, 64, 64, 1)])
 def test_fused_gemm_split_over_k_and_the_norm_that_adds_its_slabs(ops, M, N, K, S):
