@@ -1692,7 +1692,13 @@ struct MixerParams {
   int splits;
   int split_keys;
   float* partial;
+  int* arrived;           // [M, Hkv] zeros, which the launch leaves zero again: the runs are merged inside it; or null
 };
+
+// A word that another workgroup's cache must see, or may have written, without the fences that would write back and drop
+// all of a die's cache: stored through to where the dies meet, and read from there.
+__device__ __forceinline__ void store_through(float* at, float v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float load_through(const float* at) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // one dim of a rotated head: pairs (j, j + rotary_dim/2) of the first rotary_dim dims;
 // cs holds cos (first half) and sin (second half) of the token's angles, rotary_dim/2 each
@@ -1705,18 +1711,55 @@ __device__ __forceinline__ float rotated_dim(const bf16_t* head, int dim, int ro
   return dim < half ? x * c - (float)head[dim + half] * s : x * c + (float)head[dim - half] * s;
 }
 
+// sum_s exp(m_s - m) o_s / sum_s exp(m_s - m) l_s of one dim of a head over its runs that hold keys, the first count() of
+// `most`, in ascending order.  MERGE_AT_ONCE are asked for at once, the first of them before it is known how many hold keys
+// (what a run without keys left in its place is read and not used).
+template <typename Load, typename Count>
+__device__ __forceinline__ float merged_runs(const float* runs, int dh, int dim, int most, Load load, Count count) {
+  float maximum = -INFINITY, denominator = 0.f, sum = 0.f;
+  int used = most;
+  for (int s0 = 0; s0 < used; s0 += MERGE_AT_ONCE) {
+    float m_s[MERGE_AT_ONCE], l_s[MERGE_AT_ONCE], o_s[MERGE_AT_ONCE];
+#pragma unroll
+    for (int j = 0; j < MERGE_AT_ONCE; ++j) {
+      const float* run = runs + (long)min(s0 + j, most - 1) * (dh + 2);
+      m_s[j] = load(run);
+      l_s[j] = load(run + 1);
+      o_s[j] = load(run + 2 + dim);
+    }
+    if (s0 == 0) used = count();
+#pragma unroll
+    for (int j = 0; j < MERGE_AT_ONCE; ++j) {
+      if (s0 + j < used) {
+        const float larger = fmaxf(maximum, m_s[j]);
+        const float keep = __builtin_amdgcn_exp2f(maximum - larger);        // 0 the first time (maximum = -inf); units of log2
+        const float weight = __builtin_amdgcn_exp2f(m_s[j] - larger);
+        denominator = denominator * keep + weight * l_s[j];
+        sum = sum * keep + weight * o_s[j];
+        maximum = larger;
+      }
+    }
+  }
+  return sum / denominator;
+}
+
 // Latency matters more than bandwidth here (a request's K and V for one layer are about a
 // megabyte): what a workgroup does is a chain of dependent memory round trips, so the context is
 // cut into runs of split_keys keys, one workgroup per (token, kv head, run), each wave of which
 // asks for all its keys at once (64 keys: two steps of attn_mfma.h in flight, the query heads of
 // the kv head as the columns).  The waves merge through LDS and the workgroup leaves (maximum,
-// normalizer, sums) per head; a small kernel merges the runs (a merge inside this kernel would
-// need a device-wide fence, which costs more than the whole read).  The new token's rotated key
+// normalizer, sums) per head, which are merged behind the last of them.  The new token's rotated key
 // and its value are written to their cache cell by the workgroup whose run holds it, before it
 // reads, so the run reads them like any other key.
+//
+// The runs of a token's kv head are merged by the workgroup that finishes its run last, which `arrived` tells (a launch of
+// mixer_merge_kernel behind this one takes 4.7 us, the merge in the output product's prologue 3; here the counter and the
+// read of the runs take about 2 in the workgroups that the launch has anyway, beside the scan's).  The partial results are
+// stored through the die's cache, every wave waits for its stores, then the workgroup counts itself; whoever counts last
+// sees all of them with loads that pass the cache, and puts the counter back.  Nobody waits for another workgroup.
 template <int DH>
 __device__ void mixer_attention_block(const MixerParams& p, int block, int* pages_lds, float* cs,
-                                      float* merge_lds) {
+                                      float* merge_lds, int* last_lds) {
   const int G = p.Hq / p.Hkv;
   const int split = block % p.splits;
   const int kvh = (block / p.splits) % p.Hkv;
@@ -1879,58 +1922,51 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
       denominator += weight * theirs[1];
       sum += weight * theirs[2 + dim];
     }
-    if (p.splits == 1) {             // the only workgroup of this token and kv head: nothing is left to merge
+    if (p.splits == 1 || (p.arrived && runs == 1)) {  // the only workgroup of this token and kv head: nothing is left to merge
       p.attn_out[token * p.out_ld + (long)(kvh * G + g) * DH + dim] = (bf16_t)(sum / denominator);
       continue;
     }
     float* mine = p.partial + ((token * p.Hq + kvh * G + g) * p.splits + split) * (long)(DH + 2);
     if (dim == 0) {
-      mine[0] = maximum;
-      mine[1] = denominator;
+      store_through(mine, maximum);
+      store_through(mine + 1, denominator);
     }
-    mine[2 + dim] = sum;
+    store_through(mine + 2 + dim, sum);
+  }
+  if (!p.arrived || p.splits == 1 || runs == 1) return;
+  const int used = min(runs, p.splits);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                     // this wave's partial results have arrived
+  __syncthreads();
+  if (tid == 0) {
+    int* counter = p.arrived + token * p.Hkv + kvh;
+    const int before = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last_lds = before == used - 1;
+    if (before == used - 1) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*last_lds) return;
+  for (int index = tid; index < G * DH; index += MX_THREADS) {
+    const int g = index / DH;
+    const int dim = index - g * DH;
+    const float* all = p.partial + (token * p.Hq + kvh * G + g) * p.splits * (long)(DH + 2);
+    p.attn_out[token * p.out_ld + (long)(kvh * G + g) * DH + dim] = (bf16_t)merged_runs(all, DH, dim, used, [](const float* at) { return load_through(at); }, [&]() { return used; });
   }
 }
 
-// out[token, head, :] = sum_s exp(m_s - m) o_s / sum_s exp(m_s - m) l_s over the runs that hold keys.
-// Eight runs are asked for at once, before it is known how many hold keys (the position is on
-// its way too); what a run without keys left in its place is read and not used.
+// out[token, head, :] of the runs left in p.partial, in a launch of its own (a caller without counters).
 __global__ void mixer_merge_kernel(MixerParams p, int dh) {
   const long token = blockIdx.x;
   const int head = blockIdx.y;
   const int dim = min((int)threadIdx.x, dh - 1);
   const float* runs = p.partial + (token * p.Hq + head) * p.splits * (long)(dh + 2);
   const int pos = p.positions[token];
-  float maximum = -INFINITY, denominator = 0.f, sum = 0.f;
-  int used = p.splits;
-  for (int s0 = 0; s0 < used; s0 += MERGE_AT_ONCE) {
-    float m_s[MERGE_AT_ONCE], l_s[MERGE_AT_ONCE], o_s[MERGE_AT_ONCE];
-#pragma unroll
-    for (int j = 0; j < MERGE_AT_ONCE; ++j) {
-      const float* run = runs + (long)min(s0 + j, p.splits - 1) * (dh + 2);
-      m_s[j] = run[0];
-      l_s[j] = run[1];
-      o_s[j] = run[2 + dim];
-    }
-    if (s0 == 0) {
-      int first_key = 0;
-      if (p.window > 0 && pos - p.window + 1 > 0) first_key = pos - p.window + 1;
-      const int base_key = (first_key / p.page_size) * p.page_size;
-      used = min(p.splits, (pos - base_key) / p.split_keys + 1);
-    }
-#pragma unroll
-    for (int j = 0; j < MERGE_AT_ONCE; ++j) {
-      if (s0 + j < used) {
-        const float larger = fmaxf(maximum, m_s[j]);
-        const float keep = __builtin_amdgcn_exp2f(maximum - larger);        // 0 the first time (maximum = -inf); units of log2
-        const float weight = __builtin_amdgcn_exp2f(m_s[j] - larger);
-        denominator = denominator * keep + weight * l_s[j];
-        sum = sum * keep + weight * o_s[j];
-        maximum = larger;
-      }
-    }
-  }
-  if ((int)threadIdx.x < dh) p.attn_out[token * p.out_ld + (long)head * dh + dim] = (bf16_t)(sum / denominator);
+  const float merged = merged_runs(runs, dh, dim, p.splits, [](const float* at) { return *at; }, [&]() {
+    int first_key = 0;
+    if (p.window > 0 && pos - p.window + 1 > 0) first_key = pos - p.window + 1;
+    const int base_key = (first_key / p.page_size) * p.page_size;
+    return min(p.splits, (pos - base_key) / p.split_keys + 1);
+  });
+  if ((int)threadIdx.x < dh) p.attn_out[token * p.out_ld + (long)head * dh + dim] = (bf16_t)merged;
 }
 
 // One step of the selective scan for (token, head, tile of state rows); see ssm_scan_kernel.
@@ -2030,8 +2066,9 @@ __global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p)
   __shared__ int pages_lds[MX_MAX_PAGES];
   __shared__ float cs[DH];
   __shared__ float merge_lds[MX_WAVES * 8 * (DH + 2)];
+  __shared__ int last_lds;
   if ((int)blockIdx.x < p.attention_blocks)
-    mixer_attention_block<DH>(p, blockIdx.x, pages_lds, cs, merge_lds);
+    mixer_attention_block<DH>(p, blockIdx.x, pages_lds, cs, merge_lds, &last_lds);
   else if (!p.vector_scan)
     mixer_ssm_block<false, 1>(p, blockIdx.x - p.attention_blocks);
   else if (p.rows_per_thread == 1)
@@ -2091,7 +2128,9 @@ extern "C" int mi_mixer_runs(int M, int Hkv, int dh, int page_size, long span, i
 
 // merge = 0: the attended heads are not written; `partial` is left for mi_fused_gemm_merge.  (When a token and
 // kv head have one workgroup, mi_mixer_runs says runs = 1, there is nothing to merge: that workgroup writes the
-// attended heads itself, whatever `merge` says, and no merge kernel is launched.)
+// attended heads itself, whatever `merge` says, and no merge kernel is launched.)  arrived (with merge; or null: a merge
+// kernel is launched): [M, Hkv] int32 zeros, by which the runs are merged inside the launch; zeros again behind it, so that
+// the launches of a step share them one after the other.
 extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv, int dh, int q_col, int k_col,
                                int v_col, const float* inv_freq, int rotary_dim, void* k_base, void* v_base,
                                long page_stride, int page_size, const int* block_tables, int max_pages,
@@ -2099,7 +2138,7 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
                                int max_seq_len, int H, int P, int N, int G, int z_col, int x_col, int dt_col, const float* dt_bias,
                                const float* A, const float* D, float* ssm_state, const int* slot_ids,
                                void* attn_out, void* ssm_out, float* ssm_y, long out_ld, float* partial,
-                               long partial_floats, int merge, hipStream_t stream) {
+                               long partial_floats, int merge, int* arrived, hipStream_t stream) {
   if (M <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || H <= 0 || P <= 0 || N <= 0 || G <= 0 || H % G != 0)
     return ERR_BAD_ARGUMENT;
   const int group = Hq / Hkv;
@@ -2175,13 +2214,14 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
   if ((long)Hkv * M * p.splits > 0x3fffffffL || M > 65535 || Hq > 65535) return ERR_UNSUPPORTED_SIZE;
   if (!partial || partial_floats < (long)M * Hq * p.splits * (dh + 2)) return ERR_BAD_ARGUMENT;
   p.partial = partial;
+  p.arrived = merge ? arrived : nullptr;
   p.attention_blocks = Hkv * M * p.splits;
   const long total = (long)p.attention_blocks + (long)p.p_tiles * H * M;
   if (total > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
   if (dh == 64) mixer_decode_kernel<64><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
   else mixer_decode_kernel<128><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
   RETURN_IF_LAUNCH_FAILED();
-  if (!merge || p.splits == 1) return 0;
+  if (!merge || p.splits == 1 || p.arrived) return 0;
   const dim3 merge_grid(M, Hq);
   mixer_merge_kernel<<<merge_grid, dh, 0, stream>>>(p, dh);
   RETURN_IF_LAUNCH_FAILED();

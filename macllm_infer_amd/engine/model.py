@@ -153,10 +153,11 @@ class DecoderModel:
         self.query_tile = max((getattr(mixer, "query_tile", 0) for mixer in mixers), default=0)
         # and its tables of chunks for the chunk sizes the mixers name
         self.chunk_sizes = tuple(sorted({getattr(mixer, "chunk_tokens", 0) for mixer in mixers} - {0}))
-        # and the tables the mixers declare themselves; one name is one table, whichever layers read it
+        # and the tables the mixers and the layers' fusions declare themselves; one name is one table, whichever layers read it
         declared = {}
-        for mixer in mixers:
-            for table in (mixer.step_tables() if hasattr(mixer, "step_tables") else ()):
+        fusions = [getattr(block, "fusion", None) for block in self.blocks]
+        for part in mixers + fusions:
+            for table in (part.step_tables() if hasattr(part, "step_tables") else ()):
                 declared.setdefault(table.name, table)
         self.step_tables = tuple(declared.values())
 

@@ -202,7 +202,7 @@ _SIGNATURES = {
                             _c_ptr, _c_ptr, _c_long, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int,
                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                             _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long,
-                            _c_int, _c_ptr],
+                            _c_int, _c_ptr, _c_ptr],
     },
     "microbench": {
         "mi_stream_read": [_c_ptr, _c_long, _c_ptr, _c_int, _c_ptr],
@@ -2453,9 +2453,6 @@ def mixer_decode_supported(num_heads: int, num_kv_heads: int, head_dim: int, pag
             and state_size <= 512 and rotary_dim % 16 == 0)
 
 
-MERGE_AT_ONCE = 8          # runs of keys a merge asks for at once (decode.hip)
-
-
 def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: int):
     """(keys of a run, runs per token and kv head) as ``mixer_decode`` cuts the contexts of a step of M tokens
     whose requests hold up to ``span`` keys, for heads of ``head_dim``."""
@@ -2472,14 +2469,17 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
                  ssm_heads: int, ssm_head_dim: int, state_size: int, num_groups: int,
                  z_col: int, x_col: int, dt_col: int, dt_bias: torch.Tensor, A: torch.Tensor, D: torch.Tensor,
                  ssm_state: torch.Tensor, slot_ids: torch.Tensor, out: torch.Tensor,
-                 ssm_y: Optional[torch.Tensor], merge: bool = True) -> Optional[AttentionRuns]:
+                 ssm_y: Optional[torch.Tensor], merge: bool = True,
+                 arrived: Optional[torch.Tensor] = None) -> Optional[AttentionRuns]:
     """Both mixers of a decode step in one launch.  ``u`` [M, >=cols] holds each token's projected
     row (q, k, v unrotated; x, B, C after the conv).  Attention: rotates q and the new key, writes
     the new K/V into the cache cell ``slot_mapping``, attends over the request's pages, writes
     ``out[:, :Hq*dh]``.  State space: one scan step from and into ``ssm_state[slot_ids]``, writes
     ``y * SiLU(z)`` to ``out[:, Hq*dh:]``, or float32 ``y`` to ``ssm_y`` when a grouped norm
     follows.  ``max_seq_len``: an upper bound of the longest context in the batch.  With ``merge=False``
-    ``out[:, :Hq*dh]`` is not written: the runs of keys are returned unmerged, for ``fused_gemm_merge``."""
+    ``out[:, :Hq*dh]`` is not written: the runs of keys are returned unmerged, for ``fused_gemm_merge``.
+    ``arrived``: int32 zeros, one a token and kv head, which are zeros again behind the call: the runs are merged
+    inside the launch by whichever workgroup ends last (without them by a launch of their own, the same bits)."""
     u_ld = _row_major(u, "u")
     out_ld = _row_major(out, "out")
     M = u.shape[0]
@@ -2503,6 +2503,9 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
     widest = max(q_col + num_heads * head_dim, k_col + num_kv_heads * head_dim, v_col + num_kv_heads * head_dim,
                  z_col + E, x_col + E + 2 * num_groups * state_size, dt_col + ssm_heads)
     _need(u.shape[1] >= widest, "mixer_decode: u is too narrow")
+    if arrived is not None:
+        _i32(arrived, "arrived")
+        _need(arrived.numel() >= M * num_kv_heads, "mixer_decode: one counter per token and kv head")
     span = max(1, int(max_seq_len)) if not window else window + page_size
     run_keys, runs = mixer_runs(M, num_kv_heads, page_size, span, head_dim)        # the launcher's own rule
     partial = torch.empty((M * num_heads * runs * (head_dim + 2),), dtype=torch.float32, device=u.device)
@@ -2512,7 +2515,7 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
         _p(slot_mapping), float(scale), int(window or 0), int(max_seq_len), ssm_heads, ssm_head_dim, state_size,
         num_groups, z_col, x_col, dt_col, _p(dt_bias), _p(A), _p(D), _p(ssm_state), _p(slot_ids), _p(out),
         out.data_ptr() + 2 * num_heads * head_dim,
-        _p(ssm_y), out_ld, _p(partial), partial.numel(), int(merge), _stream()), "mixer_decode")
+        _p(ssm_y), out_ld, _p(partial), partial.numel(), int(merge), _p(arrived), _stream()), "mixer_decode")
     if merge or runs == 1:                  # one workgroup per token and kv head has written the heads itself
         return None
     return AttentionRuns(partial, positions, num_heads, head_dim, runs, run_keys, page_size, int(window or 0))

@@ -46,6 +46,7 @@ from typing import Dict, Optional
 
 import torch
 
+from ..engine.context import StepTable
 from ..kernels import ops
 from .base import Residual, ScaledRows
 from .block import overlap_pays, register_fusion, side_stream
@@ -111,14 +112,12 @@ PAD_FEATURES = 256
 PAD_ROWS = (256, 512, 1024, 2048, 4096)
 PAD_MARGIN = 0.95
 FORCE_PADDING: Optional[bool] = None      # tests: True or False instead of the clock
-# The attended heads of a decode step come in runs of keys that a small kernel merges; the output projection
-# can merge them in its prologue instead, every workgroup of it again: one launch less, but the projection then
-# starts behind a read of the runs.  It pays while a workgroup reads few of them (0.5B-shaped at 2,048-token
-# contexts: 1.33 -> 1.26 ms a step at 1 row, 1.39 -> 1.37 at 4, even at 6 to 8, slower from 16; 7B-shaped: faster
-# at 1 and 2 rows, slower at 4): up to MERGE_LATER_BYTES of runs a workgroup.
-MERGE_LATER_ROWS = 16
-MERGE_LATER_BYTES = 96 << 10
-FORCE_MERGE_LATER: Optional[bool] = None  # tests: True or False instead of the rule
+# The attended heads of a decode step come in runs of keys, which the mixers' launch merges itself by the counters of the
+# step (``AttentionMamba2Step.step_tables``).  The output projection can merge them in its prologue instead, every workgroup
+# of it again, and starts behind a read of the runs: the 0.5B shape at 1 row 1,032 us a step with the counters, 1,081 that way
+#,
+# at 8 rows 1,198 with the counters and 1,252 with the merge as a launch of its own.  No step takes that way by itself.
+FORCE_MERGE_LATER: Optional[bool] = None  # True: the output projection merges, where it takes the step
 _padding_wins: Dict[tuple, tuple] = {}
 # A projection whose result joins the residual stream can add it there itself (float32, in place) and leave, beside
 # the stream, its rows times the next norm's weight in bfloat16 with the partial sums of their squares; the product
@@ -339,9 +338,9 @@ def register_mixer_kernel(*kinds: str):
     this order: a kernel that runs all of them in one launch in steps of single tokens.  The kernel object
     offers ``conv`` (None, or the columns of the input projection that go through a conv step in that
     product's epilogue: {lo, hi, taps, weight, bias}), ``supported(step, caches)``,
-    ``conv_state(caches)`` and ``run(u, step, caches, mixed, merge=True)``; a kernel with ``merge_later_bytes(step,
-    caches)`` returns, when called with ``merge=False``, the runs of keys of its attended heads (the first columns of
-    ``mixed``) unmerged, as ``ops.AttentionRuns``, for the output projection to merge."""
+    ``conv_state(caches)`` and ``run(u, step, caches, mixed, merge=True)``; a kernel with ``merged_columns`` (how
+    many the attended heads are, the first columns of ``mixed``) returns, when called with ``merge=False``, their runs of
+    keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; ``step_tables()``: tables it reads in every step."""
     def decorate(factory):
         _MIXER_KERNELS[tuple(kinds)] = factory
         return factory
@@ -550,6 +549,10 @@ class LayerFusion:
         for name, value in beyond.items():
             if hasattr(self, name):
                 setattr(self, name, getattr(self, name) + (value,))
+
+    def step_tables(self):
+        """Index tables of the kernel for the layer's mixers in every step."""
+        return self.kernel.step_tables() if hasattr(self.kernel, "step_tables") else []
 
     def _row_tiles(self, weight: torch.Tensor) -> tuple:
         """The fixed rule for a projection into the stream: one tile of 16 rows a workgroup where it has few output
@@ -900,16 +903,9 @@ class LayerFusion:
 
     def _merges_later(self, kernel, step, caches) -> bool:
         """Whether the output projection merges the runs of keys of this step's attended heads itself."""
-        estimate = getattr(kernel, "merge_later_bytes", None)
-        rows = step.num_tokens
-        if estimate is None or rows > MERGE_LATER_ROWS or FORCE_MERGE_LATER is False:
-            return False
-        merged = estimate(step, caches)                  # (merged columns, bytes of runs one workgroup reads)
-        if merged is None or not ops.fused_gemm_merge_supported(rows, self.w_out.shape[1], 1, merged[0]):
-            return False
-        if FORCE_MERGE_LATER:
-            return True
-        return merged[1] <= MERGE_LATER_BYTES
+        merged_columns = getattr(kernel, "merged_columns", None)
+        return bool(FORCE_MERGE_LATER and merged_columns is not None
+                    and ops.fused_gemm_merge_supported(step.num_tokens, self.w_out.shape[1], 1, merged_columns))
 
     def _to_the_stream(self, x: torch.Tensor, weight: torch.Tensor, bias, library: bool, slabs: int, tiles: int,
                        fragments, attended=None) -> list:
@@ -977,10 +973,16 @@ class AttentionMamba2Step:
         self.z_col = second
         self.x_col = second + s.inner_size
         self.dt_col = self.x_col + s.conv_width
-        self.attended_width = q_width
+        self.attended_width = self.merged_columns = q_width
         self.inv_freq, self.rotary_dim = self.attention.position.fused_rotation()
         self.conv = dict(lo=self.x_col, hi=self.dt_col, taps=s.conv_kernel, weight=self.mamba.conv_weight,
                          bias=self.mamba.conv_bias)
+
+    def step_tables(self):
+        # zeros, uploaded with every step: by these the launch knows which workgroup merges a token's runs of keys (the
+        # launches of the step's layers use them one after the other and leave zeros)
+        heads = self.attention.spec.num_kv_heads
+        return [StepTable(f"mixer_arrived_{heads}", lambda lanes, tokens: lanes * heads, lambda out, packed: None)]
 
     def conv_state(self, caches) -> torch.Tensor:
         return caches[self.mamba_name].states["conv"]
@@ -991,14 +993,6 @@ class AttentionMamba2Step:
         return (cache.owns_kv
                 and ops.mixer_decode_supported(a.num_heads, a.num_kv_heads, a.head_dim, cache.k_cache.shape[2],
                                                self.mamba.spec.state_size, step.max_seq_len, a.window, self.rotary_dim))
-
-    def merge_later_bytes(self, step, caches):
-        """(columns of the attended heads, bytes of runs of keys a workgroup reads to merge them), or None."""
-        a = self.attention.spec
-        rows, page_size = step.num_tokens, caches[self.attention_name].k_cache.shape[2]
-        span = max(1, int(step.max_seq_len)) if not a.window else a.window + page_size
-        runs = ops.mixer_runs(rows, a.num_kv_heads, page_size, span, a.head_dim)[1]
-        return a.num_heads * a.head_dim, rows * a.num_heads * min(runs, ops.MERGE_AT_ONCE) * (a.head_dim + 2) * 4
 
     def run(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, merge: bool = True):
         a, s = self.attention.spec, self.mamba.spec
@@ -1014,7 +1008,8 @@ class AttentionMamba2Step:
             ssm_heads=s.num_heads, ssm_head_dim=s.head_dim, state_size=s.state_size,
             num_groups=s.num_groups, z_col=self.z_col, x_col=self.x_col, dt_col=self.dt_col,
             dt_bias=self.mamba.dt_bias, A=self.mamba.A, D=self.mamba.D, ssm_state=state.states["ssm"],
-            slot_ids=step.slot_ids, out=mixed, ssm_y=y, merge=merge)
+            slot_ids=step.slot_ids, out=mixed, ssm_y=y, merge=merge,
+            arrived=step.tables.get(f"mixer_arrived_{a.num_kv_heads}") if merge else None)
         if gated_norm:
             ops.gate_norm(y, u[:, self.z_col:self.z_col + s.inner_size], self.mamba.norm_weight, s.num_groups,
                           s.norm_eps, mixed[:, self.attended_width:])

@@ -1564,6 +1564,53 @@ def test_output_projection_that_merges_the_runs_of_keys(ops, Hq, Hkv, dh, E, N_o
     close(want, product, dtype, max(1.0, product.abs().max().item()))
 
 
+@pytest.mark.parametrize("Hq, Hkv, dh, window, most, lengths", [
+    (8, 2, 64, None, 0, [1, 17, 64, 65, 300, 1500, 2, 2060]), (8, 2, 64, 1100, 0, [1, 700, 1500, 2060]),
+    (12, 2, 128, None, 0, [700, 3]), (4, 4, 64, None, 0, [5000, 9000, 3] + [40 + lane for lane in range(13)]),
+    (2, 2, 128, None, 9000, [257 + 64 * lane for lane in range(40)]), (5, 1, 64, None, 12000, [2100])])
+def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, most, lengths):
+    """With counters the runs of keys are merged by whichever workgroup ends last: the bits of the merge kernel, launch
+    after launch with the same counters, which are zeros again; contexts of one run, of more runs than a merge asks for at
+    once, of runs that one workgroup walks over, a window of several runs, a launch made for far longer contexts."""
+    dtype = torch.bfloat16
+    H, P, N, G, page_size = 4, 16, 32, 1, 16
+    E, M = H * P, len(lengths)
+    pool, table = paged_setup(lengths, page_size, Hkv, dh, dtype, seed=23)
+    for lane, length in enumerate(lengths):
+        fill_cache(pool, table, lane, rand(length, Hkv, dh, seed=600 + lane, dtype=dtype),
+                   rand(length, Hkv, dh, seed=700 + lane, dtype=dtype), page_size)
+    q_col, k_col, v_col = 0, Hq * dh, (Hq + Hkv) * dh
+    z_col = (Hq + 2 * Hkv) * dh
+    x_col, dt_col = z_col + E, z_col + 2 * E + 2 * G * N
+    u = rand(M, -(-(dt_col + H) // 8) * 8, seed=610, dtype=dtype).to(DEV)
+    positions = i32([length - 1 for length in lengths]).to(DEV)
+    slot_mapping = i32([int(table[lane, (length - 1) // page_size]) * page_size + (length - 1) % page_size
+                        for lane, length in enumerate(lengths)]).to(DEV)
+    inv_freq = torch.tensor([1.0 / (1e4 ** (i / dh)) for i in range(0, dh, 2)], dtype=torch.float64).float().to(DEV)
+    vectors = [rand(H, seed=612) - 2.0, -(rand(H, seed=613).abs() + 0.1), rand(H, seed=614)]
+    arrived = torch.zeros(M * Hkv, dtype=torch.int32, device=DEV)
+
+    def run(counters):
+        dev_pool = pool.clone().to(DEV)
+        mixed = torch.full((M, Hq * dh + E), float("nan"), dtype=dtype, device=DEV)
+        ops.mixer_decode(u, num_heads=Hq, num_kv_heads=Hkv, head_dim=dh, q_col=q_col, k_col=k_col, v_col=v_col,
+                         inv_freq=inv_freq, rotary_dim=dh, k_cache=views(dev_pool, page_size)[0],
+                         v_cache=views(dev_pool, page_size)[1], block_tables=table.to(DEV), positions=positions,
+                         slot_mapping=slot_mapping, scale=0.13, window=window, max_seq_len=max(max(lengths) + 5, most),
+                         ssm_heads=H, ssm_head_dim=P, state_size=N, num_groups=G, z_col=z_col, x_col=x_col, dt_col=dt_col,
+                         dt_bias=vectors[0].to(DEV), A=vectors[1].to(DEV), D=vectors[2].to(DEV),
+                         ssm_state=rand(M, H, P, N, seed=611, scale=0.5).to(DEV), slot_ids=i32(list(range(M))).to(DEV), out=mixed,
+                         ssm_y=None, arrived=counters)
+        return mixed
+
+    want = run(None)
+    assert torch.isfinite(want.float()).all()
+    for _ in range(3):
+        assert torch.equal(run(arrived), want) and not arrived.any()
+    with pytest.raises(ops.KernelError):
+        run(arrived[:-1])
+
+
 def test_mixer_decode_over_a_long_context(ops):
     """Contexts of 5 000 and 9 000 tokens (more runs of keys than the merge takes
     at once) beside a short one; one far key per long request is made to dominate, so a run that
