@@ -1655,6 +1655,14 @@ extern "C" int mi_fused_gemm_supported(int pro, int M, int K) {
 #define MX_SCAN_PER_THREAD 8
 #define MX_FEW_BLOCKS 512       // state-space workgroups of a step up to which each takes one row per thread group
 
+// Weights that the products behind the mixers read, in tiles of 16 features one behind the other.
+#define AHEAD_MOST 4
+#define AHEAD_BLOCKS 256        // workgroups that read them, a multiple of 8
+struct AheadWeight {
+  const void* at;
+  long tiles, tile_bytes;
+};
+
 struct MixerParams {
   // the layer's projected row per token: [q | k | v | z | x B C (after conv) | dt], bfloat16
   const bf16_t* u;
@@ -1686,13 +1694,17 @@ struct MixerParams {
   bf16_t* ssm_out;        // gated y, bfloat16 (when no norm follows)
   float* ssm_y;           // or float32 y before the gate (when a grouped norm follows)
   long out_ld;
-  int attention_blocks;
+  int attention_blocks, ahead_from;        // the attention's workgroups come first; those from ahead_from on read ahead
   // the context of a request is cut into runs of split_keys keys, one workgroup each; their
   // partial results [M, Hq, splits, DH + 2] = (maximum, normalizer, sums) are merged by mixer_merge_kernel
   int splits;
   int split_keys;
   float* partial;
   int* arrived;           // [M, Hkv] zeros, which the launch leaves zero again: the runs are merged inside it; or null
+};
+
+struct MixerAhead {
+  AheadWeight weight[AHEAD_MOST];
 };
 
 // A word that another workgroup's cache must see, or may have written, without the fences that would write back and drop
@@ -2061,14 +2073,46 @@ __device__ void mixer_ssm_block(const MixerParams& p, int block) {
   }
 }
 
-template <int DH>
-__global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p) {
+// The mixers of a small step wait for round trips and leave the memory idle, and the four products behind them are as long
+// as the way of their weights from memory: these workgroups read the weights meanwhile and drop them.  What they leave is
+// in the caches: a tile is read on the die whose cache the product's workgroup of that number will ask (workgroups go to
+// the eight dies in turn), or, where the mixers' own bytes have pushed it out, in the memory-side cache.  Pieces of
+// MX_THREADS 16-byte words, dealt out to the die's workgroups in the order in which the products will read them.
+__device__ void mixer_ahead_block(const MixerAhead& p, int block) {
+  const int die = blockIdx.x % 8;
+  constexpr int PIECE = MX_THREADS * 16;
+  long u = block / 8;
+#pragma unroll
+  for (int k = 0; k < AHEAD_MOST; ++k) {
+    const AheadWeight w = p.weight[k];
+    const long tiles = (w.tiles - die + 7) / 8;                          // of this die
+    const long pieces = (w.tile_bytes + PIECE - 1) / PIECE;
+    const long count = tiles * pieces;
+    for (; u < count; u += 4 * (AHEAD_BLOCKS / 8)) {
+      floatx4 word[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const long item = min(u + j * (AHEAD_BLOCKS / 8), count - 1);
+        const long tile = item / pieces, at = (item - tile * pieces) * PIECE + threadIdx.x * 16;
+        word[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(w.at) + (die + 8 * tile) * w.tile_bytes + min(at, w.tile_bytes - 16));
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) asm volatile("" ::"v"(word[j]));
+    }
+    u = block / 8;
+  }
+}
+
+template <int DH, bool AHEAD>
+__device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const MixerAhead& ahead) {
   __shared__ int pages_lds[MX_MAX_PAGES];
   __shared__ float cs[DH];
   __shared__ float merge_lds[MX_WAVES * 8 * (DH + 2)];
   __shared__ int last_lds;
   if ((int)blockIdx.x < p.attention_blocks)
     mixer_attention_block<DH>(p, blockIdx.x, pages_lds, cs, merge_lds, &last_lds);
+  else if (AHEAD && (int)blockIdx.x >= p.ahead_from)
+    mixer_ahead_block(ahead, blockIdx.x - p.ahead_from);
   else if (!p.vector_scan)
     mixer_ssm_block<false, 1>(p, blockIdx.x - p.attention_blocks);
   else if (p.rows_per_thread == 1)
@@ -2079,6 +2123,17 @@ __global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p)
     mixer_ssm_block<true, 4>(p, blockIdx.x - p.attention_blocks);
   else
     mixer_ssm_block<true, 8>(p, blockIdx.x - p.attention_blocks);
+}
+
+template <int DH>
+__global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p) {
+  mixer_decode_block<DH, false>(p, MixerAhead{});
+}
+
+// (a kernel of its own: 64 rows pay 1.6 us a launch for the question alone)
+template <int DH>
+__global__ void __launch_bounds__(MX_THREADS) mixer_decode_ahead_kernel(MixerParams p, MixerAhead ahead) {
+  mixer_decode_block<DH, true>(p, ahead);
 }
 
 // Keys of one attention workgroup (a run).  Long runs pay the start of a workgroup (position, page ids,
@@ -2130,7 +2185,8 @@ extern "C" int mi_mixer_runs(int M, int Hkv, int dh, int page_size, long span, i
 // kv head have one workgroup, mi_mixer_runs says runs = 1, there is nothing to merge: that workgroup writes the
 // attended heads itself, whatever `merge` says, and no merge kernel is launched.)  arrived (with merge; or null: a merge
 // kernel is launched): [M, Hkv] int32 zeros, by which the runs are merged inside the launch; zeros again behind it, so that
-// the launches of a step share them one after the other.
+// the launches of a step share them one after the other.  ahead (ahead_count, up to AHEAD_MOST): weights that the launches
+// behind this one will read, brought into the caches by workgroups of their own; nothing else depends on them.
 extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv, int dh, int q_col, int k_col,
                                int v_col, const float* inv_freq, int rotary_dim, void* k_base, void* v_base,
                                long page_stride, int page_size, const int* block_tables, int max_pages,
@@ -2138,7 +2194,8 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
                                int max_seq_len, int H, int P, int N, int G, int z_col, int x_col, int dt_col, const float* dt_bias,
                                const float* A, const float* D, float* ssm_state, const int* slot_ids,
                                void* attn_out, void* ssm_out, float* ssm_y, long out_ld, float* partial,
-                               long partial_floats, int merge, int* arrived, hipStream_t stream) {
+                               long partial_floats, int merge, int* arrived, const AheadWeight* ahead, int ahead_count,
+                               hipStream_t stream) {
   if (M <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || H <= 0 || P <= 0 || N <= 0 || G <= 0 || H % G != 0)
     return ERR_BAD_ARGUMENT;
   const int group = Hq / Hkv;
@@ -2217,8 +2274,18 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
   p.arrived = merge ? arrived : nullptr;
   p.attention_blocks = Hkv * M * p.splits;
   const long total = (long)p.attention_blocks + (long)p.p_tiles * H * M;
-  if (total > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
-  if (dh == 64) mixer_decode_kernel<64><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
+  if (total > 0x7fffffffL - AHEAD_BLOCKS - 8) return ERR_UNSUPPORTED_SIZE;
+  if (ahead_count < 0 || ahead_count > AHEAD_MOST || (ahead_count && !ahead)) return ERR_BAD_ARGUMENT;
+  MixerAhead reads = {};
+  p.ahead_from = (int)total;
+  for (int k = 0; k < ahead_count; ++k) {
+    reads.weight[k] = ahead[k];
+    if (!ahead[k].at || (uintptr_t)ahead[k].at % 16 || ahead[k].tiles <= 0 || ahead[k].tile_bytes <= 0 || ahead[k].tile_bytes % 16)
+      return ERR_BAD_ARGUMENT;
+  }
+  if (ahead_count && dh == 64) mixer_decode_ahead_kernel<64><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads);
+  else if (ahead_count) mixer_decode_ahead_kernel<128><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads);
+  else if (dh == 64) mixer_decode_kernel<64><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
   else mixer_decode_kernel<128><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
   RETURN_IF_LAUNCH_FAILED();
   if (!merge || p.splits == 1 || p.arrived) return 0;

@@ -202,7 +202,7 @@ _SIGNATURES = {
                             _c_ptr, _c_ptr, _c_long, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int,
                             _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                             _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long,
-                            _c_int, _c_ptr, _c_ptr],
+                            _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     },
     "microbench": {
         "mi_stream_read": [_c_ptr, _c_long, _c_ptr, _c_int, _c_ptr],
@@ -2462,6 +2462,9 @@ def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: i
     return run_keys.value, runs.value
 
 
+AHEAD_MOST = 4             # weights that mixer_decode brings into the caches at most (decode.hip)
+
+
 def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim: int, q_col: int, k_col: int,
                  v_col: int, inv_freq: Optional[torch.Tensor], rotary_dim: int, k_cache: torch.Tensor,
                  v_cache: torch.Tensor, block_tables: torch.Tensor, positions: torch.Tensor,
@@ -2470,7 +2473,7 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
                  z_col: int, x_col: int, dt_col: int, dt_bias: torch.Tensor, A: torch.Tensor, D: torch.Tensor,
                  ssm_state: torch.Tensor, slot_ids: torch.Tensor, out: torch.Tensor,
                  ssm_y: Optional[torch.Tensor], merge: bool = True,
-                 arrived: Optional[torch.Tensor] = None) -> Optional[AttentionRuns]:
+                 arrived: Optional[torch.Tensor] = None, ahead: Sequence[torch.Tensor] = ()) -> Optional[AttentionRuns]:
     """Both mixers of a decode step in one launch.  ``u`` [M, >=cols] holds each token's projected
     row (q, k, v unrotated; x, B, C after the conv).  Attention: rotates q and the new key, writes
     the new K/V into the cache cell ``slot_mapping``, attends over the request's pages, writes
@@ -2479,7 +2482,9 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
     follows.  ``max_seq_len``: an upper bound of the longest context in the batch.  With ``merge=False``
     ``out[:, :Hq*dh]`` is not written: the runs of keys are returned unmerged, for ``fused_gemm_merge``.
     ``arrived``: int32 zeros, one a token and kv head, which are zeros again behind the call: the runs are merged
-    inside the launch by whichever workgroup ends last (without them by a launch of their own, the same bits)."""
+    inside the launch by whichever workgroup ends last (without them by a launch of their own, the same bits).
+    ``ahead``: up to four weights in fragment order that the launches behind this one read, in that order: brought
+    into the caches meanwhile."""
     u_ld = _row_major(u, "u")
     out_ld = _row_major(out, "out")
     M = u.shape[0]
@@ -2506,6 +2511,9 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
     if arrived is not None:
         _i32(arrived, "arrived")
         _need(arrived.numel() >= M * num_kv_heads, "mixer_decode: one counter per token and kv head")
+    _need(len(ahead) <= AHEAD_MOST and all(w.is_cuda and w.is_contiguous() and w.dim() == 5 for w in ahead),
+          "mixer_decode: up to four weights in fragment order ahead")
+    weights = (_c_long * (3 * AHEAD_MOST))(*(number for w in ahead for number in (w.data_ptr(), w.shape[0], w[0].numel() * w.element_size())))
     span = max(1, int(max_seq_len)) if not window else window + page_size
     run_keys, runs = mixer_runs(M, num_kv_heads, page_size, span, head_dim)        # the launcher's own rule
     partial = torch.empty((M * num_heads * runs * (head_dim + 2),), dtype=torch.float32, device=u.device)
@@ -2515,7 +2523,8 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
         _p(slot_mapping), float(scale), int(window or 0), int(max_seq_len), ssm_heads, ssm_head_dim, state_size,
         num_groups, z_col, x_col, dt_col, _p(dt_bias), _p(A), _p(D), _p(ssm_state), _p(slot_ids), _p(out),
         out.data_ptr() + 2 * num_heads * head_dim,
-        _p(ssm_y), out_ld, _p(partial), partial.numel(), int(merge), _p(arrived), _stream()), "mixer_decode")
+        _p(ssm_y), out_ld, _p(partial), partial.numel(), int(merge), _p(arrived),
+        ctypes.addressof(weights), len(ahead), _stream()), "mixer_decode")
     if merge or runs == 1:                  # one workgroup per token and kv head has written the heads itself
         return None
     return AttentionRuns(partial, positions, num_heads, head_dim, runs, run_keys, page_size, int(window or 0))

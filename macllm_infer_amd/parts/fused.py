@@ -119,6 +119,14 @@ FORCE_PADDING: Optional[bool] = None      # tests: True or False instead of the 
 # at 8 rows 1,198 with the counters and 1,252 with the merge as a launch of its own.  No step takes that way by itself.
 FORCE_MERGE_LATER: Optional[bool] = None  # True: the output projection merges, where it takes the step
 _padding_wins: Dict[tuple, tuple] = {}
+# The mixers of a small step wait for round trips and leave the memory idle, so their launch also brings the weights of the
+# products behind them, the next layer's first one included, into the caches, in the order in which they are read: as many
+# as AHEAD_BYTES hold (the dies' caches together) beside the states that the step reads and writes.  A step of the 0.5B
+# shape (25 MB a layer, 1.6 MB of states a row) in us without | out and gate-up | and down | and the next layer's input, at
+# contexts of 2,048: 1 row 1,034 | 978 | 962 | 947, 4 rows 1,096 | 1,044 | 1,033 | 1,036, 8 rows 1,203 | 1,171 | 1,153 | 1,184, 12 rows
+# 1,369 | 1,336 | 1,361 | 1,408, 16 rows 1,424 | 1,437 | 1,459 | 1,505; of 300: 1 row 1,003 | 947 | 924 | 907, 8 rows 1,148 | 1,084 | 1,113 |
+# 1,150, 16 rows 1,305 | 1,264 | 1,282 | 1,318.  The 7B shape's 28 MB of output projection: 1 row 1,098 | 1,084, 4 rows 1,196 | 1,225.
+AHEAD_BYTES = 32 << 20
 # A projection whose result joins the residual stream can add it there itself (float32, in place) and leave, beside
 # the stream, its rows times the next norm's weight in bfloat16 with the partial sums of their squares; the product
 # behind that norm then reads those rows and multiplies its float32 sums by 1 / sqrt(mean square + eps): the norm
@@ -340,7 +348,8 @@ def register_mixer_kernel(*kinds: str):
     product's epilogue: {lo, hi, taps, weight, bias}), ``supported(step, caches)``,
     ``conv_state(caches)`` and ``run(u, step, caches, mixed, merge=True)``; a kernel with ``merged_columns`` (how
     many the attended heads are, the first columns of ``mixed``) returns, when called with ``merge=False``, their runs of
-    keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; ``step_tables()``: tables it reads in every step."""
+    keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; ``step_tables()``: tables it reads in every step;
+    ``ahead``: weights that its launch may bring into the caches, if it says the ``state_bytes`` that it moves a row."""
     def decorate(factory):
         _MIXER_KERNELS[tuple(kinds)] = factory
         return factory
@@ -802,10 +811,26 @@ class LayerFusion:
         if kernel is not None:
             later = (not self.library_out[bucket] and not self.split_out[bucket]
                      and self._merges_later(kernel, step, caches))
-            attended = kernel.run(u, step, caches, mixed, merge=not later)
+            attended = kernel.run(u, step, caches, mixed, merge=not later, ahead=self._read_ahead(residual, kernel, M, bucket))
         else:
             self._mix_each(u, step, caches, mixed)
         self._after_the_mixers(residual, mixed, attended, M, bucket)
+
+    def _read_ahead(self, residual: Residual, kernel, M: int, bucket: int) -> list:
+        """The weights of the products behind the mixers that the mixers' launch brings into the caches."""
+        room = AHEAD_BYTES - M * getattr(kernel, "state_bytes", AHEAD_BYTES)
+        products = [(self.library_out[bucket], self.f_out)]
+        if self.gate_up is not None:
+            products += [(self.library_gate_up[bucket], self.f_gate_up), (self.library_down[bucket], self.f_down)]
+        weights = []
+        for library, fragments in products + [(False, residual.next_first)]:
+            if library or fragments is None:
+                continue
+            room -= fragments.numel() * fragments.element_size()
+            if room < 0:
+                break
+            weights.append(fragments)
+        return weights
 
     def _norm_prologue(self, residual: Residual, M: int, norm, rms):
         """The input of a projection: the norm in the kernel's prologue, or its own kernel before."""
@@ -974,6 +999,7 @@ class AttentionMamba2Step:
         self.x_col = second + s.inner_size
         self.dt_col = self.x_col + s.conv_width
         self.attended_width = self.merged_columns = q_width
+        self.state_bytes = 2 * 4 * s.num_heads * s.head_dim * s.state_size         # a row's states, read and written
         self.inv_freq, self.rotary_dim = self.attention.position.fused_rotation()
         self.conv = dict(lo=self.x_col, hi=self.dt_col, taps=s.conv_kernel, weight=self.mamba.conv_weight,
                          bias=self.mamba.conv_bias)
@@ -994,7 +1020,7 @@ class AttentionMamba2Step:
                 and ops.mixer_decode_supported(a.num_heads, a.num_kv_heads, a.head_dim, cache.k_cache.shape[2],
                                                self.mamba.spec.state_size, step.max_seq_len, a.window, self.rotary_dim))
 
-    def run(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, merge: bool = True):
+    def run(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, merge: bool = True, ahead=()):
         a, s = self.attention.spec, self.mamba.spec
         kv, state = caches[self.attention_name], caches[self.mamba_name]
         gated_norm = self.mamba.norm_weight is not None
@@ -1009,7 +1035,7 @@ class AttentionMamba2Step:
             num_groups=s.num_groups, z_col=self.z_col, x_col=self.x_col, dt_col=self.dt_col,
             dt_bias=self.mamba.dt_bias, A=self.mamba.A, D=self.mamba.D, ssm_state=state.states["ssm"],
             slot_ids=step.slot_ids, out=mixed, ssm_y=y, merge=merge,
-            arrived=step.tables.get(f"mixer_arrived_{a.num_kv_heads}") if merge else None)
+            arrived=step.tables.get(f"mixer_arrived_{a.num_kv_heads}") if merge else None, ahead=ahead)
         if gated_norm:
             ops.gate_norm(y, u[:, self.z_col:self.z_col + s.inner_size], self.mamba.norm_weight, s.num_groups,
                           s.norm_eps, mixed[:, self.attended_width:])

@@ -222,7 +222,7 @@ def total(costs: Dict[str, Cost]) -> Cost:
 # launched once a step is the output head; launched more often, an output or down projection (the library's
 # products carry no such mark and stay with the other kernels).
 DECODE_GROUPS: List[Tuple[str, str]] = [
-    (r"mixer_decode_kernel|mixer_merge_kernel|decode_attention_kernel|decode_merge_kernel|ssm_scan_kernel|conv_step_kernel|"
+    (r"mixer_decode_|mixer_merge_kernel|decode_attention_kernel|decode_merge_kernel|ssm_scan_kernel|conv_step_kernel|"
      r"gate_norm_kernel|rope_kv_store_kernel|paged_attention_kernel|paged_attention_tile_kernel|"
      r"paged_attention_merge_kernel|linear_state_|head_norm_gate_|wide_norm_gate_kernel|tanh_rows_kernel|latent_|rotate_heads_kernel|attention_prepare_kernel", "mixers"),
     (r"fused_gemm_kernel<\d+, \d+, 2|skinny_kernel<\d+, 2|shared_rows_gemm_kernel<\d+, \d+, 2", "input projections"),

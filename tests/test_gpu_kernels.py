@@ -1571,7 +1571,8 @@ def test_output_projection_that_merges_the_runs_of_keys(ops, Hq, Hkv, dh, E, N_o
 def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, most, lengths):
     """With counters the runs of keys are merged by whichever workgroup ends last: the bits of the merge kernel, launch
     after launch with the same counters, which are zeros again; contexts of one run, of more runs than a merge asks for at
-    once, of runs that one workgroup walks over, a window of several runs, a launch made for far longer contexts."""
+    once, of runs that one workgroup walks over, a window of several runs, a launch made for far longer contexts.  And
+    the same bits where the launch reads weights ahead (of one tile, of tiles that are no multiple of 8)."""
     dtype = torch.bfloat16
     H, P, N, G, page_size = 4, 16, 32, 1, 16
     E, M = H * P, len(lengths)
@@ -1590,7 +1591,7 @@ def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, mo
     vectors = [rand(H, seed=612) - 2.0, -(rand(H, seed=613).abs() + 0.1), rand(H, seed=614)]
     arrived = torch.zeros(M * Hkv, dtype=torch.int32, device=DEV)
 
-    def run(counters):
+    def run(counters, ahead=()):
         dev_pool = pool.clone().to(DEV)
         mixed = torch.full((M, Hq * dh + E), float("nan"), dtype=dtype, device=DEV)
         ops.mixer_decode(u, num_heads=Hq, num_kv_heads=Hkv, head_dim=dh, q_col=q_col, k_col=k_col, v_col=v_col,
@@ -1600,13 +1601,17 @@ def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, mo
                          ssm_heads=H, ssm_head_dim=P, state_size=N, num_groups=G, z_col=z_col, x_col=x_col, dt_col=dt_col,
                          dt_bias=vectors[0].to(DEV), A=vectors[1].to(DEV), D=vectors[2].to(DEV),
                          ssm_state=rand(M, H, P, N, seed=611, scale=0.5).to(DEV), slot_ids=i32(list(range(M))).to(DEV), out=mixed,
-                         ssm_y=None, arrived=counters)
+                         ssm_y=None, arrived=counters, ahead=ahead)
         return mixed
 
     want = run(None)
     assert torch.isfinite(want.float()).all()
     for _ in range(3):
         assert torch.equal(run(arrived), want) and not arrived.any()
+    weights = [ops.fragment_order(torch.ones(rows, width, dtype=dtype, device=DEV)) for rows, width in ((12, 64), (4120, 1024), (136, 96), (64, 4608))]
+    assert torch.equal(run(arrived, weights), want) and torch.equal(run(None, weights[:1]), want)
+    with pytest.raises(ops.KernelError):
+        run(arrived, weights + weights[:1])
     with pytest.raises(ops.KernelError):
         run(arrived[:-1])
 
