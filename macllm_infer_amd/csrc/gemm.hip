@@ -128,17 +128,35 @@ gemm_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict__
 }
 
 // Many rows: a group of 2 x 2 waves owns 32 MT rows x 32 NT features, stages 32 columns of both operands in LDS (two
-// buffers; the next stage is on its way to registers while this one is multiplied) and sums the four runs of chunks
+// buffers; the stages behind it are on their way to registers while this one is multiplied) and sums the four runs of chunks
 // one after the other, each from zero, adding the runs' sums in their order: bit for bit the sums above.
 // GROUPS = 4: four such groups of a workgroup take a run each and group 0 adds their tiles, for products of too few
 // tiles to fill 256 compute units one wave a SIMD (a wave's chain of products is then a quarter as long).
 // LDS: a row of a stage is eight 16-byte pieces; piece p of row r lies at r * 8 + (p ^ (r & 7)), so that the eight rows
 // that a quarter-wave reads at once fall into different banks, and a thread's stores are one run.
-// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32, 152 TFLOP/s in a large library product) where the tiles
-// fill the chip (512 x 4,096 x 1,024: 105 TFLOP/s, 86 with the waves' operands straight from the caches, each row of
-// 64 bytes a chunk), else the tiles' serial walk over K (512 x 1,024 x 2,048: 27 us, 53 before; 100 x 1,024 x 2,048: 16
-// us, 50 before).  A second stage on its way (102 TFLOP/s), 128 x 128 tiles (92) and an order of the tiles by die gain nothing.
-template <int MT, int NT, int GROUPS>
+// EVEN: the runs are whole stages (K a multiple of 128).
+// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32, 152 TFLOP/s in a large library product) and what the waves
+// do between their products, all at once in a workgroup: with the operands fetched where they are used, the stages laid
+// down and asked for in a row and the barrier behind, 512 x 4,096 x 1,024 took 47.1 us, 512 x 1,024 x 2,048 29.4, 512 x 768 x
+// 1,024 16.6, 512 x 32,784 x 1,024 331; fetched a chunk ahead, one by one between the products, 45.1, 24.2, 14.5, 321 (without
+// any of those instructions 35, 18, 11, 252).  64 x 128 tiles in two groups take 43.5, 41.1 (N = 768) and 343, 64 x 64 ones in
+// two groups 47.4; a second stage on its way, 128 x 128 tiles and an order of the tiles by die gain nothing.
+
+// The order of a chunk's instructions: stores to LDS, loads from memory and loads from LDS one by one between its products.
+template <int PRODUCTS, int STORES, int LOADS, int FETCHES>
+__device__ __forceinline__ void interleave() {
+  constexpr int OTHERS = STORES + LOADS + FETCHES;
+  constexpr int EACH = PRODUCTS / OTHERS > 0 ? PRODUCTS / OTHERS : 1;
+#pragma unroll
+  for (int i = 0; i < OTHERS; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);                        // matrix products
+    if (i < STORES) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);           // a store to LDS
+    else if (i < STORES + LOADS) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);          // a load from memory
+    else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                      // a load from LDS
+  }
+}
+
+template <int MT, int NT, int GROUPS, bool EVEN>
 __global__ void __launch_bounds__(GF_THREADS * GROUPS)
 tiled_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict__ W, long ldw,
                  const float* __restrict__ bias, float* __restrict__ out, long ldo, bool whole, int M, int N, int K) {
@@ -188,35 +206,26 @@ tiled_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict_
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = total[nt][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
   int left = run;
-  ask(0);
-  lay_down(0);
-  __syncthreads();
-  for (int stage = 0; stage < stages; ++stage) {
-    const floatx4* const staged = stage_of_group + (stage & 1) * ROWS * 8;
-    ask(stage + 1);
-    __builtin_amdgcn_sched_barrier(0);                         // the loads before the products, their stores to LDS behind them
+  floatx4 weights[2][NT], rows[2][MT];                         // the operands of a stage's two chunks
+  auto fetch = [&](int stage, int c) {                         // (a row's number and r agree modulo 8)
+    const floatx4* const staged = stage_of_group + (stage & 1) * ROWS * 8 + ((4 * c + q) ^ (r & 7));
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      if (GROUPS > 1 && 2 * stage + c >= mine) continue;
-      floatx4 weights[NT], rows[MT];
+    for (int nt = 0; nt < NT; ++nt) weights[c][nt] = staged[(first_n + nt * 16 + r) * 8];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int row = first_n + nt * 16 + r;
-        weights[nt] = staged[row * 8 + ((4 * c + q) ^ (row & 7))];
-      }
+    for (int mt = 0; mt < MT; ++mt) rows[c][mt] = staged[(BN + first_m + mt * 16 + r) * 8];
+  };
+  auto multiply = [&](int stage, int c) {
+    if (GROUPS > 1 && !EVEN && 2 * stage + c >= mine) return;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int row = BN + first_m + mt * 16 + r;
-        rows[mt] = staged[row * 8 + ((4 * c + q) ^ (row & 7))];
-      }
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(weights[nt][i], rows[mt][i], acc[nt][mt], 0, 0, 0);
-      if (GROUPS == 1 && --left == 0) {                        // a run ends
+        for (int mt = 0; mt < MT; ++mt)
+          acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(weights[c][nt][i], rows[c][mt][i], acc[nt][mt], 0, 0, 0);
+    if (GROUPS == 1 && (c == 1 || !EVEN)) {
+      left -= EVEN ? 2 : 1;
+      if (left == 0) {                                         // a run ends
         left = run;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
@@ -227,12 +236,31 @@ tiled_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict_
           }
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Every wait has products in front of it: a stage's columns leave memory a whole stage before they are laid down, and
+  // a chunk's operands leave LDS while the chunk before is multiplied.  The one barrier a stage stands between its two
+  // chunks: behind it the next stage is laid down, and nobody reads the one before any more.
+  ask(0);
+  lay_down(0);
+  ask(1);
+  __syncthreads();
+  fetch(0, 0);
+  for (int stage = 0; stage < stages; ++stage) {
     lay_down((stage + 1) & 1);
+    ask(stage + 2);
+    fetch(stage, 1);
+    multiply(stage, 0);
+    interleave<4 * NT * MT, PIECES, PIECES, NT + MT>();
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
+    fetch(stage + 1, 0);
+    multiply(stage, 1);
+    interleave<4 * NT * MT, 0, 0, NT + MT>();
+    __builtin_amdgcn_sched_barrier(0);
   }
 
-  if (GROUPS > 1) {                                            // behind the loop's last barrier: the stages are read
+  if (GROUPS > 1) {
+    __syncthreads();                                           // the stages are read
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -279,25 +307,29 @@ extern "C" int mi_gemm_f32(const float* x, long ldx, const float* W, long ldw, c
                    ((unsigned long long)W % 16) == 0;
   if (M > 32 && vec && K % 32 == 0) {
     // The tiling that the rounds of workgroups over 256 compute units make cheapest: microseconds a round at K =
-    // 1,024, in tenths, as measured over 33 to 512 rows and 768 to 32,784 features (32 x 32 in four groups: 9.1, 15.7,
-    // 22.5, 28.7 for one to four rounds; 32 x 64 in four groups: 14.3, 28; 64 x 64 in one group: 24.5, 41, then two
-    // workgroups a compute unit hide each other's waits).  From 33 rows on the best of them is at least as fast as
-    // the first kernel at every size measured (64 x 1,024 x 2,048: 16 us against 21; 33 x 3,352 x 1,024: 9.7 against 11).
+    // 1,024, in tenths, as measured over 40 to 512 rows and 768 to 32,784 features (32 x 32 in four groups: 9.0 to 9.8,
+    // 15.8, 22.5, 28.8, 37.1, 41.7 for one to six rounds; 32 x 64 in four groups: 13.4 to 15.3, 28, 38 to 40, 55; 64 x 64 in one
+    // group: 22.5 to 24.7, 41 to 45, 61.6, then 20.5 a round: workgroups of a compute unit hide each other's waits).  From 33 rows
+    // on the best of them is at least as fast as the first kernel at every size measured.
     auto rounds = [&](long rows, long features) {
       return (((M + rows - 1) / rows) * ((N + features - 1) / features) + 255) / 256;
     };
-    const long small = 25 + 66 * rounds(32, 32), middle = 5 + 139 * rounds(32, 64);
-    const long large = rounds(64, 64) == 1 ? 245 : 205 * rounds(64, 64);
+    const long small = 28 + 66 * rounds(32, 32), middle = 25 + 130 * rounds(32, 64), tall = rounds(64, 64);
+    const long large = tall == 1 ? 240 : tall == 2 ? 430 : 205 * tall;
     const bool whole = ldo % 4 == 0 && ((unsigned long long)out % 16) == 0;
     const int bm = large < small && large < middle ? 64 : 32, bn = bm == 64 || middle < small ? 64 : 32;
     const dim3 tiles((unsigned)(((long)N + bn - 1) / bn), (unsigned)(((long)M + bm - 1) / bm));
     if (((long)M + bm - 1) / bm <= 65535) {
-      if (bm == 64)
-        tiled_f32_kernel<2, 2, 1><<<tiles, GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
-      else if (bn == 64)
-        tiled_f32_kernel<1, 2, 4><<<tiles, 4 * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
-      else
-        tiled_f32_kernel<1, 1, 4><<<tiles, 4 * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
+      const bool even = K % 128 == 0;
+#define TILED(MT_, NT_, GROUPS_)                                                                                       \
+  do {                                                                                                                 \
+    if (even) tiled_f32_kernel<MT_, NT_, GROUPS_, true><<<tiles, GROUPS_ * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K); \
+    else tiled_f32_kernel<MT_, NT_, GROUPS_, false><<<tiles, GROUPS_ * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);     \
+  } while (0)
+      if (bm == 64) TILED(2, 2, 1);
+      else if (bn == 64) TILED(1, 2, 4);
+      else TILED(1, 1, 4);
+#undef TILED
       RETURN_IF_LAUNCH_FAILED();
       return 0;
     }

@@ -144,6 +144,12 @@ def test_tiled_float32_product_sums_in_the_order_of_the_small_one(ops, shape):
     assert torch.equal(ops.linear(x[:17], w, None), ops.linear(x, w, None)[:17])
 
 
+@pytest.mark.parametrize("shape", [(33, 70, 128), (70, 1000, 256), (130, 2100, 384), (448, 4100, 128)])
+def test_tiled_float32_product_of_runs_of_whole_stages(ops, shape):
+    """K a multiple of 128, from a single stage a run on, through the same three tilings: as above."""
+    test_tiled_float32_product_sums_in_the_order_of_the_small_one(ops, shape)
+
+
 def test_mixed_product_keeps_a_32bit_weight(ops):
     x, w = rand(4, 96, seed=10, dtype=torch.bfloat16), rand(50, 96, seed=11)
     got = ops.linear(x.to(DEV), w.to(DEV), None)
