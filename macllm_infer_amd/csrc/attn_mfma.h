@@ -54,6 +54,10 @@ struct AttnCache {
   int base_page;
   int value_dim;         // PADDED loads only: the width of a cached value, at most the DV the wave computes with
   int key_dim;           // PADDED_KEYS loads only: the width of a cached key, a multiple of 8 and at most DH
+  int page_shift = -1;   // log2 of page_size, for a caller that says it: a division is 16 instructions, four of them a step of 32 keys
+
+  __device__ __forceinline__ int page_of(int key) const { return page_shift >= 0 ? key >> page_shift : key / page_size; }
+  __device__ __forceinline__ int place_of(int key) const { return page_shift >= 0 ? key & (page_size - 1) : key % page_size; }
 };
 
 // The K and V fragments of STEPS steps of 32 keys from key k00 on.  K: rows of two 16-key tiles
@@ -80,17 +84,17 @@ __device__ __forceinline__ void attn_load(AttnFragments<DH, STEPS, DV>& f, int k
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int key = min(k0 + 16 * t + r, last_key);
-      const int page = cache.pages[key / cache.page_size - cache.base_page];
+      const int page = cache.pages[cache.page_of(key) - cache.base_page];
       if (PADDED_KEYS) {
         const bf16_t* row = cache.k_base + (long)page * cache.page_stride +
-                            ((long)cache.kvh * cache.page_size + key % cache.page_size) * cache.key_dim;
+                            ((long)cache.kvh * cache.page_size + cache.place_of(key)) * cache.key_dim;
 #pragma unroll
         for (int kk = 0; kk < DH / 32; ++kk)
           f.k[st][t][kk] = *reinterpret_cast<const mfma_bf16x8*>(row + min(32 * kk + 8 * q, cache.key_dim - 8));
         continue;
       }
       const bf16_t* row = cache.k_base + (long)page * cache.page_stride +
-                          ((long)cache.kvh * cache.page_size + key % cache.page_size) * DH + 8 * q;
+                          ((long)cache.kvh * cache.page_size + cache.place_of(key)) * DH + 8 * q;
 #pragma unroll
       for (int kk = 0; kk < DH / 32; ++kk) f.k[st][t][kk] = *reinterpret_cast<const mfma_bf16x8*>(row + 32 * kk);
     }
@@ -98,8 +102,8 @@ __device__ __forceinline__ void attn_load(AttnFragments<DH, STEPS, DV>& f, int k
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int key = min(k0 + 16 * t + 4 * q, last_key & ~3);
-      page[t] = cache.pages[key / cache.page_size - cache.base_page];
-      offset[t] = key % cache.page_size;
+      page[t] = cache.pages[cache.page_of(key) - cache.base_page];
+      offset[t] = cache.place_of(key);
     }
 #pragma unroll
     for (int dt = 0; dt < DV / 16; ++dt) {

@@ -1657,11 +1657,34 @@ extern "C" int mi_fused_gemm_supported(int pro, int M, int K) {
 
 // Weights that the products behind the mixers read, in tiles of 16 features one behind the other.
 #define AHEAD_MOST 4
-#define AHEAD_BLOCKS 256        // workgroups that read them, a multiple of 8
-struct AheadWeight {
+#define AHEAD_BLOCKS 128        // workgroups that read them, a multiple of 8 (a step of 1 and of 8 rows with 64 / 128 / 256: 976 / 915 / 939 and 1,210 / 1,156 / 1,159 us)
+struct AheadWeight {           // as callers give it
   const void* at;
   long tiles, tile_bytes;
 };
+struct AheadTiles {            // pieces of a tile that a workgroup reads at once, and how far on its next one is
+  const void* at;
+  int tiles, tile_bytes, pieces, step_tiles, step_pieces;
+};
+
+// Division of a workgroup's number by a size of the launch: the upper half of a product where numbers and sizes are small
+// enough for it (n * d < 2^32), which the launch checks.
+struct FastDivide {
+  unsigned divisor, magic;     // magic 0: divide
+  __device__ __forceinline__ int operator()(int n) const {
+    return magic ? (int)__umulhi((unsigned)n, magic) : divisor == 1 ? n : n / (int)divisor;
+  }
+};
+static FastDivide fast_divide(long divisor, long numbers) {
+  FastDivide d = {(unsigned)divisor, 0};
+  if (divisor > 1 && numbers * divisor < (1L << 32)) d.magic = (unsigned)(((1UL << 32) + divisor - 1) / divisor);
+  return d;
+}
+
+// A word that is the same for the whole workgroup and that no launch in flight writes: through the scalar cache, so that the
+// loads behind it do not wait for it
+__device__ __forceinline__ int scalar_word(const int* at) { return *(const __attribute__((address_space(4))) int*)at; }
+__device__ __forceinline__ float scalar_word(const float* at) { return *(const __attribute__((address_space(4))) float*)at; }
 
 struct MixerParams {
   // the layer's projected row per token: [q | k | v | z | x B C (after conv) | dt], bfloat16
@@ -1695,6 +1718,9 @@ struct MixerParams {
   float* ssm_y;           // or float32 y before the gate (when a grouped norm follows)
   long out_ld;
   int attention_blocks, ahead_from;        // the attention's workgroups come first; those from ahead_from on read ahead
+  FastDivide by_splits, by_kv_heads, by_tiles, by_heads, by_group_heads;
+  int page_shift;                          // log2 of page_size, or -1
+  int heads_a_group;                       // query heads of a kv head
   // the context of a request is cut into runs of split_keys keys, one workgroup each; their
   // partial results [M, Hq, splits, DH + 2] = (maximum, normalizer, sums) are merged by mixer_merge_kernel
   int splits;
@@ -1704,7 +1730,7 @@ struct MixerParams {
 };
 
 struct MixerAhead {
-  AheadWeight weight[AHEAD_MOST];
+  AheadTiles weight[AHEAD_MOST];
 };
 
 // A word that another workgroup's cache must see, or may have written, without the fences that would write back and drop
@@ -1769,13 +1795,17 @@ __device__ __forceinline__ float merged_runs(const float* runs, int dh, int dim,
 // read of the runs take about 2 in the workgroups that the launch has anyway, beside the scan's).  The partial results are
 // stored through the die's cache, every wave waits for its stores, then the workgroup counts itself; whoever counts last
 // sees all of them with loads that pass the cache, and puts the counter back.  Nobody waits for another workgroup.
-template <int DH>
+//
+// POW2: pages of a power of two of cells (a division is 16 instructions, and this block a chain of waits and of instructions).
+template <int DH, bool POW2>
 __device__ void mixer_attention_block(const MixerParams& p, int block, int* pages_lds, float* cs,
                                       float* merge_lds, int* last_lds) {
-  const int G = p.Hq / p.Hkv;
-  const int split = block % p.splits;
-  const int kvh = (block / p.splits) % p.Hkv;
-  const long token = block / (p.splits * p.Hkv);
+  const int G = p.heads_a_group;
+  const int pair = p.by_splits(block), split = block - pair * p.splits;
+  const int token_number = p.by_kv_heads(pair), kvh = pair - token_number * p.Hkv;
+  const long token = token_number;
+  if (POW2) __builtin_assume(p.page_shift >= 0);
+  auto pages_before = [&](int key) { return POW2 ? key >> p.page_shift : key / p.page_size; };
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
   const int wave = tid / WAVE;
@@ -1791,8 +1821,8 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
   const bool rotate = p.inv_freq != nullptr;
   // (the position first: the page ids wait for it, the keys for them, and loads come back in the order they were
   // asked for; behind the query's rows, which the kernel before has just written on other dies, it would wait for them)
-  const int pos = p.positions[token];
-  const long cell = p.slot_mapping[token];
+  const int pos = scalar_word(p.positions + token);
+  const int cell = scalar_word(p.slot_mapping + token);
   mfma_bf16x8 q_own[DH / 32], q_pair[DH / 32];
   const bool has_head = n < G;
   const bf16_t* q_head = row + p.q_col + (kvh * G + (has_head ? n : 0)) * DH;
@@ -1814,7 +1844,7 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
   // ---- this workgroup's run of keys
   int first_key = 0;
   if (p.window > 0 && pos - p.window + 1 > 0) first_key = pos - p.window + 1;
-  const int base_key = (first_key / p.page_size) * p.page_size;       // a page edge
+  const int base_key = pages_before(first_key) * p.page_size;         // a page edge
   // the request's keys are cut into runs of split_keys; this workgroup takes the runs split, split + splits,
   // split + 2 splits, ... (a large step has fewer workgroups than runs: a workgroup that finds no keys costs
   // some 30 ns of a step's time, and a graph made for long contexts would launch hundreds of them)
@@ -1824,8 +1854,8 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
   auto stage_pages = [&](int run) {
     const int lo = base_key + run * p.split_keys;
     const int hi = min(lo + p.split_keys, pos + 1);
-    const int first_page = lo / p.page_size;
-    const int last_page = (hi - 1) / p.page_size;
+    const int first_page = pages_before(lo);
+    const int last_page = pages_before(hi - 1);
     for (int t = tid; t <= last_page - first_page; t += MX_THREADS) pages_lds[t] = table[first_page + t];
   };
   stage_pages(split);
@@ -1852,8 +1882,8 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
       const int j = tid < half ? tid : tid - half;
       k = tid < half ? k_raw * cs[j] - k_raw_pair * cs[half + j] : k_raw * cs[j] + k_raw_pair * cs[half + j];
     }
-    const long page = cell / p.page_size;
-    const int offset = (int)(cell - page * p.page_size);
+    const long page = pages_before(cell);
+    const int offset = cell - (int)page * p.page_size;
     p.k_base[page * p.page_stride + ((long)kvh * p.page_size + offset) * DH + tid] = (bf16_t)k;
     p.v_base[page * p.page_stride + ((long)kvh * DH + tid) * p.page_size + offset] = (bf16_t)v_raw;
   }
@@ -1900,7 +1930,8 @@ __device__ void mixer_attention_block(const MixerParams& p, int block, int* page
       cache.page_size = p.page_size;
       cache.kvh = kvh;
       cache.pages = pages_lds;
-      cache.base_page = run_lo / p.page_size;
+      cache.base_page = pages_before(run_lo);
+      if (POW2) cache.page_shift = p.page_shift;
       const int col_pos[1] = {has_head ? pos : -1};
       attend_keys<DH, 1, 2>(acc, q_frag, col_pos, p.window, p.scale, wave_lo, wave_hi, cache);
     }
@@ -1986,14 +2017,14 @@ __global__ void mixer_merge_kernel(MixerParams p, int dh) {
 // consecutive elements: two 16-byte state loads and one 16-byte load each of B and C.
 template <bool VECTOR, int RPT>
 __device__ void mixer_ssm_block(const MixerParams& p, int block) {
-  const int tile = block % p.p_tiles;
-  const int head = (block / p.p_tiles) % p.H;
-  const long token = block / (p.p_tiles * p.H);
-  const int R = p.R;
-  const int rows_per_round = MX_THREADS / R;
-  const int row_in_round = threadIdx.x / R;
-  const int r = threadIdx.x - row_in_round * R;
-  const int group = head / (p.H / p.G);
+  const int pair = p.by_tiles(block), tile = block - pair * p.p_tiles;
+  const int token_number = p.by_heads(pair), head = pair - token_number * p.H;
+  const long token = token_number;
+  const int R = p.R, shift = __builtin_ctz(R);                          // a power of two
+  const int rows_per_round = MX_THREADS >> shift;
+  const int row_in_round = threadIdx.x >> shift;
+  const int r = threadIdx.x & (R - 1);
+  const int group = p.by_group_heads(head);
   const int N = p.N;
   const bf16_t* row = p.u + token * p.u_ld;
   const bf16_t* b_row = row + p.x_col + p.H * p.P + group * N;
@@ -2005,7 +2036,8 @@ __device__ void mixer_ssm_block(const MixerParams& p, int block) {
   int pi[RPT];
   bool active[RPT];
   float* s_row[RPT];
-  const long slot_base = ((long)p.slot_ids[token] * p.H + head) * p.P;
+  const long slot_base = ((long)scalar_word(p.slot_ids + token) * p.H + head) * p.P;
+  const float dt_bias = scalar_word(p.dt_bias + head), rate = scalar_word(p.A + head), skip = scalar_word(p.D + head);
 #pragma unroll
   for (int j = 0; j < RPT; ++j) {
     pi[j] = (tile * RPT + j) * rows_per_round + row_in_round;
@@ -2031,9 +2063,8 @@ __device__ void mixer_ssm_block(const MixerParams& p, int block) {
     x_bits[j] = row[p.x_col + column];
     z_bits[j] = row[p.z_col + column];
   }
-  const float delta = softplus_f((float)dt_bits + p.dt_bias[head]);
-  const float decay = expf(delta * p.A[head]);
-  const float skip = p.D[head];
+  const float delta = softplus_f((float)dt_bits + dt_bias);
+  const float decay = expf(delta * rate);
 #pragma unroll
   for (int j = 0; j < RPT; ++j) {
     const long column = (long)head * p.P + (active[j] ? pi[j] : 0);
@@ -2079,38 +2110,40 @@ __device__ void mixer_ssm_block(const MixerParams& p, int block) {
 // the eight dies in turn), or, where the mixers' own bytes have pushed it out, in the memory-side cache.  Pieces of
 // MX_THREADS 16-byte words, dealt out to the die's workgroups in the order in which the products will read them.
 __device__ void mixer_ahead_block(const MixerAhead& p, int block) {
-  const int die = blockIdx.x % 8;
+  const int die = blockIdx.x % 8, first = block / 8;
   constexpr int PIECE = MX_THREADS * 16;
-  long u = block / 8;
 #pragma unroll
   for (int k = 0; k < AHEAD_MOST; ++k) {
-    const AheadWeight w = p.weight[k];
-    const long tiles = (w.tiles - die + 7) / 8;                          // of this die
-    const long pieces = (w.tile_bytes + PIECE - 1) / PIECE;
-    const long count = tiles * pieces;
-    for (; u < count; u += 4 * (AHEAD_BLOCKS / 8)) {
+    const AheadTiles w = p.weight[k];
+    const int tiles = (w.tiles - die + 7) / 8;                           // of this die
+    int tile = first / w.pieces, piece = first - tile * w.pieces;
+    while (tile < tiles) {
       floatx4 word[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const long item = min(u + j * (AHEAD_BLOCKS / 8), count - 1);
-        const long tile = item / pieces, at = (item - tile * pieces) * PIECE + threadIdx.x * 16;
-        word[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(w.at) + (die + 8 * tile) * w.tile_bytes + min(at, w.tile_bytes - 16));
+        const int at = min(piece * PIECE + (int)threadIdx.x * 16, w.tile_bytes - 16);
+        word[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(w.at) + (long)(die + 8 * min(tile, tiles - 1)) * w.tile_bytes + at);
+        tile += w.step_tiles;                                            // PEERS pieces on
+        piece += w.step_pieces;
+        if (piece >= w.pieces) {
+          piece -= w.pieces;
+          ++tile;
+        }
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) asm volatile("" ::"v"(word[j]));
     }
-    u = block / 8;
   }
 }
 
-template <int DH, bool AHEAD>
+template <int DH, bool POW2, bool AHEAD>
 __device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const MixerAhead& ahead) {
   __shared__ int pages_lds[MX_MAX_PAGES];
   __shared__ float cs[DH];
   __shared__ float merge_lds[MX_WAVES * 8 * (DH + 2)];
   __shared__ int last_lds;
   if ((int)blockIdx.x < p.attention_blocks)
-    mixer_attention_block<DH>(p, blockIdx.x, pages_lds, cs, merge_lds, &last_lds);
+    mixer_attention_block<DH, POW2>(p, blockIdx.x, pages_lds, cs, merge_lds, &last_lds);
   else if (AHEAD && (int)blockIdx.x >= p.ahead_from)
     mixer_ahead_block(ahead, blockIdx.x - p.ahead_from);
   else if (!p.vector_scan)
@@ -2125,15 +2158,15 @@ __device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const M
     mixer_ssm_block<true, 8>(p, blockIdx.x - p.attention_blocks);
 }
 
-template <int DH>
+template <int DH, bool POW2>
 __global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p) {
-  mixer_decode_block<DH, false>(p, MixerAhead{});
+  mixer_decode_block<DH, POW2, false>(p, MixerAhead{});
 }
 
 // (a kernel of its own: 64 rows pay 1.6 us a launch for the question alone)
-template <int DH>
+template <int DH, bool POW2>
 __global__ void __launch_bounds__(MX_THREADS) mixer_decode_ahead_kernel(MixerParams p, MixerAhead ahead) {
-  mixer_decode_block<DH, true>(p, ahead);
+  mixer_decode_block<DH, POW2, true>(p, ahead);
 }
 
 // Keys of one attention workgroup (a run).  Long runs pay the start of a workgroup (position, page ids,
@@ -2272,21 +2305,37 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
   if (!partial || partial_floats < (long)M * Hq * p.splits * (dh + 2)) return ERR_BAD_ARGUMENT;
   p.partial = partial;
   p.arrived = merge ? arrived : nullptr;
+  p.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
+  p.heads_a_group = group;
+  p.by_splits = fast_divide(p.splits, (long)Hkv * M * p.splits);
+  p.by_kv_heads = fast_divide(Hkv, (long)Hkv * M);
+  p.by_tiles = fast_divide(p.p_tiles, (long)p.p_tiles * H * M);
+  p.by_heads = fast_divide(H, (long)H * M);
+  p.by_group_heads = fast_divide(H / G, H);
   p.attention_blocks = Hkv * M * p.splits;
   const long total = (long)p.attention_blocks + (long)p.p_tiles * H * M;
   if (total > 0x7fffffffL - AHEAD_BLOCKS - 8) return ERR_UNSUPPORTED_SIZE;
   if (ahead_count < 0 || ahead_count > AHEAD_MOST || (ahead_count && !ahead)) return ERR_BAD_ARGUMENT;
   MixerAhead reads = {};
+  for (int k = 0; k < AHEAD_MOST; ++k) reads.weight[k].pieces = 1;
   p.ahead_from = (int)total;
   for (int k = 0; k < ahead_count; ++k) {
-    reads.weight[k] = ahead[k];
-    if (!ahead[k].at || (uintptr_t)ahead[k].at % 16 || ahead[k].tiles <= 0 || ahead[k].tile_bytes <= 0 || ahead[k].tile_bytes % 16)
+    if (!ahead[k].at || (uintptr_t)ahead[k].at % 16 || ahead[k].tiles <= 0 || ahead[k].tile_bytes <= 0 || ahead[k].tile_bytes % 16 ||
+        ahead[k].tiles > (1 << 28) || ahead[k].tile_bytes > (1 << 28))
       return ERR_BAD_ARGUMENT;
+    const int pieces = (int)((ahead[k].tile_bytes + MX_THREADS * 16 - 1) / (MX_THREADS * 16)), peers = AHEAD_BLOCKS / 8;
+    reads.weight[k] = {ahead[k].at, (int)ahead[k].tiles, (int)ahead[k].tile_bytes, pieces, peers / pieces, peers % pieces};
   }
-  if (ahead_count && dh == 64) mixer_decode_ahead_kernel<64><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads);
-  else if (ahead_count) mixer_decode_ahead_kernel<128><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads);
-  else if (dh == 64) mixer_decode_kernel<64><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
-  else mixer_decode_kernel<128><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);
+#define MIXER(DH_, POW2_)                                                                                                  \
+  do {                                                                                                                     \
+    if (ahead_count) mixer_decode_ahead_kernel<DH_, POW2_><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads); \
+    else mixer_decode_kernel<DH_, POW2_><<<(unsigned)total, MX_THREADS, 0, stream>>>(p);                                   \
+  } while (0)
+  if (dh == 64 && p.page_shift >= 0) MIXER(64, true);
+  else if (dh == 64) MIXER(64, false);
+  else if (p.page_shift >= 0) MIXER(128, true);
+  else MIXER(128, false);
+#undef MIXER
   RETURN_IF_LAUNCH_FAILED();
   if (!merge || p.splits == 1 || p.arrived) return 0;
   const dim3 merge_grid(M, Hq);

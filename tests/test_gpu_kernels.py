@@ -1570,17 +1570,19 @@ def test_output_projection_that_merges_the_runs_of_keys(ops, Hq, Hkv, dh, E, N_o
     close(want, product, dtype, max(1.0, product.abs().max().item()))
 
 
-@pytest.mark.parametrize("Hq, Hkv, dh, window, most, lengths", [
-    (8, 2, 64, None, 0, [1, 17, 64, 65, 300, 1500, 2, 2060]), (8, 2, 64, 1100, 0, [1, 700, 1500, 2060]),
-    (12, 2, 128, None, 0, [700, 3]), (4, 4, 64, None, 0, [5000, 9000, 3] + [40 + lane for lane in range(13)]),
-    (2, 2, 128, None, 9000, [257 + 64 * lane for lane in range(40)]), (5, 1, 64, None, 12000, [2100])])
-def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, most, lengths):
+@pytest.mark.parametrize("Hq, Hkv, dh, window, most, page_size, lengths", [
+    (8, 2, 64, None, 0, 24, [1, 23, 24, 25, 300, 1500, 2060]), (6, 3, 128, 900, 0, 40, [700, 3, 2100]),
+    (8, 2, 64, None, 0, 16, [1, 17, 64, 65, 300, 1500, 2, 2060]), (8, 2, 64, 1100, 0, 16, [1, 700, 1500, 2060]),
+    (12, 2, 128, None, 0, 16, [700, 3]), (4, 4, 64, None, 0, 16, [5000, 9000, 3] + [40 + lane for lane in range(13)]),
+    (2, 2, 128, None, 9000, 16, [257 + 64 * lane for lane in range(40)]), (5, 1, 64, None, 12000, 16, [2100])])
+def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, most, page_size, lengths):
     """With counters the runs of keys are merged by whichever workgroup ends last: the bits of the merge kernel, launch
     after launch with the same counters, which are zeros again; contexts of one run, of more runs than a merge asks for at
-    once, of runs that one workgroup walks over, a window of several runs, a launch made for far longer contexts.  And
+    once, of runs that one workgroup walks over, a window of several runs, a launch made for far longer contexts, pages of no
+    power of two (also against the plain version).  And
     the same bits where the launch reads weights ahead (of one tile, of tiles that are no multiple of 8)."""
     dtype = torch.bfloat16
-    H, P, N, G, page_size = 4, 16, 32, 1, 16
+    H, P, N, G = 4, 16, 32, 1
     E, M = H * P, len(lengths)
     pool, table = paged_setup(lengths, page_size, Hkv, dh, dtype, seed=23)
     for lane, length in enumerate(lengths):
@@ -1612,6 +1614,15 @@ def test_mixer_decode_merges_its_runs_in_the_launch(ops, Hq, Hkv, dh, window, mo
 
     want = run(None)
     assert torch.isfinite(want.float()).all()
+    if page_size & (page_size - 1):
+        host, plain = pool.clone(), torch.empty(M, Hq * dh + E, dtype=dtype)
+        ref_ops.mixer_decode(u.cpu(), num_heads=Hq, num_kv_heads=Hkv, head_dim=dh, q_col=q_col, k_col=k_col, v_col=v_col,
+                             inv_freq=inv_freq.cpu(), rotary_dim=dh, k_cache=views(host, page_size)[0], v_cache=views(host, page_size)[1],
+                             block_tables=table, positions=positions.cpu(), slot_mapping=slot_mapping.cpu(), scale=0.13, window=window,
+                             max_seq_len=max(lengths) + 5, ssm_heads=H, ssm_head_dim=P, state_size=N, num_groups=G, z_col=z_col,
+                             x_col=x_col, dt_col=dt_col, dt_bias=vectors[0], A=vectors[1], D=vectors[2],
+                             ssm_state=rand(M, H, P, N, seed=611, scale=0.5), slot_ids=i32(list(range(M))), out=plain, ssm_y=None)
+        close(want, plain, dtype, 2.0)
     for _ in range(3):
         assert torch.equal(run(arrived), want) and not arrived.any()
     weights = [ops.fragment_order(torch.ones(rows, width, dtype=dtype, device=DEV)) for rows, width in ((12, 64), (4120, 1024), (136, 96), (64, 4608))]
