@@ -121,12 +121,12 @@ FORCE_MERGE_LATER: Optional[bool] = None  # True: the output projection merges, 
 _padding_wins: Dict[tuple, tuple] = {}
 # The mixers of a small step wait for round trips and leave the memory idle, so their launch also brings the weights of the
 # products behind them, the next layer's first one included, into the caches, in the order in which they are read: as many
-# as AHEAD_BYTES hold (the dies' caches together) beside the states that the step reads and writes.  A step of the 0.5B
-# shape (25 MB a layer, 1.6 MB of states a row) in us without | out and gate-up | and down | and the next layer's input, at
-# contexts of 2,048: 1 row 1,034 | 978 | 962 | 947, 4 rows 1,096 | 1,044 | 1,033 | 1,036, 8 rows 1,203 | 1,171 | 1,153 | 1,184, 12 rows
-# 1,369 | 1,336 | 1,361 | 1,408, 16 rows 1,424 | 1,437 | 1,459 | 1,505; of 300: 1 row 1,003 | 947 | 924 | 907, 8 rows 1,148 | 1,084 | 1,113 |
-# 1,150, 16 rows 1,305 | 1,264 | 1,282 | 1,318.  The 7B shape's 28 MB of output projection: 1 row 1,098 | 1,084, 4 rows 1,196 | 1,225.
-AHEAD_BYTES = 32 << 20
+# as AHEAD_BYTES hold (of the dies' caches of 32 MB together) beside the states that the step reads.  A step of the 0.5B
+# shape (25 MB a layer, 0.8 MB of states a row) in us without | out and gate-up | and down | and the next layer's input, at
+# contexts of 2,048: 1 row 1,018 | 956 | 937 | 915, 4 rows 1,071 | 1,036 | 1,028 | 1,025, 8 rows 1,170 | 1,159 | 1,146 | 1,167, 12 rows
+# 1,328 | 1,290 | 1,282 | 1,321, 16 rows 1,367 | 1,329 | 1,325 | 1,374; of 300: 1 row 985 | 920 | 902 | 879, 8 rows 1,123 | 1,080 | 1,074 |
+# 1,116, 16 rows 1,290 | 1,266 | 1,266 | 1,302.  (The 7B shape's 28 MB of output projection: 1 row 1,098 | 1,084, 4 rows 1,196 | 1,225: left out.)
+AHEAD_BYTES = 28 << 20
 # A projection whose result joins the residual stream can add it there itself (float32, in place) and leave, beside
 # the stream, its rows times the next norm's weight in bfloat16 with the partial sums of their squares; the product
 # behind that norm then reads those rows and multiplies its float32 sums by 1 / sqrt(mean square + eps): the norm
@@ -349,7 +349,7 @@ def register_mixer_kernel(*kinds: str):
     ``conv_state(caches)`` and ``run(u, step, caches, mixed, merge=True)``; a kernel with ``merged_columns`` (how
     many the attended heads are, the first columns of ``mixed``) returns, when called with ``merge=False``, their runs of
     keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; ``step_tables()``: tables it reads in every step;
-    ``ahead``: weights that its launch may bring into the caches, if it says the ``state_bytes`` that it moves a row."""
+    ``ahead``: weights that its launch may bring into the caches, if it says the ``state_bytes`` that it reads a row."""
     def decorate(factory):
         _MIXER_KERNELS[tuple(kinds)] = factory
         return factory
@@ -999,7 +999,7 @@ class AttentionMamba2Step:
         self.x_col = second + s.inner_size
         self.dt_col = self.x_col + s.conv_width
         self.attended_width = self.merged_columns = q_width
-        self.state_bytes = 2 * 4 * s.num_heads * s.head_dim * s.state_size         # a row's states, read and written
+        self.state_bytes = 4 * s.num_heads * s.head_dim * s.state_size         # that a row reads
         self.inv_freq, self.rotary_dim = self.attention.position.fused_rotation()
         self.conv = dict(lo=self.x_col, hi=self.dt_col, taps=s.conv_kernel, weight=self.mamba.conv_weight,
                          bias=self.mamba.conv_bias)
