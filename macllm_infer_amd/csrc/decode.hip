@@ -50,6 +50,7 @@
 // mamba2.hip; these kernels only change what runs together.
 #include "common.h"
 #include "attn_mfma.h"
+#include "read_ahead.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
@@ -1655,17 +1656,7 @@ extern "C" int mi_fused_gemm_supported(int pro, int M, int K) {
 #define MX_SCAN_PER_THREAD 8
 #define MX_FEW_BLOCKS 512       // state-space workgroups of a step up to which each takes one row per thread group
 
-// Weights that the products behind the mixers read, in tiles of 16 features one behind the other.
-#define AHEAD_MOST 4
-#define AHEAD_BLOCKS 128        // workgroups that read them, a multiple of 8 (a step of 1 and of 8 rows with 64 / 128 / 256: 976 / 915 / 939 and 1,210 / 1,156 / 1,159 us)
-struct AheadWeight {           // as callers give it
-  const void* at;
-  long tiles, tile_bytes;
-};
-struct AheadTiles {            // pieces of a tile that a workgroup reads at once, and how far on its next one is
-  const void* at;
-  int tiles, tile_bytes, pieces, step_tiles, step_pieces;
-};
+#define AHEAD_BLOCKS 128        // workgroups that read weights ahead, a multiple of 8 (a step of 1 and of 8 rows with 64 / 128 / 256: 976 / 915 / 939 and 1,210 / 1,156 / 1,159 us)
 
 // Division of a workgroup's number by a size of the launch: the upper half of a product where numbers and sizes are small
 // enough for it (n * d < 2^32), which the launch checks.
@@ -1727,10 +1718,6 @@ struct MixerParams {
   int split_keys;
   float* partial;
   int* arrived;           // [M, Hkv] zeros, which the launch leaves zero again: the runs are merged inside it; or null
-};
-
-struct MixerAhead {
-  AheadTiles weight[AHEAD_MOST];
 };
 
 // A word that another workgroup's cache must see, or may have written, without the fences that would write back and drop
@@ -2104,40 +2091,8 @@ __device__ void mixer_ssm_block(const MixerParams& p, int block) {
   }
 }
 
-// The mixers of a small step wait for round trips and leave the memory idle, and the four products behind them are as long
-// as the way of their weights from memory: these workgroups read the weights meanwhile and drop them.  What they leave is
-// in the caches: a tile is read on the die whose cache the product's workgroup of that number will ask (workgroups go to
-// the eight dies in turn), or, where the mixers' own bytes have pushed it out, in the memory-side cache.  Pieces of
-// MX_THREADS 16-byte words, dealt out to the die's workgroups in the order in which the products will read them.
-__device__ void mixer_ahead_block(const MixerAhead& p, int block) {
-  const int die = blockIdx.x % 8, first = block / 8;
-  constexpr int PIECE = MX_THREADS * 16;
-#pragma unroll
-  for (int k = 0; k < AHEAD_MOST; ++k) {
-    const AheadTiles w = p.weight[k];
-    const int tiles = (w.tiles - die + 7) / 8;                           // of this die
-    int tile = first / w.pieces, piece = first - tile * w.pieces;
-    while (tile < tiles) {
-      floatx4 word[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int at = min(piece * PIECE + (int)threadIdx.x * 16, w.tile_bytes - 16);
-        word[j] = *reinterpret_cast<const floatx4*>(reinterpret_cast<const char*>(w.at) + (long)(die + 8 * min(tile, tiles - 1)) * w.tile_bytes + at);
-        tile += w.step_tiles;                                            // PEERS pieces on
-        piece += w.step_pieces;
-        if (piece >= w.pieces) {
-          piece -= w.pieces;
-          ++tile;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) asm volatile("" ::"v"(word[j]));
-    }
-  }
-}
-
 template <int DH, bool POW2, bool AHEAD>
-__device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const MixerAhead& ahead) {
+__device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const AheadList& ahead) {
   __shared__ int pages_lds[MX_MAX_PAGES];
   __shared__ float cs[DH];
   __shared__ float merge_lds[MX_WAVES * 8 * (DH + 2)];
@@ -2145,7 +2100,7 @@ __device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const M
   if ((int)blockIdx.x < p.attention_blocks)
     mixer_attention_block<DH, POW2>(p, blockIdx.x, pages_lds, cs, merge_lds, &last_lds);
   else if (AHEAD && (int)blockIdx.x >= p.ahead_from)
-    mixer_ahead_block(ahead, blockIdx.x - p.ahead_from);
+    read_ahead_block<MX_THREADS>(ahead, blockIdx.x - p.ahead_from);
   else if (!p.vector_scan)
     mixer_ssm_block<false, 1>(p, blockIdx.x - p.attention_blocks);
   else if (p.rows_per_thread == 1)
@@ -2160,12 +2115,12 @@ __device__ __forceinline__ void mixer_decode_block(const MixerParams& p, const M
 
 template <int DH, bool POW2>
 __global__ void __launch_bounds__(MX_THREADS) mixer_decode_kernel(MixerParams p) {
-  mixer_decode_block<DH, POW2, false>(p, MixerAhead{});
+  mixer_decode_block<DH, POW2, false>(p, AheadList{});
 }
 
 // (a kernel of its own: 64 rows pay 1.6 us a launch for the question alone)
 template <int DH, bool POW2>
-__global__ void __launch_bounds__(MX_THREADS) mixer_decode_ahead_kernel(MixerParams p, MixerAhead ahead) {
+__global__ void __launch_bounds__(MX_THREADS) mixer_decode_ahead_kernel(MixerParams p, AheadList ahead) {
   mixer_decode_block<DH, POW2, true>(p, ahead);
 }
 
@@ -2314,18 +2269,11 @@ extern "C" int mi_mixer_decode(const void* u, long u_ld, int M, int Hq, int Hkv,
   p.by_group_heads = fast_divide(H / G, H);
   p.attention_blocks = Hkv * M * p.splits;
   const long total = (long)p.attention_blocks + (long)p.p_tiles * H * M;
-  if (total > 0x7fffffffL - AHEAD_BLOCKS - 8) return ERR_UNSUPPORTED_SIZE;
-  if (ahead_count < 0 || ahead_count > AHEAD_MOST || (ahead_count && !ahead)) return ERR_BAD_ARGUMENT;
-  MixerAhead reads = {};
-  for (int k = 0; k < AHEAD_MOST; ++k) reads.weight[k].pieces = 1;
+  if (total > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
+  if (total > 0x7fffffffL - AHEAD_BLOCKS) ahead_count = 0;
+  AheadList reads;
+  if (!read_ahead_list(reads, ahead, ahead_count, AHEAD_BLOCKS, MX_THREADS)) return ERR_BAD_ARGUMENT;
   p.ahead_from = (int)total;
-  for (int k = 0; k < ahead_count; ++k) {
-    if (!ahead[k].at || (uintptr_t)ahead[k].at % 16 || ahead[k].tiles <= 0 || ahead[k].tile_bytes <= 0 || ahead[k].tile_bytes % 16 ||
-        ahead[k].tiles > (1 << 28) || ahead[k].tile_bytes > (1 << 28))
-      return ERR_BAD_ARGUMENT;
-    const int pieces = (int)((ahead[k].tile_bytes + MX_THREADS * 16 - 1) / (MX_THREADS * 16)), peers = AHEAD_BLOCKS / 8;
-    reads.weight[k] = {ahead[k].at, (int)ahead[k].tiles, (int)ahead[k].tile_bytes, pieces, peers / pieces, peers % pieces};
-  }
 #define MIXER(DH_, POW2_)                                                                                                  \
   do {                                                                                                                     \
     if (ahead_count) mixer_decode_ahead_kernel<DH_, POW2_><<<(unsigned)total + AHEAD_BLOCKS, MX_THREADS, 0, stream>>>(p, reads); \

@@ -21,6 +21,7 @@
 // two products, hence the transposed copies.
 // (reference recurrence: crates/macllm-kernels/src/mamba2.rs:259-288; the reference scans token by token.)
 #include "attn_prefill.h"
+#include "read_ahead.h"
 #include "rope_rows.h"
 
 typedef __bf16 s_bf16x8 __attribute__((ext_vector_type(8)));
@@ -227,7 +228,10 @@ struct PromptBeside {
   int window, max_seq_len;
   void* out;
   long out_ld;
+  AheadWeight ahead[AHEAD_MOST];   // weights that the launches behind read, brought into the caches by the second launch
+  int ahead_count;
 };
+#define BESIDE_AHEAD_BLOCKS 128    // by so many workgroups, a multiple of 8
 
 // prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch (their code inlined in
 // both instances: as a function called from two kernels the conv took 30 us where it takes 16); with BESIDE the rows
@@ -1095,10 +1099,14 @@ ssd_single_beside_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16
                   const float* __restrict__ delta, const float* __restrict__ cum, const float* __restrict__ D,
                   const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y, long y_ld,
                   const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated, long gated_ld, const SsdSingle one,
-                         int n_chunks, int scan_groups, int passes, const PromptBeside beside) {
+                         int n_chunks, int scan_groups, int passes, int ahead_from, const PromptBeside beside, const AheadList ahead) {
   extern __shared__ __align__(16) unsigned char scan_smem[];
   if ((int)blockIdx.x < scan_groups) {
     ssd_single_block<NK, PT>(scan_smem, blockIdx.x % n_chunks, blockIdx.x / n_chunks, xbc, xbc_ld, TT, E, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld, one);
+    return;
+  }
+  if ((int)blockIdx.x >= ahead_from) {
+    read_ahead_block<SSD_SCAN_WAVES * WAVE>(ahead, blockIdx.x - ahead_from);
     return;
   }
   const int index = blockIdx.x - scan_groups;
@@ -1151,8 +1159,10 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
       const int passes = (beside->Hq / beside->Hkv + nset - 1) / nset;
       const long all = (long)grid.x * grid.y + 4L * beside->n_tiles * beside->Hkv * passes;
       if (all > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
+      AheadList ahead;
+      if (!read_ahead_list(ahead, beside->ahead, beside->ahead_count, BESIDE_AHEAD_BLOCKS, SSD_SCAN_WAVES * WAVE)) return ERR_BAD_ARGUMENT;
       const int scan_groups = (int)(grid.x * grid.y);
-      const unsigned groups = (unsigned)all;
+      const unsigned groups = (unsigned)all + (beside->ahead_count && all < 0x7fffffffL - BESIDE_AHEAD_BLOCKS ? BESIDE_AHEAD_BLOCKS : 0);
 #define BESIDE_CASE(DH_, NSET_)                                                                                             \
   if (beside->dh == DH_ && nset == NSET_) {                                                                                 \
     static bool told[64] = {};                                                                                              \
@@ -1160,7 +1170,7 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
     const int code = allow_lds(ssd_single_beside_kernel<NK, PT, DH_, NSET_>, both, told);                                   \
     if (code) return code;                                                                                                  \
     ssd_single_beside_kernel<NK, PT, DH_, NSET_><<<groups, SSD_SCAN_WAVES * WAVE, both, stream>>>(                          \
-        SINGLE_ARGUMENTS, (int)grid.x, scan_groups, passes, *beside);                                                       \
+        SINGLE_ARGUMENTS, (int)grid.x, scan_groups, passes, (int)all, *beside, ahead);                                                       \
     return 0;                                                                                                               \
   }
       BESIDE_CASE(64, 2) BESIDE_CASE(64, 3) BESIDE_CASE(64, 4) BESIDE_CASE(128, 2)

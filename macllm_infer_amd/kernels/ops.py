@@ -2000,13 +2000,23 @@ def ssd_supported(chunk_size: int, head_dim: int, state_size: int, num_groups: i
     return bool(_fn("ssd", "mi_ssd_supported")(chunk_size, head_dim, state_size, num_groups, inner_size))
 
 
+AHEAD_MOST = 4             # weights that a launch brings into the caches at most (read_ahead.h)
+
+
+def _weights_ahead(weights: Sequence[torch.Tensor], what: str):
+    """(address, tiles, bytes of a tile) of weights in fragment order, as the kernels take them."""
+    _need(len(weights) <= AHEAD_MOST and all(w.is_cuda and w.is_contiguous() and w.dim() == 5 for w in weights),
+          f"{what}: up to four weights in fragment order ahead")
+    return (_c_long * (3 * AHEAD_MOST))(*(number for w in weights for number in (w.data_ptr(), w.shape[0], w[0].numel() * w.element_size())))
+
+
 class _PromptBeside(ctypes.Structure):
     _fields_ = [("qkv", _c_ptr), ("ld", _c_long), ("T", _c_int), ("Hq", _c_int), ("Hkv", _c_int), ("dh", _c_int),
                 ("positions", _c_ptr), ("inv_freq", _c_ptr), ("rotary_dim", _c_int), ("slot_mapping", _c_ptr),
                 ("k_base", _c_ptr), ("v_base", _c_ptr), ("page_stride", _c_long), ("page_size", _c_int),
                 ("block_tables", _c_ptr), ("max_pages", _c_int), ("tiles", _c_ptr), ("n_tiles", _c_int),
                 ("cu_seqlens", _c_ptr), ("start_pos", _c_ptr), ("scale", _c_float), ("window", _c_int),
-                ("max_seq_len", _c_int), ("out", _c_ptr), ("out_ld", _c_long)]
+                ("max_seq_len", _c_int), ("out", _c_ptr), ("out_ld", _c_long), ("ahead", _c_long * (3 * 4)), ("ahead_count", _c_int)]
 
 
 @dataclass
@@ -2032,6 +2042,7 @@ class PromptBeside:
     out: torch.Tensor
     max_seq_len: int
     sizes: Optional[tuple]
+    ahead: Sequence[torch.Tensor] = ()         # weights in fragment order that the launches behind read: see ``mixer_decode``
 
     def fits(self, longest: int, ssm_state: torch.Tensor, chunk_size: int) -> bool:
         """Whether ``ssd_prefill`` of a step with lanes of up to ``longest`` tokens takes this attention in its two
@@ -2077,7 +2088,7 @@ class PromptBeside:
                              page_size, _p(self.block_tables), self.block_tables.shape[1],
                              _p(self.query_tiles), self.query_tiles.shape[0], _p(self.cu_seqlens), _p(self.start_pos),
                              float(self.scale), _span(self.window, None, "prefill_attention"), int(self.max_seq_len or 0),
-                             _p(self.out), out_ld)
+                             _p(self.out), out_ld, _weights_ahead(self.ahead, "prompt beside"), len(self.ahead))
 
 
 def ssd_prefill(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A: torch.Tensor, D: torch.Tensor,
@@ -2462,9 +2473,6 @@ def mixer_runs(M: int, num_kv_heads: int, page_size: int, span: int, head_dim: i
     return run_keys.value, runs.value
 
 
-AHEAD_MOST = 4             # weights that mixer_decode brings into the caches at most (decode.hip)
-
-
 def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim: int, q_col: int, k_col: int,
                  v_col: int, inv_freq: Optional[torch.Tensor], rotary_dim: int, k_cache: torch.Tensor,
                  v_cache: torch.Tensor, block_tables: torch.Tensor, positions: torch.Tensor,
@@ -2511,9 +2519,7 @@ def mixer_decode(u: torch.Tensor, *, num_heads: int, num_kv_heads: int, head_dim
     if arrived is not None:
         _i32(arrived, "arrived")
         _need(arrived.numel() >= M * num_kv_heads, "mixer_decode: one counter per token and kv head")
-    _need(len(ahead) <= AHEAD_MOST and all(w.is_cuda and w.is_contiguous() and w.dim() == 5 for w in ahead),
-          "mixer_decode: up to four weights in fragment order ahead")
-    weights = (_c_long * (3 * AHEAD_MOST))(*(number for w in ahead for number in (w.data_ptr(), w.shape[0], w[0].numel() * w.element_size())))
+    weights = _weights_ahead(ahead, "mixer_decode")
     span = max(1, int(max_seq_len)) if not window else window + page_size
     run_keys, runs = mixer_runs(M, num_kv_heads, page_size, span, head_dim)        # the launcher's own rule
     partial = torch.empty((M * num_heads * runs * (head_dim + 2),), dtype=torch.float32, device=u.device)

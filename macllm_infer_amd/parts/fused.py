@@ -673,15 +673,16 @@ class LayerFusion:
             return True
         return False
 
-    def _mix_each(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, order=None) -> None:
-        if order is None and self._mix_side_by_side(u, step, caches, mixed):
+    def _mix_each(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, order=None, ahead=()) -> None:
+        if order is None and self._mix_side_by_side(u, step, caches, mixed, ahead):
             return
         for index in (range(len(self.mixers)) if order is None else order):
             (lo, hi), (mixed_lo, mixed_hi) = self.in_cols[index], self.mixed_cols[index]
             self.mixers[index].mix(u[:, lo:hi], step, caches[self.names[index]], mixed[:, mixed_lo:mixed_hi])
 
-    def _mix_side_by_side(self, u: torch.Tensor, step, caches, mixed: torch.Tensor) -> bool:
-        """Short portions: an attention mixer's launches inside those of a state-space mixer (False: nothing was done)."""
+    def _mix_side_by_side(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, ahead=()) -> bool:
+        """Short portions: an attention mixer's launches inside those of a state-space mixer (False: nothing was done), which
+        bring the weights ``ahead`` into the caches."""
         if len(self.mixers) != 2 or step.max_query_len == 1:
             return False
         first, second = self.mixers
@@ -693,6 +694,7 @@ class LayerFusion:
         beside = make(*rows[0])
         if beside is None or not takes(*rows[1], beside):
             return False
+        beside.ahead = ahead
         second.mix(*rows[1], beside=beside)
         return True
 
@@ -813,12 +815,12 @@ class LayerFusion:
                      and self._merges_later(kernel, step, caches))
             attended = kernel.run(u, step, caches, mixed, merge=not later, ahead=self._read_ahead(residual, kernel, M, bucket))
         else:
-            self._mix_each(u, step, caches, mixed)
+            self._mix_each(u, step, caches, mixed, ahead=self._read_ahead(residual, self.kernel, step.num_lanes, bucket))
         self._after_the_mixers(residual, mixed, attended, M, bucket)
 
-    def _read_ahead(self, residual: Residual, kernel, M: int, bucket: int) -> list:
+    def _read_ahead(self, residual: Residual, kernel, lanes: int, bucket: int) -> list:
         """The weights of the products behind the mixers that the mixers' launch brings into the caches."""
-        room = AHEAD_BYTES - M * getattr(kernel, "state_bytes", AHEAD_BYTES)
+        room = AHEAD_BYTES - lanes * getattr(kernel, "state_bytes", AHEAD_BYTES)
         products = [(self.library_out[bucket], self.f_out)]
         if self.gate_up is not None:
             products += [(self.library_gate_up[bucket], self.f_gate_up), (self.library_down[bucket], self.f_down)]

@@ -867,6 +867,34 @@ def test_the_output_projection_may_merge_the_runs_of_keys(monkeypatch):
         assert torch.equal(rows, results[False, False]), key
 
 
+@pytest.mark.parametrize("prompt", [5, 37, 64])
+def test_weights_read_ahead_change_nothing(monkeypatch, prompt):
+    """Short prompts and single tokens whose mixers' launches bring the next products' weights into the caches, launched and
+    replayed: the logits of an engine that reads nothing ahead, bit for bit."""
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.parts import fused
+    from macllm_infer_amd.weights.random_init import random_tensors
+    config = FalconH1Config.from_dict(dict(tiny_configs.TINY_C, hidden_size=256, num_hidden_layers=3, num_attention_heads=8,
+                                           num_key_value_heads=2, head_dim=64, intermediate_size=416, mamba_n_heads=6, mamba_d_head=64,
+                                           mamba_d_ssm=384, mamba_d_state=128, mamba_n_groups=1, mamba_chunk_size=128,
+                                           max_position_embeddings=512))
+    tensors = random_tensors(config, 6, torch.bfloat16, "unit")
+    results = {}
+    for room in (0, 28 << 20):
+        monkeypatch.setattr(fused, "AHEAD_BYTES", room)
+        engine = Engine(config=config, tensors=tensors, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=2048,
+                        max_active_sequences=4, measured_paths=False)
+        rows = []
+        for name in range(4):                        # the third prompt of a size is replayed
+            engine.add_request(name)
+            rows.append(engine.step([Lane(name, tokens_for(config.vocab_size, prompt, 40 + name), [prompt - 1])]).float().cpu())
+        for turn in range(4):
+            rows.append(engine.step([Lane(name, [7 + turn], [0]) for name in range(1 + turn)]).float().cpu())
+        results[room] = torch.cat(rows)
+    assert torch.equal(results[0], results[28 << 20]) and torch.isfinite(results[0]).all()
+
+
 def test_graphs_come_in_buckets_of_context_length():
     """A model that allows long contexts: a short request decodes through a graph made for 2,048
     tokens, a longer one through a graph made for 4,096 (wider block tables, more runs of keys),
