@@ -847,7 +847,8 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
     for (int w = 0; w < WAVES; ++w) squares += parts[w][mine * 16 + r];
     const float mean = squares * p.ssq_inverse_width + p.ssq_eps;
     float inverse = __builtin_amdgcn_rsqf(mean);
-    inverse = inverse * (1.5f - 0.5f * mean * inverse * inverse);         // (a step of Newton's: as close as 1 / sqrtf)
+    const float closer = inverse * (1.5f - 0.5f * mean * inverse * inverse);           // (a step of Newton's: as close as 1 / sqrtf,
+    inverse = mean > 0.f && mean < INFINITY ? closer : inverse;                        // whose limits at 0 and infinity it has not)
     v *= inverse;
   }
   if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + n_safe);
