@@ -54,6 +54,7 @@
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 #define FG_PAD 8
@@ -681,11 +682,13 @@ __device__ __forceinline__ float quarters_sum(float v) {
   return __builtin_bit_cast(float, low) + __builtin_bit_cast(float, high);
 }
 
-// v of the lane 32 further, in the lanes below 32
-__device__ __forceinline__ float upper_half(float v) {
-  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
-  const unsigned high = halves[1];
-  return __builtin_bit_cast(float, high);
+// lower: a of the lanes below 32 where they are, b of the lanes below 32 in the lanes above; upper: a of the lanes above 32 in the
+// lanes below, b of those above where they are
+__device__ __forceinline__ void exchange_halves(float a, float b, float& lower, float& upper) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned low = halves[0], high = halves[1];
+  lower = __builtin_bit_cast(float, low);
+  upper = __builtin_bit_cast(float, high);
 }
 
 // v * v, rounded before anything is added to it (fused_gemm_kernel's squares pass through LDS)
@@ -882,19 +885,16 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
     *reinterpret_cast<floatx4*>(h_at) = updated;
     if (p.res_hb) *reinterpret_cast<bf16x4_t*>(p.res_hb + row * p.res_hb_ld + n) = rows;
   } else if (EPI == EPI_SWIGLU) {
-    // a tile is 8 gate features, then the 8 up features of the same columns: lanes q = 0, 1 take theirs from q + 2
-    floatx4 up;
+    // a tile is 8 gate features, then the 8 up features of the same columns: lane q < 2 holds four gates, lane q + 2 their ups.
+    // Each of the two finishes two of the four columns
+    float gate[2], up[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) up[i] = upper_half(v[i]);
-    if (q >= 2 || !live) return;
-    bf16x4_t packed;
+    for (int i = 0; i < 2; ++i) exchange_halves(v[i], v[i + 2], gate[i], up[i]);
+    if (!live) return;
+    bf16x2_t packed;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)(silu_bf16_f(round_bf16(v[i])) * round_bf16(up[i]));
-    if (p.gate_act) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) packed[i] = (bf16_t)gated_f(p, round_bf16(v[i]), round_bf16(up[i]));
-    }
-    *reinterpret_cast<bf16x4_t*>(reinterpret_cast<bf16_t*>(p.out) + row * p.out_ld + tile * 8 + 4 * q) = packed;
+    for (int i = 0; i < 2; ++i) packed[i] = (bf16_t)gated_f(p, round_bf16(gate[i]), round_bf16(up[i]));
+    *reinterpret_cast<bf16x2_t*>(reinterpret_cast<bf16_t*>(p.out) + row * p.out_ld + tile * 8 + 4 * (q & 1) + 2 * (q / 2)) = packed;
   } else {
     if (!live) return;
     if (EPI == EPI_PLAIN && p.out_f32) {
@@ -911,7 +911,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) sum += taps[i][k] * (float)tail[k][i];
         sum += taps[i][3] * (float)sample[i];
-        packed[i] = (bf16_t)silu_bf16_f(sum);
+        packed[i] = (bf16_t)silu_f(sum);
       }
       *reinterpret_cast<bf16x4_t*>(tail_at) = tail[1];                    // the tail rolls by one
       *reinterpret_cast<bf16x4_t*>(tail_at + channels) = tail[2];

@@ -3,6 +3,7 @@ other than the tiny models': head sizes in steps of 16, odd head and group count
 and vocabularies that are no power of two, several page sizes; and inputs built so that a
 fault that random data would hide (a far key, a window's edge, a page's edge) shows."""
 import math
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -1207,6 +1208,33 @@ def test_skinny_products_of_weights_in_fragment_order(ops, M, N, K, blocks):
         close(got_state, want_state, torch.bfloat16, 8.0)
         unused = [slot for slot in range(M + 2) if slot not in slot_ids.tolist()]
         assert torch.equal(got_state[unused].cpu(), state[unused])
+
+
+def _odd_rows(rows, columns, dtype):
+    """Room for an output whose rows are not whole fours apart: the product's general kernel writes it."""
+    return torch.full((rows, columns + 3), float("nan"), dtype=dtype, device=DEV)[:, :columns]
+
+
+@pytest.mark.parametrize("M, N, K", [(1, 65536, 512), (16, 4112, 1024), (37, 2000, 2080), (64, 1040, 2048)])
+def test_activations_of_a_product_are_the_same_bits_in_both_of_its_kernels(ops, M, N, K):
+    """SiLU behind the gate and behind the conv step, of numbers as far from zero as its exponential reaches: the kernel of
+    small steps and the general one (which takes rows that are not whole fours apart) add up in one order and end in the same
+    functions."""
+    x, W = rand(M, K, seed=370, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=371, scale=30.0 * K ** -0.5, dtype=torch.bfloat16).to(DEV)
+    fragments, lo, hi = ops.fragment_order(W), 8, N - 4
+    for gate_activation, clamp in (("silu", None), ("gelu_tanh", None), ("clamped", SimpleNamespace(limit=7.0, alpha=1.702, up_offset=1.0))):
+        got, want = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV), _odd_rows(M, N // 2, torch.bfloat16)
+        for out in (got, want):
+            ops.fused_gemm(W, None, out, x=x, epilogue=ops.EPI_SWIGLU, fragments=fragments, gate_activation=gate_activation, clamp=clamp)
+        assert torch.equal(got, want), gate_activation
+    state = rand(M + 1, 3, hi - lo, seed=372, dtype=torch.bfloat16).to(DEV)
+    conv = dict(lo=lo, hi=hi, taps=4, weight=rand(hi - lo, 4, seed=373).to(DEV), bias=rand(hi - lo, seed=374, scale=0.1).to(DEV),
+                slot_ids=torch.arange(M, dtype=torch.int32, device=DEV))
+    got, want, states = torch.empty(M, N, dtype=torch.bfloat16, device=DEV), _odd_rows(M, N, torch.bfloat16), []
+    for out in (got, want):
+        states.append(state.clone())
+        ops.fused_gemm(W, None, out, x=x, epilogue=ops.EPI_CONV, fragments=fragments, conv=dict(conv, state=states[-1]))
+    assert torch.equal(got, want) and torch.equal(*states)
 
 
 @pytest.mark.parametrize("M, N, K, S", [(64, 1024, 2048, 8), (33, 100, 2048, 16), (17, 48, 96, 3), (64, 136, 3072, 5),
