@@ -657,7 +657,7 @@ struct SkinnyParams {
   void* out;             // rows, or the residual stream (RESIDUAL, TANH: leading dimension N)
   long out_ld;
   const float* bias;
-  float out_scale, ssq_inverse_width, ssq_eps;
+  float out_scale, ssq_width, ssq_eps;
   int out_f32, gate_act;
   const float* res_w;
   bf16_t* res_hb;
@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   asm volatile("" ::"s"(p.bias), "s"(p.out), "s"(p.out_ld), "s"(p.out_scale), "s"(p.out_f32));
   if (EPI == EPI_SWIGLU) asm volatile("" ::"s"(p.gate_act));
   if (EPI == EPI_RESIDUAL) asm volatile("" ::"s"(p.res_hb), "s"(p.res_hb_ld), "s"(p.ssq_out));
-  if (SQ > 0) asm volatile("" ::"s"(p.ssq_inverse_width), "s"(p.ssq_eps));
+  if (SQ > 0) asm volatile("" ::"s"(p.ssq_width), "s"(p.ssq_eps));
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the products
@@ -848,11 +848,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
     float squares = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) squares += parts[w][mine * 16 + r];
-    const float mean = squares * p.ssq_inverse_width + p.ssq_eps;
-    float inverse = __builtin_amdgcn_rsqf(mean);
-    const float closer = inverse * (1.5f - 0.5f * mean * inverse * inverse);           // (a step of Newton's: as close as 1 / sqrtf,
-    inverse = mean > 0.f && mean < INFINITY ? closer : inverse;                        // whose limits at 0 and infinity it has not)
-    v *= inverse;
+    v *= 1.0f / sqrtf(squares / p.ssq_width + p.ssq_eps);
   }
   if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + n_safe);
   const bool live = mine * 16 + r <= last_row && n < p.N && own == tile;
@@ -982,7 +978,7 @@ static int launch_skinny(const FusedGemmParams& f, int epi, hipStream_t stream) 
   p.ssq_in = f.ssq_in;
   p.ssq_blocks = f.ssq_blocks;
   p.ssq_ld = f.ssq_ld;
-  p.ssq_inverse_width = f.ssq_width > 0 ? 1.0f / (float)f.ssq_width : 0.f;
+  p.ssq_width = (float)f.ssq_width;
   p.ssq_eps = f.ssq_eps;
   p.out = epi == EPI_RESIDUAL || epi == EPI_TANH ? (void*)f.res_h : f.out;
   p.out_ld = f.out_ld;

@@ -1237,6 +1237,22 @@ def test_activations_of_a_product_are_the_same_bits_in_both_of_its_kernels(ops, 
     assert torch.equal(got, want) and torch.equal(*states)
 
 
+@pytest.mark.parametrize("M, N, K", [(1, 4096, 1024), (16, 1028, 512), (64, 516, 2080)])
+def test_row_scale_of_a_product_is_the_same_bits_in_both_of_its_kernels(ops, M, N, K):
+    """1 / sqrt(sum of squares / width + eps) of one sum of squares a row, from 1e-44 to infinity and zero, with and without
+    an eps: the kernel of small steps and the general one."""
+    x, W = rand(M, K, seed=380, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=381, scale=0.1, dtype=torch.bfloat16).to(DEV)
+    fragments, rows = ops.fragment_order(W), 16 * (-(-M // 16))
+    for turn in range(4):
+        squares = torch.exp(rand(1, rows, seed=382 + turn, scale=25.0))
+        squares[0, :M:5], squares[0, 1:M:7], squares[0, 2:M:7] = (0.0, float("inf"), 1e-44, 1e-39)[turn], 3.0, 1e38
+        for eps in (0.0, 1e-5):
+            got, want = torch.empty(M, N, device=DEV), _odd_rows(M, N, torch.float32)
+            for out in (got, want):
+                ops.fused_gemm(W, None, out, x=x, fragments=fragments, row_scale=ops.RowScale(squares.to(DEV), 777, eps))
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(5.0), want.nan_to_num(5.0)), (turn, eps)
+
+
 @pytest.mark.parametrize("M, N, K, S", [(64, 1024, 2048, 8), (33, 100, 2048, 16), (17, 48, 96, 3), (64, 136, 3072, 5),
                                         (5, 64, 64, 1)])
 def test_fused_gemm_split_over_k_and_the_norm_that_adds_its_slabs(ops, M, N, K, S):
