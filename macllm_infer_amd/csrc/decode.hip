@@ -601,10 +601,10 @@ __global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmPa
     if (EPI == EPI_RESIDUAL) {
       __syncthreads();
       if (tid < min(MT * 16, ssq_rows)) {
-        float squares[4];                       // in the order of skinny_kernel: fours, then pairs of them
+        float squares = 0.f;
 #pragma unroll
-        for (int f = 0; f < 16; ++f) squares[f / 4] = (f % 4 ? squares[f / 4] : 0.f) + tile[f * (MT * 16) + tid];
-        p.ssq_out[(long)block_x * p.ssq_ld + tid] = (squares[0] + squares[1]) + (squares[2] + squares[3]);
+        for (int f = 0; f < 16; ++f) squares += tile[f * (MT * 16) + tid];
+        p.ssq_out[(long)block_x * p.ssq_ld + tid] = squares;
       }
     }
     if (EPI == EPI_SWIGLU) {
@@ -672,16 +672,6 @@ struct SkinnyParams {
   float act_limit, act_alpha, act_offset;
 };
 
-// the sum over the lanes 16, then 32 apart, in every lane, in the vector pipeline
-__device__ __forceinline__ float quarters_sum(float v) {
-  const auto rows = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
-  const unsigned even = rows[0], odd = rows[1];
-  const float pair = __builtin_bit_cast(float, even) + __builtin_bit_cast(float, odd);
-  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, pair), __builtin_bit_cast(unsigned, pair), false, false);
-  const unsigned low = halves[0], high = halves[1];
-  return __builtin_bit_cast(float, low) + __builtin_bit_cast(float, high);
-}
-
 // lower: a of the lanes below 32 where they are, b of the lanes below 32 in the lanes above; upper: a of the lanes above 32 in the
 // lanes below, b of those above where they are
 __device__ __forceinline__ void exchange_halves(float a, float b, float& lower, float& upper) {
@@ -691,19 +681,29 @@ __device__ __forceinline__ void exchange_halves(float a, float b, float& lower, 
   upper = __builtin_bit_cast(float, high);
 }
 
-// v * v, rounded before anything is added to it (fused_gemm_kernel's squares pass through LDS)
+// v * v, rounded before anything is added to it
 __device__ __forceinline__ float square_rounded(float v) {
 #pragma clang fp contract(off)
   return v * v;
 }
 
-// EPI_PLAIN ... EPI_TANH as above.  SQ: partial sums of squares a thread asks for early (0: no row scale).  TILED: W in
-// fragment order.  Row y of the grid takes the MT tiles of 16 rows from row 16 MT y on; with several of them a row of
+// Partial sums of squares of a row that a thread asks for early: where a wave's whole run of K is in flight, those of rows as wide
+// as that K (16 features each, SSQ_PARTS threads a row), else SSQ_EARLY; of several tiles of rows 24 in all.  (16 beside two buffers
+// leave the conv step of one tile of rows more than the 128 registers of two workgroups a compute unit: 8,728 x 3,072 at one
+// row 16.2 us, 14.3 with 12.)
+template <int MT, int WAVES, int CH, bool EXACT>
+constexpr int skinny_early_sums() {
+  constexpr int wanted = EXACT ? (2 * WAVES * CH + SSQ_PARTS - 1) / SSQ_PARTS : SSQ_EARLY, most = MT == 1 ? SSQ_EARLY : 24 / MT;
+  return wanted < most ? wanted : most;
+}
+
+// EPI_PLAIN ... EPI_TANH as above.  SCALED: behind a row scale.  TILED: W in fragment order.  Row y of the grid takes the MT tiles of 16 rows from row 16 MT y on; with several of them a row of
 // the grid is a multiple of 8 workgroups, so that those of a tile of features run on one die and its weights leave memory once.
-template <int MT, int EPI, int WAVES, int CH, bool EXACT, int SQ, bool TILED>
+template <int MT, int EPI, int WAVES, int CH, bool EXACT, bool SCALED, bool TILED>
 __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   __shared__ floatx4 red[WAVES][MT][WAVE];
-  __shared__ float parts[SQ > 0 ? WAVES : 1][MT * 16];
+  constexpr int SQ = skinny_early_sums<MT, WAVES, CH, EXACT>();
+  __shared__ float parts[SCALED ? SSQ_PARTS : 1][MT * 16];
   const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int q = lane / 16, r = lane % 16;
   // (a workgroup past the last tile, which fills up a row of the grid, does that tile's work again and stores nothing: a
@@ -748,17 +748,17 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   for (int buffer = 0; buffer < BUFFERS; ++buffer) ask_rows(buffer, buffer * CH);
 
   // ---- what the last stage needs, behind them: sums of squares, the stream's elements, conv tails
-  constexpr int PARTS = WAVES * 4;
-  const int part = threadIdx.x / 16;
-  float sq[MT][SQ > 0 ? SQ : 1];
-  if (SQ > 0) {
-    const int last = p.ssq_blocks - 1;
+  // (four waves add them up, however many tiles of rows there are: a row's sum does not depend on how a step's rows are dealt out)
+  const int part = threadIdx.x / 16, own_sums = part * p.ssq_ld, last_sums = (p.ssq_blocks - 1) * p.ssq_ld;
+  auto sum_at = [&](int mt, int block) {                       // of row mt * 16 + r, `block` blocks behind the part's first
+    return (p.ssq_in + row0)[(unsigned)(min(own_sums + block * p.ssq_ld, last_sums) + min(mt * 16 + r, ssq_rows - 1))];
+  };
+  float sq[MT][SQ];
+  if (SCALED && (WAVES == 4 || wave < 4)) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const float* at = p.ssq_in + row0 + min(mt * 16 + r, ssq_rows - 1);
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int i = 0; i < SQ; ++i) sq[mt][i] = at[(long)min(part + i * PARTS, last) * p.ssq_ld];
-    }
+      for (int i = 0; i < SQ; ++i) sq[mt][i] = sum_at(mt, i * SSQ_PARTS);
   }
   floatx4 h_old, res_w, post_w, post_b, next_w, next_b;
   float* h_at = reinterpret_cast<float*>(p.out) + (long)(row0 + m) * p.N + n_safe;
@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   asm volatile("" ::"s"(p.bias), "s"(p.out), "s"(p.out_ld), "s"(p.out_scale), "s"(p.out_f32));
   if (EPI == EPI_SWIGLU) asm volatile("" ::"s"(p.gate_act));
   if (EPI == EPI_RESIDUAL) asm volatile("" ::"s"(p.res_hb), "s"(p.res_hb_ld), "s"(p.ssq_out));
-  if (SQ > 0) asm volatile("" ::"s"(p.ssq_width), "s"(p.ssq_eps));
+  if (SCALED) asm volatile("" ::"s"(p.ssq_width), "s"(p.ssq_eps));
   __builtin_amdgcn_sched_barrier(0);
 
   // ---- the products
@@ -822,18 +822,29 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
 #pragma unroll
     for (int buffer = 0; buffer < 2; ++buffer) multiply(buffer, c + buffer * CH, false);
   }
-  if (SQ > 0) {
+  if (SCALED && (WAVES == 4 || wave < 4)) {
+    const int blocks = p.ssq_blocks - part;
+    float sums[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      float sum = 0.f;
+      sums[mt] = 0.f;
 #pragma unroll
-      for (int i = 0; i < SQ; ++i) sum += part + i * PARTS < p.ssq_blocks ? sq[mt][i] : 0.f;
-      // wider rows than SQ sums a thread: the rest now
-      for (int block = part + SQ * PARTS; block < p.ssq_blocks; block += PARTS)
-        sum += p.ssq_in[(long)block * p.ssq_ld + row0 + min(mt * 16 + r, ssq_rows - 1)];
-      sum = quarters_sum(sum);
-      if (lane < 16) parts[wave][mt * 16 + lane] = sum;
+      for (int i = 0; i < SQ; ++i) sums[mt] += i * SSQ_PARTS < blocks ? sq[mt][i] : 0.f;
     }
+    // wider rows than SQ sums a thread: the rest now
+    for (int block = SQ * SSQ_PARTS; block < blocks; block += 4 * SSQ_PARTS) {
+      float more[MT][4];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) more[mt][i] = sum_at(mt, block + i * SSQ_PARTS);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[mt] += block + i * SSQ_PARTS < blocks ? more[mt][i] : 0.f;
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) parts[part][mt * 16 + r] = sums[mt];
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) red[wave][mt][lane] = acc[mt];
@@ -844,31 +855,41 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   floatx4 v = red[0][mine][lane];
 #pragma unroll
   for (int w = 1; w < WAVES; ++w) v += red[w][mine][lane];
-  if (SQ > 0) {                                // the norm's division, on the float32 sums
+  if (SCALED) {                                // the norm's division, on the float32 sums
     float squares = 0.f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) squares += parts[w][mine * 16 + r];
+    for (int k = 0; k < SSQ_PARTS; ++k) squares += parts[k][mine * 16 + r];
     v *= 1.0f / sqrtf(squares / p.ssq_width + p.ssq_eps);
   }
   if (p.bias) v += *reinterpret_cast<const floatx4*>(p.bias + n_safe);
   const bool live = mine * 16 + r <= last_row && n < p.N && own == tile;
   const long row = row0 + m;
   if (EPI == EPI_RESIDUAL) {
-    floatx4 updated;
-    float square = 0.f;
+    floatx4 updated, squares = {0.f, 0.f, 0.f, 0.f};
     if (live) {
       bf16x4_t rows;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         updated[i] = h_old[i] + v[i];
         rows[i] = (bf16_t)(updated[i] * res_w[i]);
-        square += square_rounded(updated[i]);
+        squares[i] = square_rounded(updated[i]);
       }
       *reinterpret_cast<floatx4*>(h_at) = updated;
       *reinterpret_cast<bf16x4_t*>(p.res_hb + row * p.res_hb_ld + n) = rows;
     }
-    square = quarters_sum(square);
-    if (own == tile && lane < min(16, ssq_rows - mine * 16)) p.ssq_out[(long)tile * p.ssq_ld + row0 + mine * 16 + lane] = square;
+    // a row's squares feature by feature, by one lane: through LDS, where this wave alone has read its tile
+    red[0][mine][lane] = squares;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (own == tile && lane < min(16, ssq_rows - mine * 16)) {
+      float sum = 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const floatx4 four = red[0][mine][k * 16 + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum += four[i];
+      }
+      p.ssq_out[(long)tile * p.ssq_ld + row0 + mine * 16 + lane] = sum;
+    }
   } else if (EPI == EPI_TANH) {
     if (!live) return;
     floatx4 updated;
@@ -924,6 +945,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
 static bool skinny_takes(const FusedGemmParams& p, int epi) {
   auto aligned = [](const void* at, size_t bytes) { return ((uintptr_t)at & (bytes - 1)) == 0; };
   if (p.w_tiled ? epi == EPI_TANH : p.ssq_in || epi == EPI_CONV || epi == EPI_RESIDUAL) return false;     // forms without an instance
+  if (p.ssq_in && (long)p.ssq_blocks * p.ssq_ld > 0x3fffffffL) return false;       // 32-bit offsets
   if (p.N % 4 || p.x_ld > 0x7fffffffL || !aligned(p.W, 16) || !aligned(p.x, 16) || (p.bias && !aligned(p.bias, 16))) return false;
   if (epi == EPI_RESIDUAL || epi == EPI_TANH) {
     if (!aligned(p.res_h, 16) || (p.res_hb && (p.res_hb_ld % 4 || !aligned(p.res_hb, 8)))) return false;
@@ -940,17 +962,13 @@ static bool skinny_takes(const FusedGemmParams& p, int epi) {
 template <int MT, int EPI, int WAVES, int CH, bool EXACT>
 static void launch_skinny_scaled(const SkinnyParams& p, bool tiled, dim3 blocks, hipStream_t stream) {
   if (!tiled) {
-    if constexpr (EPI == EPI_PLAIN || EPI == EPI_SWIGLU || EPI == EPI_TANH) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, false><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+    if constexpr (EPI == EPI_PLAIN || EPI == EPI_SWIGLU || EPI == EPI_TANH) skinny_kernel<MT, EPI, WAVES, CH, EXACT, false, false><<<blocks, WAVES * WAVE, 0, stream>>>(p);
     return;
   }
   if constexpr (EPI == EPI_TANH) return;
-  else if constexpr (EPI == EPI_RESIDUAL) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
-  else {
-    if (!p.ssq_in) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 0, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
-    else if (WAVES == 4 || p.ssq_blocks <= 4 * 4 * WAVES) skinny_kernel<MT, EPI, WAVES, CH, EXACT, 4, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
-    else if (p.ssq_blocks <= 6 * 4 * 8) skinny_kernel<MT, EPI, 8, CH, EXACT, 6, true><<<blocks, 8 * WAVE, 0, stream>>>(p);
-    else skinny_kernel<MT, EPI, 8, CH, EXACT, 12, true><<<blocks, 8 * WAVE, 0, stream>>>(p);
-  }
+  else if constexpr (EPI == EPI_RESIDUAL) skinny_kernel<MT, EPI, WAVES, CH, EXACT, false, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+  else if (p.ssq_in) skinny_kernel<MT, EPI, WAVES, CH, EXACT, true, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
+  else skinny_kernel<MT, EPI, WAVES, CH, EXACT, false, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
 }
 
 // All of a wave's run of K at once where that is a fixed number of chunks (K of 512 and 1,024 over four waves, 2,048 over

@@ -1253,6 +1253,33 @@ def test_row_scale_of_a_product_is_the_same_bits_in_both_of_its_kernels(ops, M, 
             assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(5.0), want.nan_to_num(5.0)), (turn, eps)
 
 
+@pytest.mark.parametrize("M, N, K, blocks", [(1, 4096, 1024, 64), (16, 1028, 512, 32), (17, 260, 1024, 64), (40, 132, 2048, 333),
+                                             (48, 272, 96, 700), (64, 516, 2080, 193), (8, 64, 1056, 1)])
+def test_squares_of_a_row_are_added_up_in_one_order_in_both_kernels_of_a_product(ops, M, N, K, blocks):
+    """A row's squares of a tile are added up feature by feature, the tiles' sums by 16 threads and theirs one after the other:
+    the kernel of small steps, however a step's rows are dealt out, and the general one (with one tile of rows; its 256 threads
+    are fewer a row for more)."""
+    x, W = rand(M, K, seed=390, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=391, scale=0.1, dtype=torch.bfloat16).to(DEV)
+    fragments, rows = ops.fragment_order(W), 16 * (-(-M // 16))
+    h, weight = rand(M, N, seed=392, scale=2.0), torch.ones(N, device=DEV)
+    for operand in (W, fragments):
+        got_h, hb, ssq = h.clone().to(DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV), ops.residual_workspace(M, N, DEV)
+        ops.fused_gemm_residual(W, None, x, got_h, hb, weight, ssq, None if operand is W else operand)
+        squares = torch.cat([got_h.cpu() ** 2, torch.zeros(M, -N % 16)], dim=1).view(M, -1, 16)
+        want = torch.zeros(M, squares.shape[1])
+        for feature in range(16):
+            want = want + squares[:, :, feature]
+        assert torch.equal(ssq.cpu()[:, :M], want.T) and not ssq[:, M:].any()
+    sums = (rand(blocks, rows, seed=393).abs() * 16.0 + 1.0).to(DEV)
+    for first in range(0, M, 16):                    # a tile of rows by itself
+        some = slice(first, min(first + 16, M))
+        want, again = _odd_rows(some.stop - first, N, torch.float32), torch.empty(M, N, device=DEV)
+        ops.fused_gemm(W, None, want, x=x[some], fragments=fragments, row_scale=ops.RowScale(sums[:, first:first + 16].contiguous(), 16 * blocks, 1e-5))
+        for row_tiles in (1, 2, 3, 4):
+            ops.fused_gemm(W, None, again, x=x, fragments=fragments, row_tiles=row_tiles, row_scale=ops.RowScale(sums, 16 * blocks, 1e-5))
+            assert torch.equal(again[some], want), (first, row_tiles)
+
+
 @pytest.mark.parametrize("M, N, K, S", [(64, 1024, 2048, 8), (33, 100, 2048, 16), (17, 48, 96, 3), (64, 136, 3072, 5),
                                         (5, 64, 64, 1)])
 def test_fused_gemm_split_over_k_and_the_norm_that_adds_its_slabs(ops, M, N, K, S):
