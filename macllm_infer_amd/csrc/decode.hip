@@ -730,7 +730,8 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   const bf16_t* x_at[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) x_at[mt] = p.x + (long)(row0 + min(mt * 16 + r, last_row)) * p.x_ld + first * 32 + 8 * q;
-  // (no condition around a load: a chunk past the wave's run reads a valid one and is multiplied as zeros)
+  // (no condition around a load: a chunk past the wave's run reads a valid one and is not multiplied: as zeros it would make a
+  // NaN of a row's infinity)
   auto chunk_at = [&](int c) { return EXACT ? c : min(c, max(count, 1) - 1) - (count ? 0 : first); };
   auto ask_weights = [&](int buffer, int c0) {
 #pragma unroll
@@ -800,11 +801,9 @@ __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   auto multiply = [&](int buffer, int c0, bool whole) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      floatx4 weights = *reinterpret_cast<const floatx4*>(&a[buffer][j]);
-      if (!whole) weights = c0 + j < count ? weights : floatx4{0.f, 0.f, 0.f, 0.f};
+      if (!whole && c0 + j >= count) continue;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(&weights), b[buffer][j][mt], acc[mt], 0, 0, 0);
+      for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[buffer][j], b[buffer][j][mt], acc[mt], 0, 0, 0);
     }
   };
   if (EXACT) {

@@ -1280,6 +1280,22 @@ def test_squares_of_a_row_are_added_up_in_one_order_in_both_kernels_of_a_product
             assert torch.equal(again[some], want), (first, row_tiles)
 
 
+@pytest.mark.parametrize("K", [32, 96, 512, 768, 1024, 1312, 2048, 2080, 3072, 4096, 4640])
+def test_an_infinity_in_a_row_of_a_small_step_stays_one(ops, K):
+    """Runs of K that fill a wave's buffers and runs that do not: nothing is multiplied that the row does not hold."""
+    x = rand(17, K, seed=395, dtype=torch.bfloat16)
+    x[0, 0], x[3, K - 1], x[16, K // 2] = float("inf"), float("-inf"), float("inf")
+    W = rand(36, K, seed=396, dtype=torch.bfloat16)
+    W[W == 0] = 1.0
+    want = x.double() @ W.double().T
+    for rows in (1, 16, 17):
+        for fragments in (None, ops.fragment_order(W.to(DEV))):
+            got = torch.empty(rows, 36, device=DEV)
+            ops.fused_gemm(W.to(DEV), None, got, x=x[:rows].to(DEV), fragments=fragments)
+            assert torch.equal(got.isnan().cpu(), want[:rows].isnan()) and torch.equal(got.isinf().cpu(), want[:rows].isinf())
+            assert torch.equal(got.cpu()[got.isinf().cpu()].double(), want[:rows][want[:rows].isinf()])
+
+
 @pytest.mark.parametrize("M, N, K, S", [(64, 1024, 2048, 8), (33, 100, 2048, 16), (17, 48, 96, 3), (64, 136, 3072, 5),
                                         (5, 64, 64, 1)])
 def test_fused_gemm_split_over_k_and_the_norm_that_adds_its_slabs(ops, M, N, K, S):
