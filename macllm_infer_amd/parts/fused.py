@@ -348,8 +348,9 @@ def register_mixer_kernel(*kinds: str):
     product's epilogue: {lo, hi, taps, weight, bias}), ``supported(step, caches)``,
     ``conv_state(caches)`` and ``run(u, step, caches, mixed, merge=True)``; a kernel with ``merged_columns`` (how
     many the attended heads are, the first columns of ``mixed``) returns, when called with ``merge=False``, their runs of
-    keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; ``step_tables()``: tables it reads in every step;
-    ``ahead``: weights that its launch may bring into the caches, if it says the ``state_bytes`` that it reads a row."""
+    keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; one with ``step_tables()`` names the tables
+    that it reads in every step; one with ``state_bytes``, how many it reads a row, is called with ``ahead`` too: weights in
+    fragment order that its launch may bring into the caches."""
     def decorate(factory):
         _MIXER_KERNELS[tuple(kinds)] = factory
         return factory
@@ -813,7 +814,8 @@ class LayerFusion:
         if kernel is not None:
             later = (not self.library_out[bucket] and not self.split_out[bucket]
                      and self._merges_later(kernel, step, caches))
-            attended = kernel.run(u, step, caches, mixed, merge=not later, ahead=self._read_ahead(residual, kernel, M, bucket))
+            reads = dict(ahead=self._read_ahead(residual, kernel, M, bucket)) if hasattr(kernel, "state_bytes") else {}
+            attended = kernel.run(u, step, caches, mixed, merge=not later, **reads)
         else:
             self._mix_each(u, step, caches, mixed, ahead=self._read_ahead(residual, self.kernel, step.num_lanes, bucket))
         self._after_the_mixers(residual, mixed, attended, M, bucket)

@@ -895,6 +895,39 @@ def test_weights_read_ahead_change_nothing(monkeypatch, prompt):
     assert torch.equal(results[0], results[28 << 20]) and torch.isfinite(results[0]).all()
 
 
+def test_a_mixer_kernel_is_called_as_registered(monkeypatch):
+    """A kernel with the attributes that every kernel offers, and none besides, takes steps of single tokens: its ``run`` is
+    called with the step's rows, caches and output and with ``merge``, and with nothing that it did not ask for."""
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.parts import fused
+    from macllm_infer_amd.weights.random_init import random_tensors
+    calls = []
+
+    class Least:
+        def __init__(self, whole):
+            self.whole, self.conv, self.supported, self.conv_state = whole, whole.conv, whole.supported, whole.conv_state
+
+        def run(self, u, step, caches, mixed, merge=True):
+            calls.append(merge)
+            return self.whole.run(u, step, caches, mixed, merge=merge)
+
+    config = FalconH1Config.from_dict(dict(tiny_configs.TINY_C, max_position_embeddings=1024))
+    tensors = random_tensors(config, 5, torch.bfloat16, "unit")
+    whole = fused._MIXER_KERNELS["attention", "mamba2"]
+    results = []
+    for factory in (whole, lambda fusion: Least(whole(fusion))):
+        monkeypatch.setitem(fused._MIXER_KERNELS, ("attention", "mamba2"), factory)
+        engine = Engine(config=config, tensors=tensors, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=2048,
+                        max_active_sequences=2)
+        for name in range(2):
+            engine.add_request(name)
+            engine.step([Lane(name, tokens_for(config.vocab_size, 700, 50 + name), [])])
+        results.append(torch.cat([engine.step([Lane(name, [7 + turn], [0]) for name in range(2)]).float().cpu() for turn in range(4)]))
+    assert calls and all(calls)
+    assert torch.equal(*results)
+
+
 def test_graphs_come_in_buckets_of_context_length():
     """A model that allows long contexts: a short request decodes through a graph made for 2,048
     tokens, a longer one through a graph made for 4,096 (wider block tables, more runs of keys),
