@@ -136,14 +136,42 @@ __device__ __forceinline__ float gated_f(const Params& p, float gate, float up) 
   return g / (1.0f + expf(-p.act_alpha * g)) * (u + p.act_offset);
 }
 
+// What is left of a step for a workgroup that takes `rows` of its rows from row0 on (plain prologue).
+__device__ __forceinline__ void take_rows(FusedGemmParams& p, int row0, int rows) {
+  if (p.x) p.x += (long)row0 * p.x_ld;
+  if (p.out) p.out = p.out_f32 ? (void*)(reinterpret_cast<float*>(p.out) + (long)row0 * p.out_ld)
+                               : (void*)(reinterpret_cast<bf16_t*>(p.out) + (long)row0 * p.out_ld);
+  if (p.slot_ids) p.slot_ids += row0;
+  if (p.res_h) {
+    p.res_h += (long)row0 * p.N;
+    if (p.res_hb) p.res_hb += (long)row0 * p.res_hb_ld;
+    if (p.ssq_out) p.ssq_out += row0;
+  }
+  if (p.ssq_in) p.ssq_in += row0;
+  p.M = min(rows, p.M - row0);
+}
+
 __device__ __forceinline__ float round_bf16(float v) { return (float)(bf16_t)v; }
 
-template <int MT, int PRO, int EPI, int FG_WAVES, int NT>
-__global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmParams p) {
+template <int MT, int PRO, int EPI, int FG_WAVES, int NT, bool ROW_TILES = false>
+__global__ void __launch_bounds__(FG_WAVES * WAVE) fused_gemm_kernel(FusedGemmParams whole_step) {
   static_assert(NT == 1 || PRO == PRO_PLAIN, "several feature tiles a workgroup: plain prologue only");
+  // Row tiles: a workgroup takes MT tiles of 16 rows of the step and row_tiles workgroups share a tile of
+  // features.  Workgroups go to the eight dies in turn and each die has a cache of its own, so those that share
+  // weights are given numbers that are 8 apart and follow each other: the weights leave memory once.
+  FusedGemmParams p = whole_step;
   const int slab_rows = p.M;
-  const int block_x = blockIdx.x;
-  const int ssq_rows = p.ssq_ld;        // rows of the tables of partial sums of squares
+  int block_x = blockIdx.x;
+  int ssq_rows = p.ssq_ld;              // rows of the tables of partial sums of squares from this workgroup's first row on
+  if (ROW_TILES) {
+    static_assert(!ROW_TILES || (PRO == PRO_PLAIN && NT == 1), "rows dealt out: plain prologue, one tile of features");
+    const int die = block_x % 8, turn = block_x / 8;
+    block_x = (turn / p.row_tiles) * 8 + die;
+    if (block_x * 16 * NT >= p.N) return;
+    const int row0 = (turn % p.row_tiles) * MT * 16;
+    ssq_rows -= row0;
+    take_rows(p, row0, MT * 16);
+  }
   static_assert(PRO != PRO_MERGE || EPI == EPI_PLAIN || EPI == EPI_RESIDUAL, "the merge prologue comes with the plain or the residual epilogue");
   static_assert(EPI != EPI_RESIDUAL || (NT == 1 && PRO != PRO_NORM), "the residual epilogue: one tile of features, rows given as they are");
   static_assert(EPI != EPI_TANH || (NT == 1 && PRO == PRO_PLAIN), "the tanh epilogue: one tile of features, the plain prologue");
@@ -1057,13 +1085,35 @@ static int launch_fused_gemm(const FusedGemmParams& p, int pro, int epi, hipStre
 #undef FG_WIDE
     return 0;
   }
-  const dim3 blocks((p.N + 15) / 16, k_splits);
+  const int feature_blocks = (p.N + 15) / 16;
+  const dim3 blocks(p.row_tiles > 1 ? (feature_blocks + 7) / 8 * 8 * p.row_tiles : feature_blocks, k_splits);
   const int waves = fused_gemm_waves(p.K / k_splits);
 #define FG_LAUNCH(PRO_, EPI_)                                                                      \
   do {                                                                                             \
     if (waves == 8) fused_gemm_kernel<MT, PRO_, EPI_, 8, 1><<<blocks, 8 * WAVE, lds, stream>>>(p); \
     else fused_gemm_kernel<MT, PRO_, EPI_, 4, 1><<<blocks, 4 * WAVE, lds, stream>>>(p);            \
   } while (0)
+#define FG_LAUNCH_ROWS(EPI_)                                                                                  \
+  do {                                                                                                        \
+    if (waves == 8) fused_gemm_kernel<MT, PRO_PLAIN, EPI_, 8, 1, true><<<blocks, 8 * WAVE, lds, stream>>>(p); \
+    else fused_gemm_kernel<MT, PRO_PLAIN, EPI_, 4, 1, true><<<blocks, 4 * WAVE, lds, stream>>>(p);            \
+  } while (0)
+  if (p.row_tiles > 1) {           // MT of 1 or 2: the tiles of a step of up to 64 rows over two workgroups or more (forms that
+    // skinny_kernel does not take; 64 rows over 1 / 2 / 4: 1,024 x 2,048 row-major into the stream 12.7 / 9.0 / 7.0 us, with the conv step
+    // 13.5 / 9.5 / 7.6; 4,118 x 1,024 behind a row scale in fragment order 13.1 / 11.2 / 10.8)
+    if (pro != PRO_PLAIN) return ERR_BAD_ARGUMENT;
+    if constexpr (MT <= 2) {
+      if (epi == EPI_RESIDUAL) FG_LAUNCH_ROWS(EPI_RESIDUAL);
+      else if (epi == EPI_TANH) FG_LAUNCH_ROWS(EPI_TANH);
+      else if (epi == EPI_PLAIN) FG_LAUNCH_ROWS(EPI_PLAIN);
+      else if (epi == EPI_SWIGLU) FG_LAUNCH_ROWS(EPI_SWIGLU);
+      else if (epi == EPI_CONV) FG_LAUNCH_ROWS(EPI_CONV);
+      else return ERR_BAD_ARGUMENT;
+      return 0;
+    } else {
+      return ERR_BAD_ARGUMENT;
+    }
+  }
   if (pro == PRO_MERGE && epi == EPI_PLAIN) FG_LAUNCH(PRO_MERGE, EPI_PLAIN);
   else if (pro == PRO_MERGE && epi == EPI_RESIDUAL) FG_LAUNCH(PRO_MERGE, EPI_RESIDUAL);
   else if (pro == PRO_PLAIN && epi == EPI_RESIDUAL) FG_LAUNCH(PRO_PLAIN, EPI_RESIDUAL);
@@ -1076,6 +1126,7 @@ static int launch_fused_gemm(const FusedGemmParams& p, int pro, int epi, hipStre
   else if (pro == PRO_PLAIN && epi == EPI_CONV) FG_LAUNCH(PRO_PLAIN, EPI_CONV);
   else return ERR_BAD_ARGUMENT;
 #undef FG_LAUNCH
+#undef FG_LAUNCH_ROWS
   return 0;
 }
 
@@ -1089,17 +1140,18 @@ static int launch_fused_gemm_rows(FusedGemmParams& p, int pro, int epi, hipStrea
   int MT = step_tiles;
   p.ssq_ld = 16 * step_tiles;
   p.row_tiles = 1;
-  if (row_tiles > 1 && (pro != PRO_PLAIN || feature_tiles != 1)) return ERR_BAD_ARGUMENT;
-  if (pro == PRO_PLAIN && feature_tiles == 1 && k_splits == 1 && skinny_takes(p, epi)) {
+  if (row_tiles > 1) {
+    if (pro != PRO_PLAIN || feature_tiles != 1) return ERR_BAD_ARGUMENT;
     MT = (step_tiles + row_tiles - 1) / row_tiles;
     p.row_tiles = (step_tiles + MT - 1) / MT;
+  }
+  if (pro == PRO_PLAIN && feature_tiles == 1 && k_splits == 1 && skinny_takes(p, epi)) {
     if (MT == 1) return launch_skinny<1>(p, epi, stream);
     if (MT == 2) return launch_skinny<2>(p, epi, stream);
     if (MT == 3) return launch_skinny<3>(p, epi, stream);
     if (MT == 4) return launch_skinny<4>(p, epi, stream);
     return ERR_UNSUPPORTED_SIZE;
   }
-  // (features that are no whole pieces of four: every workgroup takes all rows, the same sums)
   if (MT == 1) return launch_fused_gemm<1>(p, pro, epi, stream, k_splits, feature_tiles);
   if (MT == 2) return launch_fused_gemm<2>(p, pro, epi, stream, k_splits, feature_tiles);
   if (MT == 3) return launch_fused_gemm<3>(p, pro, epi, stream, k_splits, feature_tiles);

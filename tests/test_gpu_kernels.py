@@ -1280,6 +1280,50 @@ def test_squares_of_a_row_are_added_up_in_one_order_in_both_kernels_of_a_product
             assert torch.equal(again[some], want), (first, row_tiles)
 
 
+@pytest.mark.parametrize("M, N, K", [(17, 1030, 512), (33, 50, 2080), (40, 516, 1024), (64, 1030, 2048)])
+def test_rows_dealt_out_by_the_general_kernel_of_a_product(ops, M, N, K):
+    """Forms of a product that the kernel of small steps does not take (features that are no whole fours, row-major weights that
+    join the stream, a row scale or a conv step behind row-major weights): the step's tiles of rows over as many workgroups as
+    are asked for.  A workgroup that has one tile of rows adds up its rows' sums of squares as the product of that tile alone
+    does, so dealt out to one tile each, the rows are the bits of the products by tiles."""
+    x, W = rand(M, K, seed=400, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=401, scale=0.1, dtype=torch.bfloat16).to(DEV)
+    fragments, rows, blocks = ops.fragment_order(W), 16 * (-(-M // 16)), 200
+    sums = (rand(blocks, rows, seed=402).abs() * 16.0 + 1.0).to(DEV)
+    h, weight = rand(M, N, seed=403, scale=2.0).to(DEV), torch.ones(N, device=DEV)
+    lo, hi = 6, N - 4
+    state = rand(M + 1, 3, hi - lo, seed=404, dtype=torch.bfloat16).to(DEV)
+    conv = dict(lo=lo, hi=hi, taps=4, weight=rand(hi - lo, 4, seed=405).to(DEV), bias=None)
+    slots = torch.randperm(M, generator=torch.Generator().manual_seed(M)).to(torch.int32).to(DEV)
+
+    def all_forms(some, row_tiles, out):
+        scale = ops.RowScale(sums[:, some.start:-(-some.stop // 16) * 16].contiguous(), 16 * blocks, 1e-5)
+        forms = [W] + ([fragments] if N % 4 else [])
+        for form, operand in enumerate(forms):
+            kept = None if operand is W else operand
+            ops.fused_gemm(W, None, out["plain", form][some], x=x[some], row_scale=scale, fragments=kept, row_tiles=row_tiles)
+            ops.fused_gemm(W, None, out["conv", form][some], x=x[some], row_scale=scale, fragments=kept, row_tiles=row_tiles, epilogue=ops.EPI_CONV,
+                           conv=dict(conv, state=out["tails", form], slot_ids=slots[some].contiguous()))
+            ssq = ops.residual_workspace(some.stop - some.start, N, DEV)
+            ops.fused_gemm_residual(W, None, x[some], out["h", form][some], out["hb", form][some], weight, ssq, kept, row_tiles=row_tiles)
+            out["ssq", form][:, some] = ssq[:, :some.stop - some.start]
+
+    def room():
+        out = {}
+        for form in range(2):
+            out["plain", form] = torch.full((M, N), float("nan"), device=DEV)
+            out["conv", form] = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+            out["hb", form], out["h", form] = out["conv", form].clone(), h.clone()
+            out["tails", form], out["ssq", form] = state.clone(), torch.zeros(-(-N // 16), M, device=DEV)
+        return out
+
+    want, got = room(), room()
+    for first in range(0, M, 16):
+        all_forms(slice(first, min(first + 16, M)), 1, want)
+    all_forms(slice(0, M), 4, got)
+    for key in want:
+        assert torch.equal(torch.nan_to_num(got[key].float(), 9.0), torch.nan_to_num(want[key].float(), 9.0)), key
+
+
 @pytest.mark.parametrize("K", [32, 96, 512, 768, 1024, 1312, 2048, 2080, 3072, 4096, 4640])
 def test_an_infinity_in_a_row_of_a_small_step_stays_one(ops, K):
     """Runs of K that fill a wave's buffers and runs that do not: nothing is multiplied that the row does not hold."""
