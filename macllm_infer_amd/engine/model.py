@@ -144,9 +144,9 @@ class DecoderModel:
 
         firsts = [rms_of(getattr(self.blocks[entry.layer], "first_norm", None)) for entry in spec.schedule]
         self._next_norms = firsts[1:] + [self._final_rms]
-        # and the weight that it reads first in steps of few rows, in the order in which the skinny product reads it
-        fragments = [getattr(getattr(self.blocks[entry.layer], "fusion", None), "f_in", None) for entry in spec.schedule]
-        self._next_firsts = fragments[1:] + [None]
+        # and that layer's fusion, which says what it reads first
+        fusions = [getattr(self.blocks[entry.layer], "fusion", None) for entry in spec.schedule]
+        self._next_fusions = [fusion if hasattr(fusion, "first_product") else None for fusion in fusions[1:]] + [None]
         # and the norm part itself, unless something joins the stream before that run
         parts = [getattr(self.blocks[entry.layer], "first_norm", None) if entry.before is None else None
                  for entry in spec.schedule]
@@ -211,7 +211,7 @@ class DecoderModel:
                 residual.pending = added
             caches = {name: cache.entry((index, name)) for name, _ in block.mixers}
             residual.next_norm = self._next_norms[index]
-            residual.next_first = self._next_firsts[index]
+            residual.next_fusion = self._next_fusions[index]
             residual.following = self._following[index]
             block.forward(residual, step, caches)
         wanted = step.want_rows.numel()

@@ -157,9 +157,9 @@ class Residual:
     after the last), if that norm is a root-mean-square norm, set by whoever runs the layers; a layer whose last
     projection adds to the stream itself may then leave ``scaled`` rows for it.  ``following``: the norm part that
     the layer after the one running starts with (the final norm after the last; None where something joins the stream
-    before it); a layer may leave the stream's rows through that norm in ``normed``.  ``next_first``: the weight that the layer
-    after the one running reads first in a step of few rows, in fragment order, or None: a launch that leaves the memory idle may
-    bring it into the caches.  ``scaled`` and ``normed`` are
+    before it); a layer may leave the stream's rows through that norm in ``normed``.  ``next_fusion``: the fusion of
+    the layer after the one running, or None; its ``first_product`` is the weight that it reads first, which a launch that leaves
+    the memory idle may bring into the caches.  ``scaled`` and ``normed`` are
     dropped whenever ``h`` or ``pending`` is assigned: whoever changes the stream without knowing of them makes them
     stale."""
 
@@ -168,7 +168,7 @@ class Residual:
         self._pending: List[torch.Tensor] = []
         self.scaled: Optional[ScaledRows] = None
         self.next_norm: Optional[tuple] = None
-        self.next_first: Optional[torch.Tensor] = None
+        self.next_fusion = None
         self.normed: Optional[NormedRows] = None
         self.following = None
 

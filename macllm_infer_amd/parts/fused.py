@@ -127,6 +127,10 @@ _padding_wins: Dict[tuple, tuple] = {}
 # 1,328 | 1,290 | 1,282 | 1,321, 16 rows 1,367 | 1,329 | 1,325 | 1,374; of 300: 1 row 985 | 920 | 902 | 879, 8 rows 1,123 | 1,080 | 1,074 |
 # 1,116, 16 rows 1,290 | 1,266 | 1,266 | 1,302.  (The 7B shape's 28 MB of output projection: 1 row 1,098 | 1,084, 4 rows 1,196 | 1,225: left out.)
 AHEAD_BYTES = 28 << 20
+# Where a launch has many keys to read it leaves no memory idle: nothing is read ahead beside more than AHEAD_KEY_BYTES of them a
+# layer, by the longest context that the step is made for.  The same shape without | out and gate-up, at 33 MB of keys: 8 rows behind
+# 8,000 1,337 | 1,338, 16 rows behind 4,096 1,597 | 1,586; at 49 MB (12 rows behind 8,000) 1,599 | 1,625, at 65 MB (16 rows) 1,728 | 1,771.
+AHEAD_KEY_BYTES = 40 << 20
 # A projection whose result joins the residual stream can add it there itself (float32, in place) and leave, beside
 # the stream, its rows times the next norm's weight in bfloat16 with the partial sums of their squares; the product
 # behind that norm then reads those rows and multiplies its float32 sums by 1 / sqrt(mean square + eps): the norm
@@ -350,7 +354,7 @@ def register_mixer_kernel(*kinds: str):
     many the attended heads are, the first columns of ``mixed``) returns, when called with ``merge=False``, their runs of
     keys unmerged, as ``ops.AttentionRuns``, for the output projection to merge; one with ``step_tables()`` names the tables
     that it reads in every step; one with ``state_bytes``, how many it reads a row, is called with ``ahead`` too: weights in
-    fragment order that its launch may bring into the caches."""
+    fragment order that its launch may bring into the caches (``key_bytes(step)``: of keys and values, a row, at most)."""
     def decorate(factory):
         _MIXER_KERNELS[tuple(kinds)] = factory
         return factory
@@ -814,21 +818,32 @@ class LayerFusion:
         if kernel is not None:
             later = (not self.library_out[bucket] and not self.split_out[bucket]
                      and self._merges_later(kernel, step, caches))
-            reads = dict(ahead=self._read_ahead(residual, kernel, M, bucket)) if hasattr(kernel, "state_bytes") else {}
+            reads = dict(ahead=self._read_ahead(residual, step, kernel, M, bucket)) if hasattr(kernel, "state_bytes") else {}
             attended = kernel.run(u, step, caches, mixed, merge=not later, **reads)
         else:
-            self._mix_each(u, step, caches, mixed, ahead=self._read_ahead(residual, self.kernel, step.num_lanes, bucket))
+            self._mix_each(u, step, caches, mixed, ahead=self._read_ahead(residual, step, self.kernel, step.num_lanes, bucket))
         self._after_the_mixers(residual, mixed, attended, M, bucket)
 
-    def _read_ahead(self, residual: Residual, kernel, lanes: int, bucket: int) -> list:
-        """The weights of the products behind the mixers that the mixers' launch brings into the caches."""
-        room = AHEAD_BYTES - lanes * getattr(kernel, "state_bytes", AHEAD_BYTES)
-        products = [(self.library_out[bucket], self.f_out)]
+    def first_product(self) -> tuple:
+        """How each size of step runs the product that the layer reads first (whether the library does, no slabs, its tiles), and
+        that product's weight in fragment order or None."""
+        return self.library_in, None, self.tiles_in, self.f_in
+
+    def _read_ahead(self, residual: Residual, step, kernel, rows: int, bucket: int) -> list:
+        """The weights of the products behind the mixers that the mixers' launch brings into the caches: of those that this step
+        reads in fragment order, tile by tile as the launch deals them out."""
+        room = AHEAD_BYTES - rows * getattr(kernel, "state_bytes", AHEAD_BYTES)
+        if bucket == BEYOND or (hasattr(kernel, "key_bytes") and rows * kernel.key_bytes(step) > AHEAD_KEY_BYTES):
+            return []
+        products = [(self.library_out, self.split_out, self.tiles_out, self.f_out)]
         if self.gate_up is not None:
-            products += [(self.library_gate_up[bucket], self.f_gate_up), (self.library_down[bucket], self.f_down)]
+            products += [(self.library_gate_up, None, self.tiles_gate_up, self.f_gate_up),
+                         (self.library_down, self.split_down, self.tiles_down, self.f_down)]
+        if residual.next_fusion is not None:
+            products.append(residual.next_fusion.first_product())
         weights = []
-        for library, fragments in products + [(False, residual.next_first)]:
-            if library or fragments is None:
+        for library, slabs, tiles, fragments in products:
+            if library[bucket] or (slabs and slabs[bucket]) or tiles[bucket] != 1 or fragments is None:
                 continue
             room -= fragments.numel() * fragments.element_size()
             if room < 0:
@@ -1013,6 +1028,11 @@ class AttentionMamba2Step:
         # launches of the step's layers use them one after the other and leave zeros)
         heads = self.attention.spec.num_kv_heads
         return [StepTable(f"mixer_arrived_{heads}", lambda lanes, tokens: lanes * heads, lambda out, packed: None)]
+
+    def key_bytes(self, step) -> int:
+        a = self.attention.spec
+        keys = int(step.max_seq_len) if not a.window else min(int(step.max_seq_len), a.window)
+        return keys * 2 * 2 * a.num_kv_heads * a.head_dim
 
     def conv_state(self, caches) -> torch.Tensor:
         return caches[self.mamba_name].states["conv"]

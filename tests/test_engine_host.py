@@ -157,6 +157,47 @@ def test_a_part_with_a_method_of_its_own_keeps_it_in_short_prompts():
     assert scan.takes_beside(None, step, cache, None, None) is False
 
 
+def test_weights_are_read_ahead_only_where_the_step_reads_them_so():
+    """What the launch of the mixers brings into the caches: the products behind it that this size of step runs tile by tile from
+    fragments, the next layer's first one by that layer's plan, as many as fit beside the states, none beside many keys."""
+    from types import SimpleNamespace
+
+    from macllm_infer_amd.parts import fused
+    from macllm_infer_amd.parts.base import Residual
+    sizes = fused.BUCKETS + 1
+    weight = lambda mib: torch.empty(mib << 20, dtype=torch.uint8)
+
+    def layer(**plan):
+        fusion = object.__new__(fused.LayerFusion)
+        fusion.gate_up, fusion.f_in, fusion.f_out, fusion.f_gate_up, fusion.f_down = object(), weight(6), weight(4), weight(8), weight(5)
+        for name in ("library_in", "library_out", "library_gate_up", "library_down"):
+            setattr(fusion, name, (plan.get(name, False),) * fused.BUCKETS + (True,))
+        for name in ("split_out", "split_down"):
+            setattr(fusion, name, (plan.get(name, 0),) * sizes)
+        for name in ("tiles_in", "tiles_out", "tiles_gate_up", "tiles_down"):
+            setattr(fusion, name, (plan.get(name, 1),) * sizes)
+        return fusion
+
+    kernel = SimpleNamespace(state_bytes=1 << 20, key_bytes=lambda step: step.max_seq_len * 512)
+
+    def read(own, following, rows=1, bucket=0, context=2048, kernel=kernel):
+        residual = Residual(torch.empty(1))
+        residual.next_fusion = following
+        weights = own._read_ahead(residual, SimpleNamespace(max_seq_len=context), kernel, rows, bucket)
+        names = {id(own.f_out): "out", id(own.f_gate_up): "gate_up", id(own.f_down): "down", id(following.f_in): "in"}
+        return [names[id(one)] for one in weights]
+
+    whole = ["out", "gate_up", "down", "in"]
+    assert read(layer(), layer()) == whole
+    assert read(layer(), layer(library_in=True)) == whole[:3] and read(layer(), layer(tiles_in=2)) == whole[:3]
+    assert read(layer(library_out=True), layer()) == whole[1:] and read(layer(split_down=4), layer()) == ["out", "gate_up", "in"]
+    assert read(layer(tiles_gate_up=-1), layer()) == ["out", "down", "in"]
+    assert read(layer(), layer(), bucket=fused.BEYOND) == []
+    assert read(layer(), layer(), rows=8) == whole[:3] and read(layer(), layer(), rows=24) == whole[:1] and read(layer(), layer(), rows=25) == []
+    assert read(layer(), layer(), rows=8, context=10240) == whole[:3] and read(layer(), layer(), rows=8, context=10241) == []
+    assert read(layer(), layer(), context=1 << 20) == [] and read(layer(), layer(), kernel=object()) == []
+
+
 def test_refused_steps_change_nothing(host_ops, tmp_path):
     engine, cfg, tensors = engine_for("A", tmp_path, capacity=32, page=8, requests=2)
     engine.add_request("a")

@@ -870,9 +870,11 @@ def test_the_output_projection_may_merge_the_runs_of_keys(monkeypatch):
 @pytest.mark.parametrize("prompt", [5, 37, 64])
 def test_weights_read_ahead_change_nothing(monkeypatch, prompt):
     """Short prompts and single tokens whose mixers' launches bring the next products' weights into the caches, launched and
-    replayed: the logits of an engine that reads nothing ahead, bit for bit."""
+    replayed: the logits of an engine that reads nothing ahead, bit for bit.  Both kinds of launch are given the weights of the
+    layer's other three products and of the next layer's first, and none where there is no room."""
     from macllm_infer_amd import Engine, Lane
     from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.kernels import ops
     from macllm_infer_amd.parts import fused
     from macllm_infer_amd.weights.random_init import random_tensors
     config = FalconH1Config.from_dict(dict(tiny_configs.TINY_C, hidden_size=256, num_hidden_layers=3, num_attention_heads=8,
@@ -880,7 +882,18 @@ def test_weights_read_ahead_change_nothing(monkeypatch, prompt):
                                            mamba_d_ssm=384, mamba_d_state=128, mamba_n_groups=1, mamba_chunk_size=128,
                                            max_position_embeddings=512))
     tensors = random_tensors(config, 6, torch.bfloat16, "unit")
-    results = {}
+    results, read = {}, {}
+
+    def spied(name, weights_of):
+        launch = getattr(ops, name)
+
+        def call(*args, **kwargs):
+            read.setdefault((room, name), set()).add(tuple(one.data_ptr() for one in weights_of(kwargs)))
+            return launch(*args, **kwargs)
+        monkeypatch.setattr(ops, name, call)
+
+    spied("mixer_decode", lambda kwargs: kwargs["ahead"])
+    spied("ssd_prefill", lambda kwargs: kwargs["beside"].ahead if kwargs.get("beside") is not None else (torch.empty(0),))
     for room in (0, 28 << 20):
         monkeypatch.setattr(fused, "AHEAD_BYTES", room)
         engine = Engine(config=config, tensors=tensors, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=2048,
@@ -892,6 +905,10 @@ def test_weights_read_ahead_change_nothing(monkeypatch, prompt):
         for turn in range(4):
             rows.append(engine.step([Lane(name, [7 + turn], [0]) for name in range(1 + turn)]).float().cpu())
         results[room] = torch.cat(rows)
+        weights = [[getattr(block.fusion, name).data_ptr() for name in ("f_in", "f_out", "f_gate_up", "f_down")] for block in engine.model.blocks]
+        following = [row[:1] for row in weights[1:]] + [[]]
+        want = {tuple(row[1:] + after) for row, after in zip(weights, following)} if room else {()}
+        assert read[room, "mixer_decode"] == want and read[room, "ssd_prefill"] == want
     assert torch.equal(results[0], results[28 << 20]) and torch.isfinite(results[0]).all()
 
 
