@@ -668,7 +668,7 @@ static size_t fused_gemm_lds(int MT, int pro, int K, int M, int staged = 0) {
 // layer of a decode step.  Such a launch is bound by a chain of round trips (its arguments, the weights, the rows that the
 // launch before has just written on other dies, LDS) and by its instructions (64 of them cost a wave 0.1 us), not by
 // bandwidth, so: what does not change with the sizes is fixed at compile time, all of a wave's weights and rows are asked
-// for before the first product (EXACT: CH chunks of 32 columns a wave; longer K in two buffers of CH chunks), the partial
+// for before the first product (EXACT: CH chunks of 32 columns a wave; other runs in two buffers of CH chunks), the partial
 // tiles lie in LDS as they leave the matrix cores, and one wave a tile of 16 rows finishes it, four neighbouring features
 // a lane, behind the only barrier.  The sums of a tile have the order of fused_gemm_kernel's: the waves' runs of K, each
 // in order, then the waves in order.  One behind the other, the weights of 36 layers in turn (one MI355X): 4,096 x 1,024
@@ -998,17 +998,38 @@ static void launch_skinny_scaled(const SkinnyParams& p, bool tiled, dim3 blocks,
   else skinny_kernel<MT, EPI, WAVES, CH, EXACT, false, true><<<blocks, WAVES * WAVE, 0, stream>>>(p);
 }
 
-// All of a wave's run of K at once where that is a fixed number of chunks (K of 512 and 1,024 over four waves, 2,048 over
-// eight), else two buffers of a few chunks in turn: eight waves of a long K wait for each other's registers, not for
-// latency.  At 8 rows two buffers of 2 / 3 / 4 / 6 chunks take 15.5 / 15.8 / 19.5 / 20.5 us for 8,728 x 3,072 (all 12 chunks of
-// a wave at once 16.6), 29.6 / 29.1 / 38.4 / 40.0 for 24,576 x 3,072, 7.5 / 7.4 / 8.5 / 8.9 for 3,072 x 4,608.
+// All of a wave's run of K at once where the waves' runs are the same 4 to 8 whole chunks (K of 512 to 1,024 in steps of 128
+// over four waves, of 1,280 to 2,048 in steps of 256 over eight): the instance of that many chunks, without a question what is
+// past the run.  One behind the other, two buffers (as below) | at once, of N x K with the weights of 24 layers in turn, us (one
+// MI355X): 4,096 x 512 / 768 / 1,024 / 1,280 / 1,536 / 2,048 behind a row scale at one row 3.9 | 3.4, 4.1 | 3.7, 4.3 | 4.0, 4.5 | 4.1, 5.0 |
+// 4.7, 6.4 | 5.4; at 32 rows 5.7 | 4.3, 5.9 | 5.0, 6.2 | 5.7, 7.0 | 6.2, 7.6 | 6.7, 10.7 | 8.1; 1,024 features into the stream at 8 rows
+// 2.9 | 2.6, 3.4 | 3.1, 3.5 | 3.4, 4.0 | 3.7, 4.0 | 3.9, 5.1 | 4.2.
+// Other runs in two buffers: of the fewest chunks that hold the run in both (2 / 3 / 4 chunks a buffer: 4,096 x 256 at 32 rows 4.5 / 5.0 /
+// 5.5; 1,024 x 1,056 there 5.3 / 4.9 / 5.4; 4,096 x 1,824 7.8 / 8.8 / 7.6; at one row 3.4 / 3.5 / 3.6, 3.5 / 3.4 / 3.6, 5.7 / 6.1 / 5.4; four
+// waves have no instance of 3, whose runs of 5 and 6 take 3 to 5 % less with it, and at more than 32 rows 2 for all: 4,096 x 800 5.9 /
+// 6.9 / 6.3).  Longer ones in buffers of 3: eight waves of a long K wait for each other's registers, not for latency (4,096 x
+// 2,080 at one row 6.5 / 6.4 / 6.6, x 4,128 9.5 / 8.9 / 9.5, at 32 rows 14.8 / 14.2 / 15.6; 24,576 x 3,072 at 8 rows 28.0 / 27.9 / 31.9).
 template <int MT, int EPI>
 static void launch_skinny_sized(const SkinnyParams& p, bool tiled, int waves, dim3 blocks, hipStream_t stream) {
-  if (waves == 4 && p.chunks == 32) launch_skinny_scaled<MT, EPI, 4, 8, true>(p, tiled, blocks, stream);
-  else if (waves == 8 && p.chunks == 64) launch_skinny_scaled<MT, EPI, 8, 8, true>(p, tiled, blocks, stream);
-  else if (MT == 1 && waves == 4 && p.chunks == 16) launch_skinny_scaled<1, EPI, 4, 4, true>(p, tiled, blocks, stream);
-  else if (waves == 4) launch_skinny_scaled<MT, EPI, 4, MT <= 2 ? 4 : 2, false>(p, tiled, blocks, stream);
-  else launch_skinny_scaled<MT, EPI, 8, MT == 1 ? 3 : 2, false>(p, tiled, blocks, stream);
+  const int run = (p.chunks + waves - 1) / waves;
+#define RUN(WAVES_, CH_, EXACT_) return launch_skinny_scaled<MT, EPI, WAVES_, CH_, EXACT_>(p, tiled, blocks, stream)
+  if (p.chunks % waves == 0) {
+    if (waves == 4 && run == 4) RUN(4, 4, true);
+    if (waves == 4 && run == 5) RUN(4, 5, true);
+    if (waves == 4 && run == 6) RUN(4, 6, true);
+    if (waves == 4 && run == 7) RUN(4, 7, true);
+    if (waves == 4 && run == 8) RUN(4, 8, true);
+    if (waves == 8 && run == 5) RUN(8, 5, true);
+    if (waves == 8 && run == 6) RUN(8, 6, true);
+    if (waves == 8 && run == 7) RUN(8, 7, true);
+    if (waves == 8 && run == 8) RUN(8, 8, true);
+  }
+  if (waves == 4 && (run <= 4 || MT > 2)) RUN(4, 2, false);
+  if constexpr (MT <= 2)
+    if (waves == 4) RUN(4, 4, false);
+  if (run == 7 || run == 8) RUN(8, 4, false);
+  RUN(8, 3, false);
+#undef RUN
 }
 
 template <int MT>

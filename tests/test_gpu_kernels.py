@@ -1215,6 +1215,22 @@ def _odd_rows(rows, columns, dtype):
     return torch.full((rows, columns + 3), float("nan"), dtype=dtype, device=DEV)[:, :columns]
 
 
+@pytest.mark.parametrize("M", [1, 16, 30, 48, 64])
+@pytest.mark.parametrize("K", [384, 512, 640, 672, 768, 896, 992, 1024, 1056, 1280, 1536, 1760, 1792, 2048, 2304])
+def test_a_wave_s_run_of_a_product_is_the_same_sum_in_flight_at_once_or_in_buffers(ops, M, K):
+    """Runs of 4 to 8 whole chunks a wave, shorter, longer and uneven ones: the general kernel's sums, whose waves take the same
+    runs in the same order, bit for bit; behind a row scale of the width's partial sums too (one tile of rows)."""
+    N = 148
+    x, W = rand(M, K, seed=410, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=411, scale=0.1, dtype=torch.bfloat16).to(DEV)
+    fragments, sums = ops.fragment_order(W), (rand(K // 16, 16 * (-(-M // 16)), seed=412).abs() * 16.0 + 1.0).to(DEV)
+    for scale in (None, ops.RowScale(sums, K, 1e-5)) if M <= 16 else (None,):
+        for operand in (None, fragments) if scale is None else (fragments,):
+            got, want = torch.empty(M, N, device=DEV), _odd_rows(M, N, torch.float32)
+            for out in (got, want):
+                ops.fused_gemm(W, None, out, x=x, fragments=operand, row_scale=scale)
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M, N, K", [(1, 65536, 512), (16, 4112, 1024), (37, 2000, 2080), (64, 1040, 2048)])
 def test_activations_of_a_product_are_the_same_bits_in_both_of_its_kernels(ops, M, N, K):
     """SiLU behind the gate and behind the conv step, of numbers as far from zero as its exponential reaches: the kernel of
