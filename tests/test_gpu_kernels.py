@@ -2226,6 +2226,25 @@ def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H
         assert torch.isfinite(joined.float()).all() and torch.equal(apart, joined)
 
 
+@pytest.mark.parametrize("H, P, N, Hq, Hkv, dh", [(24, 64, 128, 8, 2, 64), (3, 64, 128, 4, 1, 64), (4, 128, 256, 12, 2, 128)])
+def test_weights_read_ahead_beside_a_scan_change_no_bit(ops, monkeypatch, H, P, N, Hq, Hkv, dh):
+    """The same with weights of one tile, of fewer tiles than dies and of tiles that are no multiple of 8 or of a workgroup's piece,
+    which the second launch brings into the caches; more than four are refused."""
+    sizes = ((12, 64), (100, 32), (4120, 1024), (136, 4640))
+    weights = [ops.fragment_order(torch.ones(rows, width, dtype=torch.bfloat16, device=DEV)) for rows, width in sizes]
+    plain, given = ops.PromptBeside, []
+
+    def with_weights(*args):
+        given.append(plain(*args, ahead=weights))
+        return given[-1]
+    monkeypatch.setattr(ops, "PromptBeside", with_weights)
+    test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, [1, 5, 128, 64], [0, 700, 0, 33], None, 4096)
+    assert len(given) == 2 and all(w.eq(1).sum() == rows * width for w, (rows, width) in zip(weights, sizes))
+    weights.append(weights[0])
+    with pytest.raises(ops.KernelError):
+        test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, [37], [0], None, 2048)
+
+
 def test_prompt_attention_beside_a_scan_is_refused_where_it_does_not_fit(ops):
     state = torch.zeros(2, 4, 64, 128, device=DEV)
     q, out = torch.zeros(8, 1024, dtype=torch.bfloat16, device=DEV), torch.zeros(8, 512, dtype=torch.bfloat16, device=DEV)
