@@ -725,8 +725,9 @@ constexpr int skinny_early_sums() {
   return wanted < most ? wanted : most;
 }
 
-// EPI_PLAIN ... EPI_TANH as above.  SCALED: behind a row scale.  TILED: W in fragment order.  Row y of the grid takes the MT tiles of 16 rows from row 16 MT y on; with several of them a row of
-// the grid is a multiple of 8 workgroups, so that those of a tile of features run on one die and its weights leave memory once.
+// EPI_PLAIN ... EPI_TANH as above.  SCALED: behind a row scale.  TILED: W in fragment order.  Row y of the grid takes the MT
+// tiles of 16 rows from row 16 MT y on; with several of them a row of the grid is a multiple of 8 workgroups, so that those of a
+// tile of features run on one die and its weights leave memory once.
 template <int MT, int EPI, int WAVES, int CH, bool EXACT, bool SCALED, bool TILED>
 __global__ void __launch_bounds__(WAVES * WAVE) skinny_kernel(SkinnyParams p) {
   __shared__ floatx4 red[WAVES][MT][WAVE];
@@ -1800,7 +1801,8 @@ struct MixerParams {
   int page_shift;                          // log2 of page_size, or -1
   int heads_a_group;                       // query heads of a kv head
   // the context of a request is cut into runs of split_keys keys, one workgroup each; their
-  // partial results [M, Hq, splits, DH + 2] = (maximum, normalizer, sums) are merged by mixer_merge_kernel
+  // partial results [M, Hq, splits, DH + 2] = (maximum, normalizer, sums) are merged by the last of them (arrived), by
+  // mixer_merge_kernel or by the output product
   int splits;
   int split_keys;
   float* partial;
@@ -2217,7 +2219,10 @@ __global__ void __launch_bounds__(MX_THREADS) mixer_decode_ahead_kernel(MixerPar
 // keys.  Measured on one MI355X (mixer + merge of a layer, head size 64, 2 kv heads; runs of
 // 256 / 512 / 1,024 keys; contexts inside graphs made for 4,096 and 8,192 keys): 1 token at 2,100 keys
 // 11.3 / 12.0 / 15.0 us; 8 tokens at 2,100 keys 15.1 / 14.0 / 16.6, at 6,000 keys 20.3 / 17.2 / 17.8;
-// 64 tokens at 2,100 keys 61.0 / 56.0 / 52.0, at 6,000 keys 100 / 85 / 80.  So: the longest run that still
+// 64 tokens at 2,100 keys 61.0 / 56.0 / 52.0, at 6,000 keys 100 / 85 / 80.  (Merged inside the launch, as in a step, the runs' length
+// counts for less: 1 token at 2,100 keys 9.4 / 10.2 / 12.7, 8 at 2,100 11.6 / 11.5 / 14.0, at 6,000 13.9 / 13.9 / 14.9, 64 at 2,100 40.3 / 41.9 /
+// 41.3, at 6,000 65.7 / 65.7 / 64.9; the line costs 16 tokens at 2,100 keys 6 % and 32 tokens 7 %: 13.5 / 14.4 / 15.6 and 22.0 / 22.8 /
+// 23.7.)  So: the longest run that still
 // leaves MX_SPLIT_BLOCKS workgroups (up to 512 keys for steps of up to 16 tokens, 1,024 beyond), and never
 // more than 16 runs for a request.  `span`: the most keys a request of the step can have.
 extern "C" int mi_mixer_split_keys(int M, int Hkv, int dh, int page_size, long span) {
@@ -2237,14 +2242,15 @@ extern "C" int mi_mixer_split_keys(int M, int Hkv, int dh, int page_size, long s
 // (token, kv head): one per run while the step is small, fewer (each walks over several runs) once the step has
 // MX_WALK_BLOCKS of them anyway.  `span`: the most keys a request of the step can have.
 // A step of half as many requests as that, or of heads of 128 a quarter, gives each request's kv head to one workgroup, which
-// writes the attended heads itself: the merge's launch (4.7 us) counts for more than the longer walk, up to contexts of
-// MX_WHOLE_SPAN keys.  Mixer and merge of a layer in us, several workgroups a request | one: heads of 64, 64 tokens behind
-// 300 keys 33.8 | 29.2, 1,500 39.9 | 34.9, 4,500 62.6 | 64.3; 32 tokens behind 1,500 24.9 | 26.5.  (Contexts of all lengths up to
-// 3,500 keys wait for the longest walk: a step of 64 of them takes 2,870 and 2,884.)  Heads
-// of 128 over states of 128 x 256, 32 tokens behind 300 keys 57.1 | 54.4, 1,500 64.9 | 58.8, but 4,000 88 | 92.  The line at
-// 128 workgroups for those heads (256 before | 128): 8 tokens behind 4,500 keys 37.7 | 33.8, 16 behind 2,500 48.9 | 42.8, behind
-// 4,500 63.0 | 50.4, 32 behind 2,500 79.0 | 71.0; their runs of 512 keys from 64 workgroups on (128 before | 64): 8 tokens
-// behind 300 keys 21.8 | 18.2, behind 1,500 26.2 | 23.7, but 4 behind 2,500 17.7 | 18.8.
+// writes the attended heads itself: the partial results, their counter and the merge count for more than the longer walk, up to
+// contexts of MX_WHOLE_SPAN keys.  Mixers of a layer in us, runs merged in the launch, several workgroups a request | one: heads of
+// 64, 64 tokens behind 300 keys 30.2 | 28.6, 1,500 37.7 | 35.9, 2,000 38.5 | 37.8 (of lengths from 100 to 2,000, which wait for the longest
+// walk, 33.9 | 36.8), 4,000 51.9 | 54.3; 48 tokens behind 300 22.9 | 20.6, 1,500 28.9 | 31.8; 32 behind 300 16.9 | 16.2, 1,500 22.2 | 26.8.  Heads
+// of 128 over states of 128 x 256, 32 tokens behind 300 keys 53.9 | 53.6, 1,500 61.7 | 57.5, 2,000 59.6 | 59.9, 4,000 73.7 | 86.4; 16 behind
+// 300 30.6 | 28.5, 1,500 36.1 | 42.2, 4,000 39.5 | 76.8.  The line at 128 workgroups for those heads (256 before | 128, the merge a launch
+// of its own, as in the next): 8 tokens behind 4,500 keys 37.7 | 33.8, 16 behind 2,500 48.9 | 42.8, behind 4,500 63.0 | 50.4, 32 behind
+// 2,500 79.0 | 71.0; their runs of 512 keys from 64 workgroups on (128 before | 64): 8 tokens behind 300 keys 21.8 | 18.2, behind
+// 1,500 26.2 | 23.7, but 4 behind 2,500 17.7 | 18.8.
 extern "C" int mi_mixer_runs(int M, int Hkv, int dh, int page_size, long span, int* run_keys, int* runs) {
   const int keys = mi_mixer_split_keys(M, Hkv, dh, page_size, span);
   if (keys <= 0 || !run_keys || !runs) return ERR_BAD_ARGUMENT;

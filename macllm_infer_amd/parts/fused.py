@@ -114,9 +114,8 @@ PAD_MARGIN = 0.95
 FORCE_PADDING: Optional[bool] = None      # tests: True or False instead of the clock
 # The attended heads of a decode step come in runs of keys, which the mixers' launch merges itself by the counters of the
 # step (``AttentionMamba2Step.step_tables``).  The output projection can merge them in its prologue instead, every workgroup
-# of it again, and starts behind a read of the runs: the 0.5B shape at 1 row 1,032 us a step with the counters, 1,081 that way
-#,
-# at 8 rows 1,198 with the counters and 1,252 with the merge as a launch of its own.  No step takes that way by itself.
+# of it again, and starts behind a read of the runs: the 0.5B shape at 1 row 1,032 us a step with the counters, 1,081 that way;
+# at 8 rows 1,198 with the counters, 1,252 with the merge as a launch of its own.  No step takes that way unless it is forced.
 FORCE_MERGE_LATER: Optional[bool] = None  # True: the output projection merges, where it takes the step
 _padding_wins: Dict[tuple, tuple] = {}
 # The mixers of a small step wait for round trips and leave the memory idle, so their launch also brings the weights of the
@@ -126,6 +125,8 @@ _padding_wins: Dict[tuple, tuple] = {}
 # contexts of 2,048: 1 row 1,018 | 956 | 937 | 915, 4 rows 1,071 | 1,036 | 1,028 | 1,025, 8 rows 1,170 | 1,159 | 1,146 | 1,167, 12 rows
 # 1,328 | 1,290 | 1,282 | 1,321, 16 rows 1,367 | 1,329 | 1,325 | 1,374; of 300: 1 row 985 | 920 | 902 | 879, 8 rows 1,123 | 1,080 | 1,074 |
 # 1,116, 16 rows 1,290 | 1,266 | 1,266 | 1,302.  (The 7B shape's 28 MB of output projection: 1 row 1,098 | 1,084, 4 rows 1,196 | 1,225: left out.)
+# Beyond 16 rows, as much as fits without | with: behind 300 keys 20 rows 1,555 | 1,525, 24 1,592 | 1,558, 28 1,628 | 1,603, 32 1,655 | 1,638;
+# behind 2,000 1,668 | 1,668, 1,697 | 1,698, 1,744 | 1,745, 1,806 | 1,809; 24 rows beside a prompt of 515 tokens on the other stream 5,108 | 5,105.
 AHEAD_BYTES = 28 << 20
 # Where a launch has many keys to read it leaves no memory idle: nothing is read ahead beside more than AHEAD_KEY_BYTES of them a
 # layer, by the longest context that the step is made for.  The same shape without | out and gate-up, at 33 MB of keys: 8 rows behind
@@ -149,11 +150,12 @@ CHAIN_MARGIN = 0.97
 # Where the norms are left to the projections, a step of more than 16 rows can have its tiles of 16 rows dealt out
 # to several workgroups per tile of features instead of every workgroup taking them all.  The two projections that
 # feed the stream have few output features (1,024 of them: 64 workgroups, each of which fetches all of the step's
-# rows): with 64 rows over four workgroups 1,024 x 2,048 takes 5.9 us instead of 11.4, at 32 rows 5.7 instead of
-# 7.5, and the same bits come out, so this is a fixed rule up to ROW_TILES_FEATURES output features (3,072 x 7,680
-# gains at 64 rows only, 35 us against 41, and loses below).  The products behind the norms gain less (4,120 x 1,024
-# at 64 rows: 9.4 us against 11.8) and add their rows' partial sums of squares in another order, so for them, and
-# beyond the rule, the clock decides over the chain of layers.  A plan's number: 1 = every workgroup all rows,
+# rows): with 64 rows over four workgroups 1,024 x 2,048 takes 5.1 us instead of 10.4, at 32 rows 5.0 instead of
+# 6.7, and the same bits come out, so this is a fixed rule up to ROW_TILES_FEATURES output features (3,072 x 7,680
+# gains at 64 rows only, 32 us against 39, and loses below).  The products behind the norms gain less, or lose (4,120 x
+# 1,024 with the conv step at 64 rows over 1 / 2 / 4 workgroups: 12.1 / 11.1 / 10.2 us, 4,096 x 1,024 7.6 / 7.7 / 8.0), so for
+# them, and beyond the rule, the clock decides over the chain of layers: the same bits where the kernel of small steps takes
+# the product (the general one adds a row's partial sums of squares in another order).  A plan's number: 1 = every workgroup all rows,
 # 2 = over two workgroups, 4 = one tile of 16 rows each.
 ROW_TILES_FEATURES = 2048
 FORCE_ROW_TILES: Optional[int] = None     # tests: this number for all four projections instead of the rule and the clock
@@ -1004,8 +1006,8 @@ def attention_mamba2_step(fusion: "LayerFusion") -> Optional["AttentionMamba2Ste
 class AttentionMamba2Step:
     """Attention beside Mamba2 in steps of single tokens: the conv step of the state-space columns runs in the
     epilogue of the input product, and one launch (``mixer_decode``) rotates q and the new key, writes the new
-    key and value into their cache cell, attends over the request's pages in runs that a small kernel merges,
-    and advances the state-space state by one step with the gate on the way out."""
+    key and value into their cache cell, attends over the request's pages in runs that the workgroup which ends last
+    merges, and advances the state-space state by one step with the gate on the way out."""
 
     def __init__(self, fusion: "LayerFusion"):
         self.attention, self.mamba = fusion.mixers
