@@ -6,7 +6,8 @@
 //                    the choice to the best groups
 //   moe_plan         the step's (token, choice) rows grouped by expert, every expert's rows starting a tile of 16
 //                    places: built on the device by one workgroup, so that no count has to travel to the host and
-//                    the launches that follow depend on the number of tokens alone
+//                    the launches that follow depend on the number of tokens alone; a shared expert's rows may stand
+//                    in front of them, as one expert more
 //   moe_expert_gemm  the grouped product on the matrix cores: a tile's rows (gathered from the tokens' rows, or
 //                    the places themselves) with its expert's matrix; epilogue: plain, or the clamped gated
 //                    activation of a gate tile and an up tile
@@ -228,18 +229,20 @@ struct PlanArgs {
   int* ranks;
   const float* weights;             // with place_weight: the choices' weights, laid beside the places (padding gets 0)
   float* place_weight;
+  int shared;                       // a shared expert's rows: rows 0 .. shared - 1 of the step stand at the places of these numbers, as expert E
 };
 
 // By one workgroup; a choice of E or beyond is an identity expert and gets the place -1.
 __device__ __forceinline__ void plan_rows(const PlanArgs& a, int* counts, int* offsets) {
   const int tid = threadIdx.x;
   const int threads = blockDim.x;
+  const int shared_tiles = (a.shared + a.pad - 1) / a.pad;
   for (int e = tid; e < a.E; e += threads) counts[e] = 0;
   for (int i = tid; i < a.capacity; i += threads) {
-    a.source[i] = -1;
+    a.source[i] = i < a.shared ? i : -1;
     if (a.place_weight) a.place_weight[i] = 0.f;
   }
-  for (int t = tid; t < a.capacity / a.pad; t += threads) a.tile_expert[t] = -1;
+  for (int t = tid; t < a.capacity / a.pad; t += threads) a.tile_expert[t] = t < shared_tiles ? a.E : -1;
   __syncthreads();
   for (int i = tid; i < a.entries; i += threads) {
     const int expert = a.chosen[i];
@@ -248,7 +251,7 @@ __device__ __forceinline__ void plan_rows(const PlanArgs& a, int* counts, int* o
   __syncthreads();
   // where every expert's places begin: whole tiles, an inclusive sum over the wave in turns of 64 experts
   if (tid < WAVE) {
-    int before = 0;
+    int before = shared_tiles * a.pad;
     for (int e0 = 0; e0 < a.E; e0 += WAVE) {
       const int e = e0 + tid;
       const int places = e < a.E ? (counts[e] + a.pad - 1) / a.pad * a.pad : 0;
@@ -290,14 +293,16 @@ __global__ void __launch_bounds__(1024) moe_plan_kernel(PlanArgs a) {
 static int check_plan(const PlanArgs& a) {
   if (a.place_weight && !a.weights) return ERR_BAD_ARGUMENT;
   if (!a.chosen || !a.source || !a.place || !a.tile_expert || !a.ranks || a.entries <= 0 || a.top <= 0 || a.E <= 0 || a.pad <= 0 ||
-      a.capacity % a.pad != 0 || a.capacity < a.entries + a.E * (a.pad - 1))
+      a.capacity % a.pad != 0 || a.shared < 0 || (a.shared > 0 && a.place_weight) ||
+      a.capacity < (a.shared + a.pad - 1) / a.pad * a.pad + a.entries + a.E * (a.pad - 1))
     return ERR_BAD_ARGUMENT;
   return a.E > MOE_MAX_EXPERTS ? ERR_UNSUPPORTED_SIZE : 0;
 }
 
 extern "C" int mi_moe_plan(const int* chosen, int entries, int top, int E, int pad, int capacity, int* source, int* place,
-                           int* tile_expert, int* ranks, const float* weights, float* place_weight, hipStream_t stream) {
-  const PlanArgs a = {chosen, entries, top, E, pad, capacity, source, place, tile_expert, ranks, weights, place_weight};
+                           int* tile_expert, int* ranks, const float* weights, float* place_weight, int shared,
+                           hipStream_t stream) {
+  const PlanArgs a = {chosen, entries, top, E, pad, capacity, source, place, tile_expert, ranks, weights, place_weight, shared};
   const int code = check_plan(a);
   if (code) return code;
   moe_plan_kernel<<<1, 1024, 0, stream>>>(a);
@@ -322,9 +327,9 @@ __global__ void __launch_bounds__(1024) moe_route_plan_kernel(RouteArgs route, P
 extern "C" int mi_moe_route_plan(const float* logits, long ld, int T, int E, int top, const float* correction, float scale,
                                  float eps, int mode, int renormalize, int groups, int kept_groups, int* chosen,
                                  float* weights, float* gate, int experts, int pad, int capacity, int* source, int* place,
-                                 int* tile_expert, int* ranks, float* place_weight, hipStream_t stream) {
+                                 int* tile_expert, int* ranks, float* place_weight, int shared, hipStream_t stream) {
   const RouteArgs route = {logits, ld, T, E, top, correction, scale, eps, mode, renormalize, groups, kept_groups, chosen, weights, gate};
-  const PlanArgs plan = {chosen, T * top, top, experts, pad, capacity, source, place, tile_expert, ranks, weights, place_weight};
+  const PlanArgs plan = {chosen, T * top, top, experts, pad, capacity, source, place, tile_expert, ranks, weights, place_weight, shared};
   int code = check_route(route);
   if (!code) code = check_plan(plan);
   if (code) return code;

@@ -79,7 +79,7 @@ _SIGNATURES = {
         "mi_moe_route": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr, _c_float, _c_float, _c_int, _c_int, _c_int, _c_int,
                          _c_ptr, _c_ptr, _c_ptr, _c_ptr],
         "mi_moe_plan": [_c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
-                        _c_ptr],
+                        _c_int, _c_ptr],
         "mi_moe_expert_gemm": [_c_ptr, _c_int, _c_long, _c_int, _c_ptr, _c_long, _c_long, _c_int, _c_int, _c_ptr, _c_ptr,
                                _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_ptr, _c_ptr, _c_int,
                                _c_long, _c_ptr],
@@ -88,7 +88,7 @@ _SIGNATURES = {
                            _c_ptr],
         "mi_moe_route_plan": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr, _c_float, _c_float, _c_int, _c_int, _c_int,
                               _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
-                              _c_ptr, _c_ptr],
+                              _c_ptr, _c_int, _c_ptr],
     },
     "linear_state": {
         "mi_linear_state_scan": [_c_ptr, _c_int, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr,
@@ -958,6 +958,21 @@ def moe_tile_rows(tokens: int, top_k: int, num_experts: int, whole_pieces: bool 
     return MOE_WIDEST_TILE_ROWS if 10 * fills[0] > 11 * fills[1] else MOE_WIDE_TILE_ROWS
 
 
+def moe_shared_grouped(tokens: int, width: int, hidden: int) -> bool:
+    """Whether a shared expert like the routed ones (``width`` by ``hidden``, bfloat16) runs as one more of them in the
+    grouped products of a step: three launches less (two products and the activation between them, 10 us of small steps, 25
+    of prompts), where the matrices are small enough that those launches wait for little else.  us of the whole
+    feed-forward, apart | grouped, by tokens (experts x hidden x width, choices a token):
+
+    * 16 x 1,024 x 512, 3: 1 27.7 | 20.4, 12 35.3 | 27.4, 64 62.0 | 45.8, 256 60.9 | 44.2, 777 72.8 | 52.5, 1,554 94.5 |
+      77.5, 4,096 171 | 162
+    * 64 x 1,024 x 512, 6: 12 46.3 | 41.6, 64 110 | 91, 512 105.5 | 103.9, 1,554 159 | 167 (another tile), 2,048 209 | 167
+    * 64 x 2,048 x 1,024, 6: 12 131 | 121, 64 255 | 239, 128 302 | 296, 256 390 | 402, 1,024 325 | 353, 2,048 478 | 443
+    * 8 x 3,072 x 3,072, 2: 1 65.9 | 70.0, 12 134 | 129, 64 216 | 227, 512 258 | 225, 1,024 318 | 335, 4,096 968 | 1,000"""
+    first = 2 * width * hidden
+    return first <= 1 << 21 or (first <= 1 << 22 and tokens <= 128)
+
+
 ROUTINGS = {"softmax_then_top": 0, "top_then_softmax": 1, "sigmoid_then_top": 2}
 
 
@@ -1007,12 +1022,15 @@ class MoePlan:
     int32 [capacity / pad] = the expert of every tile of ``pad`` places (-1: an unused tile).  A choice of
     ``num_experts`` or beyond (an expert without matrices) stands nowhere: its place is -1.  Every expert's rows
     start a tile; ``capacity`` depends on the number of tokens alone.  ``place_weight`` (float32 [capacity], if asked for):
-    the weight of the choice that stands at a place (padding: 0)."""
+    the weight of the choice that stands at a place (padding: 0).  ``shared``: the step's rows stand once more in front,
+    token t at place t, as the rows of an expert of the number ``num_experts``."""
 
-    def __init__(self, tokens: int, top_k: int, num_experts: int, pad: Optional[int], device, weighted: bool = False):
+    def __init__(self, tokens: int, top_k: int, num_experts: int, pad: Optional[int], device, weighted: bool = False,
+                 shared: bool = False):
         pad = moe_tile_rows(tokens, top_k, num_experts) if pad is None else int(pad)
         self.pad, self.tokens, self.top_k = pad, tokens, top_k
-        self.capacity = -(-(tokens * top_k + num_experts * (pad - 1)) // pad) * pad
+        self.shared_rows = tokens if shared else 0
+        self.capacity = -(-self.shared_rows // pad) * pad + -(-(tokens * top_k + num_experts * (pad - 1)) // pad) * pad
         self.source = torch.empty((self.capacity,), dtype=torch.int32, device=device)
         self.place = torch.empty((tokens * top_k,), dtype=torch.int32, device=device)
         self.tile_expert = torch.empty((self.capacity // pad,), dtype=torch.int32, device=device)
@@ -1021,17 +1039,18 @@ class MoePlan:
 
 
 def moe_plan(chosen: torch.Tensor, num_experts: int, pad: Optional[int] = None,
-             weights: Optional[torch.Tensor] = None) -> MoePlan:
+             weights: Optional[torch.Tensor] = None, shared: bool = False) -> MoePlan:
     """The plan of the choices ``chosen`` int32 [T, top_k]; with ``weights`` float32 [T, top_k] their weights lie beside
-    the places."""
+    the places; with ``shared`` (and no weights) a shared expert's rows stand in front of the choices."""
     _i32(chosen, "chosen")
     tokens, top_k = chosen.shape
     _need(weights is None or (weights.dtype == torch.float32 and weights.shape == chosen.shape and weights.is_contiguous()
                               and weights.is_cuda), "moe_plan: the weights must be float32 [T, top_k] on the GPU")
-    plan = MoePlan(tokens, top_k, num_experts, pad, chosen.device, weights is not None)
+    _need(not shared or weights is None, "moe_plan: a shared expert's rows have no weights beside their places")
+    plan = MoePlan(tokens, top_k, num_experts, pad, chosen.device, weights is not None, shared)
     _check(_fn("moe", "mi_moe_plan")(_p(chosen), tokens * top_k, top_k, num_experts, plan.pad, plan.capacity, _p(plan.source),
                                      _p(plan.place), _p(plan.tile_expert), _p(plan.ranks), _p(weights),
-                                     _p(plan.place_weight), _stream()),
+                                     _p(plan.place_weight), plan.shared_rows, _stream()),
            "moe_plan", f"(experts={num_experts})")
     return plan
 
@@ -1042,18 +1061,19 @@ ROUTE_PLAN_TOKENS = 64      # steps of up to this many tokens are routed and gro
 def moe_route_plan(logits: torch.Tensor, num_experts: int, top_k: int, correction: Optional[torch.Tensor], scale: float, eps: float,
                    shared_gate: bool, *, experts_with_matrices: int, pad: Optional[int] = None,
                    routing: str = "softmax_then_top", renormalize: bool = True, groups: int = 0, kept_groups: int = 0,
-                   place_weights: bool = False):
-    """``moe_route`` and ``moe_plan`` (``place_weights``: with the weights beside the places) of a step of up to
+                   place_weights: bool = False, shared: bool = False):
+    """``moe_route`` and ``moe_plan`` (``place_weights``: with the weights beside the places; ``shared``) of a step of up to
     ROUTE_PLAN_TOKENS tokens in one launch: (chosen, weights, gate, plan).  ``experts_with_matrices``: the experts that the plan groups rows for (the router's first outputs)."""
     ld, T, chosen, weights, gate = _route_arguments(logits, num_experts, top_k, correction, shared_gate, routing, groups,
                                                     kept_groups, "moe_route_plan")
     _need(T <= ROUTE_PLAN_TOKENS and 0 < experts_with_matrices <= num_experts, "moe_route_plan: the step or its experts do not fit")
-    plan = MoePlan(T, top_k, experts_with_matrices, pad, logits.device, place_weights)
+    _need(not (shared and place_weights), "moe_route_plan: a shared expert's rows have no weights beside their places")
+    plan = MoePlan(T, top_k, experts_with_matrices, pad, logits.device, place_weights, shared)
     _check(_fn("moe", "mi_moe_route_plan")(
         _p(logits), ld, T, num_experts, top_k, _p(correction), float(scale), float(eps),
         ROUTINGS[routing], 1 if renormalize else 0, int(groups), int(kept_groups), _p(chosen),
         _p(weights), _p(gate), experts_with_matrices, plan.pad, plan.capacity, _p(plan.source), _p(plan.place),
-        _p(plan.tile_expert), _p(plan.ranks), _p(plan.place_weight), _stream()), "moe_route_plan", f"(experts={num_experts})")
+        _p(plan.tile_expert), _p(plan.ranks), _p(plan.place_weight), plan.shared_rows, _stream()), "moe_route_plan", f"(experts={num_experts})")
     return chosen, weights, gate, plan
 
 

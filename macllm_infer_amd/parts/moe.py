@@ -32,7 +32,8 @@ class RoutedExperts(FeedForward):
     activation in its epilogue, then down into float32 rows, which a last kernel weights and sums token by token, in
     the order of the token's choices, together with the gated shared expert.  A token's result does not depend on
     which other tokens share its expert's tiles: a row of a tile is summed on its own.  The output is float32.
-    Steps of up to 64 tokens are routed and grouped in one launch; a shared expert whose activation is plain SiLU runs as
+    Steps of up to 64 tokens are routed and grouped in one launch; a bfloat16 shared expert of the routed ones' size and
+    clamped activation runs as one more of them where that pays (``ops.moe_shared_grouped``); one whose activation is plain SiLU runs as
     the dense gated feed-forward does (its activation in the product's epilogue in small steps)."""
     graph_safe = True
     takes_tail = True
@@ -72,13 +73,19 @@ class RoutedExperts(FeedForward):
         # rows of 16-byte pieces for the bfloat16 matrix cores, else the float32 kernel (any width)
         keep = torch.float32 if (build.dtype == torch.float32 or hidden % 8 or inner % 8) else torch.bfloat16
         self.gated = getattr(spec.activation, "gated", True)
+        # a shared expert of the routed ones' size and activation is one more of them: its rows can stand in front of
+        # theirs in the grouped products
+        like_routed = (spec.shared_size == inner and spec.shared_activation == spec.activation != SILU_GLU and self.gated
+                       and not spec.input_weighted and keep == torch.bfloat16 and build.device.type == "cuda"
+                       and get("shared.gate.weight").dtype == get("shared.up.weight").dtype
+                       == get("shared.down.weight").dtype == torch.bfloat16)
+        names = [f"e{number}" for number in range(experts)] + (["shared"] if like_routed else [])
         if self.gated:
-            first = [torch.cat([get(f"e{number}.gate.weight"), get(f"e{number}.up.weight")]) for number in range(experts)]
+            first = [torch.cat([get(f"{name}.gate.weight"), get(f"{name}.up.weight")]) for name in names]
         else:
-            first = [get(f"e{number}.up.weight") for number in range(experts)]
+            first = [get(f"{name}.up.weight") for name in names]
         self.gate_up = torch.stack(first).to(keep).contiguous().to(build.device)
-        self.down = torch.stack([get(f"e{number}.down.weight") for number in range(experts)]) \
-            .to(keep).contiguous().to(build.device)
+        self.down = torch.stack([get(f"{name}.down.weight") for name in names]).to(keep).contiguous().to(build.device)
         # the router's product has float32 sums; a weight stored in bfloat16 beside bfloat16 rows gives exact float32
         # products on the matrix cores, so it stays as it is stored; any other keeps 32 bits and the float32 kernel
         stored = {get("router.weight").dtype} | ({get("shared.sg.weight").dtype} if spec.shared_size is not None and spec.shared_gated else set())
@@ -86,11 +93,14 @@ class RoutedExperts(FeedForward):
             else torch.float32
         router = [get("router.weight").to(route_dtype)]
         self.shared = spec.shared_size is not None
+        self.shared_grouped = like_routed
         if self.shared:
             if spec.shared_gated:
                 router.append(get("shared.sg.weight").to(route_dtype).reshape(1, hidden))
             self.shared_dense = None
-            if spec.shared_activation == SILU_GLU:
+            if like_routed:                       # (its matrices are the last of the routed experts')
+                pass
+            elif spec.shared_activation == SILU_GLU:
                 named = {f"shared.{name}_proj.weight": get(f"shared.{name}.weight") for name in ("gate", "up", "down")}
                 self.shared_dense = SwiGLU(SwiGLUSpec(intermediate_size=spec.shared_size), "shared", named, build)
             else:
@@ -110,10 +120,10 @@ class RoutedExperts(FeedForward):
         if self.shared_dense is not None:
             return self.shared_dense.forward(x)
         act = self.spec.shared_activation
-        gate_up = self.shared_gate_up(x)
+        gate_up = ops.linear(x, self.gate_up[-1], None) if self.shared_grouped else self.shared_gate_up(x)
         activated = torch.empty((x.shape[0], self.spec.shared_size), dtype=gate_up.dtype, device=x.device)
         ops.clamped_glu(gate_up, act.limit, act.alpha, act.up_offset, activated)
-        return self.shared_down(activated)
+        return ops.linear(activated, self.down[-1], None) if self.shared_grouped else self.shared_down(activated)
 
     def forward(self, x: torch.Tensor, tail=None) -> Optional[torch.Tensor]:
         spec = self.spec
@@ -122,14 +132,16 @@ class RoutedExperts(FeedForward):
         how = dict(routing=spec.routing, renormalize=spec.renormalize, groups=spec.groups, kept_groups=spec.kept_groups)
         choice = (logits, spec.router_outputs, spec.top_k, self.correction, spec.route_scale, spec.weight_eps,
                   self.shared and spec.shared_gated)
-        pad = ops.moe_tile_rows(tokens, spec.top_k, spec.num_experts, self.whole_pieces, self.gate_up.dtype,
-                                self.gate_up.shape[1])
+        grouped = self.shared_grouped and ops.moe_shared_grouped(tokens, spec.expert_size, hidden)
+        pad = ops.moe_tile_rows(tokens, spec.top_k + grouped, spec.num_experts + grouped, self.whole_pieces,
+                                self.gate_up.dtype, self.gate_up.shape[1])
+        in_front = dict(shared=True) if grouped else {}
         if tokens <= ops.ROUTE_PLAN_TOKENS:
             _, weights, gate, plan = ops.moe_route_plan(*choice, experts_with_matrices=spec.num_experts, pad=pad,
-                                                         place_weights=spec.input_weighted, **how)
+                                                         place_weights=spec.input_weighted, **how, **in_front)
         else:
             chosen, weights, gate = ops.moe_route(*choice, **how)
-            plan = ops.moe_plan(chosen, spec.num_experts, pad, weights if spec.input_weighted else None)
+            plan = ops.moe_plan(chosen, spec.num_experts, pad, weights if spec.input_weighted else None, **in_front)
         if spec.input_weighted:                # the weights are in the rows: the sum of the experts' outputs is plain
             weights = None
         rows = x if x.dtype == self.gate_up.dtype else x.to(self.gate_up.dtype)
@@ -138,7 +150,9 @@ class RoutedExperts(FeedForward):
                             squared_relu=not self.gated, row_scale=plan.place_weight if spec.input_weighted else None)
         down = torch.empty((plan.capacity, hidden), dtype=torch.float32, device=x.device)
         ops.moe_expert_gemm(inner, plan, self.down, down, gather=False, glu=None)
-        shared_rows = self._shared_rows(x) if self.shared else None
+        shared_rows = None
+        if self.shared:
+            shared_rows = down[:tokens] if grouped else self._shared_rows(x)
         own_rows = x if spec.identity_experts else None
         if tail is not None and (own_rows is None or own_rows.dtype == tail.dtype):
             ops.moe_combine(down, plan, weights, shared_rows, gate, None, own_rows, tail.stream_arguments())

@@ -214,6 +214,71 @@ def test_the_grouped_products_and_the_weighted_sum(dtype, T, experts, top, hidde
     close(got, want, torch.float32, "the weighted sum")
 
 
+@pytest.mark.parametrize("T, experts, top, pad", [(1, 4, 2, 16), (15, 5, 3, 16), (16, 5, 3, 16), (17, 3, 3, 16), (64, 70, 6, 16),
+                                                   (65, 4, 2, 64), (130, 4, 2, 64), (300, 3, 2, 128)])
+def test_a_shared_experts_rows_stand_in_front_of_the_choices(T, experts, top, pad):
+    """Token t at place t, in tiles of an expert of the number behind the last; the choices as without it, as many tiles
+    further on: through either launch."""
+    logits = rand(T, experts + 1, seed=1).to(DEV)
+    chosen, _, _ = ops().moe_route(logits, experts, top, None, 1.0, 0.0, True)
+    want = ref_ops.MoePlan(chosen.cpu(), experts, pad)
+    plans = [ops().moe_plan(chosen, experts, pad, shared=True)]
+    if T <= ops().ROUTE_PLAN_TOKENS:
+        plans.append(ops().moe_route_plan(logits, experts, top, None, 1.0, 0.0, True, experts_with_matrices=experts, pad=pad,
+                                          shared=True)[3])
+    front = -(-T // pad) * pad
+    for plan in plans:
+        assert plan.capacity == front + want.capacity
+        source, tile_expert, place = plan.source.cpu(), plan.tile_expert.cpu(), plan.place.cpu()
+        assert source[:front].tolist() == list(range(T)) + [-1] * (front - T)
+        assert tile_expert[:front // pad].tolist() == [experts] * (front // pad)
+        assert torch.equal(tile_expert[front // pad:], want.tile_expert)
+        live = want.source >= 0                                # (which of an expert's places a choice gets is left open)
+        assert torch.equal(source[front:] >= 0, live) and sorted(place.tolist()) == sorted((want.place + front).tolist())
+        assert source[place.long()].tolist() == [entry // top for entry in range(T * top)]
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 65, 130, 700])
+def test_a_shared_expert_among_the_routed_ones_gives_what_it_gives_apart(T, monkeypatch):
+    """One of the routed experts' size and activation, grouped and in launches of its own, against float64."""
+    from macllm_infer_amd.config import ClampedGLUSpec, RoutedExpertsSpec
+    from macllm_infer_amd.parts.base import BuildContext
+    from macllm_infer_amd.parts.moe import RoutedExperts
+    hidden, inner, experts, top = 72, 40, 5, 2
+    act = ClampedGLUSpec(limit=1.5)
+    spec = RoutedExpertsSpec(num_experts=experts, top_k=top, expert_size=inner, activation=act, shared_size=inner, shared_activation=act)
+    shapes = {"router": (experts, hidden), "shared.sg": (1, hidden)}
+    for name in [f"e{number}" for number in range(experts)] + ["shared"]:
+        shapes.update({f"{name}.gate": (inner, hidden), f"{name}.up": (inner, hidden), f"{name}.down": (hidden, inner)})
+    tensors = {f"m.{name}.weight": (rand(*shape, seed=20 + index) / shape[1] ** 0.5).to(torch.bfloat16)
+               for index, (name, shape) in enumerate(shapes.items())}
+    tensors["m.correction"] = rand(experts, seed=3) * 0.05
+    part = RoutedExperts(spec, "m", tensors, BuildContext(hidden, torch.bfloat16, torch.device(DEV), 4096))
+    x = rand(T, hidden, seed=9).to(torch.bfloat16)
+    double = {name[2:]: value.double() for name, value in tensors.items()}
+    scores = torch.softmax(x.double() @ double["router.weight"].T, dim=-1)
+    chosen = torch.topk(scores + double["correction"], top, dim=-1).indices
+    picked = torch.gather(scores, 1, chosen)
+    picked = picked / picked.sum(-1, keepdim=True)
+
+    def expert(name):
+        gate = (x.double() @ double[f"{name}.gate.weight"].T).clamp(max=1.5)
+        up = (x.double() @ double[f"{name}.up.weight"].T).clamp(-1.5, 1.5)
+        return (gate * torch.sigmoid(1.702 * gate) * (up + 1.0)) @ double[f"{name}.down.weight"].T
+
+    want = torch.sigmoid(x.double() @ double["shared.sg.weight"].T) * expert("shared")
+    for number in range(experts):
+        want += (picked * (chosen == number)).sum(-1, keepdim=True) * expert(f"e{number}")
+    errors = {}
+    for grouped in (True, False):
+        monkeypatch.setattr(ops(), "moe_shared_grouped", lambda *sizes: grouped)
+        got = part.forward(x.to(DEV)).double().cpu()
+        errors[grouped] = float((got - want).norm() / want.norm())
+    # the activation in bfloat16 (2^-9 at most, 2^-9 / sqrt(3) on average, of every addend of an output); apart, the
+    # products before and behind it are rounded too
+    assert errors[True] < 2.0 ** -9 and errors[False] < 3 * 2.0 ** -9, errors
+
+
 # ------------------------------------------------------------------ each mechanism alone against the plain model
 def rounded(tensors, dtype):
     return {name: value.to(dtype).to(torch.float32) for name, value in tensors.items()}
