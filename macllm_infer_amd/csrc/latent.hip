@@ -5,7 +5,8 @@
 //                    the token's cache cell (K page: [latent | turned part], V page, transposed: the latent), and,
 //                    if asked for, the heads' query parts turned into their places beside the latent-space queries
 //   rotate_heads     a part of every head's row turned by position into another matrix
-//   head_gemm        one product per head on the matrix cores (queries into the latent space, attended latents out)
+//   head_gemm        one product per head on the matrix cores (queries into the latent space, attended latents out), with
+//                    rotate_heads beside it if asked for
 //
 // Norms, angles, sines and the turn itself are float32 whatever the activations are.
 #include "mfma_tile.h"
@@ -176,16 +177,64 @@ extern "C" int mi_rotate_heads(const void* x, int dtype, long ld, int col, int h
 
 // ---------------------------------------------------------------- one product per head
 // out[m, out_col + h * out_head_stride + n] = sum_k x[m, x_col + h * x_head_stride + k] * W[h, n, k]
+// With turned.rows the launch has one slice of workgroups more, which turn the heads' position parts (as rotate_heads does,
+// beside the products in place of behind them: it reads and writes other columns).  A decode step of 12 requests over 12
+// layers 1,087 -> 1,077 us (a small launch of a graph costs 0.8 us a layer); 1,554 prompt tokens the same either way.
+template <typename T>
+struct HeadTurns {
+  TurnedHeads<T> heads;             // rows null: none
+  int width;
+  const int* positions;
+  const float* inv_freq;
+  int rotary_dim, interleaved;
+  float magnitude;
+};
+
+// The turns of tokens first .. last - 1 by one workgroup: as many tokens at a time as the LDS holds cosines and sines of.
+template <typename T>
+__device__ __forceinline__ void turn_tokens(const HeadTurns<T>& t, long first, long last) {
+  __shared__ float cosines[TURN_MAX_PAIRS], sines[TURN_MAX_PAIRS];
+  const int pairs = t.rotary_dim / 2;
+  const int together = pairs > 0 ? TURN_MAX_PAIRS / pairs : TURN_MAX_PAIRS;
+  const int each = t.heads.heads * t.width;
+  for (long from = first; from < last; from += together) {
+    const int count = (int)min((long)together, last - from);
+    if (from > first) __syncthreads();
+    for (int i = threadIdx.x; i < count * pairs; i += blockDim.x) {
+      const int token = i / pairs;
+      float s, c;
+      sincosf((float)t.positions[from + token] * t.inv_freq[i - token * pairs], &s, &c);
+      cosines[i] = c * t.magnitude;
+      sines[i] = s * t.magnitude;
+    }
+    __syncthreads();
+    for (int at = threadIdx.x; at < count * each; at += blockDim.x) {
+      const int token = at / each;
+      const int head = (at - token * each) / t.width;
+      const int j = at - token * each - head * t.width;
+      const T* row = t.heads.rows + (from + token) * t.heads.ld + t.heads.col + (long)head * t.heads.head_stride;
+      t.heads.out[(from + token) * t.heads.out_ld + t.heads.out_col + (long)head * t.heads.out_head_stride + j] =
+          from_float<T>(turned_element(row, j, t.rotary_dim, t.interleaved, cosines + token * pairs, sines + token * pairs));
+    }
+  }
+}
+
 template <typename T, int MT, bool VEC>
 __global__ void __launch_bounds__(TILE_THREADS)
 head_gemm_kernel(const T* __restrict__ x, long ldx, int x_col, const T* __restrict__ W, int x_head_stride,
-                 int out_head_stride, T* __restrict__ out, long ldo, int out_col, int M, int N, int K) {
+                 int out_head_stride, T* out, long ldo, int out_col, int M, int N, int K, int heads, HeadTurns<T> turned) {
   __shared__ float red[TILE_WAVES][256];
   const int tid = threadIdx.x;
   const int r = (tid & (WAVE - 1)) % 16;
   const int head = blockIdx.z;
   const long n0 = (long)blockIdx.x * 16;
   const long m0 = (long)blockIdx.y * 16 * MT;
+  if (head == heads) {                               // the slice that turns: its row of workgroups shares the rows of a tile
+    const int share = (16 * MT + gridDim.x - 1) / gridDim.x;
+    const long first = m0 + (long)blockIdx.x * share;
+    turn_tokens(turned, first, min(min(first + share, m0 + 16 * MT), (long)M));
+    return;
+  }
   const T* w_row[1] = {W + ((long)head * N + min(n0 + r, (long)N - 1)) * K};
   const T* x_row[MT];
 #pragma unroll
@@ -205,45 +254,59 @@ head_gemm_kernel(const T* __restrict__ x, long ldx, int x_col, const T* __restri
 
 template <typename T>
 static int launch_head_gemm(const T* x, long ldx, int x_col, const T* W, int x_head_stride, int out_head_stride, T* out,
-                            long ldo, int out_col, int M, int N, int K, int H, hipStream_t stream) {
+                            long ldo, int out_col, int M, int N, int K, int H, const HeadTurns<T>& turned, hipStream_t stream) {
   constexpr int PIECE = TileTraits<T>::PIECE;
   const bool vec = K % PIECE == 0 && ldx % PIECE == 0 && x_col % PIECE == 0 && x_head_stride % PIECE == 0 &&
                    ((unsigned long long)x % 16) == 0 && ((unsigned long long)W % 16) == 0;
   const int row_tiles = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   const long blocks_y = ((long)M + 16 * row_tiles - 1) / (16 * row_tiles);
-  if (blocks_y > 65535 || H > 65535) return ERR_UNSUPPORTED_SIZE;
-  const dim3 grid((unsigned)((N + 15) / 16), (unsigned)blocks_y, (unsigned)H);
-#define HEAD_LAUNCH(MT_)                                                                                              \
+  const int slices = H + (turned.heads.rows ? 1 : 0);
+  if (blocks_y > 65535 || slices > 65535) return ERR_UNSUPPORTED_SIZE;
+  const dim3 grid((unsigned)((N + 15) / 16), (unsigned)blocks_y, (unsigned)slices);
+#define HEAD_LAUNCH(MT_, VEC_)                                                                                        \
+  head_gemm_kernel<T, MT_, VEC_><<<grid, TILE_THREADS, 0, stream>>>(x, ldx, x_col, W, x_head_stride, out_head_stride, \
+                                                                    out, ldo, out_col, M, N, K, H, turned)
+#define HEAD_ROWS(MT_)                                                                                                \
   do {                                                                                                                \
-    if (vec)                                                                                                          \
-      head_gemm_kernel<T, MT_, true><<<grid, TILE_THREADS, 0, stream>>>(x, ldx, x_col, W, x_head_stride,              \
-                                                                        out_head_stride, out, ldo, out_col, M, N, K); \
-    else                                                                                                              \
-      head_gemm_kernel<T, MT_, false><<<grid, TILE_THREADS, 0, stream>>>(x, ldx, x_col, W, x_head_stride,             \
-                                                                         out_head_stride, out, ldo, out_col, M, N, K); \
+    if (vec) HEAD_LAUNCH(MT_, true);                                                                                  \
+    else HEAD_LAUNCH(MT_, false);                                                                                     \
   } while (0)
-  if (row_tiles == 1) HEAD_LAUNCH(1);
-  else if (row_tiles == 2) HEAD_LAUNCH(2);
-  else HEAD_LAUNCH(4);
+  if (row_tiles == 1) HEAD_ROWS(1);
+  else if (row_tiles == 2) HEAD_ROWS(2);
+  else HEAD_ROWS(4);
+#undef HEAD_ROWS
 #undef HEAD_LAUNCH
   return 0;
 }
 
+// positions not null: the heads' parts of `turn_width` numbers at x[m, turn_col + h * turn_head_stride] are turned into
+// out[m, turn_out_col + h * turn_out_head_stride] too (columns that the products neither read nor write).
 extern "C" int mi_head_gemm(const void* x, int dtype, long ldx, long x_col, const void* W, long x_head_stride,
                             long out_head_stride, void* out, long ldo, long out_col, int M, int N, int K, int H,
+                            const int* positions, const float* inv_freq, int rotary_dim, int interleaved, float magnitude,
+                            int turn_width, int turn_col, int turn_head_stride, int turn_out_col, int turn_out_head_stride,
                             hipStream_t stream) {
   if (!x || !W || !out || M <= 0 || N <= 0 || K <= 0 || H <= 0 || x_col < 0 || out_col < 0 || x_head_stride < 0 ||
       out_head_stride < 0 || ldx < x_col + (H - 1) * x_head_stride + K || ldo < out_col + (H - 1) * out_head_stride + N)
     return ERR_BAD_ARGUMENT;
-  int code;
-  if (dtype == DT_F32)
-    code = launch_head_gemm<float>((const float*)x, ldx, (int)x_col, (const float*)W, (int)x_head_stride,
-                                   (int)out_head_stride, (float*)out, ldo, (int)out_col, M, N, K, H, stream);
-  else if (dtype == DT_BF16)
-    code = launch_head_gemm<bf16_t>((const bf16_t*)x, ldx, (int)x_col, (const bf16_t*)W, (int)x_head_stride,
-                                    (int)out_head_stride, (bf16_t*)out, ldo, (int)out_col, M, N, K, H, stream);
-  else
+  if (positions && (turn_width <= 0 || rotary_dim < 0 || rotary_dim > turn_width || rotary_dim % 2 || (rotary_dim > 0 && !inv_freq) ||
+                    turn_col < 0 || turn_head_stride < 0 || turn_out_col < 0 || turn_out_head_stride < 0 ||
+                    ldx < turn_col + (long)(H - 1) * turn_head_stride + turn_width ||
+                    ldo < turn_out_col + (long)(H - 1) * turn_out_head_stride + turn_width))
     return ERR_BAD_ARGUMENT;
+  if (positions && rotary_dim > 2 * TURN_MAX_PAIRS) return ERR_UNSUPPORTED_SIZE;
+  int code;
+#define HEAD_GEMM(T_)                                                                                                 \
+  launch_head_gemm<T_>((const T_*)x, ldx, (int)x_col, (const T_*)W, (int)x_head_stride, (int)out_head_stride, (T_*)out, \
+                       ldo, (int)out_col, M, N, K, H,                                                                 \
+                       HeadTurns<T_>{{positions ? (const T_*)x : nullptr, ldx, turn_col, turn_head_stride, H, (T_*)out, ldo, \
+                                      turn_out_col, turn_out_head_stride},                                            \
+                                     turn_width, positions, inv_freq, rotary_dim, interleaved, magnitude},            \
+                       stream)
+  if (dtype == DT_F32) code = HEAD_GEMM(float);
+  else if (dtype == DT_BF16) code = HEAD_GEMM(bf16_t);
+  else return ERR_BAD_ARGUMENT;
+#undef HEAD_GEMM
   if (code) return code;
   RETURN_IF_LAUNCH_FAILED();
   return 0;

@@ -67,7 +67,8 @@ _SIGNATURES = {
         "mi_rotate_heads": [_c_ptr, _c_int, _c_long, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_int,
                             _c_float, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr],
         "mi_head_gemm": [_c_ptr, _c_int, _c_long, _c_long, _c_ptr, _c_long, _c_long, _c_ptr, _c_long, _c_long, _c_int,
-                         _c_int, _c_int, _c_int, _c_ptr],
+                         _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_int,
+                         _c_int, _c_float, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
         "mi_latent_attention": [_c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_int, _c_ptr, _c_int,
                                 _c_ptr, _c_int, _c_ptr, _c_ptr, _c_float, _c_int, _c_ptr, _c_long, _c_ptr],
         "mi_latent_attention_supported": [_c_int, _c_int],
@@ -811,9 +812,11 @@ def rotate_heads(x: torch.Tensor, col: int, head_stride: int, num_heads: int, wi
 
 
 def head_linear(x: torch.Tensor, x_col: int, x_head_stride: int, weight: torch.Tensor, out: torch.Tensor, out_col: int,
-                out_head_stride: int) -> None:
+                out_head_stride: int, turn: Optional[tuple] = None) -> None:
     """One product per head: out[:, out_col + h * out_head_stride : + N] = x[:, x_col + h * x_head_stride : + K] .
-    weight[h]^T, ``weight`` [heads, N, K], float32 sums on the matrix cores (float32 operands: true 32-bit)."""
+    weight[h]^T, ``weight`` [heads, N, K], float32 sums on the matrix cores (float32 operands: true 32-bit).
+    ``turn`` (col, head_stride, width, positions, inv_freq, rotary_dim, interleaved, out_col, out_head_stride, magnitude):
+    ``rotate_heads`` of other columns of ``x`` into other columns of ``out`` in the same launch."""
     ldx = _row_major(x, "x")
     ldo = _row_major(out, "out")
     _need(weight.dim() == 3 and weight.is_contiguous() and weight.is_cuda, "head_linear: weight must be contiguous [heads, N, K]")
@@ -823,16 +826,32 @@ def head_linear(x: torch.Tensor, x_col: int, x_head_stride: int, weight: torch.T
           and out_col + (heads - 1) * out_head_stride + N <= out.shape[1], "head_linear: shapes do not fit")
     rows = x if x.dtype == weight.dtype else x.to(weight.dtype)
     target = out if out.dtype == weight.dtype else torch.empty(out.shape, dtype=weight.dtype, device=out.device)
+    turns = [None, None, 0, 0, 1.0, 0, 0, 0, 0, 0]
+    if turn is not None:
+        col, head_stride, width, positions, inv_freq, rotary_dim, interleaved, turn_out_col, turn_out_stride, magnitude = turn
+        if rows is x and target is out:                      # (else the product's rows are copies: a launch of its own, behind it)
+            _i32(positions, "positions")
+            turned = int(rotary_dim) if inv_freq is not None else 0
+            _need(positions.numel() == T and turned % 2 == 0 and turned <= width
+                  and col + (heads - 1) * head_stride + width <= x.shape[1]
+                  and turn_out_col + (heads - 1) * turn_out_stride + width <= out.shape[1], "head_linear: the turns do not fit")
+            _need(inv_freq is None or (inv_freq.dtype == torch.float32 and inv_freq.numel() == turned // 2 and inv_freq.is_cuda),
+                  "head_linear: inv_freq must be float32 [rotary_dim / 2]")
+            turns = [_p(positions), _p(inv_freq), turned, 1 if interleaved else 0, float(magnitude), int(width), int(col),
+                     int(head_stride), int(turn_out_col), int(turn_out_stride)]
     if rows is not x:
         ldx = _row_major(rows, "x")
     if target is not out:
         ldo = _row_major(target, "out")
     _check(_fn("latent", "mi_head_gemm")(
         _p(rows), _dt(rows), ldx, int(x_col), _p(weight), int(x_head_stride), int(out_head_stride), _p(target), ldo,
-        int(out_col), T, N, K, heads, _stream()), "head_linear", f"(N={N}, K={K})")
+        int(out_col), T, N, K, heads, *turns, _stream()), "head_linear", f"(N={N}, K={K})")
     if target is not out:
-        width = (heads - 1) * out_head_stride + N
-        out[:, out_col:out_col + width] = target[:, out_col:out_col + width].to(out.dtype)
+        span = (heads - 1) * out_head_stride + N
+        out[:, out_col:out_col + span] = target[:, out_col:out_col + span].to(out.dtype)
+    if turn is not None and turns[0] is None:
+        rotate_heads(x, col, head_stride, heads, width, positions, inv_freq, rotary_dim, interleaved, out, turn_out_col,
+                     turn_out_stride, magnitude)
 
 
 def latent_attention_supported(dtype, num_heads: int, kv_rank: int, rope_dim: int, page_size: int) -> bool:

@@ -30,7 +30,8 @@ class LatentAttention(Mixer):
 
     One kernel forms both latents' RMS norms (float32), turns the shared key part, writes the token's cache cell and,
     where the queries are projected directly, turns their ``rope_dim`` parts into place beside their latent-space parts
-    (a launch of its own behind a query latent, and where there is no row to write)."""
+    (behind a query latent, and where there is no row to write, the launch that takes the queries into the latent space
+    does)."""
     graph_safe = True
     takes_tail = True
     kernel_modules = ("common", "attention", "gemm", "latent")
@@ -115,12 +116,15 @@ class LatentAttention(Mixer):
         latent_q = torch.empty((tokens, heads * width), dtype=x.dtype, device=x.device)
         if self.direct:
             q = down[:, :self.q_width]                                # [T, heads * (dim + rope)], a view
-            ops.head_linear(q, 0, dim + rope, self.into_latent, latent_q, 0, width)
+            beside = {}
+            if rope and not owns and x.is_cuda:                       # the turn beside the products, in one launch
+                beside = dict(turn=(dim, dim + rope, rope, step.positions, *turn, rank, width, self.magnitude))
+            ops.head_linear(q, 0, dim + rope, self.into_latent, latent_q, 0, width, **beside)
             if owns:
                 ops.latent_prepare(down[:, self.q_width:], 0, rank, rope, None, self.kv_norm, spec.norm_eps,
                                    step.positions, *turn, step.slot_mappings[cache.group], cache.k_cache, cache.v_cache,
                                    None, self.magnitude, (q, dim, dim + rope, heads, latent_q, rank, width))
-            elif rope:
+            elif rope and not beside:
                 ops.rotate_heads(q, dim, dim + rope, heads, rope, step.positions, *turn, latent_q, rank, width,
                                  self.magnitude)
         else:
@@ -129,8 +133,12 @@ class LatentAttention(Mixer):
                                *turn, step.slot_mappings[cache.group], cache.k_cache, cache.v_cache, query_latent,
                                self.magnitude)
             q = self.up_q(query_latent)                               # [T, heads * (dim + rope)]
-            ops.head_linear(q, 0, dim + rope, self.into_latent, latent_q, 0, width)
-            if rope:
+            if rope and x.is_cuda:                                    # the turn beside the products, in one launch
+                ops.head_linear(q, 0, dim + rope, self.into_latent, latent_q, 0, width,
+                                turn=(dim, dim + rope, rope, step.positions, *turn, rank, width, self.magnitude))
+            else:
+                ops.head_linear(q, 0, dim + rope, self.into_latent, latent_q, 0, width)
+            if rope and not x.is_cuda:
                 ops.rotate_heads(q, dim, dim + rope, heads, rope, step.positions, *turn, latent_q, rank, width,
                                  self.magnitude)
         attended = torch.empty((tokens, heads * rank), dtype=x.dtype, device=x.device)

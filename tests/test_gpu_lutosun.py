@@ -150,6 +150,26 @@ def test_one_product_per_head(dtype, T, heads, N, K, x_col, x_stride, out_col, o
     close(got.float(), want.float(), dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T, heads, dim, rope, rotary, rank, interleaved", [
+    (1, 8, 64, 32, 32, 128, True), (16, 3, 16, 8, 6, 20, False), (17, 8, 64, 32, 32, 128, True), (33, 2, 24, 12, 0, 8, False),
+    (130, 8, 64, 32, 32, 128, True), (65, 1, 40, 300, 300, 16, False), (70, 2, 8, 1024, 1024, 40, True)])
+def test_turns_beside_the_heads_products_are_those_of_a_launch_of_their_own(dtype, T, heads, dim, rope, rotary, rank, interleaved):
+    """The same bits, tokens and turns past what the LDS holds at a time among them; and a weight of another type."""
+    x = rand(T, heads * (dim + rope), seed=1).to(dtype).to(DEV)
+    weight = (rand(heads, rank, dim, seed=2) / dim ** 0.5).to(dtype).to(DEV)
+    positions = torch.randint(0, 5000, (T,), generator=torch.Generator().manual_seed(3), dtype=torch.int32).to(DEV)
+    inv_freq = (1.0 / 1e4 ** (torch.arange(0, rotary, 2).float() / max(rotary, 1))).to(DEV) if rotary else None
+    width = rank + rope
+    turn = (dim, dim + rope, rope, positions, inv_freq, rotary, interleaved, rank, width, 1.25)
+    for matrix in (weight, weight.float()):
+        apart, together = (torch.full((T, heads * width), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+        ops().head_linear(x, 0, dim + rope, matrix, apart, 0, width)
+        ops().rotate_heads(x, dim, dim + rope, heads, rope, positions, inv_freq, rotary, interleaved, apart, rank, width, 1.25)
+        ops().head_linear(x, 0, dim + rope, matrix, together, 0, width, turn=turn)
+        assert torch.equal(apart, together)
+
+
 @pytest.mark.parametrize("T, experts, top", [(1, 5, 2), (37, 12, 3), (300, 70, 8), (9, 3, 3), (64, 130, 1), (700, 6, 2)])
 def test_the_router_and_the_grouping_of_rows_by_expert(T, experts, top):
     logits = rand(T, experts + 1, seed=1) * 2.0
