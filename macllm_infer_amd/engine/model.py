@@ -71,7 +71,7 @@ class DecoderModel:
     @staticmethod
     def kernel_modules(spec: ModelSpec, dtype: torch.dtype = torch.bfloat16) -> List[str]:
         """The HIP modules that a model of this spec launches in ``dtype``."""
-        modules = ["common", "gemm"]
+        modules = ["common", "gemm", "rows_gemm"]
         for layer in spec.layers:
             modules += arrangement_class(layer.arrangement).kernel_modules(layer)
         never = kernel_build.BFLOAT16_MODULES if dtype != torch.bfloat16 else ()

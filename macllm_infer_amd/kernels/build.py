@@ -29,8 +29,8 @@ FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-shared", "-fPIC",
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option", "-Wno-pass-failed"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-Wall"]
 HOST_MODULES = ("hostcore",)                      # plain C++, no GPU code
-MODULES = ("common", "attention", "attention_widths", "attention_shared", "mamba2", "ssd", "linear_state", "linear_chunk", "linear_matrix", "latent", "moe", "gemm", "decode", "sampling", "microbench") + HOST_MODULES
-BFLOAT16_MODULES = ("attention_shared", "linear_matrix")      # kernels that take bfloat16 alone
+MODULES = ("common", "attention", "attention_widths", "attention_shared", "mamba2", "ssd", "linear_state", "linear_chunk", "linear_matrix", "latent", "moe", "gemm", "rows_gemm", "decode", "sampling", "microbench") + HOST_MODULES
+BFLOAT16_MODULES = ("attention_shared", "linear_matrix", "rows_gemm")      # kernels that take bfloat16 alone
 
 _loaded: Dict[str, ctypes.CDLL] = {}
 _lock = threading.Lock()

@@ -177,6 +177,10 @@ _SIGNATURES = {
                            _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr],
         "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int, _c_ptr],
     },
+    "rows_gemm": {
+        "mi_rows_gemm": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int,
+                         _c_ptr],
+    },
     "gemm": {
         "mi_gemm_f32": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr],
     },
@@ -464,6 +468,20 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor, tile: int = 0, activation: 
     _check(_fn("common", "mi_swiglu")(_p(gate_up), _dt(gate_up), ld, _p(out), T, two_i // 2, int(tile),
                                       GATE_ACTIVATIONS[activation], *_clamp_numbers(activation, clamp, "swiglu"),
                                       _stream()), "swiglu")
+
+
+def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+                  bias16: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """SiLU(gate) * up of the product of many rows with a weight in tiles of 8 gate and 8 up rows (bfloat16): in the
+    product's launch where that pays, else behind it."""
+    M, K = x.shape
+    N = weight.shape[0]
+    if rows_gemm_pays(M, N, K, swiglu=True) and rows_gemm_supported(x, weight):
+        return rows_gemm(x, weight, bias, swiglu=True)
+    gate_up = linear(x, weight, bias, bias16=bias16)
+    out = torch.empty((M, N // 2), dtype=gate_up.dtype, device=x.device)
+    swiglu(gate_up, out, 8)
+    return out
 
 
 def cast_rows(source: torch.Tensor, out: torch.Tensor) -> None:
@@ -1408,6 +1426,64 @@ def linear_chunk_scan(u: torch.Tensor, *, q_col: int, k_col: int, v_col: int, nu
 
 
 # --------------------------------------------------------------------------- matrix products
+GEMM_UNITS = 256          # compute units
+
+
+def rows_gemm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether ``rows_gemm`` takes these operands."""
+    return (x.is_cuda and weight.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+            and x.shape[1] % 64 == 0 and x.shape[0] > 0 and x.stride(1) == 1 and weight.stride(1) == 1
+            and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and max(x.stride(0), weight.stride(0)) <= 1 << 22
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False) -> bool:
+    """Whether this package's product of many rows is the faster one, the library the other: where tiles of 64 rows by 64
+    or 128 features fit the compute units once.  Its time | the library's over 33 to 4,096 rows and 512 to 8,192 features
+    (weights from memory), least, median and most:
+
+    * K = 512: 64 x 64 0.61 0.67 0.88, 64 x 128 0.67 0.75 0.81, 128 x 128 once 0.76 0.87 0.92, more 0.73 1.0 1.28
+    * K = 1,024: 0.67 0.74 0.81; 0.81 0.87 0.92; 128 x 128 0.88 0.98 1.05, more 0.94 1.2 1.59
+    * K = 2,048: 0.85 0.97 1.12, of more than half a million results 0.85 0.91 0.99; 64 x 128 of 512 rows on 0.88 0.95
+      1.01, of fewer 0.74 to 1.11
+    * K = 4,096: 0.85 1.16 1.73, 0.92 1.08 1.22: the library splits K over the compute units there
+
+    ``swiglu``: of a gated feed-forward, with the activation in the product | the library's product and the activation behind
+    it (features of the weight): 128 x 128 tiles at most twice a compute unit at K of up to 1,024 0.53 to 0.91 (2,048 x 4,096 x
+    1,024 25.5 -> 19.2 us, 640 rows 16.4 -> 11.4, 65 rows 11.3 -> 7.4), of 4,096 features more 0.83 to 0.94, of more features 0.86
+    to 1.18; once at K = 2,048 0.68 to 0.97, twice 0.92 to 1.1, and 1.07 to 1.39 beyond."""
+    tiles = lambda rows, features: -(-M // rows) * -(-N // features)
+    small, wide = tiles(64, 64) <= GEMM_UNITS, tiles(64, 128) <= GEMM_UNITS
+    if swiglu:
+        large = tiles(128, 128)
+        return K <= 2048 and (large <= GEMM_UNITS or (K <= 1024 and (large <= 2 * GEMM_UNITS or N <= 4096)))
+    if K <= 512:
+        return small or wide or tiles(128, 128) <= GEMM_UNITS
+    if K <= 1024:
+        return small or wide
+    return K <= 2048 and M * N >= 1 << 19 and (small or (wide and M >= 512))
+
+
+def rows_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *, swiglu: bool = False,
+              keep_float32: bool = False, tile: int = -1) -> torch.Tensor:
+    """x [M, K] . weight[N, K]^T (+ bias float32 [N]) of bfloat16 operands with float32 sums, [M, N] in bfloat16 or (``keep_float32``)
+    float32; or (``swiglu``) SiLU(gate) * up [M, N / 2] of a weight whose rows are tiles of 8 gate and 8 up rows, the
+    activation on the float32 sums.  ``tile``: the kernel's tile (0 to 3; by its rule if negative)."""
+    _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and rows_gemm_supported(x, weight)
+          and not (swiglu and keep_float32), "rows_gemm: operands not covered")
+    M, K = x.shape
+    N = weight.shape[0]
+    _need(not swiglu or N % 16 == 0, "rows_gemm: gate and up rows come in whole tiles of 8 each")
+    _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == N and bias.is_contiguous() and bias.is_cuda),
+          "rows_gemm: bias must be float32 [N]")
+    width = N // 2 if swiglu else N
+    out = torch.empty((M, width), dtype=torch.float32 if keep_float32 else torch.bfloat16, device=x.device)
+    _check(_fn("rows_gemm", "mi_rows_gemm")(
+        _p(x), _row_major(x, "x"), _p(weight), _row_major(weight, "weight"), _p(bias), _p(out), width, M, N, K,
+        1 if swiglu else 2 if keep_float32 else 0, int(tile), _stream()), "rows_gemm", f"(M={M}, N={N}, K={K})")
+    return out
+
+
 SKINNY_ROWS = 16          # steps of up to this many rows take the skinny kernel in ``linear``
 
 
@@ -1417,8 +1493,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
     ``keep_float32`` and no bias, in float32 whatever the operands are (the library writes its
     float32 sums without rounding them to bfloat16: the logits).
 
-    float32 operands: the hand-written float32 FMA kernel (true 32-bit).  bfloat16 operands:
-    the BLAS library with float32 accumulation.  A float32 weight with bfloat16 activations
+    float32 operands: the hand-written float32 FMA kernel (true 32-bit).  bfloat16 operands: float32 sums, in the skinny
+    kernel (few rows), in ``rows_gemm`` where that is the faster one, or in the BLAS library.  A float32 weight with bfloat16 activations
     (a tensor that was stored in 32-bit) runs in float32 and the result is rounded once.
     ``bias16``: the bias in bfloat16, if that holds the same numbers: the library's products of many rows then add it
     to their float32 sums themselves."""
@@ -1444,8 +1520,11 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         out = torch.empty((M, weight.shape[0]), dtype=torch.float32 if keep_float32 else torch.bfloat16, device=x.device)
         fused_gemm(weight, bias, out, x=x)
         return out
+    _need(not keep_float32 or bias is None, "linear: float32 results of bfloat16 operands come without a bias")
+    if (rows_gemm_pays(M, weight.shape[0], K) and rows_gemm_supported(x, weight)
+            and (bias is None or (bias.dtype == torch.float32 and bias.numel() == weight.shape[0] and bias.is_contiguous()))):
+        return rows_gemm(x, weight, bias, keep_float32=keep_float32)
     if keep_float32:
-        _need(bias is None, "linear: float32 results of bfloat16 operands come without a bias")
         return torch.mm(x, weight.t(), out_dtype=torch.float32)
     if bias is None:
         return torch.mm(x, weight.t())

@@ -78,6 +78,9 @@ class SwiGLU(FeedForward):
             ops.fused_gemm(self.gate_up.weight, self.gate_up.bias, activated, x=x, epilogue=ops.EPI_SWIGLU,
                            gate_activation=self.spec.activation, clamp=self.spec.clamp)
             return activated
+        if (self.tile == 8 and self.spec.activation == "silu" and x.is_cuda and x.dtype == torch.bfloat16
+                and self.gate_up.weight.dtype == torch.bfloat16):
+            return ops.linear_swiglu(x, self.gate_up.weight, self.gate_up.bias, self.gate_up.bias16)
         gate_up = self.gate_up(x)
         activated = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=gate_up.dtype, device=x.device)
         ops.swiglu(gate_up, activated, self.tile, activation=self.spec.activation, clamp=self.spec.clamp)

@@ -286,7 +286,7 @@ def _measure_split(weight: torch.Tensor, bias, rows: int, library: bool, tiles: 
     return best
 
 
-def _measure_library(weight: torch.Tensor, bias, rows: int, epilogue: int, tile: int, conv: Optional[dict],
+def _measure_library(weight: torch.Tensor, bias, rows: int, epilogue: int, conv: Optional[dict],
                      wide: bool) -> tuple:
     """(whether the library way is faster for this weight at this many rows, the skinny kernel's best number
     of feature tiles; ``wide``: more than one tile may be taken, i.e. the prologue is the plain one; negative:
@@ -314,10 +314,11 @@ def _measure_library(weight: torch.Tensor, bias, rows: int, epilogue: int, tile:
 
     def library():
         for w in weights:
-            product = ops.linear(x, w, bias)
             if epilogue == ops.EPI_SWIGLU:
-                ops.swiglu(product, out, tile)
-            elif epilogue == ops.EPI_CONV:
+                ops.linear_swiglu(x, w, bias)
+                continue
+            product = ops.linear(x, w, bias)
+            if epilogue == ops.EPI_CONV:
                 ops.conv_step(product, conv["lo"], conv["hi"] - conv["lo"], conv["weight"], conv["bias"], conv["state"],
                               conv["slot_ids"])
 
@@ -801,7 +802,7 @@ class LayerFusion:
             wide = bucket in self.wide_buckets or not normed          # the plain prologue: a workgroup may own several tiles
             key = (tuple(weight.shape), epilogue, bias is None, bucket, wide)
             if key not in _library_wins:
-                _library_wins[key] = _measure_library(weight, bias, rows, epilogue, 8, conv, wide)
+                _library_wins[key] = _measure_library(weight, bias, rows, epilogue, conv, wide)
             choices.append(_library_wins[key][0])
             tiles.append(_library_wins[key][1] if FORCE_TILES is None or bucket not in self.wide_buckets else FORCE_TILES)
         return tuple(choices), tuple(tiles)
@@ -922,17 +923,18 @@ class LayerFusion:
         if self.gate_up is None:
             residual.pending = [block.ffn.forward(block.ffn_norm.forward(residual))]
             return
-        activated = torch.empty((M, self.inner), dtype=torch.bfloat16, device=mixed.device)
         scaled = residual.scaled
         if scaled is not None and (self.ffn_scale is None or scaled.weight is not self.ffn_scale[0]):
             scaled = None
+        if scaled is None and self.library_gate_up[bucket]:
+            activated = ops.linear_swiglu(block.ffn_norm.forward(residual), self.gate_up.weight, self.gate_up.bias)
+        else:
+            activated = torch.empty((M, self.inner), dtype=torch.bfloat16, device=mixed.device)
         if scaled is not None:
             ops.fused_gemm(self.gate_up.weight, self.gate_up.bias, activated, epilogue=ops.EPI_SWIGLU,
                            fragments=self.f_gate_up, **_tiles(self.tiles_gate_up[bucket], self.rows_gate_up[bucket]),
                            **self._behind_the_norm(scaled, self.ffn_scale))
-        elif self.library_gate_up[bucket]:
-            ops.swiglu(ops.linear(block.ffn_norm.forward(residual), self.gate_up.weight, self.gate_up.bias), activated, 8)
-        else:
+        elif not self.library_gate_up[bucket]:
             arguments, h_out = self._norm_prologue(residual, M, block.ffn_norm, self.ffn_rms)
             ops.fused_gemm(self.gate_up.weight, self.gate_up.bias, activated, epilogue=ops.EPI_SWIGLU,
                            fragments=self.f_gate_up, **(_tiles(self.tiles_gate_up[bucket]) if "x" in arguments else {}),
