@@ -3,17 +3,19 @@
 //
 // A workgroup owns a tile of BM rows x BN features.  K is walked in stages of 64 columns, whole lines of 128 bytes of every
 // row, which go from memory to LDS without passing through registers (`buffer_load ... lds`), STAGES of them on their way;
-// one barrier a stage.  A wave holds the fragments of half a stage in registers and reads those of the next half while it
-// multiplies, one load between every few products.  Piece p of row r of a stage lies at 8 r + (p ^ (r & 7)): a load to LDS
+// one barrier a stage.  A wave holds the fragments of half a stage (small tiles: of a whole one) in registers and reads those of
+// the next while it multiplies.  Piece p of row r of a stage lies at 8 r + (p ^ (r & 7)): a load to LDS
 // writes 64 pieces one after the other, so it is the lanes' addresses that are exchanged (within a line), and no read of a
 // fragment meets a bank conflict.  A row's sum runs in k order in one lane, whatever the tile and the rows beside it.
 //
-// What bounds it: a stage's reads from LDS and its barrier (64 x 64 tiles: 435 cycles a stage, 128 of them products), the
-// launch and the lines written at its end (2,048 x 4,096 with K = 64: 8.9 us).  So it is at its best where the tiles fit the
-// chip once, which is where the library is at its worst: us, library | this, weights from memory: 257 x 1,024 x 1,024
-// 8.7 | 6.4, 1,024 x 1,024 x 1,024 9.1 | 6.8, 640 x 2,048 x 1,024 9.8 | 8.6, 385 x 4,096 x 1,024 10.4 | 8.9, 1,554 x 1,536 x 512
-// 9.9 | 6.9, 640 x 1,024 x 2,048 11.0 | 9.4, 2,048 x 1,024 x 2,048 16.1 | 13.1; and where it is not: 2,048 x 4,096 x 1,024 20.4 |
-// 20.5, 1,280 x 4,096 x 1,024 14.3 | 17.9, 2,048 x 6,144 x 1,024 27.7 | 39.8, 2,048 x 24,576 x 3,072 226 | 254.
+// What bounds it: a stage's reads from LDS, their latency and its barrier (64 x 64 tiles: 400 cycles a stage, 128 of them
+// products; with the next half's fragments in place of the next stage's on their way 470, with four waves in place of eight
+// 540), the launch and the lines written at its end (2,048 x 4,096 with K = 64: 8.9 us).  So it is at its best where the tiles
+// fit the chip once, which is where the library is at its worst: us, library | this, rows and weights from memory: 65 x 1,024 x
+// 1,024 8.3 | 6.5, 1,554 x 1,024 x 1,024 10.6 | 8.6, 1,554 x 1,024 x 512 8.6 | 6.4, 640 x 1,024 x 2,048 10.9 | 9.9; with the
+// activation (the library's product and the launch behind it) 256 x 4,096 x 1,024 14.0 | 6.7, 640 rows 18.1 | 13.1, 2,048 rows
+// 28 | 22.6; and where it is not: 2,048 x 1,024 x 2,048 18.0 | 17.7, 1,999 x 6,144 x 1,024 31 | 40, 2,048 x 24,576 x 3,072 with the
+// activation 253 | 310.
 #include "common.h"
 
 typedef float g_floatx4 __attribute__((ext_vector_type(4)));
@@ -37,8 +39,8 @@ struct RowsGemm {
   int whole;                         // four neighbouring outputs are one aligned piece
 };
 
-template <int BM, int BN, int WM, int WN, int STAGES, int EPI>
-__global__ void __launch_bounds__(WAVE * WM * WN, WM * WN > 4 ? 2 : 1)
+template <int BM, int BN, int WM, int WN, int STAGES, bool AHEAD, int EPI>
+__global__ void __launch_bounds__(WAVE * WM * WN, 2)
 rows_gemm_kernel(RowsGemm p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int WAVES = WM * WN;
@@ -85,61 +87,89 @@ rows_gemm_kernel(RowsGemm p) {
   for (int n = 0; n < TN; ++n)
 #pragma unroll
     for (int m = 0; m < TM; ++m) acc[n][m] = g_floatx4{0.f, 0.f, 0.f, 0.f};
-  g_bf16x8 rows[2][TM], features[2][TN];                     // the fragments of a stage's halves
-  auto fetch = [&](int stage, int half) {
+  g_bf16x8 rows[AHEAD ? 2 : 1][2][TM], features[AHEAD ? 2 : 1][2][TN];     // the fragments of a stage's halves
+  auto fetch = [&](int set, int stage, int half) {
     const unsigned char* const from = lds[stage % STAGES];
 #pragma unroll
     for (int m = 0; m < TM; ++m) {
       const int row = (wm * TM + m) * 16 + r;
-      rows[half][m] = *reinterpret_cast<const g_bf16x8*>(from + 128 * row + 16 * ((4 * half + q) ^ (row & 7)));
+      rows[set][half][m] = *reinterpret_cast<const g_bf16x8*>(from + 128 * row + 16 * ((4 * half + q) ^ (row & 7)));
     }
 #pragma unroll
     for (int n = 0; n < TN; ++n) {
       const int row = BM + (wn * TN + n) * 16 + r;
-      features[half][n] = *reinterpret_cast<const g_bf16x8*>(from + 128 * row + 16 * ((4 * half + q) ^ (row & 7)));
+      features[set][half][n] = *reinterpret_cast<const g_bf16x8*>(from + 128 * row + 16 * ((4 * half + q) ^ (row & 7)));
     }
   };
-  auto multiply = [&](int half) {
+  auto multiply = [&](int set, int half) {
 #pragma unroll
     for (int n = 0; n < TN; ++n)
 #pragma unroll
       for (int m = 0; m < TM; ++m)
-        acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(features[half][n], rows[half][m], acc[n][m], 0, 0, 0);
+        acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(features[set][half][n], rows[set][half][m], acc[n][m], 0, 0, 0);
   };
-  constexpr int PRODUCTS = TM * TN, FETCHES = TM + TN;
+  // this wave has read what it wanted of a stage, and its own part of the next one has arrived: behind the barrier the same
+  // holds for all
+  auto next_stage = [&]() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
 #pragma unroll
   for (int stage = 0; stage < STAGES; ++stage) ask(stage);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * LOADS) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  fetch(0, 0);
-  for (int stage = 0; stage < stages; ++stage) {
-    fetch(stage, 1);
-    multiply(0);
+  fetch(0, 0, 0);
+  if constexpr (AHEAD) {
+    // few products a stage: the next stage's fragments are read, into a second set, while this one is multiplied
+    fetch(0, 0, 1);
+    for (int stage = 0; stage < stages; stage += 2) {
+      next_stage();
+      ask(stage + STAGES);
+      fetch(1, stage + 1, 0);
+      fetch(1, stage + 1, 1);
+      multiply(0, 0);
+      multiply(0, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      next_stage();
+      ask(stage + 1 + STAGES);
+      fetch(0, stage + 2, 0);
+      fetch(0, stage + 2, 1);
+      if (stage + 1 < stages) {
+        multiply(1, 0);
+        multiply(1, 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    // half a stage ahead, one load between every few products
+    constexpr int PRODUCTS = TM * TN, FETCHES = TM + TN;
     constexpr int EACH = PRODUCTS / FETCHES > 0 ? PRODUCTS / FETCHES : 1;
-#pragma unroll
-    for (int i = 0; i < FETCHES; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);  // matrix products
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // a load from LDS
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    // this wave has read the stage, and its own part of the next one has arrived: behind the barrier the same holds for all
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * LOADS) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    ask(stage + STAGES);
-    fetch(stage + 1, 0);
-    multiply(1);
     constexpr int BOTH = PRODUCTS / (FETCHES + LOADS) > 0 ? PRODUCTS / (FETCHES + LOADS) : 1;
+    for (int stage = 0; stage < stages; ++stage) {
+      fetch(0, stage, 1);
+      multiply(0, 0);
 #pragma unroll
-    for (int i = 0; i < FETCHES + LOADS; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, BOTH, 0);
-      if ((i % 2 == 0 && i / 2 < FETCHES) || i - (i + 1) / 2 >= LOADS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                      // a load from memory
+      for (int i = 0; i < FETCHES; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);  // matrix products
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // a load from LDS
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      next_stage();
+      ask(stage + STAGES);
+      fetch(0, stage + 1, 0);
+      multiply(0, 1);
+#pragma unroll
+      for (int i = 0; i < FETCHES + LOADS; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, BOTH, 0);
+        if ((i % 2 == 0 && i / 2 < FETCHES) || i - (i + 1) / 2 >= LOADS) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                    // a load from memory
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, PRODUCTS, 0);
-    __builtin_amdgcn_sched_barrier(0);
   }
   // nothing of the stages past the end may still be on its way to LDS when the workgroup ends
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -206,27 +236,27 @@ rows_gemm_kernel(RowsGemm p) {
 #endif
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES>
+template <int BM, int BN, int WM, int WN, int STAGES, bool AHEAD>
 static void launch_rows_gemm(RowsGemm p, int epilogue, hipStream_t stream) {
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
   const int per_die = (int)(((long)p.tiles_m * p.tiles_n + 7) / 8);
-  if (epilogue == EPI_ROWS_SWIGLU) rows_gemm_kernel<BM, BN, WM, WN, STAGES, EPI_ROWS_SWIGLU><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
-  else if (epilogue == EPI_ROWS_F32) rows_gemm_kernel<BM, BN, WM, WN, STAGES, EPI_ROWS_F32><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
-  else rows_gemm_kernel<BM, BN, WM, WN, STAGES, EPI_ROWS_PLAIN><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
+  if (epilogue == EPI_ROWS_SWIGLU) rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_SWIGLU><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
+  else if (epilogue == EPI_ROWS_F32) rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_F32><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
+  else rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_PLAIN><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
 }
 
 // The tile with the least estimate of its time in microseconds: by the workgroups of the fullest compute unit, as measured
-// over 33 to 4,096 rows, 512 to 8,192 features and K of 512 to 4,096.  At K = 1,024, with one / two / three / four of them:
-// 64 x 64 6.3 / 9.3 / 13.5 / 16.2, 64 x 128 8.3 / 13.5 / 19.2 / 24.3, 128 x 128 with two stages, two of which run beside each
-// other, 13.2 / 18.5 / 30 / 37, with four stages, one at a time, 11.7 / 21.5.  The choice is the fastest of the four or within
-// a tenth of it wherever they are faster than the library.
+// over 33 to 4,096 rows, 256 to 8,192 features and K of 512 to 2,048 (medians).  At K = 1,024, with one / two / three / four of
+// them: 64 x 64 6.7 / 9.8 / 15.2 / 18.5, 64 x 128 8.2 / 14.2 / 22 / 28, 128 x 128 with two stages, two of which run beside each
+// other, 13.5 / 21.7 / 33 / 40, with four stages, one at a time, 11.4 / 25.  The choice is the fastest of the four or within
+// 15 % of it, 0.4 % behind it on average.
 static int rows_gemm_tile(int M, int N, int K) {
   auto fullest = [&](long rows, long features) { return (int)(((M + rows - 1) / rows * ((N + features - 1) / features) + 255) / 256); };
   const float k = K / 1024.f;
   const int large = fullest(128, 128);
-  const float time[4] = {3.2f + fullest(64, 64) * (0.4f + 2.9f * k), 3.2f + fullest(64, 128) * (0.4f + 4.9f * k),
-                         large > 1 ? 1e9f : 6.f + 5.6f * k, 2.5f + k * (16.f * (large / 2) + 10.5f * (large % 2))};
+  const float time[4] = {2.3f + fullest(64, 64) * (0.6f + 3.68f * k), 2.f + fullest(64, 128) * (1.1f + 5.5f * k),
+                         large > 1 ? 1e9f : 4.8f + 6.85f * k, 2.5f + (3.5f + 15.6f * k) * (large / 2) + (1.f + 10.5f * k) * (large % 2)};
   int best = 0;
   for (int i = 1; i < 4; ++i)
     if (time[i] < time[best]) best = i;
@@ -247,10 +277,10 @@ extern "C" int mi_rows_gemm(const void* x, long ldx, const void* w, long ldw, co
   RowsGemm p = {(const bf16_t*)x, (const bf16_t*)w, bias, out, (int)ldx, (int)ldw, ldo, M, N, K, 0, 0,
                 ldo % 4 == 0 && (uintptr_t)out % (epilogue == EPI_ROWS_F32 ? 16 : 8) == 0};
   switch (tile < 0 ? rows_gemm_tile(M, N, K) : tile) {
-    case 0: launch_rows_gemm<64, 64, 2, 2, 4>(p, epilogue, stream); break;
-    case 1: launch_rows_gemm<64, 128, 2, 2, 3>(p, epilogue, stream); break;
-    case 2: launch_rows_gemm<128, 128, 2, 4, 4>(p, epilogue, stream); break;
-    default: launch_rows_gemm<128, 128, 2, 4, 2>(p, epilogue, stream); break;
+    case 0: launch_rows_gemm<64, 64, 4, 2, 4, true>(p, epilogue, stream); break;
+    case 1: launch_rows_gemm<64, 128, 2, 4, 3, true>(p, epilogue, stream); break;
+    case 2: launch_rows_gemm<128, 128, 2, 4, 4, false>(p, epilogue, stream); break;
+    default: launch_rows_gemm<128, 128, 2, 4, 2, false>(p, epilogue, stream); break;
   }
   RETURN_IF_LAUNCH_FAILED();
   return 0;

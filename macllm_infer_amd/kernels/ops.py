@@ -1439,29 +1439,32 @@ def rows_gemm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False) -> bool:
     """Whether this package's product of many rows is the faster one, the library the other: where tiles of 64 rows by 64
-    or 128 features fit the compute units once.  Its time | the library's over 33 to 4,096 rows and 512 to 8,192 features
-    (weights from memory), least, median and most:
+    or 128 features fit the compute units once.  Its time | the library's over 33 to 4,096 rows and 256 to 8,192 features
+    (rows and weights from memory), least, median and most:
 
-    * K = 512: 64 x 64 0.61 0.67 0.88, 64 x 128 0.67 0.75 0.81, 128 x 128 once 0.76 0.87 0.92, more 0.73 1.0 1.28
-    * K = 1,024: 0.67 0.74 0.81; 0.81 0.87 0.92; 128 x 128 0.88 0.98 1.05, more 0.94 1.2 1.59
-    * K = 2,048: 0.85 0.97 1.12, of more than half a million results 0.85 0.91 0.99; 64 x 128 of 512 rows on 0.88 0.95
-      1.01, of fewer 0.74 to 1.11
-    * K = 4,096: 0.85 1.16 1.73, 0.92 1.08 1.22: the library splits K over the compute units there
+    * K = 512: 64 x 64 once 0.36 0.69 0.85, 64 x 128 once 0.65 0.73 0.79, 128 x 128 once 0.74 0.88 0.96, more 0.75 1.1 1.28
+    * K = 1,024: 0.63 0.76 0.80 (33 x 256: 1.15); 0.79 0.85 0.91; 128 x 128 once 0.81 1.0 1.09, more 0.94 1.2 1.46
+    * K = 2,048: 0.86 1.01 1.16 (of 512 rows and half a million results on 0.86 0.92 0.97), 0.78 1.02 1.15, more 1.06 to 1.59;
+      beyond, the library splits K over the compute units
 
-    ``swiglu``: of a gated feed-forward, with the activation in the product | the library's product and the activation behind
-    it (features of the weight): 128 x 128 tiles at most twice a compute unit at K of up to 1,024 0.53 to 0.91 (2,048 x 4,096 x
-    1,024 25.5 -> 19.2 us, 640 rows 16.4 -> 11.4, 65 rows 11.3 -> 7.4), of 4,096 features more 0.83 to 0.94, of more features 0.86
-    to 1.18; once at K = 2,048 0.68 to 0.97, twice 0.92 to 1.1, and 1.07 to 1.39 beyond."""
+    ``swiglu``: of a gated feed-forward, with the activation in the product | the library's product and the activation
+    behind it (2,048 to 8,192 features):
+
+    * K = 512: 0.49 to 0.8
+    * K = 1,024: 0.51 0.58 0.60; 0.59 0.63 0.67; 0.60 0.70 0.74; 128 x 128 twice 0.78 0.83 0.89, more 0.73 0.90 1.05 (of up to 4,096
+      features 0.73 to 0.96)
+    * K = 2,048: 0.70 0.77 0.86; 0.68 0.86 0.93; 0.79 0.80 0.87; twice 0.87 0.98 1.11, more 0.91 1.15 1.31"""
     tiles = lambda rows, features: -(-M // rows) * -(-N // features)
-    small, wide = tiles(64, 64) <= GEMM_UNITS, tiles(64, 128) <= GEMM_UNITS
+    small, wide, large = tiles(64, 64) <= GEMM_UNITS, tiles(64, 128) <= GEMM_UNITS, tiles(128, 128)
     if swiglu:
-        large = tiles(128, 128)
+        if K <= 512:
+            return True
         return K <= 2048 and (large <= GEMM_UNITS or (K <= 1024 and (large <= 2 * GEMM_UNITS or N <= 4096)))
     if K <= 512:
-        return small or wide or tiles(128, 128) <= GEMM_UNITS
+        return small or wide or large <= GEMM_UNITS
     if K <= 1024:
         return small or wide
-    return K <= 2048 and M * N >= 1 << 19 and (small or (wide and M >= 512))
+    return K <= 2048 and small and M >= 512 and M * N >= 1 << 19
 
 
 def rows_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *, swiglu: bool = False,
