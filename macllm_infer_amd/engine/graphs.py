@@ -269,7 +269,8 @@ class DecodeGraphs:
 
     def forks(self, key: tuple) -> bool:
         """Whether the graph of the portions' capacity ``key`` runs its mixers on two streams."""
-        return key[1] >= OVERLAP_MIN_TOKENS and any(len(getattr(block, "mixers", ())) == 2 for block in self.model.blocks)
+        least = lambda block: getattr(getattr(block, "fusion", None), "overlap_from", OVERLAP_MIN_TOKENS)
+        return any(len(getattr(block, "mixers", ())) == 2 and key[1] >= least(block) for block in self.model.blocks)
 
     def ask_beside(self, keys: Iterable[tuple], candidates: Sequence[torch.cuda.Stream]) -> None:
         """The clock's answer to which of ``candidates`` does not stand in the way of the graphs of these capacities, for

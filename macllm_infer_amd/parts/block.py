@@ -36,11 +36,11 @@ def side_stream(device: torch.device, beside: "torch.cuda.Stream") -> "torch.cud
             return streams[-1]
 
 
-def overlap_pays(mixers, rows: int, device: torch.device) -> bool:
+def overlap_pays(mixers, rows: int, device: torch.device, least: int = OVERLAP_MIN_TOKENS) -> bool:
     """Whether two mixers of a layer that read the same rows should run beside each other on two streams: in a
     captured graph only (launched one by one the step waits for the host, which the second stream costs more),
-    for portions long enough to be worth the hops between the queues, and if both only queue work."""
-    return (len(mixers) == 2 and rows >= OVERLAP_MIN_TOKENS and device.type == "cuda"
+    for portions long enough (``least`` rows) to be worth the hops between the queues, and if both only queue work."""
+    return (len(mixers) == 2 and rows >= least and device.type == "cuda"
             and torch.cuda.is_current_stream_capturing()
             and all(getattr(mixer, "graph_safe", False) for mixer in mixers))
 

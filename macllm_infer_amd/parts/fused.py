@@ -438,6 +438,11 @@ def _measure_chain(chain, bucket: int) -> dict:
 
 
 class LayerFusion:
+    # Portions from this size on run their two mixers beside each other: where a lane may be longer than the chunk that the
+    # state-space mixer's launches hold beside the attention's (us a prompt, beside | behind: 0.5B shape 144 tokens 2,971 | 3,109,
+    # 200 3,071 | 3,213, 256 3,144 | 3,305; 7B shape 144 2,783 | 2,928)
+    overlap_from = 129
+
     @staticmethod
     def build(block, build) -> Optional["LayerFusion"]:
         if build.dtype != torch.bfloat16 or build.device.type != "cuda":
@@ -764,7 +769,7 @@ class LayerFusion:
 
     def _general_mixers(self, u: torch.Tensor, step, caches) -> torch.Tensor:
         mixed = torch.empty((u.shape[0], self.mixed_width), dtype=u.dtype, device=u.device)
-        if overlap_pays(self.mixers, u.shape[0], u.device):
+        if overlap_pays(self.mixers, u.shape[0], u.device, self.overlap_from):
             # two mixers read the same rows and write different columns: the first runs on a second stream
             # beside the second (in a captured graph only: launched one by one the step waits for the host,
             # which the second stream costs more).  The mixer on the main stream is recorded first: the graph
