@@ -10,7 +10,7 @@
 // row's result is bit for bit the same alone, in a small step and in a large one.
 //
 // A step of up to 32 rows is bound by reading W once: every wave keeps its 1 KiB fragments in flight.  More rows are
-// bound by the matrix cores and go through tiled_f32_kernel, which shares its operands through LDS and keeps that
+// bound by the matrix cores and go through tiled_f32_kernel and direct_f32_kernel, which share their operands through LDS and keep that
 // order of the sums (K a multiple of 32, rows of whole 16-byte pieces; other sizes stay with the first kernel).
 #include "common.h"
 
@@ -293,6 +293,124 @@ tiled_f32_kernel(const float* __restrict__ x, long ldx, const float* __restrict_
     }
 }
 
+// The 64 x 64 tile of the above where the runs are whole stages (K a multiple of 128): the stages go from memory to LDS
+// without passing through registers (`buffer_load ... lds` writes 64 pieces one after the other, so it is the lanes'
+// addresses within a line that are exchanged), and the waves have nothing between their products but the loads of the next
+// chunk's operands.  Two stages in LDS: four workgroups a compute unit hide each other's waits (with three stages 280 us in place
+// of 273 for 32,784 features; tiles of 64 x 128 and 128 x 64 39.5 to 41.0 for the first).  512 x 4,096 x 1,024 45.2 -> 39.6 us, 512
+// x 3,352 x 1,024 43.6 -> 39.1, 512 x 32,784 x 1,024 298 -> 273, 2,048 x 1,024 x 2,048 73.3 -> 68.2; the smaller tiles in four
+// groups gain nothing this way (512 x 1,024 x 2,048 22.7 | 24.0).
+typedef __attribute__((address_space(3))) void f32_lds;
+#define DIRECT_STAGES 2
+
+__global__ void __launch_bounds__(GF_THREADS)
+direct_f32_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ W, int ldw, const float* __restrict__ bias,
+                  float* __restrict__ out, long ldo, bool whole, int M, int N, int K) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int TILE = 64, ROWS = 2 * TILE, LOADS = ROWS / 8 / GF_WAVES;       // of eight rows that a wave makes a stage
+  __shared__ floatx4 lds[DIRECT_STAGES][ROWS * 8];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int q = lane / 16, r = lane % 16;
+  const int first_m = (wave & 1) * 32, first_n = (wave >> 1) * 32;             // the wave's part of the tile
+  const int n0 = blockIdx.x * TILE, m0 = blockIdx.y * TILE;
+  const __amdgpu_buffer_rsrc_t w_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (long)n0 * ldw), 0, 0xffffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t x_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)m0 * ldx), 0, 0xffffffff, 0x00020000);
+  int offset[LOADS];                                           // (bytes within the tile's rows: the launch keeps them below 2^31)
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (i * GF_WAVES + wave) * 8 + lane / 8;
+    const int piece = (lane % 8) ^ (row & 7);
+    offset[i] = 4 * (i * GF_WAVES * 8 < TILE ? min(row, N - 1 - n0) * ldw + 4 * piece : min(row - TILE, M - 1 - m0) * ldx + 4 * piece);
+  }
+  const int stages = K / 32, run = stages / GF_WAVES;          // the sums' four runs
+  auto ask = [&](int stage) {                                  // (past the last one: the last again, never multiplied)
+    floatx4* const into = lds[stage % DIRECT_STAGES];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i * GF_WAVES * 8 < TILE ? w_rows : x_rows, (f32_lds*)(into + (i * GF_WAVES + wave) * 64), 16,
+                                               offset[i], min(stage, stages - 1) * 128, 0, 0);
+  };
+  floatx4 acc[2][2], total[2][2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int m = 0; m < 2; ++m) acc[n][m] = total[n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  floatx4 weights[2][2], rows[2][2];                           // the operands of a stage's two chunks
+  auto fetch = [&](int stage, int chunk) {
+    const floatx4* const from = lds[stage % DIRECT_STAGES] + ((4 * chunk + q) ^ (r & 7));
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      weights[chunk][t] = from[(first_n + 16 * t + r) * 8];
+      rows[chunk][t] = from[(TILE + first_m + 16 * t + r) * 8];
+    }
+  };
+  auto multiply = [&](int chunk) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(weights[chunk][n][i], rows[chunk][m][i], acc[n][m], 0, 0, 0);
+  };
+#pragma unroll
+  for (int stage = 0; stage < DIRECT_STAGES; ++stage) ask(stage);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DIRECT_STAGES - 1) * LOADS) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  fetch(0, 0);
+  int left = run;
+  for (int stage = 0; stage < stages; ++stage) {
+    fetch(stage, 1);
+    multiply(0);
+    interleave<16, 0, 0, 4>();
+    __builtin_amdgcn_sched_barrier(0);
+    // this wave has read the stage, and its own part of the next one has arrived: behind the barrier the same holds for all
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((DIRECT_STAGES - 2) * LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    ask(stage + DIRECT_STAGES);
+    fetch(stage + 1, 0);
+    multiply(1);
+    interleave<16, 0, LOADS, 4>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (--left == 0) {                                         // a run ends
+      left = run;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          total[n][m] += acc[n][m];
+          acc[n][m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  }
+  // nothing of the stages past the end may still be on its way to LDS when the workgroup ends
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      floatx4 value = total[nt][mt];
+      const int n = n0 + first_n + 16 * nt + 4 * q;
+      const long m = m0 + first_m + 16 * mt + r;
+      if (m >= M) continue;
+      if (bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) value[i] += bias[min(n + i, N - 1)];
+      }
+      if (whole && n + 3 < N) {
+        *reinterpret_cast<floatx4*>(out + m * ldo + n) = value;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) out[m * ldo + n + i] = value[i];
+      }
+    }
+#endif
+}
+
 template <int MT, int NT, int DEPTH>
 static void launch_gemm_f32(bool vec, dim3 grid, hipStream_t stream, const float* x, long ldx, const float* W,
                             long ldw, const float* bias, float* out, long ldo, int M, int N, int K) {
@@ -309,13 +427,13 @@ extern "C" int mi_gemm_f32(const float* x, long ldx, const float* W, long ldw, c
     // The tiling that the rounds of workgroups over 256 compute units make cheapest: microseconds a round at K =
     // 1,024, in tenths, as measured over 40 to 512 rows and 768 to 32,784 features (32 x 32 in four groups: 9.0 to 9.8,
     // 15.8, 22.5, 28.8, 37.1, 41.7 for one to six rounds; 32 x 64 in four groups: 13.4 to 15.3, 28, 38 to 40, 55; 64 x 64 in one
-    // group: 22.5 to 24.7, 41 to 45, 61.6, then 20.5 a round: workgroups of a compute unit hide each other's waits).  From 33 rows
+    // group: 22 to 24, 39 to 41, 56, then 18.5 a round: workgroups of a compute unit hide each other's waits).  From 33 rows
     // on the best of them is at least as fast as the first kernel at every size measured.
     auto rounds = [&](long rows, long features) {
       return (((M + rows - 1) / rows) * ((N + features - 1) / features) + 255) / 256;
     };
     const long small = 28 + 66 * rounds(32, 32), middle = 25 + 130 * rounds(32, 64), tall = rounds(64, 64);
-    const long large = tall == 1 ? 240 : tall == 2 ? 430 : 205 * tall;
+    const long large = tall == 1 ? 235 : tall == 2 ? 400 : 185 * tall;
     const bool whole = ldo % 4 == 0 && ((unsigned long long)out % 16) == 0;
     const int bm = large < small && large < middle ? 64 : 32, bn = bm == 64 || middle < small ? 64 : 32;
     const dim3 tiles((unsigned)(((long)N + bn - 1) / bn), (unsigned)(((long)M + bm - 1) / bm));
@@ -326,7 +444,9 @@ extern "C" int mi_gemm_f32(const float* x, long ldx, const float* W, long ldw, c
     if (even) tiled_f32_kernel<MT_, NT_, GROUPS_, true><<<tiles, GROUPS_ * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K); \
     else tiled_f32_kernel<MT_, NT_, GROUPS_, false><<<tiles, GROUPS_ * GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);     \
   } while (0)
-      if (bm == 64) TILED(2, 2, 1);
+      if (bm == 64 && even && ldx <= 1 << 22 && ldw <= 1 << 22)
+        direct_f32_kernel<<<tiles, GF_THREADS, 0, stream>>>(x, (int)ldx, W, (int)ldw, bias, out, ldo, whole, M, N, K);
+      else if (bm == 64) tiled_f32_kernel<2, 2, 1, false><<<tiles, GF_THREADS, 0, stream>>>(x, ldx, W, ldw, bias, out, ldo, whole, M, N, K);
       else if (bn == 64) TILED(1, 2, 4);
       else TILED(1, 1, 4);
 #undef TILED

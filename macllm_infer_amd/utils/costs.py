@@ -235,7 +235,7 @@ DECODE_GROUPS: List[Tuple[str, str]] = [
 PLAIN_PRODUCT = r"fused_gemm_kernel<\d+, [01], 0|skinny_kernel<\d+, 0"
 # (of lanes of one chunk, up to 128 tokens, the scan's two launches hold the attention too)
 PREFILL_GROUPS: List[Tuple[str, str]] = [
-    (r"^Cijk_|gemm_f32_kernel|tiled_f32_kernel|head_gemm_kernel|moe_expert_gemm", "matrix products"),
+    (r"^Cijk_|gemm_f32_kernel|tiled_f32_kernel|direct_f32_kernel|rows_gemm_kernel|head_gemm_kernel|moe_expert_gemm", "matrix products"),
     (r"prefill_attention|prefill_shared|paged_attention_kernel|paged_attention_tile_kernel|paged_attention_merge_kernel|"
      r"rope_kv_store_kernel|latent_|attention_prepare_kernel|rotate_heads_kernel", "attention"),
     (r"ssd_|ssm_scan_kernel|conv1d_silu|conv_state_update|gate_norm_kernel|linear_state_|linear_chunk_|linear_matrix_|head_norm_gate_|"
