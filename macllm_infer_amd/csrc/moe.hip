@@ -348,12 +348,17 @@ extern "C" int mi_moe_route_plan(const float* logits, long ld, int T, int E, int
 // MT = 1 (every expert's matrix is read once, by as many workgroups as it has tiles of features); prompt portions,
 // whose experts get dozens of rows each, MT = 4 and four tiles of features (the rows and the matrix come from the
 // caches, 64 x 64 results a workgroup).
+// The sums of the expert `rounded` (-1: none) are rounded to bfloat16 before anything else is done with them, as those of a product
+// of its own are: an expert gets the same bits in a launch with others as in launches of its own (up to 16 rows with K up to
+// 1,024 in tiles of 16 places, four runs of K; in tiles of 64 and 128 places those of a product of many rows, in k order).
+__device__ __forceinline__ float sum_as(float sum, bool rounded) { return rounded ? (float)(bf16_t)sum : sum; }
+
 template <typename T, typename TO, bool VEC, bool GLU, int MT, int PAIRS>
 __global__ void __launch_bounds__(TILE_THREADS)
 moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* __restrict__ W, long expert_stride, long ldw,
                        int N, int K, const int* __restrict__ source, const int* __restrict__ tile_expert, int gather,
                        float limit, float alpha, float offset, int squared_relu,
-                       const float* __restrict__ row_scale, TO* __restrict__ out, long ldo) {
+                       const float* __restrict__ row_scale, int rounded, TO* __restrict__ out, long ldo) {
   __shared__ float red[TILE_WAVES][256];
   const int tile = blockIdx.y;
   const int expert = tile_expert[tile];
@@ -387,9 +392,9 @@ moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* _
     for (int mt = 0; mt < MT; ++mt) {
       const int place = (tile * MT + mt) * 16 + (l % 16);
       const float scale = row_scale ? row_scale[place] : 1.0f;
-      float value = tile_reduce(acc[p][mt], red) * scale;
+      float value = sum_as(tile_reduce(acc[p][mt], red) * scale, expert == rounded);
       if (GLU) {
-        const float up = tile_reduce(acc[NT - PAIRS + p][mt], red) * scale;
+        const float up = sum_as(tile_reduce(acc[NT - PAIRS + p][mt], red) * scale, expert == rounded);
         const float g = fminf(value, limit);
         const float u = fminf(fmaxf(up, -limit), limit);
         value = g / (1.0f + expf(-alpha * g)) * (u + offset);
@@ -435,7 +440,7 @@ __global__ void __launch_bounds__(TILE_THREADS, 2)
 moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* __restrict__ W, long expert_stride,
                             long ldw, int N, int K, const int* __restrict__ source, const int* __restrict__ tile_expert,
                             int gather, float limit, float alpha, float offset, int squared_relu,
-                            const float* __restrict__ row_scale, TO* __restrict__ out, long ldo, int whole) {
+                            const float* __restrict__ row_scale, int rounded, TO* __restrict__ out, long ldo, int whole) {
   typedef typename TileTraits<T>::Piece Piece;
   constexpr int PIECE = TileTraits<T>::PIECE;
   constexpr int STAGE_K = 8 * PIECE;
@@ -540,8 +545,8 @@ moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const
         float value[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float g = fminf(acc[h][mt][i] * scale, limit);
-          const float u = fminf(fmaxf(acc[2 + h][mt][i] * scale, -limit), limit);
+          const float g = fminf(sum_as(acc[h][mt][i] * scale, expert == rounded), limit);
+          const float u = fminf(fmaxf(sum_as(acc[2 + h][mt][i] * scale, expert == rounded), -limit), limit);
           value[i] = live ? g / (1.0f + expf(-alpha * g)) * (u + offset) : 0.f;
         }
         store_four<TO>(row, n0 + 32 * wn + 16 * h + 4 * q, width, whole != 0, value);
@@ -552,7 +557,7 @@ moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const
         float value[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          value[i] = acc[nt][mt][i] * scale;
+          value[i] = sum_as(acc[nt][mt][i] * scale, expert == rounded);
           if (squared_relu) {
             value[i] = fmaxf(value[i], 0.f);
             value[i] *= value[i];
@@ -568,7 +573,7 @@ moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const
 template <typename T, typename TO>
 static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, long expert_stride, long ldw, int N, int K,
                                const int* source, const int* tile_expert, int tiles, int pad, int gather, int activation,
-                               float limit, float alpha, float offset, const float* row_scale, TO* out, long ldo,
+                               float limit, float alpha, float offset, const float* row_scale, int rounded, TO* out, long ldo,
                                hipStream_t stream) {
   const int glu = activation == 1;
   const int squared_relu = activation == 2;
@@ -576,7 +581,7 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
   const bool vec = K % PIECE == 0 && ldx % PIECE == 0 && ldw % PIECE == 0 && expert_stride % PIECE == 0 &&
                    ((unsigned long long)x % 16) == 0 && ((unsigned long long)W % 16) == 0;
   const int width = glu ? N / 2 : N;
-#define EXPERT_LAUNCH(VEC_, GLU_, MT_, PAIRS_)                                                                           moe_expert_gemm_kernel<T, TO, VEC_, GLU_, MT_, PAIRS_>                                                                    <<<dim3((unsigned)((width + 16 * PAIRS_ - 1) / (16 * PAIRS_)), (unsigned)tiles), TILE_THREADS, 0, stream>>>(               x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, out, ldo)
+#define EXPERT_LAUNCH(VEC_, GLU_, MT_, PAIRS_)                                                                           moe_expert_gemm_kernel<T, TO, VEC_, GLU_, MT_, PAIRS_>                                                                    <<<dim3((unsigned)((width + 16 * PAIRS_ - 1) / (16 * PAIRS_)), (unsigned)tiles), TILE_THREADS, 0, stream>>>(               x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, rounded, out, ldo)
 #define EXPERT_SHAPE(MT_, PAIRS_GLU_, PAIRS_PLAIN_)                                                                      do {                                                                                                                    if (vec && glu) EXPERT_LAUNCH(true, true, MT_, PAIRS_GLU_);                                                            else if (vec) EXPERT_LAUNCH(true, false, MT_, PAIRS_PLAIN_);                                                           else if (glu) EXPERT_LAUNCH(false, true, MT_, PAIRS_GLU_);                                                             else EXPERT_LAUNCH(false, false, MT_, PAIRS_PLAIN_);                                                                 } while (0)
   if ((pad == 128 || pad == 64) && vec) {      // (plans of 128 places are made of rows and matrices in whole pieces only)
     const dim3 grid((unsigned)((width + (glu ? 64 : 128) - 1) / (glu ? 64 : 128)), (unsigned)tiles);
@@ -584,7 +589,7 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
 #define EXPERT_WIDE(GLU_, ROWS_)                                                                                  \
   moe_expert_gemm_wide_kernel<T, TO, GLU_, ROWS_><<<grid, TILE_THREADS, 0, stream>>>(                             \
       x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, \
-      row_scale, out, ldo, whole)
+      row_scale, rounded, out, ldo, whole)
     if (pad == 128 && glu) EXPERT_WIDE(true, 128);
     else if (pad == 128) EXPERT_WIDE(false, 128);
     else if (glu) EXPERT_WIDE(true, 64);
@@ -602,7 +607,7 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
 extern "C" int mi_moe_expert_gemm(const void* x, int dtype, long ldx, int x_rows, const void* W, long expert_stride,
                                   long ldw, int N, int K, const int* source, const int* tile_expert, int tiles, int pad,
                                   int gather, int activation, float limit, float alpha, float offset,
-                                  const float* row_scale, void* out, int out_dtype, long ldo, hipStream_t stream) {
+                                  const float* row_scale, int rounded, void* out, int out_dtype, long ldo, hipStream_t stream) {
   // row_scale (or null): a number for every place that multiplies its row before the product (as the products are linear
   // in the row, the sums before the activation)
   // activation: 0 none, 1 the clamped gated one (the matrix holds gate rows then up rows), 2 max(z, 0)^2
@@ -620,13 +625,13 @@ extern "C" int mi_moe_expert_gemm(const void* x, int dtype, long ldx, int x_rows
   }
   if (dtype == DT_F32 && out_dtype == DT_F32)
     launch_expert_gemm<float, float>((const float*)x, ldx, x_rows, (const float*)W, expert_stride, ldw, N, K, source,
-                                     tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, (float*)out, ldo, stream);
+                                     tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (float*)out, ldo, stream);
   else if (dtype == DT_BF16 && out_dtype == DT_BF16)
     launch_expert_gemm<bf16_t, bf16_t>((const bf16_t*)x, ldx, x_rows, (const bf16_t*)W, expert_stride, ldw, N, K, source,
-                                       tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, (bf16_t*)out, ldo, stream);
+                                       tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (bf16_t*)out, ldo, stream);
   else if (dtype == DT_BF16 && out_dtype == DT_F32)
     launch_expert_gemm<bf16_t, float>((const bf16_t*)x, ldx, x_rows, (const bf16_t*)W, expert_stride, ldw, N, K, source,
-                                      tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, (float*)out, ldo, stream);
+                                      tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (float*)out, ldo, stream);
   else
     return ERR_BAD_ARGUMENT;
   RETURN_IF_LAUNCH_FAILED();

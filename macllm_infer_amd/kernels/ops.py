@@ -82,7 +82,7 @@ _SIGNATURES = {
         "mi_moe_plan": [_c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                         _c_int, _c_ptr],
         "mi_moe_expert_gemm": [_c_ptr, _c_int, _c_long, _c_int, _c_ptr, _c_long, _c_long, _c_int, _c_int, _c_ptr, _c_ptr,
-                               _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_ptr, _c_ptr, _c_int,
+                               _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_ptr, _c_int, _c_ptr, _c_int,
                                _c_long, _c_ptr],
         "mi_moe_combine": [_c_ptr, _c_long, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_long, _c_ptr, _c_int, _c_long, _c_ptr,
                            _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_float, _c_ptr,
@@ -997,9 +997,9 @@ def moe_tile_rows(tokens: int, top_k: int, num_experts: int, whole_pieces: bool 
     return MOE_WIDEST_TILE_ROWS if 10 * fills[0] > 11 * fills[1] else MOE_WIDE_TILE_ROWS
 
 
-def moe_shared_grouped(tokens: int, width: int, hidden: int) -> bool:
+def moe_shared_grouped(tokens: int, width: int, hidden: int, pad: int) -> bool:
     """Whether a shared expert like the routed ones (``width`` by ``hidden``, bfloat16) runs as one more of them in the
-    grouped products of a step: three launches less (two products and the activation between them, 10 us of small steps, 25
+    grouped products of a step, in tiles of ``pad`` places: three launches less (two products and the activation between them, 10 us of small steps, 25
     of prompts), where the matrices are small enough that those launches wait for little else.  us of the whole
     feed-forward, apart | grouped, by tokens (experts x hidden x width, choices a token):
 
@@ -1007,7 +1007,12 @@ def moe_shared_grouped(tokens: int, width: int, hidden: int) -> bool:
       77.5, 4,096 171 | 162
     * 64 x 1,024 x 512, 6: 12 46.3 | 41.6, 64 110 | 91, 512 105.5 | 103.9, 1,554 159 | 167 (another tile), 2,048 209 | 167
     * 64 x 2,048 x 1,024, 6: 12 131 | 121, 64 255 | 239, 128 302 | 296, 256 390 | 402, 1,024 325 | 353, 2,048 478 | 443
-    * 8 x 3,072 x 3,072, 2: 1 65.9 | 70.0, 12 134 | 129, 64 216 | 227, 512 258 | 225, 1,024 318 | 335, 4,096 968 | 1,000"""
+    * 8 x 3,072 x 3,072, 2: 1 65.9 | 70.0, 12 134 | 129, 64 216 | 227, 512 258 | 225, 1,024 318 | 335, 4,096 968 | 1,000
+
+    And only where its sums have the order of the products apart, so that a step gives the same bits either way: tiles of 16
+    places split K as the product of few rows does, wider ones sum in k order as the product of many does."""
+    if tokens > SKINNY_ROWS if pad == MOE_TILE_ROWS else tokens < 32:
+        return False
     first = 2 * width * hidden
     return first <= 1 << 21 or (first <= 1 << 22 and tokens <= 128)
 
@@ -1117,13 +1122,14 @@ def moe_route_plan(logits: torch.Tensor, num_experts: int, top_k: int, correctio
 
 
 def moe_expert_gemm(x: torch.Tensor, plan: MoePlan, weight: torch.Tensor, out: torch.Tensor, gather: bool, glu,
-                    squared_relu: bool = False, row_scale: Optional[torch.Tensor] = None) -> None:
+                    squared_relu: bool = False, row_scale: Optional[torch.Tensor] = None, rounded: Optional[int] = None) -> None:
     """The grouped product of a plan's rows with their experts' matrices ``weight`` [experts, N, K]: the row at a
     place is ``x[source[place]]`` (``gather``) or ``x[place]``; out[place] = weight[expert] . row, or with ``glu``
     (limit, alpha, up_offset; N = 2 I, gate rows then up rows) the clamped gated activation of the two halves,
     [capacity, I]; or with ``squared_relu`` max(weight[expert] . row, 0)^2.  Float32 sums on the matrix cores;
     float32 operands give a true 32-bit product.  ``row_scale`` float32 [capacity]: a number that multiplies a place's row
-    before the product (applied, in float32, to the sums before the activation)."""
+    before the product (applied, in float32, to the sums before the activation).  ``rounded``: the expert whose sums are
+    rounded to bfloat16 first, as a product of its own does."""
     _need(row_scale is None or (row_scale.dtype == torch.float32 and row_scale.numel() == plan.capacity
                                 and row_scale.is_contiguous() and row_scale.is_cuda),
           "moe_expert_gemm: row_scale must be float32 [capacity] on the GPU")
@@ -1140,7 +1146,8 @@ def moe_expert_gemm(x: torch.Tensor, plan: MoePlan, weight: torch.Tensor, out: t
         _p(x), _dt(x), ldx, x.shape[0], _p(weight), N * K, K, N, K, _p(plan.source), _p(plan.tile_expert),
         plan.tile_expert.numel(), plan.pad, 1 if gather else 0, 1 if glu is not None else (2 if squared_relu else 0),
         float(glu.limit) if glu is not None else 0.0, float(glu.alpha) if glu is not None else 0.0,
-        float(glu.up_offset) if glu is not None else 0.0, _p(row_scale), _p(out), _dt(out), ldo, _stream()),
+        float(glu.up_offset) if glu is not None else 0.0, _p(row_scale), -1 if rounded is None else int(rounded), _p(out), _dt(out), ldo,
+        _stream()),
         "moe_expert_gemm", f"(N={N}, K={K})")
 
 
@@ -1439,7 +1446,7 @@ def rows_gemm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 
 
-def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False) -> bool:
+def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False, keep_float32: bool = False) -> bool:
     """Whether this package's product of many rows is the faster one, the library the other: where tiles of 64 rows by 64
     or 128 features fit the compute units once.  Its time | the library's over 33 to 4,096 rows and 256 to 8,192 features
     (rows and weights from memory), least, median and most:
@@ -1455,7 +1462,13 @@ def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False) -> bool:
     * K = 512: 0.49 to 0.8
     * K = 1,024: 0.51 0.58 0.60; 0.59 0.63 0.67; 0.60 0.70 0.74; 128 x 128 twice 0.78 0.83 0.89, more 0.73 0.90 1.05 (of up to 4,096
       features 0.73 to 0.96)
-    * K = 2,048: 0.70 0.77 0.86; 0.68 0.86 0.93; 0.79 0.80 0.87; twice 0.87 0.98 1.11, more 0.91 1.15 1.31"""
+    * K = 2,048: 0.70 0.77 0.86; 0.68 0.86 0.93; 0.79 0.80 0.87; twice 0.87 0.98 1.11, more 0.91 1.15 1.31
+
+    ``keep_float32``: sums that are not rounded, of K up to 64 only.  The library's order of them is nearer to the exact sum (17
+    features of K = 1,024: relative error 0.95e-7, in k order 1.9e-7).  Rounded products of 32 rows and more have the library's
+    bits; it splits K where there are fewer."""
+    if M < 32 or (keep_float32 and K > 64):
+        return False
     tiles = lambda rows, features: -(-M // rows) * -(-N // features)
     small, wide, large = tiles(64, 64) <= GEMM_UNITS, tiles(64, 128) <= GEMM_UNITS, tiles(128, 128)
     if swiglu:
@@ -1558,7 +1571,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], 
         fused_gemm(weight, bias, out, x=x)
         return out
     _need(not keep_float32 or bias is None, "linear: float32 results of bfloat16 operands come without a bias")
-    if (rows_gemm_pays(M, weight.shape[0], K) and rows_gemm_supported(x, weight)
+    if (rows_gemm_pays(M, weight.shape[0], K, keep_float32=keep_float32) and rows_gemm_supported(x, weight)
             and (bias is None or (bias.dtype == torch.float32 and bias.numel() == weight.shape[0] and bias.is_contiguous()))):
         return rows_gemm(x, weight, bias, keep_float32=keep_float32)
     if keep_float32:

@@ -33,7 +33,7 @@ class RoutedExperts(FeedForward):
     the order of the token's choices, together with the gated shared expert.  A token's result does not depend on
     which other tokens share its expert's tiles: a row of a tile is summed on its own.  The output is float32.
     Steps of up to 64 tokens are routed and grouped in one launch; a bfloat16 shared expert of the routed ones' size and
-    clamped activation runs as one more of them where that pays (``ops.moe_shared_grouped``); one whose activation is plain SiLU runs as
+    clamped activation runs as one more of them where that pays (``ops.moe_shared_grouped``), with the same bits; one whose activation is plain SiLU runs as
     the dense gated feed-forward does (its activation in the product's epilogue in small steps)."""
     graph_safe = True
     takes_tail = True
@@ -132,10 +132,11 @@ class RoutedExperts(FeedForward):
         how = dict(routing=spec.routing, renormalize=spec.renormalize, groups=spec.groups, kept_groups=spec.kept_groups)
         choice = (logits, spec.router_outputs, spec.top_k, self.correction, spec.route_scale, spec.weight_eps,
                   self.shared and spec.shared_gated)
-        grouped = self.shared_grouped and ops.moe_shared_grouped(tokens, spec.expert_size, hidden)
-        pad = ops.moe_tile_rows(tokens, spec.top_k + grouped, spec.num_experts + grouped, self.whole_pieces,
-                                self.gate_up.dtype, self.gate_up.shape[1])
+        pad = ops.moe_tile_rows(tokens, spec.top_k, spec.num_experts, self.whole_pieces, self.gate_up.dtype,
+                                self.gate_up.shape[1])
+        grouped = self.shared_grouped and ops.moe_shared_grouped(tokens, spec.expert_size, hidden, pad)
         in_front = dict(shared=True) if grouped else {}
+        rounded = dict(rounded=spec.num_experts) if grouped else {}
         if tokens <= ops.ROUTE_PLAN_TOKENS:
             _, weights, gate, plan = ops.moe_route_plan(*choice, experts_with_matrices=spec.num_experts, pad=pad,
                                                          place_weights=spec.input_weighted, **how, **in_front)
@@ -147,9 +148,9 @@ class RoutedExperts(FeedForward):
         rows = x if x.dtype == self.gate_up.dtype else x.to(self.gate_up.dtype)
         inner = torch.empty((plan.capacity, spec.expert_size), dtype=rows.dtype, device=x.device)
         ops.moe_expert_gemm(rows, plan, self.gate_up, inner, gather=True, glu=spec.activation if self.gated else None,
-                            squared_relu=not self.gated, row_scale=plan.place_weight if spec.input_weighted else None)
+                            squared_relu=not self.gated, row_scale=plan.place_weight if spec.input_weighted else None, **rounded)
         down = torch.empty((plan.capacity, hidden), dtype=torch.float32, device=x.device)
-        ops.moe_expert_gemm(inner, plan, self.down, down, gather=False, glu=None)
+        ops.moe_expert_gemm(inner, plan, self.down, down, gather=False, glu=None, **rounded)
         shared_rows = None
         if self.shared:
             shared_rows = down[:tokens] if grouped else self._shared_rows(x)

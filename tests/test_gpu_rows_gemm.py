@@ -107,10 +107,11 @@ def test_rows_of_a_wider_matrix_infinities_and_what_is_refused():
         module.rows_gemm(rand(4, 96).to(torch.bfloat16).to(DEV), rand(4, 96).to(torch.bfloat16).to(DEV))     # K no multiple of 64
 
 
-@pytest.mark.parametrize("M, N, K", [(17, 48, 64), (40, 1024, 1024), (300, 260, 512), (600, 1024, 2048)])
+@pytest.mark.parametrize("M, N, K", [(32, 48, 64), (40, 1024, 1024), (300, 260, 512), (600, 1024, 2048)])
 def test_linear_takes_it_where_it_pays_and_gives_the_librarys_numbers(M, N, K):
     module = ops()
-    assert module.rows_gemm_pays(M, N, K)
+    assert module.rows_gemm_pays(M, N, K) and module.rows_gemm_pays(M, N, K, keep_float32=True) == (K == 64)
+    assert not module.rows_gemm_pays(31, N, K)
     x, w, b = rand(M, K, seed=9).to(torch.bfloat16).to(DEV), (rand(N, K, seed=10) / math.sqrt(K)).to(torch.bfloat16).to(DEV), rand(N, seed=11).to(DEV)
     # two roundings to bfloat16 of sums that differ by float32 rounding: a neighbouring value at most
     for bias in (None, b):
