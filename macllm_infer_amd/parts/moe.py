@@ -135,6 +135,9 @@ class RoutedExperts(FeedForward):
         pad = ops.moe_tile_rows(tokens, spec.top_k, spec.num_experts, self.whole_pieces, self.gate_up.dtype,
                                 self.gate_up.shape[1])
         grouped = self.shared_grouped and ops.moe_shared_grouped(tokens, spec.expert_size, hidden, pad)
+        if grouped and pad > ops.MOE_TILE_ROWS:           # (the wide tiles, which sum alike, for the rows that there are now)
+            pad = max(ops.MOE_WIDE_TILE_ROWS, ops.moe_tile_rows(tokens, spec.top_k + 1, spec.num_experts + 1, self.whole_pieces,
+                                                                self.gate_up.dtype, self.gate_up.shape[1]))
         in_front = dict(shared=True) if grouped else {}
         rounded = dict(rounded=spec.num_experts) if grouped else {}
         if tokens <= ops.ROUTE_PLAN_TOKENS:
