@@ -150,6 +150,22 @@ def test_one_product_per_head(dtype, T, heads, N, K, x_col, x_stride, out_col, o
     close(got.float(), want.float(), dtype)
 
 
+@pytest.mark.parametrize("T, heads, N, K", [(33, 2, 4, 8), (63, 1, 36, 40), (64, 8, 128, 64), (65, 3, 64, 72), (130, 8, 64, 128),
+                                            (200, 2, 32, 96), (1030, 1, 100, 64), (70, 2, 30, 64), (70, 2, 32, 136)])
+def test_a_heads_product_of_many_rows_has_the_bits_of_one_of_few(T, heads, N, K):
+    """A row's sum does not depend on how many there are, whichever kernel takes them (the last two: neither groups of four
+    features nor a K that a wave holds)."""
+    x = rand(T, heads * (K + 8), seed=1).to(torch.bfloat16).to(DEV)
+    weight = (rand(heads, N, K, seed=2) / K ** 0.5).to(torch.bfloat16).to(DEV)
+    together, apart = (torch.full((T, heads * (N + 4)), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops().head_linear(x, 0, K + 8, weight, together, 0, N + 4)
+    for row in range(0, T, 32):
+        ops().head_linear(x[row:row + 32], 0, K + 8, weight, apart[row:row + 32], 0, N + 4)
+    assert torch.equal(together, apart)
+    want = torch.stack([x.view(T, heads, K + 8)[:, head, :K].double() @ weight[head].double().T for head in range(heads)], 1)
+    close(together.view(T, heads, N + 4)[:, :, :N].float(), want.float(), torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T, heads, dim, rope, rotary, rank, interleaved", [
     (1, 8, 64, 32, 32, 128, True), (16, 3, 16, 8, 6, 20, False), (17, 8, 64, 32, 32, 128, True), (33, 2, 24, 12, 0, 8, False),
