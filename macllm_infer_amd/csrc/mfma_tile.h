@@ -60,8 +60,9 @@ __device__ __forceinline__ tile_floatx4 tile_mfma(const tile_bf16x8& a, const ti
 }
 
 // This wave's share of the products: w_row[nt] / x_row[mt] point at the weight row / the row of x that this
-// lane's column of the operands comes from (lane % 16), already clamped to valid rows.
-template <typename T, int MT, int NT, bool VEC>
+// lane's column of the operands comes from (lane % 16), already clamped to valid rows.  AT_ONCE chunks are asked for before the
+// first is used (it changes no sum).
+template <typename T, int MT, int NT, bool VEC, int AT_ONCE = 2>
 __device__ __forceinline__ void tile_accumulate(const T* const (&w_row)[NT], const T* const (&x_row)[MT], int K,
                                                 tile_floatx4 (&acc)[NT][MT]) {
   typedef typename TileTraits<T>::Piece Piece;
@@ -78,11 +79,11 @@ __device__ __forceinline__ void tile_accumulate(const T* const (&w_row)[NT], con
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = tile_floatx4{0.f, 0.f, 0.f, 0.f};
-  // two chunks are asked for before the first is used; a chunk past the wave's run reads as zeros
-  for (int first = 0; first < iterations; first += 2) {
-    Piece a[2][NT], b[2][MT];
+  // a chunk past the wave's run reads as zeros
+  for (int first = 0; first < iterations; first += AT_ONCE) {
+    Piece a[AT_ONCE][NT], b[AT_ONCE][MT];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < AT_ONCE; ++j) {
       const int k = first + j < iterations ? (first_chunk + first + j) * CHUNK + PIECE * q : K;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) a[j][nt] = tile_load<T, VEC>(w_row[nt], k, K);
@@ -90,7 +91,7 @@ __device__ __forceinline__ void tile_accumulate(const T* const (&w_row)[NT], con
       for (int mt = 0; mt < MT; ++mt) b[j][mt] = tile_load<T, VEC>(x_row[mt], k, K);
     }
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < AT_ONCE; ++j)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll

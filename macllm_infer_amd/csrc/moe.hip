@@ -342,29 +342,37 @@ extern "C" int mi_moe_route_plan(const float* logits, long ld, int T, int E, int
 }
 
 // ---------------------------------------------------------------- the grouped product
+// The sums of the expert `rounded` (-1: none) are rounded to bfloat16 before anything else is done with them, as those of a product
+// of its own are, and in the same order: an expert gets the same bits in a launch with others as in launches of its own.  In tiles
+// of 16 places that is the order of the product of few rows, four runs of K (K up to 1,024), or with in_k_order that of the
+// product of many rows, which the tiles of 64 and 128 places have anyway.  In k order a wave walks all of K, eight chunks at a time,
+// beside the routed experts' tiles: steps of twelve layers with the shared expert apart | so, us: 32 decoded tokens 1,372 | 1,253,
+// 64 1,638 | 1,477, a prompt of 40 1,391 | 1,236, 100 1,403 | 1,310.
+__device__ __forceinline__ float sum_as(float sum, bool rounded) { return rounded ? (float)(bf16_t)sum : sum; }
+
 // Tile t of 16 MT places belongs to expert tile_expert[t] (none: the workgroup leaves).  A workgroup owns the
 // tile's rows and PAIRS tiles of 16 output features.  GLU: the expert's matrix is [2 I, K], gate rows then up
 // rows; out[place, n] = act(gate tile, up tile), n < I.  Places without a row get zeros.  Steps of few rows take
 // MT = 1 (every expert's matrix is read once, by as many workgroups as it has tiles of features); prompt portions,
 // whose experts get dozens of rows each, MT = 4 and four tiles of features (the rows and the matrix come from the
-// caches, 64 x 64 results a workgroup).
-// The sums of the expert `rounded` (-1: none) are rounded to bfloat16 before anything else is done with them, as those of a product
-// of its own are: an expert gets the same bits in a launch with others as in launches of its own (up to 16 rows with K up to
-// 1,024 in tiles of 16 places, four runs of K; in tiles of 64 and 128 places those of a product of many rows, in k order).
-__device__ __forceinline__ float sum_as(float sum, bool rounded) { return rounded ? (float)(bf16_t)sum : sum; }
-
+// caches, 64 x 64 results a workgroup).  Steps of few rows are bound by the matrices (12 tokens, 16 of 17 experts of 512 x 1,024: 33 MB
+// in 9.8 us, 17 in 8.1, launch and two round trips of the tables among it); a wave's whole run of up to eight chunks is on its way
+// at once (two of them: a prompt of 40 1,254 -> 1,236 us, of 64 1,359 -> 1,343, 12 decoded tokens the same).
 template <typename T, typename TO, bool VEC, bool GLU, int MT, int PAIRS>
 __global__ void __launch_bounds__(TILE_THREADS)
 moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* __restrict__ W, long expert_stride, long ldw,
                        int N, int K, const int* __restrict__ source, const int* __restrict__ tile_expert, int gather,
                        float limit, float alpha, float offset, int squared_relu,
-                       const float* __restrict__ row_scale, int rounded, TO* __restrict__ out, long ldo) {
+                       const float* __restrict__ row_scale, int rounded, int in_k_order, TO* __restrict__ out, long ldo) {
   __shared__ float red[TILE_WAVES][256];
   const int tile = blockIdx.y;
-  const int expert = tile_expert[tile];
-  if (expert < 0) return;
   const int tid = threadIdx.x;
   const int r = (tid & (WAVE - 1)) % 16;
+  const int expert = tile_expert[tile];
+  int from[MT];                                      // the rows that stand at the tile's places, beside the expert's number
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) from[mt] = source[(tile * MT + mt) * 16 + r];
+  if (expert < 0) return;
   const int width = GLU ? N / 2 : N;
   const long n0 = (long)blockIdx.x * 16 * PAIRS;
   const T* matrix = W + (long)expert * expert_stride;
@@ -379,22 +387,57 @@ moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* _
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const int place_in = (tile * MT + mt) * 16 + r;
-    const long x_at = gather ? max(source[place_in], 0) : place_in;
+    const long x_at = gather ? max(from[mt], 0) : (tile * MT + mt) * 16 + r;
     x_row[mt] = x + min(x_at, (long)x_rows - 1) * ldx;
   }
   tile_floatx4 acc[NT][MT];
-  tile_accumulate<T, MT, NT, VEC>(w_row, x_row, K, acc);
   const int l = tid % 64;
+  bool serial = false;                               // the tiles of `rounded` whose sums run through K in one wave each
+  if constexpr (MT == 1 && PAIRS == 1 && VEC) {
+    serial = in_k_order && expert == rounded;
+    if (serial) {
+      // the NT tiles of features by as many waves, eight chunks asked for at once; the sums to where tile_reduce would read them
+      constexpr int CHUNK = TileTraits<T>::CHUNK, PIECE = TileTraits<T>::PIECE;
+      const int wave = tid / WAVE, q = (tid & (WAVE - 1)) / 16;
+      const T* const mine = w_row[NT > 1 && wave == 1 ? NT - 1 : 0];
+      tile_floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+      if (wave < NT)
+        for (int k0 = 0; k0 < K; k0 += 8 * CHUNK) {
+          typename TileTraits<T>::Piece a[8], b[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            a[j] = tile_load<T, true>(mine, k0 + j * CHUNK + PIECE * q, K);
+            b[j] = tile_load<T, true>(x_row[0], k0 + j * CHUNK + PIECE * q, K);
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sum = tile_mfma(a[j], b[j], sum);
+        }
+      if (wave < NT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][i * 64 + (tid & (WAVE - 1))] = sum[i];
+      }
+      __syncthreads();
+    }
+  }
+  if constexpr (MT == 1 && PAIRS == 1 && VEC) {
+    if (serial) {
+    } else if (K <= TILE_WAVES * 4 * TileTraits<T>::CHUNK) {
+      tile_accumulate<T, MT, NT, VEC, 4>(w_row, x_row, K, acc);
+    } else {
+      tile_accumulate<T, MT, NT, VEC, 8>(w_row, x_row, K, acc);
+    }
+  } else {
+    tile_accumulate<T, MT, NT, VEC>(w_row, x_row, K, acc);
+  }
 #pragma unroll
   for (int p = 0; p < PAIRS; ++p)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int place = (tile * MT + mt) * 16 + (l % 16);
       const float scale = row_scale ? row_scale[place] : 1.0f;
-      float value = sum_as(tile_reduce(acc[p][mt], red) * scale, expert == rounded);
+      float value = sum_as((serial ? red[0][tid] : tile_reduce(acc[p][mt], red)) * scale, expert == rounded);
       if (GLU) {
-        const float up = sum_as(tile_reduce(acc[NT - PAIRS + p][mt], red) * scale, expert == rounded);
+        const float up = sum_as((serial ? red[1][tid] : tile_reduce(acc[NT - PAIRS + p][mt], red)) * scale, expert == rounded);
         const float g = fminf(value, limit);
         const float u = fminf(fmaxf(up, -limit), limit);
         value = g / (1.0f + expf(-alpha * g)) * (u + offset);
@@ -403,7 +446,7 @@ moe_expert_gemm_kernel(const T* __restrict__ x, long ldx, int x_rows, const T* _
         value *= value;
       }
       const long n = n0 + 16 * p + 4 * (l / 16) + tid / 64;
-      if (n < width) out[(long)place * ldo + n] = from_float<TO>(source[place] >= 0 ? value : 0.f);
+      if (n < width) out[(long)place * ldo + n] = from_float<TO>(from[mt] >= 0 ? value : 0.f);
     }
 }
 
@@ -573,7 +616,7 @@ moe_expert_gemm_wide_kernel(const T* __restrict__ x, long ldx, int x_rows, const
 template <typename T, typename TO>
 static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, long expert_stride, long ldw, int N, int K,
                                const int* source, const int* tile_expert, int tiles, int pad, int gather, int activation,
-                               float limit, float alpha, float offset, const float* row_scale, int rounded, TO* out, long ldo,
+                               float limit, float alpha, float offset, const float* row_scale, int rounded, int in_k_order, TO* out, long ldo,
                                hipStream_t stream) {
   const int glu = activation == 1;
   const int squared_relu = activation == 2;
@@ -581,7 +624,7 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
   const bool vec = K % PIECE == 0 && ldx % PIECE == 0 && ldw % PIECE == 0 && expert_stride % PIECE == 0 &&
                    ((unsigned long long)x % 16) == 0 && ((unsigned long long)W % 16) == 0;
   const int width = glu ? N / 2 : N;
-#define EXPERT_LAUNCH(VEC_, GLU_, MT_, PAIRS_)                                                                           moe_expert_gemm_kernel<T, TO, VEC_, GLU_, MT_, PAIRS_>                                                                    <<<dim3((unsigned)((width + 16 * PAIRS_ - 1) / (16 * PAIRS_)), (unsigned)tiles), TILE_THREADS, 0, stream>>>(               x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, rounded, out, ldo)
+#define EXPERT_LAUNCH(VEC_, GLU_, MT_, PAIRS_)                                                                           moe_expert_gemm_kernel<T, TO, VEC_, GLU_, MT_, PAIRS_>                                                                    <<<dim3((unsigned)((width + 16 * PAIRS_ - 1) / (16 * PAIRS_)), (unsigned)tiles), TILE_THREADS, 0, stream>>>(               x, ldx, x_rows, W, expert_stride, ldw, N, K, source, tile_expert, gather, limit, alpha, offset, squared_relu, row_scale, rounded, in_k_order, out, ldo)
 #define EXPERT_SHAPE(MT_, PAIRS_GLU_, PAIRS_PLAIN_)                                                                      do {                                                                                                                    if (vec && glu) EXPERT_LAUNCH(true, true, MT_, PAIRS_GLU_);                                                            else if (vec) EXPERT_LAUNCH(true, false, MT_, PAIRS_PLAIN_);                                                           else if (glu) EXPERT_LAUNCH(false, true, MT_, PAIRS_GLU_);                                                             else EXPERT_LAUNCH(false, false, MT_, PAIRS_PLAIN_);                                                                 } while (0)
   if ((pad == 128 || pad == 64) && vec) {      // (plans of 128 places are made of rows and matrices in whole pieces only)
     const dim3 grid((unsigned)((width + (glu ? 64 : 128) - 1) / (glu ? 64 : 128)), (unsigned)tiles);
@@ -607,7 +650,7 @@ static void launch_expert_gemm(const T* x, long ldx, int x_rows, const T* W, lon
 extern "C" int mi_moe_expert_gemm(const void* x, int dtype, long ldx, int x_rows, const void* W, long expert_stride,
                                   long ldw, int N, int K, const int* source, const int* tile_expert, int tiles, int pad,
                                   int gather, int activation, float limit, float alpha, float offset,
-                                  const float* row_scale, int rounded, void* out, int out_dtype, long ldo, hipStream_t stream) {
+                                  const float* row_scale, int rounded, int in_k_order, void* out, int out_dtype, long ldo, hipStream_t stream) {
   // row_scale (or null): a number for every place that multiplies its row before the product (as the products are linear
   // in the row, the sums before the activation)
   // activation: 0 none, 1 the clamped gated one (the matrix holds gate rows then up rows), 2 max(z, 0)^2
@@ -625,13 +668,13 @@ extern "C" int mi_moe_expert_gemm(const void* x, int dtype, long ldx, int x_rows
   }
   if (dtype == DT_F32 && out_dtype == DT_F32)
     launch_expert_gemm<float, float>((const float*)x, ldx, x_rows, (const float*)W, expert_stride, ldw, N, K, source,
-                                     tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (float*)out, ldo, stream);
+                                     tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, in_k_order, (float*)out, ldo, stream);
   else if (dtype == DT_BF16 && out_dtype == DT_BF16)
     launch_expert_gemm<bf16_t, bf16_t>((const bf16_t*)x, ldx, x_rows, (const bf16_t*)W, expert_stride, ldw, N, K, source,
-                                       tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (bf16_t*)out, ldo, stream);
+                                       tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, in_k_order, (bf16_t*)out, ldo, stream);
   else if (dtype == DT_BF16 && out_dtype == DT_F32)
     launch_expert_gemm<bf16_t, float>((const bf16_t*)x, ldx, x_rows, (const bf16_t*)W, expert_stride, ldw, N, K, source,
-                                      tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, (float*)out, ldo, stream);
+                                      tile_expert, tiles, pad, gather, activation, limit, alpha, offset, row_scale, rounded, in_k_order, (float*)out, ldo, stream);
   else
     return ERR_BAD_ARGUMENT;
   RETURN_IF_LAUNCH_FAILED();

@@ -82,8 +82,8 @@ _SIGNATURES = {
         "mi_moe_plan": [_c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                         _c_int, _c_ptr],
         "mi_moe_expert_gemm": [_c_ptr, _c_int, _c_long, _c_int, _c_ptr, _c_long, _c_long, _c_int, _c_int, _c_ptr, _c_ptr,
-                               _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_ptr, _c_int, _c_ptr, _c_int,
-                               _c_long, _c_ptr],
+                               _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_ptr, _c_int, _c_int, _c_ptr,
+                               _c_int, _c_long, _c_ptr],
         "mi_moe_combine": [_c_ptr, _c_long, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_long, _c_ptr, _c_int, _c_long, _c_ptr,
                            _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_float, _c_ptr,
                            _c_ptr],
@@ -1009,9 +1009,9 @@ def moe_shared_grouped(tokens: int, width: int, hidden: int, pad: int) -> bool:
     * 64 x 2,048 x 1,024, 6: 12 131 | 121, 64 255 | 239, 128 302 | 296, 256 390 | 402, 1,024 325 | 353, 2,048 478 | 443
     * 8 x 3,072 x 3,072, 2: 1 65.9 | 70.0, 12 134 | 129, 64 216 | 227, 512 258 | 225, 1,024 318 | 335, 4,096 968 | 1,000
 
-    And only where its sums have the order of the products apart, so that a step gives the same bits either way: tiles of 16
-    places split K as the product of few rows does, wider ones sum in k order as the product of many does."""
-    if tokens > SKINNY_ROWS if pad == MOE_TILE_ROWS else tokens < 32:
+    A step gives the same bits either way, except of 17 to 31 tokens, where the library splits the K of the products apart: those
+    stay apart, and so do tiles of 16 places of rows that are not whole pieces, whose kernel has the one order only."""
+    if SKINNY_ROWS < tokens < 32 or (tokens > SKINNY_ROWS and pad == MOE_TILE_ROWS and (width % 8 or hidden % 8)):
         return False
     first = 2 * width * hidden
     return first <= 1 << 21 or (first <= 1 << 22 and tokens <= 128)
@@ -1129,7 +1129,7 @@ def moe_expert_gemm(x: torch.Tensor, plan: MoePlan, weight: torch.Tensor, out: t
     [capacity, I]; or with ``squared_relu`` max(weight[expert] . row, 0)^2.  Float32 sums on the matrix cores;
     float32 operands give a true 32-bit product.  ``row_scale`` float32 [capacity]: a number that multiplies a place's row
     before the product (applied, in float32, to the sums before the activation).  ``rounded``: the expert whose sums are
-    rounded to bfloat16 first, as a product of its own does."""
+    rounded to bfloat16 first and summed in the order of a product of its own of as many rows."""
     _need(row_scale is None or (row_scale.dtype == torch.float32 and row_scale.numel() == plan.capacity
                                 and row_scale.is_contiguous() and row_scale.is_cuda),
           "moe_expert_gemm: row_scale must be float32 [capacity] on the GPU")
@@ -1146,8 +1146,8 @@ def moe_expert_gemm(x: torch.Tensor, plan: MoePlan, weight: torch.Tensor, out: t
         _p(x), _dt(x), ldx, x.shape[0], _p(weight), N * K, K, N, K, _p(plan.source), _p(plan.tile_expert),
         plan.tile_expert.numel(), plan.pad, 1 if gather else 0, 1 if glu is not None else (2 if squared_relu else 0),
         float(glu.limit) if glu is not None else 0.0, float(glu.alpha) if glu is not None else 0.0,
-        float(glu.up_offset) if glu is not None else 0.0, _p(row_scale), -1 if rounded is None else int(rounded), _p(out), _dt(out), ldo,
-        _stream()),
+        float(glu.up_offset) if glu is not None else 0.0, _p(row_scale), -1 if rounded is None else int(rounded),
+        1 if plan.tokens > SKINNY_ROWS else 0, _p(out), _dt(out), ldo, _stream()),
         "moe_expert_gemm", f"(N={N}, K={K})")
 
 

@@ -315,7 +315,7 @@ def test_a_shared_expert_among_the_routed_ones_gives_what_it_gives_apart(T, monk
     assert max(errors.values()) < 3 * 2.0 ** -9, errors
 
 
-@pytest.mark.parametrize("T", [1, 12, 16, 171, 300, 777])
+@pytest.mark.parametrize("T", [1, 12, 16, 32, 33, 64, 65, 170, 171, 300, 777])
 def test_a_shared_expert_has_the_same_bits_grouped_and_apart(T, monkeypatch):
     from macllm_infer_amd.config import ClampedGLUSpec, RoutedExpertsSpec
     from macllm_infer_amd.parts.base import BuildContext
