@@ -204,7 +204,7 @@ __device__ __forceinline__ void ssd_conv_block(const bf16_t* __restrict__ u, lon
 // A layer whose attention and state-space mixer read the same projected rows runs two chains of small launches that do
 // not depend on each other: rotation and cache write, then the attention; conv and prepare, then the scan.  In a short
 // prompt none of them fills the GPU and each costs its launch and its round trips, so the attention's two run as further
-// workgroups of the scan's two.  37 tokens of the 0.5B shape through 36 layers: 2,314 us in four launches, 1,954 in two; 128 tokens of
+// workgroups of the scan's two, or in chunks of the first and the last of its four.  37 tokens of the 0.5B shape through 36 layers: 2,314 us in four launches, 1,954 in two; 128 tokens of
 // twelve layers of the 7B shape 3,100 and 2,872.
 struct PromptBeside {
   void* qkv;                       // rows [q | k | v] of T tokens, bfloat16
@@ -232,6 +232,18 @@ struct PromptBeside {
   int ahead_count;
 };
 #define BESIDE_AHEAD_BLOCKS 128    // by so many workgroups, a multiple of 8
+
+// workgroup `index` of the attention's
+template <int DH, int NSET>
+__device__ __forceinline__ void prompt_attention_beside(unsigned char* __restrict__ smem, const int index, const PromptBeside& beside) {
+  const int places = 4 * beside.n_tiles;
+  prefill_attention_block<DH, NSET>(smem, index % places, places, index / places % beside.Hkv, index / places / beside.Hkv,
+                                    (const bf16_t*)beside.qkv, beside.ld, beside.Hq, beside.Hkv, (const bf16_t*)beside.k_base,
+                                    (const bf16_t*)beside.v_base, beside.page_stride, beside.page_size, beside.block_tables,
+                                    beside.max_pages, beside.tiles, beside.cu_seqlens, beside.start_pos, beside.scale,
+                                    beside.window, (bf16_t*)beside.out, beside.out_ld, nullptr, nullptr, DH, nullptr, nullptr, 0,
+                                    nullptr, nullptr, 0, DH);
+}
 
 // prepare (rows 0 .. H-1 of the grid) and the conv with the transpose (the rows after) in one launch (their code inlined in
 // both instances: as a function called from two kernels the conv took 30 us where it takes 16); with BESIDE the rows
@@ -603,6 +615,7 @@ ssd_chunk_scan_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t*
 }
 
 #define SSD_SCAN_WAVES 8
+static_assert(SSD_SCAN_WAVES == PREFILL_WAVES, "workgroups of one launch");
 // The same with the operands that the eight tiles of 128 tokens share staged in LDS: one
 // workgroup of eight waves per (chunk, head, 128 tokens), a tile of 16 tokens a wave.  S_in of
 // the head (64 rows at a time), then, 64 tokens s at a time, the rows of B and the columns of
@@ -610,30 +623,27 @@ ssd_chunk_scan_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t*
 // skip and the gate are read per tile.  Rows are padded by 16 bytes so that the 16 rows a
 // matrix-core operand reads fall in different banks.  Head sizes up to 128.
 template <int NK, int PT>
-__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
-ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
-                          const bf16_t* __restrict__ state_in, const float* __restrict__ delta,
-                          const float* __restrict__ cum, const float* __restrict__ D,
-                          const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y,
-                          long y_ld, const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated,
-                          long gated_ld) {
+__device__ __forceinline__ void
+ssd_chunk_scan_block(unsigned char* __restrict__ scan_smem, const int chunk, const int head, const int part,
+                     const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                     const bf16_t* __restrict__ state_in, const float* __restrict__ delta,
+                     const float* __restrict__ cum, const float* __restrict__ D,
+                     const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y,
+                     long y_ld, const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated,
+                     long gated_ld) {
   constexpr int N = 32 * NK;
   constexpr int P = 16 * PT;
   constexpr int LD1 = N + 8;                     // row stride of the S / B buffer
   constexpr int LDX = 64 + 8;                    // row stride of the x^T buffer
   constexpr int THREADS = SSD_SCAN_WAVES * WAVE;
-  extern __shared__ __align__(16) unsigned char scan_smem[];
   bf16_t* buf1 = reinterpret_cast<bf16_t*>(scan_smem);                 // [64][LD1]: S_in rows, then B rows
   bf16_t* buf_x = buf1 + 64 * LD1;                                     // [P][LDX]
   float* L = reinterpret_cast<float*>(buf_x + (long)P * LDX);          // [Q]
   float* step = L + Q;                                                 // [Q]
-  const int chunk = blockIdx.x;
-  const int head = blockIdx.y;
   const int group = head / (H / G);
   const int t0 = chunks[4 * chunk + 1];
   const int length = chunks[4 * chunk + 2];
   if (length <= 0) return;                    // a row of the table past the step's own chunks: the whole workgroup leaves
-  const int part = gridDim.z - 1 - blockIdx.z;                         // the later 128 tokens first: they have more before them
   if (part * 128 >= length) return;
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
@@ -795,6 +805,42 @@ ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf1
     }
   }
 }
+
+#define SCAN_OPERANDS xbc, xbc_ld, TT, E, state_in, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld
+template <int NK, int PT>
+__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE)
+ssd_chunk_scan_lds_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                          const bf16_t* __restrict__ state_in, const float* __restrict__ delta,
+                          const float* __restrict__ cum, const float* __restrict__ D,
+                          const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y,
+                          long y_ld, const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated,
+                          long gated_ld) {
+  extern __shared__ __align__(16) unsigned char scan_smem[];
+  // the later 128 tokens first: they have more before them
+  ssd_chunk_scan_block<NK, PT>(scan_smem, blockIdx.x, blockIdx.y, gridDim.z - 1 - blockIdx.z, SCAN_OPERANDS);
+}
+
+// The same beside the prompt attention of the layer (see PromptBeside): workgroups 0 .. scan_groups - 1 are the scan's, those
+// after them the attention's.  Heads of 64: one a workgroup of the attention, in 128 registers (two would take 191, and the
+// compute unit one workgroup of either kind: 18 us for 515 tokens, where the whole prompt gained nothing, 12 for 300); of 128
+// two, of which none fits beside another.  Which rows share a workgroup changes no sum.
+template <int NK, int PT, int DH, int NSET>
+__global__ void __launch_bounds__(SSD_SCAN_WAVES * WAVE, DH == 64 ? 4 : 2)
+ssd_chunk_scan_beside_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __restrict__ TT, int E,
+                             const bf16_t* __restrict__ state_in, const float* __restrict__ delta,
+                             const float* __restrict__ cum, const float* __restrict__ D,
+                             const int* __restrict__ chunks, int Q, int H, int G, float* __restrict__ y,
+                             long y_ld, const bf16_t* __restrict__ z, long z_ld, bf16_t* __restrict__ gated,
+                             long gated_ld, int n_chunks, int parts, int scan_groups, const PromptBeside beside) {
+  extern __shared__ __align__(16) unsigned char scan_smem[];
+  const int number = blockIdx.x;
+  if (number < scan_groups) {
+    ssd_chunk_scan_block<NK, PT>(scan_smem, number % n_chunks, number / n_chunks % H, parts - 1 - number / n_chunks / H, SCAN_OPERANDS);
+    return;
+  }
+  prompt_attention_beside<DH, NSET>(scan_smem, number - scan_groups, beside);
+}
+#undef SCAN_OPERANDS
 
 // ---------------------------------------------------------------- lanes of one chunk
 // Every lane of the step is one chunk of at most SSD_SINGLE_TOKENS tokens, so that a chunk starts from its request's state
@@ -1084,7 +1130,6 @@ ssd_single_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16_t* __r
 
 // The same beside the prompt attention of the layer (see PromptBeside): workgroups 0 .. scan_groups - 1 are the scan's, the
 // longer ones, and those after them the attention's, of as many threads; either uses the workgroup's LDS.
-static_assert(SSD_SCAN_WAVES == PREFILL_WAVES, "workgroups of one launch");
 // Heads that share their keys and states of 64 x 128 and more: two launches are the faster way at every such size, by what the
 // launches and the attention behind the scan cost.  37 tokens | 128 | five lanes of 16 behind 700 keys, four launches and two in us, 24 heads
 // of the scan: states of 64 x 128 beside 8 / 2 heads of 64 28.5, 19.2 | 33.8, 24.2 | 33.5, 19.0; 64 x 256 beside 6 / 2 of
@@ -1109,14 +1154,7 @@ ssd_single_beside_kernel(const bf16_t* __restrict__ xbc, long xbc_ld, const bf16
     read_ahead_block<SSD_SCAN_WAVES * WAVE>(ahead, blockIdx.x - ahead_from);
     return;
   }
-  const int index = blockIdx.x - scan_groups;
-  const int places = 4 * beside.n_tiles;
-  prefill_attention_block<DH, NSET>(scan_smem, index % places, places, index / places % beside.Hkv, index / places / beside.Hkv,
-                                    (const bf16_t*)beside.qkv, beside.ld, beside.Hq, beside.Hkv, (const bf16_t*)beside.k_base,
-                                    (const bf16_t*)beside.v_base, beside.page_stride, beside.page_size, beside.block_tables,
-                                    beside.max_pages, beside.tiles, beside.cu_seqlens, beside.start_pos, beside.scale,
-                                    beside.window, (bf16_t*)beside.out, beside.out_ld, nullptr, nullptr, DH, nullptr, nullptr, 0,
-                                    nullptr, nullptr, 0, DH);
+  prompt_attention_beside<DH, NSET>(scan_smem, blockIdx.x - scan_groups, beside);
 }
 
 static size_t ssd_single_lds_bytes(int P, int N) {
@@ -1186,8 +1224,8 @@ static int launch_ssd_single(dim3 grid, hipStream_t stream, const bf16_t* xbc, l
 }
 #undef SINGLE_ARGUMENTS
 
-// Whether mi_ssd_prefill takes the attention of such heads beside its second launch (of a step that mi_ssd_single covers,
-// whose H heads of the scan may have a group each): what it would refuse is refused here, before anything is launched.
+// Whether mi_ssd_prefill takes the attention of such heads beside its last launch (of a step that mi_ssd_single or, in chunks,
+// mi_ssd_staged covers, whose H heads of the scan may have a group each): what it would refuse is refused here, before anything is launched.
 extern "C" int mi_ssd_beside(int H, int P, int N, int Hq, int Hkv, int dh, int n_tiles, int max_seq_len) {
   if (H <= 0 || Hkv <= 0 || Hkv > 256 || Hq <= Hkv || Hq % Hkv != 0 || n_tiles <= 0 || n_tiles > (1 << 20) || (dh != 64 && dh != 128) ||
       !ssd_staged_sizes(P, N) || P < BESIDE_LEAST_P || N < BESIDE_LEAST_N)
@@ -1196,11 +1234,65 @@ extern "C" int mi_ssd_beside(int H, int P, int N, int Hq, int Hkv, int dh, int n
   // rows of the first launch, with a lane's tokens beside each chunk; workgroups of the second (a lane of one chunk has a tile)
   const long own_rows = H + ((long)H * (P + 2 * N) + 63) / 64;
   const long passes = (Hq / Hkv + nset - 1) / nset;
-  return own_rows + SSD_SINGLE_TOKENS <= 65535 && n_tiles * (2 * own_rows + 4 * Hkv * passes) <= 0x7fffffffL ? 1 : 0;
+  return own_rows + SSD_MAX_Q <= 65535 && n_tiles * (2 * own_rows + 4 * Hkv * passes) <= 0x7fffffffL ? 1 : 0;
 }
 
 static size_t ssd_scan_lds_bytes(int Q, int P, int N) {
   return (size_t)64 * (N + 8) * 2 + (size_t)P * (64 + 8) * 2 + (size_t)2 * Q * 4;
+}
+
+// Whether the scan of chunks of Q tokens stages its operands in LDS: it then takes an attention beside it too.
+extern "C" int mi_ssd_staged(int Q, int P, int N) { return ssd_staged_sizes(P, N) && ssd_scan_lds_bytes(Q, P, N) <= 64 * 1024 ? 1 : 0; }
+
+// query heads of a workgroup of the attention beside the scan of chunks (see there)
+static int scan_beside_heads(int dh) { return dh == 64 ? 1 : 2; }
+
+// Whether the attention of `tokens` tokens beside the scan of n_chunks chunks is faster than on a stream of its own, whose fork and
+// join cost about 12 us a layer: us a prompt on two streams | in one launch.
+// Heads of 64, two workgroups of the launch on a compute unit (0.5B shape): 144 tokens 2,952 | 2,671, 300 3,258 | 3,023, 515 3,570 |
+// 3,411, 700 3,662 | 3,545, 800 3,785 | 3,787, 900 4,230 | 4,161, four lanes of 200 4,122 | 3,992; 300 beside four tokens behind 6,000 keys
+// 5,750 | 4,805; 4,096 in portions of 256 56,100 | 49,300, of 512 30,690 | 30,100, of 1,024 18,280 | 19,120 (18,600 with the
+// first two alone).
+// Heads of 128, one on a compute unit (twelve layers of the 7B shape): 144 2,777 | 2,677, 256 3,190 | 3,102, 300 (216 workgroups)
+// 3,268 | 3,213, 400 (288) 3,702 | 3,710; 4,096 in portions of 256 51,570 | 52,090, 200 beside four tokens behind 4,000 keys (528)
+// 3,750 | 3,959.
+extern "C" int mi_ssd_chunks_beside(int Q, int H, int P, int N, int n_chunks, int tokens, int Hq, int Hkv, int dh, int n_tiles,
+                                    int max_seq_len) {
+  if (n_chunks <= 0 || !mi_ssd_staged(Q, P, N) || !mi_ssd_beside(H, P, N, Hq, Hkv, dh, n_tiles, max_seq_len)) return 0;
+  const int nset = scan_beside_heads(dh);
+  const long groups = (long)n_chunks * H * ((Q + 127) / 128) + 4L * n_tiles * Hkv * ((Hq / Hkv + nset - 1) / nset);
+  const bool near = max_seq_len > 0 && max_seq_len <= 2048;
+  return groups <= 0x7fffffffL && (dh == 64 ? tokens <= (near ? 896 : 640) : near && groups <= 256) ? 1 : 0;
+}
+
+template <int NK, int PT>
+static int launch_ssd_scan_beside(hipStream_t stream, const bf16_t* xbc, long xbc_ld, const bf16_t* TT, int E, const bf16_t* state_in,
+                                  const float* delta, const float* cum, const float* D, const int* chunks, int n_chunks, int Q,
+                                  int H, int G, float* y, long y_ld, const bf16_t* z, long z_ld, bf16_t* gated, long gated_ld,
+                                  const PromptBeside& beside) {
+  const int nset = scan_beside_heads(beside.dh);
+  if constexpr (32 * NK >= BESIDE_LEAST_N && 16 * PT >= BESIDE_LEAST_P) {
+    const size_t lds = ssd_scan_lds_bytes(Q, 16 * PT, 32 * NK);
+    const int parts = (Q + 127) / 128, passes = (beside.Hq / beside.Hkv + nset - 1) / nset;
+    const long scan_groups = (long)n_chunks * H * parts, all = scan_groups + 4L * beside.n_tiles * beside.Hkv * passes;
+    if (all > 0x7fffffffL) return ERR_UNSUPPORTED_SIZE;
+#define BESIDE_CASE(DH_, NSET_)                                                                                             \
+  if (beside.dh == DH_ && nset == NSET_) {                                                                                  \
+    static bool told[64] = {};                                                                                              \
+    const size_t most = ssd_scan_lds_bytes(SSD_MAX_Q, 16 * PT, 32 * NK);                                                    \
+    const size_t both = most > (size_t)prefill_lds_bytes(DH_) ? most : (size_t)prefill_lds_bytes(DH_);                      \
+    const int code = allow_lds(ssd_chunk_scan_beside_kernel<NK, PT, DH_, NSET_>, both, told);                               \
+    if (code) return code;                                                                                                  \
+    ssd_chunk_scan_beside_kernel<NK, PT, DH_, NSET_>                                                                        \
+        <<<(unsigned)all, SSD_SCAN_WAVES * WAVE, lds > (size_t)prefill_lds_bytes(DH_) ? lds : (size_t)prefill_lds_bytes(DH_), stream>>>( \
+            xbc, xbc_ld, TT, E, state_in, delta, cum, D, chunks, Q, H, G, y, y_ld, z, z_ld, gated, gated_ld, n_chunks, parts, \
+            (int)scan_groups, beside);                                                                                      \
+    return 0;                                                                                                               \
+  }
+    BESIDE_CASE(64, 1) BESIDE_CASE(128, 2)
+#undef BESIDE_CASE
+  }
+  return ERR_UNSUPPORTED_SIZE;
 }
 
 // Sizes: bfloat16; Q a multiple of 32 and at most 256; head_dim P a multiple of 16; state size N a
@@ -1212,7 +1304,7 @@ extern "C" int mi_ssd_supported(int Q, int P, int N, int G, int E) {
 }
 
 // beside: null, or the attention that reads the same step's rows (bfloat16, values as wide as the keys, a cache to write to
-// or none): needs the conv here and a step that mi_ssd_single and mi_ssd_beside cover.
+// or none): needs the conv here and a step that mi_ssd_single or mi_ssd_staged, and mi_ssd_beside, cover.
 extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long dt_ld, const float* dt_bias,
                               const float* A, const float* D, float* ssm_state, const int* chunks, int n_chunks,
                               const int* lane_chunks, const int* slot_ids, int n_lanes, int Q, int H, int P, int N,
@@ -1244,7 +1336,7 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
     if (!b.block_tables || b.max_pages <= 0 || !b.tiles || b.n_tiles <= 0 || !b.cu_seqlens || !b.start_pos || !b.out || !b.k_base ||
         !b.v_base || b.page_size <= 0)
       return ERR_BAD_ARGUMENT;
-    if (!mi_ssd_single(Q, P, N, longest, ssm_state) || !mi_ssd_beside(H, P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
+    if (!(mi_ssd_single(Q, P, N, longest, ssm_state) || mi_ssd_staged(Q, P, N)) || !mi_ssd_beside(H, P, N, b.Hq, b.Hkv, b.dh, b.n_tiles, b.max_seq_len) ||
         b.page_size % 4 != 0 || b.ld % 8 != 0 || b.out_ld % 4 != 0 || (uintptr_t)b.qkv % 16 != 0 || (uintptr_t)b.out % 8 != 0)
       return ERR_UNSUPPORTED_SIZE;
     nset = prefill_head_set(b.dh, b.Hq / b.Hkv, b.n_tiles, b.Hkv, b.max_seq_len);
@@ -1326,8 +1418,20 @@ extern "C" int mi_ssd_prefill(const void* xbc, long xbc_ld, const void* dt, long
 #undef PASS_CASE
     RETURN_IF_LAUNCH_FAILED();
   }
-  const bool staged = ssd_staged_sizes(P, N) && ssd_scan_lds_bytes(Q, P, N) <= 64 * 1024;
-  if (staged) {
+  if (beside) {
+    int status = ERR_UNSUPPORTED_SIZE;
+#define SCAN_BESIDE_CASE(NK_, PT_)                                                                                \
+  if (N == 32 * NK_ && P == 16 * PT_)                                                                             \
+    status = launch_ssd_scan_beside<NK_, PT_>(stream, (const bf16_t*)xbc, xbc_ld, (const bf16_t*)TT, E, (const bf16_t*)state_in, \
+                                              delta, cum, D, chunks, n_chunks, Q, H, G, y, y_ld, (const bf16_t*)z, z_ld, \
+                                              (bf16_t*)gated, gated_ld, *beside);
+    SCAN_BESIDE_CASE(4, 4) SCAN_BESIDE_CASE(4, 8) SCAN_BESIDE_CASE(8, 4) SCAN_BESIDE_CASE(8, 8)
+#undef SCAN_BESIDE_CASE
+    if (status != 0) return status;
+    RETURN_IF_LAUNCH_FAILED();
+    return 0;
+  }
+  if (mi_ssd_staged(Q, P, N)) {
     const dim3 grid(n_chunks, H, (Q + 127) / 128);
     const size_t lds = ssd_scan_lds_bytes(Q, P, N);
 #define SCAN_LDS_CASE(NK_, PT_)                                                                                   \

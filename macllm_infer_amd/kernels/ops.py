@@ -175,6 +175,7 @@ _SIGNATURES = {
                            _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr,
                            _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_long,
                            _c_ptr, _c_long, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr],
+        "mi_ssd_chunks_beside": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
         "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int, _c_ptr],
     },
     "rows_gemm": {
@@ -2212,10 +2213,10 @@ class PromptBeside:
     sizes: Optional[tuple]
     ahead: Sequence[torch.Tensor] = ()         # weights in fragment order that the launches behind read: see ``mixer_decode``
 
-    def fits(self, longest: int, ssm_state: torch.Tensor, chunk_size: int) -> bool:
-        """Whether ``ssd_prefill`` of a step with lanes of up to ``longest`` tokens takes this attention in its two
-        launches: lanes of one chunk, heads and states of the sizes it knows, and a step that ``prefill_attention`` gives
-        to the kernel whose waves read their keys themselves."""
+    def fits(self, longest: int, ssm_state: torch.Tensor, chunk_size: int, chunks: int = 0) -> bool:
+        """Whether ``ssd_prefill`` of a step with lanes of up to ``longest`` tokens takes this attention in its
+        launches: lanes of one chunk, or ``chunks`` of them in all where that pays (0: not asked for), heads and states of the sizes
+        it knows, and a step that ``prefill_attention`` gives to the kernel whose waves read their keys themselves."""
         q, out = self.qkv, self.out
         if not (q.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and q.dim() == 2 and q.stride(1) == 1 and q.stride(0) % 8 == 0
                 and q.data_ptr() % 16 == 0 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0):
@@ -2224,9 +2225,11 @@ class PromptBeside:
         if not prefill_attention_supported(q.dtype, self.num_heads, self.num_kv_heads, self.head_dim, page_size):
             return False
         _, H, P, N = ssm_state.shape
-        if not (_fn("ssd", "mi_ssd_single")(chunk_size, P, N, int(longest), _p(ssm_state))
-                and _fn("ssd", "mi_ssd_beside")(H, P, N, self.num_heads, self.num_kv_heads, self.head_dim,
-                                                self.query_tiles.shape[0], int(self.max_seq_len or 0))):
+        attention = (self.num_heads, self.num_kv_heads, self.head_dim, self.query_tiles.shape[0], int(self.max_seq_len or 0))
+        if _fn("ssd", "mi_ssd_single")(chunk_size, P, N, int(longest), _p(ssm_state)):
+            if not _fn("ssd", "mi_ssd_beside")(H, P, N, *attention):
+                return False
+        elif not _fn("ssd", "mi_ssd_chunks_beside")(chunk_size, H, P, N, int(chunks), q.shape[0], *attention):
             return False
         if not shared_prefill_covers(self.num_kv_heads, self.head_dim, page_size, self.k_cache.stride(0), self.k_cache.data_ptr(),
                                      self.v_cache.data_ptr()):

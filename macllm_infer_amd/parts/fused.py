@@ -438,7 +438,7 @@ def _measure_chain(chain, bucket: int) -> dict:
 
 
 class LayerFusion:
-    # Portions from this size on run their two mixers beside each other: where a lane may be longer than the chunk that the
+    # Portions from this size on, if they do not share launches, run their two mixers beside each other: where a lane may be longer than the chunk that the
     # state-space mixer's launches hold beside the attention's (us a prompt, beside | behind: 0.5B shape 144 tokens 2,971 | 3,109,
     # 200 3,071 | 3,213, 256 3,144 | 3,305; 7B shape 144 2,783 | 2,928)
     overlap_from = 129
@@ -705,8 +705,8 @@ class LayerFusion:
             self.mixers[index].mix(u[:, lo:hi], step, caches[self.names[index]], mixed[:, mixed_lo:mixed_hi])
 
     def _mix_side_by_side(self, u: torch.Tensor, step, caches, mixed: torch.Tensor, ahead=()) -> bool:
-        """Short portions: an attention mixer's launches inside those of a state-space mixer (False: nothing was done), which
-        bring the weights ``ahead`` into the caches."""
+        """Portions of up to several hundred tokens (``ops.PromptBeside.fits``): an attention mixer's launches inside those of a
+        state-space mixer (False: nothing was done), which bring the weights ``ahead`` into the caches where lanes are one chunk."""
         if len(self.mixers) != 2 or step.max_query_len == 1:
             return False
         first, second = self.mixers
@@ -769,6 +769,8 @@ class LayerFusion:
 
     def _general_mixers(self, u: torch.Tensor, step, caches) -> torch.Tensor:
         mixed = torch.empty((u.shape[0], self.mixed_width), dtype=u.dtype, device=u.device)
+        if self._mix_side_by_side(u, step, caches, mixed):
+            return mixed
         if overlap_pays(self.mixers, u.shape[0], u.device, self.overlap_from):
             # two mixers read the same rows and write different columns: the first runs on a second stream
             # beside the second (in a captured graph only: launched one by one the step waits for the host,

@@ -119,7 +119,7 @@ class Mamba2(Mixer):
         return (getattr(self.mix, "__func__", None) is Mamba2.mix and self.norm_weight is None
                 and self._chunked(u, step) and u.stride(0) % 4 == 0 and gated.stride(0) % 4 == 0
                 and ops.ssd_conv_supported(spec.conv_kernel, spec.conv_width, u[:, spec.inner_size:spec.inner_size + spec.conv_width])
-                and beside.fits(step.max_query_len, cache.states["ssm"], spec.chunk_size))
+                and beside.fits(step.max_query_len, cache.states["ssm"], spec.chunk_size, self._chunk_table(step).num_chunks))
 
     def mix(self, u: torch.Tensor, step, cache, gated: torch.Tensor, beside=None) -> None:
         """From the projected rows [z | x B C | dt] to the gated (and normed) scan output

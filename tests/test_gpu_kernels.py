@@ -2176,10 +2176,12 @@ def test_layer_norm_of_the_stream_and_its_branches(ops, dtype, T, d):
                                                   (5, 128, 256, 2, 1, 64), (2, 64, 128, 4, 2, 128), (3, 64, 256, 6, 2, 64),
                                                   (4, 128, 128, 10, 2, 64), (3, 64, 256, 12, 2, 128), (2, 128, 128, 4, 1, 64)])
 @pytest.mark.parametrize("counts, starts, window, longest", [([37], [0], None, 2048), ([1, 5, 128, 64], [0, 700, 0, 33], None, 4096),
-                                                             ([16] * 5, [3, 0, 950, 16, 690], 600, 2048)])
+                                                             ([16] * 5, [3, 0, 950, 16, 690], 600, 2048),
+                                                             ([129], [0], None, 2048), ([300, 1, 128], [0, 700, 33], None, 2048),
+                                                             ([256], [777], 600, 2048)])
 def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, window, longest):
-    """Lanes of one chunk of up to 128 tokens behind contexts: the rotation, the cache, the attended rows, the scan's outputs,
-    states and tails are the same bits in two launches and in four; a row of the table of runs that holds none."""
+    """Lanes of one chunk of up to 128 tokens, and of several, behind contexts: the rotation, the cache, the attended rows, the scan's outputs,
+    states and tails are the same bits in the scan's launches and in launches of their own; a row of the table of runs that holds none."""
     page_size, G, K, Q = 16, 1, 4, 128
     E, GN, T, lanes = H * P, G * N, sum(counts), len(counts)
     C, A_cols = E + 2 * GN, (Hq + 2 * Hkv) * dh
@@ -2217,7 +2219,7 @@ def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H
             ops.prefill_attention(qkv, Hq, Hkv, dh, *views(pages, page_size), block_table, beside.query_tiles, beside.cu_seqlens,
                                   beside.start_pos, 0.11, window, beside.out, longest, sizes=beside.sizes)
         else:
-            assert beside.fits(max(counts), s, Q)
+            assert beside.fits(max(counts), s, Q, table.num_chunks) and (max(counts) <= Q or not beside.fits(max(counts), s, Q))
         xbc = torch.empty(T, C, dtype=torch.bfloat16, device=DEV)
         ops.ssd_prefill(xbc, dt, dt_bias, A, D, s, table, slots, G, None, z=z, gated=mixed[:, Hq * dh:], longest=max(counts),
                         conv=dict(u=raw, weight=weight, bias=bias, state=t), beside=beside if together else None)
