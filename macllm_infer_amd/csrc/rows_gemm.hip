@@ -1,5 +1,5 @@
 // Products of many rows in bfloat16 on the matrix cores: out[M, N] = x[M, K] . W[N, K]^T (+ bias[N], float32), rounded once,
-// SiLU(gate) * up of a W whose rows lie in tiles of 8 gate rows and 8 up rows, or the float32 sums.
+// SiLU(gate) * up of the rounded results of a W whose rows lie in tiles of 8 gate rows and 8 up rows, or the float32 sums.
 //
 // A workgroup owns a tile of BM rows x BN features.  K is walked in stages of 64 columns, whole lines of 128 bytes of every
 // row, which go from memory to LDS without passing through registers (`buffer_load ... lds`), STAGES of them on their way;
@@ -230,7 +230,10 @@ rows_gemm_kernel(RowsGemm p) {
             b += p.bias[min(first + 16 + 4 * q + i, p.N - 1)];
           }
           const auto swapped = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
-          const float gate = __builtin_bit_cast(float, (unsigned)swapped[0]), up = __builtin_bit_cast(float, (unsigned)swapped[1]);
+          // (rounded as by a product of its own with the activation behind it: the same bits either way, for 0.3 us, 640 x 4,096 x
+          // 1,024 11.1 -> 11.4)
+          const float gate = (float)(bf16_t)__builtin_bit_cast(float, (unsigned)swapped[0]);
+          const float up = (float)(bf16_t)__builtin_bit_cast(float, (unsigned)swapped[1]);
           packed[i] = (bf16_t)(silu_bf16_f(gate) * up);
         }
         const int mine = first + 16 * (q / 2);               // the tile this lane has now (whole, as N is a multiple of 16)

@@ -476,7 +476,7 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor, tile: int = 0, activation: 
 def linear_swiglu(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                   bias16: Optional[torch.Tensor] = None) -> torch.Tensor:
     """SiLU(gate) * up of the product of many rows with a weight in tiles of 8 gate and 8 up rows (bfloat16): in the
-    product's launch where that pays, else behind it."""
+    product's launch where that pays, else behind it (of the same rounded numbers)."""
     M, K = x.shape
     N = weight.shape[0]
     if rows_gemm_pays(M, N, K, swiglu=True) and rows_gemm_supported(x, weight):
@@ -1492,7 +1492,7 @@ def rows_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
               keep_float32: bool = False, tile: int = -1, row_scale: Optional["RowScale"] = None) -> torch.Tensor:
     """x [M, K] . weight[N, K]^T (+ bias float32 [N]) of bfloat16 operands with float32 sums, [M, N] in bfloat16 or (``keep_float32``)
     float32; or (``swiglu``) SiLU(gate) * up [M, N / 2] of a weight whose rows are tiles of 8 gate and 8 up rows, the
-    activation on the float32 sums.  ``tile``: the kernel's tile (0 to 3; by its rule if negative).  ``row_scale``: a norm left
+    activation on the rounded results, as ``swiglu`` behind the product forms it.  ``tile``: the kernel's tile (0 to 3; by its rule if negative).  ``row_scale``: a norm left
     to the product (``rows_gemm_residual``): a row's sums are divided by its root mean square before the bias."""
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and rows_gemm_supported(x, weight)
           and not (swiglu and keep_float32), "rows_gemm: operands not covered")

@@ -50,13 +50,33 @@ def test_the_gated_activation_in_the_product(M, inner, K):
         sums = x.double() @ w.double().T + (0.0 if bias is None else bias.double())
         gate, up = sums.view(M, inner // 8, 2, 8).unbind(2)
         want = (gate * torch.sigmoid(gate) * up).reshape(M, inner)
-        # the sums' error e reaches the result by at most (1.1 |up| + |silu(gate)|) e, the activation adds four ulps
+        # the sums' error e and their rounding (2^-8 of either) reach the result by at most 1.1 |up| of the gate's and |silu(gate)| of the
+        # up half's, the activation adds four ulps
         e = float((x.double().abs() @ w.double().abs().T).max() * K * 2.0 ** -24 + 1e-6)
         most = float((1.1 * up.abs() + gate.abs()).max())
         for tile in (0, 1, 2, 3, -1):
             got = ops().rows_gemm(x.to(DEV), w.to(DEV), None if bias is None else bias.to(DEV), swiglu=True, tile=tile)
             assert got.shape == (M, inner)
-            assert bool(((got.cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + most * e).all()), tile
+            rounded = 2.0 ** -8 * (1.1 * up.abs() * gate.abs() + (gate * torch.sigmoid(gate)).abs() * up.abs()).reshape(M, inner)
+            assert bool(((got.cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + rounded * 1.01 + most * e).all()), tile
+
+
+@pytest.mark.parametrize("M, N, K", [(32, 128, 64), (33, 4096, 1024), (65, 80, 192), (130, 1040, 512), (515, 4096, 1024), (2048, 4096, 1024),
+                                     (600, 512, 2048)])
+def test_the_gated_activation_in_the_product_has_the_bits_of_a_launch_behind_it(M, N, K):
+    """Of this package's product, and of the library's, where that sums in k order too (64 features and more, K up to 1,024)."""
+    module = ops()
+    x, b = rand(M, K, seed=4).to(torch.bfloat16).to(DEV), rand(N, seed=6).to(DEV)
+    w = (rand(N, K, seed=5) * 2.0 / math.sqrt(K)).to(torch.bfloat16).to(DEV)
+    for bias in (None, b):
+        products = [module.rows_gemm(x, w, bias)]
+        if bias is None and K <= 1024:
+            products.append(torch.mm(x, w.t()))
+        got = [module.rows_gemm(x, w, bias, swiglu=True, tile=tile) for tile in (0, 1, 2, 3)] + [module.linear_swiglu(x, w, bias)]
+        for product in products:
+            behind = torch.empty(M, N // 2, dtype=torch.bfloat16, device=DEV)
+            module.swiglu(product, behind, 8)
+            assert all(torch.equal(one, behind) for one in got)
 
 
 @pytest.mark.parametrize("M, N, K", [(1, 16, 64), (64, 64, 128), (65, 80, 192), (130, 1040, 64), (300, 128, 320), (129, 272, 1024)])
@@ -88,7 +108,8 @@ def test_a_norm_left_to_the_products_around_it(M, N, K):
             want_act = (gate * torch.sigmoid(gate) * up).reshape(M, 40)
             act = module.rows_gemm(rows, behind.to(DEV), swiglu=True, row_scale=scale, tile=tile).cpu().double()
             most = float((1.1 * up.abs() + gate.abs()).max() * slack.max() + 1e-6)
-            assert bool(((act - want_act).abs() <= 2.0 ** -8 * want_act.abs() + most).all()), tile
+            rounded = 2.0 ** -8 * (1.1 * up.abs() * gate.abs() + (gate * torch.sigmoid(gate)).abs() * up.abs()).reshape(M, 40)
+            assert bool(((act - want_act).abs() <= 2.0 ** -8 * want_act.abs() + rounded * 1.01 + most).all()), tile
 
 
 def test_rows_of_a_wider_matrix_infinities_and_what_is_refused():
