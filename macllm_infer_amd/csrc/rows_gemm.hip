@@ -27,7 +27,6 @@ typedef __attribute__((address_space(3))) void g_lds;
 #define EPI_ROWS_PLAIN 0
 #define EPI_ROWS_SWIGLU 1
 #define EPI_ROWS_F32 2               // the sums as they are
-#define EPI_ROWS_RESIDUAL 3          // added to the residual stream, with what the product behind the next norm needs
 
 struct RowsGemm {
   const bf16_t* x;
@@ -38,17 +37,6 @@ struct RowsGemm {
   long ldo;
   int M, N, K, tiles_m, tiles_n;
   int whole;                         // four neighbouring outputs are one aligned piece
-  // A norm before the product, left to it: x are the stream's rows times the norm's weight, and a row's sums are multiplied by
-  // 1 / sqrt(sum of squares / scale_width + scale_eps); its sum of squares is the sum of scale_parts numbers scale_ld apart.
-  const float* scale;                // or null
-  int scale_parts;
-  long scale_ld;
-  float scale_width, scale_eps;
-  // EPI_ROWS_RESIDUAL: h [M, N] += the product; out = h * next_weight; squares[feature / 16, row] the sum of squares of 16 of h
-  float* h;
-  const float* next_weight;
-  float* squares;
-  long squares_ld;
 };
 
 template <int BM, int BN, int WM, int WN, int STAGES, bool AHEAD, int EPI>
@@ -129,15 +117,6 @@ rows_gemm_kernel(RowsGemm p) {
   };
 #pragma unroll
   for (int stage = 0; stage < STAGES; ++stage) ask(stage);
-  // a share of a row's sum of squares, GROUPS threads a row, behind the first stages' loads (it waits in a register: a second
-  // array in LDS would make the compiler wait for every load to LDS before a read of it)
-  constexpr int GROUPS = WAVE * WAVES / BM;
-  float share = 0.f;
-  if (p.scale) {
-    const float* const parts = p.scale + min(m0 + (int)threadIdx.x % BM, p.M - 1);
-#pragma unroll 8
-    for (int part = threadIdx.x / BM; part < p.scale_parts; part += GROUPS) share += parts[part * p.scale_ld];
-  }
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * LOADS) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -194,22 +173,6 @@ rows_gemm_kernel(RowsGemm p) {
   }
   // nothing of the stages past the end may still be on its way to LDS when the workgroup ends
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  float factor[TM];
-#pragma unroll
-  for (int m = 0; m < TM; ++m) factor[m] = 1.f;
-  if (p.scale) {
-    float* const shares = reinterpret_cast<float*>(&lds[0][0]);
-    __syncthreads();                                         // every stage has arrived and is read
-    shares[threadIdx.x] = share;
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < TM; ++m) {
-      float sum = 0.f;
-#pragma unroll
-      for (int group = 0; group < GROUPS; ++group) sum += shares[group * BM + (wm * TM + m) * 16 + r];
-      factor[m] = 1.0f / sqrtf(sum / p.scale_width + p.scale_eps);
-    }
-  }
   // a lane holds four neighbouring features (4 q ..) of row r of every tile
 #pragma unroll
   for (int m = 0; m < TM; ++m) {
@@ -224,7 +187,7 @@ rows_gemm_kernel(RowsGemm p) {
         g_bf16x4 packed;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float a = acc[n][m][i] * factor[m], b = acc[n + 1][m][i] * factor[m];
+          float a = acc[n][m][i], b = acc[n + 1][m][i];
           if (p.bias) {
             a += p.bias[min(first + 4 * q + i, p.N - 1)];
             b += p.bias[min(first + 16 + 4 * q + i, p.N - 1)];
@@ -244,32 +207,9 @@ rows_gemm_kernel(RowsGemm p) {
       for (int n = 0; n < TN; ++n) {
         const int feature = n0 + (wn * TN + n) * 16 + 4 * q;
         g_floatx4 value = acc[n][m];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) value[i] *= factor[m];
         if (p.bias) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) value[i] += p.bias[min(feature + i, p.N - 1)];
-        }
-        if (EPI == EPI_ROWS_RESIDUAL) {
-          const bool there = row < p.M && feature < p.N;     // (N is a multiple of 16: four features or none)
-          const int column = min(feature, p.N - 4);
-          float* const h = p.h + min(row, (long)p.M - 1) * p.N + column;
-          value += *reinterpret_cast<const g_floatx4*>(h);
-          const g_floatx4 weight = *reinterpret_cast<const g_floatx4*>(p.next_weight + column);
-          g_bf16x4 packed;
-          float squares = 0.f;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            packed[i] = (bf16_t)(value[i] * weight[i]);
-            squares = fmaf(value[i], value[i], squares);
-          }
-          squares += __shfl_xor(squares, 16, WAVE);
-          squares += __shfl_xor(squares, 32, WAVE);
-          if (!there) continue;
-          *reinterpret_cast<g_floatx4*>(h) = value;
-          *reinterpret_cast<g_bf16x4*>(out + feature) = packed;
-          if (q == 0) p.squares[feature / 16 * p.squares_ld + row] = squares;
-          continue;
         }
         if (row >= p.M) continue;
         if (EPI == EPI_ROWS_F32) {
@@ -305,7 +245,6 @@ static void launch_rows_gemm(RowsGemm p, int epilogue, hipStream_t stream) {
   p.tiles_n = (p.N + BN - 1) / BN;
   const int per_die = (int)(((long)p.tiles_m * p.tiles_n + 7) / 8);
   if (epilogue == EPI_ROWS_SWIGLU) rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_SWIGLU><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
-  else if (epilogue == EPI_ROWS_RESIDUAL) rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_RESIDUAL><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
   else if (epilogue == EPI_ROWS_F32) rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_F32><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
   else rows_gemm_kernel<BM, BN, WM, WN, STAGES, AHEAD, EPI_ROWS_PLAIN><<<8 * per_die, WAVE * WM * WN, 0, stream>>>(p);
 }
@@ -327,20 +266,20 @@ static int rows_gemm_tile(int M, int N, int K) {
   return best;
 }
 
-static int run_rows_gemm(RowsGemm p, int epilogue, int tile, long ldx, long ldw, hipStream_t stream) {
-  if (!p.x || !p.w || !p.out || p.M <= 0 || p.N <= 0 || p.K <= 0 || ldx < p.K || ldw < p.K || tile < -1 || tile > 3 ||
-      p.ldo < (epilogue == EPI_ROWS_SWIGLU ? p.N / 2 : p.N) ||
-      (p.scale && (p.scale_parts <= 0 || p.scale_ld < p.M || !(p.scale_width > 0.f))))
+// K a multiple of 64; rows of x and W start at 16 bytes.  epilogue 1: N features in tiles of 8 gate and 8 up rows, out
+// [M, N / 2] bfloat16; 2: out float32.  tile: 0 .. 3, or -1 for the rule's choice.
+extern "C" int mi_rows_gemm(const void* x, long ldx, const void* w, long ldw, const float* bias, void* out, long ldo, int M,
+                            int N, int K, int epilogue, int tile, hipStream_t stream) {
+  const bool swiglu = epilogue == EPI_ROWS_SWIGLU;
+  if (!x || !w || !out || M <= 0 || N <= 0 || K <= 0 || ldx < K || ldw < K || ldo < (swiglu ? N / 2 : N) || tile < -1 || tile > 3 || epilogue < 0 ||
+      epilogue > EPI_ROWS_F32)
     return ERR_BAD_ARGUMENT;
-  const long results = epilogue == EPI_ROWS_F32 ? 16 : 8;
-  if (p.K % GEMM_STAGE || ldx % 8 || ldw % 8 || (uintptr_t)p.x % 16 || (uintptr_t)p.w % 16 || ldx > (1 << 22) || ldw > (1 << 22) ||
-      (long)(p.M / 64 + 1) * (p.N / 64 + 1) > (1 << 28) ||
-      ((epilogue == EPI_ROWS_SWIGLU || epilogue == EPI_ROWS_RESIDUAL) && (p.N % 16 || p.ldo % 4 || (uintptr_t)p.out % 8)))
+  if (K % GEMM_STAGE || ldx % 8 || ldw % 8 || (uintptr_t)x % 16 || (uintptr_t)w % 16 || ldx > (1 << 22) || ldw > (1 << 22) ||
+      (long)(M / 64 + 1) * (N / 64 + 1) > (1 << 28) || (swiglu && (N % 16 || ldo % 4 || (uintptr_t)out % 8)))
     return ERR_UNSUPPORTED_SIZE;
-  p.ldx = (int)ldx;
-  p.ldw = (int)ldw;
-  p.whole = p.ldo % 4 == 0 && (uintptr_t)p.out % results == 0;
-  switch (tile < 0 ? rows_gemm_tile(p.M, p.N, p.K) : tile) {
+  RowsGemm p = {(const bf16_t*)x, (const bf16_t*)w, bias, out, (int)ldx, (int)ldw, ldo, M, N, K, 0, 0,
+                ldo % 4 == 0 && (uintptr_t)out % (epilogue == EPI_ROWS_F32 ? 16 : 8) == 0};
+  switch (tile < 0 ? rows_gemm_tile(M, N, K) : tile) {
     case 0: launch_rows_gemm<64, 64, 4, 2, 4, true>(p, epilogue, stream); break;
     case 1: launch_rows_gemm<64, 128, 2, 4, 3, true>(p, epilogue, stream); break;
     case 2: launch_rows_gemm<128, 128, 2, 4, 4, false>(p, epilogue, stream); break;
@@ -348,51 +287,4 @@ static int run_rows_gemm(RowsGemm p, int epilogue, int tile, long ldx, long ldw,
   }
   RETURN_IF_LAUNCH_FAILED();
   return 0;
-}
-
-// K a multiple of 64; rows of x and W start at 16 bytes.  epilogue 1: N features in tiles of 8 gate and 8 up rows, out
-// [M, N / 2] bfloat16; 2: out float32.  scale (or null): the sums of squares of a norm left to the product (RowsGemm).  tile:
-// 0 .. 3, or -1 for the rule's choice.
-extern "C" int mi_rows_gemm(const void* x, long ldx, const void* w, long ldw, const float* bias, void* out, long ldo, int M,
-                            int N, int K, int epilogue, const float* scale, int scale_parts, long scale_ld, int scale_width,
-                            float scale_eps, int tile, hipStream_t stream) {
-  if (epilogue < 0 || epilogue > EPI_ROWS_F32) return ERR_BAD_ARGUMENT;
-  RowsGemm p = {};
-  p.x = (const bf16_t*)x;
-  p.w = (const bf16_t*)w;
-  p.bias = bias;
-  p.out = out;
-  p.ldo = ldo;
-  p.M = M;
-  p.N = N;
-  p.K = K;
-  p.scale = scale;
-  p.scale_parts = scale_parts;
-  p.scale_ld = scale_ld;
-  p.scale_width = (float)scale_width;
-  p.scale_eps = scale_eps;
-  return run_rows_gemm(p, epilogue, tile, ldx, ldw, stream);
-}
-
-// h [M, N] float32 += x . W^T (+ bias); rows [M, N] bfloat16 = h * next_weight; squares [N / 16, squares_ld] the sums of squares of
-// h over every 16 features.  N a multiple of 16.
-extern "C" int mi_rows_gemm_residual(const void* x, long ldx, const void* w, long ldw, const float* bias, int M, int N, int K,
-                                     float* h, void* rows, long rows_ld, const float* next_weight, float* squares,
-                                     long squares_ld, int tile, hipStream_t stream) {
-  if (!h || !next_weight || !squares || squares_ld < M) return ERR_BAD_ARGUMENT;
-  if ((uintptr_t)h % 16 || (uintptr_t)next_weight % 16) return ERR_UNSUPPORTED_SIZE;
-  RowsGemm p = {};
-  p.x = (const bf16_t*)x;
-  p.w = (const bf16_t*)w;
-  p.bias = bias;
-  p.out = rows;
-  p.ldo = rows_ld;
-  p.M = M;
-  p.N = N;
-  p.K = K;
-  p.h = h;
-  p.next_weight = next_weight;
-  p.squares = squares;
-  p.squares_ld = squares_ld;
-  return run_rows_gemm(p, EPI_ROWS_RESIDUAL, tile, ldx, ldw, stream);
 }

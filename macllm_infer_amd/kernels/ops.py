@@ -179,10 +179,8 @@ _SIGNATURES = {
         "mi_ssd_single": [_c_int, _c_int, _c_int, _c_int, _c_ptr],
     },
     "rows_gemm": {
-        "mi_rows_gemm": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_ptr,
-                         _c_int, _c_long, _c_int, _c_float, _c_int, _c_ptr],
-        "mi_rows_gemm_residual": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_long,
-                                  _c_ptr, _c_ptr, _c_long, _c_int, _c_ptr],
+        "mi_rows_gemm": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_int, _c_int,
+                         _c_ptr],
     },
     "gemm": {
         "mi_gemm_f32": [_c_ptr, _c_long, _c_ptr, _c_long, _c_ptr, _c_ptr, _c_long, _c_int, _c_int, _c_int, _c_ptr],
@@ -1483,17 +1481,12 @@ def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False, keep_float32: b
     return K <= 2048 and small and M >= 512 and M * N >= 1 << 19
 
 
-def rows_gemm_fits_once(M: int, N: int) -> bool:
-    """Whether tiles of 128 rows by 128 features fit the compute units once."""
-    return -(-M // 128) * -(-N // 128) <= GEMM_UNITS
-
-
 def rows_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, *, swiglu: bool = False,
-              keep_float32: bool = False, tile: int = -1, row_scale: Optional["RowScale"] = None) -> torch.Tensor:
+              keep_float32: bool = False, tile: int = -1) -> torch.Tensor:
     """x [M, K] . weight[N, K]^T (+ bias float32 [N]) of bfloat16 operands with float32 sums, [M, N] in bfloat16 or (``keep_float32``)
     float32; or (``swiglu``) SiLU(gate) * up [M, N / 2] of a weight whose rows are tiles of 8 gate and 8 up rows, the
-    activation on the rounded results, as ``swiglu`` behind the product forms it.  ``tile``: the kernel's tile (0 to 3; by its rule if negative).  ``row_scale``: a norm left
-    to the product (``rows_gemm_residual``): a row's sums are divided by its root mean square before the bias."""
+    activation on the rounded results, as ``swiglu`` behind the product forms it.  ``tile``: the kernel's tile (0 to 3; by its
+    rule if negative)."""
     _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1] and rows_gemm_supported(x, weight)
           and not (swiglu and keep_float32), "rows_gemm: operands not covered")
     M, K = x.shape
@@ -1505,34 +1498,8 @@ def rows_gemm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
     out = torch.empty((M, width), dtype=torch.float32 if keep_float32 else torch.bfloat16, device=x.device)
     _check(_fn("rows_gemm", "mi_rows_gemm")(
         _p(x), _row_major(x, "x"), _p(weight), _row_major(weight, "weight"), _p(bias), _p(out), width, M, N, K,
-        1 if swiglu else 2 if keep_float32 else 0, *_row_scale_arguments(row_scale, M, K), int(tile), _stream()),
-        "rows_gemm", f"(M={M}, N={N}, K={K})")
+        1 if swiglu else 2 if keep_float32 else 0, int(tile), _stream()), "rows_gemm", f"(M={M}, N={N}, K={K})")
     return out
-
-
-def _row_scale_arguments(row_scale: Optional["RowScale"], M: int, K: int) -> list:
-    if row_scale is None:
-        return [None, 0, 0, 0, 0.0]
-    ssq = row_scale.ssq
-    _need(ssq.dtype == torch.float32 and ssq.dim() == 2 and ssq.is_contiguous() and ssq.is_cuda and ssq.shape[1] >= M
-          and row_scale.width == K, "rows_gemm: the row scale does not fit the rows")
-    return [_p(ssq), ssq.shape[0], ssq.shape[1], K, float(row_scale.eps)]
-
-
-def rows_gemm_residual(weight: torch.Tensor, bias: Optional[torch.Tensor], x: torch.Tensor, h: torch.Tensor,
-                       rows: torch.Tensor, next_weight: torch.Tensor, ssq: torch.Tensor, tile: int = -1) -> None:
-    """``fused_gemm_residual`` of any number of rows: h [M, N] float32 += x . weight^T (+ bias) in place, with the new rows times
-    the next norm's weight in bfloat16 (``rows``) and the sums of squares of the new rows over every 16 features (``ssq``, of
-    ``residual_workspace``) beside it, for a product with ``row_scale``.  N a multiple of 16."""
-    M, K = x.shape
-    N = weight.shape[0]
-    _need(rows_gemm_supported(x, weight) and weight.shape[1] == K and N % 16 == 0, "rows_gemm_residual: operands not covered")
-    _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == N and bias.is_contiguous()),
-          "rows_gemm_residual: bias must be float32 [N]")
-    rows_ld = _residual_arguments(h, rows, next_weight, ssq, M, N, "rows_gemm_residual")
-    _check(_fn("rows_gemm", "mi_rows_gemm_residual")(
-        _p(x), _row_major(x, "x"), _p(weight), _row_major(weight, "weight"), _p(bias), M, N, K, _p(h), _p(rows), rows_ld,
-        _p(next_weight), _p(ssq), ssq.shape[1], int(tile), _stream()), "rows_gemm_residual", f"(M={M}, N={N}, K={K})")
 
 
 SKINNY_ROWS = 16          # steps of up to this many rows take the skinny kernel in ``linear``

@@ -158,10 +158,6 @@ CHAIN_MARGIN = 0.97
 # the product (the general one adds a row's partial sums of squares in another order).  A plan's number: 1 = every workgroup all rows,
 # 2 = over two workgroups, 4 = one tile of 16 rows each.
 ROW_TILES_FEATURES = 2048
-# Prompt portions leave their norms to the products too, where all four are of K up to this and fit the compute units once
-# (``LayerFusion._leaves_norms``)
-ROWS_NORM_WIDTH = 2048
-FORCE_ROWS_NORM: Optional[bool] = None    # tests: True or False instead of that rule
 FORCE_ROW_TILES: Optional[int] = None     # tests: this number for all four projections instead of the rule and the clock
 PLAN_FIELDS = ("library_in", "library_out", "library_gate_up", "library_down", "split_out", "split_down",
                "tiles_in", "tiles_out", "tiles_gate_up", "tiles_down", "deferred",
@@ -524,13 +520,6 @@ class LayerFusion:
         # the same two norms for the products that take them as a row scale (any width)
         self.mixer_scale = _rms_prologue(block.mixer_norm) if self.decode_ok else None
         self.ffn_scale = _rms_prologue(block.ffn_norm) if self.decode_ok else None
-        # the features of a prompt portion's four products, where they can leave the norms to each other
-        self.rows_products = None
-        if (self.gate_up is not None and self.general and self.mixer_scale is not None and self.ffn_scale is not None
-                and self.hidden % 64 == 0 and self.mixed_width % 64 == 0 and self.inner % 64 == 0
-                and max(self.hidden, self.mixed_width, self.inner) <= ROWS_NORM_WIDTH
-                and self.w_in.dtype == self.w_out.dtype == torch.bfloat16):
-            self.rows_products = (self.in_width, self.hidden, 2 * self.inner, self.hidden)
         # a kernel for this set of mixers, if one is registered and takes these sizes
         factory = _MIXER_KERNELS.get(tuple(getattr(mixer, "kind", None) for mixer in self.mixers))
         self.kernel = factory(self) if factory is not None and self.decode_ok else None
@@ -722,50 +711,16 @@ class LayerFusion:
         second.mix(*rows[1], beside=beside)
         return True
 
-    def _leaves_norms(self, rows: int) -> bool:
-        """Whether a prompt portion of this many rows leaves its norms to the products around them, as small steps do: the two
-        that feed the stream add to it and leave the next norm's rows, those behind them divide.  Two launches of 5 us a layer
-        less where each of the four products is this package's own anyway or as fast as the library's (``ops.rows_gemm``:
-        128 x 128 tiles that fit the compute units once)."""
-        if FORCE_ROWS_NORM is False or self.rows_products is None:
-            return False
-        return bool(FORCE_ROWS_NORM) or all(ops.rows_gemm_fits_once(rows, N) for N in self.rows_products)
-
     def forward_general(self, residual: Residual, step, caches) -> None:
         block = self.block
-        rows = step.num_tokens
-        leaves = self._leaves_norms(rows)
-        scaled = residual.scaled
-        if (leaves and scaled is not None and scaled.weight is self.mixer_scale[0] and not residual.pending):
-            u = ops.rows_gemm(scaled.rows, self.w_in, self.b_in,
-                              row_scale=ops.RowScale(scaled.ssq, self.hidden, self.mixer_scale[1]))
-        else:
-            u = self._general_input(block.mixer_norm.forward(residual))
-        mixed = self._general_mixers(u, step, caches)
-        if not leaves or residual.pending:
-            residual.pending = [ops.linear(mixed, self.w_out, self.b_out)]
-            normed = block.ffn_norm.forward(residual)
-            residual.pending = [block.ffn.forward(normed)]
-            return
-        self._rows_to_the_stream(residual, mixed, self.w_out, self.b_out, self.ffn_scale[0])
-        activated = ops.rows_gemm(residual.scaled.rows, self.gate_up.weight, self.gate_up.bias, swiglu=True,
-                                  row_scale=ops.RowScale(residual.scaled.ssq, self.hidden, self.ffn_scale[1]))
-        if residual.next_norm is not None:
-            self._rows_to_the_stream(residual, activated, self.down.weight, self.down.bias, residual.next_norm[0])
-        else:
-            residual.pending = [self.down(activated)]
-
-    def _rows_to_the_stream(self, residual: Residual, x, weight, bias, next_weight) -> None:
-        """``_add_to_the_stream`` of a prompt portion's rows."""
-        rows = torch.empty((x.shape[0], self.hidden), dtype=torch.bfloat16, device=x.device)
-        ssq = ops.residual_workspace(x.shape[0], self.hidden, x.device)
-        ops.rows_gemm_residual(weight, bias, x, residual.h, rows, next_weight, ssq)
-        residual.scaled = ScaledRows(rows, ssq, next_weight)
-
-    def _general_input(self, normed: torch.Tensor) -> torch.Tensor:
+        normed = block.mixer_norm.forward(residual)
         if self.padding_pays[_portion_bucket(normed.shape[0])]:
-            return ops.linear(normed, self.w_in_wide, self.b_in_wide)
-        return ops.linear(normed, self.w_in, self.b_in)
+            u = ops.linear(normed, self.w_in_wide, self.b_in_wide)
+        else:
+            u = ops.linear(normed, self.w_in, self.b_in)
+        residual.pending = [ops.linear(self._general_mixers(u, step, caches), self.w_out, self.b_out)]
+        normed = block.ffn_norm.forward(residual)
+        residual.pending = [block.ffn.forward(normed)]
 
     def _general_mixers(self, u: torch.Tensor, step, caches) -> torch.Tensor:
         mixed = torch.empty((u.shape[0], self.mixed_width), dtype=u.dtype, device=u.device)

@@ -1380,6 +1380,63 @@ def test_long_portions_overlap_their_mixers(tmp_path, name):
     assert engine.graphs.counts["bucket_replays"] >= 5
 
 
+def shared_launches_config(chunk=128):
+    """Heads and states of the sizes at which the two mixers of a portion share launches, in widths of whole stages of 64."""
+    return dict(tiny_configs.TINY_C, hidden_size=256, num_hidden_layers=3, intermediate_size=320, mamba_n_heads=8, mamba_d_head=64,
+                mamba_d_ssm=512, mamba_d_state=128, mamba_chunk_size=chunk, max_position_embeddings=2048)
+
+
+@pytest.mark.parametrize("counts, chunk", [([65], 128), ([300, 5], 128), ([129, 150, 1], 128), ([600], 256)])
+def test_portions_have_the_bits_of_the_launches_that_theirs_replace(tmp_path, monkeypatch, counts, chunk):
+    """A layer's own products with the activation inside and its mixers in shared launches give what the library's products, the
+    activation and the mixers in launches of their own give, bit for bit, launched kernel by kernel and from the graph of the
+    step's capacity (padding lanes and rows among its); the former against the plain model too."""
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.kernels import ops
+    from macllm_infer_amd.weights.random_init import write_random_model
+    raw = shared_launches_config(chunk)
+    folder = write_random_model(FalconH1Config.from_dict(raw), 5, str(tmp_path), torch.bfloat16, "unit")
+    cfg, tensors = plain_impl.load_model_dir(folder)
+    places = lambda some: sorted({0, (len(some) - 1) // 2, len(some) - 2})       # of all tokens but the last
+    longer, products = [], []
+    fits, product = ops.PromptBeside.fits, ops.rows_gemm
+
+    def run(apart):
+        monkeypatch.setattr(ops.PromptBeside, "fits", lambda self, longest, *rest: not apart and fits(self, longest, *rest)
+                            and (longer.append(longest) or True))
+        monkeypatch.setattr(ops, "rows_gemm_pays", (lambda *sizes, **how: False) if apart else pays)
+        monkeypatch.setattr(ops, "rows_gemm", lambda *operands, **how: products.append(how.get("swiglu", False)) or product(*operands, **how))
+        engine = Engine(folder, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=4096,
+                        max_active_sequences=8, measured_paths=False)
+        out = []
+        for turn in range(4):
+            tokens = [tokens_for(cfg["vocab_size"], count + 1, 50 * turn + index) for index, count in enumerate(counts)]
+            for index in range(len(counts)):
+                engine.add_request(f"{turn}-{index}")
+            lanes = [Lane(f"{turn}-{index}", some[:-1], places(some)) for index, some in enumerate(tokens)]
+            rows = engine.step(lanes).float().cpu()
+            rows = torch.cat([rows, engine.step([Lane(f"{turn}-{index}", some[-1:], [0]) for index, some in enumerate(tokens)]).float().cpu()])
+            out.append((tokens, rows))
+            for index in range(len(counts)):
+                engine.finish(f"{turn}-{index}")
+        assert engine.graphs.counts["bucket_replays"] >= 1 and engine.model.blocks[0].fusion.general
+        return out
+
+    pays = ops.rows_gemm_pays
+    together = run(False)
+    assert max(longer) >= max(counts) and {True, False} <= set(products)
+    del longer[:], products[:]
+    apart = run(True)
+    assert not longer and not products
+    for (tokens, ours), (_, theirs) in zip(together, apart):
+        assert torch.equal(ours, theirs)
+        want = [plain_impl.falcon_h1_logits(cfg, tensors, some) for some in tokens]
+        want = torch.cat([torch.cat([one[places(some)] for one, some in zip(want, tokens)]),
+                          torch.cat([one[-1:] for one in want])])
+        assert (ours - want).abs().max().item() <= 6e-2 * want.abs().max().item()
+
+
 @pytest.mark.parametrize("name, dtype", [("A", "float32"), ("D", "bfloat16")])
 @pytest.mark.parametrize("count", [40, 130])
 def test_single_tokens_beside_portions_give_the_bits_of_one_batch_behind_the_other(tmp_path, monkeypatch, name, dtype, count):

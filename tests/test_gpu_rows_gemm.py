@@ -79,39 +79,6 @@ def test_the_gated_activation_in_the_product_has_the_bits_of_a_launch_behind_it(
             assert all(torch.equal(one, behind) for one in got)
 
 
-@pytest.mark.parametrize("M, N, K", [(1, 16, 64), (64, 64, 128), (65, 80, 192), (130, 1040, 64), (300, 128, 320), (129, 272, 1024)])
-def test_a_norm_left_to_the_products_around_it(M, N, K):
-    """h += the product, the rows times the next norm's weight, and the product behind them divided by the root mean square."""
-    module = ops()
-    x, w, b = rand(M, K, seed=1).to(torch.bfloat16), (rand(N, K, seed=2) / math.sqrt(K)).to(torch.bfloat16), rand(N, seed=3)
-    h, weight = rand(M, N, seed=4) * 3.0, rand(N, seed=5) * 0.1 + 1.0
-    behind = (rand(80, 64 * -(-N // 64), seed=6)[:, :N] / math.sqrt(N)).to(torch.bfloat16)
-    want = h.double() + x.double() @ w.double().T + b.double()
-    error = bound(x, w, want * 0.0) + 2.0 ** -22 * want.abs()
-    for tile in (0, 1, 2, 3, -1):
-        got, rows = h.clone().to(DEV), torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
-        ssq = module.residual_workspace(M, N, DEV)
-        module.rows_gemm_residual(w.to(DEV), b.to(DEV), x.to(DEV), got, rows, weight.to(DEV), ssq, tile=tile)
-        assert bool(((got.cpu().double() - want).abs() <= error).all()), tile
-        new = got.cpu().double()
-        assert bool(((rows.cpu().double() - new * weight.double()).abs() <= 2.0 ** -8 * (new * weight.double()).abs() + 1e-30).all())
-        squares = ssq.cpu().double().sum(0)[:M]
-        assert torch.allclose(squares, new.pow(2).sum(-1), rtol=N * 2.0 ** -23)
-        if N % 64 == 0:
-            scale = module.RowScale(ssq, N, 1e-5)
-            factor = 1.0 / torch.sqrt(new.pow(2).mean(-1, keepdim=True) + 1e-5)
-            sums = (rows.cpu().double() @ behind.double().T) * factor
-            out = module.rows_gemm(rows, behind.to(DEV), row_scale=scale, tile=tile).cpu().double()
-            slack = bound(rows.cpu(), behind, sums * 0.0) * factor + 2.0 ** -20 * sums.abs()
-            assert bool(((out - sums).abs() <= slack + 2.0 ** -8 * sums.abs()).all()), tile
-            gate, up = sums.view(M, 5, 2, 8).unbind(2)
-            want_act = (gate * torch.sigmoid(gate) * up).reshape(M, 40)
-            act = module.rows_gemm(rows, behind.to(DEV), swiglu=True, row_scale=scale, tile=tile).cpu().double()
-            most = float((1.1 * up.abs() + gate.abs()).max() * slack.max() + 1e-6)
-            rounded = 2.0 ** -8 * (1.1 * up.abs() * gate.abs() + (gate * torch.sigmoid(gate)).abs() * up.abs()).reshape(M, 40)
-            assert bool(((act - want_act).abs() <= 2.0 ** -8 * want_act.abs() + rounded * 1.01 + most).all()), tile
-
-
 def test_rows_of_a_wider_matrix_infinities_and_what_is_refused():
     module = ops()
     wide = rand(70, 200, seed=7).to(torch.bfloat16).to(DEV)
