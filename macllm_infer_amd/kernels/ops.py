@@ -1438,9 +1438,11 @@ GEMM_UNITS = 256          # compute units
 
 
 def rows_gemm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether ``rows_gemm`` takes these operands."""
+    """Whether ``rows_gemm`` takes these operands (rows behind each other: none that overlap, as expanded ones do)."""
+    K = x.shape[1]
     return (x.is_cuda and weight.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-            and x.shape[1] % 64 == 0 and x.shape[0] > 0 and x.stride(1) == 1 and weight.stride(1) == 1
+            and K > 0 and K % 64 == 0 and x.shape[0] > 0 and weight.shape[0] > 0 and x.stride(1) == 1 and weight.stride(1) == 1
+            and (x.shape[0] == 1 or x.stride(0) >= K) and (weight.shape[0] == 1 or weight.stride(0) >= K)
             and x.stride(0) % 8 == 0 and weight.stride(0) % 8 == 0 and max(x.stride(0), weight.stride(0)) <= 1 << 22
             and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
 

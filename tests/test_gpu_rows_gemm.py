@@ -108,3 +108,20 @@ def test_linear_takes_it_where_it_pays_and_gives_the_librarys_numbers(M, N, K):
         assert bool(((got.float() - library).abs() <= 2.0 ** -8 * library.abs() + K * 2.0 ** -22).all())
     sums = module.linear(x, w, None, keep_float32=True)
     assert sums.dtype == torch.float32 and float((sums - torch.mm(x.float(), w.float().T)).abs().max()) < K * 2.0 ** -22
+
+
+def test_linear_takes_rows_that_overlap_and_operands_without_elements():
+    """Expanded rows and rows of a sliding window are the library's, as they are where no product of this package pays; so is a
+    product with no features or of nothing."""
+    module = ops()
+    x, w = rand(70, 128, seed=12).to(torch.bfloat16).to(DEV), rand(48, 128, seed=13).to(torch.bfloat16).to(DEV)
+    assert module.rows_gemm_pays(70, 48, 128) and module.rows_gemm_supported(x, w)
+    row, window = x[5:6].expand(70, 128), x.view(-1).as_strided((70, 128), (64, 1))
+    for rows in (row, window):
+        assert not module.rows_gemm_supported(rows, w)
+        assert torch.equal(module.linear(rows, w, None), torch.mm(rows.contiguous(), w.t()))
+        # (W [70, 128] against x's first rows: the same numbers the other way round)
+        assert torch.equal(module.linear(x[:48], rows, None), torch.mm(x[:48], rows.contiguous().t()))
+    assert module.linear(x, w[:0], None).shape == (70, 0)
+    empty = module.linear(x[:, :0], w[:, :0], None)
+    assert empty.shape == (70, 48) and not bool(empty.any())
