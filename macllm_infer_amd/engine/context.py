@@ -296,6 +296,7 @@ class StaticStep:
       slot, the first ones of one token and the last one with the remainder.
 
     ``fill`` rewrites the arrays for the real lanes of a step."""
+    forks = False                    # whether the graph that was recorded on them runs a part of the step on a second stream
 
     def __init__(self, cache, lanes: int, max_seq_len: int, device, lengths: Sequence[int] = (),
                  want_rows: Sequence[int] = (), query_tile: int = 0, chunk_sizes: Sequence[int] = (),

@@ -29,7 +29,6 @@ from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 import torch
 
 from ..kernels import ops
-from ..parts.block import OVERLAP_MIN_TOKENS
 from ..parts.streams import PORTIONS, SECOND_HALF, SINGLES, batch_streams
 from .context import _NO_LANES, Lane, LoweredLanes, StaticStep, apply_feeds, longest_context
 
@@ -267,20 +266,15 @@ class DecodeGraphs:
             main.wait_stream(beside)
         return self._clock(side_by_side, replays)
 
-    def forks(self, key: tuple) -> bool:
-        """Whether the graph of the portions' capacity ``key`` runs its mixers on two streams."""
-        least = lambda block: getattr(getattr(block, "fusion", None), "overlap_from", OVERLAP_MIN_TOKENS)
-        return any(len(getattr(block, "mixers", ())) == 2 and key[1] >= least(block) for block in self.model.blocks)
-
     def ask_beside(self, keys: Iterable[tuple], candidates: Sequence[torch.cuda.Stream]) -> None:
         """The clock's answer to which of ``candidates`` does not stand in the way of the graphs of these capacities, for
         those that fork and have no answer yet (nothing but padding is touched).  Such a graph takes two hardware queues, of
         which the second is the runtime's choice when the graph is made, another one from graph to graph: a stream that
-        lies on it makes the graph wait (640 tokens of the 0.5B shape beside 24 decoded ones: 4.5 ms on two of four streams,
-        5.6 on the others, which are others for the graph of 1,024 tokens).  Asked by a kernel that does nothing but wait, for
+        lies on it makes the graph wait (640 tokens of the 0.5B shape with their mixers on two streams, beside 24 decoded ones: 4.5 ms
+        on two of four streams, 5.6 on the others, which are others for the graph of 1,024 tokens).  Asked by a kernel that does nothing but wait, for
         a quarter of the graph's time: five to seven replays, about what the capture cost."""
         for key in keys:
-            if key not in self._bucket_graphs or key in self._besides or not self.forks(key):
+            if key not in self._bucket_graphs or key in self._besides or not self._bucket_graphs[key][0].forks:
                 continue
             static, graph, _ = self._bucket_graphs[key]
             static.fill(_NO_LANES)
@@ -362,6 +356,8 @@ class DecodeGraphs:
             pool = self._pools.setdefault(kind, torch.cuda.graph_pool_handle())
         with torch.cuda.graph(graph, pool=pool, stream=self.streams.recording[kind]):
             logits = self.model.forward(static.context, self.cache)
+            with torch.cuda.stream(self.streams.side[kind]):         # (part of the recording from its fork to the recording's end)
+                static.forks = torch.cuda.is_current_stream_capturing()
         return static, graph, logits
 
     def run(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> torch.Tensor:

@@ -741,7 +741,7 @@ class LayerFusion:
                 self._mix_each(u, step, caches, mixed, order=(0,))
             main.wait_stream(side)
         else:
-            self._mix_each(u, step, caches, mixed)
+            self._mix_each(u, step, caches, mixed, order=range(len(self.mixers)))
         return mixed
 
     def _tune(self, weight: torch.Tensor, bias, epilogue: int, conv: Optional[dict] = None,

@@ -1437,6 +1437,38 @@ def test_portions_have_the_bits_of_the_launches_that_theirs_replace(tmp_path, mo
         assert (ours - want).abs().max().item() <= 6e-2 * want.abs().max().item()
 
 
+@pytest.mark.parametrize("name, count, forks", [("shared launches", 300, False), ("D", 300, True), ("D", 64, False)])
+def test_a_graph_is_asked_for_its_second_queue_where_it_forks(tmp_path, monkeypatch, name, count, forks):
+    """Portions whose mixers share launches fork nowhere, whatever their size: no replay is spent on the choice of a stream
+    beside them.  A graph forks where a layer took a second stream in its recording."""
+    from macllm_infer_amd import Engine, Lane
+    from macllm_infer_amd.config import FalconH1Config
+    from macllm_infer_amd.parts import block, fused
+    from macllm_infer_amd.weights.random_init import write_random_model
+    if name == "D":
+        folder = tiny_configs.make_model_dir("D", tmp_path, torch.bfloat16)
+    else:
+        folder = write_random_model(FalconH1Config.from_dict(shared_launches_config()), 5, str(tmp_path), torch.bfloat16, "unit")
+    took, asked = [], []
+    real = block.side_stream
+    monkeypatch.setattr(fused, "side_stream", lambda device, beside: (took.append(1), real(device, beside))[1])
+    engine = Engine(folder, dtype="bfloat16", kv_cache_block_tokens=16, kv_cache_capacity_tokens=4096, max_active_sequences=8,
+                    measured_paths=False)
+    graphs = engine.graphs
+    clock = graphs._clock_behind_wait
+    monkeypatch.setattr(graphs, "_clock_behind_wait", lambda *arguments: (asked.append(1), clock(*arguments))[1])
+    for turn in range(3):
+        engine.add_request("a")
+        engine.step([Lane("a", tokens_for(100, count, 60 + turn), [count - 1])])
+        engine.finish("a")
+    assert len(graphs._bucket_graphs) == 1 and bool(took) == forks
+    (key, (static, _, _)), = graphs._bucket_graphs.items()
+    assert static.forks == forks
+    graphs.ask_beside([key], graphs.streams.beside)
+    assert bool(asked) == forks and (key in graphs._besides) == forks
+    assert graphs.stream_beside(key, graphs.streams.beside) in graphs.streams.beside
+
+
 @pytest.mark.parametrize("name, dtype", [("A", "float32"), ("D", "bfloat16")])
 @pytest.mark.parametrize("count", [40, 130])
 def test_single_tokens_beside_portions_give_the_bits_of_one_batch_behind_the_other(tmp_path, monkeypatch, name, dtype, count):
