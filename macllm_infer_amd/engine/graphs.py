@@ -354,10 +354,10 @@ class DecodeGraphs:
         # one pool for every graph of a kind: their replays never overlap, so their intermediate buffers may share memory
         if pool is None:
             pool = self._pools.setdefault(kind, torch.cuda.graph_pool_handle())
+        forks = self.streams.forks[kind]
         with torch.cuda.graph(graph, pool=pool, stream=self.streams.recording[kind]):
             logits = self.model.forward(static.context, self.cache)
-            with torch.cuda.stream(self.streams.side[kind]):         # (part of the recording from its fork to the recording's end)
-                static.forks = torch.cuda.is_current_stream_capturing()
+        static.forks = self.streams.forks[kind] > forks
         return static, graph, logits
 
     def run(self, lanes: Sequence[Lane], lowered: LoweredLanes) -> torch.Tensor:

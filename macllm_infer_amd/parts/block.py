@@ -23,7 +23,7 @@ def side_stream(device: torch.device, beside: "torch.cuda.Stream") -> "torch.cud
     to one of two that belong to no such batch."""
     index = device.index if device.index is not None else torch.cuda.current_device()
     batches = batch_streams(device)
-    side = batches.side_of(beside)
+    side = batches.fork(beside)
     if side is not None:
         return side
     streams = _side_streams.setdefault(index, [])

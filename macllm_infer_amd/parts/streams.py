@@ -32,6 +32,7 @@ class BatchStreams:
         self._draw = draw
         self._taken = []
         self.recording, self.side = {}, {}
+        self.forks = dict.fromkeys(KINDS, 0)             # how often a recording of the kind took its second stream
         if usual is not None:
             self.recording[SINGLES] = usual
             self._taken.append(usual)
@@ -58,6 +59,13 @@ class BatchStreams:
             if main == self.recording[kind]:
                 return self.side[kind]
         return None
+
+    def fork(self, main: "torch.cuda.Stream") -> Optional["torch.cuda.Stream"]:
+        """``side_of(main)`` for work that is recorded there now."""
+        for kind in KINDS:
+            if main == self.recording[kind]:
+                self.forks[kind] += 1
+        return self.side_of(main)
 
     def belongs_to(self, kind: str, stream: "torch.cuda.Stream") -> bool:
         return stream == self.recording[kind] or stream == self.side[kind]

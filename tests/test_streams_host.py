@@ -102,6 +102,18 @@ def test_no_capture_of_portions_works_on_a_stream_of_the_single_tokens(cuda, dra
         assert not singles & capture()
 
 
+@pytest.mark.parametrize("kind", ["singles", "portions"])
+def test_a_recording_says_whether_it_forked(cuda, kind):
+    """By the second stream that was handed out during it, not by its size or by what other kinds of batches do."""
+    for forks in (True, False, True):
+        def forward(context, cache):
+            if forks:                                        # (a warm-up, on another stream, forks as well)
+                block.side_stream(DEVICE, cuda.current)
+        bank = graphs_module.DecodeGraphs(SimpleNamespace(forward=forward, blocks=[], step_layout={}), None, DEVICE, 4096)
+        static = SimpleNamespace(capacity=kind == "portions", context=None)
+        assert bank._capture(0, static)[0] is static and static.forks == forks
+
+
 def test_every_kind_of_batch_has_streams_of_its_own(cuda):
     of_device = streams.batch_streams(DEVICE)
     assert streams.batch_streams(DEVICE) is of_device
