@@ -998,22 +998,25 @@ def moe_tile_rows(tokens: int, top_k: int, num_experts: int, whole_pieces: bool 
 
 def moe_shared_grouped(tokens: int, width: int, hidden: int, pad: int) -> bool:
     """Whether a shared expert like the routed ones (``width`` by ``hidden``, bfloat16) runs as one more of them in the
-    grouped products of a step, in tiles of ``pad`` places: three launches less (two products and the activation between them, 10 us of small steps, 25
-    of prompts), where the matrices are small enough that those launches wait for little else.  us of the whole
-    feed-forward, apart | grouped, by tokens (experts x hidden x width, choices a token):
+    grouped products of a step, in tiles of ``pad`` places: three launches less (two products and the activation between them).
+    A step gives the same bits either way: it is grouped only where the shared expert's sums are added up in the order of
+    products of their own.  Those of up to 16 rows deal K over four waves as tiles of 16 places do, a K beyond 1,024 over eight; those
+    of 32 rows and more walk K in order, as the wider tiles do and a wave of the small ones can, but the library splits a K beyond
+    1,024, and that of 17 to 31 rows, over compute units.  K (``hidden``, then ``width``) in whole chunks of 32 (few rows of any other
+    are the library's), and tiles of 16, 64 or 128 places.  us of the whole feed-forward, replayed, apart | grouped, by tokens (experts x hidden
+    x width, choices a token):
 
-    * 16 x 1,024 x 512, 3: 1 27.7 | 20.4, 12 35.3 | 27.4, 64 62.0 | 45.8, 256 60.9 | 44.2, 777 72.8 | 52.5, 1,554 94.5 |
-      77.5, 4,096 171 | 162
-    * 64 x 1,024 x 512, 6: 12 46.3 | 41.6, 64 110 | 91, 512 105.5 | 103.9, 1,554 159 | 167 (another tile), 2,048 209 | 167
-    * 64 x 2,048 x 1,024, 6: 12 131 | 121, 64 255 | 239, 128 302 | 296, 256 390 | 402, 1,024 325 | 353, 2,048 478 | 443
-    * 8 x 3,072 x 3,072, 2: 1 65.9 | 70.0, 12 134 | 129, 64 216 | 227, 512 258 | 225, 1,024 318 | 335, 4,096 968 | 1,000
-
-    A step gives the same bits either way, except of 17 to 31 tokens, where the library splits the K of the products apart: those
-    stay apart, and so do tiles of 16 places of rows that are not whole pieces, whose kernel has the one order only."""
-    if SKINNY_ROWS < tokens < 32 or (tokens > SKINNY_ROWS and pad == MOE_TILE_ROWS and (width % 8 or hidden % 8)):
+    * 16 x 1,024 x 512, 3: 1 25.3 | 19.3, 12 30.1 | 22.1, 64 58.1 | 49.0, 256 56.9 | 44.4, 777 64.8 | 52.7, 1,554 84.2 | 75.7,
+      4,096 160 | 149
+    * 64 x 1,024 x 512, 6: 12 37.7 | 29.8, 64 71.6 | 62.5, 256 102.6 | 101.3, 512 77.3 | 65.0, 777 81.5 | 81.5, 1,554 124.1 |
+      123.5, 2,048 149 | 135
+    * 8 x 1,024 x 1,024, 2: 1 26.7 | 19.5, 12 29.7 | 21.4, 128 62.6 | 47.3, 1,024 81.0 | 69.5, 4,096 176 | 175
+    * 32 x 1,024 x 1,024, 4: 12 38.7 | 29.3, 64 75.8 | 66.7, 192 107.3 | 108.3, 512 90.0 | 75.1, 1,554 157 | 143
+    * 64 x 512 x 256, 8: 1 26.1 | 21.7, 64 62.1 | 54.7, 512 55.1 | 45.2, 2,048 92.8 | 83.4, 4,096 149 | 151
+    * 128 x 1,024 x 256, 8: 1 30.0 | 24.7, 64 81.6 | 72.1, 512 75.5 | 63.0, 4,096 249 | 249"""
+    if max(width, hidden) > 1024 or width % 32 or hidden % 32 or pad not in (MOE_TILE_ROWS, MOE_WIDE_TILE_ROWS, MOE_WIDEST_TILE_ROWS):
         return False
-    first = 2 * width * hidden
-    return first <= 1 << 21 or (first <= 1 << 22 and tokens <= 128)
+    return not SKINNY_ROWS < tokens < 32
 
 
 ROUTINGS = {"softmax_then_top": 0, "top_then_softmax": 1, "sigmoid_then_top": 2}
@@ -1128,7 +1131,7 @@ def moe_expert_gemm(x: torch.Tensor, plan: MoePlan, weight: torch.Tensor, out: t
     [capacity, I]; or with ``squared_relu`` max(weight[expert] . row, 0)^2.  Float32 sums on the matrix cores;
     float32 operands give a true 32-bit product.  ``row_scale`` float32 [capacity]: a number that multiplies a place's row
     before the product (applied, in float32, to the sums before the activation).  ``rounded``: the expert whose sums are
-    rounded to bfloat16 first and summed in the order of a product of its own of as many rows."""
+    rounded to bfloat16 first and summed in the order of a product of its own of as many rows (K up to 1,024, in chunks of 32)."""
     _need(row_scale is None or (row_scale.dtype == torch.float32 and row_scale.numel() == plan.capacity
                                 and row_scale.is_contiguous() and row_scale.is_cuda),
           "moe_expert_gemm: row_scale must be float32 [capacity] on the GPU")

@@ -33,7 +33,7 @@ class RoutedExperts(FeedForward):
     the order of the token's choices, together with the gated shared expert.  A token's result does not depend on
     which other tokens share its expert's tiles: a row of a tile is summed on its own.  The output is float32.
     Steps of up to 64 tokens are routed and grouped in one launch; a bfloat16 shared expert of the routed ones' size and
-    clamped activation runs as one more of them where that pays (``ops.moe_shared_grouped``), with the same bits; one whose activation is plain SiLU runs as
+    clamped activation runs as one more of them where that gives the same bits (``ops.moe_shared_grouped``); one whose activation is plain SiLU runs as
     the dense gated feed-forward does (its activation in the product's epilogue in small steps)."""
     graph_safe = True
     takes_tail = True

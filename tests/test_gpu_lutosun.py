@@ -335,6 +335,29 @@ def test_a_shared_expert_has_the_same_bits_grouped_and_apart(T, monkeypatch):
     assert torch.equal(grouped, part.forward(x))
 
 
+@pytest.mark.parametrize("hidden, inner, experts, top, grouped", [
+    (2048, 1024, 4, 2, False), (1024, 2048, 2, 1, False), (512, 1088, 3, 2, False), (1000, 488, 16, 3, False), (136, 200, 7, 1, False),
+    (72, 40, 5, 2, False), (1024, 1024, 4, 2, True), (1024, 96, 4, 2, True), (32, 64, 5, 2, True), (992, 480, 8, 4, True), (256, 704, 3, 1, True)])
+def test_a_shared_expert_is_grouped_where_its_bits_stay(hidden, inner, experts, top, grouped, monkeypatch):
+    """Whatever the sizes, a step gives what the shared expert's launches apart give: grouped where both orders of the sums are one."""
+    from macllm_infer_amd.config import ClampedGLUSpec, RoutedExpertsSpec
+    from macllm_infer_amd.parts.base import BuildContext
+    from macllm_infer_amd.parts.moe import RoutedExperts
+    act = ClampedGLUSpec(limit=7.0)
+    spec = RoutedExpertsSpec(num_experts=experts, top_k=top, expert_size=inner, activation=act, shared_size=inner, shared_activation=act)
+    tensors = {one.name: (rand(*one.shapes[0], seed=40 + index) / one.shapes[0][-1] ** 0.5).to(torch.bfloat16)
+               for index, one in enumerate(RoutedExperts.expected_tensors(spec, "m", hidden))}
+    part = RoutedExperts(spec, "m", tensors, BuildContext(hidden, torch.bfloat16, torch.device(DEV), 4096))
+    rule, taken = ops().moe_shared_grouped, []
+    for T in (1, 16, 17, 31, 32, 33, 64, 65, 128, 300, 1554):
+        x = rand(T, hidden, seed=T).to(torch.bfloat16).to(DEV)
+        monkeypatch.setattr(ops(), "moe_shared_grouped", lambda *sizes: taken.append(rule(*sizes)) or taken[-1])
+        ours = part.forward(x)
+        monkeypatch.setattr(ops(), "moe_shared_grouped", lambda *sizes: False)
+        assert torch.equal(ours, part.forward(x)), T
+    assert taken[0] == taken[4] == grouped and not taken[2] and not taken[3]
+
+
 # ------------------------------------------------------------------ each mechanism alone against the plain model
 def rounded(tensors, dtype):
     return {name: value.to(dtype).to(torch.float32) for name, value in tensors.items()}

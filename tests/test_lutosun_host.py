@@ -190,3 +190,15 @@ def test_tiles_of_the_grouped_products_go_by_the_matrices_too():
         assert [tile(rows, 8, columns, torch.float32) for rows in (63, 64, 255, 256)] == [16, 64, 64, 128]
         assert [tile(rows, 8, columns, torch.float32, False) for rows in (63, 64, 255, 256)] == [16, 64, 64, 64]
         assert [tile(rows, 8, columns, torch.bfloat16, False) for rows in (63, 64, 255, 256)] == [16, 64, 64, 64]
+
+
+def test_a_shared_expert_joins_the_routed_ones_where_its_sums_keep_their_order():
+    """Both products' K whole chunks of 32 and at most 1,024 (a longer one is dealt to more waves, or compute units, in launches of
+    its own), and not in steps of 17 to 31 tokens."""
+    from macllm_infer_amd.kernels import ops
+    grouped = lambda tokens, width, hidden, pad=16: ops.moe_shared_grouped(tokens, width, hidden, pad)
+    assert [tokens for tokens in range(1, 40) if not grouped(tokens, 512, 1024)] == list(range(17, 32))
+    for tokens, pad in ((1, 16), (16, 16), (32, 16), (128, 64), (4096, 128)):
+        assert all(grouped(tokens, *sizes, pad) for sizes in ((512, 1024), (1024, 1024), (32, 64), (1024, 96), (320, 992)))
+        assert not any(grouped(tokens, *sizes, pad) for sizes in ((1024, 2048), (2048, 1024), (512, 2048), (1056, 512), (200, 1024), (512, 72)))
+        assert not grouped(tokens, 512, 1024, 32)
