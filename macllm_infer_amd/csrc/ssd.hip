@@ -1248,12 +1248,21 @@ extern "C" int mi_ssd_staged(int Q, int P, int N) { return ssd_staged_sizes(P, N
 static int scan_beside_heads(int dh) { return dh == 64 ? 1 : 2; }
 
 // Whether the attention of `tokens` tokens beside the scan of n_chunks chunks is faster than on a stream of its own, whose fork and
-// join cost about 12 us a layer: us a prompt on two streams | in one launch.
-// Heads of 64, two workgroups of the launch on a compute unit (0.5B shape): 144 tokens 2,952 | 2,671, 300 3,258 | 3,023, 515 3,570 |
-// 3,411, 700 3,662 | 3,545, 800 3,785 | 3,787, 900 4,230 | 4,161, four lanes of 200 4,122 | 3,992; 300 beside four tokens behind 6,000 keys
-// 5,750 | 4,805; 4,096 in portions of 256 56,100 | 49,300, of 512 30,690 | 30,100, of 1,024 18,280 | 19,120 (18,600 with the
-// first two alone).
-// Heads of 128, one on a compute unit (twelve layers of the 7B shape): 144 2,777 | 2,677, 256 3,190 | 3,102, 300 (216 workgroups)
+// join cost about 12 us a layer: two streams | one launch in us a prompt, eight layers or more, at the workgroups of the launch in brackets.
+// Heads of 64, two workgroups on a compute unit; 24 heads of the scan beside 8 / 2 of the attention (A), 48 and 96 beside 8 / 2 (B, C), 24
+// beside 16 / 2 and 32 / 2 (D, E), 48 beside 16 / 4 (F), 96 beside 32 / 8 (G).
+// Behind contexts of up to 2,048 the line lies by the tokens, as the longest rows of keys end the launch: to 768 the one launch is
+// the faster at every number of heads (640 tokens A (496) 3,723 | 3,529, C (928) 1,727 | 1,674, E (1,552) 1,346 | 1,276; 768 A (584) 3,822 |
+// 3,768, B (752) 1,358 | 1,347, C (1,088) 1,758 | 1,753, E (1,832) 1,426 | 1,361; 150 G (1,024) 1,249 | 1,187; four lanes of 200 A (1,064)
+// 4,295 | 4,139, C (2,144) 2,196 | 2,148), to 896 where the scan's workgroups have a compute unit each (A (672) 3,912 | 3,896, two lanes of
+// 400 4,200 | 4,038, D (1,152) 2,055 | 2,032, E (2,112) 1,518 | 1,477, but B 1,359 | 1,384, C 1,791 | 1,828; 1,024 A 4,128 | 4,199, D
+// 2,125 | 2,142).  Far more
+// workgroups than that gain nothing (five lanes of 150 E (2,896) 1,431 | 1,447, four of 200 beside 192 heads (3,584) 3,497 | 3,531).
+// Behind longer ones a workgroup of the attention takes longer than one of the scan, and the line lies by their number: 4,096 tokens
+// in portions of 256 A (232) 12,508 | 10,929, F (464) 13,711 | 12,843, G (928) 20,892 | 22,592; of 384 D (392) 19,762 | 19,185, C (608) 15,459 |
+// 15,825, E (992) 14,043 | 15,073; of 512 A (408) 32,450 | 31,932, B (528) 9,909 | 9,648, D (696) 15,180 | 16,026; of 576 A (552) 32,550 |
+// 32,070; of 640 A (496) 29,093 | 27,746, B (640) 9,510 | 9,767, F (992) 15,080 | 16,531.  (States of 64 x 256 and 128 x 128 have the lines of A.)
+// Heads of 128, one on a compute unit (twelve layers of the 7B shape): 144 tokens 2,777 | 2,677, 256 3,190 | 3,102, 300 (216)
 // 3,268 | 3,213, 400 (288) 3,702 | 3,710; 4,096 in portions of 256 51,570 | 52,090, 200 beside four tokens behind 4,000 keys (528)
 // 3,750 | 3,959.
 extern "C" int mi_ssd_chunks_beside(int Q, int H, int P, int N, int n_chunks, int tokens, int Hq, int Hkv, int dh, int n_tiles,
@@ -1261,8 +1270,10 @@ extern "C" int mi_ssd_chunks_beside(int Q, int H, int P, int N, int n_chunks, in
   if (n_chunks <= 0 || !mi_ssd_staged(Q, P, N) || !mi_ssd_beside(H, P, N, Hq, Hkv, dh, n_tiles, max_seq_len)) return 0;
   const int nset = scan_beside_heads(dh);
   const long groups = (long)n_chunks * H * ((Q + 127) / 128) + 4L * n_tiles * Hkv * ((Hq / Hkv + nset - 1) / nset);
+  const long scan = (long)((tokens + Q - 1) / Q) * H * ((Q + 127) / 128);      // that work: chunks past the step's own leave at once
   const bool near = max_seq_len > 0 && max_seq_len <= 2048;
-  return groups <= 0x7fffffffL && (dh == 64 ? tokens <= (near ? 896 : 640) : near && groups <= 256) ? 1 : 0;
+  if (dh != 64) return near && groups <= 256 ? 1 : 0;
+  return near ? groups <= 2304 && tokens <= (scan <= 256 ? 896 : 768) : groups <= 560;
 }
 
 template <int NK, int PT>

@@ -162,3 +162,24 @@ def test_the_streams_of_a_callers_stream_begin_with_the_one_the_clock_found(cuda
     assert found[0] == engine.graphs.streams.beside[-1] and set(found) == set(engine.graphs.streams.beside)
     monkeypatch.setattr(engine_module.ops, "stream_beside", None)               # not asked again
     assert engine._streams_beside() is found
+
+
+def test_an_attention_rides_beside_a_scan_in_chunks_where_their_workgroups_share_the_chip():
+    """Behind long contexts the number of workgroups decides, whichever of heads, chunks and tokens they come from: a model with four
+    times the heads stops at a quarter of the tokens.  Behind short ones the tokens do, a little earlier where the scan's heads
+    are more than the compute units hold."""
+    from macllm_infer_amd.kernels import ops
+
+    def rides(tokens, longest, heads=24, query_heads=8, kv_heads=2, dh=64, lanes=1):
+        chunks, tiles = -(-tokens // 128) + lanes - 1, -(-tokens // 64) + lanes          # (of a captured step)
+        return bool(ops._fn("ssd", "mi_ssd_chunks_beside")(128, heads, 64, 128, chunks, tokens, query_heads, kv_heads, dh, tiles, longest))
+    assert [rides(tokens, 4096) for tokens in (150, 256, 640, 896)] == [True, True, True, False]
+    assert [rides(tokens, 4096, 48, 16, 4) for tokens in (150, 256, 512, 640)] == [True, True, False, False]
+    assert [rides(tokens, 4096, 96, 32, 8) for tokens in (64, 150, 256, 640)] == [True, False, False, False]
+    assert [rides(tokens, 4096, 96) for tokens in (256, 448, 640)] == [True, False, False]
+    assert [rides(tokens, 4096, query_heads=32) for tokens in (129, 256, 640)] == [True, False, False]
+    assert [rides(tokens, 2048) for tokens in (150, 768, 896, 1024)] == [True, True, True, False]
+    assert [rides(tokens, 2048, 48) for tokens in (150, 768, 896, 1024)] == [True, True, False, False]
+    assert [rides(tokens, 2048, query_heads=32) for tokens in (150, 896, 1024)] == [True, True, False]
+    assert not rides(768, 2048, query_heads=32, lanes=16) and not rides(768, 2048, 192, 32, 8)      # far more than the chip holds
+    assert not any(rides(tokens, 0, dh=128) for tokens in (129, 300))        # heads of 128 behind contexts of unknown length
