@@ -2179,10 +2179,10 @@ def test_layer_norm_of_the_stream_and_its_branches(ops, dtype, T, d):
                                                              ([16] * 5, [3, 0, 950, 16, 690], 600, 2048),
                                                              ([129], [0], None, 2048), ([300, 1, 128], [0, 700, 33], None, 2048),
                                                              ([256], [777], 600, 2048)])
-def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, window, longest):
+def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, window, longest, Q=128):
     """Lanes of one chunk of up to 128 tokens, and of several, behind contexts: the rotation, the cache, the attended rows, the scan's outputs,
     states and tails are the same bits in the scan's launches and in launches of their own; a row of the table of runs that holds none."""
-    page_size, G, K, Q = 16, 1, 4, 128
+    page_size, G, K = 16, 1, 4
     E, GN, T, lanes = H * P, G * N, sum(counts), len(counts)
     C, A_cols = E + 2 * GN, (Hq + 2 * Hkv) * dh
     lengths = [start + count for start, count in zip(starts, counts)]
@@ -2226,6 +2226,14 @@ def test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H
         results.append((rows, pages, s, t, mixed))
     for apart, joined in zip(*results):
         assert torch.isfinite(joined.float()).all() and torch.equal(apart, joined)
+
+
+@pytest.mark.parametrize("H, P, N, Hq, Hkv, dh", [(24, 64, 128, 8, 2, 64), (3, 64, 128, 4, 1, 64), (4, 128, 256, 12, 2, 128), (3, 64, 256, 6, 2, 64)])
+@pytest.mark.parametrize("Q, counts, starts", [(256, [300, 5], [0, 700]), (256, [200], [0]), (256, [450], [40]),
+                                               (32, [100, 33, 1], [0, 5, 9]), (96, [200, 97], [3, 0])])
+def test_prompt_attention_beside_a_scan_in_chunks_of_other_sizes(ops, H, P, N, Hq, Hkv, dh, Q, counts, starts):
+    """Chunks of 256 tokens, whose scan is two workgroups a head, with a last chunk that fills one of them or both, and small ones."""
+    test_prompt_attention_in_the_scans_launches_gives_the_bits_of_its_own(ops, H, P, N, Hq, Hkv, dh, counts, starts, None, 2048, Q)
 
 
 @pytest.mark.parametrize("H, P, N, Hq, Hkv, dh", [(24, 64, 128, 8, 2, 64), (3, 64, 128, 4, 1, 64), (4, 128, 256, 12, 2, 128)])

@@ -250,6 +250,35 @@ def test_the_grouped_products_and_the_weighted_sum(dtype, T, experts, top, hidde
     close(got, want, torch.float32, "the weighted sum")
 
 
+@pytest.mark.parametrize("T, experts, top, identity, how", [
+    (1024, 5, 8, 3, "weighted"), (8193, 3, 1, 1, "weighted"), (1366, 64, 6, 0, "shared"), (2048, 16, 6, 4, "weighted"), (2048, 16, 6, 4, "shared"),
+    (4096, 130, 3, 2, "plain"), (777, 4, 20, 2, "shared")])
+def test_the_plan_of_more_choices_than_its_workgroup_keeps(T, experts, top, identity, how):
+    """Up to 8,192 choices stay in registers and the ones behind go through memory: 8,192, one more, and thousands more, with choices of
+    experts without matrices, weights beside the places and a shared expert's rows in front."""
+    generator = torch.Generator().manual_seed(T + top)
+    chosen = torch.randint(0, experts + identity, (T, top), generator=generator, dtype=torch.int32)
+    weights = torch.rand(T, top, generator=generator) + 0.5
+    plan = ops().moe_plan(chosen.to(DEV), experts, 64, weights.to(DEV) if how == "weighted" else None, shared=how == "shared")
+    source, place, tile_expert, flat = plan.source.cpu(), plan.place.cpu().long(), plan.tile_expert.cpu(), chosen.reshape(-1)
+    stands, entries = flat < experts, torch.arange(T * top)
+    front = -(-T // 64) * 64 if how == "shared" else 0
+    assert torch.equal(place >= 0, stands)
+    at = place[stands]
+    assert at.unique().numel() == at.numel() and (not at.numel() or int(at.min()) >= front)
+    assert torch.equal(source[at].long(), entries[stands] // top) and torch.equal(tile_expert[at // 64], flat[stands])
+    assert int((source >= 0).sum()) == at.numel() + (T if front else 0)
+    counts = torch.bincount(flat[stands].long(), minlength=experts)
+    assert tile_expert[front // 64:].tolist() == (
+        lambda tiles: tiles + [-1] * (tile_expert.numel() - front // 64 - len(tiles)))([e for e in range(experts) for _ in range(-(-int(counts[e]) // 64))])
+    if front:
+        assert source[:front].tolist() == list(range(T)) + [-1] * (front - T) and tile_expert[:front // 64].eq(experts).all()
+    if how == "weighted":
+        beside = torch.zeros(plan.capacity)
+        beside[at] = weights.reshape(-1)[stands]
+        assert torch.equal(plan.place_weight.cpu(), beside)
+
+
 @pytest.mark.parametrize("T, experts, top, pad", [(1, 4, 2, 16), (15, 5, 3, 16), (16, 5, 3, 16), (17, 3, 3, 16), (64, 70, 6, 16),
                                                    (65, 4, 2, 64), (130, 4, 2, 64), (300, 3, 2, 128)])
 def test_a_shared_experts_rows_stand_in_front_of_the_choices(T, experts, top, pad):
