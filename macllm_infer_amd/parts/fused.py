@@ -713,14 +713,17 @@ class LayerFusion:
 
     def forward_general(self, residual: Residual, step, caches) -> None:
         block = self.block
-        normed = block.mixer_norm.forward(residual)
-        if self.padding_pays[_portion_bucket(normed.shape[0])]:
-            u = ops.linear(normed, self.w_in_wide, self.b_in_wide)
-        else:
-            u = ops.linear(normed, self.w_in, self.b_in)
-        residual.pending = [ops.linear(self._general_mixers(u, step, caches), self.w_out, self.b_out)]
+        # (no normed rows are held past their product: what is allocated next takes their place, and the layer fewer lines of the caches)
+        u = self._general_input(block.mixer_norm.forward(residual))
+        mixed = self._general_mixers(u, step, caches)
+        residual.pending = [ops.linear(mixed, self.w_out, self.b_out)]
         normed = block.ffn_norm.forward(residual)
         residual.pending = [block.ffn.forward(normed)]
+
+    def _general_input(self, normed: torch.Tensor) -> torch.Tensor:
+        if self.padding_pays[_portion_bucket(normed.shape[0])]:
+            return ops.linear(normed, self.w_in_wide, self.b_in_wide)
+        return ops.linear(normed, self.w_in, self.b_in)
 
     def _general_mixers(self, u: torch.Tensor, step, caches) -> torch.Tensor:
         mixed = torch.empty((u.shape[0], self.mixed_width), dtype=u.dtype, device=u.device)
