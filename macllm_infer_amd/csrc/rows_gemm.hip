@@ -13,8 +13,8 @@
 // 540), the launch and the lines written at its end (2,048 x 4,096 with K = 64: 8.9 us).  So it is at its best where the tiles
 // fit the chip once, which is where the library is at its worst: us, library | this, rows and weights from memory: 65 x 1,024 x
 // 1,024 8.3 | 6.5, 1,554 x 1,024 x 1,024 10.6 | 8.6, 1,554 x 1,024 x 512 8.6 | 6.4, 640 x 1,024 x 2,048 10.9 | 9.9; with the
-// activation (the library's product and the launch behind it) 256 x 4,096 x 1,024 14.0 | 6.7, 640 rows 18.1 | 13.1, 2,048 rows
-// 28 | 22.6; and where it is not: 2,048 x 1,024 x 2,048 18.0 | 17.7, 1,999 x 6,144 x 1,024 31 | 40, 2,048 x 24,576 x 3,072 with the
+// activation (the library's product and the launch behind it) 256 x 4,096 x 1,024 15.1 | 8.0, 640 rows 19.0 | 13.9, 2,048 rows
+// 27 | 23.0; and where it is not: 2,048 x 1,024 x 2,048 18.0 | 17.7, 1,999 x 6,144 x 1,024 31 | 40, 2,048 x 24,576 x 3,072 with the
 // activation 253 | 310.
 #include "common.h"
 

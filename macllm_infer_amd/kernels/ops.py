@@ -1461,16 +1461,15 @@ def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False, keep_float32: b
       beyond, the library splits K over the compute units
 
     ``swiglu``: of a gated feed-forward, with the activation in the product | the library's product and the activation
-    behind it (2,048 to 8,192 features):
+    behind it (33 to 8,192 rows, 1,024 to 16,384 features):
 
-    * K = 512: 0.49 to 0.8
-    * K = 1,024: 0.51 0.58 0.60; 0.59 0.63 0.67; 0.60 0.70 0.74; 128 x 128 twice 0.78 0.83 0.89, more 0.73 0.90 1.05 (of up to 4,096
-      features 0.73 to 0.96)
-    * K = 2,048: 0.70 0.77 0.86; 0.68 0.86 0.93; 0.79 0.80 0.87; twice 0.87 0.98 1.11, more 0.91 1.15 1.31
+    * K = 512: 0.41 0.49 0.53; 0.43 0.50 0.51; 0.52 0.55 0.58; 128 x 128 twice 0.53 0.57 0.70, more 0.54 0.82 0.99
+    * K = 1,024: 0.52 0.54 0.58; 0.58 0.64 0.68; 0.66 0.69 0.73; twice 0.82 0.87 0.95, more 0.78 1.04 1.14
+    * K = 2,048: 0.75 0.80 0.82; 0.67 0.85 0.97; 0.79 0.81 0.86; twice 0.91 0.95 1.07, more 1.15 1.22 1.28
 
     ``keep_float32``: sums that are not rounded, of K up to 64 only.  The library's order of them is nearer to the exact sum (17
-    features of K = 1,024: relative error 0.95e-7, in k order 1.9e-7).  Rounded products of 32 rows and more have the library's
-    bits; it splits K where there are fewer."""
+    features of K = 1,024: relative error 0.95e-7, in k order 1.9e-7).  Rounded products of 32 rows and 64 features or more have the
+    library's bits at K up to 1,024 (and plain ones wherever they are taken beyond); it splits K where there are fewer, or K is longer."""
     if M < 32 or (keep_float32 and K > 64):
         return False
     tiles = lambda rows, features: -(-M // rows) * -(-N // features)
@@ -1478,7 +1477,7 @@ def rows_gemm_pays(M: int, N: int, K: int, swiglu: bool = False, keep_float32: b
     if swiglu:
         if K <= 512:
             return True
-        return K <= 2048 and (large <= GEMM_UNITS or (K <= 1024 and (large <= 2 * GEMM_UNITS or N <= 4096)))
+        return K <= 2048 and large <= (2 if K <= 1024 else 1) * GEMM_UNITS
     if K <= 512:
         return small or wide or large <= GEMM_UNITS
     if K <= 1024:
