@@ -202,3 +202,12 @@ def test_a_shared_expert_joins_the_routed_ones_where_its_sums_keep_their_order()
         assert all(grouped(tokens, *sizes, pad) for sizes in ((512, 1024), (1024, 1024), (32, 64), (1024, 96), (320, 992)))
         assert not any(grouped(tokens, *sizes, pad) for sizes in ((1024, 2048), (2048, 1024), (512, 2048), (1056, 512), (200, 1024), (512, 72)))
         assert not grouped(tokens, 512, 1024, 32)
+
+
+def test_the_gated_product_of_many_rows_is_taken_up_to_two_tiles_a_compute_unit():
+    """Beyond, at K of more than 512, the library's product with the activation behind it is as fast."""
+    from macllm_infer_amd.kernels import ops
+    gated = lambda rows, features, K: ops.rows_gemm_pays(rows, features, K, swiglu=True)
+    assert [rows for rows in (31, 32, 2048, 2049, 4096) if gated(rows, 4096, 1024)] == [32, 2048]
+    assert gated(4096, 2048, 1024) and not gated(4097, 2048, 1024) and gated(8192, 16384, 512)
+    assert gated(1024, 4096, 2048) and not gated(1025, 4096, 2048) and not gated(64, 4096, 2112)
